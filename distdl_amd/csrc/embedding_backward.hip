@@ -6,27 +6,37 @@
 //
 // for the rows r of the shard window [lo, hi); tokens outside the window and
 // tokens equal to padding_idx contribute nothing.  No atomics on the gradient:
-// the tokens are first bucketed by table row (a counting sort on 32-bit
-// counters), then one wavefront per (row, column chunk) adds the dy rows of its
-// bucket in fp32, in ascending token order, and writes every element of
-// dweight exactly once -- rows nobody looked up get their zeros from the same
+// the tokens are first bucketed by table row, then every bucket's dy rows are
+// added in fp32, in ascending token order, and every element of dweight is
+// written exactly once -- rows nobody looked up get their zeros from the same
 // pass, so dweight needs no clearing.
 //
-//   emb_bwd_clear    count = cursor = 0
+//   emb_bwd_clear    counters = 0
 //   emb_bwd_count    count[row]++ per token in the window
-//   emb_bwd_fill     begin = exclusive prefix sum of count, formed by every workgroup for itself in LDS
-//                    (no launch of its own, no kernel boundary to wait behind); bucket[begin[row] + cursor[row]++] = t
-//   emb_bwd_reduce   a workgroup per row (or per few rows of a narrow table): buckets longer than a wavefront are put
-//                    in ascending token order first (bitonic network over the workgroup), short ones in registers;
-//                    then sum, scale, convert, store
+//   emb_bwd_place    a stretch of the bucket array for every row.  The stretches lie in no particular order, so
+//                    no prefix sum over the whole table is needed: a workgroup scans its own 1024 counters and takes its
+//                    place with one atomic.  Rows of more than kHotAbove tokens go on the list of hot rows.
+//   emb_bwd_fill     bucket[end[row]++] = t
+//   emb_bwd_hot      the sums of hot rows: a workgroup per row and 256 bytes of columns (hot_row); not launched
+//                    when there are too few tokens for a hot row
+//   emb_bwd_reduce   the sums of all other rows: one wavefront (half a wavefront for narrow tables) per row and group
+//                    of columns, the bucket ordered in registers
 //
 // The order in which the fill kernel's atomics hand out bucket slots varies
-// from run to run; both sorts exist so that the fp32 sums do not.  Tables of
-// more rows than a workgroup's LDS holds counters for get their prefix sum from
-// a kernel of its own (emb_bwd_scan) in front of the fill kernel.
+// from run to run; the reduce kernel orders every bucket so that the fp32 sums
+// do not.
+//
+// What bounds it: the gradient rows read once and the table written once, plus
+// the four short kernels in front (2-5 us each, launch and memory latency).
+// Token ids as they occur in text make a few rows hot: of 8192 tokens over
+// 50304 rows with ids distributed log-uniformly, 483 share one row.  A single
+// wavefront walking that bucket one token at a time -- a memory round trip per
+// token -- took 1140 us for [50304,512] fp32 where the whole call can take 25.
 #include "ddl_common.h"
 
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 // Workspace of ddl_embedding_backward_static: the counters, bucket cursors, bucket starts and
 // token buckets of one call, for callers that cannot hand over (or allocate)
@@ -40,12 +50,11 @@ namespace {
 constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
-constexpr int kScanBlock = 1024;
-constexpr int kChunk = 512;    // columns per wavefront of the reduce kernel: 8 per lane
 
-__global__ __launch_bounds__(kBlock) void emb_bwd_clear(int32_t* __restrict__ p, int64_t n) {
+__global__ __launch_bounds__(kBlock) void emb_bwd_clear(int32_t* __restrict__ count, int64_t rows, int32_t* __restrict__ totals) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i < n) p[i] = 0;
+    if (i < rows) count[i] = 0;
+    if (i < 2) totals[i] = 0;
 }
 
 template <typename IdT>
@@ -54,445 +63,510 @@ __device__ inline int64_t token_row(const IdT* __restrict__ ids, int64_t t, int6
     return (id >= lo && id < hi && id != padding_idx) ? id - lo : -1;
 }
 
+// The lanes of a wavefront whose tokens share a row take their places with one
+// atomic: `first` receives the lane that issues it, `before` the number of such
+// lanes below this one, and the number of such lanes is returned.  Ids as in text
+// put hundreds of tokens on one counter, which serves them one after the other
+// (8192 such tokens over 50304 rows: count and fill 10 + 11 us without this).
+__device__ inline int same_row_lanes(int32_t row, bool on, int lane, int* first, int* before) {
+    uint64_t todo = __ballot(on);
+    int size = 0;
+    *first = lane, *before = 0;
+    while (todo) {                                    // the same in all lanes
+        const int leader = __ffsll(static_cast<unsigned long long>(todo)) - 1;
+        const int32_t r = __builtin_amdgcn_readlane(row, leader);
+        const uint64_t same = __ballot(row == r) & todo;
+        if ((same >> lane) & 1) {
+            *first = leader;
+            *before = __popcll(same & ((1ull << lane) - 1));
+            size = __popcll(same);
+        }
+        todo &= ~same;
+    }
+    return size;
+}
+
 template <typename IdT>
 __global__ __launch_bounds__(kBlock) void emb_bwd_count(const IdT* __restrict__ ids, int64_t n_ids, int64_t lo, int64_t hi,
                                                         int64_t padding_idx, int32_t* __restrict__ count) {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (t >= n_ids) return;
-    const int64_t r = token_row(ids, t, lo, hi, padding_idx);
-    if (r >= 0) atomicAdd(&count[r], 1);
+    const int32_t r = t < n_ids ? static_cast<int32_t>(token_row(ids, t, lo, hi, padding_idx)) : -1;
+    const int lane = threadIdx.x & (kWave - 1);
+    int first, before;
+    const int size = same_row_lanes(r, r >= 0, lane, &first, &before);
+    if (r >= 0 && before == 0) atomicAdd(&count[r], size);
 }
 
-// Exclusive prefix sum of count[0..n) into start[0..n), one workgroup, 16384
-// counters per round.  The counters come in and the sums go out with
-// consecutive lanes on consecutive addresses; in between they sit in LDS, where
-// a thread owns 16 consecutive ones (pitch 17 keeps the lanes on different
-// banks).  Thread totals are scanned across the wavefront with shuffles, the 16
-// wavefront totals through LDS.
-constexpr int kScanItems = 16;
-constexpr int kScanWaves = kScanBlock / kWave;
-constexpr int kScanRound = kScanBlock * kScanItems;
-__device__ inline int scan_slot(int i) { return i + (i >> 4); }
-__global__ __launch_bounds__(kScanBlock) void emb_bwd_scan(const int32_t* __restrict__ count, int64_t n, int32_t* __restrict__ start) {
-    __shared__ int32_t stage[kScanRound + kScanRound / 16];
-    __shared__ int32_t wave_total[kScanWaves];
-    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-    int32_t carry = 0;                                         // sum of all earlier rounds, the same in every thread
-    for (int64_t base = 0; base < n; base += kScanRound) {
+// Stretches of the bucket array.  end[row] is where the row's stretch begins;
+// the fill kernel advances it to where it ends.  totals[0]: slots handed out so
+// far, totals[1]: entries of the hot list.  The last row of the table never goes
+// on the list (it is looked at in any case), so the list has at most rows - 1 entries.
+constexpr int kPlaceRows = 4;                     // consecutive rows of a thread
+__global__ __launch_bounds__(kBlock) void emb_bwd_place(const int32_t* __restrict__ count, int64_t rows, int32_t hot_above,
+                                                        int32_t* __restrict__ end, int32_t* __restrict__ hot, int32_t* __restrict__ totals) {
+    __shared__ int32_t wave_total[kWavesPerBlock];
+    __shared__ int32_t base;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * kPlaceRows;
+    int32_t n[kPlaceRows], total = 0;
 #pragma unroll
-        for (int j = 0; j < kScanItems; ++j) {
-            const int i = j * kScanBlock + t;
-            stage[scan_slot(i)] = base + i < n ? count[base + i] : 0;
-        }
-        __syncthreads();
-        int32_t v[kScanItems];
-        int32_t total = 0;
+    for (int k = 0; k < kPlaceRows; ++k) {
+        n[k] = r0 + k < rows ? count[r0 + k] : 0;
+        total += n[k];
+    }
+    int32_t incl = total;                                      // inclusive scan over the wavefront
 #pragma unroll
-        for (int k = 0; k < kScanItems; ++k) {
-            v[k] = stage[scan_slot(t * kScanItems + k)];
-            total += v[k];
-        }
-        int32_t incl = total;                                  // inclusive scan over the wavefront
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t up = __shfl_up(incl, off, kWave);
+        if (lane >= off) incl += up;
+    }
+    if (lane == kWave - 1) wave_total[wave] = incl;
+    __syncthreads();
+    int32_t before = 0, all = 0;
 #pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-            const int32_t up = __shfl_up(incl, off, kWave);
-            if (lane >= off) incl += up;
-        }
-        if (lane == kWave - 1) wave_total[wave] = incl;
-        __syncthreads();
-        int32_t before = 0, all = 0;
+    for (int k = 0; k < kWavesPerBlock; ++k) {
+        before += k < wave ? wave_total[k] : 0;
+        all += wave_total[k];
+    }
+    if (threadIdx.x == 0) base = all ? atomicAdd(&totals[0], all) : 0;
+    __syncthreads();
+    int32_t run = base + before + incl - total;
 #pragma unroll
-        for (int k = 0; k < kScanWaves; ++k) {
-            const int32_t wt = wave_total[k];
-            before += k < wave ? wt : 0;
-            all += wt;
-        }
-        int32_t run = carry + before + incl - total;
-#pragma unroll
-        for (int k = 0; k < kScanItems; ++k) {
-            stage[scan_slot(t * kScanItems + k)] = run;
-            run += v[k];
-        }
-        carry += all;
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kScanItems; ++j) {
-            const int i = j * kScanBlock + t;
-            if (base + i < n) start[base + i] = stage[scan_slot(i)];
-        }
-        __syncthreads();                                       // stage and wave_total are rewritten by the next round
+    for (int k = 0; k < kPlaceRows; ++k) {
+        if (r0 + k >= rows) break;
+        end[r0 + k] = run;
+        run += n[k];
+        if (n[k] > hot_above && r0 + k < rows - 1) hot[atomicAdd(&totals[1], 1)] = static_cast<int32_t>(r0 + k);
     }
 }
 
-// Bucket fill.  SCAN: every workgroup forms the exclusive prefix sum of the
-// counters for itself, in LDS (a thread owns ceil(rows / 1024) consecutive
-// counters; thread totals are scanned across the wavefront with shuffles, the
-// 16 wavefront totals through LDS), workgroup 0 also writes it to `begin` for the
-// reduce kernel; otherwise `begin` has been filled by emb_bwd_scan.  A token's
-// slot is begin[row] plus the number of tokens of that row that came before it
-// in this run (an atomic counter per row, zero on entry).
-constexpr int kFillBlock = 1024;
-constexpr int kFillWaves = kFillBlock / kWave;
-constexpr int64_t kFillScanRows = 32768;  // counters a workgroup scans in LDS (128 KiB)
-
-template <typename IdT, bool SCAN>
-__global__ __launch_bounds__(kFillBlock) void emb_bwd_fill(const IdT* __restrict__ ids, int64_t n_ids, int64_t lo, int64_t hi,
-                                                           int64_t padding_idx, const int32_t* __restrict__ count,
-                                                           int32_t* __restrict__ begin, int32_t* __restrict__ cursor,
-                                                           int32_t* __restrict__ bucket) {
-    // Counter i sits in slot i + i / per, per = counters per thread (a power of two): a thread walks consecutive slots,
-    // the lanes of a wavefront are per + 1 slots apart and so on different banks.
-    __shared__ int32_t base[SCAN ? kFillScanRows + kFillBlock : 1];
-    __shared__ int32_t wave_total[kFillWaves];
-    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-    // The token's row and its place among the tokens of that row first: neither waits for the prefix sum.
-    const int64_t tok = static_cast<int64_t>(blockIdx.x) * kFillBlock + t;
-    const int64_t r = tok < n_ids ? token_row(ids, tok, lo, hi, padding_idx) : -1;
-    const int32_t place = r >= 0 ? atomicAdd(&cursor[r], 1) : 0;
-    int per_log = 0;
-    if (SCAN) {
-        const int32_t rows = static_cast<int32_t>(hi - lo);
-        while ((kFillBlock << per_log) < rows) ++per_log;
-        const int32_t per = 1 << per_log;
-        for (int32_t i = t; i < rows; i += kFillBlock) base[i + (i >> per_log)] = count[i];
-        __syncthreads();
-        const int32_t i0 = t << per_log, i1 = i0 + per < rows ? i0 + per : rows;
-        int32_t* const mine = base + i0 + t;                   // slot of counter i0
-        int32_t total = 0;
-        for (int32_t i = i0; i < i1; ++i) total += mine[i - i0];
-        int32_t incl = total;                                  // inclusive scan over the wavefront
-#pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-            const int32_t up = __shfl_up(incl, off, kWave);
-            if (lane >= off) incl += up;
-        }
-        if (lane == kWave - 1) wave_total[wave] = incl;
-        __syncthreads();
-        int32_t before = 0, all = 0;
-#pragma unroll
-        for (int k = 0; k < kFillWaves; ++k) {
-            const int32_t wt = wave_total[k];
-            before += k < wave ? wt : 0;
-            all += wt;
-        }
-        int32_t run = before + incl - total;
-        for (int32_t i = i0; i < i1; ++i) {
-            const int32_t c = mine[i - i0];
-            mine[i - i0] = run;
-            run += c;
-        }
-        __syncthreads();
-        if (blockIdx.x == 0) {
-            for (int32_t i = t; i < rows; i += kFillBlock) begin[i] = base[i + (i >> per_log)];
-            if (t == 0) begin[rows] = all;
-        }
-    }
-    if (r >= 0) bucket[(SCAN ? base[r + (r >> per_log)] : begin[r]) + place] = static_cast<int32_t>(tok);
+template <typename IdT>
+__global__ __launch_bounds__(kBlock) void emb_bwd_fill(const IdT* __restrict__ ids, int64_t n_ids, int64_t lo, int64_t hi,
+                                                       int64_t padding_idx, int32_t* __restrict__ end, int32_t* __restrict__ bucket) {
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const int32_t r = t < n_ids ? static_cast<int32_t>(token_row(ids, t, lo, hi, padding_idx)) : -1;
+    const int lane = threadIdx.x & (kWave - 1);
+    int first, before;
+    const int size = same_row_lanes(r, r >= 0, lane, &first, &before);
+    int32_t slot = 0;
+    if (r >= 0 && before == 0) slot = atomicAdd(&end[r], size);
+    slot = __shfl(slot, first, kWave) + before;
+    if (r >= 0) bucket[slot] = static_cast<int32_t>(t);
 }
 
-// Ascending order of a bucket of more than 64 tokens, by the whole workgroup.
-// The network is the bitonic sort in the form whose exchanges all put the
-// smaller key first: partner of i is its mirror image inside blocks of k in the
-// first pass of a merge, i + j in the others.  Keys beyond the end of the bucket
-// count as +infinity and never move, so any length works.  Buckets of up to
-// kSortLds tokens are sorted in LDS and written back, longer ones where they
-// lie (a workgroup's stores are visible to its own later loads once the barrier
-// between the passes has been passed; the loads are volatile so that none is
-// served from a stale cache line).
-constexpr int kSortLds = 4096;
+// Elements: bf16 or fp16 bits or float; all are summed in fp32 and rounded once on the way out.
+struct Bf16 {
+    typedef uint16_t word;
+    static __device__ float widen(uint16_t u) { return __uint_as_float(static_cast<uint32_t>(u) << 16); }
+    static __device__ uint16_t round(float f) {
+        const __bf16 b = static_cast<__bf16>(f);
+        uint16_t u;
+        __builtin_memcpy(&u, &b, 2);
+        return u;
+    }
+};
+struct F16 {
+    typedef uint16_t word;
+    static __device__ float widen(uint16_t u) {
+        _Float16 h;
+        __builtin_memcpy(&h, &u, 2);
+        return static_cast<float>(h);
+    }
+    static __device__ uint16_t round(float f) {
+        const _Float16 h = static_cast<_Float16>(f);
+        uint16_t u;
+        __builtin_memcpy(&u, &h, 2);
+        return u;
+    }
+};
+struct F32 {
+    typedef float word;
+    static __device__ float widen(float f) { return f; }
+    static __device__ float round(float f) { return f; }
+};
 
-template <typename P>
-__device__ inline void bitonic_passes(P a, int32_t n) {
-    int32_t pow2 = 1;
-    while (pow2 < n) pow2 <<= 1;
-    for (int32_t k = 2; k <= pow2; k <<= 1) {
-        for (int32_t j = k >> 1; j > 0; j >>= 1) {
-            const bool mirror = j == (k >> 1);
-            for (int32_t t = threadIdx.x; t < (pow2 >> 1); t += kBlock) {
-                int32_t i, l;
-                if (mirror) {
-                    const int32_t blk = t / j, off = t - blk * j;
-                    i = blk * k + off;
-                    l = blk * k + k - 1 - off;
-                } else {
-                    const int32_t blk = t / j, off = t - blk * j;
-                    i = blk * 2 * j + off;
-                    l = i + j;
-                }
-                if (l < n) {
-                    const int32_t lo = a[i], hi = a[l];
-                    if (lo > hi) {
-                        a[i] = hi;
-                        a[l] = lo;
-                    }
-                }
+// V consecutive elements in one access, aligned to an element only (gfx950 serves
+// 16-byte accesses at any alignment, and a copy of rows of odd length runs at
+// nine tenths of the aligned rate).
+template <typename W, int V>
+struct Pack {
+    W e[V];
+};
+template <typename W, int V>
+__device__ inline Pack<W, V> load_pack(const W* p) {
+    typedef W raw __attribute__((ext_vector_type(V)));
+    typedef raw loose __attribute__((aligned(sizeof(W))));
+    const raw r = *reinterpret_cast<const loose*>(p);
+    Pack<W, V> out;
+    __builtin_memcpy(&out, &r, sizeof(out));
+    return out;
+}
+template <typename W, int V>
+__device__ inline void store_pack(W* p, const Pack<W, V>& v) {   // streaming: the gradient is not read again here
+    typedef W raw __attribute__((ext_vector_type(V)));
+    typedef raw loose __attribute__((aligned(sizeof(W))));
+    raw r;
+    __builtin_memcpy(&r, &v, sizeof(r));
+    __builtin_nontemporal_store(r, reinterpret_cast<loose*>(p));
+}
+
+struct ReduceArgs {
+    const void* dy;
+    void* dw;
+    int64_t dim, ld_dy, ld_dw, rows;
+    const int32_t* count;
+    const int32_t* end;
+    const int32_t* bucket;
+    const int32_t* hot;
+    const int32_t* totals;
+    int64_t n_ids;
+    int32_t nv;             // vectors of V elements per row; the last one is moved back to end with the row
+    int32_t passes;         // groups of columns per row of the ordinary path
+    int32_t rows_per_block;
+    int32_t hot_above;      // rows of more tokens are hot
+    int32_t hot_chunks;     // 256-byte pieces of a row
+    int32_t scale_by_freq;
+};
+
+// ---- hot rows ----
+// A workgroup owns 256 bytes of columns of one row.  What takes time is the
+// memory round trip, not the additions, so all threads fetch the pieces of the
+// next two batches of 64 tokens -- 16 lanes a token, 16 bytes a lane -- while one
+// wavefront adds a batch in token order out of LDS, a column (or two 16-bit ones)
+// per lane: the sums stay strictly sequential per column with 128 tokens in
+// flight.  (A wavefront that walks its columns alone keeps 32 in flight in the
+// same registers: 55 us instead of 20 for 483 tokens of 2 KiB.)
+// The order of the tokens: up to 512 by counting the smaller ones, more through
+// a bit per token number in LDS (the stage's 16 KiB hold 131072 of them) that is
+// read back in ascending order, kListTokens at a time.
+constexpr int kHotAbove = 32;                        // rows of more tokens are hot: what half a wavefront's lanes order, and as long as
+                                                     // the ordinary walk stays below the time of everything else (with 64: 24 us, with 32: 17)
+constexpr int kHotBytes = 256;
+constexpr int kHotBatch = 64;                        // tokens per batch
+constexpr int kListTokens = 1024;
+constexpr int kRankTokens = 2 * kBlock;
+constexpr int kBitWords = kHotBytes * kHotBatch / 4;
+constexpr int kBitsPerWindow = kBitWords * 32;
+constexpr int kWordsPerThread = kBitWords / kBlock;
+
+struct HotShared {
+    uint32_t bits[kBitWords];                        // pieces of a batch, a bit per token number, or the bucket being ordered
+    int32_t list[kListTokens];                       // tokens in ascending order
+    int32_t wave_total[kWavesPerBlock];
+};
+
+// Adds the first m tokens of the list to the columns from col0 on; called by all threads.
+template <typename E>
+__device__ inline void hot_accumulate(HotShared& sh, const ReduceArgs& a, int64_t col0, int m, float (&acc)[2]) {
+    typedef typename E::word W;
+    constexpr int V = 16 / sizeof(W);
+    constexpr int kLanesPerToken = 16, kTokensPerLoad = kBlock / kLanesPerToken, kLoads = kHotBatch / kTokensPerLoad;
+    const int t = threadIdx.x, part = t % kLanesPerToken, tok0 = t / kLanesPerToken;
+    const int64_t col = col0 + part * V, left = a.dim - col;
+    const W* const dy = static_cast<const W*>(a.dy) + col;
+    uint4 piece[2][kLoads];
+    auto fetch = [&](uint4 (&to)[kLoads], int base) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const int i = base + u * kTokensPerLoad + tok0;
+            to[u] = make_uint4(0, 0, 0, 0);
+            if (i >= m || left <= 0) continue;
+            const W* src = dy + static_cast<int64_t>(sh.list[i]) * a.ld_dy;
+            Pack<W, V> v;
+            if (left >= V) {
+                v = load_pack<W, V>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < V; ++e) v.e[e] = e < left ? src[e] : W(0);
             }
-            __syncthreads();
+            __builtin_memcpy(&to[u], &v, 16);
         }
+    };
+    auto batch = [&](uint4 (&from)[kLoads], int base) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+            *reinterpret_cast<uint4*>(&sh.bits[(u * kTokensPerLoad + tok0) * (kHotBytes / 4) + part * 4]) = from[u];
+        __syncthreads();
+        if (base + 2 * kHotBatch < m) fetch(from, base + 2 * kHotBatch);
+        if (t < kWave) {
+            const int here = m - base < kHotBatch ? m - base : kHotBatch;
+            auto add = [&](uint32_t w) {
+                if constexpr (sizeof(W) == 4) {
+                    acc[0] += __uint_as_float(w);
+                } else {
+                    acc[0] += E::widen(static_cast<uint16_t>(w));
+                    acc[1] += E::widen(static_cast<uint16_t>(w >> 16));
+                }
+            };
+            int k = 0;
+            for (; k + 16 <= here; k += 16) {
+                uint32_t w[16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) w[u] = sh.bits[(k + u) * (kHotBytes / 4) + t];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) add(w[u]);
+            }
+            for (; k < here; ++k) add(sh.bits[k * (kHotBytes / 4) + t]);
+        }
+        __syncthreads();
+    };
+    fetch(piece[0], 0);
+    if (kHotBatch < m) fetch(piece[1], kHotBatch);
+    for (int base = 0; base < m; base += 2 * kHotBatch) {
+        batch(piece[0], base);
+        if (base + kHotBatch < m) batch(piece[1], base + kHotBatch);
     }
 }
 
 // Called by every thread of the workgroup with the same arguments.
-__device__ inline void sort_bucket_long(int32_t* stage, int32_t* bucket, int32_t n) {
-    if (n <= kSortLds) {
-        for (int32_t i = threadIdx.x; i < n; i += kBlock) stage[i] = bucket[i];
+template <typename E>
+__device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, int chunk) {
+    typedef typename E::word W;
+    const int32_t n = a.count[row];
+    const int32_t* const bucket = a.bucket + (a.end[row] - n);
+    const int t = threadIdx.x;
+    const int64_t col0 = static_cast<int64_t>(chunk) * (kHotBytes / sizeof(W));
+    float acc[2] = {0.f, 0.f};
+    if (n <= kRankTokens) {
+        int32_t* const raw = reinterpret_cast<int32_t*>(sh.bits);
+        // two tokens per thread; INT_MAX behind the bucket's end is smaller than nothing
+        const int32_t t0 = t < n ? bucket[t] : 0x7FFFFFFF, t1 = t + kBlock < n ? bucket[t + kBlock] : 0x7FFFFFFF;
+        raw[t] = t0, raw[t + kBlock] = t1;
         __syncthreads();
-        bitonic_passes(stage, n);
-        for (int32_t i = threadIdx.x; i < n; i += kBlock) bucket[i] = stage[i];
+        int rank0 = 0, rank1 = 0;
+#pragma unroll 4
+        for (int k = 0; k < n; k += 4) {
+            const int4 q = *reinterpret_cast<const int4*>(&raw[k]);
+            rank0 += (q.x < t0) + (q.y < t0) + (q.z < t0) + (q.w < t0);
+            rank1 += (q.x < t1) + (q.y < t1) + (q.z < t1) + (q.w < t1);
+        }
+        if (t < n) sh.list[rank0] = t0;
+        if (t + kBlock < n) sh.list[rank1] = t1;
+        __syncthreads();
+        hot_accumulate<E>(sh, a, col0, n, acc);
     } else {
-        bitonic_passes(static_cast<volatile int32_t*>(bucket), n);
-    }
-    __syncthreads();   // the bucket is in order for every wavefront of the workgroup; stage may be refilled
-}
-
-// Elements: uint16_t holds bf16 bits, f16_bits fp16 bits; both are summed in fp32 and rounded once on the way out.
-struct f16_bits {
-    uint16_t u;
-};
-__device__ inline float f16_to_f32(uint16_t u) {
-    _Float16 h;
-    __builtin_memcpy(&h, &u, 2);
-    return static_cast<float>(h);
-}
-__device__ inline uint16_t f32_to_f16(float f) {
-    const _Float16 h = static_cast<_Float16>(f);
-    uint16_t u;
-    __builtin_memcpy(&u, &h, 2);
-    return u;
-}
-__device__ inline float load_as_f32(const uint16_t* p) { return __uint_as_float(static_cast<uint32_t>(*p) << 16); }
-__device__ inline float load_as_f32(const f16_bits* p) { return f16_to_f32(p->u); }
-__device__ inline float load_as_f32(const float* p) { return *p; }
-
-__device__ inline void store_from_f32(uint16_t* p, float f) {
-    uint32_t u = __float_as_uint(f);
-    uint16_t b = 0x7FC0;
-    if (f == f) {
-        u += 0x7FFFu + ((u >> 16) & 1u);
-        b = static_cast<uint16_t>(u >> 16);
-    }
-    *p = b;
-}
-__device__ inline void store_from_f32(f16_bits* p, float f) { p->u = f32_to_f16(f); }
-__device__ inline void store_from_f32(float* p, float f) { *p = f; }
-
-// Order of the tokens of a bucket of at most 64: lane i holds one token and
-// counts the smaller ones (its rank), then every lane picks the token whose
-// rank is its own lane number.  Ascending token order makes the sums
-// independent of how the fill kernel's atomics interleaved; longer buckets are
-// put in order by sort_bucket_long.
-__device__ inline int32_t sort_bucket(int32_t mine, int32_t m, int lane) {
-    int32_t rank = 0;
-    for (int k = 0; k < m; ++k) rank += __shfl(mine, k, kWave) < mine ? 1 : 0;
-    int32_t sorted = 0x7FFFFFFF;
-    for (int k = 0; k < m; ++k) {
-        const int32_t tk = __shfl(mine, k, kWave), rk = __shfl(rank, k, kWave);
-        if (rk == lane) sorted = tk;
-    }
-    return sorted;
-}
-
-// Both reduce kernels: a workgroup owns rows_per_block consecutive rows
-// (one when a row has work for all four wavefronts, more for narrow tables).
-// First its long buckets are sorted, one after the other, by all its threads;
-// then wavefront w takes the items (row, group of columns) w, w + 4, ...
-struct RowsOfBlock {
-    int64_t row0;
-    int n_rows;        // rows of this workgroup that exist
-    int32_t n0, b0;    // tokens and first slot of row0 (fetched once: most workgroups own one row)
-};
-__device__ inline RowsOfBlock sort_long_buckets_of_block(const int32_t* __restrict__ count, const int32_t* __restrict__ begin,
-                                                        int32_t* bucket, int64_t rows, int rows_per_block, int32_t* stage) {
-    RowsOfBlock rb;
-    rb.row0 = static_cast<int64_t>(blockIdx.x) * rows_per_block;
-    const int64_t left = rows - rb.row0;
-    rb.n_rows = left < rows_per_block ? static_cast<int>(left) : rows_per_block;
-    rb.n0 = count[rb.row0];                                   // the grid has no workgroup without a row
-    rb.b0 = begin[rb.row0];
-    if (rb.n0 > kWave) sort_bucket_long(stage, bucket + rb.b0, rb.n0);
-    for (int q = 1; q < rb.n_rows; ++q) {                     // the same trip count and branches in every thread
-        const int32_t n = count[rb.row0 + q];
-        if (n > kWave) sort_bucket_long(stage, bucket + begin[rb.row0 + q], n);
-    }
-    return rb;
-}
-
-// Tokens base .. base + 63 of a bucket, one per lane.  A bucket that this
-// workgroup has just sorted is read around the vector cache.
-__device__ inline int32_t bucket_tokens(const int32_t* bucket, int32_t b0, int32_t base, int32_t m, int32_t n, int lane) {
-    if (lane >= m) return 0x7FFFFFFF;
-    if (n > kWave) return *static_cast<const volatile int32_t*>(bucket + b0 + base + lane);
-    return bucket[b0 + base + lane];
-}
-
-// Wavefront item (row, chunk): columns chunk * kChunk + lane + 64 j, j = 0..7.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void emb_bwd_reduce(const T* __restrict__ dy, int64_t dim, int64_t ld_dy,
-                                                         const int32_t* __restrict__ count, const int32_t* __restrict__ begin,
-                                                         int32_t* bucket, int64_t rows, int chunks, int rows_per_block,
-                                                         T* __restrict__ dw, int64_t ld_dw, int scale_by_freq) {
-    __shared__ int32_t stage[kSortLds];
-    const RowsOfBlock rb = sort_long_buckets_of_block(count, begin, bucket, rows, rows_per_block, stage);
-    const int lane = threadIdx.x & (kWave - 1);
-    for (int item = threadIdx.x / kWave; item < rb.n_rows * chunks; item += kWavesPerBlock) {
-        const int q = item / chunks, chunk = item - q * chunks;
-        const int64_t row = rb.row0 + q;
-        const int32_t b0 = q ? begin[row] : rb.b0, n = q ? count[row] : rb.n0;
-        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        const int64_t c0 = static_cast<int64_t>(chunk) * kChunk + lane;
-        for (int32_t base = 0; base < n; base += kWave) {
-            const int32_t m = n - base < kWave ? n - base : kWave;
-            int32_t mine = bucket_tokens(bucket, b0, base, m, n, lane);
-            if (n <= kWave) mine = sort_bucket(mine, m, lane);
-            for (int k = 0; k < m; ++k) {
-                const int64_t t = __shfl(mine, k, kWave);
-                const T* src = dy + t * ld_dy;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int64_t c = c0 + 64 * j;
-                    if (c < dim) acc[j] += load_as_f32(src + c);
+        const int lane = t & (kWave - 1), wave = t / kWave;
+        for (int64_t w0 = 0; w0 < a.n_ids; w0 += kBitsPerWindow) {
+            for (int32_t first = 0, in_window = 1; first < in_window; first += kListTokens) {
+                for (int i = t; i < kBitWords; i += kBlock) sh.bits[i] = 0;
+                __syncthreads();
+                for (int32_t i = t; i < n; i += kBlock) {
+                    const int64_t at = bucket[i] - w0;
+                    if (at >= 0 && at < kBitsPerWindow) atomicOr(&sh.bits[at >> 5], 1u << (at & 31));
                 }
+                __syncthreads();
+                int32_t mine = 0;
+                for (int k = 0; k < kWordsPerThread; ++k) mine += __popc(sh.bits[t * kWordsPerThread + k]);
+                int32_t incl = mine;
+#pragma unroll
+                for (int off = 1; off < kWave; off <<= 1) {
+                    const int32_t up = __shfl_up(incl, off, kWave);
+                    if (lane >= off) incl += up;
+                }
+                if (lane == kWave - 1) sh.wave_total[wave] = incl;
+                __syncthreads();
+                int32_t rank = incl - mine;
+                in_window = 0;
+#pragma unroll
+                for (int k = 0; k < kWavesPerBlock; ++k) {
+                    rank += k < wave ? sh.wave_total[k] : 0;
+                    in_window += sh.wave_total[k];
+                }
+                for (int k = 0; k < kWordsPerThread; ++k) {
+                    uint32_t bits = sh.bits[t * kWordsPerThread + k];
+                    while (bits) {
+                        const int b = __ffs(bits) - 1;
+                        bits &= bits - 1;
+                        if (rank >= first && rank < first + kListTokens)
+                            sh.list[rank - first] = static_cast<int32_t>(w0) + (t * kWordsPerThread + k) * 32 + b;
+                        ++rank;
+                    }
+                }
+                __syncthreads();
+                const int32_t here = in_window - first;
+                if (here > 0) hot_accumulate<E>(sh, a, col0, here < kListTokens ? here : kListTokens, acc);
             }
         }
-        T* dst = dw + row * ld_dw;
-        const float scale = (scale_by_freq && n > 1) ? 1.0f / static_cast<float>(n) : 1.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int64_t c = c0 + 64 * j;
-            if (c < dim) store_from_f32(dst + c, acc[j] * scale);
+    }
+    if (t < kWave) {
+        const float scale = (a.scale_by_freq && n > 1) ? 1.0f / static_cast<float>(n) : 1.0f;
+        W* const dst = static_cast<W*>(a.dw) + row * a.ld_dw + col0;
+        if constexpr (sizeof(W) == 4) {
+            if (col0 + t < a.dim) dst[t] = acc[0] * scale;
+        } else {
+            if (col0 + 2 * t < a.dim) dst[2 * t] = E::round(acc[0] * scale);
+            if (col0 + 2 * t + 1 < a.dim) dst[2 * t + 1] = E::round(acc[1] * scale);
         }
+    }
+    __syncthreads();                                 // the list is rewritten by the workgroup's next row
+}
+
+// A launch of its own: with the hot rows' registers and LDS the ordinary rows,
+// which live on many wavefronts, took 64 us instead of 50 for [16032,4096] bf16.
+template <typename E>
+__global__ __launch_bounds__(kBlock) void emb_bwd_hot(const ReduceArgs a) {
+    __shared__ HotShared sh;
+    // the list, and the last row of the table if it is hot
+    const int32_t listed = a.totals[1];
+    const int32_t items = (listed + (a.count[a.rows - 1] > a.hot_above ? 1 : 0)) * a.hot_chunks;
+    for (int32_t item = static_cast<int32_t>(blockIdx.x); item < items; item += static_cast<int32_t>(gridDim.x)) {
+        const int32_t which = item / a.hot_chunks;
+        hot_row<E>(sh, a, which < listed ? a.hot[which] : a.rows - 1, item - which * a.hot_chunks);
     }
 }
 
-// The same for bf16 or fp16 (HALF) rows that can be moved 16 bytes at a time: a lane owns the
-// eight consecutive columns chunk * kChunk + 8 lane .. + 7, so one load
-// instruction of the wavefront covers a chunk, and an item is a group of CPW
-// chunks of its row so that the loads of a token overlap and the walk through
-// the bucket is paid once for all of them.
-template <int CPW, bool HALF>
-__global__ __launch_bounds__(kBlock) void emb_bwd_reduce_bf16x8(const uint16_t* __restrict__ dy, int64_t dim, int64_t ld_dy,
-                                                                const int32_t* __restrict__ count, const int32_t* __restrict__ begin,
-                                                                int32_t* bucket, int64_t rows, int groups, int rows_per_block,
-                                                                uint16_t* __restrict__ dw, int64_t ld_dw, int scale_by_freq) {
-    __shared__ int32_t stage[kSortLds];
-    const RowsOfBlock rb = sort_long_buckets_of_block(count, begin, bucket, rows, rows_per_block, stage);
-    const int lane = threadIdx.x & (kWave - 1);
-    for (int item = threadIdx.x / kWave; item < rb.n_rows * groups; item += kWavesPerBlock) {
-        const int q = item / groups, group = item - q * groups;
-        const int64_t row = rb.row0 + q;
-        const int32_t b0 = q ? begin[row] : rb.b0, n = q ? count[row] : rb.n0;
-        float acc[CPW][8];
+// ---- ordinary rows ----
+// V: elements per vector (16 bytes, or 1 for rows shorter than that).  LPR lanes
+// share a row (32: two rows per wavefront, for rows of at most 32 vectors), CPW
+// vectors per lane and pass.  Buckets (of at most kHotAbove tokens) are ordered in
+// registers: lane i holds one token, counts the smaller ones (its rank) and sends
+// it to the lane of that number (lanes without a token send theirs, larger than
+// any, to the lane behind the last).
+template <typename E, int V, int LPR, int CPW>
+__global__ __launch_bounds__(kBlock, 8) void emb_bwd_reduce(const ReduceArgs a) {
+    typedef typename E::word W;
+    constexpr int kGroups = kWave / LPR;
+    const int lane = threadIdx.x & (kWave - 1), g = lane / LPR, gl = lane % LPR;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * a.rows_per_block;
+    const int items = a.rows_per_block / kGroups * a.passes;
+    const W* const dy = static_cast<const W*>(a.dy);
+    for (int item = threadIdx.x / kWave; item < items; item += kWavesPerBlock) {
+        const int q = item / a.passes, pass = item - q * a.passes;
+        const int64_t row = row0 + q * kGroups + g;
+        const bool real = row < a.rows;
+        int32_t n = real ? a.count[row] : 0;
+        const bool mine_to_write = real && n <= a.hot_above;
+        if (!mine_to_write) n = 0;
+        int32_t m = __builtin_amdgcn_readlane(n, 0);
+        if (kGroups == 2) {
+            const int32_t m1 = __builtin_amdgcn_readlane(n, kWave - 1);
+            m = m > m1 ? m : m1;
+        }
+        float acc[CPW][V];
 #pragma unroll
         for (int j = 0; j < CPW; ++j)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[j][e] = 0.f;
-        const int64_t c0 = static_cast<int64_t>(group) * CPW * kChunk + lane * 8;   // dim is a multiple of 8 on this path
-        for (int32_t base = 0; base < n; base += kWave) {
-            const int32_t m = n - base < kWave ? n - base : kWave;
-            int32_t mine = bucket_tokens(bucket, b0, base, m, n, lane);
-            if (n <= kWave) mine = sort_bucket(mine, m, lane);
-            for (int k = 0; k < m; ++k) {
-                const int64_t t = __shfl(mine, k, kWave);
-                const uint16_t* src = dy + t * ld_dy + c0;
-                uint4 q[CPW];
-#pragma unroll
-                for (int j = 0; j < CPW; ++j) q[j] = c0 + j * kChunk < dim ? *reinterpret_cast<const uint4*>(src + j * kChunk) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-                for (int j = 0; j < CPW; ++j) {
-                    const uint32_t w4[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        acc[j][2 * e] += HALF ? f16_to_f32(static_cast<uint16_t>(w4[e])) : __uint_as_float(w4[e] << 16);
-                        acc[j][2 * e + 1] += HALF ? f16_to_f32(static_cast<uint16_t>(w4[e] >> 16)) : __uint_as_float(w4[e] & 0xFFFF0000u);
-                    }
-                }
-            }
-        }
-        uint16_t* dst = dw + row * ld_dw + c0;
-        const float scale = (scale_by_freq && n > 1) ? 1.0f / static_cast<float>(n) : 1.0f;
+            for (int e = 0; e < V; ++e) acc[j][e] = 0.f;
+        int64_t col[CPW];
+        bool on[CPW];
 #pragma unroll
         for (int j = 0; j < CPW; ++j) {
-            if (c0 + j * kChunk >= dim) continue;
-            uint16_t o[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (HALF)
-                    o[e] = f32_to_f16(acc[j][e] * scale);
-                else
-                    store_from_f32(&o[e], acc[j][e] * scale);
+            const int64_t v = static_cast<int64_t>(pass) * (LPR * CPW) + j * LPR + gl;
+            on[j] = v < a.nv;
+            col[j] = v * V;
+            if (col[j] > a.dim - V) col[j] = a.dim - V;          // the last vector ends with the row (or a lane has none)
+        }
+        if (m > 0) {                                             // the same in all lanes
+            int32_t tok = gl < n ? a.bucket[a.end[row] - n + gl] : 0x7FFFFFFF;
+            if (m > 1) {
+                int rank = 0;
+                for (int k = 0; k < m; ++k) rank += __shfl(tok, g * LPR + k, kWave) < tok ? 1 : 0;
+                tok = __builtin_amdgcn_ds_permute((g * LPR + rank) << 2, tok);
             }
-            uint4 q;
-            q.x = o[0] | (static_cast<uint32_t>(o[1]) << 16);
-            q.y = o[2] | (static_cast<uint32_t>(o[3]) << 16);
-            q.z = o[4] | (static_cast<uint32_t>(o[5]) << 16);
-            q.w = o[6] | (static_cast<uint32_t>(o[7]) << 16);
-            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));   // streaming store: the gradient is not read again here
-            u32x4 nv;
-            nv[0] = q.x, nv[1] = q.y, nv[2] = q.z, nv[3] = q.w;
-            __builtin_nontemporal_store(nv, reinterpret_cast<u32x4*>(dst + j * kChunk));
+            auto add_tokens = [&](int k0, auto count) {
+                constexpr int U = decltype(count)::value;
+                Pack<W, V> v[U][CPW];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int32_t at = __shfl(tok, g * LPR + k0 + u, kWave);
+                    const W* src = dy + static_cast<int64_t>(kGroups == 1 || k0 + u < n ? at : 0) * a.ld_dy;   // token 0 exists
+#pragma unroll
+                    for (int j = 0; j < CPW; ++j) v[u][j] = load_pack<W, V>(src + col[j]);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int j = 0; j < CPW; ++j)
+#pragma unroll
+                        for (int e = 0; e < V; ++e) acc[j][e] += (kGroups == 1 || k0 + u < n) ? E::widen(v[u][j].e[e]) : 0.f;
+            };
+            int k = 0;
+            constexpr int kMost = (CPW == 1 ? 4 : 2) * (sizeof(W) == 4 ? 2 : 1);   // what 64 registers hold
+            for (; k + kMost <= m; k += kMost) add_tokens(k, std::integral_constant<int, kMost>{});
+            if (kMost > 4 && k + 4 <= m) {
+                add_tokens(k, std::integral_constant<int, 4>{});
+                k += 4;
+            }
+            if (kMost > 2 && k + 2 <= m) {
+                add_tokens(k, std::integral_constant<int, 2>{});
+                k += 2;
+            }
+            if (k < m) add_tokens(k, std::integral_constant<int, 1>{});
+        }
+        if (!mine_to_write) continue;
+        W* const dst = static_cast<W*>(a.dw) + row * a.ld_dw;
+        const float scale = (a.scale_by_freq && n > 1) ? 1.0f / static_cast<float>(n) : 1.0f;
+#pragma unroll
+        for (int j = 0; j < CPW; ++j) {
+            if (!on[j]) continue;
+            Pack<W, V> o;
+#pragma unroll
+            for (int e = 0; e < V; ++e) o.e[e] = E::round(acc[j][e] * scale);
+            store_pack<W, V>(dst + col[j], o);
         }
     }
 }
 
-// Rows a workgroup of the reduce kernels takes: one when a row has items for
-// all four wavefronts (or three), else as many as fill them.
-inline int rows_per_block_for(int items_per_row) { return items_per_row >= 3 ? 1 : kWavesPerBlock / items_per_row; }
-
-template <int CPW>
-void launch_reduce_x8(const void* dy, int64_t dim, int64_t ld_dy, const int32_t* count, const int32_t* begin, int32_t* bucket,
-                      int64_t rows, int chunks, void* dw, int64_t ld_dw, int scale_by_freq, bool half, hipStream_t s) {
-    const int groups = (chunks + CPW - 1) / CPW;
-    const int rpb = rows_per_block_for(groups);
-    const dim3 grid(static_cast<uint32_t>((rows + rpb - 1) / rpb));
-    if (half)
-        hipLaunchKernelGGL((emb_bwd_reduce_bf16x8<CPW, true>), grid, dim3(kBlock), 0, s, static_cast<const uint16_t*>(dy), dim, ld_dy, count,
-                           begin, bucket, rows, groups, rpb, static_cast<uint16_t*>(dw), ld_dw, scale_by_freq);
+template <typename E, int V>
+void launch_reduce(ReduceArgs a, hipStream_t s) {
+    a.nv = static_cast<int32_t>((a.dim + V - 1) / V);
+    auto go = [&](auto kernel, int lpr, int cpw) {
+        a.passes = (a.nv + lpr * cpw - 1) / (lpr * cpw);
+        // One row per workgroup when a row has work for three or four wavefronts, else as many rows as fill them.
+        a.rows_per_block = a.passes >= 3 ? 1 : (kWave / lpr) * (kWavesPerBlock / a.passes);
+        const int64_t blocks = (a.rows + a.rows_per_block - 1) / a.rows_per_block;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0, s, a);
+    };
+    if (a.nv <= 32)
+        go(emb_bwd_reduce<E, V, 32, 1>, 32, 1);
+    else if (a.nv <= 64)
+        go(emb_bwd_reduce<E, V, 64, 1>, 64, 1);
     else
-        hipLaunchKernelGGL((emb_bwd_reduce_bf16x8<CPW, false>), grid, dim3(kBlock), 0, s, static_cast<const uint16_t*>(dy), dim, ld_dy, count,
-                           begin, bucket, rows, groups, rpb, static_cast<uint16_t*>(dw), ld_dw, scale_by_freq);
+        go(emb_bwd_reduce<E, V, 64, 2>, 64, 2);
+}
+
+template <typename E>
+void launch_reduce_any(const ReduceArgs& a, uint32_t hot_blocks, hipStream_t s) {
+    constexpr int V = 16 / sizeof(typename E::word);
+    if (hot_blocks > 0) hipLaunchKernelGGL(emb_bwd_hot<E>, dim3(hot_blocks), dim3(kBlock), 0, s, a);
+    if (a.dim >= V)
+        launch_reduce<E, V>(a, s);
+    else
+        launch_reduce<E, 1>(a, s);
 }
 
 template <typename IdT>
 int run(const void* dy, int dtype, int64_t dim, int64_t ld_dy, const IdT* ids, int64_t n_ids, int64_t lo, int64_t hi,
         int64_t padding_idx, int scale_by_freq, void* dw, int64_t ld_dw, int32_t* ws, hipStream_t s) {
     const int64_t rows = hi - lo;
-    int32_t* count = ws;                 // [rows]      tokens of each row
-    int32_t* cursor = ws + rows;         // [rows]      slots of each bucket handed out so far
-    int32_t* begin = cursor + rows;      // [rows + 1]  first slot of each bucket
-    int32_t* bucket = begin + rows + 1;  // [n_ids]
+    const int es = dtype == DDL_DT_F32 ? 4 : 2;
+    ReduceArgs a{};
+    a.dy = dy, a.dw = dw, a.dim = dim, a.ld_dy = ld_dy, a.ld_dw = ld_dw, a.rows = rows, a.n_ids = n_ids;
+    a.scale_by_freq = scale_by_freq;
+    a.hot_above = kHotAbove;
+    // 3 rows + 1 + n_ids integers: the hot list has at most rows - 1 entries
+    int32_t* const count = ws;                              // [rows]      tokens of each row
+    int32_t* const end = ws + rows;                         // [rows]      next free slot of each row's stretch
+    int32_t* const totals = end + rows;                     // [2]
+    int32_t* const bucket = totals + 2;                     // [n_ids]
+    int32_t* const hot = bucket + n_ids;                    // [rows - 1]
+    a.count = count, a.end = end, a.bucket = bucket, a.hot = hot, a.totals = totals;
+    const int64_t most_hot = std::min(rows, n_ids / (a.hot_above + 1));
+    a.hot_chunks = static_cast<int32_t>((dim * es + kHotBytes - 1) / kHotBytes);
+    const uint32_t hot_blocks = static_cast<uint32_t>(std::min<int64_t>(most_hot * a.hot_chunks, 1024));
     auto grid = [](int64_t n) { return dim3(static_cast<uint32_t>((n + kBlock - 1) / kBlock)); };
-    hipLaunchKernelGGL(emb_bwd_clear, grid(2 * rows), dim3(kBlock), 0, s, count, 2 * rows);
-    if (n_ids > 0) hipLaunchKernelGGL((emb_bwd_count<IdT>), grid(n_ids), dim3(kBlock), 0, s, ids, n_ids, lo, hi, padding_idx, count);
-    const dim3 fgrid(static_cast<uint32_t>((n_ids + kFillBlock - 1) / kFillBlock));
-    if (rows <= kFillScanRows) {
-        // Without tokens one workgroup still runs: it writes `begin` (all zeros).
-        hipLaunchKernelGGL((emb_bwd_fill<IdT, true>), n_ids > 0 ? fgrid : dim3(1), dim3(kFillBlock), 0, s, ids, n_ids, lo, hi, padding_idx,
-                           count, begin, cursor, bucket);
-    } else {
-        hipLaunchKernelGGL(emb_bwd_scan, dim3(1), dim3(kScanBlock), 0, s, count, rows, begin);
-        if (n_ids > 0)
-            hipLaunchKernelGGL((emb_bwd_fill<IdT, false>), fgrid, dim3(kFillBlock), 0, s, ids, n_ids, lo, hi, padding_idx, count, begin,
-                               cursor, bucket);
+    hipLaunchKernelGGL(emb_bwd_clear, grid(std::max<int64_t>(rows, 2)), dim3(kBlock), 0, s, count, rows, totals);
+    if (n_ids > 0) {
+        hipLaunchKernelGGL((emb_bwd_count<IdT>), grid(n_ids), dim3(kBlock), 0, s, ids, n_ids, lo, hi, padding_idx, count);
+        hipLaunchKernelGGL(emb_bwd_place, grid((rows + kPlaceRows - 1) / kPlaceRows), dim3(kBlock), 0, s, count, rows, a.hot_above, end, hot, totals);
+        hipLaunchKernelGGL((emb_bwd_fill<IdT>), grid(n_ids), dim3(kBlock), 0, s, ids, n_ids, lo, hi, padding_idx, end, bucket);
     }
-    const int chunks = static_cast<int>((dim + kChunk - 1) / kChunk);
-    const bool half = dtype == DDL_DT_F16;
-    const bool vec = (dtype == DDL_DT_BF16 || half) && dim % 8 == 0 && ld_dy % 8 == 0 && ld_dw % 8 == 0 && aligned_to(dy, 16) && aligned_to(dw, 16);
-    if (vec) {
-        if (chunks >= 2) launch_reduce_x8<2>(dy, dim, ld_dy, count, begin, bucket, rows, chunks, dw, ld_dw, scale_by_freq, half, s);
-        else launch_reduce_x8<1>(dy, dim, ld_dy, count, begin, bucket, rows, chunks, dw, ld_dw, scale_by_freq, half, s);
-    } else {
-        const int rpb = rows_per_block_for(chunks);
-        const dim3 rgrid(static_cast<uint32_t>((rows + rpb - 1) / rpb));
-        if (half)
-            hipLaunchKernelGGL((emb_bwd_reduce<f16_bits>), rgrid, dim3(kBlock), 0, s, static_cast<const f16_bits*>(dy), dim, ld_dy, count,
-                               begin, bucket, rows, chunks, rpb, static_cast<f16_bits*>(dw), ld_dw, scale_by_freq);
-        else if (dtype == DDL_DT_BF16)
-            hipLaunchKernelGGL((emb_bwd_reduce<uint16_t>), rgrid, dim3(kBlock), 0, s, static_cast<const uint16_t*>(dy), dim, ld_dy, count,
-                               begin, bucket, rows, chunks, rpb, static_cast<uint16_t*>(dw), ld_dw, scale_by_freq);
-        else
-            hipLaunchKernelGGL((emb_bwd_reduce<float>), rgrid, dim3(kBlock), 0, s, static_cast<const float*>(dy), dim, ld_dy, count, begin,
-                               bucket, rows, chunks, rpb, static_cast<float*>(dw), ld_dw, scale_by_freq);
-    }
+    if (dtype == DDL_DT_F16)
+        launch_reduce_any<F16>(a, hot_blocks, s);
+    else if (dtype == DDL_DT_BF16)
+        launch_reduce_any<Bf16>(a, hot_blocks, s);
+    else
+        launch_reduce_any<F32>(a, hot_blocks, s);
     return check_launch("embedding backward");
 }
 
@@ -562,7 +636,7 @@ extern "C" int ddl_embedding_backward(const void* dy, int dtype, int64_t dim, in
     if (workspace_elems < need)
         return fail(DDL_E_ARG, "embedding backward: workspace of %lld int32 is smaller than the %lld needed (3 rows + 1 + tokens)",
                     (long long)workspace_elems, (long long)need);
-    const int64_t chunks = (dim + kChunk - 1) / kChunk;
+    const int64_t chunks = (dim + 63) / 64;
     if (rows >= 0x7FFFFFFFll || chunks > 0xFFFFFF) return fail(DDL_E_UNSUPP, "embedding backward: too many workgroups or columns");
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (ids_is_i64)

@@ -1026,6 +1026,29 @@ def test_embedding_backward_long_buckets_are_summed_in_token_order(ops, dtype):
         assert torch.equal(again.view(as_bits), first.view(as_bits))
 
 
+@pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 5), (torch.bfloat16, 8), (torch.bfloat16, 255), (torch.float16, 264),
+                                       (torch.bfloat16, 515), (torch.float16, 1999), (torch.float32, 3), (torch.float32, 127),
+                                       (torch.float32, 129), (torch.float32, 259), (torch.float32, 770)])
+@pytest.mark.parametrize("misses", [0, 150000])
+def test_embedding_backward_bucket_lengths(ops, dtype, dim, misses):
+    """Buckets of the lengths at which their handling changes (in registers up
+    to 32 tokens, by counting up to 512, by bits per token number beyond, 1024 of
+    them at a time; token numbers beyond 131072 need a second window), rows of
+    whole and partial vectors and more than one group of columns, the last row of
+    the table hot.  Small integers: every sum is exact in fp32, so the result is
+    the exact sum rounded once."""
+    lengths = [1, 2, 3, 31, 32, 33, 64, 65, 0, 511, 512, 513, 1024, 1025, 2500, 40]
+    gen = torch.Generator().manual_seed(dim)
+    if misses and dim > 8:
+        pytest.skip("the second window does not depend on the width of the rows")
+    ids = torch.cat([torch.full((n,), r) for r, n in enumerate(lengths)] + [torch.full((misses,), 99)])
+    ids = ids[torch.randperm(ids.numel(), generator=gen)]
+    dy = torch.randint(-1, 2, (ids.numel(), dim), generator=gen)
+    got = ops.embedding_backward(dy.to(dtype).cuda(), ids.cuda(), 0, len(lengths))
+    want = torch.zeros(100, dim, dtype=torch.float64).index_add_(0, ids, dy.double())[:len(lengths)]
+    assert torch.equal(got.cpu(), want.to(dtype))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_embedding_backward_scale_grad_by_freq(ops, dtype):
     """Each row's sum divided by its number of contributing tokens, against the
