@@ -115,6 +115,9 @@ SIGNATURES = {
                            c_int64, c_void_p]),
     "ddl_gemm": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64, c_int64,
                          c_int64, c_int64, c_void_p]),
+    "ddl_gemm_ws": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64, c_int64,
+                            c_int64, c_int64, c_void_p, c_int64, c_void_p]),
+    "ddl_gemm_workspace": (c_int64, [c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64]),
     "ddl_gemm_f32": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64,
                              c_int64, c_int64, c_void_p]),
     "ddl_colsum": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p]),

@@ -56,26 +56,13 @@
 //              Workgroup ids are regrouped so that the 32 workgroups resident on
 //              one XCD cover a compact patch of the tile grid and share their
 //              operand panels in that XCD's L2
-#include "gemm_tiles.h"
-#include <hip/hip_fp16.h>
+#include "gemm16_small.h"
 #include <type_traits>
 
 namespace ddl {
 namespace {
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
-
 constexpr int BK = kRowBytes / 2;   // 16-bit elements of a k-tile
-
-__device__ inline uint16_t f32_to_bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if (f != f) return 0x7FC0;
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
-}
-
-__device__ inline float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
 
 // acc += a . b (16 x 16 x 32, bf16 in, fp32 accumulate).  Written as assembly
 // so that the accumulators live in the accumulation registers ("a" operands):
@@ -90,27 +77,6 @@ __device__ inline void mfma_16x16x32(floatx4& acc, const bf16x8& a, const bf16x8
         asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
     else
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-
-// 16-bit element <-> fp32, round to nearest even on the way back.
-template <bool F16>
-__device__ inline float elem_to_f32(uint16_t b) {
-    if (F16) {
-        __half h;
-        __builtin_memcpy(&h, &b, 2);
-        return __half2float(h);
-    }
-    return bf16_bits_to_f32(b);
-}
-template <bool F16>
-__device__ inline uint16_t f32_to_elem(float f) {
-    if (F16) {
-        const __half h = __float2half_rn(f);
-        uint16_t b;
-        __builtin_memcpy(&b, &h, 2);
-        return b;
-    }
-    return f32_to_bf16_bits(f);
 }
 
 // NWM x NWN wavefronts, each owning TM x TN sub-tiles of 16 x 16: the workgroup
@@ -153,14 +119,14 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     // buffers that start at the tile's first row: a 32-bit byte offset per lane,
     // the k-tile offset in a scalar.
     //
-    // Operand contiguous along k: instruction j of this wavefront fills rows
+    // Operand16 contiguous along k: instruction j of this wavefront fills rows
     // (J wave + j) 8 .. +7 of an operand tile (J instructions per wavefront);
     // lane l lands on row l / 8, physical chunk l % 8 of that row, i.e. logical
     // chunk (l % 8) ^ ((row >> 1) & 7): the eight lanes of a row fetch one whole
     // 128-byte line.  Rows past the end of the matrix repeat its last row (their
     // products are never stored).
     //
-    // Operand contiguous along its rows ("transposed": element (row, k) lies at
+    // Operand16 contiguous along its rows ("transposed": element (row, k) lies at
     // k ld + row): the tile is kept in LDS as panels of 64 rows, each panel 64
     // k-lines of 128 bytes.  Instruction j of wavefront v fills k-lines 8 v .. +7
     // of panel j; lane l lands on k-line l / 8, physical chunk l % 8, and fetches
@@ -232,7 +198,7 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     const std::integral_constant<bool, WT> w_kind{};
     const std::integral_constant<bool, XT> x_kind{};
 
-    // Fragment addresses.  Operand contiguous along k: row (sub-tile origin +
+    // Fragment addresses.  Operand16 contiguous along k: row (sub-tile origin +
     // l16), logical chunk 4 ks + kg; sub-tile origins are multiples of 16, so the
     // swizzle term is (l16 >> 1) & 7.
     const int frag_row = l16 * (BK * 2);
@@ -523,17 +489,8 @@ const Kernel kKernels[8] = {
 
 std::atomic<bool> lds_reserved[kMaxDevices][16];   // the dynamic LDS size of kKernels[i] (8 + i: kLowKernels[i]) has been raised on that device (first use, any thread)
 
-// One operand of the product: element (row, k) at p[row * row_stride + k * k_stride],
-// one of the strides being 1.
-struct Operand {
-    const uint16_t* p;
-    int64_t row_stride, k_stride;
-    bool transposed() const { return row_stride == 1 && k_stride != 1; }
-    int64_t ld() const { return transposed() ? k_stride : row_stride; }
-};
-
 // What the kernel asks of an operand with `rows` rows; 0 or an error code.
-int check_operand(const char* who, const char* name, const Operand& o, int64_t rows, int64_t K) {
+int check_operand(const char* who, const char* name, const Operand16& o, int64_t rows, int64_t K) {
     if (o.row_stride != 1 && o.k_stride != 1)
         return fail(DDL_E_UNSUPP, "%s: operand %s has no unit stride (row stride %lld, k stride %lld)", who, name, (long long)o.row_stride,
                     (long long)o.k_stride);
@@ -552,9 +509,40 @@ int check_operand(const char* who, const char* name, const Operand& o, int64_t r
     return 0;
 }
 
-// y[M, N] = a[M, K] . b[N, K]^T + bias in 16-bit elements.
-int gemm16(const char* who, bool f16, Operand a, Operand b, const uint16_t* bias, uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
-           void* stream) {
+// Estimated duration of the large tiles' schedule in microseconds (fits of a sweep, as in linear_small.hip): per k-tile
+// 0.47 (tiles of 128 x 256) or 0.95 us while few CUs work, up to 0.74 or 1.43 when all do and the chip runs into its
+// power limit.  `cost` is the schedule's length in tile rows or columns (see wide_tile_columns), `tiles` the workgroups.
+double large_us(bool low, int64_t cost, int64_t tiles, int64_t K, int cus) {
+    const double rounds = cost / (low ? 128.0 : 256.0), fill = tiles < cus ? static_cast<double>(tiles) / cus : 1.0;
+    return 6.5 + static_cast<double>((K + BK - 1) / BK) * rounds * (low ? 0.47 + 0.27 * fill * fill : 0.95 + 0.48 * fill * fill);
+}
+
+struct Plan16 {
+    Small16 small;            // kind other than kNone: linear_small.hip computes the product
+    int64_t low_tiles = 0;    // otherwise this many tiles of 128 x 256, if not 0
+    int64_t wide_cols = 0;    // otherwise 256 x 256 tiles for the first columns, 256 x 192 for the rest
+};
+
+Plan16 plan16(bool at, bool bt, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace) {
+    Plan16 plan;
+    const int64_t tiles_m = (M + 255) / 256, cols = (N + 255) / 256;
+    int64_t cost = 0;
+    plan.wide_cols = wide_tile_columns(tiles_m, N, cus, &cost);
+    // Tiles of half the height: twice the workgroups.  Taken when that shortens
+    // the schedule by more than the 10 % a smaller tile loses in efficiency.
+    const int64_t low_tiles = ((M + 127) / 128) * cols;
+    const int64_t low_cost = (low_tiles + cus - 1) / cus * 128;
+    const bool low = low_cost * 11 < cost * 10;
+    if (low) plan.low_tiles = low_tiles;
+    // Products that leave most of the chip idle either way.
+    plan.small = plan_small16(at, bt, M, N, K, cus, workspace,
+                              large_us(low, low ? low_cost : cost, low ? low_tiles : tiles_m * cols, K, cus));
+    return plan;
+}
+
+// y[M, N] = a[M, K] . b[N, K]^T + bias in 16-bit elements.  `workspace` (may be null) for the sums of a split reduction.
+int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* bias, uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
+           float* workspace, int64_t workspace_elems, void* stream) {
     if (M < 0 || N < 0 || K < 0 || ldy < N)
         return fail(DDL_E_ARG, "%s: M=%lld N=%lld K=%lld ldy=%lld", who, (long long)M, (long long)N, (long long)K, (long long)ldy);
     if (M == 0 || N == 0) return 0;
@@ -572,8 +560,8 @@ int gemm16(const char* who, bool f16, Operand a, Operand b, const uint16_t* bias
     const int64_t tiles_m = (M + 255) / 256, cols = (N + 255) / 256;
     if (tiles_m > 0x7FFFFFll || cols > 0x7FFFFFll || tiles_m * (cols + 1) > 0x7FFFFFFFll)
         return fail(DDL_E_UNSUPP, "%s: too many output tiles", who);
-    int64_t cost = 0;
-    const int64_t wide_cols = wide_tile_columns(tiles_m, N, cus, &cost);
+    const Plan16 plan = plan16(at, bt, M, N, K, cus, workspace_elems);
+    const int64_t wide_cols = plan.wide_cols;
     // Columns [n_begin, n_begin + n_count) of the output with tiles of bm x bn.
     auto part = [&](int bm, int bn, int64_t n_begin, int64_t n_count) {
         Part p{};
@@ -591,13 +579,11 @@ int gemm16(const char* who, bool f16, Operand a, Operand b, const uint16_t* bias
         }
         return 0;
     };
-    // Tiles of half the height: twice the workgroups.  Taken when that shortens
-    // the schedule by more than the 10 % a smaller tile loses in efficiency.
-    const int64_t low_tiles = ((M + 127) / 128) * cols;
-    const int64_t low_cost = (low_tiles + cus - 1) / cus * 128;
-    if (low_cost * 11 < cost * 10) {
+    if (plan.small.kind != Small16::kNone)
+        return run_small16(who, plan.small, f16, at, bt, part(64, 64, 0, N), workspace, dev, static_cast<hipStream_t>(stream));
+    if (plan.low_tiles) {
         if (int rc = reserve_lds(8 + k, reinterpret_cast<const void*>(kLowKernels[k]))) return rc;
-        hipLaunchKernelGGL(kLowKernels[k], dim3(static_cast<uint32_t>(low_tiles)), dim3(kThreads), kLdsBytes, static_cast<hipStream_t>(stream),
+        hipLaunchKernelGGL(kLowKernels[k], dim3(static_cast<uint32_t>(plan.low_tiles)), dim3(kThreads), kLdsBytes, static_cast<hipStream_t>(stream),
                            part(128, 256, 0, N));
         return check_launch("gemm16_low_tiles");
     }
@@ -635,12 +621,30 @@ extern "C" int ddl_linear(const void* x, const void* w, const void* bias, void* 
 
 extern "C" int ddl_gemm(const void* a, int64_t a_row_stride, int64_t a_k_stride, const void* b, int64_t b_row_stride, int64_t b_k_stride,
                         const void* bias, void* y, int dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, void* stream) {
+    return ddl_gemm_ws(a, a_row_stride, a_k_stride, b, b_row_stride, b_k_stride, bias, y, dtype, ldy, M, N, K, nullptr, 0, stream);
+}
+
+extern "C" int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride, int64_t b_k_stride,
+                                      int64_t M, int64_t N, int64_t K) {
     using namespace ddl;
+    if (M <= 0 || N <= 0 || K <= 0 || (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16)) return 0;
+    int dev = 0;
+    const int cus = compute_units(dev);
+    const Operand16 a{nullptr, a_row_stride, a_k_stride}, b{nullptr, b_row_stride, b_k_stride};
+    return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;
+}
+
+extern "C" int ddl_gemm_ws(const void* a, int64_t a_row_stride, int64_t a_k_stride, const void* b, int64_t b_row_stride, int64_t b_k_stride,
+                           const void* bias, void* y, int dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, float* workspace,
+                           int64_t workspace_elems, void* stream) {
+    using namespace ddl;
+    if (workspace && !aligned_to(workspace, 16)) return fail(DDL_E_ALIGN, "gemm: workspace must be 16-byte aligned");
     if (dtype == DDL_DT_F32)
         return ddl_gemm_f32(static_cast<const float*>(a), a_row_stride, a_k_stride, static_cast<const float*>(b), b_row_stride, b_k_stride,
                             static_cast<const float*>(bias), static_cast<float*>(y), ldy, M, N, K, stream);
     if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return fail(DDL_E_UNSUPP, "gemm: dtype %d (bf16, f16 and f32 only)", dtype);
-    const Operand oa{static_cast<const uint16_t*>(a), a_row_stride, a_k_stride};
-    const Operand ob{static_cast<const uint16_t*>(b), b_row_stride, b_k_stride};
-    return gemm16("gemm", dtype == DDL_DT_F16, oa, ob, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K, stream);
+    const Operand16 oa{static_cast<const uint16_t*>(a), a_row_stride, a_k_stride};
+    const Operand16 ob{static_cast<const uint16_t*>(b), b_row_stride, b_k_stride};
+    return gemm16("gemm", dtype == DDL_DT_F16, oa, ob, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K, workspace,
+                  workspace ? workspace_elems : 0, stream);
 }

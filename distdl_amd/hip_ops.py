@@ -4,6 +4,7 @@ into ``libdistdl_hip.so`` and raises when that is impossible.
 """
 
 import ctypes
+import functools
 
 import torch
 
@@ -682,6 +683,21 @@ def _padded_k(t, k8):
     return out
 
 
+@functools.lru_cache(maxsize=4096)
+def _gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k):
+    """Floats a product of these sizes and strides can use for partial sums (a function of its arguments alone)."""
+    return _lib.load().ddl_gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k)
+
+
+def _gemm(a, a_row, a_k, b, b_row, b_k, bias, out, dt, m, n, k):
+    """``out[m, n] = sum_k a b + bias`` on operands addressed by two strides each; ``out`` is contiguous."""
+    elems = _gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k)
+    work = torch.empty(elems, dtype=torch.float32, device=out.device) if elems else None
+    rc = _lib.load().ddl_gemm_ws(a.data_ptr(), a_row, a_k, b.data_ptr(), b_row, b_k, _ptr(bias), out.data_ptr(), dt, n, m, n, k,
+                                 _ptr(work), elems, _stream())
+    _lib.check(rc, "ddl_gemm")
+
+
 def linear(x, weight, bias=None, out=None):
     """y = x @ weight.T + bias with fp32 accumulation; operands and result
     bfloat16, float16 or float32 (all the same).  The 16-bit kernel wants the
@@ -719,9 +735,7 @@ def linear(x, weight, bias=None, out=None):
         if not (fits(x2, m) and fits(weight, n)):
             k8 = _round_up(k, 8)
             x2, weight, k = _padded_k(x2, k8), _padded_k(weight, k8), k8
-    rc = _lib.load().ddl_linear(x2.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(), dt, m, n, k,
-                                x2.stride(0) if m > 1 else k, weight.stride(0) if n > 1 else k, n, _stream())
-    _lib.check(rc, "ddl_linear")
+    _gemm(x2, x2.stride(0) if m > 1 else k, 1, weight, weight.stride(0) if n > 1 else k, 1, bias, out, dt, m, n, k)
     return out
 
 
@@ -804,25 +818,20 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
             x2 = contiguous(x2)
         if weight.stride(1) != 1 and k > 1:
             weight = contiguous(weight)
-        lib = _lib.load()
         ld_dy, ld_x, ld_w = (dy.stride(0) if m > 1 else n), (x2.stride(0) if m > 1 else k), (weight.stride(0) if n > 1 else k)
         if need_input:
             dx = torch.empty((m, k), dtype=x.dtype, device=x.device)
             if n == 0:
                 dx.zero_()
             else:   # dx[m, j] = sum_n dy[m, n] w[n, j]: rows of the second operand are the columns of w
-                rc = lib.ddl_gemm_f32(dy.data_ptr(), ld_dy, 1, weight.data_ptr(), 1, ld_w, None, dx.data_ptr(), k, m, k, n,
-                                      _stream())
-                _lib.check(rc, "ddl_gemm_f32")
+                _gemm(dy, ld_dy, 1, weight, 1, ld_w, None, dx, dt, m, k, n)
             dx = dx.reshape(x.shape)
         if need_weight:
             dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
             if m == 0:
                 dw.zero_()
             else:   # dw[i, j] = sum_m dy[m, i] x[m, j]: both operands are read down their columns
-                rc = lib.ddl_gemm_f32(dy.data_ptr(), 1, ld_dy, x2.data_ptr(), 1, ld_x, None, dw.data_ptr(), k, n, k, m,
-                                      _stream())
-                _lib.check(rc, "ddl_gemm_f32")
+                _gemm(dy, 1, ld_dy, x2, 1, ld_x, None, dw, dt, n, k, m)
         if need_bias:
             db = colsum(dy)
         return dx, dw, db
@@ -835,9 +844,7 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
         # dx[m, j] = sum_n dy[m, n] w[n, j]: dy is read along n, w down its columns
         if m and n and k and _along_k_ok(dy, ld_dy, n) and _along_rows_ok(weight, ld_w, k, n):
             dx = torch.empty((m, k), dtype=x.dtype, device=x.device)
-            rc = _lib.load().ddl_gemm(dy.data_ptr(), ld_dy, 1, weight.data_ptr(), 1, ld_w, None, dx.data_ptr(), dt, k, m, k, n,
-                                      _stream())
-            _lib.check(rc, "ddl_gemm")
+            _gemm(dy, ld_dy, 1, weight, 1, ld_w, None, dx, dt, m, k, n)
             dx = dx.reshape(x.shape)
         else:   # operands dy[M, N] and wT[K, N], padded
             np8 = _round_up(n, 8)
@@ -850,9 +857,7 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
         # dw[i, j] = sum_m dy[m, i] x[m, j]: both operands are read down their columns
         if m and n and k and _along_rows_ok(dy, ld_dy, n, m) and _along_rows_ok(x2, ld_x, k, m):
             dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
-            rc = _lib.load().ddl_gemm(dy.data_ptr(), 1, ld_dy, x2.data_ptr(), 1, ld_x, None, dw.data_ptr(), dt, k, n, k, m,
-                                      _stream())
-            _lib.check(rc, "ddl_gemm")
+            _gemm(dy, 1, ld_dy, x2, 1, ld_x, None, dw, dt, n, k, m)
         else:   # operands dyT[N, M] and xT[K, M], padded
             mp8 = _round_up(m, 8)
             dy_t = transpose_2d(dy, mp8)                          # [N, mp8]
@@ -886,7 +891,5 @@ def _linear_padded(a, b, m, n, k_padded, dt):
     out = torch.empty((m, n), dtype=a.dtype, device=a.device)
     if k_padded == 0 or m == 0 or n == 0:
         return out.zero_()
-    rc = _lib.load().ddl_linear(a.data_ptr(), b.data_ptr(), None, out.data_ptr(), dt, m, n, k_padded,
-                                a.stride(0) if m > 1 else k_padded, b.stride(0) if n > 1 else k_padded, n, _stream())
-    _lib.check(rc, "ddl_linear")
+    _gemm(a, a.stride(0) if m > 1 else k_padded, 1, b, b.stride(0) if n > 1 else k_padded, 1, None, out, dt, m, n, k_padded)
     return out

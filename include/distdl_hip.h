@@ -490,6 +490,20 @@ int ddl_gemm(const void* a, int64_t a_row_stride, int64_t a_k_stride,
              const void* b, int64_t b_row_stride, int64_t b_k_stride,
              const void* bias, void* y, int dtype, int64_t ldy,
              int64_t M, int64_t N, int64_t K, void* stream);
+/* ddl_gemm with room for the partial sums of a reduction that is split over
+ * workgroups: `workspace` (16-byte aligned, may be null) holds
+ * `workspace_elems` floats, as many as ddl_gemm_workspace says for the fastest
+ * way (0: none needed; with fewer, a way that needs no more is taken).  Its
+ * contents on entry do not matter; the result is the same up to the order of
+ * the fp32 sums. */
+int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride,
+                           int64_t b_row_stride, int64_t b_k_stride, int64_t M,
+                           int64_t N, int64_t K);
+int ddl_gemm_ws(const void* a, int64_t a_row_stride, int64_t a_k_stride,
+                const void* b, int64_t b_row_stride, int64_t b_k_stride,
+                const void* bias, void* y, int dtype, int64_t ldy, int64_t M,
+                int64_t N, int64_t K, float* workspace, int64_t workspace_elems,
+                void* stream);
 int ddl_gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride,
                  const float* b, int64_t b_row_stride, int64_t b_k_stride,
                  const float* bias, float* y, int64_t ldy,

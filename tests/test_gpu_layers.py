@@ -1535,6 +1535,45 @@ def test_gemm_16_bit_reads_operands_where_they_lie(ops, dtype, a_t, b_t, M, N, K
     assert (got[:, N:] == 77.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("a_t,b_t,M,N,K,splits", [
+    # up to 64 rows: one to eight pieces of eight rows, odd columns, one step per wavefront and many, a straddling step
+    (False, False, 1, 1, 8, False), (False, False, 8, 17, 512, False), (False, False, 9, 40, 1032, False),
+    (False, False, 17, 333, 4104, False), (False, False, 33, 16, 520, False), (False, False, 64, 100, 2056, False),
+    # small tiles: one workgroup and several per CU, one k-tile and an odd number of them
+    (False, False, 65, 65, 64, False), (False, True, 72, 136, 200, False), (True, False, 136, 67, 456, False),
+    (True, True, 2056, 1032, 136, False),
+    # the reduction split over workgroups: unequal shares, a share that straddles K
+    (False, False, 100, 130, 4168, True), (False, True, 72, 136, 2120, True), (True, False, 200, 264, 4104, True),
+    (True, True, 128, 64, 8191, True)])
+def test_gemm_16_bit_products_that_leave_the_chip_idle(ops, dtype, a_t, b_t, M, N, K, splits):
+    """The skinny and small-tile kernels on integer operands (every sum is exact), with and without the workspace that
+    lets them split the reduction; the workspace's contents on entry do not matter."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(M * 7 + N * 3 + K)
+    a = torch.randint(-1, 2, (M, K), generator=gen).to(dtype)
+    b = torch.randint(-1, 2, (N, K), generator=gen).to(dtype)
+    b = b * (torch.rand(N, K, generator=gen) < min(1.0, 64.0 / K)).to(dtype)
+    bias = torch.randint(-3, 4, (N,), generator=gen).to(dtype)
+    ag, a_rs, a_ks = _gemm_operand(a, a_t, 0)
+    bg, b_rs, b_ks = _gemm_operand(b, b_t, 0)
+    want = a.double() @ b.double().T + bias.double()
+    assert want.abs().max() <= 256
+    lib, dt, stream = _lib.load(), _lib.DDL_DT_BF16 if dtype == torch.bfloat16 else _lib.DDL_DT_F16, torch.cuda.current_stream().cuda_stream
+    elems = lib.ddl_gemm_workspace(dt, a_rs, a_ks, b_rs, b_ks, M, N, K)
+    assert (elems > 0) == splits
+    ldy = N + 8
+    for n in {0, elems // 2, elems}:
+        work = torch.full((n,), float("nan"), device="cuda") if n else None
+        out = torch.full((M, ldy), 77.0, dtype=dtype, device="cuda")
+        rc = lib.ddl_gemm_ws(ag.data_ptr(), a_rs, a_ks, bg.data_ptr(), b_rs, b_ks, bias.cuda().data_ptr(), out.data_ptr(), dt, ldy, M, N,
+                             K, None if work is None else work.data_ptr(), n, stream)
+        _lib.check(rc, "ddl_gemm_ws")
+        got = out.cpu().double()
+        assert torch.equal(got[:, :N], want)
+        assert (got[:, N:] == 77.0).all()
+
+
 @pytest.mark.parametrize("a_t,b_t", [(False, True), (True, True)])
 def test_gemm_16_bit_random_within_tolerance_and_ragged_depth(ops, a_t, b_t):
     """Random operands, a reduction length that is no multiple of the k-tile
