@@ -328,25 +328,30 @@ struct Operand {
     int64_t ld() const { return transposed() ? k_stride : row_stride; }
 };
 
-// Can the tiled kernel read this operand (`rows` rows) where it lies?
-bool operand_ok(const Operand& o, int64_t rows, int64_t K) {
-    if (o.row_stride != 1 && o.k_stride != 1) return false;
-    const int64_t ld = o.ld();
-    if (!aligned_to(o.p, 16) || ld % 4 != 0 || ld > 0x1FFFFF) return false;   // 32-bit byte offsets inside a tile
-    if (o.transposed()) return ld >= rows && rows % 4 == 0 && (K + BK) * ld <= 0x1FFFFFFF;
+// Can the tiled kernel read this operand (`rows` rows, base aligned to 16 bytes) where it lies?
+bool operand_ok(int64_t row_stride, int64_t k_stride, int64_t rows, int64_t K) {
+    if (row_stride != 1 && k_stride != 1) return false;
+    const bool transposed = row_stride == 1 && k_stride != 1;
+    const int64_t ld = transposed ? k_stride : row_stride;
+    if (ld % 4 != 0 || ld > 0x1FFFFF) return false;   // 32-bit byte offsets inside a tile
+    if (transposed) return ld >= rows && rows % 4 == 0 && (K + BK) * ld <= 0x1FFFFFFF;
     return ld >= K && K % 4 == 0 && K <= 0x1FFFFFFF;
 }
 
 }  // namespace
 
-// y = a . b^T + bias through the tiled kernel; false if the operands do not
-// qualify (the caller then takes the strided kernel), otherwise *rc is the result.
-bool gemm_f32_tiled(const float* a, int64_t a_rs, int64_t a_ks, const float* b, int64_t b_rs, int64_t b_ks, const float* bias, float* y,
-                    int64_t ldy, int64_t M, int64_t N, int64_t K, void* stream, int* rc) {
-    const Operand oa{a, a_rs, a_ks}, ob{b, b_rs, b_ks};
-    if (!operand_ok(oa, M, K) || !operand_ok(ob, N, K)) return false;
+// Does the tiled kernel take this product?  At least a quarter of the CUs' worth of tiles, operands it can read.
+bool gemm_f32_tiled_ok(bool aligned, int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K) {
     const int64_t tiles_m = (M + 255) / 256, cols = (N + 255) / 256;
-    if (tiles_m > 0x7FFFFFll || cols > 0x7FFFFFll || tiles_m * (cols + 1) > 0x7FFFFFFFll) return false;
+    return aligned && tiles_m * cols >= 64 && operand_ok(a_rs, a_ks, M, K) && operand_ok(b_rs, b_ks, N, K) && tiles_m <= 0x7FFFFFll &&
+           cols <= 0x7FFFFFll && tiles_m * (cols + 1) <= 0x7FFFFFFFll;
+}
+
+// y = a . b^T + bias through the tiled kernel, for products that gemm_f32_tiled_ok accepts.
+int gemm_f32_tiled(const float* a, int64_t a_rs, int64_t a_ks, const float* b, int64_t b_rs, int64_t b_ks, const float* bias, float* y,
+                   int64_t ldy, int64_t M, int64_t N, int64_t K, void* stream) {
+    const Operand oa{a, a_rs, a_ks}, ob{b, b_rs, b_ks};
+    const int64_t tiles_m = (M + 255) / 256;
     int dev = 0;
     const int cus = compute_units(dev);
     const int64_t wide_cols = wide_tile_columns(tiles_m, N, cus);
@@ -365,16 +370,12 @@ bool gemm_f32_tiled(const float* a, int64_t a_rs, int64_t a_ks, const float* b, 
     const int k = (oa.transposed() ? 2 : 0) + (ob.transposed() ? 1 : 0);
     if (!lds_reserved[dev][k].load(std::memory_order_acquire)) {   // the attribute sticks to the function on this device
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kKernels[k]), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-        if (e != hipSuccess) {
-            *rc = fail(static_cast<int>(e), "gemm f32: cannot reserve %d bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
-            return true;
-        }
+        if (e != hipSuccess) return fail(static_cast<int>(e), "gemm f32: cannot reserve %d bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
         lds_reserved[dev][k].store(true, std::memory_order_release);
     }
     hipLaunchKernelGGL(kKernels[k], dim3(static_cast<uint32_t>(n_wide > n_narrow ? n_wide : n_narrow)), dim3(kThreads), kLdsBytes,
                        static_cast<hipStream_t>(stream), parts);
-    *rc = check_launch("gemm32_tiles");
-    return true;
+    return check_launch("gemm32_tiles");
 }
 
 }  // namespace ddl

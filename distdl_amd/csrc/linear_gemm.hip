@@ -57,6 +57,7 @@
 //              one XCD cover a compact patch of the tile grid and share their
 //              operand panels in that XCD's L2
 #include "gemm16_small.h"
+#include "gemm32_small.h"
 #include <type_traits>
 
 namespace ddl {
@@ -600,9 +601,13 @@ int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* 
 }  // namespace
 }  // namespace ddl
 
-extern "C" int ddl_gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride, const float* b, int64_t b_row_stride,
-                            int64_t b_k_stride, const float* bias, float* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
-                            void* stream);
+namespace ddl {
+int gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride, const float* b, int64_t b_row_stride, int64_t b_k_stride,
+             const float* bias, float* y, int64_t ldy, int64_t M, int64_t N, int64_t K, float* workspace, int64_t workspace_elems,
+             void* stream);
+Small32 plan32(bool aligned, int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K, int cus,
+               int64_t workspace);
+}  // namespace ddl
 
 extern "C" int ddl_linear_bf16(const void* x, const void* w, const void* bias, void* y, int64_t M, int64_t N, int64_t K,
                                int64_t ldx, int64_t ldw, int64_t ldy, void* stream) {
@@ -627,9 +632,11 @@ extern "C" int ddl_gemm(const void* a, int64_t a_row_stride, int64_t a_k_stride,
 extern "C" int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride, int64_t b_k_stride,
                                       int64_t M, int64_t N, int64_t K) {
     using namespace ddl;
-    if (M <= 0 || N <= 0 || K <= 0 || (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16)) return 0;
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
     int dev = 0;
     const int cus = compute_units(dev);
+    if (dtype == DDL_DT_F32) return plan32(true, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, INT64_MAX).workspace;
+    if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return 0;
     const Operand16 a{nullptr, a_row_stride, a_k_stride}, b{nullptr, b_row_stride, b_k_stride};
     return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;
 }
@@ -640,8 +647,8 @@ extern "C" int ddl_gemm_ws(const void* a, int64_t a_row_stride, int64_t a_k_stri
     using namespace ddl;
     if (workspace && !aligned_to(workspace, 16)) return fail(DDL_E_ALIGN, "gemm: workspace must be 16-byte aligned");
     if (dtype == DDL_DT_F32)
-        return ddl_gemm_f32(static_cast<const float*>(a), a_row_stride, a_k_stride, static_cast<const float*>(b), b_row_stride, b_k_stride,
-                            static_cast<const float*>(bias), static_cast<float*>(y), ldy, M, N, K, stream);
+        return gemm_f32(static_cast<const float*>(a), a_row_stride, a_k_stride, static_cast<const float*>(b), b_row_stride, b_k_stride,
+                        static_cast<const float*>(bias), static_cast<float*>(y), ldy, M, N, K, workspace, workspace_elems, stream);
     if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return fail(DDL_E_UNSUPP, "gemm: dtype %d (bf16, f16 and f32 only)", dtype);
     const Operand16 oa{static_cast<const uint16_t*>(a), a_row_stride, a_k_stride};
     const Operand16 ob{static_cast<const uint16_t*>(b), b_row_stride, b_k_stride};

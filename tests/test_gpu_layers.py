@@ -1617,6 +1617,41 @@ def test_gemm_f32_tiled_kernel_reads_every_operand_layout(ops, a_t, b_t, M, N, K
     assert (got[:, N:] == 77.0).all()
 
 
+@pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K,pad,splits", [
+    # tiles of 64 x 64, 32 x 64 and 32 x 32; odd lengths and pitches; one k-tile, a straddling one, an odd number of rounds
+    (4, 4, 1, 0, False), (5, 7, 9, 1, False), (33, 31, 33, 3, False), (64, 64, 64, 0, False), (130, 65, 96, 5, False),
+    (1030, 517, 131, 0, False), (2050, 1027, 100, 2, False),
+    # the reduction split over workgroups, unequal shares
+    (201, 263, 1033, 1, True), (64, 100, 4095, 0, True),
+    # enough work for the 256 x 256 tiles, wide and narrow ones
+    (4096, 4352, 1540, 4, False)])
+def test_gemm_f32_products_of_every_size_and_pitch(ops, a_t, b_t, M, N, K, pad, splits):
+    """Integer operands (every sum is exact in fp32) at the sizes where the small fp32 tiles can go wrong, with and
+    without the workspace that lets them split the reduction, on buffers that end where the operands end."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(M + 3 * N + K + 2 * a_t + b_t)
+    a = torch.randint(-3, 4, (M, K), generator=gen).float()
+    b = torch.randint(-3, 4, (N, K), generator=gen).float()
+    bias = torch.randint(-5, 6, (N,), generator=gen).float()
+    ag, a_rs, a_ks = _gemm_operand(a, a_t, pad)
+    bg, b_rs, b_ks = _gemm_operand(b, b_t, pad)
+    want = a.double() @ b.double().T + bias.double()
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    elems = lib.ddl_gemm_workspace(_lib.DDL_DT_F32, a_rs, a_ks, b_rs, b_ks, M, N, K)
+    assert (elems > 0) == splits
+    ldy = N + 4 + (M & 1)
+    for n in {0, elems}:
+        work = torch.full((n,), float("nan"), device="cuda") if n else None
+        out = torch.full((M, ldy), 77.0, device="cuda")
+        rc = lib.ddl_gemm_ws(ag.data_ptr(), a_rs, a_ks, bg.data_ptr(), b_rs, b_ks, bias.cuda().data_ptr(), out.data_ptr(), _lib.DDL_DT_F32,
+                             ldy, M, N, K, None if work is None else work.data_ptr(), n, stream)
+        _lib.check(rc, "ddl_gemm_ws")
+        got = out.cpu().double()
+        assert torch.equal(got[:, :N], want)
+        assert (got[:, N:] == 77.0).all()
+
+
 def test_gemm_f32_tiled_kernel_random_and_odd_depth(ops):
     """Random operands through the tiled fp32 kernel: both operands read along
     their rows, so the reduction length may be anything (here 1003, no multiple
