@@ -89,6 +89,8 @@ SIGNATURES = {
     "ddl_ln_bwd_input_params": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,
                                         c_void_p, c_void_p, c_int, c_float, c_void_p, c_int64, c_void_p, c_int64,
                                         c_void_p, c_void_p, c_void_p]),
+    "ddl_ln_bwd_whole_rows": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
+                                      c_float, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
     "ddl_ln_bwd_one_pass": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                                     c_void_p, c_int, c_int, c_float, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
                                     c_void_p]),

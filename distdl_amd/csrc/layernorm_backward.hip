@@ -382,6 +382,184 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
     }
 }
 
+// Rows that do not fit a wavefront's registers, or are no multiple of four
+// elements: the pass of ln_bwd_partial_cols with a workgroup per row.  Thread t
+// keeps the V-element pieces t + THREADS k, k < NV, of gamma and of the column
+// sums in registers for all rows of its split; RU rows are loaded while the RU rows
+// before them are summed, and the only barrier per RU rows is the exchange of the
+// wavefronts' row sums (double-buffered in LDS).  Bound by HBM: dy and x are read
+// once and dx written once.  [8192, 8192] bf16 measured, row sums + column sums + dx
+// in separate passes 45 + 65 + 82 us, here together (see ddl_ln_bwd_whole_rows).
+template <typename T, int V>
+struct Piece;
+template <typename T>
+struct Piece<T, 4> {
+    typedef std::conditional_t<sizeof(T) == 4, float4, uint2> raw;
+    static __device__ void get(const raw& r, float (&f)[4]) {
+        const float4 q = load4(reinterpret_cast<const T*>(&r));
+        f[0] = q.x, f[1] = q.y, f[2] = q.z, f[3] = q.w;
+    }
+    static __device__ void put(T* p, const float (&f)[4]) { store4(p, make_float4(f[0], f[1], f[2], f[3])); }
+};
+template <typename T>
+struct Piece<T, 1> {
+    typedef T raw;
+    static __device__ void get(const raw& r, float (&f)[1]) { f[0] = load1(&r); }
+    static __device__ void put(T* p, const float (&f)[1]) { store1(p, f[0]); }
+};
+
+template <typename T, int THREADS, int V, int NV, int RU, bool WITH_DX>
+__global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows, int64_t cols,
+                                                             int64_t ld_dy, int64_t ld_x, const float* __restrict__ mean,
+                                                             const float* __restrict__ rstd, const T* __restrict__ gamma,
+                                                             float* __restrict__ sums, int64_t rows_per_split, float* __restrict__ partial,
+                                                             float weight, T* __restrict__ dx, int64_t ld_dx) {
+#pragma clang fp contract(off)   // both instantiations round alike
+    typedef Piece<T, V> P;
+    typedef typename P::raw Raw;
+    constexpr int kWaves = THREADS / kWave;
+    __shared__ float2 row_sums[2][RU][kWaves];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int pieces = static_cast<int>(cols / V);
+    const int64_t r_begin = static_cast<int64_t>(blockIdx.x) * rows_per_split;
+    const int64_t r_end = r_begin + rows_per_split < rows ? r_begin + rows_per_split : rows;
+    Raw g[NV];
+    float ca[NV][V], cb[NV][V];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int c = threadIdx.x + k * THREADS;
+        if (gamma && c < pieces) g[k] = *reinterpret_cast<const Raw*>(gamma + V * c);
+#pragma unroll
+        for (int e = 0; e < V; ++e) ca[k][e] = cb[k][e] = 0.f;
+    }
+    auto fetch = [&](int64_t r0, Raw (&d)[RU][NV], Raw (&v)[RU][NV], float (&m)[RU], float (&rs)[RU]) {
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            const int64_t r = r0 + u < r_end ? r0 + u : r_end - 1;   // a row past the end repeats the last one and is not used
+            m[u] = mean[r], rs[u] = rstd[r];
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const int c = threadIdx.x + k * THREADS;
+                if (c < pieces) {
+                    d[u][k] = *reinterpret_cast<const Raw*>(dy + r * ld_dy + V * c);
+                    v[u][k] = *reinterpret_cast<const Raw*>(x + r * ld_x + V * c);
+                }
+            }
+        }
+    };
+    auto gain = [&](int k, float (&f)[V]) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) f[e] = 1.f;
+        if (gamma) P::get(g[k], f);
+    };
+    Raw d[RU][NV], v[RU][NV];
+    float m[RU], rs[RU];
+    if (r_begin < r_end) fetch(r_begin, d, v, m, rs);
+    int parity = 0;
+    for (int64_t r0 = r_begin; r0 < r_end; r0 += RU, parity ^= 1) {
+        Raw d_next[RU][NV], v_next[RU][NV];
+        float m_next[RU], rs_next[RU];
+        const bool more = r0 + RU < r_end;
+        if (more) fetch(r0 + RU, d_next, v_next, m_next, rs_next);
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            if (r0 + u >= r_end) break;   // the same in all threads
+            float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                if (static_cast<int>(threadIdx.x) + k * THREADS >= pieces) continue;
+                float dd[V], vv[V], gg[V];
+                P::get(d[u][k], dd);
+                P::get(v[u][k], vv);
+                gain(k, gg);
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const float h = (vv[e] - m[u]) * rs[u], t = dd[e] * gg[e];
+                    s1 += t;
+                    s2 += t * h;
+                    ca[k][e] += dd[e] * h;
+                    cb[k][e] += dd[e];
+                }
+            }
+            s1 = wave_sum(s1);
+            s2 = wave_sum(s2);
+            if (lane == 0) row_sums[parity][u][wave] = make_float2(s1, s2);
+        }
+        // Only LDS is exchanged: the loads of the next rows stay in flight.
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            const int64_t r = r0 + u;
+            if (r >= r_end) break;
+            const float2 p = lane < kWaves ? row_sums[parity][u][lane] : make_float2(0.f, 0.f);
+            const float s1 = wave_sum(p.x), s2 = wave_sum(p.y);
+            if (threadIdx.x == 0 && sums) reinterpret_cast<float2*>(sums)[r] = make_float2(s1, s2);
+            if (WITH_DX) {
+                const float S1 = s1 * weight, S2 = s2 * weight;
+#pragma unroll
+                for (int k = 0; k < NV; ++k) {
+                    const int c = threadIdx.x + k * THREADS;
+                    if (c >= pieces) continue;
+                    float dd[V], vv[V], gg[V], o[V];
+                    P::get(d[u][k], dd);
+                    P::get(v[u][k], vv);
+                    gain(k, gg);
+#pragma unroll
+                    for (int e = 0; e < V; ++e) o[e] = dx_value(dd[e], gg[e], vv[e], m[u], rs[u], S1, S2);
+                    P::put(dx + r * ld_dx + V * c, o);
+                }
+            }
+        }
+        if (more) {
+#pragma unroll
+            for (int u = 0; u < RU; ++u) {
+                m[u] = m_next[u], rs[u] = rs_next[u];
+#pragma unroll
+                for (int k = 0; k < NV; ++k) d[u][k] = d_next[u][k], v[u][k] = v_next[u][k];
+            }
+        }
+    }
+    float* out = partial + static_cast<int64_t>(blockIdx.x) * 2 * cols;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int c = threadIdx.x + k * THREADS;
+        if (c >= pieces) continue;
+#pragma unroll
+        for (int e = 0; e < V; ++e) out[V * c + e] = ca[k][e], out[cols + V * c + e] = cb[k][e];
+    }
+}
+
+// The longest rows that ln_bwd_block_rows takes: what a workgroup's registers hold.
+constexpr int64_t block_rows_cols(bool vec) { return vec ? 16384 : 8192; }
+
+template <typename T, bool WITH_DX>
+void launch_block_rows(bool vec, const T* dy, const T* x, int64_t rows, int64_t cols, int64_t ld_dy, int64_t ld_x, const float* mean,
+                       const float* rstd, const T* gamma, float* sums, int64_t splits, float* partial, float weight, T* dx, int64_t ld_dx,
+                       hipStream_t s) {
+    const int64_t rows_per_split = (rows + splits - 1) / splits;
+    auto go = [&](auto threads, auto v, auto nv, auto ru) {
+        constexpr int kThreads = decltype(threads)::value;
+        hipLaunchKernelGGL((ln_bwd_block_rows<T, kThreads, decltype(v)::value, decltype(nv)::value, decltype(ru)::value, WITH_DX>),
+                           dim3(static_cast<uint32_t>(splits)), dim3(kThreads), 0, s, dy, x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, sums,
+                           rows_per_split, partial, weight, dx, ld_dx);
+    };
+    const std::integral_constant<int, 1> c1{};
+    const std::integral_constant<int, 2> c2{};
+    const std::integral_constant<int, 4> c4{};
+    const std::integral_constant<int, 8> c8{};
+    const std::integral_constant<int, 512> c512{};
+    const std::integral_constant<int, 1024> c1024{};
+    if (vec) {
+        if (cols <= 2048) go(c512, c4, c1, c4);
+        else if (cols <= 4096) go(c1024, c4, c1, c4);
+        else if (cols <= 8192) go(c1024, c4, c2, c2);
+        else go(c1024, c4, c4, c1);
+    } else {
+        if (cols <= 4096) go(c1024, c1, c4, c2);
+        else go(c1024, c1, c8, c1);
+    }
+}
+
 // Can rows be read four elements at a time?  elem = bytes per element.
 bool vectorizable(int elem, int64_t cols, std::initializer_list<int64_t> lds, std::initializer_list<const void*> ptrs) {
     if (cols % 4 != 0) return false;
@@ -410,12 +588,12 @@ bool elems_aligned(int elem, std::initializer_list<const void*> ptrs) {
 }
 
 // Row splits of the parameter gradients: as many as the workspace holds, at most
-// 256 and at least 32 rows each.  0 when the workspace cannot hold one split.
-int64_t param_splits(int64_t rows, int64_t cols, int64_t workspace_elems) {
+// 256 and at least `fewest` rows each.  0 when the workspace cannot hold one split.
+int64_t param_splits(int64_t rows, int64_t cols, int64_t workspace_elems, int64_t fewest = 32) {
     int64_t splits = workspace_elems / (2 * cols);
     if (splits < 1) return 0;
     if (splits > 256) splits = 256;
-    const int64_t by_rows = (rows + 31) / 32;
+    const int64_t by_rows = (rows + fewest - 1) / fewest;
     if (splits > by_rows) splits = by_rows > 0 ? by_rows : 1;
     return splits;
 }
@@ -537,7 +715,18 @@ extern "C" int ddl_ln_bwd_partial_params(const void* dy, const void* x, int dtyp
         });
         return check_launch("ln_bwd_partial_cols");
     }
-    // long or unaligned rows: the two passes separately, same results in the same places
+    const bool vec = vectorizable(elem, cols, {ld_dy, ld_x}, {dy, x, gamma});
+    // One read of dy and x instead of two, where every CU gets a split: [8192, 8192] bf16 with the dx launch 187 -> 132 us,
+    // but [1024, 8192] (32 splits) 43 -> 58 and rows of a few hundred elements 10.6 -> 24.
+    if (splits == 256 && cols > 4 * kWave * 4 && cols <= block_rows_cols(vec)) {
+        with_ln_element(dtype, [&](auto* tag) {
+            using T = std::remove_pointer_t<decltype(tag)>;
+            launch_block_rows<T, false>(vec, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, splits, workspace, 0.f,
+                                        static_cast<T*>(nullptr), 0, s);
+        });
+        return check_launch("ln_bwd_block_rows");
+    }
+    // everything else: the two passes separately, same results in the same places
     if (rows > 0) {
         if (int rc = ddl_ln_bwd_partial(dy, x, dtype, rows, cols, ld_dy, ld_x, mean, rstd, gamma, sums, stream)) return rc;
     }
@@ -631,6 +820,42 @@ extern "C" int ddl_ln_bwd_one_pass(const void* dy, const void* x, int dtype, int
     with_ln_element(dtype, [&](auto* tag) {
         using T = std::remove_pointer_t<decltype(tag)>;
         hipLaunchKernelGGL(ln_bwd_params_final<T>, dim3(static_cast<uint32_t>(strips)), dim3(kBlock), 0, s, workspace, cols,
+                           static_cast<int>(rows > 0 ? splits : 0), as<T>(dgamma), as<T>(dbeta));
+    });
+    return check_launch("ln_bwd_params_final");
+}
+
+extern "C" int ddl_ln_bwd_whole_rows(const void* dy, const void* x, int dtype, int64_t rows, int64_t cols, int64_t ld_dy, int64_t ld_x,
+                                     const float* mean, const float* rstd, const void* gamma, float weight, void* dx, int64_t ld_dx,
+                                     float* workspace, int64_t workspace_elems, void* dgamma, void* dbeta, void* stream) {
+    using namespace ddl;
+    const int elem = elem_bytes(dtype);
+    if (!elem) return fail(DDL_E_UNSUPP, "ln backward (whole rows): dtype %d (f32, bf16, f16 only)", dtype);
+    if (int rc = check_rows("ln backward (whole rows)", rows, cols, ld_dy, ld_x)) return rc;
+    if (ld_dx < cols) return fail(DDL_E_ARG, "ln backward (whole rows): ld_dx=%lld below cols=%lld", (long long)ld_dx, (long long)cols);
+    const bool vec = vectorizable(elem, cols, {ld_dy, ld_x, ld_dx}, {dy, x, gamma, dx});
+    if (cols <= 4 * kWave * 4 || cols > block_rows_cols(vec))
+        return fail(DDL_E_UNSUPP, "ln backward (whole rows): rows of %d to %lld columns", 4 * kWave * 4 + 1, (long long)block_rows_cols(vec));
+    if (!workspace) return fail(DDL_E_ARG, "ln backward (whole rows): null workspace");
+    // Four rows per split already pay: a split's column sums are 8 bytes per column next to 4 rows x 3 tensors of elements.
+    const int64_t splits = param_splits(rows, cols, workspace_elems, 4);
+    if (splits < 1) return fail(DDL_E_ARG, "ln backward (whole rows): workspace of %lld floats is smaller than 2 x %lld", (long long)workspace_elems, (long long)cols);
+    if (rows > 0 && (!dy || !x || !mean || !rstd || !dx)) return fail(DDL_E_ARG, "ln backward (whole rows): null pointer");
+    if (!elems_aligned(elem, {dy, x, gamma, dx, dgamma, dbeta}) || !aligned_to(mean, 4) || !aligned_to(rstd, 4) || !aligned_to(workspace, 4))
+        return fail(DDL_E_ALIGN, "ln backward (whole rows): elements must be aligned to their size, fp32 arrays to 4 bytes");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (rows > 0) {
+        with_ln_element(dtype, [&](auto* tag) {
+            using T = std::remove_pointer_t<decltype(tag)>;
+            launch_block_rows<T, true>(vec, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), nullptr, splits, workspace, weight,
+                                       as<T>(dx), ld_dx, s);
+        });
+        if (int rc = check_launch("ln_bwd_block_rows")) return rc;
+    }
+    if (!dgamma && !dbeta) return 0;
+    with_ln_element(dtype, [&](auto* tag) {
+        using T = std::remove_pointer_t<decltype(tag)>;
+        hipLaunchKernelGGL(ln_bwd_params_final<T>, dim3(static_cast<uint32_t>((cols + kStrip - 1) / kStrip)), dim3(kBlock), 0, s, workspace, cols,
                            static_cast<int>(rows > 0 ? splits : 0), as<T>(dgamma), as<T>(dbeta));
     });
     return check_launch("ln_bwd_params_final");

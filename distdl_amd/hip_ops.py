@@ -589,6 +589,36 @@ def ln_backward_one_pass(dy2d, x2d, mean, rstd, gamma, weight, part_sums=None, m
     return dx, dg, db
 
 
+def ln_backward_whole_rows_supported(dy2d, x2d, gamma):
+    """Whether ``ln_backward_whole_rows`` takes these rows: 1025 to 8192
+    columns, or 16384 when columns and pitches are multiples of 4 and dy, x and
+    gamma aligned to four elements."""
+    rows, cols = x2d.shape
+    if cols <= 8192:
+        return cols > 1024
+    quad = 4 * x2d.element_size()
+    return (cols <= 16384 and cols % 4 == 0 and (rows <= 1 or (x2d.stride(0) % 4 == 0 and dy2d.stride(0) % 4 == 0)) and
+            x2d.data_ptr() % quad == 0 and dy2d.data_ptr() % quad == 0 and (gamma is None or gamma.data_ptr() % quad == 0))
+
+
+def ln_backward_whole_rows(dy2d, x2d, mean, rstd, gamma, weight, want_gamma=True, want_beta=True):
+    """dx and (dgamma, dbeta) in one pass over dy and x, for rows this worker
+    holds whole (a workgroup per row)."""
+    _require_gpu(dy2d, x2d, mean, rstd, gamma)
+    ld_dy, ld_x = _rows2d(dy2d, "ln_backward_whole_rows"), _rows2d(x2d, "ln_backward_whole_rows")
+    rows, cols = x2d.shape
+    dt = _ln_bwd_dtype("ln_backward_whole_rows", dy2d, x2d, gamma)
+    work = torch.empty(2 * max(1, min(256, (rows + 3) // 4)) * cols, dtype=torch.float32, device=x2d.device)
+    dx = torch.empty((rows, cols), dtype=x2d.dtype, device=x2d.device)
+    dg = torch.empty(cols, dtype=x2d.dtype, device=x2d.device) if want_gamma else None
+    db = torch.empty(cols, dtype=x2d.dtype, device=x2d.device) if want_beta else None
+    rc = _lib.load().ddl_ln_bwd_whole_rows(dy2d.data_ptr(), x2d.data_ptr(), dt, rows, cols, ld_dy, ld_x, mean.data_ptr(),
+                                           rstd.data_ptr(), _ptr(gamma), float(weight), dx.data_ptr(), cols, work.data_ptr(),
+                                           work.numel(), _ptr(dg), _ptr(db), _stream())
+    _lib.check(rc, "ddl_ln_bwd_whole_rows")
+    return dx, dg, db
+
+
 def embedding_gather(weight, ids, lo, hi, out=None):
     """out[t] = weight[ids[t] - lo] if lo <= ids[t] < hi else 0."""
     _require_gpu(weight, ids)

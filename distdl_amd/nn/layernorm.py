@@ -102,6 +102,9 @@ class _LayerNormShard(torch.autograd.Function):
             dx, dw, db = hip_ops.ln_backward_one_pass(dy2d, x2d, mean, rstd, gamma, 1.0 / ctx.cols, want_gamma=want_w,
                                                       want_beta=want_b)
             dx = dx.view(grad_output.shape)
+        elif fused and ctx.nparts == 1 and hip_ops.ln_backward_whole_rows_supported(dy2d, x2d, gamma):
+            dx, dw, db = hip_ops.ln_backward_whole_rows(dy2d, x2d, mean, rstd, gamma, 1.0 / ctx.cols, want_w, want_b)
+            dx = dx.view(grad_output.shape)
         elif need_x:
             if fused:
                 sums, work = hip_ops.ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma)

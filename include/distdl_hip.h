@@ -359,6 +359,18 @@ int ddl_ln_bwd_one_pass(const void* dy, const void* x, int dtype, int64_t rows,
                         void* dx, int64_t ld_dx, float* workspace,
                         int64_t workspace_elems, void* dgamma, void* dbeta,
                         void* stream);
+/* The same for longer rows a worker holds whole (any pitch): a workgroup per
+ * row.  More than 1024 columns, at most 16384 when columns and
+ * pitches are multiples of 4 and pointers aligned to 4 elements, 8192 otherwise
+ * (else DDL_E_UNSUPP: take the two calls).
+ * dgamma and dbeta may be NULL.  Uses up to 512 * cols floats of workspace. */
+int ddl_ln_bwd_whole_rows(const void* dy, const void* x, int dtype, int64_t rows,
+                          int64_t cols, int64_t ld_dy, int64_t ld_x,
+                          const float* mean, const float* rstd,
+                          const void* gamma, float weight, void* dx,
+                          int64_t ld_dx, float* workspace,
+                          int64_t workspace_elems, void* dgamma, void* dbeta,
+                          void* stream);
 int ddl_ln_bwd_partial_params_f32(const float* dy, const float* x, int64_t rows,
                                   int64_t cols, int64_t ld_dy, int64_t ld_x,
                                   const float* mean, const float* rstd,

@@ -503,6 +503,38 @@ def test_layer_norm_backward_of_whole_rows_in_one_pass(ops, rows, cols, dtype):
     assert dg5 is None and db5 is None and torch.equal(dx5, dx)
 
 
+@pytest.mark.parametrize("rows,cols,pad", [(1, 1028, 0), (5, 1025, 0), (37, 2048, 4), (3, 2052, 0), (66, 4096, 1), (1029, 4097, 0),
+                                           (9, 8192, 0), (7, 8191, 0), (6, 8196, 0), (10, 16384, 8), (8200, 1032, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_layer_norm_backward_of_long_whole_rows(ops, rows, cols, pad, dtype):
+    """Rows a workgroup owns: dx, dgamma and dbeta in one pass against float64 autograd of the same inputs, at the widths
+    where the kernel's shape changes, aligned and not, with a pitch, with one row per split and with several; and the row
+    sums and column sums of the split form (a split per CU from 8161 rows on)."""
+    gen = torch.Generator().manual_seed(rows * 7 + cols)
+    store = torch.randn(2, rows, cols + pad, generator=gen).to(dtype)
+    x, dy = store[0, :, :cols], store[1, :, :cols]
+    gamma = (1 + 0.1 * torch.randn(cols, generator=gen)).to(dtype)
+    beta = torch.zeros(cols).to(dtype)
+    sg, gg = store.cuda(), gamma.cuda()
+    xg, dyg = sg[0, :, :cols], sg[1, :, :cols]
+    _, mean, rstd = ops.layer_norm(xg, gg, beta.cuda(), 1e-5, want_stats=True)
+    assert ops.ln_backward_whole_rows_supported(dyg, xg, gg)
+    dx, dg, db = ops.ln_backward_whole_rows(dyg, xg, mean, rstd, gg, 1.0 / cols)
+    only_dx = ops.ln_backward_whole_rows(dyg, xg, mean, rstd, gg, 1.0 / cols, want_gamma=False, want_beta=False)
+    assert torch.equal(only_dx[0], dx) and only_dx[1] is None and only_dx[2] is None
+    sums, work = ops.ln_backward_partial_params(dyg, xg, mean, rstd, gg)
+    dx2, dg2, db2 = ops.ln_backward_input_params(dyg, xg, mean, rstd, gg, sums.unsqueeze(0).contiguous(), 1.0 / cols, work)
+    xr, gr, br = x.double().requires_grad_(True), gamma.double().requires_grad_(True), beta.double().requires_grad_(True)
+    F.layer_norm(xr, (cols,), gr, br, 1e-5).backward(dy.double())
+    # one rounding of the result (half a unit in the last of 24, 8 or 11 bits: 2^-24, 2^-8, 2^-11 of it), and fp32 sums: a
+    # few units of the sums' size (dx: of its terms; parameters: sqrt(rows) of dy xhat)
+    ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for got_dx, got_dg, got_db in ((dx, dg, db), (dx2, dg2, db2)):
+        for got, want, size in ((got_dx, xr.grad, 4.0), (got_dg, gr.grad, 4.0 * rows ** 0.5), (got_db, br.grad, 4.0 * rows ** 0.5)):
+            err = (got.cpu().double() - want).abs()
+            assert bool((err <= ulp * want.abs() + 2e-6 * size).all()), float(err.max())
+
+
 @pytest.mark.parametrize("dtype,ulp", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)])
 @pytest.mark.parametrize("cols", [[256, 256], [300, 212], [7, 9], [2048], [1030]])
 def test_layernorm_backward_16_bit_elements(ops, dtype, ulp, cols):
