@@ -24,6 +24,7 @@ DDL_MAX_DIMS = 8
 
 DDL_OP_COPY = 0
 DDL_OP_ADD = 1
+DDL_OP_MOVE = 3
 
 DDL_DT_BITS = 0
 DDL_DT_F32 = 1

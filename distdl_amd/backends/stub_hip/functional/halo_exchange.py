@@ -2,17 +2,19 @@
 
 Dimension-ordered exchange of the reference
 (backends/mpi_numpy/functional/halo_exchange.py:13-78 forward, :81-144
-adjoint).  Per exchange dimension the two bulk slabs are packed by one launch,
-the transport swaps them with the neighbours, and the two ghost slabs are
-unpacked by one launch; dimension i sees the ghosts of dimensions < i, which is
-what makes the corners right.  The adjoint walks the dimensions backwards:
-pack the ghosts, clear them, swap, ADD what arrives into the bulk.
+adjoint).  Per exchange dimension the two bulk slabs are packed by one launch (the first
+dimension's by the launch that copies the input), the transport swaps them with
+the neighbours, and the two ghost slabs are unpacked by one launch; dimension i
+sees the ghosts of dimensions < i, which is what makes the corners right.  The
+adjoint walks the dimensions backwards: move the ghosts out (pack and clear, one
+launch), swap, ADD what arrives into the bulk.
 """
 
 __all__ = ["HaloExchangeFunction"]
 
 import torch
 
+from .... import _lib
 from .... import hip_ops
 from ....utilities.slicing import compute_nd_slice_shape
 from ....utilities.torch import zero_volume_tensor
@@ -31,22 +33,90 @@ class SliceTable(list):
         self.plans = {}
 
 
-def _plans(slices, tensor, i):
-    """(bulk plan, ghost plan) of exchange dimension ``i``; each plan holds the
-    left and the right box."""
+_INPUT, _TENSOR = 0, 1     # slots of a launch's base addresses; buffer j of dimension i has 2 + 4 i + j
+_LEFT_BULK, _LEFT_GHOST, _RIGHT_BULK, _RIGHT_GHOST = range(4)
+
+
+class _Plan:
+    """The launches of one direction for one structure of the tensor, lowered
+    once.  Buffers are looked up on every call (a pooled buffer may have been
+    reallocated); what is kept is geometry only."""
+
+    def __init__(self, slices, buffers, shape, strides, elem_size, forward):
+        self.dims = []
+        tensor_strides = hip_ops.contiguous_strides(shape)
+
+        def boxes(i, sides, to_buffer, from_input=False):
+            """Boxes between the strips ``sides`` of dimension ``i`` and their buffers."""
+            out = []
+            for j in sides:
+                if buffers[i][j] is None:
+                    continue
+                box = slices[i][j]
+                extent = [int(s.stop) - int(s.start) for s in box]
+                own = strides if from_input else tensor_strides
+                offset = sum(int(s.start) * t for s, t in zip(box, own))
+                packed = hip_ops.contiguous_strides(extent)
+                slot = 2 + 4 * i + j
+                if to_buffer:
+                    out.append((_INPUT if from_input else _TENSOR, offset, slot, 0, extent, own, packed))
+                else:
+                    out.append((slot, 0, _TENSOR, offset, extent, packed, own))
+            return out
+
+        bulk, ghost = (_LEFT_BULK, _RIGHT_BULK), (_LEFT_GHOST, _RIGHT_GHOST)
+        # The copy of the input takes the strips of the first dimension that sends any along: nothing has been written over
+        # them yet, and no other dimension's strips are in the buffers, which all dimensions share.
+        first = [(_INPUT, 0, _TENSOR, 0, list(shape), strides, tensor_strides)]
+        untouched = True
+        for i in range(len(slices)):
+            views = [None if b is None else (b, compute_nd_slice_shape(s)) for s, b in zip(slices[i], buffers[i])]
+            if forward:
+                pack, unpack = boxes(i, bulk, True, untouched), boxes(i, ghost, False)
+                merged = untouched
+                untouched = untouched and not pack and not unpack
+                if merged:
+                    first += pack
+                    pack = []
+                self.dims.append((views, [hip_ops.BoxLaunch(pack, elem_size)], [hip_ops.BoxLaunch(unpack, elem_size)]))
+            else:
+                add = boxes(i, bulk, False)
+                if len(add) == 2 and slices[i][0][i].stop > slices[i][2][i].start:
+                    # Narrow shards: the left and right bulk strips share elements, so
+                    # the two accumulations must not run in one launch.
+                    adds = [hip_ops.BoxLaunch(add[:1], elem_size), hip_ops.BoxLaunch(add[1:], elem_size)]
+                else:
+                    adds = [hip_ops.BoxLaunch(add, elem_size)]
+                self.dims.append((views, [hip_ops.BoxLaunch(boxes(i, ghost, True), elem_size)], adds))
+        self.first = hip_ops.BoxLaunch(first, elem_size) if forward else None
+
+
+def _plan(slices, buffers, tensor, forward):
     cache = getattr(slices, "plans", None)
-    key = (i, tuple(tensor.shape), tuple(tensor.stride()))
-    if cache is not None and key in cache:
-        return cache[key]
-    lbs, lgs, rbs, rgs = slices[i]
-    plans = (hip_ops.BoxPlan.from_slices(tensor, [lbs, rbs]), hip_ops.BoxPlan.from_slices(tensor, [lgs, rgs]))
-    if cache is not None:
-        cache[key] = plans
-    return plans
+    key = (forward, tensor.shape, tensor.stride(), tensor.element_size(), tuple([b is None for side in buffers for b in side]))
+    plan = None if cache is None else cache.get(key)
+    if plan is None:
+        plan = _Plan(slices, buffers, tuple(int(n) for n in tensor.shape), [int(s) for s in tensor.stride()], tensor.element_size(), forward)
+        if cache is not None:
+            cache[key] = plan
+    return plan
 
 
-def _dim_views(slices_i, buffers_i):
-    return [None if b is None else b.get_view(compute_nd_slice_shape(s)) for s, b in zip(slices_i, buffers_i)]
+def _dim_views(views, tensor, bases):
+    """The four buffer views of a dimension; their addresses go into ``bases``."""
+    out = []
+    for v in views:
+        if v is None:
+            out.append(None)
+            bases.append(0)
+            continue
+        buffer, shape = v
+        view = buffer.get_view(shape)
+        if view.dtype != tensor.dtype or not view.is_cuda:
+            raise ValueError(f"buffer {tuple(view.shape)}/{view.dtype} on {view.device} does not match a tensor of {tensor.dtype}")
+        out.append(view)
+        bases.append(view.data_ptr())
+    return out
 
 
 def _swap(P_x, neighbor_ranks_i, out_left, out_right, in_left, in_right):
@@ -83,20 +153,20 @@ class HaloExchangeFunction(torch.autograd.Function):
 
         # The reference works on a copy because marking the input dirty breaks
         # some downstream layers (halo_exchange.py:26-30); the copy runs on the
-        # box kernel as one contiguous box.
+        # box kernel, which packs the first dimension's strips in the same launch.
         src = input.detach()
+        hip_ops._require_gpu(src)
         output = torch.empty_like(src, memory_format=torch.contiguous_format)
-        full = tuple(slice(0, int(s)) for s in src.shape)
-        hip_ops.copy_box(src, full, output, full)
-
-        for i in range(P_x.dim):
-            lbb, lgb, rbb, rgb = _dim_views(slices[i], buffers[i])
-            bulk_plan, ghost_plan = _plans(slices, output, i)
-            if lbb is not None or rbb is not None:
-                bulk_plan.pack(output, [lbb, rbb])
+        plan = _plan(slices, buffers, src, True)
+        bases = [src.data_ptr(), output.data_ptr()]
+        views = [_dim_views(dim[0], output, bases) for dim in plan.dims]
+        plan.first.run(bases)
+        for i, (lbb, lgb, rbb, rgb) in enumerate(views):
+            for launch in plan.dims[i][1]:
+                launch.run(bases)
             _swap(P_x, neighbor_ranks[i], lbb, rbb, lgb, rgb)
-            if lgb is not None or rgb is not None:
-                ghost_plan.unpack(output, [lgb, rgb])
+            for launch in plan.dims[i][2]:
+                launch.run(bases)
         return output
 
     @staticmethod
@@ -112,18 +182,18 @@ class HaloExchangeFunction(torch.autograd.Function):
         if not grad_output.is_contiguous():
             raise ValueError("HaloExchange adjoint needs a contiguous gradient")
 
-        for i in reversed(range(P_x.dim)):
-            lbb, lgb, rbb, rgb = _dim_views(slices[i], buffers[i])
-            bulk_plan, ghost_plan = _plans(slices, grad_output, i)
-            if lgb is not None or rgb is not None:
-                ghost_plan.pack(grad_output, [lgb, rgb])
-                ghost_plan.zero(grad_output)
+        hip_ops._require_gpu(grad_output)
+        if grad_output.dtype not in hip_ops._ADD_DTYPES:
+            raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
+        add_dtype = hip_ops._ADD_DTYPES[grad_output.dtype]
+        plan = _plan(slices, buffers, grad_output, False)
+        bases = [0, grad_output.data_ptr()]
+        views = [_dim_views(dim[0], grad_output, bases) for dim in plan.dims]
+        for i in reversed(range(len(views))):
+            lbb, lgb, rbb, rgb = views[i]
+            for launch in plan.dims[i][1]:
+                launch.run(bases, op=_lib.DDL_OP_MOVE)
             _swap(P_x, ctx.neighbor_ranks[i], lgb, rgb, lbb, rbb)
-            if lbb is not None and rbb is not None and slices[i][0][i].stop > slices[i][2][i].start:
-                # Narrow shards: the left and right bulk strips share elements, so
-                # the two accumulations must not run in one launch.
-                bulk_plan.unpack(grad_output, [lbb, None], accumulate=True)
-                bulk_plan.unpack(grad_output, [None, rbb], accumulate=True)
-            elif lbb is not None or rbb is not None:
-                bulk_plan.unpack(grad_output, [lbb, rbb], accumulate=True)
+            for launch in plan.dims[i][2]:
+                launch.run(bases, op=_lib.DDL_OP_ADD, dtype=add_dtype)
         return grad_output, None, None, None, None

@@ -38,7 +38,7 @@ constexpr uint32_t kPersistentBlocks = 4096;  // 16 per CU
 constexpr uint64_t kMaxVecs = (1ull << 31) - kTileVecs;
 constexpr uint64_t kLongRunBytes = 64 << 10;   // boxes whose innermost runs are at least this long are interleaved within a launch
 
-enum Op { OP_COPY = 0, OP_ADD = 1, OP_ZERO = 2 };
+enum Op { OP_COPY = 0, OP_ADD = 1, OP_ZERO = 2, OP_MOVE = 3 };   // OP_MOVE: dst = src, src = 0
 
 // Multi-dword vectors are only promised dword alignment (see lower_box).
 typedef unsigned int u32x4_a __attribute__((ext_vector_type(4)));
@@ -310,6 +310,18 @@ __device__ inline void move_tile(DevBoxPtr bx, uint32_t tile) {
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u)
             if (live[u]) *reinterpret_cast<V*>(dst + doff[u]) = val[u];
+        return;
+    }
+    if constexpr (OP == OP_MOVE) {
+        // Once per element: lanes past the box repeat another lane's position and may have loaded what that one has cleared.
+        V z;
+        __builtin_memset(&z, 0, sizeof(V));
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+            if (live[u]) {
+                *reinterpret_cast<V*>(dst + doff[u]) = val[u];
+                *reinterpret_cast<V*>(const_cast<char*>(src) + soff[u]) = z;
+            }
         return;
     }
 #pragma unroll
@@ -975,7 +987,7 @@ int run_boxes(const ddl_box_t* boxes, int nbox, int elem_size, int op, int dtype
     if (op == DDL_OP_ADD) {
         if (dtype < DDL_DT_F32 || dtype > DDL_DT_I64) return fail(DDL_E_ARG, "DDL_OP_ADD needs an arithmetic dtype, got %d", dtype);
         if (dt_size[dtype] != elem_size) return fail(DDL_E_ARG, "dtype %d does not have element size %d", dtype, elem_size);
-    } else if (op != DDL_OP_COPY && op != OP_ZERO) {
+    } else if (op != DDL_OP_COPY && op != OP_ZERO && op != OP_MOVE) {
         return fail(DDL_E_ARG, "unknown box operation %d", op);
     }
     std::vector<DevBox> dev;
@@ -984,6 +996,7 @@ int run_boxes(const ddl_box_t* boxes, int nbox, int elem_size, int op, int dtype
         if (int rc = lower_box(boxes[b], elem_size, has_src, &dev)) return rc;
     if (dev.empty()) return 0;
     if (op == OP_ZERO) return launch_batches<OP_ZERO, uint8_t>(dev, stream);
+    if (op == OP_MOVE) return launch_batches<OP_MOVE, uint8_t>(dev, stream);
     if (op == DDL_OP_COPY) return launch_batches<OP_COPY, uint8_t>(dev, stream);
     switch (dtype) {
         case DDL_DT_F32: return launch_batches<OP_ADD, float>(dev, stream);
@@ -1139,7 +1152,7 @@ int ddl_sum_boxes(const ddl_box_t* box, const void* const* srcs, int nsrc, int e
 }
 
 int ddl_copy_boxes(const ddl_box_t* boxes, int nbox, int elem_size, int op, int dtype, void* stream) {
-    if (op != DDL_OP_COPY && op != DDL_OP_ADD) return ddl::fail(DDL_E_ARG, "unknown box operation %d", op);
+    if (op != DDL_OP_COPY && op != DDL_OP_ADD && op != DDL_OP_MOVE) return ddl::fail(DDL_E_ARG, "unknown box operation %d", op);
     return ddl::run_boxes(boxes, nbox, elem_size, op, dtype, true, static_cast<hipStream_t>(stream));
 }
 

@@ -146,6 +146,49 @@ class BoxPlan:
         _lib.check(rc, "ddl_zero_boxes")
 
 
+def contiguous_strides(shape):
+    strides, run = [], 1
+    for n in reversed(shape):
+        strides.append(run)
+        run *= int(n)
+    return strides[::-1]
+
+
+class BoxLaunch:
+    """The boxes of one ``ddl_copy_boxes`` call, lowered once.
+
+    ``entries`` are ``(src slot, src offset, dst slot, dst offset, shape, src
+    strides, dst strides)``, offsets and strides in elements of ``elem_size``
+    bytes; a slot is an index into the base addresses that a call supplies.
+    Boxes without elements are left out.  A call fills a copy of the
+    descriptors, so threads may share an object."""
+
+    def __init__(self, entries, elem_size):
+        entries = [e for e in entries if all(int(n) > 0 for n in e[4])]
+        self.elem_size = elem_size
+        self.n = len(entries)
+        self._type = _lib.ddl_box_t * max(self.n, 1)
+        boxes = self._type()
+        self._bases = []
+        for i, (src, src_off, dst, dst_off, shape, src_strides, dst_strides) in enumerate(entries):
+            boxes[i].ndim = len(shape)
+            for d, (n, s, t) in enumerate(zip(shape, src_strides, dst_strides)):
+                boxes[i].shape[d], boxes[i].src_stride[d], boxes[i].dst_stride[d] = int(n), int(s), int(t)
+            self._bases.append((src, int(src_off) * elem_size, dst, int(dst_off) * elem_size))
+        self._template = bytes(boxes)
+
+    def run(self, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
+        if self.n == 0:
+            return
+        boxes = self._type.from_buffer_copy(self._template)
+        for box, (src, src_off, dst, dst_off) in zip(boxes, self._bases):
+            box.src = bases[src] + src_off
+            box.dst = bases[dst] + dst_off
+        rc = _lib.load().ddl_copy_boxes(boxes, self.n, self.elem_size, op, dtype, _stream())
+        if rc:
+            _lib.check(rc, "ddl_copy_boxes")
+
+
 def copy_box(src, src_slices, dst, dst_slices, accumulate=False):
     """dst[dst_slices] (+)= src[src_slices]; both strided, same box shape."""
     _require_gpu(src, dst)

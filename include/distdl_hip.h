@@ -60,6 +60,8 @@ typedef struct ddl_box {
 
 #define DDL_OP_COPY 0   /* dst  = src                                          */
 #define DDL_OP_ADD  1   /* dst += src  (needs `dtype`; boxes must not alias)   */
+#define DDL_OP_MOVE 3   /* dst  = src, src = 0 (ddl_copy_boxes only; a source
+                           element must belong to one box)                     */
 
 #define DDL_DT_BITS 0   /* opaque elements of elem_size bytes (copy only)      */
 #define DDL_DT_F32  1
@@ -77,7 +79,9 @@ typedef struct ddl_box {
  *   backends/mpi_numpy/functional/repartition.py:179-190 (np.copyto(output[ysl], input[xsl])),
  *   backends/nccl_cupy/functional/repartition.py:186,
  * and, with DDL_OP_ADD, the adjoint accumulation of HaloExchange,
- *   backends/mpi_numpy/functional/halo_exchange.py:138,140 (grad_output[lbs] += lbb). */
+ *   backends/mpi_numpy/functional/halo_exchange.py:138,140 (grad_output[lbs] += lbb).
+ * DDL_OP_MOVE is the adjoint's other half, ghosts packed and cleared
+ * (halo_exchange.py:108-115), in one pass. */
 int ddl_copy_boxes(const ddl_box_t* boxes, int nbox, int elem_size,
                    int op, int dtype, void* stream);
 

@@ -53,6 +53,34 @@ def random_boxes(shape, nbox, rng):
 
 
 @pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32, torch.float64])
+@pytest.mark.parametrize("shape,column", [((37,), False), ((5, 1030), False), ((70, 33), True), ((9, 64, 66), True), ((3, 2, 4096), False)])
+def test_boxes_moved_out_and_cleared(ops, dtype, shape, column):
+    """DDL_OP_MOVE: two disjoint strips of a tensor (along rows, or single columns: one element per row) end up in their
+    buffers, the strips are zero afterwards and the rest of the tensor is untouched; strips that end inside a tile have
+    lanes that repeat an element, which must still be read before it is cleared."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(sum(shape))
+    x_cpu = random_bits(shape, dtype, gen)
+    x = x_cpu.cuda()
+    d = len(shape) - 1 if column else 0
+    whole = [slice(0, m) for m in shape]
+    strips = [list(whole), list(whole)]
+    strips[0][d], strips[1][d] = slice(0, 1), slice(shape[d] - 2 if shape[d] > 2 else 1, shape[d])
+    strides = ops.contiguous_strides(shape)
+    entries, bufs = [], []
+    for k, sl in enumerate(strips):
+        extent = [s.stop - s.start for s in sl]
+        bufs.append(torch.full(extent, 0, dtype=dtype, device="cuda"))
+        entries.append((0, sum(s.start * t for s, t in zip(sl, strides)), 1 + k, 0, extent, strides, ops.contiguous_strides(extent)))
+    ops.BoxLaunch(entries, x.element_size()).run([x.data_ptr()] + [b.data_ptr() for b in bufs], op=_lib.DDL_OP_MOVE)
+    want = bits(x_cpu).clone()
+    for sl, buf in zip(strips, bufs):
+        assert torch.equal(bits(buf.cpu()), bits(x_cpu)[tuple(sl)])
+        want[tuple(sl)] = 0
+    assert torch.equal(bits(x.cpu()), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32, torch.float64])
 @pytest.mark.parametrize("shape", [(37,), (5, 130), (6, 7, 64), (3, 4, 5, 6, 7), (2, 3, 2, 3, 2, 3, 2, 5)])
 def test_pack_unpack_random_boxes(ops, dtype, shape):
     gen = torch.Generator().manual_seed(sum(shape) * 64 + torch.empty((), dtype=dtype).element_size())
