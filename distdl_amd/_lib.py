@@ -121,6 +121,9 @@ SIGNATURES = {
     "ddl_gemm_ws": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int, c_int64, c_int64,
                             c_int64, c_int64, c_void_p, c_int64, c_void_p]),
     "ddl_gemm_workspace": (c_int64, [c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64]),
+    "ddl_linear_backward_workspace": (c_int64, [c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_int]),
+    "ddl_linear_backward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64,
+                                    c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p]),
     "ddl_gemm_f32": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64,
                              c_int64, c_int64, c_void_p]),
     "ddl_colsum": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p]),

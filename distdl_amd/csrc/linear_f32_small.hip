@@ -282,7 +282,8 @@ int launch_shape(const char* who, const Small32& plan, const Part32& part, float
 
 // The estimates are fits to a sweep over M, N, K of 5 .. 16384 on all operand layouts, in microseconds: 4 + per k-tile (per
 // round of one k-tile for every group) 0.68 for a lone 64 x 64 tile, 0.52 for each that a CU has to work through, 0.78 in
-// two or four groups + the epilogue of every further tile + for splits a second launch and the partial tiles at 5 TB/s.
+// two or four groups + the epilogue of every further tile + for splits a second launch (2.3, and 5 for
+// what it and the workspace cost the host, which many callers wait for) and the partial tiles at 5 TB/s.
 // Measured, general kernel of 128 x 128 tiles -> here: M 777, N 333, K 1024 107.2 -> 15.7 (three splits; 17.7 in two
 // groups); its adjoint M 777, N 1024, K 333 45.4 -> 12.4 and M 333, N 1024, K 777, both operands along their rows, 84.1 ->
 // 15.6; M 8, N 4096, K 4096 365 -> 20.  256 x 256 tiles -> here: M = N = K = 2048 351 -> 153, M 4096, N 4096, K 1024 310 ->
@@ -297,7 +298,7 @@ Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace
         for (const int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
             if (splits > 1 && (tiles * splits > 4 * static_cast<int64_t>(cus) || ktiles < 2 * splits * groups || tiles * splits * bm * bn > workspace)) break;
             const int64_t per_cu = (tiles * splits + cus - 1) / cus, kt = (ktiles + splits - 1) / splits;
-            double us = 4 + (splits > 1 ? 2.3 + static_cast<double>(tiles) * splits * bm * bn * 8 / 5e6 : 0);
+            double us = 4 + (splits > 1 ? 7.5 + static_cast<double>(tiles) * splits * bm * bn * 8 / 5e6 : 0);
             if (groups == 1)
                 us += kt * (per_cu > 1 ? 0.52 * per_cu + 0.1 : 0.68) + (per_cu > 2 ? per_cu - 2 : 0) * 1.8;
             else

@@ -457,7 +457,8 @@ int launch16(const char* who, const Small16& plan, bool xt, bool wt, const Part1
 //   tiles    3.8 + per k-tile 0.19 for each tile a CU has (0.30 for a lone workgroup, whose waits nothing hides;
 //            0.375 per pair of k-tiles with two groups, which hide each other's) + 1.4 for the epilogue of every tile
 //            beyond those resident at the start
-//   splits   2.3 for the second launch + the partial tiles (16 KiB, written and read) at 5 TB/s
+//   splits   2.3 for the second launch and 5 for what it and the workspace cost the host, which many callers wait for
+//            (M 6964, N 136, K 5632: 39.5 in two splits, 38 without) + the partial tiles (16 KiB, written and read) at 5 TB/s
 // Measured, large tiles -> here: M 8, N 3584, K 8192 69.0 -> 13.1 us (skinny; 14.2 as tiles in two groups and four splits);
 // M 64 of the same 69.5 -> 15.4 (two groups, four splits; 20.7 skinny); M 1024, N 1024, K 4096 (x w^T with w read down its
 // columns) 39.1 -> 19.5 (two groups; 21.4 in two splits); M 1024, N 512, K 512 10.8 -> 6.0.  Large tiles stay where they
@@ -483,7 +484,7 @@ Small16 plan_small16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus,
     for (const int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
         if (splits > 1 && (tiles * splits > 4 * static_cast<int64_t>(cus) || ktiles < 4 * splits || tiles * splits * 4096 > workspace)) break;
         const int64_t per_cu = (tiles * splits + cus - 1) / cus, kt = (ktiles + splits - 1) / splits;
-        const double sum = splits > 1 ? 2.3 + tiles * splits * 0.0066 : 0;
+        const double sum = splits > 1 ? 7.5 + tiles * splits * 0.0066 : 0;
         const double step = per_cu > 1 ? 0.19 * per_cu : 0.30;
         take(3.8 + kt * step + (per_cu > 2 ? per_cu - 2 : 0) * 1.4 + sum, Small16::kTiles, 1, splits);
         take(3.9 + ((kt + 1) / 2) * 0.375 * per_cu + (per_cu - 1) * 1.4 + sum, Small16::kTiles, 2, splits);

@@ -240,8 +240,9 @@ def sum_boxes(srcs, src_slices, dst, dst_slices, divisor=1):
     first = srcs[0]
     _require_gpu(dst, *srcs)
     nd = first.dim()
+    dtype, shape, strides, dst_shape, dst_strides = dst.dtype, first.shape, first.stride(), dst.shape, dst.stride()
     for t in srcs:
-        if t.dtype != dst.dtype or tuple(t.shape) != tuple(first.shape) or t.stride() != first.stride():
+        if t.dtype != dtype or t.shape != shape or t.stride() != strides:
             raise ValueError("sum_boxes: sources must agree in dtype, shape and strides with each other (dtype: and with dst)")
     if dst.dtype not in _ADD_DTYPES:
         raise ValueError(f"sums are not available for {dst.dtype}")
@@ -251,17 +252,15 @@ def sum_boxes(srcs, src_slices, dst, dst_slices, divisor=1):
     box.ndim = nd
     soff = doff = 0
     for d in range(nd):
-        n = int(src_slices[d].stop) - int(src_slices[d].start)
-        if n != int(dst_slices[d].stop) - int(dst_slices[d].start):
+        s, t = src_slices[d], dst_slices[d]
+        n = int(s.stop) - int(s.start)
+        if n != int(t.stop) - int(t.start):
             raise ValueError("sum_boxes: source and destination boxes differ in shape")
-        if src_slices[d].start < 0 or src_slices[d].stop > first.shape[d] or \
-           dst_slices[d].start < 0 or dst_slices[d].stop > dst.shape[d]:
+        if s.start < 0 or s.stop > shape[d] or t.start < 0 or t.stop > dst_shape[d]:
             raise ValueError("sum_boxes: box outside tensor")
-        box.shape[d] = n
-        box.src_stride[d] = first.stride(d)
-        box.dst_stride[d] = dst.stride(d)
-        soff += int(src_slices[d].start) * first.stride(d)
-        doff += int(dst_slices[d].start) * dst.stride(d)
+        box.shape[d], box.src_stride[d], box.dst_stride[d] = n, strides[d], dst_strides[d]
+        soff += int(s.start) * strides[d]
+        doff += int(t.start) * dst_strides[d]
     es = dst.element_size()
     box.dst = dst.data_ptr() + doff * es
     ptrs = [t.data_ptr() + soff * es for t in srcs]
@@ -276,13 +275,13 @@ def sum_boxes(srcs, src_slices, dst, dst_slices, divisor=1):
     # temporary of the box's shape and added to dst by an accumulating copy.
     rc = lib.ddl_sum_boxes(ctypes.byref(box), _lib.ptr_array(ptrs[:1]), 1, es, dt, float(divisor), _stream())
     _lib.check(rc, "ddl_sum_boxes")
-    shape = [int(box.shape[d]) for d in range(nd)]
-    whole = [slice(0, n) for n in shape]
+    extent = [int(box.shape[d]) for d in range(nd)]
+    whole = [slice(0, n) for n in extent]
     for t in srcs[1:]:
         if divisor == 1:
             copy_box(t, src_slices, dst, dst_slices, accumulate=True)
             continue
-        tmp = torch.empty(shape, dtype=dst.dtype, device=dst.device)
+        tmp = torch.empty(extent, dtype=dst.dtype, device=dst.device)
         sum_boxes([t], src_slices, tmp, whole, divisor)
         copy_box(tmp, whole, dst, dst_slices, accumulate=True)
 
@@ -867,6 +866,12 @@ def colsum_bf16(a):
     return colsum(a)
 
 
+@functools.lru_cache(maxsize=4096)
+def _linear_backward_workspace(dt, m, n, k, ld_x, ld_w, ld_dy, need_input, need_weight, need_bias):
+    """Floats the adjoint of these sizes and pitches can use (a function of its arguments alone)."""
+    return _lib.load().ddl_linear_backward_workspace(dt, m, n, k, ld_x, ld_w, ld_dy, bool(need_input), bool(need_weight), bool(need_bias))
+
+
 def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, need_bias=True):
     """Adjoint of :func:`linear`: ``(dx, dw, db)`` for ``y = x @ weight.T + bias``
     (entries not asked for are None).  Both products read their operands where
@@ -886,33 +891,38 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
         dy = contiguous(dy)
     m = x2.shape[0]
     dx = dw = db = None
-    if dt == _lib.DDL_DT_F32:
-        if x2.stride(1) != 1 and k > 1:
-            x2 = contiguous(x2)
-        if weight.stride(1) != 1 and k > 1:
-            weight = contiguous(weight)
-        ld_dy, ld_x, ld_w = (dy.stride(0) if m > 1 else n), (x2.stride(0) if m > 1 else k), (weight.stride(0) if n > 1 else k)
-        if need_input:
-            dx = torch.empty((m, k), dtype=x.dtype, device=x.device)
-            if n == 0:
-                dx.zero_()
-            else:   # dx[m, j] = sum_n dy[m, n] w[n, j]: rows of the second operand are the columns of w
-                _gemm(dy, ld_dy, 1, weight, 1, ld_w, None, dx, dt, m, k, n)
-            dx = dx.reshape(x.shape)
-        if need_weight:
-            dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
-            if m == 0:
-                dw.zero_()
-            else:   # dw[i, j] = sum_m dy[m, i] x[m, j]: both operands are read down their columns
-                _gemm(dy, 1, ld_dy, x2, 1, ld_x, None, dw, dt, n, k, m)
-        if need_bias:
-            db = colsum(dy)
-        return dx, dw, db
     if x2.stride(1) != 1 and k > 1:
         x2 = contiguous(x2)
     if weight.stride(1) != 1 and k > 1:
         weight = contiguous(weight)
     ld_dy, ld_x, ld_w = (dy.stride(0) if m > 1 else n), (x2.stride(0) if m > 1 else k), (weight.stride(0) if n > 1 else k)
+    if dt == _lib.DDL_DT_F32:
+        if not (m and n and k):
+            if need_input:
+                dx = torch.zeros((m, k), dtype=x.dtype, device=x.device).reshape(x.shape)
+            if need_weight:
+                dw = torch.zeros((n, k), dtype=x.dtype, device=x.device)
+            if need_bias:
+                db = colsum(dy)
+            return dx, dw, db
+        direct = True
+    else:
+        direct = (bool(m and n and k) and
+                  (not need_input or (_along_k_ok(dy, ld_dy, n) and _along_rows_ok(weight, ld_w, k, n))) and
+                  (not need_weight or (_along_rows_ok(dy, ld_dy, n, m) and _along_rows_ok(x2, ld_x, k, m))))
+    if direct:      # every operand is read where it lies: one call for all that is wanted
+        if need_input:
+            dx = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+        if need_weight:
+            dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
+        if need_bias:
+            db = torch.empty(n, dtype=x.dtype, device=x.device)
+        elems = _linear_backward_workspace(dt, m, n, k, ld_x, ld_w, ld_dy, need_input, need_weight, need_bias)
+        work = torch.empty(elems, dtype=torch.float32, device=x.device) if elems else None
+        rc = _lib.load().ddl_linear_backward(x2.data_ptr(), weight.data_ptr(), dy.data_ptr(), _ptr(dx), _ptr(dw), _ptr(db), dt, m, n, k,
+                                             ld_x, ld_w, ld_dy, _ptr(work), elems, _stream())
+        _lib.check(rc, "ddl_linear_backward")
+        return dx, dw, db
     if need_input:
         # dx[m, j] = sum_n dy[m, n] w[n, j]: dy is read along n, w down its columns
         if m and n and k and _along_k_ok(dy, ld_dy, n) and _along_rows_ok(weight, ld_w, k, n):

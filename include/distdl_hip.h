@@ -519,6 +519,17 @@ int ddl_gemm_ws(const void* a, int64_t a_row_stride, int64_t a_k_stride,
                 const void* bias, void* y, int dtype, int64_t ldy, int64_t M,
                 int64_t N, int64_t K, float* workspace, int64_t workspace_elems,
                 void* stream);
+/* The adjoint of ddl_linear in one call, on operands that ddl_gemm can read
+ * where they lie (row pitches ldx, ldw, lddy; dx, dw and db contiguous): dx, dw
+ * and db may each be NULL.  `workspace` as for ddl_gemm_ws, with as many floats
+ * as ddl_linear_backward_workspace says for those wanted. */
+int64_t ddl_linear_backward_workspace(int dtype, int64_t M, int64_t N, int64_t K,
+                                      int64_t ldx, int64_t ldw, int64_t lddy,
+                                      int want_dx, int want_dw, int want_db);
+int ddl_linear_backward(const void* x, const void* w, const void* dy, void* dx,
+                        void* dw, void* db, int dtype, int64_t M, int64_t N,
+                        int64_t K, int64_t ldx, int64_t ldw, int64_t lddy,
+                        float* workspace, int64_t workspace_elems, void* stream);
 int ddl_gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride,
                  const float* b, int64_t b_row_stride, int64_t b_k_stride,
                  const float* bias, float* y, int64_t ldy,

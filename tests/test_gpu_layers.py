@@ -1576,7 +1576,7 @@ def test_gemm_16_bit_reads_operands_where_they_lie(ops, dtype, a_t, b_t, M, N, K
     (False, False, 65, 65, 64, False), (False, True, 72, 136, 200, False), (True, False, 136, 67, 456, False),
     (True, True, 2056, 1032, 136, False),
     # the reduction split over workgroups: unequal shares, a share that straddles K
-    (False, False, 100, 130, 4168, True), (False, True, 72, 136, 2120, True), (True, False, 200, 264, 4104, True),
+    (False, False, 100, 130, 4168, True), (False, True, 72, 136, 4168, True), (True, False, 200, 264, 4104, True),
     (True, True, 128, 64, 8191, True)])
 def test_gemm_16_bit_products_that_leave_the_chip_idle(ops, dtype, a_t, b_t, M, N, K, splits):
     """The skinny and small-tile kernels on integer operands (every sum is exact), with and without the workspace that
@@ -1654,8 +1654,8 @@ def test_gemm_f32_tiled_kernel_reads_every_operand_layout(ops, a_t, b_t, M, N, K
     # tiles of 64 x 64, 32 x 64 and 32 x 32; odd lengths and pitches; one k-tile, a straddling one, an odd number of rounds
     (4, 4, 1, 0, False), (5, 7, 9, 1, False), (33, 31, 33, 3, False), (64, 64, 64, 0, False), (130, 65, 96, 5, False),
     (1030, 517, 131, 0, False), (2050, 1027, 100, 2, False),
-    # the reduction split over workgroups, unequal shares
-    (201, 263, 1033, 1, True), (64, 100, 4095, 0, True),
+    # the reduction split over groups of wavefronts, and over workgroups, unequal shares
+    (201, 263, 1033, 1, False), (201, 263, 2501, 1, True), (64, 100, 4095, 0, True),
     # enough work for the 256 x 256 tiles, wide and narrow ones
     (4096, 4352, 1540, 4, False)])
 def test_gemm_f32_products_of_every_size_and_pitch(ops, a_t, b_t, M, N, K, pad, splits):
