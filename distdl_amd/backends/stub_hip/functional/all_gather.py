@@ -9,6 +9,8 @@ launch of the sum kernel (strided reads of the P slabs, one write)."""
 
 __all__ = ["AllGatherFunction", "gather_slabs", "reduce_scatter_slabs", "single_axis"]
 
+import functools
+
 import numpy as np
 import torch
 
@@ -16,22 +18,47 @@ from .... import hip_ops
 from ....utilities.slicing import compute_subshape
 
 
+@functools.lru_cache(maxsize=512)
+def _gather_launch(shapes, axis, elem_size):
+    """(output shape, launch) that joins contiguous pieces of these shapes along
+    ``axis``; the output is slot 0 of the launch, piece q slot 1 + q.  Geometry
+    only: a function of its arguments."""
+    shape = list(shapes[0])
+    shape[axis] = sum(s[axis] for s in shapes)
+    strides = hip_ops.contiguous_strides(shape)
+    entries, start = [], 0
+    for q, piece in enumerate(shapes):
+        entries.append((1 + q, 0, 0, start * strides[axis], piece, hip_ops.contiguous_strides(piece), strides))
+        start += piece[axis]
+    return tuple(shape), hip_ops.BoxLaunch(entries, elem_size)
+
+
+@functools.lru_cache(maxsize=512)
+def _slab(size, rank, shape, axis):
+    """(shape, source slices, destination slices) of the balanced slab that
+    worker ``rank`` of ``size`` keeps of a tensor along ``axis``."""
+    sizes = [int(np.asarray(compute_subshape(size, r, shape[axis])).reshape(-1)[0]) for r in range(size)]
+    start = sum(sizes[:rank])
+    out = list(shape)
+    out[axis] = sizes[rank]
+    src = [slice(0, n) for n in shape]
+    src[axis] = slice(start, start + sizes[rank])
+    return tuple(out), src, [slice(0, n) for n in out]
+
+
 def gather_slabs(P, local, axis, tag):
     """``local`` of every worker of ``P``, concatenated along ``axis`` in rank order."""
     transport = P._world.transport
     x = hip_ops.contiguous(local)
     parts = transport.gather_list(P, x, tag=tag)
-    extent = sum(int(p.shape[axis]) for p in parts)
-    shape = list(x.shape)
-    shape[axis] = extent
-    out = torch.empty(shape, dtype=x.dtype, device=x.device)
-    boxes, start = [], 0
+    hip_ops._require_gpu(x, *parts)
     for p in parts:
-        origin = [0] * out.dim()
-        origin[axis] = start
-        boxes.append((origin, list(p.shape)))
-        start += int(p.shape[axis])
-    hip_ops.BoxPlan(out.shape, out.stride(), boxes).unpack(out, parts)
+        if p.dtype != x.dtype or not p.is_contiguous():
+            raise ValueError(f"gathered piece {tuple(p.shape)}/{p.dtype} does not match {x.dtype} or is not contiguous")
+    axis = axis % x.dim()
+    shape, launch = _gather_launch(tuple([tuple(p.shape) for p in parts]), axis, x.element_size())
+    out = torch.empty(shape, dtype=x.dtype, device=x.device)
+    launch.run([out.data_ptr()] + [p.data_ptr() for p in parts])
     transport.release(P, tag=tag)
     return out
 
@@ -44,16 +71,8 @@ def reduce_scatter_slabs(P, full, axis, tag, divisor=1):
     transport = P._world.transport
     g = hip_ops.contiguous(full)
     grads = transport.gather_list(P, g, tag=tag)
-    me = int(P.rank)
-    extent = int(g.shape[axis])
-    sizes = [int(np.asarray(compute_subshape(P.size, r, extent)).reshape(-1)[0]) for r in range(P.size)]
-    start = sum(sizes[:me])
-    shape = list(g.shape)
-    shape[axis] = sizes[me]
+    shape, src, dst = _slab(int(P.size), int(P.rank), tuple(g.shape), axis % g.dim())
     out = torch.empty(shape, dtype=g.dtype, device=g.device)
-    src = [slice(0, int(n)) for n in g.shape]
-    src[axis] = slice(start, start + sizes[me])
-    dst = [slice(0, int(n)) for n in shape]
     if out.numel():
         hip_ops.sum_boxes(grads, src, out, dst, divisor)
     transport.release(P, tag=tag)
