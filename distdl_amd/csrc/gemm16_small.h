@@ -8,7 +8,7 @@ namespace ddl {
 typedef PartOf<uint16_t> Part16;
 
 struct Small16 {
-    enum Kind { kNone, kSkinny, kTiles };
+    enum Kind { kNone, kSkinny, kTiles, kAny };
     Kind kind = kNone;
     int groups = 1;              // kTiles: groups of wavefronts of a workgroup the reduction is split over (1 or 2)
     int splits = 1;              // kTiles: workgroups the reduction of a tile is split over
@@ -18,6 +18,9 @@ struct Small16 {
 // The cheapest way linear_small.hip has for this product within `workspace` floats, kNone if that is not below
 // `large_us`, the estimate for the large tiles (microseconds).
 Small16 plan_small16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double large_us);
+
+// The same for operands that are not aligned to 16 bytes (kAny, or kNone): against `large_us` and copying both operands.
+Small16 plan_any16(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double large_us);
 
 // Launches the product of `part` (its tile counts are set here) as planned; `partial` holds the splits' sums.
 int run_small16(const char* who, const Small16& plan, bool f16, bool xt, bool wt, const Part16& part, float* partial, int dev, hipStream_t s);

@@ -518,9 +518,13 @@ double large_us(bool low, int64_t cost, int64_t tiles, int64_t K, int cus) {
     return 6.5 + static_cast<double>((K + BK - 1) / BK) * rounds * (low ? 0.47 + 0.27 * fill * fill : 0.95 + 0.48 * fill * fill);
 }
 
+// Are the pitch and the lengths of an operand multiples of 16 bytes, as the aligned kernels ask?
+bool pitches_ok(const Operand16& o, int64_t rows, int64_t K) { return o.ld() % 8 == 0 && (o.transposed() ? rows : K) % 8 == 0; }
+
 struct Plan16 {
     Small16 small;            // kind other than kNone: linear_small.hip computes the product
     int64_t low_tiles = 0;    // otherwise this many tiles of 128 x 256, if not 0
+    double large = 0;         // estimate for the large tiles, microseconds
     int64_t wide_cols = 0;    // otherwise 256 x 256 tiles for the first columns, 256 x 192 for the rest
 };
 
@@ -536,19 +540,44 @@ Plan16 plan16(bool at, bool bt, int64_t M, int64_t N, int64_t K, int cus, int64_
     const bool low = low_cost * 11 < cost * 10;
     if (low) plan.low_tiles = low_tiles;
     // Products that leave most of the chip idle either way.
-    plan.small = plan_small16(at, bt, M, N, K, cus, workspace,
-                              large_us(low, low ? low_cost : cost, low ? low_tiles : tiles_m * cols, K, cus));
+    plan.large = large_us(low, low ? low_cost : cost, low ? low_tiles : tiles_m * cols, K, cus);
+    plan.small = plan_small16(at, bt, M, N, K, cus, workspace, plan.large);
     return plan;
 }
 
-// y[M, N] = a[M, K] . b[N, K]^T + bias in 16-bit elements.  `workspace` (may be null) for the sums of a split reduction.
+// Can an operand with `rows` rows be read from wherever it lies (gemm16_any)?
+bool readable_anywhere(const Operand16& o, int64_t rows, int64_t K) {
+    if (o.row_stride != 1 && o.k_stride != 1) return false;
+    return o.transposed() ? rows >= 8 && o.ld() >= rows : rows == 1 || o.ld() >= K;
+}
+
+// How gemm16_any computes the product of such operands, if it does.
+Small16 plan_anywhere(const Operand16& a, const Operand16& b, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace) {
+    if (!readable_anywhere(a, M, K) || !readable_anywhere(b, N, K)) return Small16{};
+    return plan_any16(M, N, K, cus, workspace, plan16(a.transposed(), b.transposed(), M, N, K, cus, 0).large);
+}
+
+// y[M, N] = a[M, K] . b[N, K]^T + bias in 16-bit elements.  `workspace` (may be null) for the sums of a split reduction;
+// `anywhere`: operands that are not aligned to 16 bytes are taken where gemm16_any is the way to read them.
 int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* bias, uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
-           float* workspace, int64_t workspace_elems, void* stream) {
+           float* workspace, int64_t workspace_elems, bool anywhere, void* stream) {
     if (M < 0 || N < 0 || K < 0 || ldy < N)
         return fail(DDL_E_ARG, "%s: M=%lld N=%lld K=%lld ldy=%lld", who, (long long)M, (long long)N, (long long)K, (long long)ldy);
     if (M == 0 || N == 0) return 0;
     if (!a.p || !b.p || !y) return fail(DDL_E_ARG, "%s: null pointer", who);
     if (K == 0) return fail(DDL_E_UNSUPP, "%s: K = 0", who);
+    if (anywhere && aligned_to(a.p, 2) && aligned_to(b.p, 2) && aligned_to(y, 2) && aligned_to(bias, 2) &&
+        !(aligned_to(a.p, 16) && aligned_to(b.p, 16) && pitches_ok(a, M, K) && pitches_ok(b, N, K))) {
+        int dev = 0;
+        const int cus = compute_units(dev);
+        const Small16 any = plan_anywhere(a, b, M, N, K, cus, workspace ? workspace_elems : 0);
+        if (any.kind != Small16::kNone) {
+            Part16 p{};
+            p.x = a.p, p.w = b.p, p.bias = bias, p.y = y, p.M = M, p.N = N, p.K = K, p.ldx = a.ld(), p.ldw = b.ld(), p.ldy = ldy;
+            p.vec_store = ldy % 4 == 0 && aligned_to(y, 8);
+            return run_small16(who, any, f16, a.transposed(), b.transposed(), p, workspace, dev, static_cast<hipStream_t>(stream));
+        }
+    }
     if (int rc = check_operand(who, "a", a, M, K)) return rc;
     if (int rc = check_operand(who, "b", b, N, K)) return rc;
     if (!aligned_to(y, 2) || (bias && !aligned_to(bias, 2))) return fail(DDL_E_ALIGN, "%s: y / bias misaligned", who);
@@ -624,9 +653,43 @@ extern "C" int ddl_linear(const void* x, const void* w, const void* bias, void* 
     return ddl_gemm(x, ldx, 1, w, ldw, 1, bias, y, dtype, ldy, M, N, K, stream);
 }
 
+namespace ddl {
+namespace {
+
+int gemm(const void* a, int64_t a_row_stride, int64_t a_k_stride, const void* b, int64_t b_row_stride, int64_t b_k_stride, const void* bias,
+         void* y, int dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, float* workspace, int64_t workspace_elems, bool anywhere,
+         void* stream) {
+    if (workspace && !aligned_to(workspace, 16)) return fail(DDL_E_ALIGN, "gemm: workspace must be 16-byte aligned");
+    if (dtype == DDL_DT_F32)
+        return gemm_f32(static_cast<const float*>(a), a_row_stride, a_k_stride, static_cast<const float*>(b), b_row_stride, b_k_stride,
+                        static_cast<const float*>(bias), static_cast<float*>(y), ldy, M, N, K, workspace, workspace_elems, stream);
+    if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return fail(DDL_E_UNSUPP, "gemm: dtype %d (bf16, f16 and f32 only)", dtype);
+    const Operand16 oa{static_cast<const uint16_t*>(a), a_row_stride, a_k_stride};
+    const Operand16 ob{static_cast<const uint16_t*>(b), b_row_stride, b_k_stride};
+    return gemm16("gemm", dtype == DDL_DT_F16, oa, ob, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K, workspace,
+                  workspace ? workspace_elems : 0, anywhere, stream);
+}
+
+}  // namespace
+}  // namespace ddl
+
 extern "C" int ddl_gemm(const void* a, int64_t a_row_stride, int64_t a_k_stride, const void* b, int64_t b_row_stride, int64_t b_k_stride,
                         const void* bias, void* y, int dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, void* stream) {
-    return ddl_gemm_ws(a, a_row_stride, a_k_stride, b, b_row_stride, b_k_stride, bias, y, dtype, ldy, M, N, K, nullptr, 0, stream);
+    return ddl::gemm(a, a_row_stride, a_k_stride, b, b_row_stride, b_k_stride, bias, y, dtype, ldy, M, N, K, nullptr, 0, false, stream);
+}
+
+extern "C" int ddl_gemm_in_place(int dtype, int aligned, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride, int64_t b_k_stride,
+                                 int64_t M, int64_t N, int64_t K) {
+    using namespace ddl;
+    if (dtype == DDL_DT_F32) return 1;
+    if (M <= 0 || N <= 0 || K <= 0 || (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16)) return 0;
+    const Operand16 a{nullptr, a_row_stride, a_k_stride}, b{nullptr, b_row_stride, b_k_stride};
+    // a null pointer is aligned: what is left to check are the sizes
+    if (aligned && pitches_ok(a, M, K) && pitches_ok(b, N, K))
+        return check_operand("gemm", "a", a, M, K) == 0 && check_operand("gemm", "b", b, N, K) == 0;
+    int dev = 0;
+    const int cus = compute_units(dev);
+    return plan_anywhere(a, b, M, N, K, cus, INT64_MAX).kind != Small16::kNone;
 }
 
 extern "C" int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride, int64_t b_k_stride,
@@ -638,20 +701,13 @@ extern "C" int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a
     if (dtype == DDL_DT_F32) return plan32(true, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, INT64_MAX).workspace;
     if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return 0;
     const Operand16 a{nullptr, a_row_stride, a_k_stride}, b{nullptr, b_row_stride, b_k_stride};
-    return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;
+    if (pitches_ok(a, M, K) && pitches_ok(b, N, K)) return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;
+    return plan_anywhere(a, b, M, N, K, cus, INT64_MAX).workspace;
 }
 
 extern "C" int ddl_gemm_ws(const void* a, int64_t a_row_stride, int64_t a_k_stride, const void* b, int64_t b_row_stride, int64_t b_k_stride,
                            const void* bias, void* y, int dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, float* workspace,
                            int64_t workspace_elems, void* stream) {
-    using namespace ddl;
-    if (workspace && !aligned_to(workspace, 16)) return fail(DDL_E_ALIGN, "gemm: workspace must be 16-byte aligned");
-    if (dtype == DDL_DT_F32)
-        return gemm_f32(static_cast<const float*>(a), a_row_stride, a_k_stride, static_cast<const float*>(b), b_row_stride, b_k_stride,
-                        static_cast<const float*>(bias), static_cast<float*>(y), ldy, M, N, K, workspace, workspace_elems, stream);
-    if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return fail(DDL_E_UNSUPP, "gemm: dtype %d (bf16, f16 and f32 only)", dtype);
-    const Operand16 oa{static_cast<const uint16_t*>(a), a_row_stride, a_k_stride};
-    const Operand16 ob{static_cast<const uint16_t*>(b), b_row_stride, b_k_stride};
-    return gemm16("gemm", dtype == DDL_DT_F16, oa, ob, static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K, workspace,
-                  workspace ? workspace_elems : 0, stream);
+    return ddl::gemm(a, a_row_stride, a_k_stride, b, b_row_stride, b_k_stride, bias, y, dtype, ldy, M, N, K, workspace, workspace_elems, true,
+                     stream);
 }

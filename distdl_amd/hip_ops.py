@@ -761,6 +761,13 @@ def _gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k):
     return _lib.load().ddl_gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k)
 
 
+@functools.lru_cache(maxsize=4096)
+def _gemm_in_place(dt, aligned, a_row, a_k, b_row, b_k, m, n, k):
+    """Does the product read operands of these sizes and strides (and alignment) where they lie?  (A function of its
+    arguments alone.)"""
+    return bool(_lib.load().ddl_gemm_in_place(dt, aligned, a_row, a_k, b_row, b_k, m, n, k))
+
+
 def _gemm(a, a_row, a_k, b, b_row, b_k, bias, out, dt, m, n, k):
     """``out[m, n] = sum_k a b + bias`` on operands addressed by two strides each; ``out`` is contiguous."""
     elems = _gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k)
@@ -774,8 +781,9 @@ def linear(x, weight, bias=None, out=None):
     """y = x @ weight.T + bias with fp32 accumulation; operands and result
     bfloat16, float16 or float32 (all the same).  The 16-bit kernel wants the
     reduction length and the row pitches to be multiples of 8 and 16-byte
-    aligned operands; operands that are not are copied into zero-padded
-    temporaries first (zeros add nothing to the sums)."""
+    aligned operands; of operands that are not, small products are read as they
+    are by a kernel of their own, and those of large ones are copied into
+    zero-padded temporaries first (zeros add nothing to the sums)."""
     _require_gpu(x, weight, bias)
     dt = _LINEAR_DTYPES.get(x.dtype)
     if dt is None or weight.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
@@ -804,7 +812,9 @@ def linear(x, weight, bias=None, out=None):
     if dt != _lib.DDL_DT_F32:
         def fits(t, rows):
             return k % 8 == 0 and t.data_ptr() % 16 == 0 and (rows <= 1 or t.stride(0) % 8 == 0)
-        if not (fits(x2, m) and fits(weight, n)):
+        if not (fits(x2, m) and fits(weight, n)) and not _gemm_in_place(
+                dt, x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0, x2.stride(0) if m > 1 else k, 1,
+                weight.stride(0) if n > 1 else k, 1, m, n, k):
             k8 = _round_up(k, 8)
             x2, weight, k = _padded_k(x2, k8), _padded_k(weight, k8), k8
     _gemm(x2, x2.stride(0) if m > 1 else k, 1, weight, weight.stride(0) if n > 1 else k, 1, bias, out, dt, m, n, k)
@@ -877,8 +887,8 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
     (entries not asked for are None).  Both products read their operands where
     they lie: the float32 one through strides, the 16-bit one through
     transposing LDS reads, which need row counts and pitches that are multiples
-    of 8; 16-bit operands that do not qualify are transposed into temporaries
-    whose row pitch is padded to a multiple of 8 with zeros, and the forward
+    of 8 (small products: any); 16-bit operands that do not qualify are transposed
+    into temporaries whose row pitch is padded to a multiple of 8 with zeros, and the forward
     kernel runs on those."""
     _require_gpu(x, weight, grad_output)
     dt = _LINEAR_DTYPES.get(x.dtype)
@@ -907,9 +917,15 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
             return dx, dw, db
         direct = True
     else:
-        direct = (bool(m and n and k) and
-                  (not need_input or (_along_k_ok(dy, ld_dy, n) and _along_rows_ok(weight, ld_w, k, n))) and
-                  (not need_weight or (_along_rows_ok(dy, ld_dy, n, m) and _along_rows_ok(x2, ld_x, k, m))))
+        whole = bool(m and n and k)
+
+        def aligned(a, b):
+            return a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
+        dx_direct = need_input and whole and ((_along_k_ok(dy, ld_dy, n) and _along_rows_ok(weight, ld_w, k, n)) or
+                                              _gemm_in_place(dt, aligned(dy, weight), ld_dy, 1, 1, ld_w, m, k, n))
+        dw_direct = need_weight and whole and ((_along_rows_ok(dy, ld_dy, n, m) and _along_rows_ok(x2, ld_x, k, m)) or
+                                               _gemm_in_place(dt, aligned(dy, x2), 1, ld_dy, 1, ld_x, n, k, m))
+        direct = whole and dx_direct == bool(need_input) and dw_direct == bool(need_weight)
     if direct:      # every operand is read where it lies: one call for all that is wanted
         if need_input:
             dx = torch.empty(x.shape, dtype=x.dtype, device=x.device)
@@ -925,7 +941,7 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
         return dx, dw, db
     if need_input:
         # dx[m, j] = sum_n dy[m, n] w[n, j]: dy is read along n, w down its columns
-        if m and n and k and _along_k_ok(dy, ld_dy, n) and _along_rows_ok(weight, ld_w, k, n):
+        if dx_direct:
             dx = torch.empty((m, k), dtype=x.dtype, device=x.device)
             _gemm(dy, ld_dy, 1, weight, 1, ld_w, None, dx, dt, m, k, n)
             dx = dx.reshape(x.shape)
@@ -938,7 +954,7 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
             dx = _linear_padded(dy_p, w_t, m, k, np8, dt).reshape(x.shape)
     if need_weight:
         # dw[i, j] = sum_m dy[m, i] x[m, j]: both operands are read down their columns
-        if m and n and k and _along_rows_ok(dy, ld_dy, n, m) and _along_rows_ok(x2, ld_x, k, m):
+        if dw_direct:
             dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
             _gemm(dy, 1, ld_dy, x2, 1, ld_x, None, dw, dt, n, k, m)
         else:   # operands dyT[N, M] and xT[K, M], padded

@@ -1606,6 +1606,42 @@ def test_gemm_16_bit_products_that_leave_the_chip_idle(ops, dtype, a_t, b_t, M, 
         assert (got[:, N:] == 77.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K,pad", [
+    # every operand shape whose pitch, length or address is no multiple of eight: one k-tile that straddles K, whole k-tiles, an
+    # odd number of them, a reduction split over workgroups; tiles that straddle M and N by one and by seven
+    (8, 8, 1, 0), (9, 11, 3, 1), (65, 63, 65, 0), (71, 137, 640, 3), (201, 263, 1033, 0), (1030, 1023, 127, 0), (15, 66, 8191, 2)])
+def test_gemm_16_bit_operands_at_any_pitch(ops, dtype, a_t, b_t, M, N, K, pad):
+    """The kernel for unaligned 16-bit operands on integers (every sum is exact), read where they lie and against the
+    refusal of the aligned entry point; the operands end where their buffers end."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(M * 7 + N * 3 + K + 2 * a_t + b_t)
+    a = torch.randint(-1, 2, (M, K), generator=gen).to(dtype)
+    b = torch.randint(-1, 2, (N, K), generator=gen).to(dtype)
+    b = b * (torch.rand(N, K, generator=gen) < min(1.0, 64.0 / K)).to(dtype)
+    bias = torch.randint(-3, 4, (N,), generator=gen).to(dtype)
+    ag, a_rs, a_ks = _gemm_operand(a, a_t, pad)
+    bg, b_rs, b_ks = _gemm_operand(b, b_t, pad)
+    shift_a = torch.empty(ag.numel() + 1, dtype=dtype, device="cuda")      # the same operand one element further on
+    shift_a[1:] = ag.reshape(-1)
+    lib, dt, stream = _lib.load(), _lib.DDL_DT_BF16 if dtype == torch.bfloat16 else _lib.DDL_DT_F16, torch.cuda.current_stream().cuda_stream
+    want = a.double() @ b.double().T + bias.double()
+    assert want.abs().max() <= 256
+    elems = max(1 << 20, lib.ddl_gemm_workspace(dt, a_rs, a_ks, b_rs, b_ks, M, N, K))
+    assert lib.ddl_gemm_in_place(dt, 0, a_rs, a_ks, b_rs, b_ks, M, N, K) == 1
+    work, ldy = torch.full((elems,), float("nan"), device="cuda"), N + 3
+    for ptr in (ag.data_ptr(), shift_a.data_ptr() + 2):
+        out = torch.full((M, ldy), 77.0, dtype=dtype, device="cuda")
+        args = (ptr, a_rs, a_ks, bg.data_ptr(), b_rs, b_ks, bias.cuda().data_ptr(), out.data_ptr(), dt, ldy, M, N, K)
+        if ptr % 16:
+            assert lib.ddl_gemm(*args, stream) == -3
+        _lib.check(lib.ddl_gemm_ws(*args, work.data_ptr(), elems, stream), "ddl_gemm_ws")
+        got = out.cpu().double()
+        assert torch.equal(got[:, :N], want)
+        assert (got[:, N:] == 77.0).all()
+
+
 @pytest.mark.parametrize("a_t,b_t", [(False, True), (True, True)])
 def test_gemm_16_bit_random_within_tolerance_and_ragged_depth(ops, a_t, b_t):
     """Random operands, a reduction length that is no multiple of the k-tile
