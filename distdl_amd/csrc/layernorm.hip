@@ -18,9 +18,9 @@
 //   workgroup rows  up to 16384 columns: a 256-thread workgroup owns a row, still
 //                   in registers (up to 16 pieces of four per thread), sums go
 //                   through the wavefronts and four words of LDS
-//   streamed rows   anything longer, or rows whose length, pitch or address
-//                   rule out four-element accesses: a workgroup walks the row
-//                   once per reduction
+//   streamed rows   anything longer: a workgroup walks the row once per reduction
+// Rows whose length, pitch or address are no multiples of four elements are held in
+// the same way; only the end of such a row is fetched element by element.
 #include "ddl_common.h"
 
 #include "ln_elements.h"
@@ -43,6 +43,12 @@ __device__ inline float sum4(float4 v) { return (v.x + v.y) + (v.z + v.w); }
 __device__ inline float sq4(float4 v, float m) {
     const float a = v.x - m, b = v.y - m, c = v.z - m, d = v.w - m;
     return (a * a + b * b) + (c * c + d * d);
+}
+template <bool ANY>
+__device__ inline float sq_piece(float4 v, float m, int n) {   // of the first n elements
+    if (!ANY || n >= 4) return sq4(v, m);
+    const float a = v.x - m, b = n > 1 ? v.y - m : 0.f, c = n > 2 ? v.z - m : 0.f;
+    return (a * a + b * b) + c * c;
 }
 __device__ inline float4 norm4(float4 v, float mean, float rstd) {
     return make_float4((v.x - mean) * rstd, (v.y - mean) * rstd, (v.z - mean) * rstd, (v.w - mean) * rstd);
@@ -122,9 +128,9 @@ struct LnArgs {
 
 // --------------------------------------------------------- wavefront rows --
 
-// One wavefront per row, NV pieces of four per lane (cols <= 256 NV, cols % 4
-// == 0), RPW rows of a wavefront in flight at once.
-template <typename T, int NV, int RPW, int MODE, bool AFFINE>
+// One wavefront per row, NV pieces of four per lane (cols <= 256 NV), RPW rows of a
+// wavefront in flight at once.  ANY: rows of any length, pitch and address.
+template <typename T, int NV, int RPW, int MODE, bool AFFINE, bool ANY>
 __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int64_t rows_first, int64_t ld_first, int cols_first,
                                                        const LnArgs a_rest, const PartCounts pc) {
     // The leading arguments repeat four fields of the block that follows: plain
@@ -139,15 +145,15 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
     const int64_t wave = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + threadIdx.x / kWave;
     const int64_t r0 = wave * RPW;
     const int64_t rows = a.rows;
-    const int nv = a.cols >> 2;
+    const int nv = (a.cols + 3) >> 2;
     float4 g[NV], b[NV];
     if (MODE != kStats && AFFINE) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int c = lane + k * kWave;
             if (c < nv) {
-                g[k] = load4(static_cast<const T*>(a.gamma) + 4 * c);
-                b[k] = load4(static_cast<const T*>(a.beta) + 4 * c);
+                g[k] = load_piece<ANY>(static_cast<const T*>(a.gamma) + 4 * c, a.cols - 4 * c);
+                b[k] = load_piece<ANY>(static_cast<const T*>(a.beta) + 4 * c, a.cols - 4 * c);
             }
         }
     }
@@ -171,7 +177,7 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int c = lane + k * kWave;
-            v[i][k] = (r < rows && c < nv) ? load4(x + r * a.ld + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[i][k] = (r < rows && c < nv) ? load_piece<ANY>(x + r * a.ld + 4 * c, a.cols - 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
     const float inv = 1.0f / static_cast<float>(a.cols);
@@ -190,7 +196,7 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
             float q = 0.f;
 #pragma unroll
             for (int k = 0; k < NV; ++k)
-                if (lane + k * kWave < nv) q += sq4(v[i][k], mean);
+                if (lane + k * kWave < nv) q += sq_piece<ANY>(v[i][k], mean, a.cols - 4 * (lane + k * kWave));
             q = wave_sum(q);
             if (MODE == kStats || MODE == kJoined) {
                 if (lane == 0) reinterpret_cast<float2*>(a.stats)[r] = make_float2(mean, q);
@@ -212,7 +218,7 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
             if (c < nv) {
                 float4 o = norm4(v[i][k], mean, rstd);
                 if (AFFINE) o = affine4(g[k], o, b[k]);
-                store4(y + r * a.ldy + 4 * c, o);
+                store_piece<ANY>(y + r * a.ldy + 4 * c, o, a.cols - 4 * c);
             }
         }
     }
@@ -220,15 +226,15 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
 
 // --------------------------------------------------------- workgroup rows --
 
-// One workgroup per row, NV pieces of four per thread (cols <= 1024 NV, cols
-// % 4 == 0); the grid walks the rows.
-template <typename T, int NV, int MODE, bool AFFINE>
+// One workgroup per row, NV pieces of four per thread (cols <= 1024 NV); the grid
+// walks the rows.  ANY as above.
+template <typename T, int NV, int MODE, bool AFFINE, bool ANY>
 __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const PartCounts pc) {
     __shared__ float scratch[kWavesPerBlock];
     const T* __restrict__ x = static_cast<const T*>(a.x);
     T* __restrict__ y = static_cast<T*>(a.y);
     const int t = threadIdx.x, lane = t & (kWave - 1);
-    const int nv = a.cols >> 2;
+    const int nv = (a.cols + 3) >> 2;
     const float inv = 1.0f / static_cast<float>(a.cols);
     for (int64_t r = blockIdx.x; r < a.rows; r += gridDim.x) {
         float2 first = make_float2(0.f, 0.f);
@@ -237,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const Pa
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int c = t + k * kBlock;
-            v[k] = c < nv ? load4(x + r * a.ld + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[k] = c < nv ? load_piece<ANY>(x + r * a.ld + 4 * c, a.cols - 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         float mean, rstd;
         if (MODE == kNorm) {
@@ -252,7 +258,7 @@ __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const Pa
             float q = 0.f;
 #pragma unroll
             for (int k = 0; k < NV; ++k)
-                if (t + k * kBlock < nv) q += sq4(v[k], mean);
+                if (t + k * kBlock < nv) q += sq_piece<ANY>(v[k], mean, a.cols - 4 * (t + k * kBlock));
             q = block_sum(q, scratch);
             if (MODE == kStats || MODE == kJoined) {
                 if (t == 0) reinterpret_cast<float2*>(a.stats)[r] = make_float2(mean, q);
@@ -273,8 +279,9 @@ __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const Pa
             const int c = t + k * kBlock;
             if (c < nv) {
                 float4 o = norm4(v[k], mean, rstd);
-                if (AFFINE) o = affine4(load4(static_cast<const T*>(a.gamma) + 4 * c), o, load4(static_cast<const T*>(a.beta) + 4 * c));
-                store4(y + r * a.ldy + 4 * c, o);
+                if (AFFINE) o = affine4(load_piece<ANY>(static_cast<const T*>(a.gamma) + 4 * c, a.cols - 4 * c), o,
+                                        load_piece<ANY>(static_cast<const T*>(a.beta) + 4 * c, a.cols - 4 * c));
+                store_piece<ANY>(y + r * a.ldy + 4 * c, o, a.cols - 4 * c);
             }
         }
     }
@@ -353,43 +360,52 @@ __global__ __launch_bounds__(kBlock) void ln_stream_rows(const LnArgs a, const P
 // rows per wavefront stream a long input a little faster.
 constexpr int64_t kSmallRows = 65536;
 
-template <typename T, int MODE, bool AFFINE, int NV, int RPW>
+template <typename T, int MODE, bool AFFINE, bool ANY, int NV, int RPW>
 void launch_wave_rpw(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     const int64_t waves = (a.rows + RPW - 1) / RPW;
     const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
-    hipLaunchKernelGGL((ln_wave_rows<T, NV, RPW, MODE, AFFINE>), dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0, s, a.x, a.rows, a.ld,
+    hipLaunchKernelGGL((ln_wave_rows<T, NV, RPW, MODE, AFFINE, ANY>), dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0, s, a.x, a.rows, a.ld,
                        a.cols, a, pc);
 }
 
-template <typename T, int MODE, bool AFFINE, int NV>
+template <typename T, int MODE, bool AFFINE, bool ANY, int NV>
 void launch_wave(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     if (NV <= 2 && a.rows > kSmallRows)
-        launch_wave_rpw<T, MODE, AFFINE, NV, 2>(a, pc, s);
+        launch_wave_rpw<T, MODE, AFFINE, ANY, NV, 2>(a, pc, s);
     else
-        launch_wave_rpw<T, MODE, AFFINE, NV, 1>(a, pc, s);
+        launch_wave_rpw<T, MODE, AFFINE, ANY, NV, 1>(a, pc, s);
 }
 
-template <typename T, int MODE, bool AFFINE, int NV>
+template <typename T, int MODE, bool AFFINE, bool ANY, int NV>
 void launch_block(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     const uint32_t blocks = static_cast<uint32_t>(a.rows < (1 << 20) ? a.rows : (1 << 20));
-    hipLaunchKernelGGL((ln_block_rows<T, NV, MODE, AFFINE>), dim3(blocks), dim3(kBlock), 0, s, a, pc);
+    hipLaunchKernelGGL((ln_block_rows<T, NV, MODE, AFFINE, ANY>), dim3(blocks), dim3(kBlock), 0, s, a, pc);
+}
+
+// Rows of up to kBlockRowCols columns, held in registers.
+template <typename T, int MODE, bool AFFINE, bool ANY>
+int launch_held(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
+    const int cols = a.cols;
+    if (cols <= kWaveRowCols) {
+        if (cols <= 256) launch_wave<T, MODE, AFFINE, ANY, 1>(a, pc, s);
+        else if (cols <= 512) launch_wave<T, MODE, AFFINE, ANY, 2>(a, pc, s);
+        else if (cols <= 1024) launch_wave<T, MODE, AFFINE, ANY, 4>(a, pc, s);
+        else launch_wave<T, MODE, AFFINE, ANY, 8>(a, pc, s);
+        return check_launch("ln_wave_rows");
+    }
+    if (cols <= 4096) launch_block<T, MODE, AFFINE, ANY, 4>(a, pc, s);
+    else if (cols <= 8192) launch_block<T, MODE, AFFINE, ANY, 8>(a, pc, s);
+    else launch_block<T, MODE, AFFINE, ANY, 16>(a, pc, s);
+    return check_launch("ln_block_rows");
 }
 
 template <typename T, int MODE, bool AFFINE>
 int launch_typed(const LnArgs& a, const PartCounts& pc, bool vec, hipStream_t s) {
     const int cols = a.cols;
-    if (vec && cols <= kWaveRowCols) {
-        if (cols <= 256) launch_wave<T, MODE, AFFINE, 1>(a, pc, s);
-        else if (cols <= 512) launch_wave<T, MODE, AFFINE, 2>(a, pc, s);
-        else if (cols <= 1024) launch_wave<T, MODE, AFFINE, 4>(a, pc, s);
-        else launch_wave<T, MODE, AFFINE, 8>(a, pc, s);
-        return check_launch("ln_wave_rows");
-    }
-    if (vec && cols <= kBlockRowCols) {
-        if (cols <= 4096) launch_block<T, MODE, AFFINE, 4>(a, pc, s);
-        else if (cols <= 8192) launch_block<T, MODE, AFFINE, 8>(a, pc, s);
-        else launch_block<T, MODE, AFFINE, 16>(a, pc, s);
-        return check_launch("ln_block_rows");
+    if (vec && cols <= kBlockRowCols) return launch_held<T, MODE, AFFINE, false>(a, pc, s);
+    if constexpr (MODE != kJoined) {
+        // Rows that start at any element: held as well, instead of read element by element once per reduction.
+        if (cols <= kBlockRowCols) return launch_held<T, MODE, AFFINE, true>(a, pc, s);
     }
     if constexpr (MODE == kJoined) {
         return fail(DDL_E_UNSUPP, "ln stats+normalize: rows of more than %d columns take the two-launch form", kBlockRowCols);

@@ -4,6 +4,7 @@
 #define DDL_LN_ELEMENTS_H
 #include "ddl_common.h"
 #include <hip/hip_fp16.h>
+#include <type_traits>
 
 namespace ddl {
 
@@ -80,6 +81,51 @@ __device__ inline float load1(const __half* p) { return __half2float(*p); }
 __device__ inline void store1(float* p, float v) { *p = v; }
 __device__ inline void store1(bf16_t* p, float v) { p->bits = static_cast<uint16_t>(f32_to_bf16(v)); }
 __device__ inline void store1(__half* p, float v) { *p = __float2half_rn(v); }
+
+// Up to four elements at any address: a piece of a row whose length, pitch or
+// start is no multiple of four elements.  Whole pieces are one load or store
+// (global memory takes them at element alignment), the last n < 4 elements of a
+// row one by one; elements past n read as zeros.
+template <typename T>
+struct PieceBits {
+    typedef std::conditional_t<sizeof(T) == 4, float4, uint2> raw;
+    struct __attribute__((packed, aligned(sizeof(T)))) Any {
+        uint32_t word[sizeof(T)];   // four elements
+    };
+};
+template <bool ANY, typename T>
+__device__ inline float4 load_piece(const T* p, int n) {
+    if (!ANY) return load4(p);
+    if (n >= 4) {
+        typename PieceBits<T>::raw r;
+        const typename PieceBits<T>::Any a = *reinterpret_cast<const typename PieceBits<T>::Any*>(p);
+        __builtin_memcpy(&r, &a, sizeof(r));
+        return load4(reinterpret_cast<const T*>(&r));
+    }
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (n > 0) v.x = load1(p);
+    if (n > 1) v.y = load1(p + 1);
+    if (n > 2) v.z = load1(p + 2);
+    return v;
+}
+template <bool ANY, typename T>
+__device__ inline void store_piece(T* p, float4 v, int n) {
+    if (!ANY) {
+        store4(p, v);
+        return;
+    }
+    if (n >= 4) {
+        T e[4];
+        store1(e, v.x), store1(e + 1, v.y), store1(e + 2, v.z), store1(e + 3, v.w);
+        typename PieceBits<T>::Any a;
+        __builtin_memcpy(&a, e, sizeof(a));
+        *reinterpret_cast<typename PieceBits<T>::Any*>(p) = a;
+        return;
+    }
+    if (n > 0) store1(p, v.x);
+    if (n > 1) store1(p + 1, v.y);
+    if (n > 2) store1(p + 2, v.z);
+}
 
 // Calls fn(T{}) with the element type that `dtype` names; false for any other dtype.
 template <typename Fn>

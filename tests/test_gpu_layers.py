@@ -503,6 +503,38 @@ def test_layer_norm_backward_of_whole_rows_in_one_pass(ops, rows, cols, dtype):
     assert dg5 is None and db5 is None and torch.equal(dx5, dx)
 
 
+@pytest.mark.parametrize("cols", [1, 2, 3, 5, 255, 257, 511, 514, 1023, 1027, 2047, 2049, 4095, 4098, 8191, 8193, 16383, 16385])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_layer_norm_rows_of_any_length_and_address(ops, dtype, cols):
+    """Rows that are no multiple of four elements, whole and split over two workers, at the widths where the kernel's shape
+    changes: rows with an odd pitch that start one element into their buffer and end where it ends, whose neighbours hold
+    NaN, against float64; what lies between the rows of the output stays untouched."""
+    rows, pad = 7, 3
+    gen = torch.Generator().manual_seed(cols)
+    x = (torch.randn(rows, cols, generator=gen) * 2 + 0.5).to(dtype)
+    gamma = (1 + 0.1 * torch.randn(cols, generator=gen)).to(dtype)
+    beta = (0.1 * torch.randn(cols, generator=gen)).to(dtype)
+    store = torch.full((1 + rows * (cols + pad) - pad,), float("nan"), dtype=dtype, device="cuda")
+    xg = store[1:].as_strided((rows, cols), (cols + pad, 1), 1)
+    xg.copy_(x)
+    shifted = [torch.empty(cols + 1, dtype=dtype, device="cuda")[1:].copy_(t) for t in (gamma, beta)]
+    y, mean, rstd = ops.layer_norm(xg, *shifted, 1e-3, want_stats=True)
+    stats = ops.ln_partial_stats(xg)
+    other = torch.stack([torch.full((rows,), 0.25), torch.full((rows,), 3.0)], dim=1).cuda()
+    y2 = ops.ln_normalize_affine(xg, torch.stack([stats, other]).contiguous(), [cols, 5], *shifted, 1e-3)
+    x64 = x.double()
+    m, q = x64.mean(1), ((x64 - x64.mean(1, keepdim=True)) ** 2).sum(1)
+    ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+
+    def check(got, want, size):     # one rounding of the result and a few units of fp32 sums
+        assert bool(((got.cpu().double() - want).abs() <= ulp * want.abs() + 4e-6 * size).all())
+    assert bool(((stats.cpu().double()[:, 0] - m).abs() <= 4e-6 * 4).all()) and bool(((stats.cpu().double()[:, 1] - q).abs() <= 4e-6 * (q + 4)).all())
+    check(y, (x64 - m[:, None]) / (q / cols + 1e-3).sqrt()[:, None] * gamma.double() + beta.double(), 8.0 * (1 + float((q / cols + 1e-3).rsqrt().max())))
+    m2 = (m + 0.25) / 2
+    v2 = (q / cols + (m - m2) ** 2 + 3.0 / 5 + (0.25 - m2) ** 2) / 2
+    check(y2, (x64 - m2[:, None]) / (v2 + 1e-3).sqrt()[:, None] * gamma.double() + beta.double(), 8.0)
+
+
 @pytest.mark.parametrize("rows,cols,pad", [(1, 1028, 0), (5, 1025, 0), (37, 2048, 4), (3, 2052, 0), (66, 4096, 1), (1029, 4097, 0),
                                            (9, 8192, 0), (7, 8191, 0), (6, 8196, 0), (10, 16384, 8), (8200, 1032, 0)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
