@@ -281,8 +281,8 @@ struct DxArgs {
 // partial has the layout of ln_bwd_params_partial.  WITH_DX: the sums of the
 // whole row are complete once this worker's are (it holds the row whole, or the
 // other workers' pairs are in memory), so dx is written in the same pass, from
-// the registers that hold the row.
-template <typename T, int NV, bool WITH_DX>
+// the registers that hold the row.  ANY: rows of any length, pitch and address.
+template <typename T, int NV, bool WITH_DX, bool ANY>
 __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows,
                                                               int64_t cols, int64_t ld_dy, int64_t ld_x,
                                                               const float* __restrict__ mean, const float* __restrict__ rstd,
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
 #pragma clang fp contract(off)   // both instantiations round alike: sums, column sums and dx do not depend on WITH_DX
     __shared__ float fold[2][kFusedWaves][NV * kWave * 4];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int nv = static_cast<int>(cols >> 2);
+    const int nv = static_cast<int>((cols + 3) >> 2), n = static_cast<int>(cols);
     const int64_t r_begin = static_cast<int64_t>(blockIdx.x) * rows_per_split;
     const int64_t r_end = r_begin + rows_per_split < rows ? r_begin + rows_per_split : rows;
     float4 g[NV], ca[NV], cb[NV];
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
     for (int k = 0; k < NV; ++k) {
         const int c = lane + k * kWave;
         g[k] = make_float4(1.f, 1.f, 1.f, 1.f);
-        if (gamma && c < nv) g[k] = load4(gamma + 4 * c);
+        if (gamma && c < nv) g[k] = load_piece<ANY>(gamma + 4 * c, n - 4 * c);
         ca[k] = cb[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     constexpr int RU = NV <= 2 ? 4 : 2;   // rows whose loads are in flight together
@@ -321,8 +321,8 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
                 const int c = lane + k * kWave;
                 d[u][k] = v[u][k] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (on && c < nv) {
-                    d[u][k] = load4(dy + r * ld_dy + 4 * c);
-                    v[u][k] = load4(x + r * ld_x + 4 * c);
+                    d[u][k] = load_piece<ANY>(dy + r * ld_dy + 4 * c, n - 4 * c);
+                    v[u][k] = load_piece<ANY>(x + r * ld_x + 4 * c, n - 4 * c);
                 }
             }
         }
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
                     o.y = dx_value(dd.y, g[k].y, vv.y, m[u], rs[u], S1, S2);
                     o.z = dx_value(dd.z, g[k].z, vv.z, m[u], rs[u], S1, S2);
                     o.w = dx_value(dd.w, g[k].w, vv.w, m[u], rs[u], S1, S2);
-                    store4(dxr + 4 * c, o);
+                    store_piece<ANY>(dxr + 4 * c, o, n - 4 * c);
                 }
             }
         }
@@ -380,6 +380,25 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
         for (int w = 0; w < kFusedWaves; ++w) t += fold[which][w][c];
         partial[(static_cast<int64_t>(blockIdx.x) * 2 + which) * cols + c] = t;
     }
+}
+
+// Unaligned rows of fewer columns stay with the separate passes: [30000, 801] bf16 107 -> 71 us in one pass, [8192, 1023]
+// fp32 49 -> 27, but [2048, 333] 10.4 -> 14 and [100000, 63] bf16 68 -> 92 (few lanes have a piece, and most rows' ends).
+constexpr int64_t kAnyCols = 512;
+
+template <typename T, bool WITH_DX, bool ANY>
+void launch_partial_cols(const T* dy, const T* x, int64_t rows, int64_t cols, int64_t ld_dy, int64_t ld_x, const float* mean, const float* rstd,
+                         const T* gamma, float* sums, int64_t splits, float* partial, const DxArgs& dxa, hipStream_t s) {
+    const int64_t rows_per_split = (rows + splits - 1) / splits;
+    auto go = [&](auto nv) {
+        hipLaunchKernelGGL((ln_bwd_partial_cols<T, decltype(nv)::value, WITH_DX, ANY>), dim3(static_cast<uint32_t>(splits)), dim3(kFusedBlock), 0, s, dy,
+                           x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, sums, rows_per_split, partial, dxa);
+    };
+    if constexpr (!ANY) {
+        if (cols <= kWave * 4) return go(std::integral_constant<int, 1>{});
+        if (cols <= 2 * kWave * 4) return go(std::integral_constant<int, 2>{});
+    }
+    go(std::integral_constant<int, 4>{});
 }
 
 // Rows that do not fit a wavefront's registers, or are no multiple of four
@@ -702,20 +721,17 @@ extern "C" int ddl_ln_bwd_partial_params(const void* dy, const void* x, int dtyp
         return fail(DDL_E_ALIGN, "ln backward sums: elements must be aligned to their size, fp32 arrays to 4 bytes, the sums to 8");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t rows_per_split = rows > 0 ? (rows + splits - 1) / splits : 1;
-    if (rows > 0 && cols <= 4 * kWave * 4 && vectorizable(elem, cols, {ld_dy, ld_x}, {dy, x, gamma})) {
-        const dim3 grid(static_cast<uint32_t>(splits));
+    const bool vec = vectorizable(elem, cols, {ld_dy, ld_x}, {dy, x, gamma});
+    if (rows > 0 && cols <= 4 * kWave * 4 && (vec || cols > kAnyCols)) {
         with_ln_element(dtype, [&](auto* tag) {
             using T = std::remove_pointer_t<decltype(tag)>;
-            if (cols <= kWave * 4)
-                hipLaunchKernelGGL((ln_bwd_partial_cols<T, 1, false>), grid, dim3(kFusedBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, rows_per_split, workspace, DxArgs{});
-            else if (cols <= 2 * kWave * 4)
-                hipLaunchKernelGGL((ln_bwd_partial_cols<T, 2, false>), grid, dim3(kFusedBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, rows_per_split, workspace, DxArgs{});
+            if (vec)
+                launch_partial_cols<T, false, false>(as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, splits, workspace, DxArgs{}, s);
             else
-                hipLaunchKernelGGL((ln_bwd_partial_cols<T, 4, false>), grid, dim3(kFusedBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, rows_per_split, workspace, DxArgs{});
+                launch_partial_cols<T, false, true>(as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, splits, workspace, DxArgs{}, s);
         });
         return check_launch("ln_bwd_partial_cols");
     }
-    const bool vec = vectorizable(elem, cols, {ld_dy, ld_x}, {dy, x, gamma});
     // One read of dy and x instead of two, where every CU gets a split: [8192, 8192] bf16 with the dx launch 187 -> 132 us,
     // but [1024, 8192] (32 splits) 43 -> 58 and rows of a few hundred elements 10.6 -> 24.
     if (splits == 256 && cols > 4 * kWave * 4 && cols <= block_rows_cols(vec)) {
@@ -801,18 +817,11 @@ extern "C" int ddl_ln_bwd_one_pass(const void* dy, const void* x, int dtype, int
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t strips = (dgamma || dbeta) ? (cols + kStrip - 1) / kStrip : 0;
     if (rows > 0) {
-        const int64_t rows_per_split = (rows + splits - 1) / splits;
         float* sums = part_sums ? part_sums + static_cast<int64_t>(my_part) * rows * 2 : nullptr;
         const DxArgs dxa{part_sums, nparts, my_part, weight, dx, ld_dx};
-        const dim3 grid(static_cast<uint32_t>(splits));
         with_ln_element(dtype, [&](auto* tag) {
             using T = std::remove_pointer_t<decltype(tag)>;
-            if (cols <= kWave * 4)
-                hipLaunchKernelGGL((ln_bwd_partial_cols<T, 1, true>), grid, dim3(kFusedBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, rows_per_split, workspace, dxa);
-            else if (cols <= 2 * kWave * 4)
-                hipLaunchKernelGGL((ln_bwd_partial_cols<T, 2, true>), grid, dim3(kFusedBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, rows_per_split, workspace, dxa);
-            else
-                hipLaunchKernelGGL((ln_bwd_partial_cols<T, 4, true>), grid, dim3(kFusedBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, rows_per_split, workspace, dxa);
+            launch_partial_cols<T, true, false>(as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, splits, workspace, dxa, s);
         });
         if (int rc = check_launch("ln_bwd_partial_cols")) return rc;
     }
@@ -834,11 +843,13 @@ extern "C" int ddl_ln_bwd_whole_rows(const void* dy, const void* x, int dtype, i
     if (int rc = check_rows("ln backward (whole rows)", rows, cols, ld_dy, ld_x)) return rc;
     if (ld_dx < cols) return fail(DDL_E_ARG, "ln backward (whole rows): ld_dx=%lld below cols=%lld", (long long)ld_dx, (long long)cols);
     const bool vec = vectorizable(elem, cols, {ld_dy, ld_x, ld_dx}, {dy, x, gamma, dx});
-    if (cols <= 4 * kWave * 4 || cols > block_rows_cols(vec))
-        return fail(DDL_E_UNSUPP, "ln backward (whole rows): rows of %d to %lld columns", 4 * kWave * 4 + 1, (long long)block_rows_cols(vec));
+    if (cols <= kAnyCols || cols > block_rows_cols(vec))
+        return fail(DDL_E_UNSUPP, "ln backward (whole rows): rows of %lld to %lld columns", (long long)kAnyCols + 1, (long long)block_rows_cols(vec));
     if (!workspace) return fail(DDL_E_ARG, "ln backward (whole rows): null workspace");
-    // Four rows per split already pay: a split's column sums are 8 bytes per column next to 4 rows x 3 tensors of elements.
-    const int64_t splits = param_splits(rows, cols, workspace_elems, 4);
+    // A workgroup per row: four rows per split already pay (a split's column sums are 8 bytes per column next to 4 rows x 3
+    // tensors of elements).  A wavefront per row: eight rows at once.
+    const bool by_wave = cols <= 4 * kWave * 4;
+    const int64_t splits = param_splits(rows, cols, workspace_elems, by_wave ? 32 : 4);
     if (splits < 1) return fail(DDL_E_ARG, "ln backward (whole rows): workspace of %lld floats is smaller than 2 x %lld", (long long)workspace_elems, (long long)cols);
     if (rows > 0 && (!dy || !x || !mean || !rstd || !dx)) return fail(DDL_E_ARG, "ln backward (whole rows): null pointer");
     if (!elems_aligned(elem, {dy, x, gamma, dx, dgamma, dbeta}) || !aligned_to(mean, 4) || !aligned_to(rstd, 4) || !aligned_to(workspace, 4))
@@ -847,8 +858,12 @@ extern "C" int ddl_ln_bwd_whole_rows(const void* dy, const void* x, int dtype, i
     if (rows > 0) {
         with_ln_element(dtype, [&](auto* tag) {
             using T = std::remove_pointer_t<decltype(tag)>;
-            launch_block_rows<T, true>(vec, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), nullptr, splits, workspace, weight,
-                                       as<T>(dx), ld_dx, s);
+            if (by_wave)
+                launch_partial_cols<T, true, true>(as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), nullptr, splits, workspace,
+                                                   DxArgs{nullptr, 1, 0, weight, dx, ld_dx}, s);
+            else
+                launch_block_rows<T, true>(vec, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), nullptr, splits, workspace,
+                                           weight, as<T>(dx), ld_dx, s);
         });
         if (int rc = check_launch("ln_bwd_block_rows")) return rc;
     }

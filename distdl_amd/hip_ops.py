@@ -632,12 +632,12 @@ def ln_backward_one_pass(dy2d, x2d, mean, rstd, gamma, weight, part_sums=None, m
 
 
 def ln_backward_whole_rows_supported(dy2d, x2d, gamma):
-    """Whether ``ln_backward_whole_rows`` takes these rows: 1025 to 8192
+    """Whether ``ln_backward_whole_rows`` takes these rows: 513 to 8192
     columns, or 16384 when columns and pitches are multiples of 4 and dy, x and
     gamma aligned to four elements."""
     rows, cols = x2d.shape
     if cols <= 8192:
-        return cols > 1024
+        return cols > 512
     quad = 4 * x2d.element_size()
     return (cols <= 16384 and cols % 4 == 0 and (rows <= 1 or (x2d.stride(0) % 4 == 0 and dy2d.stride(0) % 4 == 0)) and
             x2d.data_ptr() % quad == 0 and dy2d.data_ptr() % quad == 0 and (gamma is None or gamma.data_ptr() % quad == 0))
@@ -645,7 +645,7 @@ def ln_backward_whole_rows_supported(dy2d, x2d, gamma):
 
 def ln_backward_whole_rows(dy2d, x2d, mean, rstd, gamma, weight, want_gamma=True, want_beta=True):
     """dx and (dgamma, dbeta) in one pass over dy and x, for rows this worker
-    holds whole (a workgroup per row)."""
+    holds whole (of more than 1024 columns, or not aligned to four elements)."""
     _require_gpu(dy2d, x2d, mean, rstd, gamma)
     ld_dy, ld_x = _rows2d(dy2d, "ln_backward_whole_rows"), _rows2d(x2d, "ln_backward_whole_rows")
     rows, cols = x2d.shape

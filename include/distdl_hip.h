@@ -363,8 +363,8 @@ int ddl_ln_bwd_one_pass(const void* dy, const void* x, int dtype, int64_t rows,
                         void* dx, int64_t ld_dx, float* workspace,
                         int64_t workspace_elems, void* dgamma, void* dbeta,
                         void* stream);
-/* The same for longer rows a worker holds whole (any pitch): a workgroup per
- * row.  More than 1024 columns, at most 16384 when columns and
+/* The same for rows a worker holds whole that ddl_ln_bwd_one_pass does not take:
+ * longer ones, and any pitch.  More than 512 columns, at most 16384 when columns and
  * pitches are multiples of 4 and pointers aligned to 4 elements, 8192 otherwise
  * (else DDL_E_UNSUPP: take the two calls).
  * dgamma and dbeta may be NULL.  Uses up to 512 * cols floats of workspace. */

@@ -536,7 +536,8 @@ def test_layer_norm_rows_of_any_length_and_address(ops, dtype, cols):
 
 
 @pytest.mark.parametrize("rows,cols,pad", [(1, 1028, 0), (5, 1025, 0), (37, 2048, 4), (3, 2052, 0), (66, 4096, 1), (1029, 4097, 0),
-                                           (9, 8192, 0), (7, 8191, 0), (6, 8196, 0), (10, 16384, 8), (8200, 1032, 0)])
+                                           (9, 8192, 0), (7, 8191, 0), (6, 8196, 0), (10, 16384, 8), (8200, 1032, 0),
+                                           (1, 513, 0), (70, 514, 3), (65, 1023, 0), (300, 768, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_layer_norm_backward_of_long_whole_rows(ops, rows, cols, pad, dtype):
     """Rows a workgroup owns: dx, dgamma and dbeta in one pass against float64 autograd of the same inputs, at the widths
