@@ -253,16 +253,27 @@ __global__ __launch_bounds__(kOneBlock) void colsum_one_kernel(const typename El
     __syncthreads();
     constexpr int kParts = kOneBlock / kNarrow;   // threads per column
     const int col = t % kNarrow, part = t / kNarrow;
-    float s = 0.f;
+    // Sums of many partial sums go pairwise: added one after the other, 64 of them lose a third more to rounding in fp32 than
+    // the two stages do.
+    constexpr int kMine = kGroups / kParts;
+    float mine[kMine];
 #pragma unroll
-    for (int k = 0; k < kGroups / kParts; ++k) s += fold[part + k * kParts][col];
-    half[part][col] = s;
+    for (int k = 0; k < kMine; ++k) mine[k] = fold[part + k * kParts][col];
+#pragma unroll
+    for (int d = kMine / 2; d > 0; d /= 2)
+#pragma unroll
+        for (int k = 0; k < d; ++k) mine[k] += mine[k + d];
+    half[part][col] = mine[0];
     __syncthreads();
     if (t < kNarrow && static_cast<int64_t>(blockIdx.x) * kNarrow + t < cols) {
-        float r = 0.f;
+        float r[kParts];
 #pragma unroll
-        for (int k = 0; k < kParts; ++k) r += half[k][t];
-        Elem<DT>::store(out + static_cast<int64_t>(blockIdx.x) * kNarrow + t, r);
+        for (int k = 0; k < kParts; ++k) r[k] = half[k][t];
+#pragma unroll
+        for (int d = kParts / 2; d > 0; d /= 2)
+#pragma unroll
+            for (int k = 0; k < d; ++k) r[k] += r[k + d];
+        Elem<DT>::store(out + static_cast<int64_t>(blockIdx.x) * kNarrow + t, r[0]);
     }
 }
 
