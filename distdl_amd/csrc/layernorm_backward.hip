@@ -205,23 +205,44 @@ __device__ inline void ln_bwd_params_final_body(uint32_t block, const float* __r
     const int64_t c = static_cast<int64_t>(block) * kStrip + t;
     float a = 0.f, b = 0.f;
     if (c < cols) {
-        int k = g;
-        for (; k + (kInFlight - 1) * kWavesPerBlock < splits; k += kInFlight * kWavesPerBlock) {
-            float va[kInFlight], vb[kInFlight];
+        // Eight splits at a time, pairwise, whatever is in flight: a chain of 64 additions lost half as much again to rounding
+        // ([3000, 2048] fp32 in 256 splits), and both callers add in the same order.
+        auto fetch = [&](int k, float (&va)[8], float (&vb)[8]) {
 #pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
+            for (int u = 0; u < 8; ++u) {
                 va[u] = partial[(static_cast<int64_t>(k + u * kWavesPerBlock) * 2) * cols + c];
                 vb[u] = partial[(static_cast<int64_t>(k + u * kWavesPerBlock) * 2 + 1) * cols + c];
             }
+        };
+        auto eight = [](const float (&v)[8]) { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); };
+        constexpr int kEights = kInFlight / 8;
+        int k = g;
+        for (; k + (kInFlight - 1) * kWavesPerBlock < splits; k += kInFlight * kWavesPerBlock) {
+            float va[kEights][8], vb[kEights][8];
 #pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
-                a += va[u];
-                b += vb[u];
+            for (int e = 0; e < kEights; ++e) fetch(k + e * 8 * kWavesPerBlock, va[e], vb[e]);
+#pragma unroll
+            for (int e = 0; e < kEights; ++e) {
+                a += eight(va[e]);
+                b += eight(vb[e]);
             }
         }
-        for (; k < splits; k += kWavesPerBlock) {
-            a += partial[(static_cast<int64_t>(k) * 2) * cols + c];
-            b += partial[(static_cast<int64_t>(k) * 2 + 1) * cols + c];
+        for (; k + 7 * kWavesPerBlock < splits; k += 8 * kWavesPerBlock) {
+            float va[8], vb[8];
+            fetch(k, va, vb);
+            a += eight(va);
+            b += eight(vb);
+        }
+        if (k < splits) {   // the last one to seven
+            float va[8], vb[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int q = k + u * kWavesPerBlock;
+                va[u] = q < splits ? partial[(static_cast<int64_t>(q) * 2) * cols + c] : 0.f;
+                vb[u] = q < splits ? partial[(static_cast<int64_t>(q) * 2 + 1) * cols + c] : 0.f;
+            }
+            a += eight(va);
+            b += eight(vb);
         }
     }
     fold[0][g][t] = a;
@@ -229,9 +250,8 @@ __device__ inline void ln_bwd_params_final_body(uint32_t block, const float* __r
     __syncthreads();
     if (threadIdx.x < 2 * kStrip && c < cols) {
         const int which = threadIdx.x / kStrip;
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < kWavesPerBlock; ++k) s += fold[which][k][t];
+        static_assert(kWavesPerBlock == 4, "four lane groups");
+        const float s = (fold[which][0][t] + fold[which][1][t]) + (fold[which][2][t] + fold[which][3][t]);
         T* out = which == 0 ? dgamma : dbeta;
         if (out) store1(out + c, s);
     }
