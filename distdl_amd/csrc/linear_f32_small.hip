@@ -284,8 +284,8 @@ int launch_shape(const char* who, const Small32& plan, const Part32& part, float
 // round of one k-tile for every group) 0.68 for a lone 64 x 64 tile, 0.52 for each that a CU has to work through, 0.78 in
 // two or four groups + the epilogue of every further tile + for splits a second launch (2.3, and 5 for
 // what it and the workspace cost the host, which many callers wait for) and the partial tiles at 5 TB/s.
-// Measured, general kernel of 128 x 128 tiles -> here: M 777, N 333, K 1024 107.2 -> 15.7 (three splits; 17.7 in two
-// groups); its adjoint M 777, N 1024, K 333 45.4 -> 12.4 and M 333, N 1024, K 777, both operands along their rows, 84.1 ->
+// Measured, general kernel of 128 x 128 tiles -> here: M 777, N 333, K 1024 107.2 -> 17.7 (two groups; 15.7 in three
+// splits, which the host's share makes the slower call); its adjoint M 777, N 1024, K 333 45.4 -> 12.4 and M 333, N 1024, K 777, both operands along their rows, 84.1 ->
 // 15.6; M 8, N 4096, K 4096 365 -> 20.  256 x 256 tiles -> here: M = N = K = 2048 351 -> 153, M 4096, N 4096, K 1024 310 ->
 // 294; M = N = K = 4096 973, here 1060: those stay.
 Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double other_us) {
