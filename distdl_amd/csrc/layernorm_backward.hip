@@ -20,7 +20,12 @@
 //                    workspace, for dgamma and dbeta
 // One wavefront owns a row and strides over its columns (four elements at a time
 // when the row is aligned); nothing is kept between passes, so rows of any length
-// work.  dy, x, gamma, dx, dgamma and dbeta are float, bf16 or fp16 (one type per
+// work.  Callers that want dx and the parameter gradients get fewer passes:
+//   ln_bwd_partial_cols   row sums, column sums and (rows held whole, or the other
+//                         workers' sums in memory) dx in one pass, a wavefront per
+//                         row of at most 1024 columns
+//   ln_bwd_block_rows     the same with a workgroup per longer row
+// dy, x, gamma, dx, dgamma and dbeta are float, bf16 or fp16 (one type per
 // call); the arithmetic, the saved mean and rstd, the row sums and the workspace
 // are fp32.
 #include "ln_elements.h"

@@ -5,11 +5,10 @@
 //   dw[N,K] = dy[M,N]^T . x[M,K]        reduction over M
 //   db[N]   = sum over m of dy[m,N]
 //
-// The shard GEMM multiplies two operands that are contiguous along the
-// reduction dimension.  dy is (for dx); w, dy and x (for dx and dw) are not, so
-// they are transposed once into a workspace -- a pass over 2 bytes per element
-// each way, small next to the GEMM -- and the same GEMM kernel does the rest.
-// db is a column sum with fp32 accumulation.
+// ddl_linear_backward runs what is wanted of the three: the products read w, dy
+// and x where they lie (ddl_gemm_ws), db is a column sum with fp32 accumulation.
+// Large 16-bit products whose operands cannot be read in place are transposed
+// into temporaries by the caller (ddl_transpose_2d) and go through ddl_linear.
 #include "ddl_common.h"
 
 #include <hip/hip_fp16.h>
