@@ -53,6 +53,9 @@ class _Plan:
                 if buffers[i][j] is None:
                     continue
                 box = slices[i][j]
+                for d, (s, n) in enumerate(zip(box, shape)):
+                    if not 0 <= s.start <= s.stop <= n:     # a shard narrower than its strips; the copies know no extents
+                        raise RuntimeError(f"halo strip {j} of dim {i}: [{s.start},{s.stop}) outside extent {n} of dim {d}")
                 extent = [int(s.stop) - int(s.start) for s in box]
                 own = strides if from_input else tensor_strides
                 offset = sum(int(s.start) * t for s, t in zip(box, own))

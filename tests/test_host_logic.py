@@ -705,3 +705,29 @@ def test_bench_refuses_more_than_one_gpu():
                           timeout=300)
     assert done.returncode != 0
     assert "ONE GPU" in (done.stderr + done.stdout)
+
+
+def _halo_plan(shape, recv, send, forward, present=None):
+    """The launches of one direction of an exchange, built on the host (no addresses yet)."""
+    from distdl_amd.backends.stub_hip.functional import halo_exchange as h
+    recv, send = np.asarray(recv), np.asarray(send)
+    slices = h.SliceTable(assemble_halo_slices(shape, recv, send))
+    if present is None:
+        present = [(send[i, 0] > 0, recv[i, 0] > 0, send[i, 1] > 0, recv[i, 1] > 0) for i in range(len(shape))]
+    buffers = [[ExpandableBuffer(torch.float32, device="cpu") if p else None for p in row] for row in present]
+    return h._plan(slices, buffers, torch.zeros(shape), forward)
+
+
+@pytest.mark.parametrize("forward", [True, False])
+@pytest.mark.parametrize("shape,recv,send", [
+    ((4, 3), [[0, 0], [2, 0]], [[0, 0], [2, 0]]),        # a shard of one column under a kernel of 5: the left bulk strip ends behind it
+    ((4, 3), [[0, 0], [0, 2]], [[0, 0], [0, 2]]),        # the right one starts in front of it
+    ((4, 3), [[1, 1], [2, 2]], [[1, 1], [0, 0]]),        # ghosts of another dimension leave no bulk
+    ((5,), [[0, 6]], [[0, 0]])])                         # a ghost wider than the tensor
+def test_halo_strips_outside_the_tensor_are_refused(shape, recv, send, forward):
+    """Copies of boxes know addresses and strides only, so a strip that leaves the tensor has to be refused when the
+    launches are built; strips that just fit are accepted."""
+    with pytest.raises(RuntimeError, match="outside extent"):
+        _halo_plan(shape, recv, send, forward)
+    _halo_plan(tuple(n + 8 for n in shape), recv, send, forward)
+    _halo_plan((4, 4), [[0, 0], [2, 0]], [[0, 0], [2, 0]], forward)
