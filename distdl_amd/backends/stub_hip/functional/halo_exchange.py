@@ -39,10 +39,11 @@ _LEFT_BULK, _LEFT_GHOST, _RIGHT_BULK, _RIGHT_GHOST = range(4)
 
 class _Plan:
     """The launches of one direction for one structure of the tensor, lowered
-    once.  Buffers are looked up on every call (a pooled buffer may have been
-    reallocated); what is kept is geometry only."""
+    once.  ``present[i][j]`` says whether strip ``j`` of dimension ``i`` has a
+    buffer.  What is kept is geometry only: the buffers are those of the call
+    (and a pooled buffer may have been reallocated since the last one)."""
 
-    def __init__(self, slices, buffers, shape, strides, elem_size, forward):
+    def __init__(self, slices, present, shape, strides, elem_size, forward):
         self.dims = []
         tensor_strides = hip_ops.contiguous_strides(shape)
 
@@ -50,7 +51,7 @@ class _Plan:
             """Boxes between the strips ``sides`` of dimension ``i`` and their buffers."""
             out = []
             for j in sides:
-                if buffers[i][j] is None:
+                if not present[i][j]:
                     continue
                 box = slices[i][j]
                 for d, (s, n) in enumerate(zip(box, shape)):
@@ -73,7 +74,7 @@ class _Plan:
         first = [(_INPUT, 0, _TENSOR, 0, list(shape), strides, tensor_strides)]
         untouched = True
         for i in range(len(slices)):
-            views = [None if b is None else (b, compute_nd_slice_shape(s)) for s, b in zip(slices[i], buffers[i])]
+            extents = [compute_nd_slice_shape(s) for s in slices[i]]
             if forward:
                 pack, unpack = boxes(i, bulk, True, untouched), boxes(i, ghost, False)
                 merged = untouched
@@ -81,7 +82,7 @@ class _Plan:
                 if merged:
                     first += pack
                     pack = []
-                self.dims.append((views, [hip_ops.BoxLaunch(pack, elem_size)], [hip_ops.BoxLaunch(unpack, elem_size)]))
+                self.dims.append((extents, [hip_ops.BoxLaunch(pack, elem_size)], [hip_ops.BoxLaunch(unpack, elem_size)]))
             else:
                 add = boxes(i, bulk, False)
                 if len(add) == 2 and slices[i][0][i].stop > slices[i][2][i].start:
@@ -90,33 +91,34 @@ class _Plan:
                     adds = [hip_ops.BoxLaunch(add[:1], elem_size), hip_ops.BoxLaunch(add[1:], elem_size)]
                 else:
                     adds = [hip_ops.BoxLaunch(add, elem_size)]
-                self.dims.append((views, [hip_ops.BoxLaunch(boxes(i, ghost, True), elem_size)], adds))
+                self.dims.append((extents, [hip_ops.BoxLaunch(boxes(i, ghost, True), elem_size)], adds))
         self.first = hip_ops.BoxLaunch(first, elem_size) if forward else None
 
 
 def _plan(slices, buffers, tensor, forward):
     cache = getattr(slices, "plans", None)
-    key = (forward, tensor.shape, tensor.stride(), tensor.element_size(), tuple([b is None for side in buffers for b in side]))
+    present = tuple([tuple([b is not None for b in sides]) for sides in buffers])
+    key = (forward, tensor.shape, tensor.stride(), tensor.element_size(), present)
     plan = None if cache is None else cache.get(key)
     if plan is None:
-        plan = _Plan(slices, buffers, tuple(int(n) for n in tensor.shape), [int(s) for s in tensor.stride()], tensor.element_size(), forward)
+        plan = _Plan(slices, present, tuple(int(n) for n in tensor.shape), [int(s) for s in tensor.stride()], tensor.element_size(), forward)
         if cache is not None:
             cache[key] = plan
     return plan
 
 
-def _dim_views(views, tensor, bases):
-    """The four buffer views of a dimension; their addresses go into ``bases``."""
+def _dim_views(buffers, extents, tensor, bases):
+    """The views of a dimension's four buffers; their addresses go into ``bases``."""
     out = []
-    for v in views:
-        if v is None:
+    for buffer, extent in zip(buffers, extents):
+        if buffer is None:
             out.append(None)
             bases.append(0)
             continue
-        buffer, shape = v
-        view = buffer.get_view(shape)
-        if view.dtype != tensor.dtype or not view.is_cuda:
-            raise ValueError(f"buffer {tuple(view.shape)}/{view.dtype} on {view.device} does not match a tensor of {tensor.dtype}")
+        view = buffer.get_view(extent)
+        hip_ops._require_gpu(view)
+        if view.dtype != tensor.dtype:
+            raise ValueError(f"buffer {tuple(view.shape)}/{view.dtype} does not match a tensor of {tensor.dtype}")
         out.append(view)
         bases.append(view.data_ptr())
     return out
@@ -162,7 +164,7 @@ class HaloExchangeFunction(torch.autograd.Function):
         output = torch.empty_like(src, memory_format=torch.contiguous_format)
         plan = _plan(slices, buffers, src, True)
         bases = [src.data_ptr(), output.data_ptr()]
-        views = [_dim_views(dim[0], output, bases) for dim in plan.dims]
+        views = [_dim_views(row, dim[0], output, bases) for row, dim in zip(buffers, plan.dims)]
         plan.first.run(bases)
         for i, (lbb, lgb, rbb, rgb) in enumerate(views):
             for launch in plan.dims[i][1]:
@@ -191,7 +193,7 @@ class HaloExchangeFunction(torch.autograd.Function):
         add_dtype = hip_ops._ADD_DTYPES[grad_output.dtype]
         plan = _plan(slices, buffers, grad_output, False)
         bases = [0, grad_output.data_ptr()]
-        views = [_dim_views(dim[0], grad_output, bases) for dim in plan.dims]
+        views = [_dim_views(row, dim[0], grad_output, bases) for row, dim in zip(buffers, plan.dims)]
         for i in reversed(range(len(views))):
             lbb, lgb, rbb, rgb = views[i]
             for launch in plan.dims[i][1]:

@@ -731,3 +731,74 @@ def test_halo_strips_outside_the_tensor_are_refused(shape, recv, send, forward):
         _halo_plan(shape, recv, send, forward)
     _halo_plan(tuple(n + 8 for n in shape), recv, send, forward)
     _halo_plan((4, 4), [[0, 0], [2, 0]], [[0, 0], [2, 0]], forward)
+
+
+@pytest.fixture
+def boxes_on_the_cpu(monkeypatch):
+    """Box launches carried out on host memory, element by element of what their descriptors say."""
+    from distdl_amd import hip_ops
+
+    def run(launch, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
+        assert launch.elem_size == 4 and (op != _lib.DDL_OP_ADD or dtype == _lib.DDL_DT_F32)
+        boxes = (launch._type).from_buffer_copy(launch._template)
+        sides = []
+        for box, (src, src_off, dst, dst_off) in zip(boxes, launch._bases):
+            at = []
+            for base, strides in ((bases[src] + src_off, box.src_stride), (bases[dst] + dst_off, box.dst_stride)):
+                one = np.ctypeslib.as_array((ctypes.c_float * 1).from_address(base))
+                at.append(np.lib.stride_tricks.as_strided(one, list(box.shape)[:box.ndim], [4 * v for v in list(strides)[:box.ndim]]))
+            sides.append(at)
+        for src, dst in sides:
+            dst[...] = dst + src if op == _lib.DDL_OP_ADD else src
+            if op == _lib.DDL_OP_MOVE:
+                src[...] = 0
+
+    def zero(plan, tensor):
+        assert plan.matches(tensor)
+        for k, shape in enumerate(plan.box_shapes):
+            start = list(plan.start_arr)[k * plan.ndim:(k + 1) * plan.ndim]
+            if shape is not None:
+                tensor[tuple(slice(a, a + n) for a, n in zip(start, shape))] = 0
+
+    monkeypatch.setattr(hip_ops, "_require_gpu", lambda *tensors: None)
+    monkeypatch.setattr(hip_ops.BoxLaunch, "run", run)
+    monkeypatch.setattr(hip_ops.BoxPlan, "zero", zero)
+
+
+class _Exchange:
+    """An interior worker of a row of three with one exchanged dimension, without its neighbours: nothing is sent, and what
+    would arrive is what the ghost (adjoint: bulk) buffers hold."""
+
+    def __init__(self, shape, recv, send):
+        from distdl_amd.backends.stub_hip.functional import halo_exchange as h
+        self.function, self.shape = h.HaloExchangeFunction, shape
+        self.P = SimWorld(3 ** len(shape), device="cpu").partition(3 ** len(shape) // 2).create_cartesian_topology_partition([3] * len(shape))
+        self.recv, self.send = np.asarray(recv), np.asarray(send)
+        self.slices = h.SliceTable(assemble_halo_slices(shape, self.recv, self.send))
+
+    def buffers(self, fill, dtype=torch.float32):
+        from distdl_amd.backends.stub_hip.buffer_allocator import allocate_halo_exchange_buffers
+        manager = BufferManager(device="cpu")
+        out = allocate_halo_exchange_buffers(manager, self.slices, self.recv, self.send, dtype)
+        for k, buf in enumerate(manager.buffers_map[dtype]):
+            buf.raw_buffer.fill_(fill + k)
+        return out
+
+    def forward(self, x, buffers):
+        return self.function.apply(x, self.P, self.slices, buffers, self.P.neighbor_ranks(self.P.rank))
+
+
+def test_halo_exchange_uses_the_buffers_it_is_handed(boxes_on_the_cpu):
+    """One table of slices, two sets of buffers: each call packs into and unpacks from its own."""
+    e = _Exchange((6,), [[1, 1]], [[2, 2]])
+    x = torch.arange(6.0)
+    for fill in (10.0, 20.0):
+        buffers = e.buffers(fill)
+        xin = x.clone().requires_grad_(True)
+        y = e.forward(xin, buffers)
+        assert y.tolist() == [fill + 1, 1, 2, 3, 4, fill + 3]
+        assert buffers[0][0].raw_buffer.tolist() == [1, 2] and buffers[0][2].raw_buffer.tolist() == [3, 4]
+        dx, = torch.autograd.grad(y, xin, torch.arange(6.0))
+        # the ghosts leave, what arrived in the bulk buffers (still what the forward packed) is added
+        assert buffers[0][1].raw_buffer.tolist() == [0] and buffers[0][3].raw_buffer.tolist() == [5]
+        assert dx.tolist() == [0, 1 + 1, 2 + 2, 3 + 3, 4 + 4, 0]
