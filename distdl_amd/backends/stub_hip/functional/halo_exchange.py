@@ -39,11 +39,11 @@ _LEFT_BULK, _LEFT_GHOST, _RIGHT_BULK, _RIGHT_GHOST = range(4)
 
 class _Plan:
     """The launches of one direction for one structure of the tensor, lowered
-    once.  ``present[i][j]`` says whether strip ``j`` of dimension ``i`` has a
-    buffer.  What is kept is geometry only: the buffers are those of the call
+    once, for the first ``dims`` dimensions (those of the partition).
+    ``present[i][j]`` says whether strip ``j`` of dimension ``i`` has a buffer.  What is kept is geometry only: the buffers are those of the call
     (and a pooled buffer may have been reallocated since the last one)."""
 
-    def __init__(self, slices, present, shape, strides, elem_size, forward):
+    def __init__(self, dims, slices, present, shape, strides, elem_size, forward):
         self.dims = []
         tensor_strides = hip_ops.contiguous_strides(shape)
 
@@ -73,7 +73,7 @@ class _Plan:
         # them yet, and no other dimension's strips are in the buffers, which all dimensions share.
         first = [(_INPUT, 0, _TENSOR, 0, list(shape), strides, tensor_strides)]
         untouched = True
-        for i in range(len(slices)):
+        for i in range(dims):
             extents = [compute_nd_slice_shape(s) for s in slices[i]]
             if forward:
                 pack, unpack = boxes(i, bulk, True, untouched), boxes(i, ghost, False)
@@ -95,13 +95,14 @@ class _Plan:
         self.first = hip_ops.BoxLaunch(first, elem_size) if forward else None
 
 
-def _plan(slices, buffers, tensor, forward):
+def _plan(dims, slices, buffers, tensor, forward):
     cache = getattr(slices, "plans", None)
     present = tuple([tuple([b is not None for b in sides]) for sides in buffers])
-    key = (forward, tensor.shape, tensor.stride(), tensor.element_size(), present)
+    key = (dims, forward, tensor.shape, tensor.stride(), tensor.element_size(), present)
     plan = None if cache is None else cache.get(key)
     if plan is None:
-        plan = _Plan(slices, present, tuple(int(n) for n in tensor.shape), [int(s) for s in tensor.stride()], tensor.element_size(), forward)
+        plan = _Plan(dims, slices, present, tuple(int(n) for n in tensor.shape), [int(s) for s in tensor.stride()],
+                     tensor.element_size(), forward)
         if cache is not None:
             cache[key] = plan
     return plan
@@ -162,7 +163,7 @@ class HaloExchangeFunction(torch.autograd.Function):
         src = input.detach()
         hip_ops._require_gpu(src)
         output = torch.empty_like(src, memory_format=torch.contiguous_format)
-        plan = _plan(slices, buffers, src, True)
+        plan = _plan(P_x.dim, slices, buffers, src, True)
         bases = [src.data_ptr(), output.data_ptr()]
         views = [_dim_views(row, dim[0], output, bases) for row, dim in zip(buffers, plan.dims)]
         plan.first.run(bases)
@@ -191,7 +192,7 @@ class HaloExchangeFunction(torch.autograd.Function):
         if grad_output.dtype not in hip_ops._ADD_DTYPES:
             raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
         add_dtype = hip_ops._ADD_DTYPES[grad_output.dtype]
-        plan = _plan(slices, buffers, grad_output, False)
+        plan = _plan(P_x.dim, slices, buffers, grad_output, False)
         bases = [0, grad_output.data_ptr()]
         views = [_dim_views(row, dim[0], grad_output, bases) for row, dim in zip(buffers, plan.dims)]
         for i in reversed(range(len(views))):

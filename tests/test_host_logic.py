@@ -715,7 +715,7 @@ def _halo_plan(shape, recv, send, forward, present=None):
     if present is None:
         present = [(send[i, 0] > 0, recv[i, 0] > 0, send[i, 1] > 0, recv[i, 1] > 0) for i in range(len(shape))]
     buffers = [[ExpandableBuffer(torch.float32, device="cpu") if p else None for p in row] for row in present]
-    return h._plan(slices, buffers, torch.zeros(shape), forward)
+    return h._plan(len(shape), slices, buffers, torch.zeros(shape), forward)
 
 
 @pytest.mark.parametrize("forward", [True, False])
@@ -766,13 +766,14 @@ def boxes_on_the_cpu(monkeypatch):
 
 
 class _Exchange:
-    """An interior worker of a row of three with one exchanged dimension, without its neighbours: nothing is sent, and what
+    """An interior worker of a grid with three workers along each dimension, without its neighbours: nothing is sent, and what
     would arrive is what the ghost (adjoint: bulk) buffers hold."""
 
-    def __init__(self, shape, recv, send):
+    def __init__(self, shape, recv, send, dims=None):
         from distdl_amd.backends.stub_hip.functional import halo_exchange as h
-        self.function, self.shape = h.HaloExchangeFunction, shape
-        self.P = SimWorld(3 ** len(shape), device="cpu").partition(3 ** len(shape) // 2).create_cartesian_topology_partition([3] * len(shape))
+        dims = len(shape) if dims is None else dims
+        self.function = h.HaloExchangeFunction
+        self.P = SimWorld(3 ** dims, device="cpu").partition(3 ** dims // 2).create_cartesian_topology_partition([3] * dims)
         self.recv, self.send = np.asarray(recv), np.asarray(send)
         self.slices = h.SliceTable(assemble_halo_slices(shape, self.recv, self.send))
 
@@ -802,3 +803,14 @@ def test_halo_exchange_uses_the_buffers_it_is_handed(boxes_on_the_cpu):
         # the ghosts leave, what arrived in the bulk buffers (still what the forward packed) is added
         assert buffers[0][1].raw_buffer.tolist() == [0] and buffers[0][3].raw_buffer.tolist() == [5]
         assert dx.tolist() == [0, 1 + 1, 2 + 2, 3 + 3, 4 + 4, 0]
+
+
+def test_halo_exchange_of_a_tensor_with_more_dimensions_than_the_partition(boxes_on_the_cpu):
+    """The dimensions of the partition are exchanged, those behind them are left alone."""
+    e = _Exchange((4, 2), [[1, 0], [0, 0]], [[1, 0], [0, 0]], dims=1)
+    x = torch.arange(8.0).reshape(4, 2).requires_grad_(True)
+    buffers = e.buffers(10.0)
+    y = e.forward(x, buffers)
+    assert y.tolist() == [[11, 11], [2, 3], [4, 5], [6, 7]]
+    dx, = torch.autograd.grad(y, x, torch.ones(4, 2))
+    assert dx.tolist() == [[0, 0], [3, 4], [1, 1], [1, 1]]
