@@ -189,12 +189,12 @@ class HaloExchangeFunction(torch.autograd.Function):
             raise ValueError("HaloExchange adjoint needs a contiguous gradient")
 
         hip_ops._require_gpu(grad_output)
-        if grad_output.dtype not in hip_ops._ADD_DTYPES:
-            raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
-        add_dtype = hip_ops._ADD_DTYPES[grad_output.dtype]
         plan = _plan(P_x.dim, slices, buffers, grad_output, False)
         bases = [0, grad_output.data_ptr()]
         views = [_dim_views(row, dim[0], grad_output, bases) for row, dim in zip(buffers, plan.dims)]
+        add_dtype = hip_ops._ADD_DTYPES.get(grad_output.dtype)
+        if add_dtype is None and any(lbb is not None or rbb is not None for lbb, _, rbb, _ in views):
+            raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
         for i in reversed(range(len(views))):
             lbb, lgb, rbb, rgb = views[i]
             for launch in plan.dims[i][1]:

@@ -735,18 +735,22 @@ def test_halo_strips_outside_the_tensor_are_refused(shape, recv, send, forward):
 
 @pytest.fixture
 def boxes_on_the_cpu(monkeypatch):
-    """Box launches carried out on host memory, element by element of what their descriptors say."""
+    """Box launches carried out on host memory, as their descriptors say."""
     from distdl_amd import hip_ops
 
     def run(launch, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
-        assert launch.elem_size == 4 and (op != _lib.DDL_OP_ADD or dtype == _lib.DDL_DT_F32)
-        boxes = (launch._type).from_buffer_copy(launch._template)
+        if launch.n == 0:
+            return
+        element = {4: ctypes.c_float, 8: ctypes.c_double}[launch.elem_size]
+        assert op != _lib.DDL_OP_ADD or dtype == _lib.DDL_DT_F32
+        boxes = launch._type.from_buffer_copy(launch._template)
         sides = []
         for box, (src, src_off, dst, dst_off) in zip(boxes, launch._bases):
             at = []
             for base, strides in ((bases[src] + src_off, box.src_stride), (bases[dst] + dst_off, box.dst_stride)):
-                one = np.ctypeslib.as_array((ctypes.c_float * 1).from_address(base))
-                at.append(np.lib.stride_tricks.as_strided(one, list(box.shape)[:box.ndim], [4 * v for v in list(strides)[:box.ndim]]))
+                one = np.ctypeslib.as_array((element * 1).from_address(base))
+                steps = [launch.elem_size * v for v in list(strides)[:box.ndim]]
+                at.append(np.lib.stride_tricks.as_strided(one, list(box.shape)[:box.ndim], steps))
             sides.append(at)
         for src, dst in sides:
             dst[...] = dst + src if op == _lib.DDL_OP_ADD else src
@@ -814,3 +818,15 @@ def test_halo_exchange_of_a_tensor_with_more_dimensions_than_the_partition(boxes
     assert y.tolist() == [[11, 11], [2, 3], [4, 5], [6, 7]]
     dx, = torch.autograd.grad(y, x, torch.ones(4, 2))
     assert dx.tolist() == [[0, 0], [3, 4], [1, 1], [1, 1]]
+
+
+def test_halo_adjoint_refuses_element_types_only_where_something_is_added(boxes_on_the_cpu):
+    """Ghosts move out as bytes; sums need an arithmetic type."""
+    x = torch.tensor([1 + 2j, 3 + 4j, 5 + 6j], dtype=torch.complex64).requires_grad_(True)
+    y = _Exchange((3,), [[0, 0]], [[0, 0]]).forward(x, [[None] * 4])
+    dx, = torch.autograd.grad(y, x, torch.ones(3, dtype=torch.complex64))
+    assert dx.tolist() == [1, 1, 1]
+    e = _Exchange((3,), [[0, 0]], [[1, 0]])
+    y = e.forward(x, e.buffers(0.0, torch.complex64))
+    with pytest.raises(ValueError, match="not available"):
+        torch.autograd.grad(y, x, torch.ones(3, dtype=torch.complex64))
