@@ -82,7 +82,7 @@ class _Plan:
                 if merged:
                     first += pack
                     pack = []
-                self.dims.append((extents, [hip_ops.BoxLaunch(pack, elem_size)], [hip_ops.BoxLaunch(unpack, elem_size)]))
+                self.dims.append((extents, hip_ops.BoxLaunch(pack, elem_size), hip_ops.BoxLaunch(unpack, elem_size)))
             else:
                 add = boxes(i, bulk, False)
                 if len(add) == 2 and slices[i][0][i].stop > slices[i][2][i].start:
@@ -91,7 +91,15 @@ class _Plan:
                     adds = [hip_ops.BoxLaunch(add[:1], elem_size), hip_ops.BoxLaunch(add[1:], elem_size)]
                 else:
                     adds = [hip_ops.BoxLaunch(add, elem_size)]
-                self.dims.append((extents, [hip_ops.BoxLaunch(boxes(i, ghost, True), elem_size)], adds))
+                out = hip_ops.BoxLaunch(boxes(i, ghost, True), elem_size)
+                left, right = slices[i][_LEFT_GHOST], slices[i][_RIGHT_GHOST]
+                clear = None
+                # A ghost leaves and is cleared in one launch.  Not where the two share elements (one box would read what
+                # the other has cleared), nor where a ghost has no buffer and is cleared all the same.
+                if out.n and (left[i].stop > right[i].start or any(not present[i][j] and min(extents[j]) > 0 for j in ghost)):
+                    clear = hip_ops.BoxPlan(shape, strides, [([int(s.start) for s in b], [int(s.stop) - int(s.start) for s in b])
+                                                             for b in (left, right)])
+                self.dims.append((extents, out, clear, adds))
         self.first = hip_ops.BoxLaunch(first, elem_size) if forward else None
 
 
@@ -168,11 +176,10 @@ class HaloExchangeFunction(torch.autograd.Function):
         views = [_dim_views(row, dim[0], output, bases) for row, dim in zip(buffers, plan.dims)]
         plan.first.run(bases)
         for i, (lbb, lgb, rbb, rgb) in enumerate(views):
-            for launch in plan.dims[i][1]:
-                launch.run(bases)
+            _, pack, unpack = plan.dims[i]
+            pack.run(bases)
             _swap(P_x, neighbor_ranks[i], lbb, rbb, lgb, rgb)
-            for launch in plan.dims[i][2]:
-                launch.run(bases)
+            unpack.run(bases)
         return output
 
     @staticmethod
@@ -197,9 +204,11 @@ class HaloExchangeFunction(torch.autograd.Function):
             raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
         for i in reversed(range(len(views))):
             lbb, lgb, rbb, rgb = views[i]
-            for launch in plan.dims[i][1]:
-                launch.run(bases, op=_lib.DDL_OP_MOVE)
+            _, out, clear, adds = plan.dims[i]
+            out.run(bases, op=_lib.DDL_OP_COPY if clear else _lib.DDL_OP_MOVE)
+            if clear:
+                clear.zero(grad_output)
             _swap(P_x, ctx.neighbor_ranks[i], lgb, rgb, lbb, rbb)
-            for launch in plan.dims[i][2]:
+            for launch in adds:
                 launch.run(bases, op=_lib.DDL_OP_ADD, dtype=add_dtype)
         return grad_output, None, None, None, None

@@ -830,3 +830,19 @@ def test_halo_adjoint_refuses_element_types_only_where_something_is_added(boxes_
     y = e.forward(x, e.buffers(0.0, torch.complex64))
     with pytest.raises(ValueError, match="not available"):
         torch.autograd.grad(y, x, torch.ones(3, dtype=torch.complex64))
+
+
+def test_halo_adjoint_of_ghosts_that_share_elements_or_have_no_buffer(boxes_on_the_cpu):
+    """Both ghosts leave as they came in before either is cleared, and a ghost without a buffer is cleared with the other."""
+    e = _Exchange((3,), [[2, 2]], [[0, 0]])
+    x = torch.zeros(3).requires_grad_(True)
+    buffers = e.buffers(7.0)
+    dx, = torch.autograd.grad(e.forward(x, buffers), x, torch.tensor([1.0, 2.0, 3.0]))
+    assert buffers[0][1].raw_buffer.tolist() == [1, 2] and buffers[0][3].raw_buffer.tolist() == [2, 3]
+    assert dx.tolist() == [0, 0, 0]
+    e = _Exchange((4,), [[1, 1]], [[0, 0]])
+    x = torch.zeros(4).requires_grad_(True)
+    buffers = [[None, e.buffers(7.0)[0][1], None, None]]
+    dx, = torch.autograd.grad(e.forward(x, buffers), x, torch.tensor([1.0, 2.0, 3.0, 4.0]))
+    assert buffers[0][1].raw_buffer.tolist() == [1]
+    assert dx.tolist() == [0, 2, 3, 0]
