@@ -19,11 +19,15 @@ from ....utilities.slicing import compute_subshape
 
 
 @functools.lru_cache(maxsize=512)
-def _gather_launch(shapes, axis, elem_size):
+def _gather_launch(local_shape, shapes, axis, elem_size):
     """(output shape, launch) that joins contiguous pieces of these shapes along
-    ``axis``; the output is slot 0 of the launch, piece q slot 1 + q.  Geometry
-    only: a function of its arguments."""
-    shape = list(shapes[0])
+    ``axis``; the output is slot 0 of the launch, piece q slot 1 + q, and has the
+    extents of ``local_shape`` off the axis, as every piece must have that is not
+    empty along it.  Geometry only: a function of its arguments."""
+    shape = list(local_shape)
+    for piece in shapes:
+        if len(piece) != len(shape) or (piece[axis] and any(n != m for d, (n, m) in enumerate(zip(piece, shape)) if d != axis)):
+            raise ValueError(f"gathered piece of shape {piece} does not fit {tuple(local_shape)} along axis {axis}")
     shape[axis] = sum(s[axis] for s in shapes)
     strides = hip_ops.contiguous_strides(shape)
     entries, start = [], 0
@@ -56,7 +60,7 @@ def gather_slabs(P, local, axis, tag):
         if p.dtype != x.dtype or not p.is_contiguous():
             raise ValueError(f"gathered piece {tuple(p.shape)}/{p.dtype} does not match {x.dtype} or is not contiguous")
     axis = axis % x.dim()
-    shape, launch = _gather_launch(tuple([tuple(p.shape) for p in parts]), axis, x.element_size())
+    shape, launch = _gather_launch(tuple(x.shape), tuple([tuple(p.shape) for p in parts]), axis, x.element_size())
     out = torch.empty(shape, dtype=x.dtype, device=x.device)
     launch.run([out.data_ptr()] + [p.data_ptr() for p in parts])
     transport.release(P, tag=tag)

@@ -846,3 +846,15 @@ def test_halo_adjoint_of_ghosts_that_share_elements_or_have_no_buffer(boxes_on_t
     dx, = torch.autograd.grad(e.forward(x, buffers), x, torch.tensor([1.0, 2.0, 3.0, 4.0]))
     assert buffers[0][1].raw_buffer.tolist() == [1]
     assert dx.tolist() == [0, 2, 3, 0]
+
+
+def test_gathered_pieces_of_other_extents_are_refused():
+    """The launch that joins pieces knows addresses and strides only: a piece whose extents off the axis are not the
+    local ones would be written past the output."""
+    from distdl_amd.backends.stub_hip.functional.all_gather import _gather_launch
+    assert _gather_launch((2, 3, 4), ((2, 3, 4), (2, 3, 1), (2, 3, 0)), 2, 4)[0] == (2, 3, 5)
+    for shapes in ((2, 3, 4), (5, 3, 4)), ((5, 3, 4), (5, 3, 4)), ((2, 3, 4), (2, 2, 4)), ((2, 3, 4), (6, 4)), ((2, 3, 4), (2, 3, 4, 1)):
+        with pytest.raises(ValueError, match="does not fit"):
+            _gather_launch((2, 3, 4), shapes, 2, 4)
+    out, launch = _gather_launch((2, 3, 4), ((2, 3, 4), (5, 3, 0)), 2, 4)
+    assert out == (2, 3, 4) and launch.n == 1
