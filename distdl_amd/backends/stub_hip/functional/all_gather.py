@@ -59,7 +59,7 @@ def gather_slabs(P, local, axis, tag):
     for p in parts:
         if p.dtype != x.dtype or not p.is_contiguous():
             raise ValueError(f"gathered piece {tuple(p.shape)}/{p.dtype} does not match {x.dtype} or is not contiguous")
-    axis = axis % x.dim()
+    axis = range(x.dim())[axis]      # an axis the tensor has not is an IndexError
     shape, launch = _gather_launch(tuple(x.shape), tuple([tuple(p.shape) for p in parts]), axis, x.element_size())
     out = torch.empty(shape, dtype=x.dtype, device=x.device)
     launch.run([out.data_ptr()] + [p.data_ptr() for p in parts])
@@ -75,7 +75,7 @@ def reduce_scatter_slabs(P, full, axis, tag, divisor=1):
     transport = P._world.transport
     g = hip_ops.contiguous(full)
     grads = transport.gather_list(P, g, tag=tag)
-    shape, src, dst = _slab(int(P.size), int(P.rank), tuple(g.shape), axis % g.dim())
+    shape, src, dst = _slab(int(P.size), int(P.rank), tuple(g.shape), range(g.dim())[axis])
     out = torch.empty(shape, dtype=g.dtype, device=g.device)
     if out.numel():
         hip_ops.sum_boxes(grads, src, out, dst, divisor)

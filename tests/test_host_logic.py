@@ -858,3 +858,18 @@ def test_gathered_pieces_of_other_extents_are_refused():
             _gather_launch((2, 3, 4), shapes, 2, 4)
     out, launch = _gather_launch((2, 3, 4), ((2, 3, 4), (5, 3, 0)), 2, 4)
     assert out == (2, 3, 4) and launch.n == 1
+
+
+@pytest.mark.parametrize("relayout", ["gather_slabs", "reduce_scatter_slabs"])
+@pytest.mark.parametrize("axis", [3, 5, -4])
+def test_relayouts_along_an_axis_the_tensor_has_not_are_refused(monkeypatch, relayout, axis):
+    from distdl_amd import hip_ops
+    from distdl_amd.backends.stub_hip.functional import all_gather
+    monkeypatch.setattr(hip_ops, "_require_gpu", lambda *tensors: None)
+    monkeypatch.setattr(hip_ops.BoxLaunch, "run", lambda *args: None)
+    monkeypatch.setattr(hip_ops, "sum_boxes", lambda *args: None)
+    P = SimWorld(2, device="cpu").partition(0)
+    with pytest.raises(IndexError):
+        getattr(all_gather, relayout)(P, torch.zeros(2, 4, 6), axis, None)
+    out = getattr(all_gather, relayout)(P, torch.zeros(2, 4, 6), -1, None)
+    assert tuple(out.shape) == ((2, 4, 12) if relayout == "gather_slabs" else (2, 4, 3))
