@@ -122,6 +122,9 @@ SIGNATURES = {
                             c_int64, c_int64, c_void_p, c_int64, c_void_p]),
     "ddl_gemm_in_place": (c_int, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64]),
     "ddl_gemm_workspace": (c_int64, [c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64]),
+    "ddl_gemm_workspace_at": (c_int64, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64]),
+    "ddl_linear_backward_workspace_at": (c_int64, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int,
+                                                   c_int]),
     "ddl_linear_backward_workspace": (c_int64, [c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_int]),
     "ddl_linear_backward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64,
                                     c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p]),

@@ -358,19 +358,27 @@ extern "C" int ddl_colsum(const void* a, int dtype, int64_t rows, int64_t cols, 
     return run_colsum<2>(a, rows, cols, ld, out, workspace, splits, rows_per_split, strips, s);
 }
 
-extern "C" int64_t ddl_linear_backward_workspace(int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy,
-                                                 int want_dx, int want_dw, int want_db) {
-    // The products and the column sum run one after the other, so they share the workspace.
+extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                                    int64_t lddy, int want_dx, int want_dw, int want_db) {
+    // The products and the column sum run one after the other, so they share the workspace.  If not all operands are
+    // aligned, a product may still have two that are.
     int64_t most = 0;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     auto take = [&](int64_t elems) { most = elems > most ? elems : most; };
-    if (want_dx) take(ddl_gemm_workspace(dtype, lddy, 1, 1, ldw, M, K, N));
-    if (want_dw) take(ddl_gemm_workspace(dtype, 1, lddy, 1, ldx, N, K, M));
+    for (int both = aligned ? 1 : 0; both < 2; ++both) {
+        if (want_dx) take(ddl_gemm_workspace_at(dtype, both, lddy, 1, 1, ldw, M, K, N));
+        if (want_dw) take(ddl_gemm_workspace_at(dtype, both, 1, lddy, 1, ldx, N, K, M));
+    }
     if (want_db && !ddl::colsum_in_one_launch(M, dtype == DDL_DT_F32 ? 4 : 2)) {
         const int64_t splits = (M + 127) / 128;
         take((splits < 64 ? splits : 64) * N);
     }
     return most;
+}
+
+extern "C" int64_t ddl_linear_backward_workspace(int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy,
+                                                 int want_dx, int want_dw, int want_db) {
+    return ddl_linear_backward_workspace_at(dtype, 1, M, N, K, ldx, ldw, lddy, want_dx, want_dw, want_db);
 }
 
 extern "C" int ddl_linear_backward(const void* x, const void* w, const void* dy, void* dx, void* dw, void* db, int dtype, int64_t M, int64_t N,

@@ -551,10 +551,13 @@ bool readable_anywhere(const Operand16& o, int64_t rows, int64_t K) {
     return o.transposed() ? rows >= 8 && o.ld() >= rows : rows == 1 || o.ld() >= K;
 }
 
-// How gemm16_any computes the product of such operands, if it does.
+// How gemm16_any computes the product of such operands, if it does.  Whether it does is a matter of sizes and strides (the
+// caller copies the operands otherwise, and has no such way out later); the workspace only decides how.
 Small16 plan_anywhere(const Operand16& a, const Operand16& b, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace) {
     if (!readable_anywhere(a, M, K) || !readable_anywhere(b, N, K)) return Small16{};
-    return plan_any16(M, N, K, cus, workspace, plan16(a.transposed(), b.transposed(), M, N, K, cus, 0).large);
+    const double large = plan16(a.transposed(), b.transposed(), M, N, K, cus, 0).large;
+    const Small16 best = plan_any16(M, N, K, cus, INT64_MAX, large);
+    return best.kind == Small16::kNone || best.workspace <= workspace ? best : plan_any16(M, N, K, cus, workspace, 1e30);
 }
 
 // y[M, N] = a[M, K] . b[N, K]^T + bias in 16-bit elements.  `workspace` (may be null) for the sums of a split reduction;
@@ -692,17 +695,22 @@ extern "C" int ddl_gemm_in_place(int dtype, int aligned, int64_t a_row_stride, i
     return plan_anywhere(a, b, M, N, K, cus, INT64_MAX).kind != Small16::kNone;
 }
 
-extern "C" int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride, int64_t b_k_stride,
-                                      int64_t M, int64_t N, int64_t K) {
+extern "C" int64_t ddl_gemm_workspace_at(int dtype, int aligned, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride,
+                                         int64_t b_k_stride, int64_t M, int64_t N, int64_t K) {
     using namespace ddl;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     int dev = 0;
     const int cus = compute_units(dev);
-    if (dtype == DDL_DT_F32) return plan32(true, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, INT64_MAX).workspace;
+    if (dtype == DDL_DT_F32) return plan32(aligned != 0, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, INT64_MAX).workspace;
     if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return 0;
     const Operand16 a{nullptr, a_row_stride, a_k_stride}, b{nullptr, b_row_stride, b_k_stride};
-    if (pitches_ok(a, M, K) && pitches_ok(b, N, K)) return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;
+    if (aligned && pitches_ok(a, M, K) && pitches_ok(b, N, K)) return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;
     return plan_anywhere(a, b, M, N, K, cus, INT64_MAX).workspace;
+}
+
+extern "C" int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride, int64_t b_k_stride,
+                                      int64_t M, int64_t N, int64_t K) {
+    return ddl_gemm_workspace_at(dtype, 1, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K);
 }
 
 extern "C" int ddl_gemm_ws(const void* a, int64_t a_row_stride, int64_t a_k_stride, const void* b, int64_t b_row_stride, int64_t b_k_stride,

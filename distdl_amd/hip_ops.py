@@ -756,9 +756,10 @@ def _padded_k(t, k8):
 
 
 @functools.lru_cache(maxsize=4096)
-def _gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k):
-    """Floats a product of these sizes and strides can use for partial sums (a function of its arguments alone)."""
-    return _lib.load().ddl_gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k)
+def _gemm_workspace(dt, aligned, a_row, a_k, b_row, b_k, m, n, k):
+    """Floats a product of these sizes and strides (and alignment) can use for partial sums (a function of its arguments
+    alone)."""
+    return _lib.load().ddl_gemm_workspace_at(dt, aligned, a_row, a_k, b_row, b_k, m, n, k)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -770,9 +771,10 @@ def _gemm_in_place(dt, aligned, a_row, a_k, b_row, b_k, m, n, k):
 
 def _gemm(a, a_row, a_k, b, b_row, b_k, bias, out, dt, m, n, k):
     """``out[m, n] = sum_k a b + bias`` on operands addressed by two strides each; ``out`` is contiguous."""
-    elems = _gemm_workspace(dt, a_row, a_k, b_row, b_k, m, n, k)
+    pa, pb = a.data_ptr(), b.data_ptr()
+    elems = _gemm_workspace(dt, (pa | pb) % 16 == 0, a_row, a_k, b_row, b_k, m, n, k)
     work = torch.empty(elems, dtype=torch.float32, device=out.device) if elems else None
-    rc = _lib.load().ddl_gemm_ws(a.data_ptr(), a_row, a_k, b.data_ptr(), b_row, b_k, _ptr(bias), out.data_ptr(), dt, n, m, n, k,
+    rc = _lib.load().ddl_gemm_ws(pa, a_row, a_k, pb, b_row, b_k, _ptr(bias), out.data_ptr(), dt, n, m, n, k,
                                  _ptr(work), elems, _stream())
     _lib.check(rc, "ddl_gemm")
 
@@ -877,9 +879,10 @@ def colsum_bf16(a):
 
 
 @functools.lru_cache(maxsize=4096)
-def _linear_backward_workspace(dt, m, n, k, ld_x, ld_w, ld_dy, need_input, need_weight, need_bias):
-    """Floats the adjoint of these sizes and pitches can use (a function of its arguments alone)."""
-    return _lib.load().ddl_linear_backward_workspace(dt, m, n, k, ld_x, ld_w, ld_dy, bool(need_input), bool(need_weight), bool(need_bias))
+def _linear_backward_workspace(dt, aligned, m, n, k, ld_x, ld_w, ld_dy, need_input, need_weight, need_bias):
+    """Floats the adjoint of these sizes and pitches (and alignment) can use (a function of its arguments alone)."""
+    return _lib.load().ddl_linear_backward_workspace_at(dt, aligned, m, n, k, ld_x, ld_w, ld_dy, bool(need_input), bool(need_weight),
+                                                        bool(need_bias))
 
 
 def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, need_bias=True):
@@ -933,9 +936,10 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
             dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
         if need_bias:
             db = torch.empty(n, dtype=x.dtype, device=x.device)
-        elems = _linear_backward_workspace(dt, m, n, k, ld_x, ld_w, ld_dy, need_input, need_weight, need_bias)
+        px, pw, pdy = x2.data_ptr(), weight.data_ptr(), dy.data_ptr()
+        elems = _linear_backward_workspace(dt, (px | pw | pdy) % 16 == 0, m, n, k, ld_x, ld_w, ld_dy, need_input, need_weight, need_bias)
         work = torch.empty(elems, dtype=torch.float32, device=x.device) if elems else None
-        rc = _lib.load().ddl_linear_backward(x2.data_ptr(), weight.data_ptr(), dy.data_ptr(), _ptr(dx), _ptr(dw), _ptr(db), dt, m, n, k,
+        rc = _lib.load().ddl_linear_backward(px, pw, pdy, _ptr(dx), _ptr(dw), _ptr(db), dt, m, n, k,
                                              ld_x, ld_w, ld_dy, _ptr(work), elems, _stream())
         _lib.check(rc, "ddl_linear_backward")
         return dx, dw, db

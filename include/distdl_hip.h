@@ -507,16 +507,20 @@ int ddl_gemm(const void* a, int64_t a_row_stride, int64_t a_k_stride,
              int64_t M, int64_t N, int64_t K, void* stream);
 /* ddl_gemm with room for the partial sums of a reduction that is split over
  * workgroups: `workspace` (16-byte aligned, may be null) holds
- * `workspace_elems` floats, as many as ddl_gemm_workspace says for the fastest
+ * `workspace_elems` floats, as many as ddl_gemm_workspace_at says for the fastest
  * way (0: none needed; with fewer, a way that needs no more is taken).  Its
  * contents on entry do not matter; the result is the same up to the order of
  * the fp32 sums.  16-bit operands that ddl_gemm refuses for their alignment are
- * taken as they are where ddl_gemm_in_place says 1 (`aligned`: both start on 16
- * bytes): one unit stride, the other at least the length of a row or line, and
- * for an operand contiguous along its rows at least eight of them. */
+ * taken as they are where ddl_gemm_in_place says 1, whatever the workspace: one
+ * unit stride, the other at least the length of a row or line, and for an operand
+ * contiguous along its rows at least eight of them.  `aligned`: both operands start
+ * on 16 bytes (ddl_gemm_workspace: they do). */
 int ddl_gemm_in_place(int dtype, int aligned, int64_t a_row_stride,
                       int64_t a_k_stride, int64_t b_row_stride,
                       int64_t b_k_stride, int64_t M, int64_t N, int64_t K);
+int64_t ddl_gemm_workspace_at(int dtype, int aligned, int64_t a_row_stride,
+                              int64_t a_k_stride, int64_t b_row_stride,
+                              int64_t b_k_stride, int64_t M, int64_t N, int64_t K);
 int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride,
                            int64_t b_row_stride, int64_t b_k_stride, int64_t M,
                            int64_t N, int64_t K);
@@ -528,7 +532,12 @@ int ddl_gemm_ws(const void* a, int64_t a_row_stride, int64_t a_k_stride,
 /* The adjoint of ddl_linear in one call, on operands that ddl_gemm_ws can read
  * where they lie (row pitches ldx, ldw, lddy; dx, dw and db contiguous): dx, dw
  * and db may each be NULL.  `workspace` as for ddl_gemm_ws, with as many floats
- * as ddl_linear_backward_workspace says for those wanted. */
+ * as ddl_linear_backward_workspace_at says for those wanted (`aligned`: x, w and dy
+ * all start on 16 bytes; ddl_linear_backward_workspace: they do). */
+int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int64_t M,
+                                         int64_t N, int64_t K, int64_t ldx,
+                                         int64_t ldw, int64_t lddy, int want_dx,
+                                         int want_dw, int want_db);
 int64_t ddl_linear_backward_workspace(int dtype, int64_t M, int64_t N, int64_t K,
                                       int64_t ldx, int64_t ldw, int64_t lddy,
                                       int want_dx, int want_dw, int want_db);

@@ -1675,6 +1675,40 @@ def test_gemm_16_bit_operands_at_any_pitch(ops, dtype, a_t, b_t, M, N, K, pad):
         assert (got[:, N:] == 77.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(8, 64, 32768), (2, 128, 28672), (1, 8, 57344), (8, 3584, 8192), (64, 256, 4096)])
+def test_linear_of_operands_off_a_16_byte_boundary(ops, dtype, M, N, K):
+    """x one element into its buffer, pitches that are multiples of eight: the product and its adjoint through the front end,
+    which sizes the workspace, and the product with that workspace, half of it and none.  Integers, every sum is exact."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(M + N + K)
+    x = torch.randint(-1, 2, (M, K), generator=gen).to(dtype)
+    w = (torch.randint(-1, 2, (N, K), generator=gen) * (torch.rand(N, K, generator=gen) < 64.0 / K)).to(dtype)
+    dy = torch.randint(-1, 2, (M, N), generator=gen) * (torch.rand(M, N, generator=gen) < min(1.0, 64.0 / N))
+    dy = dy.to(dtype)
+
+    def shifted(t):
+        return torch.empty(t.numel() + 1, dtype=dtype, device="cuda")[1:].copy_(t.reshape(-1)).view(t.shape)
+    xg, wg, dyg = shifted(x), w.cuda(), shifted(dy)
+    assert xg.data_ptr() % 16 == 2
+    want = x.double() @ w.double().T
+    assert torch.equal(ops.linear(xg, wg).cpu().double(), want)
+    dx, dw, db = ops.linear_backward(xg, wg, dyg)
+    assert torch.equal(dx.cpu().double(), dy.double() @ w.double())
+    assert torch.equal(dw.cpu().double(), dy.double().T @ x.double())
+    assert torch.equal(db.cpu().double(), dy.double().sum(0))
+    lib, dt = _lib.load(), _lib.DDL_DT_BF16 if dtype == torch.bfloat16 else _lib.DDL_DT_F16
+    assert lib.ddl_gemm_in_place(dt, 0, K, 1, K, 1, M, N, K) == 1
+    elems = lib.ddl_gemm_workspace_at(dt, 0, K, 1, K, 1, M, N, K)
+    for n in {0, elems // 2, elems}:
+        work = torch.full((n,), float("nan"), device="cuda") if n else None
+        out = torch.full((M, N), 77.0, dtype=dtype, device="cuda")
+        rc = lib.ddl_gemm_ws(xg.data_ptr(), K, 1, wg.data_ptr(), K, 1, None, out.data_ptr(), dt, N, M, N, K,
+                             None if work is None else work.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "ddl_gemm_ws")
+        assert torch.equal(out.cpu().double(), want)
+
+
 @pytest.mark.parametrize("a_t,b_t", [(False, True), (True, True)])
 def test_gemm_16_bit_random_within_tolerance_and_ragged_depth(ops, a_t, b_t):
     """Random operands, a reduction length that is no multiple of the k-tile

@@ -873,3 +873,18 @@ def test_relayouts_along_an_axis_the_tensor_has_not_are_refused(monkeypatch, rel
         getattr(all_gather, relayout)(P, torch.zeros(2, 4, 6), axis, None)
     out = getattr(all_gather, relayout)(P, torch.zeros(2, 4, 6), -1, None)
     assert tuple(out.shape) == ((2, 4, 12) if relayout == "gather_slabs" else (2, 4, 3))
+
+
+def test_gemm_workspace_follows_the_alignment_of_the_operands():
+    """The floats asked for are those of the way that will be taken: the kernel for operands off a 16-byte boundary splits
+    long reductions that the aligned ones do not, alone and inside the adjoint."""
+    lib, dt = _lib.load(), _lib.DDL_DT_BF16
+    for M, N, K in (8, 64, 32768), (2, 128, 28672), (8, 3584, 8192):
+        strides = (K, 1, K, 1, M, N, K)
+        assert lib.ddl_gemm_in_place(dt, 0, *strides) == 1
+        assert lib.ddl_gemm_workspace_at(dt, 1, *strides) == lib.ddl_gemm_workspace(dt, *strides) == 0
+        assert lib.ddl_gemm_workspace_at(dt, 0, *strides) > 0
+        # dx[M, K'] with K' = 64: a reduction over N' = K down w's columns
+        backward = (M, K, N, N, N, K, 1, 0, 0)
+        unaligned = lib.ddl_gemm_workspace_at(dt, 0, K, 1, 1, N, M, N, K)
+        assert lib.ddl_linear_backward_workspace_at(dt, 0, *backward) == max(unaligned, lib.ddl_linear_backward_workspace(dt, *backward))
