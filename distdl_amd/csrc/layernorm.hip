@@ -18,7 +18,8 @@
 //   workgroup rows  up to 16384 columns: a 256-thread workgroup owns a row, still
 //                   in registers (up to 16 pieces of four per thread), sums go
 //                   through the wavefronts and four words of LDS
-//   streamed rows   anything longer: a workgroup walks the row once per reduction
+//   streamed rows   anything longer, and more rows than one launch has wavefronts for: a
+//                   workgroup walks the row once per reduction
 // Rows whose length, pitch or address are no multiples of four elements are held in
 // the same way; only the end of such a row is fetched element by element.
 #include "ddl_common.h"
@@ -402,10 +403,12 @@ int launch_held(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
 template <typename T, int MODE, bool AFFINE>
 int launch_typed(const LnArgs& a, const PartCounts& pc, bool vec, hipStream_t s) {
     const int cols = a.cols;
-    if (vec && cols <= kBlockRowCols) return launch_held<T, MODE, AFFINE, false>(a, pc, s);
+    // A launch has fewer than 2^32 threads, which wavefront rows (one or two per wavefront) use up; streamed rows do not.
+    const bool one_launch = cols > kWaveRowCols || (cols > 512 ? a.rows : (a.rows + 1) / 2) * kWave <= 0xFFFFFF00ll;
+    if (vec && cols <= kBlockRowCols && (one_launch || MODE == kJoined)) return launch_held<T, MODE, AFFINE, false>(a, pc, s);
     if constexpr (MODE != kJoined) {
         // Rows that start at any element: held as well, instead of read element by element once per reduction.
-        if (cols <= kBlockRowCols) return launch_held<T, MODE, AFFINE, true>(a, pc, s);
+        if (cols <= kBlockRowCols && one_launch) return launch_held<T, MODE, AFFINE, true>(a, pc, s);
     }
     if constexpr (MODE == kJoined) {
         return fail(DDL_E_UNSUPP, "ln stats+normalize: rows of more than %d columns take the two-launch form", kBlockRowCols);

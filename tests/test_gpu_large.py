@@ -190,3 +190,23 @@ def test_linear_backward_rows_beyond_2_31_elements(ops):
     assert float((dw.float() - want_dw).abs().max()) <= 2e-2 * float(want_dw.abs().max())
     want_db = dy.float().sum(0)
     assert float((db.float() - want_db).abs().max()) <= 2e-2 * float(want_db.abs().max())
+
+
+def test_layer_norm_of_more_short_rows_than_one_launch_has_wavefronts_for(ops):
+    """2^27 + 5 rows of 3 bf16 columns: two rows per wavefront would be more than 2^32 threads.  Every row, in fp32 by torch,
+    within one rounding of the result and the difference of two fp32 means (1e-6 of elements up to 6) at the largest
+    1 / sqrt(eps) x gamma (32 x 4, twice)."""
+    rows, cols = 2 ** 27 + 5, 3
+    gen = torch.Generator(device="cuda").manual_seed(27)
+    x = torch.randn(rows, cols, device="cuda", generator=gen, dtype=torch.bfloat16)
+    gamma, beta = (torch.randn(cols, device="cuda", generator=gen, dtype=torch.bfloat16) for _ in range(2))
+    y = ops.layer_norm(x, gamma, beta, 1e-3)
+    stats = ops.ln_partial_stats(x)
+    for lo in range(0, rows, 2 ** 25):
+        hi = min(rows, lo + 2 ** 25)
+        v = x[lo:hi].float()
+        mean = v.mean(1, keepdim=True)
+        sq = ((v - mean) ** 2).sum(1, keepdim=True)
+        want = (v - mean) * (sq / cols + 1e-3).rsqrt() * gamma.float() + beta.float()
+        assert bool(((y[lo:hi].float() - want).abs() <= 2.0 ** -8 * want.abs() + 3e-4).all())
+        assert bool(((stats[lo:hi] - torch.cat((mean, sq), 1)).abs() <= 1e-5 * (1 + sq)).all())
