@@ -300,8 +300,10 @@ extern "C" int ddl_transpose_2d(const void* src, void* dst, int64_t rows, int64_
 
 namespace ddl {
 
-// Up to 128 KiB per workgroup of 16 columns: about 4 us on one CU.
-bool colsum_in_one_launch(int64_t rows, int64_t elem_size) { return rows * kNarrow * elem_size <= 131072; }
+// Up to 128 KiB per workgroup of 16 columns: about 4 us on one CU; and fewer than the 2^32 threads a launch may have.
+bool colsum_in_one_launch(int64_t rows, int64_t cols, int64_t elem_size) {
+    return rows <= 131072 / (kNarrow * elem_size) && (cols + kNarrow - 1) / kNarrow <= 0xFFFFFFFFll / kOneBlock;
+}
 
 }  // namespace ddl
 
@@ -312,7 +314,7 @@ template <int DT>
 int run_colsum(const void* a, int64_t rows, int64_t cols, int64_t ld, void* out, float* workspace, int64_t splits,
                int64_t rows_per_split, int64_t strips, hipStream_t s) {
     typedef typename Elem<DT>::type T;
-    if (colsum_in_one_launch(rows, sizeof(T))) {
+    if (colsum_in_one_launch(rows, cols, sizeof(T))) {
         const dim3 grid(static_cast<uint32_t>((cols + kNarrow - 1) / kNarrow));
         if (aligned_to(a, 16) && (ld * sizeof(T)) % 16 == 0)
             hipLaunchKernelGGL((colsum_one_kernel<DT, true>), grid, dim3(kOneBlock), 0, s, static_cast<const T*>(a), rows, cols, ld, static_cast<T*>(out));
@@ -340,7 +342,7 @@ extern "C" int ddl_colsum(const void* a, int dtype, int64_t rows, int64_t cols, 
     if (rows < 0 || cols < 0 || ld < cols) return fail(DDL_E_ARG, "colsum: rows=%lld cols=%lld ld=%lld", (long long)rows, (long long)cols, (long long)ld);
     if (cols == 0) return 0;
     const int es = dtype == DDL_DT_F32 ? 4 : 2;
-    const bool one_launch = colsum_in_one_launch(rows, es);
+    const bool one_launch = colsum_in_one_launch(rows, cols, es);
     if (!out || (!workspace && !one_launch) || (rows > 0 && !a)) return fail(DDL_E_ARG, "colsum: null pointer");
     if (!aligned_to(a, es) || !aligned_to(out, es) || !aligned_to(workspace, 4)) return fail(DDL_E_ALIGN, "colsum: pointer misaligned");
     // as many row splits as the workspace holds, up to 64 and to 128 rows per split
@@ -369,7 +371,7 @@ extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int6
         if (want_dx) take(ddl_gemm_workspace_at(dtype, both, lddy, 1, 1, ldw, M, K, N));
         if (want_dw) take(ddl_gemm_workspace_at(dtype, both, 1, lddy, 1, ldx, N, K, M));
     }
-    if (want_db && !ddl::colsum_in_one_launch(M, dtype == DDL_DT_F32 ? 4 : 2)) {
+    if (want_db && !ddl::colsum_in_one_launch(M, N, dtype == DDL_DT_F32 ? 4 : 2)) {
         const int64_t splits = (M + 127) / 128;
         take((splits < 64 ? splits : 64) * N);
     }

@@ -210,3 +210,11 @@ def test_layer_norm_of_more_short_rows_than_one_launch_has_wavefronts_for(ops):
         want = (v - mean) * (sq / cols + 1e-3).rsqrt() * gamma.float() + beta.float()
         assert bool(((y[lo:hi].float() - want).abs() <= 2.0 ** -8 * want.abs() + 3e-4).all())
         assert bool(((stats[lo:hi] - torch.cat((mean, sq), 1)).abs() <= 1e-5 * (1 + sq)).all())
+
+
+def test_column_sums_of_more_columns_than_one_launch_has_threads_for(ops):
+    """Small integers: every sum is exact."""
+    rows, cols = 3, 2 ** 26 + 21
+    a = torch.randint(-20, 21, (rows, cols), device="cuda", dtype=torch.int8)
+    got = ops.colsum(a.to(torch.bfloat16))
+    assert torch.equal(got, a.sum(0, dtype=torch.int32).to(torch.bfloat16))

@@ -888,3 +888,14 @@ def test_gemm_workspace_follows_the_alignment_of_the_operands():
         backward = (M, K, N, N, N, K, 1, 0, 0)
         unaligned = lib.ddl_gemm_workspace_at(dt, 0, K, 1, 1, N, M, N, K)
         assert lib.ddl_linear_backward_workspace_at(dt, 0, *backward) == max(unaligned, lib.ddl_linear_backward_workspace(dt, *backward))
+
+
+def test_column_sums_of_more_columns_than_one_launch_has_threads_for_take_two():
+    """64 threads per column: from 2^26 columns on the one launch would have 2^32 threads, and the two-launch form needs its
+    partial sums."""
+    lib = _lib.load()
+    for dt, rows in (_lib.DDL_DT_F32, 2048), (_lib.DDL_DT_BF16, 4096):
+        for cols, floats in (2 ** 26 - 16, 0), (2 ** 26 - 15, 2 ** 26 - 15):
+            assert lib.ddl_linear_backward_workspace(dt, 8, cols, 1, 1, 1, cols, 0, 0, 1) == floats
+        assert lib.ddl_linear_backward_workspace(dt, rows, 64, 1, 1, 1, 64, 0, 0, 1) == 0
+        assert lib.ddl_linear_backward_workspace(dt, rows + 1, 64, 1, 1, 1, 64, 0, 0, 1) == -(-(rows + 1) // 128) * 64
