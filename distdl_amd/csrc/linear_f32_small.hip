@@ -294,7 +294,7 @@ Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace
     double best_us = other_us * 0.95;   // what the fits are unsure of
     for (const int groups : {1, 2, 4}) {
         const int64_t bm = groups == 1 ? 64 : 32, bn = groups == 4 ? 32 : 64, tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        if (tiles > 0x7FFFFFF) continue;
+        if (tiles > 0xFFFFFF) continue;   // a launch has fewer than 2^32 threads, 256 per tile
         for (const int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
             if (splits > 1 && (tiles * splits > 4 * static_cast<int64_t>(cus) || ktiles < 2 * splits * groups || tiles * splits * bm * bn > workspace)) break;
             const int64_t per_cu = (tiles * splits + cus - 1) / cus, kt = (ktiles + splits - 1) / splits;

@@ -218,3 +218,11 @@ def test_column_sums_of_more_columns_than_one_launch_has_threads_for(ops):
     a = torch.randint(-20, 21, (rows, cols), device="cuda", dtype=torch.int8)
     got = ops.colsum(a.to(torch.bfloat16))
     assert torch.equal(got, a.sum(0, dtype=torch.int32).to(torch.bfloat16))
+
+
+def test_linear_of_more_rows_than_small_tiles_have_workgroups_for(ops):
+    """2^30 + 3 rows of one fp32 column: 2^24 tiles of 64 rows would be 2^32 threads.  One product per row, exact."""
+    x = torch.randn(2 ** 30 + 3, 1, device="cuda")
+    w = torch.full((1, 1), 1.5, device="cuda")
+    y = ops.linear(x, w)
+    assert y.shape == x.shape and torch.equal(y, x.mul_(1.5))
