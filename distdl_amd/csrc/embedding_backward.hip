@@ -237,20 +237,23 @@ struct ReduceArgs {
 // flight.  (A wavefront that walks its columns alone keeps 32 in flight in the
 // same registers: 55 us instead of 20 for 483 tokens of 2 KiB.)
 // The order of the tokens: up to 512 by counting the smaller ones, more through
-// a bit per token number in LDS (the stage's 16 KiB hold 131072 of them) that is
-// read back in ascending order, kListTokens at a time.
+// a bit per token number in LDS (16 KiB for a window of 131072 of them) that is
+// read back in ascending order, kListTokens at a time.  The bits have LDS of their
+// own: in the stage's they had to be set again, by a walk over the whole bucket,
+// for every kListTokens (2^20 tokens of one row, 256 bytes each: 1267 ms, now 59).
 constexpr int kHotAbove = 32;                        // rows of more tokens are hot: what half a wavefront's lanes order, and as long as
                                                      // the ordinary walk stays below the time of everything else (with 64: 24 us, with 32: 17)
 constexpr int kHotBytes = 256;
 constexpr int kHotBatch = 64;                        // tokens per batch
 constexpr int kListTokens = 1024;
 constexpr int kRankTokens = 2 * kBlock;
-constexpr int kBitWords = kHotBytes * kHotBatch / 4;
+constexpr int kBitWords = 4096;
 constexpr int kBitsPerWindow = kBitWords * 32;
 constexpr int kWordsPerThread = kBitWords / kBlock;
 
 struct HotShared {
-    uint32_t bits[kBitWords];                        // pieces of a batch, a bit per token number, or the bucket being ordered
+    uint32_t pieces[kHotBytes * kHotBatch / 4];      // of a batch
+    uint32_t bits[kBitWords];                        // a bit per token number, or the bucket being ordered
     int32_t list[kListTokens];                       // tokens in ascending order
     int32_t wave_total[kWavesPerBlock];
 };
@@ -285,7 +288,7 @@ __device__ inline void hot_accumulate(HotShared& sh, const ReduceArgs& a, int64_
     auto batch = [&](uint4 (&from)[kLoads], int base) {
 #pragma unroll
         for (int u = 0; u < kLoads; ++u)
-            *reinterpret_cast<uint4*>(&sh.bits[(u * kTokensPerLoad + tok0) * (kHotBytes / 4) + part * 4]) = from[u];
+            *reinterpret_cast<uint4*>(&sh.pieces[(u * kTokensPerLoad + tok0) * (kHotBytes / 4) + part * 4]) = from[u];
         __syncthreads();
         if (base + 2 * kHotBatch < m) fetch(from, base + 2 * kHotBatch);
         if (t < kWave) {
@@ -302,11 +305,11 @@ __device__ inline void hot_accumulate(HotShared& sh, const ReduceArgs& a, int64_
             for (; k + 16 <= here; k += 16) {
                 uint32_t w[16];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) w[u] = sh.bits[(k + u) * (kHotBytes / 4) + t];
+                for (int u = 0; u < 16; ++u) w[u] = sh.pieces[(k + u) * (kHotBytes / 4) + t];
 #pragma unroll
                 for (int u = 0; u < 16; ++u) add(w[u]);
             }
-            for (; k < here; ++k) add(sh.bits[k * (kHotBytes / 4) + t]);
+            for (; k < here; ++k) add(sh.pieces[k * (kHotBytes / 4) + t]);
         }
         __syncthreads();
     };
@@ -347,44 +350,47 @@ __device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, 
     } else {
         const int lane = t & (kWave - 1), wave = t / kWave;
         for (int64_t w0 = 0; w0 < a.n_ids; w0 += kBitsPerWindow) {
-            for (int32_t first = 0, in_window = 1; first < in_window; first += kListTokens) {
-                for (int i = t; i < kBitWords; i += kBlock) sh.bits[i] = 0;
-                __syncthreads();
-                for (int32_t i = t; i < n; i += kBlock) {
-                    const int64_t at = bucket[i] - w0;
-                    if (at >= 0 && at < kBitsPerWindow) atomicOr(&sh.bits[at >> 5], 1u << (at & 31));
-                }
-                __syncthreads();
-                int32_t mine = 0;
-                for (int k = 0; k < kWordsPerThread; ++k) mine += __popc(sh.bits[t * kWordsPerThread + k]);
-                int32_t incl = mine;
+            for (int i = t; i < kBitWords; i += kBlock) sh.bits[i] = 0;
+            __syncthreads();
+#pragma unroll 4
+            for (int32_t i = t; i < n; i += kBlock) {
+                const int64_t at = bucket[i] - w0;
+                if (at >= 0 && at < kBitsPerWindow) atomicOr(&sh.bits[at >> 5], 1u << (at & 31));
+            }
+            __syncthreads();
+            int32_t mine = 0;
+            for (int k = 0; k < kWordsPerThread; ++k) mine += __popc(sh.bits[t * kWordsPerThread + k]);
+            int32_t incl = mine;
 #pragma unroll
-                for (int off = 1; off < kWave; off <<= 1) {
-                    const int32_t up = __shfl_up(incl, off, kWave);
-                    if (lane >= off) incl += up;
-                }
-                if (lane == kWave - 1) sh.wave_total[wave] = incl;
-                __syncthreads();
-                int32_t rank = incl - mine;
-                in_window = 0;
+            for (int off = 1; off < kWave; off <<= 1) {
+                const int32_t up = __shfl_up(incl, off, kWave);
+                if (lane >= off) incl += up;
+            }
+            if (lane == kWave - 1) sh.wave_total[wave] = incl;
+            __syncthreads();
+            int32_t rank0 = incl - mine, in_window = 0;
 #pragma unroll
-                for (int k = 0; k < kWavesPerBlock; ++k) {
-                    rank += k < wave ? sh.wave_total[k] : 0;
-                    in_window += sh.wave_total[k];
-                }
-                for (int k = 0; k < kWordsPerThread; ++k) {
-                    uint32_t bits = sh.bits[t * kWordsPerThread + k];
-                    while (bits) {
-                        const int b = __ffs(bits) - 1;
-                        bits &= bits - 1;
-                        if (rank >= first && rank < first + kListTokens)
-                            sh.list[rank - first] = static_cast<int32_t>(w0) + (t * kWordsPerThread + k) * 32 + b;
-                        ++rank;
+            for (int k = 0; k < kWavesPerBlock; ++k) {
+                rank0 += k < wave ? sh.wave_total[k] : 0;
+                in_window += sh.wave_total[k];
+            }
+            for (int32_t first = 0; first < in_window; first += kListTokens) {   // the same in all threads
+                if (rank0 < first + kListTokens && rank0 + mine > first) {
+                    int32_t rank = rank0;
+                    for (int k = 0; k < kWordsPerThread; ++k) {
+                        uint32_t bits = sh.bits[t * kWordsPerThread + k];
+                        while (bits) {
+                            const int b = __ffs(bits) - 1;
+                            bits &= bits - 1;
+                            if (rank >= first && rank < first + kListTokens)
+                                sh.list[rank - first] = static_cast<int32_t>(w0) + (t * kWordsPerThread + k) * 32 + b;
+                            ++rank;
+                        }
                     }
                 }
                 __syncthreads();
                 const int32_t here = in_window - first;
-                if (here > 0) hot_accumulate<E>(sh, a, col0, here < kListTokens ? here : kListTokens, acc);
+                hot_accumulate<E>(sh, a, col0, here < kListTokens ? here : kListTokens, acc);
             }
         }
     }

@@ -1114,6 +1114,28 @@ def test_embedding_backward_bucket_lengths(ops, dtype, dim, misses):
     assert torch.equal(got.cpu(), want.to(dtype))
 
 
+def test_embedding_backward_of_one_row_takes_time_in_proportion_to_its_tokens(ops):
+    """Every token the same id: exact sums (small integers), and four times the tokens take about four times as long (4.5
+    measured; ordering the bucket anew for every 1024 of its tokens made it 22)."""
+    dy = torch.randint(-3, 4, (2 ** 20, 16), device="cuda", generator=torch.Generator(device="cuda").manual_seed(20)).float()
+    ids = torch.full((2 ** 20,), 7, device="cuda")
+    took = []
+    for n in (2 ** 18, 2 ** 20):
+        times = []
+        for _ in range(3):
+            start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            dw = ops.embedding_backward(dy[:n], ids[:n], 0, 9)
+            stop.record()
+            stop.synchronize()
+            times.append(start.elapsed_time(stop))
+        took.append(min(times))
+        want = torch.zeros(9, 16, device="cuda")
+        want[7] = dy[:n].double().sum(0).float()
+        assert torch.equal(dw, want)
+    assert took[1] < 10 * took[0], took
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_embedding_backward_scale_grad_by_freq(ops, dtype):
     """Each row's sum divided by its number of contributing tokens, against the
