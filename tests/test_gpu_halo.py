@@ -560,6 +560,55 @@ def test_buffer_manager_shared_by_a_network_of_layers(repartitions_share_the_man
     _adjoint_tight([r[1:] for r in res])
 
 
+def test_buffer_manager_shared_by_halo_exchanges_and_repartitions(ops):
+    """A scatter, three halo exchanges of different widths over a 2x2 partition and a gather with one buffer manager, four
+    workers moving real data: pooled buffers after every layer, values forward and backward against the oracle's exchanges
+    (integers, so that the adjoint's sums are exact)."""
+    from distdl_amd.backends.stub_hip import BufferManager
+    from distdl_amd.backends.stub_hip import SimWorld
+    from distdl_amd.nn import HaloExchange
+    from distdl_amd.nn import Repartition
+    from distdl_amd.utilities.torch import zero_volume_tensor
+    gen = torch.Generator().manual_seed(22)
+    x0, dy0 = (torch.randint(-9, 10, (1, 3, 12, 14), generator=gen).float() for _ in range(2))
+    P, indices = [1, 1, 2, 2], [(0, 0, i, j) for i in range(2) for j in range(2)]
+
+    def widths(index, w):
+        return np.array([[0, 0], [0, 0]] + [[w * (i > 0), w * (i < 1)] for i in index[2:]])
+
+    def body(P_world):
+        manager = BufferManager()
+        P_1 = P_world.create_partition_inclusive([0]).create_cartesian_topology_partition([1, 1, 1, 1])
+        P_22 = P_world.create_partition_inclusive([0, 1, 2, 3]).create_cartesian_topology_partition(P)
+        layers = [Repartition(P_1, P_22, buffer_manager=manager)]
+        for w in (1, 2, 1):
+            mine = widths(tuple(int(i) for i in P_22.index), w)
+            layers.append(HaloExchange(P_22, mine, mine, mine, buffer_manager=manager))
+        layers.append(Repartition(P_22, P_1, buffer_manager=manager))
+        x = (x0.cuda() if P_1.active else zero_volume_tensor(1, device="cuda")).requires_grad_(True)
+        h, counts = x, []
+        for layer in layers:
+            h = layer(h)
+            counts.append(len(manager.buffers_map.get(torch.float32, [])))
+        h.backward(dy0.cuda() if P_1.active else zero_volume_tensor(1, device="cuda"))
+        torch.cuda.synchronize()
+        return counts, h.detach().cpu().numpy(), x.grad.cpu().numpy()
+
+    res = SimWorld(4).run(body)
+    assert [counts for counts, _, _ in res] == [[3, 4, 4, 4, 4]] + 3 * [[1, 4, 4, 4, 4]]
+    y = dict(zip(indices, o_rep.scatter(x0.numpy(), P)))
+    dx = dict(zip(indices, o_rep.scatter(dy0.numpy(), P)))
+    for w in (1, 2, 1):
+        each = {i: widths(i, w).tolist() for i in indices}
+        y = o_halo.forward_all(y, P, each, each)
+    for w in (1, 2, 1):
+        each = {i: widths(i, w).tolist() for i in indices}
+        dx = o_halo.adjoint_all(dx, P, each, each)
+    for got, parts in ((res[0][1], y), (res[0][2], dx)):
+        for part, i in zip(o_rep.scatter(got, P), indices):
+            assert np.array_equal(part, parts[i])
+
+
 K2S2_1D = {"id": "kernel-2-stride-2-1d", "P_x_shape": [1, 1, 4], "x_global_shape": [1, 1, 10], "kernel_size": [2],
            "stride": [2], "padding": [0], "dilation": [1]}
 
