@@ -120,14 +120,14 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     // buffers that start at the tile's first row: a 32-bit byte offset per lane,
     // the k-tile offset in a scalar.
     //
-    // Operand16 contiguous along k: instruction j of this wavefront fills rows
+    // Operand contiguous along k: instruction j of this wavefront fills rows
     // (J wave + j) 8 .. +7 of an operand tile (J instructions per wavefront);
     // lane l lands on row l / 8, physical chunk l % 8 of that row, i.e. logical
     // chunk (l % 8) ^ ((row >> 1) & 7): the eight lanes of a row fetch one whole
     // 128-byte line.  Rows past the end of the matrix repeat its last row (their
     // products are never stored).
     //
-    // Operand16 contiguous along its rows ("transposed": element (row, k) lies at
+    // Operand contiguous along its rows ("transposed": element (row, k) lies at
     // k ld + row): the tile is kept in LDS as panels of 64 rows, each panel 64
     // k-lines of 128 bytes.  Instruction j of wavefront v fills k-lines 8 v .. +7
     // of panel j; lane l lands on k-line l / 8, physical chunk l % 8, and fetches
@@ -199,7 +199,7 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     const std::integral_constant<bool, WT> w_kind{};
     const std::integral_constant<bool, XT> x_kind{};
 
-    // Fragment addresses.  Operand16 contiguous along k: row (sub-tile origin +
+    // Fragment addresses.  Operand contiguous along k: row (sub-tile origin +
     // l16), logical chunk 4 ks + kg; sub-tile origins are multiples of 16, so the
     // swizzle term is (l16 >> 1) & 7.
     const int frag_row = l16 * (BK * 2);
