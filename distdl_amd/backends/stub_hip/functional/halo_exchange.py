@@ -101,14 +101,16 @@ class _Plan:
                                                              for b in (left, right)])
                 self.dims.append((extents, out, clear, adds))
         self.first = hip_ops.BoxLaunch(first, elem_size) if forward else None
+        self.adds = any(present[i][j] for i in range(dims) for j in bulk)
 
 
 def _plan(dims, slices, buffers, tensor, forward):
     cache = getattr(slices, "plans", None)
-    present = tuple([tuple([b is not None for b in sides]) for sides in buffers])
+    present = tuple([b is not None for sides in buffers for b in sides])
     key = (dims, forward, tensor.shape, tensor.stride(), tensor.element_size(), present)
     plan = None if cache is None else cache.get(key)
     if plan is None:
+        present = [[b is not None for b in sides] for sides in buffers]
         plan = _Plan(dims, slices, present, tuple(int(n) for n in tensor.shape), [int(s) for s in tensor.stride()],
                      tensor.element_size(), forward)
         if cache is not None:
@@ -116,20 +118,23 @@ def _plan(dims, slices, buffers, tensor, forward):
     return plan
 
 
-def _dim_views(buffers, extents, tensor, bases):
-    """The views of a dimension's four buffers; their addresses go into ``bases``."""
-    out = []
-    for buffer, extent in zip(buffers, extents):
-        if buffer is None:
-            out.append(None)
-            bases.append(0)
-            continue
-        view = buffer.get_view(extent)
-        hip_ops._require_gpu(view)
-        if view.dtype != tensor.dtype:
-            raise ValueError(f"buffer {tuple(view.shape)}/{view.dtype} does not match a tensor of {tensor.dtype}")
-        out.append(view)
-        bases.append(view.data_ptr())
+def _views(buffers, plan, tensor, bases):
+    """The views of every dimension's four buffers; their addresses go into ``bases``."""
+    out, dtype = [], tensor.dtype
+    for sides, dim in zip(buffers, plan.dims):
+        views = []
+        for buffer, extent in zip(sides, dim[0]):
+            if buffer is None:
+                views.append(None)
+                bases.append(0)
+                continue
+            view = buffer.get_view(extent)
+            if view.dtype != dtype:
+                raise ValueError(f"buffer {tuple(view.shape)}/{view.dtype} does not match a tensor of {dtype}")
+            views.append(view)
+            bases.append(view.data_ptr())
+        hip_ops._require_gpu(*views)
+        out.append(views)
     return out
 
 
@@ -173,7 +178,7 @@ class HaloExchangeFunction(torch.autograd.Function):
         output = torch.empty_like(src, memory_format=torch.contiguous_format)
         plan = _plan(P_x.dim, slices, buffers, src, True)
         bases = [src.data_ptr(), output.data_ptr()]
-        views = [_dim_views(row, dim[0], output, bases) for row, dim in zip(buffers, plan.dims)]
+        views = _views(buffers, plan, output, bases)
         plan.first.run(bases)
         for i, (lbb, lgb, rbb, rgb) in enumerate(views):
             _, pack, unpack = plan.dims[i]
@@ -198,9 +203,9 @@ class HaloExchangeFunction(torch.autograd.Function):
         hip_ops._require_gpu(grad_output)
         plan = _plan(P_x.dim, slices, buffers, grad_output, False)
         bases = [0, grad_output.data_ptr()]
-        views = [_dim_views(row, dim[0], grad_output, bases) for row, dim in zip(buffers, plan.dims)]
+        views = _views(buffers, plan, grad_output, bases)
         add_dtype = hip_ops._ADD_DTYPES.get(grad_output.dtype)
-        if add_dtype is None and any(lbb is not None or rbb is not None for lbb, _, rbb, _ in views):
+        if add_dtype is None and plan.adds:
             raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
         for i in reversed(range(len(views))):
             lbb, lgb, rbb, rgb = views[i]
