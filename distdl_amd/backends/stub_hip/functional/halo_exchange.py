@@ -12,6 +12,8 @@ launch), swap, ADD what arrives into the bulk.
 
 __all__ = ["HaloExchangeFunction"]
 
+import operator
+
 import torch
 
 from .... import _lib
@@ -53,13 +55,13 @@ class _Plan:
             for j in sides:
                 if not present[i][j]:
                     continue
-                box = slices[i][j]
-                for d, (s, n) in enumerate(zip(box, shape)):
-                    if not 0 <= s.start <= s.stop <= n:     # a shard narrower than its strips; the copies know no extents
-                        raise RuntimeError(f"halo strip {j} of dim {i}: [{s.start},{s.stop}) outside extent {n} of dim {d}")
-                extent = [int(s.stop) - int(s.start) for s in box]
+                start, stop = [int(s.start) for s in slices[i][j]], [int(s.stop) for s in slices[i][j]]
+                extent = list(map(operator.sub, stop, start))
+                if min(start) < 0 or min(extent) < 0 or any(map(operator.gt, stop, shape)):
+                    # a shard narrower than its strips; the copies know no extents
+                    raise RuntimeError(f"halo strip {j} of dim {i}, {list(zip(start, stop))}, is outside extents {tuple(shape)}")
                 own = strides if from_input else tensor_strides
-                offset = sum(int(s.start) * t for s, t in zip(box, own))
+                offset = sum(map(operator.mul, start, own))
                 packed = hip_ops.contiguous_strides(extent)
                 slot = 2 + 4 * i + j
                 if to_buffer:

@@ -5,6 +5,7 @@ into ``libdistdl_hip.so`` and raises when that is impossible.
 
 import ctypes
 import functools
+import struct
 
 import torch
 
@@ -154,6 +155,11 @@ def contiguous_strides(shape):
     return strides[::-1]
 
 
+# A box descriptor (ddl_box_t) in one piece: field by field through ctypes it takes ten times as long.
+_BOX = struct.Struct("PPii%dq" % (3 * _lib.DDL_MAX_DIMS))
+assert _BOX.size == ctypes.sizeof(_lib.ddl_box_t)
+
+
 class BoxLaunch:
     """The boxes of one ``ddl_copy_boxes`` call, lowered once.
 
@@ -164,18 +170,19 @@ class BoxLaunch:
     descriptors, so threads may share an object."""
 
     def __init__(self, entries, elem_size):
-        entries = [e for e in entries if all(int(n) > 0 for n in e[4])]
+        entries = [e for e in entries if min(e[4], default=1) > 0]
         self.elem_size = elem_size
         self.n = len(entries)
-        self._type = _lib.ddl_box_t * max(self.n, 1)
-        boxes = self._type()
-        self._bases = []
-        for i, (src, src_off, dst, dst_off, shape, src_strides, dst_strides) in enumerate(entries):
-            boxes[i].ndim = len(shape)
-            for d, (n, s, t) in enumerate(zip(shape, src_strides, dst_strides)):
-                boxes[i].shape[d], boxes[i].src_stride[d], boxes[i].dst_stride[d] = int(n), int(s), int(t)
+        self._type = _lib.ddl_box_t * self.n
+        self._bases, packed = [], []
+        for src, src_off, dst, dst_off, shape, src_strides, dst_strides in entries:
+            nd = len(shape)
+            if nd > _lib.DDL_MAX_DIMS:
+                raise ValueError(f"tensors of rank {nd} are not supported (1..{_lib.DDL_MAX_DIMS})")
+            rest = (0,) * (_lib.DDL_MAX_DIMS - nd)
+            packed.append(_BOX.pack(0, 0, nd, 0, *shape, *rest, *src_strides, *rest, *dst_strides, *rest))
             self._bases.append((src, int(src_off) * elem_size, dst, int(dst_off) * elem_size))
-        self._template = bytes(boxes)
+        self._template = b"".join(packed)
 
     def run(self, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
         if self.n == 0:

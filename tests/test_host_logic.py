@@ -727,7 +727,7 @@ def _halo_plan(shape, recv, send, forward, present=None):
 def test_halo_strips_outside_the_tensor_are_refused(shape, recv, send, forward):
     """Copies of boxes know addresses and strides only, so a strip that leaves the tensor has to be refused when the
     launches are built; strips that just fit are accepted."""
-    with pytest.raises(RuntimeError, match="outside extent"):
+    with pytest.raises(RuntimeError, match="outside extents"):
         _halo_plan(shape, recv, send, forward)
     _halo_plan(tuple(n + 8 for n in shape), recv, send, forward)
     _halo_plan((4, 4), [[0, 0], [2, 0]], [[0, 0], [2, 0]], forward)
