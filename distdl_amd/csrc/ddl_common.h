@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -20,6 +21,24 @@ int check_launch(const char* what);
 
 inline bool aligned_to(const void* p, uint64_t a) {
     return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
+}
+
+constexpr int kMaxDevices = 64;
+
+// Compute units of the current device (asked once per device; any thread may
+// get there first, the value is the same for all).  `dev` receives the device.
+inline int compute_units(int& dev) {
+    static std::atomic<int> cu_count[kMaxDevices];   // 0: not asked yet
+    dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) dev = 0;
+    int cus = cu_count[dev].load(std::memory_order_relaxed);
+    if (cus == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+        cus = n;
+        cu_count[dev].store(n, std::memory_order_relaxed);
+    }
+    return cus;
 }
 
 // Division of a 31-bit unsigned dividend by a fixed divisor as one multiply-high

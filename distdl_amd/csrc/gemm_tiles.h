@@ -15,7 +15,6 @@ constexpr int kUnitBytes = kMaxTileRows * kRowBytes;     // ring slot for one op
 constexpr int kUnits = 5;                                // ring of operand tiles: W0 X0 W1 X1 W2 | X2 W3 ...
 constexpr int kLdsBytes = kUnits * kUnitBytes;           // 160 KiB: all of a CU's LDS
 constexpr int kXcds = 8;
-constexpr int kMaxDevices = 64;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -82,22 +81,6 @@ __device__ inline void tile_of_workgroup(int id, int tiles_m, int tiles_n, int& 
     const int in_band = id - band * kBand * tiles_n;
     tm = band_m0 + in_band % band_h;
     tn = in_band / band_h;
-}
-
-// Compute units of the current device (asked once per device; any thread may
-// get there first, the value is the same for all).  `dev` receives the device.
-inline int compute_units(int& dev) {
-    static std::atomic<int> cu_count[kMaxDevices];   // 0: not asked yet
-    dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) dev = 0;
-    int cus = cu_count[dev].load(std::memory_order_relaxed);
-    if (cus == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-        cus = n;
-        cu_count[dev].store(n, std::memory_order_relaxed);
-    }
-    return cus;
 }
 
 // One workgroup per CU is resident, so the tiles run in rounds of one per CU

@@ -15,9 +15,9 @@
 //                   holds pieces of four elements, sums go through shuffle
 //                   butterflies; a long input keeps two rows per wavefront in
 //                   flight
-//   workgroup rows  up to 16384 columns: a 256-thread workgroup owns a row, still
-//                   in registers (up to 16 pieces of four per thread), sums go
-//                   through the wavefronts and four words of LDS
+//   workgroup rows  up to 16384 columns: a workgroup of 256 to 1024 threads owns
+//                   a row, still in registers, sums go through the wavefronts
+//                   and a word of LDS for each; it walks up to eight rows
 //   streamed rows   anything longer, and more rows than one launch has wavefronts for: a
 //                   workgroup walks the row once per reduction
 // Rows whose length, pitch or address are no multiples of four elements are held in
@@ -227,9 +227,159 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
 
 // --------------------------------------------------------- workgroup rows --
 
-// One workgroup per row, NV pieces of four per thread (cols <= 1024 NV); the grid
-// walks the rows.  ANY as above.
-template <typename T, int NV, int MODE, bool AFFINE, bool ANY>
+// V elements of a row as they lie in memory, 8 or 16 bytes; global memory takes them at the alignment of four elements.
+template <typename T, int V>
+struct RowPiece {
+    static_assert(V % 4 == 0, "pieces are quartets of elements");
+    struct __attribute__((packed, aligned(4 * sizeof(T)))) Raw {
+        uint32_t word[V * sizeof(T) / 4];
+    };
+    static __device__ Raw load(const T* p) { return *reinterpret_cast<const Raw*>(p); }
+    static __device__ float4 quad(const Raw& r, int q) {
+        struct __attribute__((aligned(4 * sizeof(T)))) Quad {
+            uint32_t word[sizeof(T)];
+        } w;
+#pragma unroll
+        for (int i = 0; i < static_cast<int>(sizeof(T)); ++i) w.word[i] = r.word[q * sizeof(T) + i];
+        return load4(reinterpret_cast<const T*>(&w));
+    }
+    // The same streaming stores as store4, as one access.
+    static __device__ void store(T* p, const float4 (&v)[V / 4]) {
+        typedef uint32_t words __attribute__((ext_vector_type(V * sizeof(T) / 4)));
+        typedef words any __attribute__((aligned(4 * sizeof(T))));
+        words o;
+#pragma unroll
+        for (int q = 0; q < V / 4; ++q) {
+            if constexpr (sizeof(T) == 4) {
+                o[4 * q] = __float_as_uint(v[q].x), o[4 * q + 1] = __float_as_uint(v[q].y);
+                o[4 * q + 2] = __float_as_uint(v[q].z), o[4 * q + 3] = __float_as_uint(v[q].w);
+            } else if constexpr (std::is_same_v<T, bf16_t>) {
+                o[2 * q] = f32x2_to_bf16(v[q].x, v[q].y), o[2 * q + 1] = f32x2_to_bf16(v[q].z, v[q].w);
+            } else {
+                const __half2 a = __floats2half2_rn(v[q].x, v[q].y), b = __floats2half2_rn(v[q].z, v[q].w);
+                o[2 * q] = *reinterpret_cast<const uint32_t*>(&a), o[2 * q + 1] = *reinterpret_cast<const uint32_t*>(&b);
+            }
+        }
+        __builtin_nontemporal_store(o, reinterpret_cast<any*>(p));
+    }
+};
+
+// Sum over a workgroup of THREADS, the same value in every thread.  `scratch` (one float per wavefront) must not be read by
+// an earlier sum that another barrier does not separate from this one.
+template <int THREADS>
+__device__ inline float group_sum(float v, float* scratch) {
+    v = wave_sum(v);
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    if (lane == 0) scratch[wave] = v;
+    // Only LDS is exchanged: the loads of the next row stay in flight.
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < THREADS / kWave; ++w) t += scratch[w];
+    return t;
+}
+
+// Rows whose columns, pitch and address are multiples of four elements: a workgroup per row, thread t holding the V-element
+// pieces t + THREADS k, k < NP, as they lie in memory.  A workgroup walks several rows; gamma and beta stay in its registers
+// and the next row is on its way while this one is summed.  Bound by HBM.  With one row per workgroup gamma and beta were
+// twice the row's own traffic in L2, the loads 8 bytes a lane in 16-bit types, and nothing was in flight while the row was
+// reduced: [8192, 8192] bf16 with statistics 68 to 82 us, here 48 (5.6 TB/s; a copy reaches 5.9); [4096, 8192] fp32 53 -> 48;
+// [20000, 2560] bf16 41 -> 33, with the other workers' statistics in memory 69 -> 39; [64, 8192] bf16 6.0 -> 3.9.
+template <typename T, int V, int THREADS, int NP, int MODE, bool AFFINE>
+__global__ __launch_bounds__(THREADS) void ln_group_rows(const LnArgs a, const PartCounts pc) {
+    typedef RowPiece<T, V> P;
+    typedef typename P::Raw Raw;
+    __shared__ float scratch[2][THREADS / kWave];
+    const T* __restrict__ x = static_cast<const T*>(a.x);
+    T* __restrict__ y = static_cast<T*>(a.y);
+    const int t = threadIdx.x, lane = t & (kWave - 1);
+    const int pieces = a.cols / V;
+    const float inv = 1.0f / static_cast<float>(a.cols);
+    constexpr bool kPairs = MODE == kNorm || MODE == kJoined;   // takes the workers' {mean, M2} from memory
+    Raw v[NP], g[NP], b[NP];
+    float2 first = make_float2(0.f, 0.f);
+    auto fetch = [&](int64_t r, Raw (&to)[NP], float2& pair) {
+        if (kPairs && lane < a.nparts) pair = load_part(a.part_stats, a.rows, r, lane);
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            const int c = t + k * THREADS;
+            if (c < pieces) to[k] = P::load(x + r * a.ld + V * c);
+        }
+    };
+    int64_t r = blockIdx.x;
+    if (r < a.rows) fetch(r, v, first);
+    if (MODE != kStats && AFFINE) {
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            const int c = t + k * THREADS;
+            if (c < pieces) {
+                g[k] = P::load(static_cast<const T*>(a.gamma) + V * c);
+                b[k] = P::load(static_cast<const T*>(a.beta) + V * c);
+            }
+        }
+    }
+    const float inv_n = kPairs && lane < a.nparts ? pc.inv_n[lane] : 0.f;
+    for (; r < a.rows; r += gridDim.x) {
+        Raw v_next[NP];
+        float2 first_next = make_float2(0.f, 0.f);
+        const bool more = r + gridDim.x < a.rows;
+        if (more) fetch(r + gridDim.x, v_next, first_next);
+        float mean, rstd;
+        if (MODE == kNorm) {
+            // every wavefront combines the pairs for itself: no exchange needed
+            combine_parts(a.part_stats, a.rows, r, a.nparts, pc, a.eps, lane, first, inv_n, &mean, &rstd);
+        } else {
+            float s = 0.f;
+#pragma unroll
+            for (int k = 0; k < NP; ++k)
+                if (t + k * THREADS < pieces)
+#pragma unroll
+                    for (int q = 0; q < V / 4; ++q) s += sum4(P::quad(v[k], q));
+            mean = group_sum<THREADS>(s, scratch[0]) * inv;
+            float m2 = 0.f;
+#pragma unroll
+            for (int k = 0; k < NP; ++k)
+                if (t + k * THREADS < pieces)
+#pragma unroll
+                    for (int q = 0; q < V / 4; ++q) m2 += sq4(P::quad(v[k], q), mean);
+            m2 = group_sum<THREADS>(m2, scratch[1]);
+            if ((MODE == kStats || MODE == kJoined) && t == 0) reinterpret_cast<float2*>(a.stats)[r] = make_float2(mean, m2);
+            if (MODE == kJoined)
+                combine_parts(a.part_stats, a.rows, r, a.nparts, pc, a.eps, lane, lane == a.my_part ? make_float2(mean, m2) : first, inv_n,
+                              &mean, &rstd);
+            else
+                rstd = 1.0f / sqrtf(m2 * inv + a.eps);
+        }
+        if (MODE != kStats) {
+            if (t == 0) {
+                if (a.mean_out) a.mean_out[r] = mean;
+                if (a.rstd_out) a.rstd_out[r] = rstd;
+            }
+#pragma unroll
+            for (int k = 0; k < NP; ++k) {
+                const int c = t + k * THREADS;
+                if (c < pieces) {
+                    float4 o[V / 4];
+#pragma unroll
+                    for (int q = 0; q < V / 4; ++q) {
+                        o[q] = norm4(P::quad(v[k], q), mean, rstd);
+                        if (AFFINE) o[q] = affine4(P::quad(g[k], q), o[q], P::quad(b[k], q));
+                    }
+                    P::store(y + r * a.ldy + V * c, o);
+                }
+            }
+        }
+        if (more) {
+            first = first_next;
+#pragma unroll
+            for (int k = 0; k < NP; ++k) v[k] = v_next[k];
+        }
+    }
+}
+
+// Rows of any length, pitch and address: one workgroup per row, NV pieces of four per thread (cols <= 1024 NV); the grid
+// walks the rows.
+template <typename T, int NV, int MODE, bool AFFINE>
 __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const PartCounts pc) {
     __shared__ float scratch[kWavesPerBlock];
     const T* __restrict__ x = static_cast<const T*>(a.x);
@@ -244,7 +394,7 @@ __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const Pa
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int c = t + k * kBlock;
-            v[k] = c < nv ? load_piece<ANY>(x + r * a.ld + 4 * c, a.cols - 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[k] = c < nv ? load_piece<true>(x + r * a.ld + 4 * c, a.cols - 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         float mean, rstd;
         if (MODE == kNorm) {
@@ -259,7 +409,7 @@ __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const Pa
             float q = 0.f;
 #pragma unroll
             for (int k = 0; k < NV; ++k)
-                if (t + k * kBlock < nv) q += sq_piece<ANY>(v[k], mean, a.cols - 4 * (t + k * kBlock));
+                if (t + k * kBlock < nv) q += sq_piece<true>(v[k], mean, a.cols - 4 * (t + k * kBlock));
             q = block_sum(q, scratch);
             if (MODE == kStats || MODE == kJoined) {
                 if (t == 0) reinterpret_cast<float2*>(a.stats)[r] = make_float2(mean, q);
@@ -280,9 +430,9 @@ __global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const Pa
             const int c = t + k * kBlock;
             if (c < nv) {
                 float4 o = norm4(v[k], mean, rstd);
-                if (AFFINE) o = affine4(load_piece<ANY>(static_cast<const T*>(a.gamma) + 4 * c, a.cols - 4 * c), o,
-                                        load_piece<ANY>(static_cast<const T*>(a.beta) + 4 * c, a.cols - 4 * c));
-                store_piece<ANY>(y + r * a.ldy + 4 * c, o, a.cols - 4 * c);
+                if (AFFINE) o = affine4(load_piece<true>(static_cast<const T*>(a.gamma) + 4 * c, a.cols - 4 * c), o,
+                                        load_piece<true>(static_cast<const T*>(a.beta) + 4 * c, a.cols - 4 * c));
+                store_piece<true>(y + r * a.ldy + 4 * c, o, a.cols - 4 * c);
             }
         }
     }
@@ -377,10 +527,32 @@ void launch_wave(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
         launch_wave_rpw<T, MODE, AFFINE, ANY, NV, 1>(a, pc, s);
 }
 
-template <typename T, int MODE, bool AFFINE, bool ANY, int NV>
+template <typename T, int MODE, bool AFFINE, int NV>
 void launch_block(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     const uint32_t blocks = static_cast<uint32_t>(a.rows < (1 << 20) ? a.rows : (1 << 20));
-    hipLaunchKernelGGL((ln_block_rows<T, NV, MODE, AFFINE, ANY>), dim3(blocks), dim3(kBlock), 0, s, a, pc);
+    hipLaunchKernelGGL((ln_block_rows<T, NV, MODE, AFFINE>), dim3(blocks), dim3(kBlock), 0, s, a, pc);
+}
+
+// Rows per workgroup of ln_group_rows: enough to share gamma and beta, few enough that every CU has several workgroups.
+constexpr int64_t kGroupRows = 8;
+
+template <typename T, int MODE, bool AFFINE, int V, int THREADS, int NP>
+void launch_group(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
+    int dev = 0;
+    const int64_t waves = 16 * compute_units(dev);
+    int64_t per = a.rows * (THREADS / kWave) / waves;
+    per = per < 1 ? 1 : per > kGroupRows ? kGroupRows : per;
+    const int64_t blocks = (a.rows + per - 1) / per;
+    hipLaunchKernelGGL((ln_group_rows<T, V, THREADS, NP, MODE, AFFINE>), dim3(static_cast<uint32_t>(blocks < (1 << 20) ? blocks : (1 << 20))), dim3(THREADS), 0, s, a, pc);
+}
+
+template <typename T, int MODE, bool AFFINE, int V>
+void launch_group_pieces(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
+    const int pieces = a.cols / V;   // up to 16384 / V
+    if (pieces <= 512) launch_group<T, MODE, AFFINE, V, 256, 2>(a, pc, s);
+    else if (pieces <= 1024) launch_group<T, MODE, AFFINE, V, 256, 4>(a, pc, s);
+    else if (pieces <= 2048) launch_group<T, MODE, AFFINE, V, 512, 4>(a, pc, s);
+    else launch_group<T, MODE, AFFINE, V, 1024, 4>(a, pc, s);
 }
 
 // Rows of up to kBlockRowCols columns, held in registers.
@@ -394,10 +566,16 @@ int launch_held(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
         else launch_wave<T, MODE, AFFINE, ANY, 8>(a, pc, s);
         return check_launch("ln_wave_rows");
     }
-    if (cols <= 4096) launch_block<T, MODE, AFFINE, ANY, 4>(a, pc, s);
-    else if (cols <= 8192) launch_block<T, MODE, AFFINE, ANY, 8>(a, pc, s);
-    else launch_block<T, MODE, AFFINE, ANY, 16>(a, pc, s);
-    return check_launch("ln_block_rows");
+    if constexpr (!ANY) {
+        if (sizeof(T) == 2 && cols % 8 == 0) launch_group_pieces<T, MODE, AFFINE, 16 / static_cast<int>(sizeof(T))>(a, pc, s);
+        else launch_group_pieces<T, MODE, AFFINE, 4>(a, pc, s);
+        return check_launch("ln_group_rows");
+    } else {
+        if (cols <= 4096) launch_block<T, MODE, AFFINE, 4>(a, pc, s);
+        else if (cols <= 8192) launch_block<T, MODE, AFFINE, 8>(a, pc, s);
+        else launch_block<T, MODE, AFFINE, 16>(a, pc, s);
+        return check_launch("ln_block_rows");
+    }
 }
 
 template <typename T, int MODE, bool AFFINE>

@@ -535,6 +535,43 @@ def test_layer_norm_rows_of_any_length_and_address(ops, dtype, cols):
     check(y2, (x64 - m2[:, None]) / (v2 + 1e-3).sqrt()[:, None] * gamma.double() + beta.double(), 8.0)
 
 
+@pytest.mark.parametrize("rows,cols,pad", [(1, 2052, 0), (3, 2056, 4), (4097, 2052, 4), (8191, 2056, 0), (9001, 4096, 0), (70, 4100, 0),
+                                           (5000, 8192, 8), (33, 8196, 0), (2100, 8200, 0), (1025, 16384, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_layer_norm_of_long_rows_walked_by_workgroups(ops, dtype, rows, cols, pad):
+    """Rows a workgroup holds in pieces of four and eight elements, where a workgroup has one row, several, and one less than
+    the others: y, mean and rstd against float64, with a pitch and a row of infinities that must not reach its neighbours;
+    the statistics alone, and statistics and result in one launch, give the same bits."""
+    gen = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x = (torch.randn(rows, cols + pad, generator=gen, device="cuda") * 2 + 0.5).to(dtype)[:, :cols]
+    gamma = (1 + 0.1 * torch.randn(cols, generator=gen, device="cuda")).to(dtype)
+    beta = (0.1 * torch.randn(cols, generator=gen, device="cuda")).to(dtype)
+    bad = rows // 2
+    if rows > 1:
+        x[bad, 1] = float("inf")
+    y, mean, rstd = ops.layer_norm(x, gamma, beta, 1e-3, want_stats=True)
+    stats = ops.ln_partial_stats(x)
+    pairs = torch.stack([torch.zeros_like(stats), stats]).contiguous()
+    joined = pairs.clone()
+    joined[1] = 0
+    two = ops.ln_normalize_affine(x, pairs, [cols, cols], gamma, beta, 1e-3)
+    one = ops.ln_stats_normalize(x, joined, 1, [cols, cols], gamma, beta, 1e-3)
+    keep = torch.ones(rows, dtype=torch.bool, device="cuda")
+    if rows > 1:
+        keep[bad] = False
+        assert bool(y[bad].isnan().any()) and not bool(y[keep].isnan().any())
+    assert torch.equal(joined[1][keep], stats[keep]) and torch.equal(one[keep], two[keep])
+    ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for part in keep.nonzero().flatten().split(1024):
+        x64 = x[part].double()
+        m = x64.mean(1)
+        r = ((x64 - m[:, None]).square().mean(1) + 1e-3).rsqrt()
+        want = (x64 - m[:, None]) * r[:, None] * gamma.double() + beta.double()
+        # one rounding of the result and a few units of fp32 sums (values up to 12, |x| rstd up to 6)
+        assert bool(((y[part].double() - want).abs() <= ulp * want.abs() + 4e-6 * 8).all())
+        assert bool(((mean[part].double() - m).abs() <= 4e-6 * 4).all()) and bool(((rstd[part].double() - r).abs() <= 4e-6 * r).all())
+
+
 @pytest.mark.parametrize("rows,cols,pad", [(1, 1028, 0), (5, 1025, 0), (37, 2048, 4), (3, 2052, 0), (66, 4096, 1), (1029, 4097, 0),
                                            (9, 8192, 0), (7, 8191, 0), (6, 8196, 0), (10, 16384, 8), (8200, 1032, 0),
                                            (1, 513, 0), (70, 514, 3), (65, 1023, 0), (300, 768, 1)])
