@@ -11,23 +11,28 @@
 // written exactly once -- rows nobody looked up get their zeros from the same
 // pass, so dweight needs no clearing.
 //
+//   emb_bwd_split    tokens of a chunk of ids sorted by segment; segment s owns the rows s, s + G, s + 2 G, ... of the
+//                    table (frequent ids are neighbours in a vocabulary sorted by frequency: so they spread)
+//   emb_bwd_buckets  a workgroup per segment: counts and places its tokens with counters in LDS.  Nothing has to be cleared,
+//                    and a row that many tokens share costs LDS atomics of one workgroup
+//   with less workspace than these take, or a table of more than 2^23 rows, four launches instead:
 //   emb_bwd_clear    counters = 0
 //   emb_bwd_count    count[row]++ per token in the window
 //   emb_bwd_place    a stretch of the bucket array for every row.  The stretches lie in no particular order, so
 //                    no prefix sum over the whole table is needed: a workgroup scans its own 1024 counters and takes its
 //                    place with one atomic.  Rows of more than kHotAbove tokens go on the list of hot rows.
 //   emb_bwd_fill     bucket[end[row]++] = t
-//   emb_bwd_hot      the sums of hot rows: a workgroup per row and 256 bytes of columns (hot_row); not launched
+//   then
+//   emb_bwd_hot      the sums of hot rows: a workgroup per row and 64 bytes of columns (hot_row); not launched
 //                    when there are too few tokens for a hot row
 //   emb_bwd_reduce   the sums of all other rows: one wavefront (half a wavefront for narrow tables) per row and group
 //                    of columns, the bucket ordered in registers
 //
-// The order in which the fill kernel's atomics hand out bucket slots varies
-// from run to run; the reduce kernel orders every bucket so that the fp32 sums
-// do not.
+// The order in which atomics hand out bucket slots varies from run to run; the
+// kernels that add order every bucket so that the fp32 sums do not.
 //
 // What bounds it: the gradient rows read once and the table written once, plus
-// the four short kernels in front (2-5 us each, launch and memory latency).
+// the short kernels in front (2-5 us each, launch and memory latency).
 // Token ids as they occur in text make a few rows hot: of 8192 tokens over
 // 50304 rows with ids distributed log-uniformly, 483 share one row.  A single
 // wavefront walking that bucket one token at a time -- a memory round trip per
@@ -51,9 +56,14 @@ constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 
-__global__ __launch_bounds__(kBlock) void emb_bwd_clear(int32_t* __restrict__ count, int64_t rows, int32_t* __restrict__ totals) {
+// What is known of a row: its number of tokens, and the end of its stretch of the bucket array.
+struct Row {
+    int32_t count, end;
+};
+
+__global__ __launch_bounds__(kBlock) void emb_bwd_clear(Row* __restrict__ meta, int64_t rows, int32_t* __restrict__ totals) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i < rows) count[i] = 0;
+    if (i < rows) meta[i].count = 0;
     if (i < 2) totals[i] = 0;
 }
 
@@ -88,22 +98,22 @@ __device__ inline int same_row_lanes(int32_t row, bool on, int lane, int* first,
 
 template <typename IdT>
 __global__ __launch_bounds__(kBlock) void emb_bwd_count(const IdT* __restrict__ ids, int64_t n_ids, int64_t lo, int64_t hi,
-                                                        int64_t padding_idx, int32_t* __restrict__ count) {
+                                                        int64_t padding_idx, Row* __restrict__ meta) {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     const int32_t r = t < n_ids ? static_cast<int32_t>(token_row(ids, t, lo, hi, padding_idx)) : -1;
     const int lane = threadIdx.x & (kWave - 1);
     int first, before;
     const int size = same_row_lanes(r, r >= 0, lane, &first, &before);
-    if (r >= 0 && before == 0) atomicAdd(&count[r], size);
+    if (r >= 0 && before == 0) atomicAdd(&meta[r].count, size);
 }
 
-// Stretches of the bucket array.  end[row] is where the row's stretch begins;
+// Stretches of the bucket array.  A row's `end` is set to where its stretch begins;
 // the fill kernel advances it to where it ends.  totals[0]: slots handed out so
 // far, totals[1]: entries of the hot list.  The last row of the table never goes
 // on the list (it is looked at in any case), so the list has at most rows - 1 entries.
 constexpr int kPlaceRows = 4;                     // consecutive rows of a thread
-__global__ __launch_bounds__(kBlock) void emb_bwd_place(const int32_t* __restrict__ count, int64_t rows, int32_t hot_above,
-                                                        int32_t* __restrict__ end, int32_t* __restrict__ hot, int32_t* __restrict__ totals) {
+__global__ __launch_bounds__(kBlock) void emb_bwd_place(Row* __restrict__ meta, int64_t rows, int32_t hot_above, int32_t* __restrict__ hot,
+                                                        int32_t* __restrict__ totals) {
     __shared__ int32_t wave_total[kWavesPerBlock];
     __shared__ int32_t base;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -111,7 +121,7 @@ __global__ __launch_bounds__(kBlock) void emb_bwd_place(const int32_t* __restric
     int32_t n[kPlaceRows], total = 0;
 #pragma unroll
     for (int k = 0; k < kPlaceRows; ++k) {
-        n[k] = r0 + k < rows ? count[r0 + k] : 0;
+        n[k] = r0 + k < rows ? meta[r0 + k].count : 0;
         total += n[k];
     }
     int32_t incl = total;                                      // inclusive scan over the wavefront
@@ -134,7 +144,7 @@ __global__ __launch_bounds__(kBlock) void emb_bwd_place(const int32_t* __restric
 #pragma unroll
     for (int k = 0; k < kPlaceRows; ++k) {
         if (r0 + k >= rows) break;
-        end[r0 + k] = run;
+        meta[r0 + k].end = run;
         run += n[k];
         if (n[k] > hot_above && r0 + k < rows - 1) hot[atomicAdd(&totals[1], 1)] = static_cast<int32_t>(r0 + k);
     }
@@ -142,16 +152,288 @@ __global__ __launch_bounds__(kBlock) void emb_bwd_place(const int32_t* __restric
 
 template <typename IdT>
 __global__ __launch_bounds__(kBlock) void emb_bwd_fill(const IdT* __restrict__ ids, int64_t n_ids, int64_t lo, int64_t hi,
-                                                       int64_t padding_idx, int32_t* __restrict__ end, int32_t* __restrict__ bucket) {
+                                                       int64_t padding_idx, Row* __restrict__ meta, int32_t* __restrict__ bucket) {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     const int32_t r = t < n_ids ? static_cast<int32_t>(token_row(ids, t, lo, hi, padding_idx)) : -1;
     const int lane = threadIdx.x & (kWave - 1);
     int first, before;
     const int size = same_row_lanes(r, r >= 0, lane, &first, &before);
     int32_t slot = 0;
-    if (r >= 0 && before == 0) slot = atomicAdd(&end[r], size);
+    if (r >= 0 && before == 0) slot = atomicAdd(&meta[r].end, size);
     slot = __shfl(slot, first, kWave) + before;
     if (r >= 0) bucket[slot] = static_cast<int32_t>(t);
+}
+
+// ---- bucketing in two launches ----
+// Bound by latency: launches, LDS atomics, a few dependent trips to L2.  Measured, four launches -> two: 131072 uniform
+// tokens over 128256 ids, 16032 of them rows, 20 -> 10.5 us; as in text (11000 tokens on one row) 92 -> 28 us; 8192 tokens as
+// in text over 50304 rows 19 -> 16 us with the buckets left in order, which takes the hot rows' kernel 6 us less; 16 tokens
+// 7.6 -> 7.3 us.  (One launch whose workgroups each look at all tokens: 7 us for 8192 tokens, but 24 for 131072, 79 as in text.)
+constexpr int kSplitBlock = 256;
+constexpr int kBucketBlock = 1024;
+constexpr int kChunks = 1024;                     // chunks of tokens, at most
+constexpr int kSegmentRows = 4096;                // rows of a segment, at most
+constexpr int kSegments = 2048;                   // segments, at most; a power of two from 256 on
+constexpr int kHeldTokens = 4096;                 // tokens of a segment that are placed in LDS first
+constexpr int kLongRows = 256;
+constexpr int32_t kOrdered = 0x40000000;          // in an entry of the hot list: the row's bucket is in ascending order
+constexpr int kRankTokens = 2 * kBlock;           // up to so many tokens of a row are ordered by counting the smaller ones
+constexpr int kBitWords = 4096;                   // more of them by a bit per token number
+constexpr int kBitsPerWindow = kBitWords * 32;
+
+struct SplitArgs {
+    int64_t n_ids, lo, padding_idx, chunk_tokens;
+    int32_t rows, segments, shift;                // segments = 1 << shift
+    int32_t segment_rows, chunks, hot_above;
+    int32_t* offsets;                             // [chunks][segments + 1]: first token of the segment in the chunk
+    int32_t* token;                               // [n_ids] tokens of a chunk by segment
+    int32_t* row;                                 // [n_ids] their rows inside the segment
+    Row* meta;                                    // [segments][segment_rows]
+    int32_t* bucket;
+    int32_t* hot;
+    int32_t* totals;                              // entries at the end of the hot list, entries at its front
+    int32_t hot_most;                             // entries the hot list has room for
+};
+
+template <typename IdT>
+__global__ __launch_bounds__(kSplitBlock) void emb_bwd_split(const IdT* __restrict__ ids, const SplitArgs a) {
+    __shared__ int32_t cursor[kSegments];
+    __shared__ int32_t wave_total[kSplitBlock / kWave];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+    const int64_t t0 = blockIdx.x * a.chunk_tokens, t1 = t0 + a.chunk_tokens < a.n_ids ? t0 + a.chunk_tokens : a.n_ids;
+    for (int s = t; s < a.segments; s += kSplitBlock) cursor[s] = 0;
+    if (blockIdx.x == 0 && t < 2) a.totals[t] = 0;
+    __syncthreads();
+    for (int64_t i = t0 + t; i < t1; i += kSplitBlock) {
+        const int32_t r = static_cast<int32_t>(token_row(ids, i, a.lo, a.lo + a.rows, a.padding_idx));
+        if (r >= 0) atomicAdd(&cursor[r & (a.segments - 1)], 1);
+    }
+    __syncthreads();
+    constexpr int kPer = kSegments / kSplitBlock;
+    const int per = a.segments / kSplitBlock;      // 1 to kPer segments per thread
+    int32_t n[kPer], total = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        n[k] = k < per ? cursor[t * per + k] : 0;
+        total += n[k];
+    }
+    int32_t incl = total;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t up = __shfl_up(incl, off, kWave);
+        if (lane >= off) incl += up;
+    }
+    if (lane == kWave - 1) wave_total[wave] = incl;
+    __syncthreads();
+    int32_t run = incl - total;
+#pragma unroll
+    for (int k = 0; k < kSplitBlock / kWave; ++k) run += k < wave ? wave_total[k] : 0;
+    int32_t* const offsets = a.offsets + static_cast<int64_t>(blockIdx.x) * (a.segments + 1);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        if (k >= per) break;
+        cursor[t * per + k] = run;
+        offsets[t * per + k] = run;
+        run += n[k];
+    }
+    if (t == kSplitBlock - 1) offsets[a.segments] = run;
+    __syncthreads();
+    for (int64_t i = t0 + t; i < t1; i += kSplitBlock) {
+        const int32_t r = static_cast<int32_t>(token_row(ids, i, a.lo, a.lo + a.rows, a.padding_idx));
+        if (r < 0) continue;
+        const int64_t at = t0 + atomicAdd(&cursor[r & (a.segments - 1)], 1);
+        a.token[at] = static_cast<int32_t>(i);
+        a.row[at] = r >> a.shift;
+    }
+}
+
+// One counter takes the lanes of a wavefront that share the first active lane's row in one atomic: a bucket of thousands of
+// tokens is mostly such lanes.  Returns what the counter held, plus the lane's place among them.
+__device__ inline int32_t count_up(int32_t* counters, int32_t row) {
+    const int32_t first = __builtin_amdgcn_readfirstlane(row);
+    const uint64_t same = __ballot(row == first);
+    if (row != first) return atomicAdd(&counters[row], 1);
+    const int32_t before = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(same >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(same), 0));
+    int32_t base = 0;
+    if (before == 0) base = atomicAdd(&counters[first], __popcll(same));
+    return __builtin_amdgcn_readfirstlane(base) + before;
+}
+
+static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const SplitArgs a) {
+    __shared__ int32_t counters[kSegmentRows];
+    __shared__ int32_t upto[kChunks + 1], from[kChunks];   // tokens of this segment in the chunks below; where its own begin
+    __shared__ int32_t wave_total[kBucketBlock / kWave], wave_base[kBucketBlock / kWave];
+    __shared__ int32_t held[kHeldTokens];
+    __shared__ uint16_t held_row[kHeldTokens];
+    __shared__ int32_t long_begin[kLongRows], long_end[kLongRows], long_rows;
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+    const int32_t s = static_cast<int32_t>(blockIdx.x);
+    if (t == 0) long_rows = 0;
+    const int32_t rows = s < a.rows ? ((a.rows - 1 - s) >> a.shift) + 1 : 0;   // of this segment
+    for (int i = t; i < rows; i += kBucketBlock) counters[i] = 0;
+    // A thread per chunk.  The tokens of lower segments in all chunks are the place of this segment's stretch.
+    static_assert(kChunks == kBucketBlock, "a thread per chunk");
+    int32_t len = 0, lower = 0;
+    if (t < a.chunks) {
+        const int32_t* const o = a.offsets + static_cast<int64_t>(t) * (a.segments + 1) + s;
+        lower = o[0];
+        len = o[1] - lower;
+        from[t] = lower;
+    }
+    int32_t incl = len, base = lower;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t up = __shfl_up(incl, off, kWave);
+        if (lane >= off) incl += up;
+        base += __shfl_xor(base, off, kWave);
+    }
+    if (lane == kWave - 1) wave_total[wave] = incl, wave_base[wave] = base;
+    __syncthreads();
+    int32_t before = 0, tokens = 0, run = 0;
+#pragma unroll
+    for (int k = 0; k < kBucketBlock / kWave; ++k) {
+        before += k < wave ? wave_total[k] : 0;
+        tokens += wave_total[k];
+        run += wave_base[k];
+    }
+    upto[t + 1] = before + incl;
+    if (t == 0) upto[0] = 0;
+    __syncthreads();
+    // Where this segment's token i < tokens is: in the chunk c with upto[c] <= i < upto[c + 1].
+    auto place = [&](int32_t i) {
+        int32_t c = 0;
+#pragma unroll
+        for (int32_t half = kChunks / 2; half > 0; half >>= 1)
+            if (upto[c + half] <= i) c += half;
+        return c * a.chunk_tokens + from[c] + (i - upto[c]);
+    };
+    // The first kBucketBlock tokens, mostly all, stay in registers.
+    int32_t row_first = -1, token_first = 0;
+    if (t < tokens) {
+        const int64_t at = place(t);
+        row_first = a.row[at], token_first = a.token[at];
+        count_up(counters, row_first);
+    }
+    for (int32_t i = t + kBucketBlock; i < tokens; i += kBucketBlock) count_up(counters, a.row[place(i)]);
+    __syncthreads();
+    constexpr int kRows = kSegmentRows / kBucketBlock;
+    const int per = (rows + kBucketBlock - 1) / kBucketBlock;   // consecutive rows of a thread
+    int32_t n[kRows], begins[kRows], long_at[kRows], total = 0;
+    const int32_t run_first = run;                              // where this segment's stretch begins
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+        long_at[k] = -1, begins[k] = 0;
+        n[k] = k < per && t * per + k < rows ? counters[t * per + k] : 0;
+        total += n[k];
+    }
+    incl = total;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t up = __shfl_up(incl, off, kWave);
+        if (lane >= off) incl += up;
+    }
+    __syncthreads();                                            // wave_total has been read
+    if (lane == kWave - 1) wave_total[wave] = incl;
+    __syncthreads();
+    run += incl - total;
+#pragma unroll
+    for (int k = 0; k < kBucketBlock / kWave; ++k) run += k < wave ? wave_total[k] : 0;
+    Row* const meta = a.meta + static_cast<int64_t>(s) * a.segment_rows;
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+        const int32_t r = t * per + k;
+        if (k >= per || r >= rows) break;
+        counters[r] = begins[k] = run;
+        run += n[k];
+        meta[r].count = n[k], meta[r].end = run;
+        // Long rows from the front of the list, so that their workgroups start first; the others from its end.
+        if (n[k] > kRankTokens) {
+            if (a.n_ids <= kBitsPerWindow) long_at[k] = atomicAdd(&long_rows, 1);
+            a.hot[atomicAdd(&a.totals[1], 1)] = ((r << a.shift) + s) | (a.n_ids <= kBitsPerWindow ? kOrdered : 0);
+        } else if (n[k] > a.hot_above) {
+            a.hot[a.hot_most - 1 - atomicAdd(&a.totals[0], 1)] = ((r << a.shift) + s) | (tokens <= kHeldTokens ? kOrdered : 0);
+        }
+    }
+    __syncthreads();
+    // The buckets, in ascending order where that is cheap: the workgroups that share a hot row's columns need not each do it.
+    const int32_t stretch = run_first;
+    if (tokens <= kHeldTokens) {
+        auto hold = [&](int32_t row, int32_t token) {
+            const int32_t at = count_up(counters, row) - stretch;
+            held[at] = token, held_row[at] = static_cast<uint16_t>(row);
+        };
+        if (row_first >= 0) hold(row_first, token_first);
+        for (int32_t i = t + kBucketBlock; i < tokens; i += kBucketBlock) {
+            const int64_t at = place(i);
+            hold(a.row[at], a.token[at]);
+        }
+        __syncthreads();
+        for (int32_t i = t; i < tokens; i += kBucketBlock) {   // a counter holds the end of its row now, which is where the next begins
+            const int32_t r = held_row[i], begin = r ? counters[r - 1] - stretch : 0, end = counters[r] - stretch;
+            int32_t to = i;
+            if (end - begin > 1 && end - begin <= kRankTokens) {
+                const int32_t mine = held[i];
+                to = begin;
+#pragma unroll 8
+                for (int32_t j = begin; j < end; ++j) to += held[j] < mine ? 1 : 0;
+            }
+            a.bucket[stretch + to] = held[i];
+        }
+    } else {
+        if (row_first >= 0) a.bucket[count_up(counters, row_first)] = token_first;
+        for (int32_t i = t + kBucketBlock; i < tokens; i += kBucketBlock) {
+            const int64_t at = place(i);
+            a.bucket[count_up(counters, a.row[at])] = a.token[at];
+        }
+    }
+    __syncthreads();
+    const int32_t all_long = long_rows;
+    for (int32_t first = 0; first < all_long; first += kLongRows) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kRows; ++k)
+            if (long_at[k] >= first && long_at[k] < first + kLongRows) {
+                long_begin[long_at[k] - first] = begins[k];
+                long_end[long_at[k] - first] = begins[k] + n[k];
+            }
+        const int32_t here = all_long - first < kLongRows ? all_long - first : kLongRows;
+        for (int32_t h = 0; h < here; ++h) {
+            uint32_t* const bits = reinterpret_cast<uint32_t*>(counters);
+            static_assert(kBitWords == kSegmentRows, "a bit per token number where the counters were");
+            constexpr int kWords = kBitWords / kBucketBlock;
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < kWords; ++k) bits[t + k * kBucketBlock] = 0;
+            __syncthreads();
+            const int32_t begin = long_begin[h], end = long_end[h];
+            for (int32_t i = begin + t; i < end; i += kBucketBlock) {
+                const int32_t at = tokens <= kHeldTokens ? held[i - stretch] : a.bucket[i];
+                atomicOr(&bits[at >> 5], 1u << (at & 31));
+            }
+            __syncthreads();
+            uint32_t mine[kWords];
+            int32_t sum = 0;
+#pragma unroll
+            for (int k = 0; k < kWords; ++k) {
+                mine[k] = bits[t * kWords + k];
+                sum += __popc(mine[k]);
+            }
+            int32_t up_to = sum;
+#pragma unroll
+            for (int off = 1; off < kWave; off <<= 1) {
+                const int32_t up = __shfl_up(up_to, off, kWave);
+                if (lane >= off) up_to += up;
+            }
+            if (lane == kWave - 1) wave_total[wave] = up_to;
+            __syncthreads();
+            int32_t rank = begin + up_to - sum;
+#pragma unroll
+            for (int k = 0; k < kBucketBlock / kWave; ++k) rank += k < wave ? wave_total[k] : 0;
+#pragma unroll
+            for (int k = 0; k < kWords; ++k)
+                for (uint32_t w = mine[k]; w; w &= w - 1) a.bucket[rank++] = (t * kWords + k) * 32 + __ffs(w) - 1;
+        }
+    }
 }
 
 // Elements: bf16 or fp16 bits or float; all are summed in fp32 and rounded once on the way out.
@@ -214,11 +496,13 @@ struct ReduceArgs {
     const void* dy;
     void* dw;
     int64_t dim, ld_dy, ld_dw, rows;
-    const int32_t* count;
-    const int32_t* end;
+    const Row* meta;
     const int32_t* bucket;
     const int32_t* hot;
     const int32_t* totals;
+    int32_t shift, segment_rows;   // of the segments that `meta` is ordered by
+    int32_t hot_most;              // entries the hot list has room for: long rows from its front, others from its end; 0: all
+                                   // from its front, and the last row of the table on no list
     int64_t n_ids;
     int32_t nv;             // vectors of V elements per row; the last one is moved back to end with the row
     int32_t passes;         // groups of columns per row of the ordinary path
@@ -226,95 +510,100 @@ struct ReduceArgs {
     int32_t hot_above;      // rows of more tokens are hot
     int32_t hot_chunks;     // 256-byte pieces of a row
     int32_t scale_by_freq;
+    __device__ Row of(int64_t row) const { return meta[(row & ((1 << shift) - 1)) * segment_rows + (row >> shift)]; }
 };
 
 // ---- hot rows ----
-// A workgroup owns 256 bytes of columns of one row.  What takes time is the
+// A workgroup owns 64 bytes of columns of one row.  What takes time is the
 // memory round trip, not the additions, so all threads fetch the pieces of the
-// next two batches of 64 tokens -- 16 lanes a token, 16 bytes a lane -- while one
-// wavefront adds a batch in token order out of LDS, a column (or two 16-bit ones)
-// per lane: the sums stay strictly sequential per column with 128 tokens in
-// flight.  (A wavefront that walks its columns alone keeps 32 in flight in the
-// same registers: 55 us instead of 20 for 483 tokens of 2 KiB.)
-// The order of the tokens: up to 512 by counting the smaller ones, more through
+// next two batches of 256 tokens -- four lanes a token, 16 bytes a lane -- while one
+// wavefront adds a batch in token order out of LDS, a column per lane: the sums stay strictly sequential per column with 512 tokens in
+// flight.  (With 256 bytes of columns and batches of 64 tokens a row of 11000 tokens
+// of 512 bytes took 370 us, here 100; 483 tokens of 2 KiB 20 us, here 9.  A wavefront
+// that walks its columns alone keeps 32 tokens in flight in the same registers: 55 us.)
+// The order of the tokens, where emb_bwd_buckets has not made it: up to 512 by counting the smaller ones, more through
 // a bit per token number in LDS (16 KiB for a window of 131072 of them) that is
 // read back in ascending order, kListTokens at a time.  The bits have LDS of their
 // own: in the stage's they had to be set again, by a walk over the whole bucket,
 // for every kListTokens (2^20 tokens of one row, 256 bytes each: 1267 ms, now 59).
 constexpr int kHotAbove = 32;                        // rows of more tokens are hot: what half a wavefront's lanes order, and as long as
                                                      // the ordinary walk stays below the time of everything else (with 64: 24 us, with 32: 17)
-constexpr int kHotBytes = 256;
-constexpr int kHotBatch = 64;                        // tokens per batch
+constexpr int kHotBytes = 64;
+constexpr int kHotBatch = 256;                       // tokens per batch
+constexpr int kHotPitch = kHotBatch + 4;             // 16 floats apart for the four lanes that store a token: no two on one bank
 constexpr int kListTokens = 1024;
-constexpr int kRankTokens = 2 * kBlock;
-constexpr int kBitWords = 4096;
-constexpr int kBitsPerWindow = kBitWords * 32;
 constexpr int kWordsPerThread = kBitWords / kBlock;
 
 struct HotShared {
-    uint32_t pieces[kHotBytes * kHotBatch / 4];      // of a batch
+    float column[kHotBytes / 2][kHotPitch];          // a batch in fp32, column by column: the adding wavefront reads four tokens at once
     uint32_t bits[kBitWords];                        // a bit per token number, or the bucket being ordered
     int32_t list[kListTokens];                       // tokens in ascending order
     int32_t wave_total[kWavesPerBlock];
 };
 
-// Adds the first m tokens of the list to the columns from col0 on; called by all threads.
+// Adds the m tokens of the list (in LDS or in global memory) to the columns from col0 on, thread t's to column col0 + t; called by all
+// threads.
 template <typename E>
-__device__ inline void hot_accumulate(HotShared& sh, const ReduceArgs& a, int64_t col0, int m, float (&acc)[2]) {
+__device__ inline void hot_accumulate(HotShared& sh, const ReduceArgs& a, const int32_t* list, int64_t col0, int m, float& acc) {
     typedef typename E::word W;
-    constexpr int V = 16 / sizeof(W);
-    constexpr int kLanesPerToken = 16, kTokensPerLoad = kBlock / kLanesPerToken, kLoads = kHotBatch / kTokensPerLoad;
+    constexpr int V = 16 / sizeof(W), kCols = kHotBytes / sizeof(W);
+    constexpr int kLanesPerToken = kHotBytes / 16, kTokensPerLoad = kBlock / kLanesPerToken, kLoads = kHotBatch / kTokensPerLoad;
     const int t = threadIdx.x, part = t % kLanesPerToken, tok0 = t / kLanesPerToken;
     const int64_t col = col0 + part * V, left = a.dim - col;
     const W* const dy = static_cast<const W*>(a.dy) + col;
-    uint4 piece[2][kLoads];
-    auto fetch = [&](uint4 (&to)[kLoads], int base) {
+    Pack<W, V> piece[2][kLoads];
+    int32_t token[kLoads];                           // of the batch that is fetched next
+    auto look = [&](int base) {
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
             const int i = base + u * kTokensPerLoad + tok0;
-            to[u] = make_uint4(0, 0, 0, 0);
+            token[u] = i < m ? list[i] : 0;
+        }
+    };
+    auto fetch = [&](Pack<W, V> (&to)[kLoads], int base) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const int i = base + u * kTokensPerLoad + tok0;
             if (i >= m || left <= 0) continue;
-            const W* src = dy + static_cast<int64_t>(sh.list[i]) * a.ld_dy;
-            Pack<W, V> v;
+            const W* src = dy + static_cast<int64_t>(token[u]) * a.ld_dy;
             if (left >= V) {
-                v = load_pack<W, V>(src);
+                to[u] = load_pack<W, V>(src);
             } else {
 #pragma unroll
-                for (int e = 0; e < V; ++e) v.e[e] = e < left ? src[e] : W(0);
+                for (int e = 0; e < V; ++e) to[u].e[e] = e < left ? src[e] : W(0);
             }
-            __builtin_memcpy(&to[u], &v, 16);
         }
     };
-    auto batch = [&](uint4 (&from)[kLoads], int base) {
+    auto batch = [&](Pack<W, V> (&from)[kLoads], int base) {
 #pragma unroll
         for (int u = 0; u < kLoads; ++u)
-            *reinterpret_cast<uint4*>(&sh.pieces[(u * kTokensPerLoad + tok0) * (kHotBytes / 4) + part * 4]) = from[u];
+#pragma unroll
+            for (int e = 0; e < V; ++e) sh.column[part * V + e][u * kTokensPerLoad + tok0] = E::widen(from[u].e[e]);
         __syncthreads();
         if (base + 2 * kHotBatch < m) fetch(from, base + 2 * kHotBatch);
-        if (t < kWave) {
+        if (base + 3 * kHotBatch < m) look(base + 3 * kHotBatch);
+        if (t < kCols) {
             const int here = m - base < kHotBatch ? m - base : kHotBatch;
-            auto add = [&](uint32_t w) {
-                if constexpr (sizeof(W) == 4) {
-                    acc[0] += __uint_as_float(w);
-                } else {
-                    acc[0] += E::widen(static_cast<uint16_t>(w));
-                    acc[1] += E::widen(static_cast<uint16_t>(w >> 16));
-                }
-            };
+            const float* const mine = sh.column[t];
             int k = 0;
-            for (; k + 16 <= here; k += 16) {
-                uint32_t w[16];
+            for (; k + 32 <= here; k += 32) {
+                float4 q[8];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) w[u] = sh.pieces[(k + u) * (kHotBytes / 4) + t];
+                for (int u = 0; u < 8; ++u) q[u] = *reinterpret_cast<const float4*>(&mine[k + 4 * u]);
 #pragma unroll
-                for (int u = 0; u < 16; ++u) add(w[u]);
+                for (int u = 0; u < 8; ++u) acc += q[u].x, acc += q[u].y, acc += q[u].z, acc += q[u].w;
             }
-            for (; k < here; ++k) add(sh.pieces[k * (kHotBytes / 4) + t]);
+            for (; k < here; ++k) acc += mine[k];
         }
         __syncthreads();
     };
+    look(0);
     fetch(piece[0], 0);
-    if (kHotBatch < m) fetch(piece[1], kHotBatch);
+    if (kHotBatch < m) {
+        look(kHotBatch);
+        fetch(piece[1], kHotBatch);
+    }
+    if (2 * kHotBatch < m) look(2 * kHotBatch);
     for (int base = 0; base < m; base += 2 * kHotBatch) {
         batch(piece[0], base);
         if (base + kHotBatch < m) batch(piece[1], base + kHotBatch);
@@ -323,14 +612,17 @@ __device__ inline void hot_accumulate(HotShared& sh, const ReduceArgs& a, int64_
 
 // Called by every thread of the workgroup with the same arguments.
 template <typename E>
-__device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, int chunk) {
+__device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, bool ordered, int chunk) {
     typedef typename E::word W;
-    const int32_t n = a.count[row];
-    const int32_t* const bucket = a.bucket + (a.end[row] - n);
+    const Row meta = a.of(row);
+    const int32_t n = meta.count;
+    const int32_t* const bucket = a.bucket + (meta.end - n);
     const int t = threadIdx.x;
     const int64_t col0 = static_cast<int64_t>(chunk) * (kHotBytes / sizeof(W));
-    float acc[2] = {0.f, 0.f};
-    if (n <= kRankTokens) {
+    float acc = 0.f;
+    if (ordered) {
+        hot_accumulate<E>(sh, a, bucket, col0, n, acc);
+    } else if (n <= kRankTokens) {
         int32_t* const raw = reinterpret_cast<int32_t*>(sh.bits);
         // two tokens per thread; INT_MAX behind the bucket's end is smaller than nothing
         const int32_t t0 = t < n ? bucket[t] : 0x7FFFFFFF, t1 = t + kBlock < n ? bucket[t + kBlock] : 0x7FFFFFFF;
@@ -346,7 +638,7 @@ __device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, 
         if (t < n) sh.list[rank0] = t0;
         if (t + kBlock < n) sh.list[rank1] = t1;
         __syncthreads();
-        hot_accumulate<E>(sh, a, col0, n, acc);
+        hot_accumulate<E>(sh, a, sh.list, col0, n, acc);
     } else {
         const int lane = t & (kWave - 1), wave = t / kWave;
         for (int64_t w0 = 0; w0 < a.n_ids; w0 += kBitsPerWindow) {
@@ -390,19 +682,13 @@ __device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, 
                 }
                 __syncthreads();
                 const int32_t here = in_window - first;
-                hot_accumulate<E>(sh, a, col0, here < kListTokens ? here : kListTokens, acc);
+                hot_accumulate<E>(sh, a, sh.list, col0, here < kListTokens ? here : kListTokens, acc);
             }
         }
     }
-    if (t < kWave) {
+    if (t < static_cast<int>(kHotBytes / sizeof(W)) && col0 + t < a.dim) {
         const float scale = (a.scale_by_freq && n > 1) ? 1.0f / static_cast<float>(n) : 1.0f;
-        W* const dst = static_cast<W*>(a.dw) + row * a.ld_dw + col0;
-        if constexpr (sizeof(W) == 4) {
-            if (col0 + t < a.dim) dst[t] = acc[0] * scale;
-        } else {
-            if (col0 + 2 * t < a.dim) dst[2 * t] = E::round(acc[0] * scale);
-            if (col0 + 2 * t + 1 < a.dim) dst[2 * t + 1] = E::round(acc[1] * scale);
-        }
+        static_cast<W*>(a.dw)[row * a.ld_dw + col0 + t] = E::round(acc * scale);
     }
     __syncthreads();                                 // the list is rewritten by the workgroup's next row
 }
@@ -412,12 +698,14 @@ __device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, 
 template <typename E>
 __global__ __launch_bounds__(kBlock) void emb_bwd_hot(const ReduceArgs a) {
     __shared__ HotShared sh;
-    // the list, and the last row of the table if it is hot
     const int32_t listed = a.totals[1];
-    const int32_t items = (listed + (a.count[a.rows - 1] > a.hot_above ? 1 : 0)) * a.hot_chunks;
+    const int32_t more = a.hot_most ? a.totals[0] : a.of(a.rows - 1).count > a.hot_above ? 1 : 0;
+    const int32_t items = (listed + more) * a.hot_chunks;
     for (int32_t item = static_cast<int32_t>(blockIdx.x); item < items; item += static_cast<int32_t>(gridDim.x)) {
         const int32_t which = item / a.hot_chunks;
-        hot_row<E>(sh, a, which < listed ? a.hot[which] : a.rows - 1, item - which * a.hot_chunks);
+        const int32_t entry = which < listed ? a.hot[which] : a.hot_most ? a.hot[a.hot_most - 1 - (which - listed)] : static_cast<int32_t>(a.rows) - 1;
+        const bool ordered = a.hot_most && (entry & kOrdered);
+        hot_row<E>(sh, a, ordered ? entry & ~kOrdered : entry, ordered, item - which * a.hot_chunks);
     }
 }
 
@@ -440,7 +728,8 @@ __global__ __launch_bounds__(kBlock, 8) void emb_bwd_reduce(const ReduceArgs a) 
         const int q = item / a.passes, pass = item - q * a.passes;
         const int64_t row = row0 + q * kGroups + g;
         const bool real = row < a.rows;
-        int32_t n = real ? a.count[row] : 0;
+        const Row meta = real ? a.of(row) : Row{0, 0};
+        int32_t n = meta.count;
         const bool mine_to_write = real && n <= a.hot_above;
         if (!mine_to_write) n = 0;
         int32_t m = __builtin_amdgcn_readlane(n, 0);
@@ -463,7 +752,7 @@ __global__ __launch_bounds__(kBlock, 8) void emb_bwd_reduce(const ReduceArgs a) 
             if (col[j] > a.dim - V) col[j] = a.dim - V;          // the last vector ends with the row (or a lane has none)
         }
         if (m > 0) {                                             // the same in all lanes
-            int32_t tok = gl < n ? a.bucket[a.end[row] - n + gl] : 0x7FFFFFFF;
+            int32_t tok = gl < n ? a.bucket[meta.end - n + gl] : 0x7FFFFFFF;
             if (m > 1) {
                 int rank = 0;
                 for (int k = 0; k < m; ++k) rank += __shfl(tok, g * LPR + k, kWave) < tok ? 1 : 0;
@@ -541,31 +830,71 @@ void launch_reduce_any(const ReduceArgs& a, uint32_t hot_blocks, hipStream_t s) 
         launch_reduce<E, 1>(a, s);
 }
 
+// Chunks, segments and workspace (elems int32; 0: too many rows) of the bucketing in two launches.
+struct Split {
+    int64_t elems, chunk_tokens;
+    int shift, segment_rows, chunks;
+};
+
+Split plan_split(int64_t n_ids, int64_t rows) {
+    Split p{};
+    if (n_ids < 1 || rows > static_cast<int64_t>(kSegments) * kSegmentRows) return p;
+    p.shift = 8;
+    while ((rows - 1) >> p.shift >= kSegmentRows) ++p.shift;
+    p.segment_rows = static_cast<int>(((rows - 1) >> p.shift) + 1);
+    p.chunk_tokens = (n_ids + kChunks - 1) / kChunks;
+    if (p.chunk_tokens < 1024) p.chunk_tokens = 1024;
+    p.chunks = static_cast<int>((n_ids + p.chunk_tokens - 1) / p.chunk_tokens);
+    const int64_t segments = 1ll << p.shift;
+    p.elems = 2 * segments * p.segment_rows + 2 + 3 * n_ids + p.chunks * (segments + 1) + n_ids / (kHotAbove + 1) + 1;
+    return p;
+}
+
 template <typename IdT>
 int run(const void* dy, int dtype, int64_t dim, int64_t ld_dy, const IdT* ids, int64_t n_ids, int64_t lo, int64_t hi,
-        int64_t padding_idx, int scale_by_freq, void* dw, int64_t ld_dw, int32_t* ws, hipStream_t s) {
+        int64_t padding_idx, int scale_by_freq, void* dw, int64_t ld_dw, int32_t* ws, int64_t ws_elems, hipStream_t s) {
     const int64_t rows = hi - lo;
     const int es = dtype == DDL_DT_F32 ? 4 : 2;
     ReduceArgs a{};
     a.dy = dy, a.dw = dw, a.dim = dim, a.ld_dy = ld_dy, a.ld_dw = ld_dw, a.rows = rows, a.n_ids = n_ids;
     a.scale_by_freq = scale_by_freq;
     a.hot_above = kHotAbove;
-    // 3 rows + 1 + n_ids integers: the hot list has at most rows - 1 entries
-    int32_t* const count = ws;                              // [rows]      tokens of each row
-    int32_t* const end = ws + rows;                         // [rows]      next free slot of each row's stretch
-    int32_t* const totals = end + rows;                     // [2]
-    int32_t* const bucket = totals + 2;                     // [n_ids]
-    int32_t* const hot = bucket + n_ids;                    // [rows - 1]
-    a.count = count, a.end = end, a.bucket = bucket, a.hot = hot, a.totals = totals;
     const int64_t most_hot = std::min(rows, n_ids / (a.hot_above + 1));
     a.hot_chunks = static_cast<int32_t>((dim * es + kHotBytes - 1) / kHotBytes);
-    const uint32_t hot_blocks = static_cast<uint32_t>(std::min<int64_t>(most_hot * a.hot_chunks, 1024));
-    auto grid = [](int64_t n) { return dim3(static_cast<uint32_t>((n + kBlock - 1) / kBlock)); };
-    hipLaunchKernelGGL(emb_bwd_clear, grid(std::max<int64_t>(rows, 2)), dim3(kBlock), 0, s, count, rows, totals);
-    if (n_ids > 0) {
-        hipLaunchKernelGGL((emb_bwd_count<IdT>), grid(n_ids), dim3(kBlock), 0, s, ids, n_ids, lo, hi, padding_idx, count);
-        hipLaunchKernelGGL(emb_bwd_place, grid((rows + kPlaceRows - 1) / kPlaceRows), dim3(kBlock), 0, s, count, rows, a.hot_above, end, hot, totals);
-        hipLaunchKernelGGL((emb_bwd_fill<IdT>), grid(n_ids), dim3(kBlock), 0, s, ids, n_ids, lo, hi, padding_idx, end, bucket);
+    const uint32_t hot_blocks = static_cast<uint32_t>(std::min<int64_t>(most_hot * a.hot_chunks, 2048));
+    const Split split = plan_split(n_ids, rows);
+    if (split.elems && split.elems <= ws_elems) {
+        SplitArgs b{};
+        b.n_ids = n_ids, b.lo = lo, b.padding_idx = padding_idx, b.chunk_tokens = split.chunk_tokens;
+        b.rows = static_cast<int32_t>(rows), b.segments = 1 << split.shift, b.shift = split.shift;
+        b.hot_most = static_cast<int32_t>(n_ids / (kHotAbove + 1) + 1);
+        b.segment_rows = split.segment_rows, b.chunks = split.chunks, b.hot_above = a.hot_above;
+        b.meta = reinterpret_cast<Row*>(ws);
+        b.totals = ws + 2 * static_cast<int64_t>(b.segments) * b.segment_rows;
+        b.bucket = b.totals + 2;
+        b.token = b.bucket + n_ids;
+        b.row = b.token + n_ids;
+        b.offsets = b.row + n_ids;
+        b.hot = b.offsets + static_cast<int64_t>(b.chunks) * (b.segments + 1);
+        a.meta = b.meta, a.bucket = b.bucket, a.hot = b.hot, a.totals = b.totals;
+        a.shift = b.shift, a.segment_rows = b.segment_rows, a.hot_most = b.hot_most;
+        hipLaunchKernelGGL((emb_bwd_split<IdT>), dim3(static_cast<uint32_t>(b.chunks)), dim3(kSplitBlock), 0, s, ids, b);
+        hipLaunchKernelGGL(emb_bwd_buckets, dim3(static_cast<uint32_t>(b.segments)), dim3(kBucketBlock), 0, s, b);
+    } else {
+        // 3 rows + 1 + n_ids integers: the hot list has at most rows - 1 entries
+        Row* const meta = reinterpret_cast<Row*>(ws);           // [rows]
+        int32_t* const totals = ws + 2 * rows;                  // [2]
+        int32_t* const bucket = totals + 2;                     // [n_ids]
+        int32_t* const hot = bucket + n_ids;                    // [rows - 1]
+        a.meta = meta, a.bucket = bucket, a.hot = hot, a.totals = totals;
+        a.shift = 0, a.segment_rows = 0, a.hot_most = 0;
+        auto grid = [](int64_t n) { return dim3(static_cast<uint32_t>((n + kBlock - 1) / kBlock)); };
+        hipLaunchKernelGGL(emb_bwd_clear, grid(std::max<int64_t>(rows, 2)), dim3(kBlock), 0, s, meta, rows, totals);
+        if (n_ids > 0) {
+            hipLaunchKernelGGL((emb_bwd_count<IdT>), grid(n_ids), dim3(kBlock), 0, s, ids, n_ids, lo, hi, padding_idx, meta);
+            hipLaunchKernelGGL(emb_bwd_place, grid((rows + kPlaceRows - 1) / kPlaceRows), dim3(kBlock), 0, s, meta, rows, a.hot_above, hot, totals);
+            hipLaunchKernelGGL((emb_bwd_fill<IdT>), grid(n_ids), dim3(kBlock), 0, s, ids, n_ids, lo, hi, padding_idx, meta, bucket);
+        }
     }
     if (dtype == DDL_DT_F16)
         launch_reduce_any<F16>(a, hot_blocks, s);
@@ -576,7 +905,6 @@ int run(const void* dy, int dtype, int64_t dim, int64_t ld_dy, const IdT* ids, i
     return check_launch("embedding backward");
 }
 
-constexpr int kMaxDevices = 64;
 std::mutex scratch_mutex;
 int32_t* scratch_address[kMaxDevices] = {};   // device address of `scratch` on each GPU, filled on first use
 
@@ -622,6 +950,12 @@ extern "C" int ddl_embedding_backward_static(const void* dy, int dtype, int64_t 
                                   ld_dw, ws, DDL_EMBEDDING_BACKWARD_STATIC_MAX_ELEMS, stream);
 }
 
+extern "C" int64_t ddl_embedding_backward_workspace(int64_t n_ids, int64_t rows) {
+    using namespace ddl;
+    if (n_ids < 0 || rows < 0 || n_ids > 0x7FFFFFFFll || rows > 0x3FFFFFFFll) return 0;
+    return std::max(plan_split(n_ids, rows).elems, 3 * rows + 1 + n_ids);
+}
+
 extern "C" int ddl_embedding_backward(const void* dy, int dtype, int64_t dim, int64_t ld_dy, const void* ids, int ids_is_i64,
                                       int64_t n_ids, int64_t lo, int64_t hi, int64_t padding_idx, int scale_grad_by_freq,
                                       void* dweight, int64_t ld_dw, int32_t* workspace, int64_t workspace_elems, void* stream) {
@@ -647,7 +981,7 @@ extern "C" int ddl_embedding_backward(const void* dy, int dtype, int64_t dim, in
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (ids_is_i64)
         return run(dy, dtype, dim, ld_dy, static_cast<const int64_t*>(ids), n_ids, lo, hi, padding_idx, scale_grad_by_freq != 0, dweight,
-                   ld_dw, workspace, s);
+                   ld_dw, workspace, workspace_elems, s);
     return run(dy, dtype, dim, ld_dy, static_cast<const int32_t*>(ids), n_ids, lo, hi, padding_idx, scale_grad_by_freq != 0, dweight, ld_dw,
-               workspace, s);
+               workspace, workspace_elems, s);
 }

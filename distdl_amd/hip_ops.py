@@ -717,6 +717,12 @@ def embedding_renorm(weight, ids, lo, hi, max_norm, norm_type=2.0):
     return weight
 
 
+@functools.lru_cache(maxsize=4096)
+def _embedding_backward_workspace(n_ids, rows):
+    """int32 words with which the adjoint takes the fewest launches (a function of its arguments alone)."""
+    return _lib.load().ddl_embedding_backward_workspace(n_ids, rows)
+
+
 def embedding_backward(grad_output, ids, lo, hi, padding_idx=None, scale_grad_by_freq=False):
     """Gradient of :func:`embedding_gather` with respect to the ``[hi-lo, dim]``
     table; with ``scale_grad_by_freq`` every row's sum is divided by the number
@@ -735,7 +741,8 @@ def embedding_backward(grad_output, ids, lo, hi, padding_idx=None, scale_grad_by
     ids_c = contiguous(ids)
     rows, n_ids = int(hi) - int(lo), ids_c.numel()
     dw = torch.empty((rows, dim), dtype=grad_output.dtype, device=grad_output.device)
-    work = torch.empty(3 * rows + 1 + n_ids, dtype=torch.int32, device=grad_output.device)
+    work = torch.empty(max(3 * rows + 1 + n_ids, _embedding_backward_workspace(n_ids, rows)), dtype=torch.int32,
+                       device=grad_output.device)
     dt = _LN_DTYPES[grad_output.dtype]
     rc = _lib.load().ddl_embedding_backward(dy.data_ptr(), dt, dim, dy.stride(0) if n_ids > 1 else dim, ids_c.data_ptr(),
                                             1 if ids.dtype == torch.int64 else 0, n_ids, int(lo), int(hi),

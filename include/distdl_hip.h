@@ -433,7 +433,9 @@ int ddl_embedding_renorm(void* weight, int dtype, int64_t dim, int64_t ldw,
  * Every element of dweight is written, so it needs no clearing.  `workspace`:
  * device memory for at least 3 (hi-lo) + 1 + n_ids int32 (token counts, bucket
  * cursors and bucket starts of the rows, then the buckets), contents on entry
- * do not matter. */
+ * do not matter.  With ddl_embedding_backward_workspace(n_ids, hi-lo) int32 the
+ * tokens are bucketed in fewer launches; the results are the same. */
+int64_t ddl_embedding_backward_workspace(int64_t n_ids, int64_t rows);
 int ddl_embedding_backward(const void* dy, int dtype, int64_t dim, int64_t ld_dy,
                            const void* ids, int ids_is_i64, int64_t n_ids,
                            int64_t lo, int64_t hi, int64_t padding_idx,

@@ -1151,6 +1151,38 @@ def test_embedding_backward_bucket_lengths(ops, dtype, dim, misses):
     assert torch.equal(got.cpu(), want.to(dtype))
 
 
+@pytest.mark.parametrize("rows,tokens,hot", [(1, 1, 0), (255, 1023, 40), (257, 1025, 513), (300, 1024, 1024), (5000, 20000, 4000), (5000, 20000, 4200),
+                                             (2 ** 20, 70000, 600), (2 ** 20 + 1, 5000, 33), (700, 131072, 9000), (700, 131073, 9000)])
+def test_embedding_backward_bucketing_by_segments(ops, rows, tokens, hot):
+    """The bucketing in two launches against the four that need less workspace (but for large tables), bit for bit, and both
+    against float64: one
+    row and one token, a chunk of tokens and one more or less, segments with as many tokens as are held in LDS and with
+    more (two hot rows share a segment), rows on either side of the lengths at which their ordering changes, table sizes
+    on either side of a doubling of the segments, more tokens than one window of bits."""
+    from distdl_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(rows + tokens)
+    lo, pad, dim = 9, 9 + rows // 3, 5
+    ids = torch.randint(0, rows + 20, (tokens,), generator=gen, device="cuda")
+    where = torch.randperm(tokens, generator=gen, device="cuda")
+    ids[where[:hot]] = lo + rows - 1
+    ids[where[hot:hot + min(hot, 300)]] = lo + max(0, rows - 257)       # the same segment as the last row
+    dy = torch.randn(tokens, dim, generator=gen, device="cuda")
+    got = ops.embedding_backward(dy, ids, lo, lo + rows, padding_idx=pad)
+    few = torch.full((rows, dim), 7.0, device="cuda")
+    work = torch.full((3 * rows + 1 + tokens,), -1, dtype=torch.int32, device="cuda")
+    assert rows >= 2 ** 20 or ops._embedding_backward_workspace(tokens, rows) > work.numel()
+    rc = lib.ddl_embedding_backward(dy.data_ptr(), _lib.DDL_DT_F32, dim, dim, ids.data_ptr(), 1, tokens, lo, lo + rows, pad, 0,
+                                    few.data_ptr(), dim, work.data_ptr(), work.numel(), ops._stream())
+    assert rc == 0
+    assert torch.equal(got.view(torch.int32), few.view(torch.int32))
+    keep = (ids >= lo) & (ids < lo + rows) & (ids != pad)
+    want = torch.zeros(rows, dim, dtype=torch.float64, device="cuda").index_add_(0, ids[keep] - lo, dy[keep].double())
+    size = torch.zeros(rows, dim, dtype=torch.float64, device="cuda").index_add_(0, ids[keep] - lo, dy[keep].double().abs())
+    count = torch.bincount(ids[keep] - lo, minlength=rows)[:, None]
+    assert bool(((got.double() - want).abs() <= 2.0 ** -24 * count * size).all())    # one rounding per addition
+
+
 def test_embedding_backward_of_one_row_takes_time_in_proportion_to_its_tokens(ops):
     """Every token the same id: exact sums (small integers), and four times the tokens take about four times as long (4.5
     measured; ordering the bucket anew for every 1024 of its tokens made it 22)."""
