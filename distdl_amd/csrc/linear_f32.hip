@@ -21,14 +21,10 @@
 //              and stores them to the other stage
 //
 // This kernel takes any strides and size.  Products whose operands have a unit
-// stride go to the kernels of linear_f32_small.hip or, where those fill the chip and
-// the operands are aligned to 16 bytes, of linear_f32_tiles.hip instead.
+// stride go to the kernels of linear_f32_small.hip and linear_f32_split.hip instead.
 #include "gemm32_small.h"
 
 namespace ddl {
-
-int gemm_f32_tiled(const float* a, int64_t a_rs, int64_t a_ks, const float* b, int64_t b_rs, int64_t b_ks, const float* bias, float* y,
-                   int64_t ldy, int64_t M, int64_t N, int64_t K, void* stream);
 
 namespace {
 
@@ -201,9 +197,6 @@ bool vector_ok(const Operand& o, bool along_k) {
 
 namespace ddl {
 
-// gemm_f32_tiled takes the product (`aligned`: as far as the pointers go).
-bool gemm_f32_tiled_ok(bool aligned, int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K);
-
 namespace {
 
 // Can linear_f32_small.hip read this operand (`rows` rows)?  Offsets inside a tile are 32-bit bytes; an operand read along
@@ -215,20 +208,13 @@ bool small_ok(int64_t rs, int64_t ks, int64_t rows, int64_t K) {
 
 }  // namespace
 
-// How linear_f32_small.hip computes the product, if it does (sizes and strides as in ddl_gemm_f32).
-Small32 plan32(bool aligned, int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K, int cus,
-               int64_t workspace) {
-    if (!small_ok(a_rs, a_ks, M, K) || !small_ok(b_rs, b_ks, N, K)) return Small32{};
-    double other_us = 1e30;   // the general kernel: never faster
-    if (gemm_f32_tiled_ok(aligned, a_rs, a_ks, b_rs, b_ks, M, N, K)) {
-        // 256 x 256 tiles: per round 45 us and 5 (few CUs at work) to 7.25 us per k-tile
-        int64_t cost = 0;
-        const int64_t tiles_m = (M + 255) / 256, tiles = tiles_m * ((N + 255) / 256);
-        wide_tile_columns(tiles_m, N, cus, &cost);
-        const double fill = tiles < cus ? static_cast<double>(tiles) / cus : 1.0;
-        other_us = cost / 256.0 * (45 + static_cast<double>((K + 31) / 32) * (5 + 2.25 * fill * fill));
-    }
-    return plan_small32(M, N, K, cus, workspace, other_us);
+// How linear_f32_small.hip or linear_f32_split.hip computes the product, if one does (sizes and strides as in ddl_gemm_f32).
+Small32 plan32(int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace) {
+    if ((a_ks != 1 && a_rs != 1) || (b_ks != 1 && b_rs != 1)) return Small32{};
+    Small32 small;
+    if (small_ok(a_rs, a_ks, M, K) && small_ok(b_rs, b_ks, N, K)) small = plan_small32(M, N, K, cus, workspace);
+    const Small32 split = plan_split32(M, N, K, cus, workspace, small);
+    return split.edge ? split : small;
 }
 
 // ddl_gemm_f32 with room for the sums of a split reduction (may be null).
@@ -244,18 +230,15 @@ int gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride, const flo
     if (!aligned_to(a, 4) || !aligned_to(b, 4) || !aligned_to(y, 4) || !aligned_to(bias, 4)) return fail(DDL_E_ALIGN, "gemm f32: pointer misaligned");
     int dev = 0;
     const int cus = compute_units(dev);
-    const bool aligned = aligned_to(a, 16) && aligned_to(b, 16);
-    const Small32 small = plan32(aligned, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, workspace ? workspace_elems : 0);
-    if (small.groups) {
+    const Small32 small = plan32(a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, workspace ? workspace_elems : 0);
+    if (small.groups || small.edge) {
         const bool at = a_k_stride != 1, bt = b_k_stride != 1;
         PartOf<float> part{};
         part.x = a, part.w = b, part.bias = bias, part.y = y, part.M = M, part.N = N, part.K = K;
         part.ldx = at ? a_k_stride : a_row_stride, part.ldw = bt ? b_k_stride : b_row_stride, part.ldy = ldy;
-        part.vec_store = ldy % 4 == 0 && aligned_to(y, 16);
+        if (small.edge) return run_split32(small, at, bt, part, workspace, static_cast<hipStream_t>(stream));
         return run_small32("gemm f32", small, at, bt, part, workspace, dev, static_cast<hipStream_t>(stream));
     }
-    if (gemm_f32_tiled_ok(aligned, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K))
-        return gemm_f32_tiled(a, a_row_stride, a_k_stride, b, b_row_stride, b_k_stride, bias, y, ldy, M, N, K, stream);
     const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     if (tiles_m * tiles_n > 0x7FFFFFFFll || tiles_m > 0x7FFFFFFFll) return fail(DDL_E_UNSUPP, "gemm f32: too many output tiles");
     const Operand oa{a, a_row_stride, a_k_stride, M}, ob{b, b_row_stride, b_k_stride, N};

@@ -1,6 +1,5 @@
-// fp32 linear products that 256 x 256 tiles leave most of the chip idle for, and
-// those whose pitches or lengths are no multiples of four floats:
-// y[M,N] = a[M,K] . b[N,K]^T + bias[N] on v_mfma_f32_32x32x2_f32.
+// fp32 linear products too small to fill the chip with the 128 x 128 tiles of
+// linear_f32_split.hip: y[M,N] = a[M,K] . b[N,K]^T + bias[N] on v_mfma_f32_32x32x2_f32.
 //
 // Bound by the matrix cores of the CUs that have work (a 64 x 64 tile of K 1024 is
 // 14 us on one CU), so tiles are small and the reduction is split wherever that
@@ -10,9 +9,15 @@
 // `splits` workgroups share the reduction of a tile through a workspace;
 // gemm32_small_sum adds their sums in the order of the splits.
 //
-// Tiles go from global memory straight into LDS through a ring of stages, in the
-// layouts of linear_f32_tiles.hip (k-tiles of 32 floats; rows with swizzled chunks,
-// or panels of 32 rows x 32 k-lines for an operand contiguous along its rows).  A
+// Tiles go from global memory straight into LDS through a ring of stages: k-tiles of
+// 32 floats; an operand contiguous along k in rows of 128 bytes whose 16-byte chunks are
+// XOR-ed with (row >> 1) & 7 (lane (r = lane % 32, h = lane / 32) reads chunk 2 g + h of row
+// r and feeds its four floats to the four matrix instructions of k-group g: any
+// assignment of k to lanes and steps is valid if both operands use the same one); an
+// operand contiguous along its rows as it lies in memory, in panels of 32 rows x 32
+// k-lines of 128 bytes (lane (r, h) reads element r of k-line 8 g + 4 h + e; lines k and
+// k + 4 would start on the same bank, so the lines 4..7 of every eight are stored with
+// neighbours swapped).  A
 // request reads 16 bytes per lane from any 4-byte-aligned address, so pitches and
 // lengths are free: only the k-tile that straddles K, and the last one of an operand
 // read along rows whose number is no multiple of four (a chunk there runs over into
@@ -28,33 +33,9 @@ namespace ddl {
 namespace {
 
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 constexpr int BK = kRowBytes / 4;   // floats of a k-tile
 typedef PartOf<float> Part32;
-
-__device__ inline void store_four(float* __restrict__ dst, int64_t n, int64_t N, const floatx4& v, bool vec) {
-    if (vec && n + 3 < N) {
-        *reinterpret_cast<floatx4*>(dst) = v;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (n + e < N) dst[e] = v[e];
-    }
-}
-
-// The bias of columns n .. n + 3 (zeros without one, and past the end).
-__device__ inline floatx4 bias_of(const float* __restrict__ bias, int64_t n, int64_t N) {
-    float b[4] = {0.f, 0.f, 0.f, 0.f};
-    if (bias) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float f = bias[n + e < N ? n + e : N - 1];
-            b[e] = n + e < N ? f : 0.f;
-        }
-    }
-    return floatx4{b[0], b[1], b[2], b[3]};
-}
 
 template <bool XT, bool WT, int NWM, int NWN, int KG, int STAGES>
 __global__ __launch_bounds__(256) void gemm32_small(const Part32 p, int splits, float* __restrict__ partial) {
@@ -220,7 +201,7 @@ __global__ __launch_bounds__(256) void gemm32_small(const Part32 p, int splits, 
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const int64_t n = n0 + sub_w * 32 + 8 * g + 4 * kh;
-        store_four(p.y + m * p.ldy + n, n, N, quad[g] + bias_of(p.bias, n, N), p.vec_store != 0);
+        store_four(p.y + m * p.ldy + n, n, N, quad[g] + bias_of(p.bias, n, N));
     }
 }
 
@@ -248,7 +229,13 @@ __global__ __launch_bounds__(256) void gemm32_small_sum(const Part32 p, int spli
         for (int u = 0; u < 4; ++u) s += v[u];
     }
     for (; k < splits; ++k) s += src[k * stride];
-    store_four(p.y + m * p.ldy + n, n, p.N, s + bias_of(p.bias, n, p.N), p.vec_store != 0);
+    store_four(p.y + m * p.ldy + n, n, p.N, s + bias_of(p.bias, n, p.N));
+}
+
+template <int NWM, int NWN>
+int launch_sum(const Part32& part, int splits, const float* partial, hipStream_t s) {
+    hipLaunchKernelGGL((gemm32_small_sum<NWM, NWN>), dim3(static_cast<uint32_t>(part.tiles_m * part.tiles_n * NWM * NWN)), dim3(256), 0, s, part, splits, partial);
+    return check_launch("gemm32_small_sum");
 }
 
 template <bool XT, bool WT, int NWM, int NWN, int KG>
@@ -265,10 +252,7 @@ int launch(const char* who, Part32 part, int splits, float* partial, int dev, hi
     const int ntiles = part.tiles_m * part.tiles_n;
     hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(ntiles * splits)), dim3(256), lds_bytes, s, part, splits, partial);
     if (int rc = check_launch("gemm32_small")) return rc;
-    if (splits == 1) return 0;
-    hipLaunchKernelGGL((gemm32_small_sum<NWM, NWN>), dim3(static_cast<uint32_t>(ntiles * NWM * NWN)), dim3(256), 0, s, part, splits,
-                       static_cast<const float*>(partial));
-    return check_launch("gemm32_small_sum");
+    return splits == 1 ? 0 : launch_sum<NWM, NWN>(part, splits, partial, s);
 }
 
 template <bool XT, bool WT>
@@ -286,12 +270,11 @@ int launch_shape(const char* who, const Small32& plan, const Part32& part, float
 // what it and the workspace cost the host, which many callers wait for) and the partial tiles at 5 TB/s.
 // Measured, general kernel of 128 x 128 tiles -> here: M 777, N 333, K 1024 107.2 -> 17.7 (two groups; 15.7 in three
 // splits, which the host's share makes the slower call); its adjoint M 777, N 1024, K 333 45.4 -> 12.4 and M 333, N 1024, K 777, both operands along their rows, 84.1 ->
-// 15.6; M 8, N 4096, K 4096 365 -> 20.  256 x 256 tiles -> here: M = N = K = 2048 351 -> 153, M 4096, N 4096, K 1024 310 ->
-// 294; M = N = K = 4096 973, here 1060: those stay.
-Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double other_us) {
+// 15.6; M 8, N 4096, K 4096 365 -> 20.
+Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace) {
     Small32 best;
     const int64_t ktiles = (K + BK - 1) / BK;
-    double best_us = other_us * 0.95;   // what the fits are unsure of
+    double best_us = 1e30;
     for (const int groups : {1, 2, 4}) {
         const int64_t bm = groups == 1 ? 64 : 32, bn = groups == 4 ? 32 : 64, tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
         if (tiles > 0xFFFFFF) continue;   // a launch has fewer than 2^32 threads, 256 per tile
@@ -304,7 +287,7 @@ Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace
             else
                 us += ((kt + groups - 1) / groups) * 0.78 * per_cu + (per_cu - 1) * (groups == 2 ? 1.5 : 3.0);
             if (us >= best_us) continue;
-            best_us = us;
+            best_us = best.us = us;
             best.groups = groups, best.splits = splits, best.workspace = splits > 1 ? tiles * splits * bm * bn : 0;
         }
     }
@@ -316,6 +299,10 @@ int run_small32(const char* who, const Small32& plan, bool xt, bool wt, const Pa
     if (xt) return launch_shape<true, false>(who, plan, part, partial, dev, s);
     if (wt) return launch_shape<false, true>(who, plan, part, partial, dev, s);
     return launch_shape<false, false>(who, plan, part, partial, dev, s);
+}
+
+int sum_small32(const PartOf<float>& part, int blocks, int splits, const float* partial, hipStream_t s) {
+    return blocks == 2 ? launch_sum<2, 2>(part, splits, partial, s) : launch_sum<4, 4>(part, splits, partial, s);
 }
 
 }  // namespace ddl

@@ -637,8 +637,7 @@ namespace ddl {
 int gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride, const float* b, int64_t b_row_stride, int64_t b_k_stride,
              const float* bias, float* y, int64_t ldy, int64_t M, int64_t N, int64_t K, float* workspace, int64_t workspace_elems,
              void* stream);
-Small32 plan32(bool aligned, int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K, int cus,
-               int64_t workspace);
+Small32 plan32(int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace);
 }  // namespace ddl
 
 extern "C" int ddl_linear_bf16(const void* x, const void* w, const void* bias, void* y, int64_t M, int64_t N, int64_t K,
@@ -701,7 +700,7 @@ extern "C" int64_t ddl_gemm_workspace_at(int dtype, int aligned, int64_t a_row_s
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     int dev = 0;
     const int cus = compute_units(dev);
-    if (dtype == DDL_DT_F32) return plan32(aligned != 0, a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, INT64_MAX).workspace;
+    if (dtype == DDL_DT_F32) return plan32(a_row_stride, a_k_stride, b_row_stride, b_k_stride, M, N, K, cus, INT64_MAX).workspace;
     if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return 0;
     const Operand16 a{nullptr, a_row_stride, a_k_stride}, b{nullptr, b_row_stride, b_k_stride};
     if (aligned && pitches_ok(a, M, K) && pitches_ok(b, N, K)) return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;

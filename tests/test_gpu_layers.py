@@ -1878,6 +1878,65 @@ def test_gemm_f32_products_of_every_size_and_pitch(ops, a_t, b_t, M, N, K, pad, 
         assert (got[:, N:] == 77.0).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(1300, 1411, 1), (1281, 1408, 15), (1280, 1409, 16), (1300, 1411, 17), (1279, 1410, 33), (1300, 1411, 79), (129, 1411, 4099),
+                                   (2049, 130, 1000), (128, 128, 8200)])
+@pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
+def test_gemm_f32_by_exact_bf16_parts(ops, a_t, b_t, M, N, K):
+    """Products large enough for 128 x 128 tiles on the bf16 matrix cores: partial tiles, every remainder of the k-tiles, the
+    reduction in one piece and split, rows of odd length that start anywhere, operands as they lie.  The error against float64
+    is that of fp32 sums (K/16 additions of six parts, each rounded once), and no larger than the fp32 matrix instruction's
+    was (1.5e-6 for the longest of these sums, in the 2-norm)."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+
+    def operand(rows, transposed):
+        shape = (K, rows) if transposed else (rows, K)
+        store = torch.full((shape[0] * (shape[1] + 3) + 1,), float("nan"), device="cuda")
+        t = store[1:].as_strided(shape, (shape[1] + 3, 1), 1)
+        t.copy_(torch.randn(shape, generator=gen, device="cuda"))
+        return t, (1, shape[1] + 3) if transposed else (shape[1] + 3, 1)
+    a, sa = operand(M, a_t)
+    b, sb = operand(N, b_t)
+    bias = torch.randn(N, generator=gen, device="cuda")
+    out = torch.empty(M, N, device="cuda")
+    ops._gemm(a, *sa, b, *sb, bias, out, ops._LINEAR_DTYPES[torch.float32], M, N, K)
+    a64, b64 = (a.t() if a_t else a).double(), (b.t() if b_t else b).double()
+    want = a64 @ b64.t() + bias.double()
+    assert float((out.double() - want).norm() / want.norm()) <= 1.5e-6
+    assert bool(((out.double() - want).abs() <= (K + 2) * 2.0 ** -24 * (a64.abs() @ b64.abs().t() + bias.double().abs())).all())
+
+
+@pytest.mark.parametrize("K", [48, 1000])
+def test_gemm_f32_of_values_that_bf16_parts_cannot_carry(ops, K):
+    """Infinities, NaN, values next to the largest float and large ones, rows so small that their parts would be denormal, and zeros: the
+    products are those of fp32 arithmetic, and tiles without such values are not touched by the others."""
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    M = N = 1400
+    x, w = torch.randn(M, K, generator=gen, device="cuda"), torch.randn(N, K, generator=gen, device="cuda")
+    plain = ops.linear(x, w)
+    x[5, 3], x[6, 4], x[140, 7] = float("inf"), float("-inf"), float("nan")
+    x[300] *= 2.0 ** -120
+    x[301] = 0
+    x[600] = 2.0 ** 127 * 1.99999
+    w[0] = 1.0                    # exactly bf16: its smaller parts are zero, and infinity times zero is not a number
+    w[1] = 0
+    w[900] *= 2.0 ** -110
+    w[1399, 0] = 1e37
+    got = ops.linear(x, w).cpu()
+    want = x.cpu().double() @ w.cpu().double().t()
+    as32 = want.float()           # overflow to infinity as fp32 has it, where no partial sum is close to it
+    size = x.cpu().double().abs() @ w.cpu().double().abs().t()
+    sure = ~((size > 3.0e38) & (size < float("inf")))
+    assert torch.equal(got.isnan()[sure], as32.isnan()[sure]) and torch.equal(got.isinf()[sure], as32.isinf()[sure])
+    assert torch.equal(got[as32.isinf() & sure], as32[as32.isinf() & sure])
+    ok = sure & as32.isfinite()
+    assert bool(((got.double() - want).abs()[ok] <= (K + 2) * 2.0 ** -24 * size[ok] + 2.0 ** -149 * K).all())
+    untouched = torch.ones(M, dtype=torch.bool)
+    untouched[:256] = untouched[256:384] = untouched[512:640] = False     # the tiles' rows
+    columns = torch.ones(N, dtype=torch.bool)
+    columns[:128] = columns[896:1024] = columns[1280:] = False
+    assert torch.equal(got[untouched][:, columns], plain.cpu()[untouched][:, columns])
+
+
 def test_gemm_f32_tiled_kernel_random_and_odd_depth(ops):
     """Random operands through the tiled fp32 kernel: both operands read along
     their rows, so the reduction length may be anything (here 1003, no multiple
