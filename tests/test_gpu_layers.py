@@ -1878,7 +1878,7 @@ def test_gemm_f32_products_of_every_size_and_pitch(ops, a_t, b_t, M, N, K, pad, 
         assert (got[:, N:] == 77.0).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(1300, 1411, 1), (1281, 1408, 15), (1280, 1409, 16), (1300, 1411, 17), (1279, 1410, 33), (1300, 1411, 79), (129, 1411, 4099),
+@pytest.mark.parametrize("M,N,K", [(1300, 1411, 3), (1281, 1408, 15), (1280, 1409, 16), (1300, 1411, 17), (1279, 1410, 33), (1300, 1411, 79), (129, 1411, 4099),
                                    (2049, 130, 1000), (128, 128, 8200)])
 @pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
 def test_gemm_f32_by_exact_bf16_parts(ops, a_t, b_t, M, N, K):
