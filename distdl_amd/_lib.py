@@ -163,6 +163,23 @@ def load():
     return lib
 
 
+_front = None
+
+
+def front():
+    """The extension with the tensor front ends (csrc/front.cpp), loaded once."""
+    global _front
+    if _front is None:
+        load()
+        try:
+            from . import _front as module
+        except ImportError as e:
+            raise HipLibraryMissing(f"distdl_amd._front is not built or does not load ({e}); run `make -C "
+                                    f"{os.path.join(_HERE, 'csrc')}` (or __graft_entry__.build()).") from e
+        _front = module
+    return _front
+
+
 def check(rc, what):
     if rc != 0:
         msg = load().ddl_last_error().decode("utf-8", "replace")

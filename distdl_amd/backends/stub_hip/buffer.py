@@ -52,8 +52,10 @@ class ExpandableBuffer:
         self.get_view(tuple(view_shape))
 
     def get_view(self, view_shape):
-        view_shape = tuple(int(s) for s in view_shape)
-        view = self.views.get(view_shape)
+        view = self.views.get(view_shape) if type(view_shape) is tuple else None
+        if view is None:
+            view_shape = tuple(int(s) for s in view_shape)
+            view = self.views.get(view_shape)
         if view is None:
             volume = int(np.prod(view_shape, dtype=np.int64))
             if volume > self.capacity:

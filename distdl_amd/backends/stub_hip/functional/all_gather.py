@@ -14,6 +14,7 @@ import functools
 import numpy as np
 import torch
 
+from .... import _lib
 from .... import hip_ops
 from ....utilities.slicing import compute_subshape
 
@@ -55,11 +56,15 @@ def gather_slabs(P, local, axis, tag):
     transport = P._world.transport
     x = hip_ops.contiguous(local)
     parts = transport.gather_list(P, x, tag=tag)
+    axis = range(x.dim())[axis]      # an axis the tensor has not is an IndexError
+    out = _lib.front().join(x, parts, axis)
+    if out is not None:
+        transport.release(P, tag=tag)
+        return out
     hip_ops._require_gpu(x, *parts)
     for p in parts:
         if p.dtype != x.dtype or not p.is_contiguous():
             raise ValueError(f"gathered piece {tuple(p.shape)}/{p.dtype} does not match {x.dtype} or is not contiguous")
-    axis = range(x.dim())[axis]      # an axis the tensor has not is an IndexError
     shape, launch = _gather_launch(tuple(x.shape), tuple([tuple(p.shape) for p in parts]), axis, x.element_size())
     out = torch.empty(shape, dtype=x.dtype, device=x.device)
     launch.run([out.data_ptr()] + [p.data_ptr() for p in parts])
@@ -75,7 +80,13 @@ def reduce_scatter_slabs(P, full, axis, tag, divisor=1):
     transport = P._world.transport
     g = hip_ops.contiguous(full)
     grads = transport.gather_list(P, g, tag=tag)
-    shape, src, dst = _slab(int(P.size), int(P.rank), tuple(g.shape), range(g.dim())[axis])
+    axis = range(g.dim())[axis]
+    shape, src, dst = _slab(int(P.size), int(P.rank), tuple(g.shape), axis)
+    out = _lib.front().sum_slab(grads, axis, src[axis].start, shape[axis], divisor) if len(grads) and grads[0].shape == g.shape and \
+        grads[0].dtype == g.dtype else None
+    if out is not None:
+        transport.release(P, tag=tag)
+        return out
     out = torch.empty(shape, dtype=g.dtype, device=g.device)
     if out.numel():
         hip_ops.sum_boxes(grads, src, out, dst, divisor)

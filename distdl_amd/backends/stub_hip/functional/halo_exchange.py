@@ -76,7 +76,7 @@ class _Plan:
         first = [(_INPUT, 0, _TENSOR, 0, list(shape), strides, tensor_strides)]
         untouched = True
         for i in range(dims):
-            extents = [compute_nd_slice_shape(s) for s in slices[i]]
+            extents = [tuple(int(n) for n in compute_nd_slice_shape(s)) for s in slices[i]]
             if forward:
                 pack, unpack = boxes(i, bulk, True, untouched), boxes(i, ghost, False)
                 merged = untouched

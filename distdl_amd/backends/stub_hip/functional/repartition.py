@@ -15,12 +15,9 @@ always do for a valid pair of partitions).
 
 __all__ = ["RepartitionFunction"]
 
-import ctypes
-
 import numpy as np
 import torch
 
-from .... import _lib
 from .... import hip_ops
 from ....utilities.torch import zero_volume_tensor
 from .. import buffer as _buffer
@@ -86,15 +83,7 @@ def _covered(overlaps, shape):
     return covered
 
 
-def _contiguous_strides(shape):
-    strides, run = [], 1
-    for n in reversed(shape):
-        strides.append(run)
-        run *= int(n)
-    return strides[::-1]
-
-
-_BOX_WORDS = ctypes.sizeof(_lib.ddl_box_t) // 8     # a box descriptor as 8-byte words; words 0 and 1 are src and dst
+_SRC, _OUT, _FIXED = 0, 1, 2     # base addresses of a launch: the source tensor, the output, 0 (buffers, by their address)
 
 
 class _MovePlan:
@@ -105,8 +94,8 @@ class _MovePlan:
               worker keeps copied straight into the output
       second  every receive buffer unpacked into the output
 
-    The box descriptors are built here; a call only writes the addresses that
-    change (the source tensor, the fresh output) into them.  Buffer views have
+    The box descriptors are built here; a call only adds the addresses that
+    change (the source tensor, the fresh output).  Buffer views have
     fixed addresses until some pooled buffer is reallocated, which invalidates
     the plan (``stale``).
     """
@@ -121,82 +110,40 @@ class _MovePlan:
         self.keep = (src_overlaps, src_buffers, dst_overlaps, dst_buffers)     # ids of these are part of the cache key
         self.out_shape = None if dst_shape is None else tuple(int(n) for n in dst_shape)
         self.zero_fill = dst_active and not _covered(dst_overlaps, self.out_shape)
-        es = self.elem_size
         src_strides = [int(v) for v in src.stride()]
-        out_strides = _contiguous_strides(self.out_shape) if dst_active else None
+        out_strides = hip_ops.contiguous_strides(self.out_shape) if dst_active else None
 
         def offset(slices, strides):
-            return sum(int(sl.start) * st for sl, st in zip(slices, strides)) * es
+            return sum(int(sl.start) * st for sl, st in zip(slices, strides))
 
-        first, second = [], []      # (src address or None, src offset, dst address or None, dst offset, shape, sstr, dstr)
+        def at(view):
+            return view.data_ptr() // self.elem_size      # in elements from address 0; views start at a multiple of their elements
+
+        first, second = [], []
         if src_active:
             for (sl, sh, partner), view in zip(src_overlaps, self.send_views):
                 if view is not None and view.numel() > 0:
                     shape = [int(n) for n in sh]
-                    first.append((None, offset(sl, src_strides), view.data_ptr(), 0, shape, src_strides,
-                                  _contiguous_strides(shape)))
+                    first.append((_SRC, offset(sl, src_strides), _FIXED, at(view), shape, src_strides, hip_ops.contiguous_strides(shape)))
             s_self, d_self = _self_slices(src_overlaps), (_self_slices(dst_overlaps) if dst_active else None)
             if s_self is not None and d_self is not None:
                 shape = [int(sl.stop) - int(sl.start) for sl in s_self]
                 if int(np.prod(shape, dtype=np.int64)) > 0:
-                    first.append((None, offset(s_self, src_strides), None, offset(d_self, out_strides), shape, src_strides,
-                                  out_strides))
+                    first.append((_SRC, offset(s_self, src_strides), _OUT, offset(d_self, out_strides), shape, src_strides, out_strides))
         if dst_active:
             for (sl, sh, partner), view in zip(dst_overlaps, self.recv_views):
                 if view is not None and view.numel() > 0:
                     shape = [int(n) for n in sh]
-                    second.append((view.data_ptr(), 0, None, offset(sl, out_strides), shape, _contiguous_strides(shape),
-                                   out_strides))
-        self.first = self._lower(first)
-        self.second = self._lower(second)
+                    second.append((_FIXED, at(view), _OUT, offset(sl, out_strides), shape, hip_ops.contiguous_strides(shape), out_strides))
+        self.first = hip_ops.BoxLaunch(first, self.elem_size)
+        self.second = hip_ops.BoxLaunch(second, self.elem_size)
         self.sends = [(partner, view) for (sl, sh, partner), view in zip(src_overlaps, self.send_views) if view is not None] \
             if src_active else []
         self.recvs = [(partner, view) for (sl, sh, partner), view in zip(dst_overlaps, self.recv_views) if view is not None] \
             if dst_active else []
 
-    @staticmethod
-    def _lower(entries):
-        """(box array, its words as a NumPy table, rows / offsets of the
-        addresses that follow the source tensor, the same for the output)."""
-        n = len(entries)
-        if n == 0:
-            return None
-        boxes = (_lib.ddl_box_t * n)()
-        words = np.frombuffer(boxes, dtype=np.int64).reshape(n, _BOX_WORDS)
-        from_src, from_out = ([], []), ([], [])
-        for i, (sa, so, da, do, shape, sstr, dstr) in enumerate(entries):
-            box = boxes[i]
-            box.ndim = len(shape)
-            for d, (nd, s1, s2) in enumerate(zip(shape, sstr, dstr)):
-                box.shape[d], box.src_stride[d], box.dst_stride[d] = nd, s1, s2
-            if sa is None:
-                from_src[0].append(i)
-                from_src[1].append(so)
-            else:
-                box.src = sa
-            if da is None:
-                from_out[0].append(i)
-                from_out[1].append(do)
-            else:
-                box.dst = da
-        return (boxes, words, n,
-                (np.asarray(from_src[0], dtype=np.intp), np.asarray(from_src[1], dtype=np.int64)),
-                (np.asarray(from_out[0], dtype=np.intp), np.asarray(from_out[1], dtype=np.int64)))
-
     def stale(self):
         return self.reallocations != _buffer.reallocations()
-
-    def launch(self, which, src_ptr, out_ptr, stream):
-        if which is None:
-            return
-        boxes, words, n, (src_rows, src_offs), (out_rows, out_offs) = which
-        if len(src_rows):
-            words[src_rows, 0] = src_offs + src_ptr
-        if len(out_rows):
-            words[out_rows, 1] = out_offs + out_ptr
-        rc = _lib.load().ddl_copy_boxes(boxes, n, self.elem_size, _lib.DDL_OP_COPY, _lib.DDL_DT_BITS, stream)
-        if rc:
-            _lib.check(rc, "ddl_copy_boxes")
 
 
 def _move_plan(src, dtype, P_src, src_overlaps, src_buffers, P_dst, dst_overlaps, dst_buffers, dst_shape):
@@ -234,12 +181,12 @@ def _move(src, P_union, dtype, P_src, src_overlaps, src_buffers, P_dst, dst_over
         out = zero_volume_tensor(src.shape[0], dtype=dtype, device=device) if preserve_batch else \
             zero_volume_tensor(dtype=dtype, device=device)
         out_ptr = 0
-    stream = hip_ops._stream()
-    plan.launch(plan.first, src.data_ptr() if P_src.active else 0, out_ptr, stream)
+    bases = [src.data_ptr() if P_src.active else 0, out_ptr, 0]
+    plan.first.run(bases)
     if P_union.active and (plan.sends or plan.recvs):
         P_union._world.transport.exchange(P_union, [(p, v, tag) for p, v in plan.sends],
                                           [(p, v, tag) for p, v in plan.recvs])
-    plan.launch(plan.second, 0, out_ptr, stream)
+    plan.second.run(bases)
     return out
 
 

@@ -1,6 +1,8 @@
 """Torch-tensor front end of the C ABI: device checks, pointer extraction and
 the current HIP stream.  Nothing here computes; every function ends in one call
-into ``libdistdl_hip.so`` and raises when that is impossible.
+into ``libdistdl_hip.so`` and raises when that is impossible.  The functions that
+layers call step by step first offer their operands to their native counterpart
+(``_lib.front()``), which takes the usual forms and answers None to any other.
 """
 
 import ctypes
@@ -166,8 +168,8 @@ class BoxLaunch:
     ``entries`` are ``(src slot, src offset, dst slot, dst offset, shape, src
     strides, dst strides)``, offsets and strides in elements of ``elem_size``
     bytes; a slot is an index into the base addresses that a call supplies.
-    Boxes without elements are left out.  A call fills a copy of the
-    descriptors, so threads may share an object."""
+    Boxes without elements are left out.  A call only reads the object, so
+    threads may share it."""
 
     def __init__(self, entries, elem_size):
         entries = [e for e in entries if min(e[4], default=1) > 0]
@@ -183,17 +185,15 @@ class BoxLaunch:
             packed.append(_BOX.pack(0, 0, nd, 0, *shape, *rest, *src_strides, *rest, *dst_strides, *rest))
             self._bases.append((src, int(src_off) * elem_size, dst, int(dst_off) * elem_size))
         self._template = b"".join(packed)
+        self._boxes = None
 
     def run(self, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
         if self.n == 0:
             return
-        boxes = self._type.from_buffer_copy(self._template)
-        for box, (src, src_off, dst, dst_off) in zip(boxes, self._bases):
-            box.src = bases[src] + src_off
-            box.dst = bases[dst] + dst_off
-        rc = _lib.load().ddl_copy_boxes(boxes, self.n, self.elem_size, op, dtype, _stream())
-        if rc:
-            _lib.check(rc, "ddl_copy_boxes")
+        boxes = self._boxes
+        if boxes is None:
+            boxes = self._boxes = _lib.front().Boxes(self._template, self._bases, self.elem_size)
+        boxes.run(bases, op, dtype)
 
 
 def copy_box(src, src_slices, dst, dst_slices, accumulate=False):
@@ -331,6 +331,10 @@ class HaloPadPlan:
         self.pad_arr = _lib.i64_array([v for p in self.pad for v in p])
         self.recv_arr = _lib.i64_array([v for p in self.recv for v in p])
         self.send_arr = _lib.i64_array([v for p in self.send for v in p])
+        # (place among the pointers, dimension, side, shape) of the slabs that exist
+        self._slabs = {kind: [(2 * d + s, d, s, self.slab_shape(d, s, kind)) for d in range(self.ndim) for s in range(2)
+                              if self.slab_shape(d, s, kind) is not None] for kind in ("ghost", "bulk")}
+        self._crops = {}        # element size -> launch of ``crop``
 
     def slab_shape(self, dim, side, kind):
         """Shape of the ghost (kind='ghost') or bulk slab of (dim, side); None if empty."""
@@ -359,24 +363,41 @@ class HaloPadPlan:
             out = torch.empty(self.padded_shape, dtype=x.dtype, device=x.device)
         elif tuple(out.shape) != self.padded_shape or not out.is_contiguous() or out.dtype != x.dtype:
             raise ValueError("halo_pad_exchange: bad output tensor")
-        gptr, bptr = [], []
-        for d in range(self.ndim):
-            for s in range(2):
-                for kind, bufs, ptrs in (("ghost", ghost_bufs, gptr), ("bulk", bulk_bufs, bptr)):
-                    buf = None if bufs is None else bufs[d][s]
-                    shape = self.slab_shape(d, s, kind)
-                    if buf is None or shape is None:
-                        ptrs.append(None)
-                        continue
-                    _require_gpu(buf)
-                    if tuple(buf.shape) != shape or not buf.is_contiguous() or buf.dtype != x.dtype:
-                        raise ValueError(f"halo_pad_exchange: {kind} slab ({d},{s}) must be contiguous {shape}, "
-                                         f"got {tuple(buf.shape)}")
-                    ptrs.append(buf.data_ptr())
+        gptr, bptr = [None] * (2 * self.ndim), [None] * (2 * self.ndim)
+        dtype = x.dtype
+        for kind, bufs, ptrs in (("ghost", ghost_bufs, gptr), ("bulk", bulk_bufs, bptr)):
+            if bufs is None:
+                continue
+            for place, d, s, shape in self._slabs[kind]:
+                buf = bufs[d][s]
+                if buf is None:
+                    continue
+                _require_gpu(buf)
+                if buf.shape != shape or not buf.is_contiguous() or buf.dtype != dtype:
+                    raise ValueError(f"halo_pad_exchange: {kind} slab ({d},{s}) must be contiguous {shape}, "
+                                     f"got {tuple(buf.shape)}")
+                ptrs[place] = buf.data_ptr()
         rc = _lib.load().ddl_halo_pad_exchange(x.data_ptr(), out.data_ptr(), self.shape_arr, self.ndim,
                                                x.element_size(), self.pad_arr, self.recv_arr, self.send_arr,
                                                _lib.ptr_array(gptr), _lib.ptr_array(bptr), int(kernel), _stream())
         _lib.check(rc, "ddl_halo_pad_exchange")
+        return out
+
+    def crop(self, padded):
+        """The part of a tensor of the padded shape that the shard fills, as a new tensor."""
+        out = torch.empty(self.x_shape, dtype=padded.dtype, device=padded.device)
+        if padded.shape == self.padded_shape and padded.is_contiguous():
+            _require_gpu(padded)
+            launch = self._crops.get(padded.element_size())
+            if launch is None:
+                strides = contiguous_strides(self.padded_shape)
+                launch = self._crops[padded.element_size()] = BoxLaunch(
+                    [(0, sum(p[0] * st for p, st in zip(self.pad, strides)), 1, 0, self.x_shape, strides, contiguous_strides(self.x_shape))],
+                    padded.element_size())
+            launch.run([padded.data_ptr(), out.data_ptr()])
+            return out
+        inner = [slice(p[0], p[0] + n) for p, n in zip(self.pad, self.x_shape)]
+        copy_box(padded, inner, out, [slice(0, n) for n in self.x_shape])
         return out
 
 
@@ -564,6 +585,9 @@ def ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma):
     """``ln_backward_partial`` plus, in the same pass, the partial column sums
     for the parameter gradients.  Returns (sums [rows, 2], workspace); hand the
     workspace to ``ln_backward_input_params``."""
+    res = _lib.front().ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma)
+    if res is not None:
+        return res
     _require_gpu(dy2d, x2d, mean, rstd, gamma)
     ld_dy, ld_x = _rows2d(dy2d, "ln_backward_partial_params"), _rows2d(x2d, "ln_backward_partial_params")
     rows, cols = x2d.shape
@@ -580,6 +604,12 @@ def ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma):
 def ln_backward_input_params(dy2d, x2d, mean, rstd, gamma, part_sums, weight, work, want_gamma=True, want_beta=True):
     """dx as ``ln_backward_input`` and, in the same launch, (dgamma, dbeta) from
     the workspace that ``ln_backward_partial_params`` filled."""
+    if x2d.dim() == 2:
+        cols = [x2d.shape[1]]
+        res = _lib.front().ln_backward_input_params(dy2d, x2d, mean, rstd, gamma, part_sums, weight, work, cols if want_gamma else None,
+                                                    cols if want_beta else None)
+        if res is not None:
+            return res
     _require_gpu(dy2d, x2d, mean, rstd, gamma, part_sums, work)
     ld_dy, ld_x = _rows2d(dy2d, "ln_backward_input_params"), _rows2d(x2d, "ln_backward_input_params")
     rows, cols = x2d.shape
@@ -670,6 +700,11 @@ def ln_backward_whole_rows(dy2d, x2d, mean, rstd, gamma, weight, want_gamma=True
 
 def embedding_gather(weight, ids, lo, hi, out=None):
     """out[t] = weight[ids[t] - lo] if lo <= ids[t] < hi else 0."""
+    if out is None:
+        out = _lib.front().embedding_gather(weight, ids, int(lo), int(hi))
+        if out is not None:
+            return out
+    weight = weight.detach()
     _require_gpu(weight, ids)
     if weight.dim() != 2 or (weight.shape[1] > 1 and weight.stride(1) != 1):
         raise ValueError("embedding_gather: weight must be 2-D with unit column stride")
@@ -727,6 +762,11 @@ def embedding_backward(grad_output, ids, lo, hi, padding_idx=None, scale_grad_by
     """Gradient of :func:`embedding_gather` with respect to the ``[hi-lo, dim]``
     table; with ``scale_grad_by_freq`` every row's sum is divided by the number
     of tokens that looked the row up."""
+    dw = _lib.front().embedding_backward(grad_output, ids, int(lo), int(hi), -1 if padding_idx is None else int(padding_idx),
+                                         bool(scale_grad_by_freq))
+    if dw is not None:
+        return dw
+    grad_output = grad_output.detach()
     _require_gpu(grad_output, ids)
     if grad_output.dtype not in _LN_DTYPES:
         raise ValueError("embedding_backward: bfloat16, float16 or float32 gradients only")
@@ -800,6 +840,11 @@ def linear(x, weight, bias=None, out=None):
     aligned operands; of operands that are not, small products are read as they
     are by a kernel of their own, and those of large ones are copied into
     zero-padded temporaries first (zeros add nothing to the sums)."""
+    if out is None:
+        y = _lib.front().linear(x, weight, bias)
+        if y is not None:
+            return y
+    x, weight, bias = x.detach(), weight.detach(), None if bias is None else bias.detach()
     _require_gpu(x, weight, bias)
     dt = _LINEAR_DTYPES.get(x.dtype)
     if dt is None or weight.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
@@ -907,6 +952,10 @@ def linear_backward(x, weight, grad_output, need_input=True, need_weight=True, n
     of 8 (small products: any); 16-bit operands that do not qualify are transposed
     into temporaries whose row pitch is padded to a multiple of 8 with zeros, and the forward
     kernel runs on those."""
+    grads = _lib.front().linear_backward(x, weight, grad_output, bool(need_input), bool(need_weight), bool(need_bias))
+    if grads is not None:
+        return grads
+    x, weight, grad_output = x.detach(), weight.detach(), grad_output.detach()
     _require_gpu(x, weight, grad_output)
     dt = _LINEAR_DTYPES.get(x.dtype)
     if dt is None or weight.dtype != x.dtype or grad_output.dtype != x.dtype:

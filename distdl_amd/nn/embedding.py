@@ -27,13 +27,13 @@ class _EmbeddingShard(torch.autograd.Function):
     def forward(ctx, weight, ids, lo, hi, padding_idx=None, scale_grad_by_freq=False):
         ctx.save_for_backward(ids)
         ctx.window = (lo, hi, padding_idx, scale_grad_by_freq)
-        return hip_ops.embedding_gather(weight.detach(), ids, lo, hi)
+        return hip_ops.embedding_gather(weight, ids, lo, hi)
 
     @staticmethod
     def backward(ctx, grad_output):
         (ids,) = ctx.saved_tensors
         lo, hi, padding_idx, scale_grad_by_freq = ctx.window
-        dw = hip_ops.embedding_backward(grad_output.detach(), ids, lo, hi, padding_idx, scale_grad_by_freq)
+        dw = hip_ops.embedding_backward(grad_output, ids, lo, hi, padding_idx, scale_grad_by_freq)
         return dw, None, None, None, None, None
 
 

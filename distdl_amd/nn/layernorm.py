@@ -38,6 +38,11 @@ def _shard_forward(input, weight, bias, P_reduce, part_cols, eps, part_cols_arr,
     None unless ``keep``.  ``stats_buffers``: the layer's cache of gathered
     statistics buffers ``[P, rows, 2]`` by row count (the stats kernel writes
     this worker's slot in place, the transport fills the others)."""
+    nparts = len(part_cols)
+    if keep and nparts == 1:
+        res = _lib.front().layer_norm(input, weight, bias, part_cols[0], eps)
+        if res is not None:
+            return res
     x = input.detach()
     cols = int(part_cols[P_reduce.rank if P_reduce.active else 0])
     x2d = x.reshape(-1, cols)
@@ -45,7 +50,6 @@ def _shard_forward(input, weight, bias, P_reduce, part_cols, eps, part_cols_arr,
         x2d = hip_ops.contiguous(x2d)
     gamma = None if weight is None else weight.detach().reshape(-1)
     beta = None if bias is None else bias.detach().reshape(-1)
-    nparts = len(part_cols)
     if nparts > 1:
         rows = x2d.shape[0]
         gathered = stats_buffers.get(rows)
@@ -88,14 +92,19 @@ class _LayerNormShard(torch.autograd.Function):
     def backward(ctx, grad_output):
         x2d, mean, rstd, gamma = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad[:3]
+        w_shape, b_shape = ctx.param_shapes
+        want_w, want_b = need_w and w_shape is not None, need_b and b_shape is not None
+        if need_x and ctx.nparts == 1:
+            grads = _lib.front().ln_backward_whole(grad_output, x2d, mean, rstd, gamma, w_shape if want_w else None,
+                                                   b_shape if want_b else None)
+            if grads is not None:
+                return grads + (None, None, None, None, None)
         dy2d = grad_output.detach().reshape(-1, ctx.cols)
         if dy2d.dtype != x2d.dtype:
             dy2d = dy2d.to(x2d.dtype)
         if dy2d.shape[1] > 1 and dy2d.stride(1) != 1:
             dy2d = hip_ops.contiguous(dy2d)
         dx = dw = db = None
-        w_shape, b_shape = ctx.param_shapes
-        want_w, want_b = need_w and w_shape is not None, need_b and b_shape is not None
         fused = need_x and (want_w or want_b)        # two launches instead of four
         if need_x and ctx.nparts == 1 and hip_ops.ln_backward_one_pass_supported(dy2d, x2d, gamma):
             # rows held whole: this worker's sums are the row's sums, so dx comes out of the pass that forms them

@@ -22,15 +22,15 @@ class _LinearShard(torch.autograd.Function):
     def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
-        return hip_ops.linear(x.detach(), weight.detach(), None if bias is None else bias.detach())
+        return hip_ops.linear(x, weight, bias)
 
     @staticmethod
     def backward(ctx, grad_output):
         x, weight = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad
-        dx, dw, db = hip_ops.linear_backward(x.detach(), weight.detach(), grad_output.detach().to(x.dtype),
-                                             need_x, need_w, need_b and ctx.has_bias)
-        return dx, dw, db
+        if grad_output.dtype != x.dtype:
+            grad_output = grad_output.detach().to(x.dtype)
+        return hip_ops.linear_backward(x, weight, grad_output, need_x, need_w, need_b and ctx.has_bias)
 
 
 def linear_shard(x, weight, bias):
