@@ -56,7 +56,7 @@ struct PartOf {
     const E* bias;
     E* y;
     int64_t M, N, K, ldx, ldw, ldy;
-    int tiles_m, tiles_n, vec_store;
+    int tiles_m, tiles_n;
 };
 
 // The two kinds of tiles of one product.

@@ -87,6 +87,16 @@ __device__ inline uint16_t f32_to_bf16(float f) {
     return static_cast<uint16_t>(u >> 16);
 }
 
+// 16 bytes at the alignment of an element, which global memory takes.
+template <typename T>
+__device__ inline uint4 load16(const T* p) {
+    struct __attribute__((packed, aligned(sizeof(T)))) Any {
+        uint32_t word[4];
+    };
+    const Any w = *reinterpret_cast<const Any*>(p);
+    return make_uint4(w.word[0], w.word[1], w.word[2], w.word[3]);
+}
+
 // Element types of the column sum: 0 = bf16, 1 = fp16, 2 = fp32.
 template <int DT>
 struct Elem;
@@ -96,7 +106,7 @@ struct Elem<0> {
     static __device__ float load(const uint16_t* p) { return bf16_to_f32(*p); }
     static __device__ void store(uint16_t* p, float f) { *p = f32_to_bf16(f); }
     static __device__ void load8(const uint16_t* p, float (&v)[8]) {
-        const uint4 q = *reinterpret_cast<const uint4*>(p);
+        const uint4 q = load16(p);
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -111,7 +121,7 @@ struct Elem<1> {
     static __device__ float load(const __half* p) { return __half2float(*p); }
     static __device__ void store(__half* p, float f) { *p = __float2half_rn(f); }
     static __device__ void load8(const __half* p, float (&v)[8]) {
-        const uint4 q = *reinterpret_cast<const uint4*>(p);
+        const uint4 q = load16(p);
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -127,8 +137,12 @@ struct Elem<2> {
     static __device__ float load(const float* p) { return *p; }
     static __device__ void store(float* p, float f) { *p = f; }
     static __device__ void load8(const float* p, float (&v)[8]) {
-        const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+        load4(p, *reinterpret_cast<float(*)[4]>(&v[0]));
+        load4(p + 4, *reinterpret_cast<float(*)[4]>(&v[4]));
+    }
+    static __device__ void load4(const float* p, float (&v)[4]) {
+        const uint4 q = load16(p);
+        v[0] = __uint_as_float(q.x), v[1] = __uint_as_float(q.y), v[2] = __uint_as_float(q.z), v[3] = __uint_as_float(q.w);
     }
 };
 
@@ -139,7 +153,7 @@ struct Elem<2> {
 template <int DT>
 __global__ __launch_bounds__(kBlock) void colsum_partial_kernel(const typename Elem<DT>::type* __restrict__ a, int64_t rows, int64_t cols,
                                                                 int64_t ld, int64_t rows_per_split, float* __restrict__ partial,
-                                                                int strips, int vec_ok) {
+                                                                int strips) {
     __shared__ float fold[32][kTile + 1];
     const int split = blockIdx.x / strips, strip = blockIdx.x - split * strips;
     const int t = threadIdx.x;
@@ -148,7 +162,7 @@ __global__ __launch_bounds__(kBlock) void colsum_partial_kernel(const typename E
     const int64_t r_begin = split * rows_per_split;
     const int64_t r_end = r_begin + rows_per_split < rows ? r_begin + rows_per_split : rows;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (vec_ok && gc + 8 <= cols) {
+    if (gc + 8 <= cols) {
         for (int64_t r = r_begin + g; r < r_end; r += 32) {
             float v[8];
             Elem<DT>::load8(a + r * ld + gc, v);
@@ -208,47 +222,52 @@ __global__ __launch_bounds__(kBlock) void colsum_final_kernel(const float* __res
 }
 
 // The column sum of few rows in one launch: a workgroup per 16 columns adds all
-// rows, 16 / E lanes per row (E elements of 16 bytes each, or one element per
-// lane where rows are not aligned), LDS folds the row groups.  The two stages
-// above are two launches and a workspace for what is a few microseconds of
-// reading: [777, 333] fp32 5.0 + 4.7 us, [1024, 4096] bf16 4.9 + 3.9 us.
-constexpr int kNarrow = 16, kOneBlock = 1024;
+// rows, 16 / E lanes per row (E elements of 16 bytes each, at any address), LDS
+// folds the row groups.  The two stages above are two launches and a workspace
+// for what is a few microseconds of reading: [777, 333] fp32 5.0 + 4.7 us, [1024,
+// 4096] bf16 4.9 + 3.9 us.  Neighbouring strips go to one XCD, so that a 128-byte line
+// they share comes from memory once and not for each of four L2 caches, and rows that
+// are not aligned are read 16 bytes a lane like others: [1024, 4096] bf16 5.7 ->
+// 3.8 us, [944, 16382] 22 -> 10.
+constexpr int kNarrow = 16, kOneBlock = 1024, kXcds = 8;
 
-template <int DT, bool VEC>
+template <int DT>
 __global__ __launch_bounds__(kOneBlock) void colsum_one_kernel(const typename Elem<DT>::type* __restrict__ a, int64_t rows, int64_t cols,
                                                                int64_t ld, typename Elem<DT>::type* __restrict__ out) {
     typedef typename Elem<DT>::type T;
-    constexpr int E = VEC ? 16 / static_cast<int>(sizeof(T)) : 1, kPieces = kNarrow / E, kGroups = kOneBlock / kPieces;
+    constexpr int E = 16 / static_cast<int>(sizeof(T)), kPieces = kNarrow / E, kGroups = kOneBlock / kPieces;
     __shared__ float fold[kGroups][kNarrow + 1];
     __shared__ float half[kOneBlock / kNarrow][kNarrow];
     const int t = threadIdx.x, g = t / kPieces, c = t % kPieces * E;
-    const int64_t gc = static_cast<int64_t>(blockIdx.x) * kNarrow + c;
+    const uint32_t per = gridDim.x / kXcds, whole = per * kXcds;   // hardware deals workgroups round-robin over the XCDs
+    const int64_t c0 = static_cast<int64_t>(blockIdx.x < whole ? blockIdx.x % kXcds * per + blockIdx.x / kXcds : blockIdx.x) * kNarrow;
+    const int64_t gc = c0 + c;
     float acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = 0.f;
-    if (VEC ? gc + E <= cols : gc < cols) {
+    // The last vector of a row ends with it: its first `back` columns are the vector's before it, added there.
+    const int back = gc + E > cols ? static_cast<int>(gc + E - cols) : 0;
+    if (back < E && gc >= back) {
+        const T* const first = a + (gc - back);
 #pragma unroll 4
         for (int64_t r = g; r < rows; r += kGroups) {
-            if constexpr (VEC && sizeof(T) == 2) {
-                float v[8];
-                Elem<DT>::load8(a + r * ld + gc, v);
+            float v[E];
+            if constexpr (sizeof(T) == 2) Elem<DT>::load8(first + r * ld, v);
+            else Elem<DT>::load4(first + r * ld, v);
 #pragma unroll
-                for (int e = 0; e < E; ++e) acc[e] += v[e];
-            } else if constexpr (VEC) {
-                const float4 v = *reinterpret_cast<const float4*>(a + r * ld + gc);
-                acc[0] += v.x, acc[1] += v.y, acc[2] += v.z, acc[3] += v.w;
-            } else {
-                acc[0] += Elem<DT>::load(a + r * ld + gc);
-            }
+            for (int e = 0; e < E; ++e) acc[e] += v[e];
         }
-    } else if (VEC) {   // the last columns, fewer than a vector
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (e >= back) fold[g][c + e - back] = acc[e];
+    } else if (back < E) {   // rows shorter than a vector
         for (int64_t r = g; r < rows; r += kGroups)
 #pragma unroll
             for (int e = 0; e < E; ++e)
                 if (gc + e < cols) acc[e] += Elem<DT>::load(a + r * ld + gc + e);
-    }
 #pragma unroll
-    for (int e = 0; e < E; ++e) fold[g][c + e] = acc[e];
+        for (int e = 0; e < E; ++e) fold[g][c + e] = acc[e];
+    }
     __syncthreads();
     constexpr int kParts = kOneBlock / kNarrow;   // threads per column
     const int col = t % kNarrow, part = t / kNarrow;
@@ -264,7 +283,7 @@ __global__ __launch_bounds__(kOneBlock) void colsum_one_kernel(const typename El
         for (int k = 0; k < d; ++k) mine[k] += mine[k + d];
     half[part][col] = mine[0];
     __syncthreads();
-    if (t < kNarrow && static_cast<int64_t>(blockIdx.x) * kNarrow + t < cols) {
+    if (t < kNarrow && c0 + t < cols) {
         float r[kParts];
 #pragma unroll
         for (int k = 0; k < kParts; ++k) r[k] = half[k][t];
@@ -272,7 +291,7 @@ __global__ __launch_bounds__(kOneBlock) void colsum_one_kernel(const typename El
         for (int d = kParts / 2; d > 0; d /= 2)
 #pragma unroll
             for (int k = 0; k < d; ++k) r[k] += r[k + d];
-        Elem<DT>::store(out + static_cast<int64_t>(blockIdx.x) * kNarrow + t, r[0]);
+        Elem<DT>::store(out + c0 + t, r[0]);
     }
 }
 
@@ -316,15 +335,11 @@ int run_colsum(const void* a, int64_t rows, int64_t cols, int64_t ld, void* out,
     typedef typename Elem<DT>::type T;
     if (colsum_in_one_launch(rows, cols, sizeof(T))) {
         const dim3 grid(static_cast<uint32_t>((cols + kNarrow - 1) / kNarrow));
-        if (aligned_to(a, 16) && (ld * sizeof(T)) % 16 == 0)
-            hipLaunchKernelGGL((colsum_one_kernel<DT, true>), grid, dim3(kOneBlock), 0, s, static_cast<const T*>(a), rows, cols, ld, static_cast<T*>(out));
-        else
-            hipLaunchKernelGGL((colsum_one_kernel<DT, false>), grid, dim3(kOneBlock), 0, s, static_cast<const T*>(a), rows, cols, ld, static_cast<T*>(out));
+        hipLaunchKernelGGL((colsum_one_kernel<DT>), grid, dim3(kOneBlock), 0, s, static_cast<const T*>(a), rows, cols, ld, static_cast<T*>(out));
         return check_launch("colsum_one_kernel");
     }
-    const int vec_ok = (aligned_to(a, 8 * sizeof(T)) && (ld * sizeof(T)) % 16 == 0) ? 1 : 0;
     hipLaunchKernelGGL((colsum_partial_kernel<DT>), dim3(static_cast<uint32_t>(strips * splits)), dim3(kBlock), 0, s,
-                       static_cast<const T*>(a), rows, cols, ld, rows_per_split, workspace, static_cast<int>(strips), vec_ok);
+                       static_cast<const T*>(a), rows, cols, ld, rows_per_split, workspace, static_cast<int>(strips));
     const int rc = check_launch("colsum_partial_kernel");
     if (rc) return rc;
     hipLaunchKernelGGL((colsum_final_kernel<DT>), dim3(static_cast<uint32_t>(strips)), dim3(kBlock), 0, s, workspace, cols,

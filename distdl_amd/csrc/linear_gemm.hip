@@ -92,7 +92,7 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     const uint16_t* __restrict__ bias = part.bias;
     uint16_t* __restrict__ y = part.y;
     const int64_t M = part.M, N = part.N, K = part.K, ldx = part.ldx, ldw = part.ldw, ldy = part.ldy;
-    const int tiles_m = part.tiles_m, tiles_n = part.tiles_n, vec_store = part.vec_store;
+    const int tiles_m = part.tiles_m, tiles_n = part.tiles_n;
 
     int tm, tn;
     tile_of_workgroup(tile_id, tiles_m, tiles_n, tm, tn);
@@ -353,97 +353,69 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     // Epilogue.  Lane holds, per 16x16 tile, output row m = l16 and the columns
     // n = 4 kg + {0,1,2,3} in acc[...][0..3].
-    if (vec_store == 2) {
-        // Through LDS, so that global stores are 16 bytes per lane and whole
-        // 128-byte (or longer) row segments per instruction.  Each wavefront
-        // transposes its own (16 TM) x (16 TN) block in a private LDS region:
-        // row pitch 32 TN bytes, the 16-byte chunk index XOR-ed with a function
-        // of the row so that neither the 8-byte writes (16 rows, four column
-        // groups) nor the 16-byte reads (whole rows) pile up on banks.
-        constexpr int kChunks = TN * 2;              // 16-byte chunks per row of the block
-        constexpr bool kPow2 = (kChunks & (kChunks - 1)) == 0;
-        // A power-of-two row is swizzled; any other row length is padded by one
-        // chunk instead, which staggers consecutive rows over the banks.
-        constexpr int kPitch = kPow2 ? TN * 32 : TN * 32 + 16;
-        auto swz = [](int row) { return !kPow2 ? 0 : kChunks == 8 ? ((row >> 1) & 7) : (row & (kChunks - 1)); };
-        __syncthreads();   // every wavefront is done with the operand stages (and every request has landed)
-        char* region = lds + wave * (TM * 16 * kPitch);
+    // Through LDS, so that global stores are 16 bytes per lane and whole
+    // 128-byte (or longer) row segments per instruction, whatever the pitch (rows
+    // that are no multiple of eight went out element by element: M 944, N 16382, K 72
+    // 36 us, here 18; M 214, N 15141, K 64 20 -> 9.6).  Each wavefront
+    // transposes its own (16 TM) x (16 TN) block in a private LDS region:
+    // row pitch 32 TN bytes, the 16-byte chunk index XOR-ed with a function
+    // of the row so that neither the 8-byte writes (16 rows, four column
+    // groups) nor the 16-byte reads (whole rows) pile up on banks.
+    constexpr int kChunks = TN * 2;              // 16-byte chunks per row of the block
+    constexpr bool kPow2 = (kChunks & (kChunks - 1)) == 0;
+    // A power-of-two row is swizzled; any other row length is padded by one
+    // chunk instead, which staggers consecutive rows over the banks.
+    constexpr int kPitch = kPow2 ? TN * 32 : TN * 32 + 16;
+    auto swz = [](int row) { return !kPow2 ? 0 : kChunks == 8 ? ((row >> 1) & 7) : (row & (kChunks - 1)); };
+    __syncthreads();   // every wavefront is done with the operand stages (and every request has landed)
+    char* region = lds + wave * (TM * 16 * kPitch);
 #pragma unroll
-        for (int a = 0; a < TN; ++a) {
-            const int64_t n = n0 + wn + a * 16 + 4 * kg;
-            float bv[4] = {0.f, 0.f, 0.f, 0.f};
-            if (bias) {
+    for (int a = 0; a < TN; ++a) {
+        const int64_t n = n0 + wn + a * 16 + 4 * kg;
+        float bv[4] = {0.f, 0.f, 0.f, 0.f};
+        if (bias) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (n + e < N) bv[e] = elem_to_f32<F16>(bias[n + e]);
-            }
-#pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                const int row = b * 16 + l16;
-                uint16_t o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = f32_to_elem<F16>(acc[a][b][e] + bv[e]);
-                uint2 pk;
-                pk.x = static_cast<uint32_t>(o[0]) | (static_cast<uint32_t>(o[1]) << 16);
-                pk.y = static_cast<uint32_t>(o[2]) | (static_cast<uint32_t>(o[3]) << 16);
-                // columns a 16 + 4 kg .. + 3 of the block: chunk 2 a + kg / 2, half kg % 2
-                *reinterpret_cast<uint2*>(region + row * kPitch + (((a * 2 + (kg >> 1)) ^ swz(row)) << 4) + (kg & 1) * 8) = pk;
-            }
+            for (int e = 0; e < 4; ++e)
+                if (n + e < N) bv[e] = elem_to_f32<F16>(bias[n + e]);
         }
-        // LDS operations of one wavefront complete in order, so its reads below
-        // see its writes above; no other wavefront touches this region.
-        asm volatile("" ::: "memory");
-        static_assert((TM * 16 * kChunks) % 64 == 0, "block does not split into whole wavefront passes");
+#pragma unroll
+        for (int b = 0; b < TM; ++b) {
+            const int row = b * 16 + l16;
+            uint16_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = f32_to_elem<F16>(acc[a][b][e] + bv[e]);
+            uint2 pk;
+            pk.x = static_cast<uint32_t>(o[0]) | (static_cast<uint32_t>(o[1]) << 16);
+            pk.y = static_cast<uint32_t>(o[2]) | (static_cast<uint32_t>(o[3]) << 16);
+            // columns a 16 + 4 kg .. + 3 of the block: chunk 2 a + kg / 2, half kg % 2
+            *reinterpret_cast<uint2*>(region + row * kPitch + (((a * 2 + (kg >> 1)) ^ swz(row)) << 4) + (kg & 1) * 8) = pk;
+        }
+    }
+    // LDS operations of one wavefront complete in order, so its reads below
+    // see its writes above; no other wavefront touches this region.
+    asm volatile("" ::: "memory");
+    static_assert((TM * 16 * kChunks) % 64 == 0, "block does not split into whole wavefront passes");
 #pragma unroll 4
-        for (int p = 0; p < TM * 16 * kChunks / 64; ++p) {
-            const int idx = p * 64 + lane;
-            const int row = idx / kChunks, chunk = idx % kChunks;
-            const int64_t m = m0 + wm + row;
-            const int64_t n = n0 + wn + chunk * 8;
-            const uint4 v = *reinterpret_cast<const uint4*>(region + row * kPitch + ((chunk ^ swz(row)) << 4));
-            if (m >= M || n >= N) continue;
-            uint16_t* dst = y + m * ldy + n;
-            if (n + 8 <= N) {
-                typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));   // y is not read again here: streaming store
-                u32x4 nv;
-                nv[0] = v.x, nv[1] = v.y, nv[2] = v.z, nv[3] = v.w;
-                __builtin_nontemporal_store(nv, reinterpret_cast<u32x4*>(dst));
-            } else {
-                const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+    for (int p = 0; p < TM * 16 * kChunks / 64; ++p) {
+        const int idx = p * 64 + lane;
+        const int row = idx / kChunks, chunk = idx % kChunks;
+        const int64_t m = m0 + wm + row;
+        const int64_t n = n0 + wn + chunk * 8;
+        const uint4 v = *reinterpret_cast<const uint4*>(region + row * kPitch + ((chunk ^ swz(row)) << 4));
+        if (m >= M || n >= N) continue;
+        uint16_t* dst = y + m * ldy + n;
+        if (n + 8 <= N) {
+            // y is not read again here: a streaming store, at the alignment of an element (global memory takes any)
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            typedef u32x4 any __attribute__((aligned(2)));
+            u32x4 nv;
+            nv[0] = v.x, nv[1] = v.y, nv[2] = v.z, nv[3] = v.w;
+            __builtin_nontemporal_store(nv, reinterpret_cast<any*>(dst));
+        } else {
+            const uint32_t words[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (n + e < N) dst[e] = static_cast<uint16_t>(words[e >> 1] >> (16 * (e & 1)));
-            }
-        }
-    } else {
-#pragma unroll
-        for (int a = 0; a < TN; ++a) {
-            const int64_t n = n0 + wn + a * 16 + 4 * kg;
-            float bv[4] = {0.f, 0.f, 0.f, 0.f};
-            if (bias) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (n + e < N) bv[e] = elem_to_f32<F16>(bias[n + e]);
-            }
-#pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                const int64_t m = m0 + wm + b * 16 + l16;
-                if (m >= M) continue;
-                uint16_t o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = f32_to_elem<F16>(acc[a][b][e] + bv[e]);
-                uint16_t* dst = y + m * ldy + n;
-                if (vec_store && n + 3 < N) {
-                    uint2 pk;
-                    pk.x = static_cast<uint32_t>(o[0]) | (static_cast<uint32_t>(o[1]) << 16);
-                    pk.y = static_cast<uint32_t>(o[2]) | (static_cast<uint32_t>(o[3]) << 16);
-                    *reinterpret_cast<uint2*>(dst) = pk;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n + e < N) dst[e] = o[e];
-                }
-            }
+            for (int e = 0; e < 8; ++e)
+                if (n + e < N) dst[e] = static_cast<uint16_t>(words[e >> 1] >> (16 * (e & 1)));
         }
     }
 }
@@ -577,15 +549,12 @@ int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* 
         if (any.kind != Small16::kNone) {
             Part16 p{};
             p.x = a.p, p.w = b.p, p.bias = bias, p.y = y, p.M = M, p.N = N, p.K = K, p.ldx = a.ld(), p.ldw = b.ld(), p.ldy = ldy;
-            p.vec_store = ldy % 4 == 0 && aligned_to(y, 8);
             return run_small16(who, any, f16, a.transposed(), b.transposed(), p, workspace, dev, static_cast<hipStream_t>(stream));
         }
     }
     if (int rc = check_operand(who, "a", a, M, K)) return rc;
     if (int rc = check_operand(who, "b", b, N, K)) return rc;
     if (!aligned_to(y, 2) || (bias && !aligned_to(bias, 2))) return fail(DDL_E_ALIGN, "%s: y / bias misaligned", who);
-    // 2: rows of y can be stored 16 bytes at a time, 1: 8 bytes, 0: element by element
-    const int vec_store = (ldy % 8 == 0 && aligned_to(y, 16)) ? 2 : (ldy % 4 == 0 && aligned_to(y, 8)) ? 1 : 0;
     const bool at = a.transposed(), bt = b.transposed();
 
     int dev = 0;
@@ -600,7 +569,7 @@ int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* 
         Part p{};
         p.x = a.p, p.w = b.p + n_begin * b.row_stride, p.bias = bias ? bias + n_begin : nullptr, p.y = y + n_begin;
         p.M = M, p.N = n_count, p.K = K, p.ldx = a.ld(), p.ldw = b.ld(), p.ldy = ldy;
-        p.tiles_m = static_cast<int>((M + bm - 1) / bm), p.tiles_n = static_cast<int>((n_count + bn - 1) / bn), p.vec_store = vec_store;
+        p.tiles_m = static_cast<int>((M + bm - 1) / bm), p.tiles_n = static_cast<int>((n_count + bn - 1) / bn);
         return p;
     };
     const int k = (f16 ? 4 : 0) + (at ? 2 : 0) + (bt ? 1 : 0);

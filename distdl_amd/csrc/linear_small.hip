@@ -47,16 +47,18 @@ __device__ inline floatx4 mfma(const bf16x8& a, const bf16x8& b, const floatx4& 
 
 // Four consecutive columns n .. n + 3 of output row m.
 template <bool F16>
-__device__ inline void store_four(uint16_t* __restrict__ y, int64_t ldy, int64_t m, int64_t n, int64_t N, const float* v, bool vec) {
+__device__ inline void store_four(uint16_t* __restrict__ y, int64_t ldy, int64_t m, int64_t n, int64_t N, const float* v) {
     uint16_t o[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = f32_to_elem<F16>(v[e]);
     uint16_t* dst = y + m * ldy + n;
-    if (vec && n + 3 < N) {
-        uint2 pk;
-        pk.x = static_cast<uint32_t>(o[0]) | (static_cast<uint32_t>(o[1]) << 16);
-        pk.y = static_cast<uint32_t>(o[2]) | (static_cast<uint32_t>(o[3]) << 16);
-        *reinterpret_cast<uint2*>(dst) = pk;
+    if (n + 3 < N) {   // global memory takes the eight bytes at any alignment
+        typedef uint32_t words __attribute__((ext_vector_type(2)));
+        typedef words any __attribute__((aligned(2)));
+        words pk;
+        pk[0] = static_cast<uint32_t>(o[0]) | (static_cast<uint32_t>(o[1]) << 16);
+        pk[1] = static_cast<uint32_t>(o[2]) | (static_cast<uint32_t>(o[3]) << 16);
+        *reinterpret_cast<any*>(dst) = pk;
     } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(KG * NWM * NWN * 64) void gemm16_small(const Part16
             const int64_t m = m0 + (sub_x + b) * 16 + l16;
             if (m >= M) continue;
             const float v[4] = {acc[a][b][0] + bv[0], acc[a][b][1] + bv[1], acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]};
-            store_four<F16>(p.y, p.ldy, m, n, N, v, p.vec_store != 0);
+            store_four<F16>(p.y, p.ldy, m, n, N, v);
         }
     }
 }
@@ -389,7 +391,7 @@ __global__ __launch_bounds__(256) void gemm16_small_sum(const Part16 p, int spli
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = s[e] + (p.bias && n + e < p.N ? elem_to_f32<F16>(p.bias[n + e]) : 0.f);
-    store_four<F16>(p.y, p.ldy, m, n, p.N, v, p.vec_store != 0);
+    store_four<F16>(p.y, p.ldy, m, n, p.N, v);
 }
 
 // ---- small tiles of operands at any address and pitch ------------------------
@@ -576,7 +578,7 @@ __global__ __launch_bounds__(512) void gemm16_any(const Part16 p, int splits, fl
             const int64_t m = m0 + (sub_x + b) * 16 + l16;
             if (m >= M) continue;
             const float v[4] = {acc[a][b][0] + bv[0], acc[a][b][1] + bv[1], acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]};
-            store_four<F16>(p.y, p.ldy, m, n, N, v, p.vec_store != 0);
+            store_four<F16>(p.y, p.ldy, m, n, N, v);
         }
     }
 }

@@ -1406,6 +1406,20 @@ def test_colsum_bf16(ops, rows, cols):
         assert torch.equal(ops.colsum_bf16(ai.cuda()).cpu().double(), want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols,pad", [(1, 1, 0), (3, 3, 2), (70, 5, 0), (513, 7, 0), (600, 8, 1), (64, 9, 0), (1000, 15, 0), (1025, 16, 3), (33, 17, 0),
+                                           (777, 333, 0), (4096, 143, 5), (4097, 143, 5), (2100, 70, 1), (129, 4103, 0)])
+def test_colsum_of_rows_at_any_address(ops, dtype, rows, cols, pad):
+    """Rows of odd length and pitch that start one element into their buffer and end where it ends, in one launch and in two;
+    columns whose last vector starts inside the one before it, rows shorter than a vector.  NaN lies between the rows.  Small
+    integers: the sums are exact."""
+    a = torch.randint(-2, 3, (rows, cols), generator=torch.Generator().manual_seed(rows + cols)).to(dtype)
+    store = torch.full((1 + rows * (cols + pad) - pad,), float("nan"), dtype=dtype, device="cuda")
+    ag = store[1:].as_strided((rows, cols), (cols + pad, 1), 1)
+    ag.copy_(a)
+    assert torch.equal(ops.colsum(ag).cpu(), a.double().sum(0).to(dtype))
+
+
 @pytest.mark.parametrize("M,N,K", [(8, 8, 8), (96, 80, 128), (300, 200, 72), (257, 36, 40), (5, 3, 16), (64, 1000, 256)])
 def test_linear_backward_small_integer_cases_are_exact(ops, M, N, K):
     """dx = dy w, dw = dy^T x, db = sum dy with small integers: every sum is
