@@ -4,13 +4,20 @@
 // HaloExchange (backends/mpi_numpy/functional/halo_exchange.py:50-74, 115-140).
 //
 // Host side: every box is rewritten in BYTES, unit dimensions are dropped,
-// dimensions that are contiguous on both sides are merged, and the widest
-// power-of-two vector (<= 16 B) that divides the innermost run, both base
-// addresses and every remaining stride is chosen.  A box is then a matrix of
+// dimensions that are contiguous on both sides are merged, and a power-of-two
+// vector (<= 16 B) is chosen.  Where an element may be written twice (copies and
+// clears) that is the widest that fits the innermost run, at any address: the last
+// vector of a run ends with it and moves some bytes of the one before once more.
+// Where it may not (accumulation, move and clear) it is the widest that divides the
+// run, both base addresses and every remaining stride.  A box is then a matrix of
 // R rows (the flattened outer dimensions) by C vectors (the innermost one).
+// (By vectors that divide the run, runs of odd length went 2 or 4 bytes a lane:
+// [44, 101, 101, 101] fp32 out of a frame of one took 139 us, now 71, at 5 TB/s; the
+// four launches of a repartition of [8, 4001, 6001] bf16 over four workers and its
+// adjoint 278, now 146; of [5, 1531, 3077] 43, now 31.)
 //
 // Device side: a workgroup moves tiles of 1024 vectors shaped TR rows x TC
-// columns, TC the power of two covering C (at most 1024), so a vector's row and
+// columns, TC a power of two (see columns_of_tile), so a vector's row and
 // column inside its tile are bit fields of its number; only the row needs
 // multiply-high divisions, and only when more than one outer dimension is left.
 // Workgroups are persistent (they stride over the tile sequence of the launch),
@@ -35,16 +42,19 @@ constexpr uint32_t kTileVecs = kThreads * kUnroll;
 constexpr uint32_t kTileLog = 10;  // log2(kTileVecs)
 static_assert((1u << kTileLog) == kTileVecs, "tile size must be 2^kTileLog");
 constexpr uint32_t kPersistentBlocks = 4096;  // 16 per CU
+constexpr uint32_t kXcds = 8;                 // workgroups are dealt to the XCDs in turn
 constexpr uint64_t kMaxVecs = (1ull << 31) - kTileVecs;
 constexpr uint64_t kLongRunBytes = 64 << 10;   // boxes whose innermost runs are at least this long are interleaved within a launch
 
 enum Op { OP_COPY = 0, OP_ADD = 1, OP_ZERO = 2, OP_MOVE = 3 };   // OP_MOVE: dst = src, src = 0
 
-// Multi-dword vectors are only promised dword alignment (see lower_box).
+// Vectors lie at any address (see lower_box); global memory takes them.
 typedef unsigned int u32x4_a __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2_a __attribute__((ext_vector_type(2)));
-typedef u32x4_a u32x4 __attribute__((aligned(4)));
-typedef u32x2_a u32x2 __attribute__((aligned(4)));
+typedef u32x4_a u32x4 __attribute__((aligned(1)));
+typedef u32x2_a u32x2 __attribute__((aligned(1)));
+typedef uint32_t u32x1 __attribute__((aligned(1)));
+typedef uint16_t u16x1 __attribute__((aligned(1)));
 
 struct DevDim {
     int64_t ss;  // source stride, bytes
@@ -64,7 +74,7 @@ struct DevBox {
     uint32_t vlog;        // log2(vector bytes)
     uint32_t first_tile;  // first tile of this box in the launch
     uint32_t ct_mul, ct_shr;  // multiply-high division by col_tiles
-    uint32_t pad;
+    uint32_t shift;       // bytes by which the last vector of a run starts earlier than its column says
     DevDim dim[kMaxDevDims];  // outer dimensions, 0 = slowest
 };
 
@@ -73,7 +83,8 @@ struct Batch {
     uint32_t first_tile[kBatch];  // copy of box[i].first_tile, contiguous for one wide scalar load
     uint32_t nbox;
     uint32_t ntiles;
-    FastDiv rr;   // div = nbox when the launch walks its boxes round-robin (tile b belongs to box b % nbox), else 0
+    FastDiv rr;   // div = nbox when the launch walks its boxes round-robin (tile b belongs to box b % nbox), else 0;
+                  // pad != 0: in groups of eight tiles of each box, and a box has pad tiles (see share_lines)
 };
 
 static_assert(sizeof(Batch) <= 4096, "box table must fit the kernel-argument segment");
@@ -207,6 +218,7 @@ __device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_
     const uint32_t ct_mul = bx->ct_mul, ct_shr = bx->ct_shr;
     const uint32_t rows = bx->rows, cols = bx->cols;
     const int64_t css = bx->css, cds = bx->cds;
+    const uint32_t shift = bx->shift;
     int64_t dss[ND > 0 ? ND : 1], dds[ND > 0 ? ND : 1];
     uint32_t ddiv[ND > 0 ? ND : 1], dmul[ND > 0 ? ND : 1], dshr[ND > 0 ? ND : 1];
 #pragma unroll
@@ -222,7 +234,8 @@ __device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_
     const uint32_t row0 = row_tile << (kTileLog - tc_log);
     const uint32_t col0 = col_tile << tc_log;
     const uint32_t tc = 1u << tc_log;
-    const bool interior = col0 + tc <= cols && row0 + (kTileVecs >> tc_log) <= rows;   // wave-uniform
+    // wave-uniform; not a tile with a vector that starts earlier
+    const bool interior = col0 + tc + (shift != 0 ? 1u : 0u) <= cols && row0 + (kTileVecs >> tc_log) <= rows;
     if (ND <= 1 && interior) {
         // Whole tile inside the box and rows addressed by one stride: the four
         // vectors of a lane differ by wave-uniform steps, so one position is
@@ -262,7 +275,8 @@ __device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_
             // every load and store unconditional.
             col = col < cols ? col : cols - 1;
             r = r < rows ? r : rows - 1;
-            int64_t so = static_cast<int64_t>(col) * css, dof = static_cast<int64_t>(col) * cds;
+            const int64_t earlier = col == cols - 1 ? shift : 0;
+            int64_t so = static_cast<int64_t>(col) * css - earlier, dof = static_cast<int64_t>(col) * cds - earlier;
 #pragma unroll
             for (int d = ND - 1; d > 0; --d) {
                 const uint32_t q = ddiv[d] == 1 ? r : (__umulhi(r, dmul[d]) >> dshr[d]);
@@ -352,9 +366,15 @@ __global__ __launch_bounds__(kThreads) void box_kernel(const Batch bt_by_value) 
     const uint32_t nbox = bt->nbox;
     const uint32_t ntiles = bt->ntiles;
     const uint32_t rr_div = bt->rr.div, rr_mul = bt->rr.mul, rr_shr = bt->rr.shr;
+    const uint32_t box_tiles = bt->rr.pad;
     for (uint32_t b = blockIdx.x; b < ntiles; b += gridDim.x) {
         uint32_t bi = 0, tile;
-        if (rr_div != 0) {   // boxes of equal tile counts, interleaved
+        if (box_tiles != 0) {   // the same tile of all boxes on one XCD
+            const uint32_t group = __umulhi(b / kXcds, rr_mul) >> rr_shr;
+            bi = b / kXcds - group * rr_div;
+            tile = group * kXcds + b % kXcds;
+            if (tile >= box_tiles) continue;
+        } else if (rr_div != 0) {   // boxes of equal tile counts, interleaved
             tile = __umulhi(b, rr_mul) >> rr_shr;
             bi = b - tile * rr_div;
         } else {
@@ -367,8 +387,8 @@ __global__ __launch_bounds__(kThreads) void box_kernel(const Batch bt_by_value) 
         switch (bx->vlog) {
             case 4: move_tile_nd<OP, T, u32x4>(bx, tile, nd); break;
             case 3: move_tile_nd<OP, T, u32x2>(bx, tile, nd); break;
-            case 2: move_tile_nd<OP, T, uint32_t>(bx, tile, nd); break;
-            case 1: move_tile_nd<OP, T, uint16_t>(bx, tile, nd); break;
+            case 2: move_tile_nd<OP, T, u32x1>(bx, tile, nd); break;
+            case 1: move_tile_nd<OP, T, u16x1>(bx, tile, nd); break;
             default: move_tile_nd<OP, T, uint8_t>(bx, tile, nd); break;
         }
     }
@@ -643,9 +663,9 @@ __global__ __launch_bounds__(kThreads) void sum_kernel(const SumArgs args_by_val
         else if (vlog == 3) {
             if constexpr (sizeof(T) <= 8) sum_tile_nd<T, u32x2, MODE>(sa, tile, nd);
         } else if (vlog == 2) {
-            if constexpr (sizeof(T) <= 4) sum_tile_nd<T, uint32_t, MODE>(sa, tile, nd);
+            if constexpr (sizeof(T) <= 4) sum_tile_nd<T, u32x1, MODE>(sa, tile, nd);
         } else {
-            if constexpr (sizeof(T) <= 2) sum_tile_nd<T, uint16_t, MODE>(sa, tile, nd);
+            if constexpr (sizeof(T) <= 2) sum_tile_nd<T, u16x1, MODE>(sa, tile, nd);
         }
     }
 }
@@ -754,9 +774,27 @@ struct HostDim {
     int64_t n, ss, ds;
 };
 
+// log2 of the columns of a tile of vectors of 2^vlog bytes: the power of two that covers the box, at most 1024; or a smaller
+// one of at least 512 bytes, the widest of which no more than an eighth lies past the box, or the one of which the least
+// does.  Lanes past the box repeat its last vector.  (Narrower tiles cover a box still better and make a wavefront's
+// addresses scatter: strips of 43 fp32 in tiles of 16 columns 12 us, in one of 64 8 to 10.)
+inline uint32_t columns_of_tile(uint32_t cols, uint32_t vlog) {
+    uint32_t log = 0;
+    while (log < kTileLog && (1u << log) < cols) ++log;
+    uint32_t best = log;
+    uint64_t least = ~0ull;
+    for (uint32_t l = log; l == log || l + vlog >= 9; --l) {
+        const uint64_t covered = ((static_cast<uint64_t>(cols) + (1u << l) - 1) >> l) << l;
+        if (covered < least) least = covered, best = l;
+        if (covered * 8 <= static_cast<uint64_t>(cols) * 9) return best;
+    }
+    return best;
+}
+
 // Rewrites one box in bytes, merges what can be merged and appends the
 // resulting device boxes (more than one only when a box must be split).
-int lower_box(const ddl_box_t& in, int elem_size, bool has_src, std::vector<DevBox>* out) {
+// `twice`: bytes may be written twice.
+int lower_box(const ddl_box_t& in, int elem_size, bool has_src, bool twice, std::vector<DevBox>* out) {
     if (in.ndim < 1 || in.ndim > DDL_MAX_DIMS) return fail(DDL_E_DIMS, "box ndim %d outside [1,%d]", in.ndim, DDL_MAX_DIMS);
     std::vector<HostDim> dims;
     for (int d = 0; d < in.ndim; ++d) {
@@ -784,26 +822,30 @@ int lower_box(const ddl_box_t& in, int elem_size, bool has_src, std::vector<DevB
         m.push_back(dims[d]);
     }
     std::reverse(m.begin(), m.end());  // m[0] outermost, m.back() = innermost byte run
-    // Vector width: the widest power of two (<= 16 B) dividing the innermost run.
-    // Base addresses and outer strides only have to be multiples of 4 bytes for
-    // the 8- and 16-byte vectors: gfx950 executes dword-aligned multi-dword
-    // global accesses at nearly the speed of aligned ones (measured: a copy
-    // whose destination is shifted by 4 bytes runs at 5.68 instead of 5.88 TB/s).
-    uint64_t align_bits = reinterpret_cast<uintptr_t>(in.dst);
-    if (has_src) align_bits |= reinterpret_cast<uintptr_t>(in.src);
-    for (size_t d = 0; d + 1 < m.size(); ++d) {
-        align_bits |= static_cast<uint64_t>(m[d].ds < 0 ? -m[d].ds : m[d].ds);
-        if (has_src) align_bits |= static_cast<uint64_t>(m[d].ss < 0 ? -m[d].ss : m[d].ss);
-    }
+    // Vector width (see the head of the file).
+    const uint64_t run = static_cast<uint64_t>(m.back().n);
     uint32_t vlog = 0;
-    while (vlog < 4 && ((static_cast<uint64_t>(m.back().n) >> vlog) & 1u) == 0) ++vlog;
-    if ((align_bits & 3u) != 0) {
-        uint32_t alog = 0;
-        while (alog < 2 && ((align_bits >> alog) & 1u) == 0) ++alog;
-        vlog = vlog < alog ? vlog : alog;
+    if (twice && run / 16 < kMaxVecs / 2) {
+        while (vlog < 4 && (2ull << vlog) <= run) ++vlog;
+    } else {
+        // Where the last vector ends with the run, base addresses and outer strides have to be multiples of 4 bytes for the 8-
+        // and 16-byte vectors, and of the vector for narrower ones.
+        uint64_t align_bits = reinterpret_cast<uintptr_t>(in.dst);
+        if (has_src) align_bits |= reinterpret_cast<uintptr_t>(in.src);
+        for (size_t d = 0; d + 1 < m.size(); ++d) {
+            align_bits |= static_cast<uint64_t>(m[d].ds < 0 ? -m[d].ds : m[d].ds);
+            if (has_src) align_bits |= static_cast<uint64_t>(m[d].ss < 0 ? -m[d].ss : m[d].ss);
+        }
+        while (vlog < 4 && ((run >> vlog) & 1u) == 0) ++vlog;
+        if ((align_bits & 3u) != 0) {
+            uint32_t alog = 0;
+            while (alog < 2 && ((align_bits >> alog) & 1u) == 0) ++alog;
+            vlog = vlog < alog ? vlog : alog;
+        }
     }
     const int64_t vbytes = 1ll << vlog;
-    m.back().n /= vbytes;
+    m.back().n = static_cast<int64_t>((run + vbytes - 1) >> vlog);
+    const uint32_t shift = static_cast<uint32_t>((m.back().n << vlog) - run);
     m.back().ss = has_src ? vbytes : 0;
     m.back().ds = vbytes;
     if (m.back().n == 1 && m.size() > 1) m.pop_back();  // element == vector: the next dimension becomes the columns
@@ -853,9 +895,9 @@ int lower_box(const ddl_box_t& in, int elem_size, bool has_src, std::vector<DevB
         db.css = inner.ss;
         db.cds = inner.ds;
         db.rows = static_cast<uint32_t>(total / static_cast<uint64_t>(inner.n));
-        uint32_t tc_log = 0;
-        while (tc_log < kTileLog && (1u << tc_log) < db.cols) ++tc_log;
+        const uint32_t tc_log = columns_of_tile(db.cols, vlog);
         db.tc_log = tc_log;
+        db.shift = shift;
         db.col_tiles = (db.cols + (1u << tc_log) - 1) >> tc_log;
         const FastDiv ct = make_fastdiv(db.col_tiles);
         db.ct_mul = ct.mul;
@@ -889,12 +931,12 @@ constexpr uint64_t kUniformMaxTiles = 16384;   // 256 MiB a launch: beyond that 
 inline bool uniform_batch(const Batch& bt, uint32_t n, uint64_t tiles) {
     const DevBox& a = bt.box[0];
     if (n < 1 || tiles > kUniformMaxTiles || tiles % n != 0 || tiles / n > 65535) return false;
-    if (a.vlog != 4 || a.nd > 1 || a.css != 16 || a.cds != 16) return false;
+    if (a.vlog != 4 || a.nd > 1 || a.css != 16 || a.cds != 16 || a.shift != 0) return false;
     const uint32_t tc = 1u << a.tc_log, tr = kTileVecs >> a.tc_log;
     if (a.cols % tc != 0 || a.rows % tr != 0) return false;
     for (uint32_t k = 1; k < n; ++k) {
         const DevBox& b = bt.box[k];
-        if (b.vlog != a.vlog || b.nd != a.nd || b.css != a.css || b.cds != a.cds || b.cols != a.cols || b.rows != a.rows) return false;
+        if (b.vlog != a.vlog || b.nd != a.nd || b.css != a.css || b.cds != a.cds || b.cols != a.cols || b.rows != a.rows || b.shift != 0) return false;
         if (a.nd == 1 && (b.dim[0].ss != a.dim[0].ss || b.dim[0].ds != a.dim[0].ds)) return false;
     }
     return true;
@@ -921,6 +963,38 @@ inline int launch_uniform(const Batch& bt, uint32_t n, uint32_t tiles_per_box, b
     else
         hipLaunchKernelGGL((uniform_copy_kernel<false, false>), grid, dim3(kThreads), 0, stream, ub);
     return check_launch("uniform_copy_kernel");
+}
+
+// Boxes of equal shape whose runs are shorter than a memory line and lie in the same rows of a tensor -- the left and right
+// strips of a halo along the last dimension: the right strip of a row and the left one of the next are mostly on one line.
+// The tiles are then dealt so that workgroups kXcds apart, which run on one XCD, move the same tile of the boxes, and the
+// line is in their L2 when the second needs it.  (Strips of one fp32 column of [8, 41, 43, 43, 43] in a frame of one: pack
+// 32 -> 23 us, move 54 -> 49, add 46 -> 36; unpack 55 either way, bound by lines written in part.)
+inline bool share_lines(const Batch& bt, uint32_t n, bool equal) {
+    const DevBox& a = bt.box[0];
+    if (!equal || n < 2) return false;
+    auto span = [](int64_t v) { return v < 0 ? -v : v; };
+    bool src = true, dst = true;
+    for (uint32_t k = 0; k < n; ++k) {
+        const DevBox& b = bt.box[k];
+        if (b.nd != a.nd || b.cols != a.cols || b.rows != a.rows || b.vlog != a.vlog || b.css != a.css || b.cds != a.cds) return false;
+        for (int d = 0; d < kMaxDevDims; ++d) {
+            src = src && b.dim[d].ss == a.dim[d].ss;
+            dst = dst && b.dim[d].ds == a.dim[d].ds;
+        }
+    }
+    // A run that fits its vector leaves the rows as columns.
+    const bool columns = span(a.css) > (1 << a.vlog) || span(a.cds) > (1 << a.vlog);
+    const int64_t run = columns ? 1ll << a.vlog : static_cast<int64_t>(a.cols) << a.vlog;
+    if (!columns && a.nd == 0) return false;
+    const int last = a.nd > 2 ? kMaxDevDims - 1 : static_cast<int>(a.nd) - 1;
+    const int64_t srow = span(columns ? a.css : a.dim[last].ss), drow = span(columns ? a.cds : a.dim[last].ds);
+    if (run >= 128) return false;
+    for (uint32_t k = 1; k < n; ++k) {
+        src = src && srow > run && span(bt.box[k].src - a.src) < srow;
+        dst = dst && drow > run && span(bt.box[k].dst - a.dst) < drow;
+    }
+    return src || dst;
 }
 
 template <int OP, typename T>
@@ -973,7 +1047,15 @@ int launch_batches(const std::vector<DevBox>& boxes, hipStream_t stream) {
             if (int rc = launch_uniform(bt, n, static_cast<uint32_t>(tiles / n), interleave, stream)) return rc;
             continue;
         }
-        const uint32_t blocks = tiles < kPersistentBlocks ? static_cast<uint32_t>(tiles) : kPersistentBlocks;
+        uint32_t most = kPersistentBlocks;
+        if (tiles < 0x40000000ull && share_lines(bt, n, equal)) {
+            bt.rr = make_fastdiv(n);
+            bt.rr.pad = static_cast<uint32_t>(tiles / n);
+            tiles = (tiles / n + kXcds - 1) / kXcds * kXcds * n;
+            bt.ntiles = static_cast<uint32_t>(tiles);
+            most = kPersistentBlocks / (kXcds * n) * (kXcds * n);
+        }
+        const uint32_t blocks = tiles < most ? static_cast<uint32_t>(tiles) : most;
         hipLaunchKernelGGL((box_kernel<OP, T>), dim3(blocks), dim3(kThreads), 0, stream, bt);
         if (int rc = check_launch("box_kernel")) return rc;
     }
@@ -993,7 +1075,7 @@ int run_boxes(const ddl_box_t* boxes, int nbox, int elem_size, int op, int dtype
     std::vector<DevBox> dev;
     dev.reserve(nbox);
     for (int b = 0; b < nbox; ++b)
-        if (int rc = lower_box(boxes[b], elem_size, has_src, &dev)) return rc;
+        if (int rc = lower_box(boxes[b], elem_size, has_src, op == DDL_OP_COPY || op == OP_ZERO, &dev)) return rc;
     if (dev.empty()) return 0;
     if (op == OP_ZERO) return launch_batches<OP_ZERO, uint8_t>(dev, stream);
     if (op == OP_MOVE) return launch_batches<OP_MOVE, uint8_t>(dev, stream);
@@ -1084,7 +1166,7 @@ int launch_sum(const std::vector<DevBox>& pieces, const void* const* srcs, int n
         const uint64_t tiles = static_cast<uint64_t>(db.col_tiles) * ((db.rows + tr - 1) / tr);
         sa.ntiles = static_cast<uint32_t>(tiles);
         const bool whole_tiles = db.cols % (1u << db.tc_log) == 0 && db.rows % tr == 0;
-        if (nsrc >= kSumPiecesSources && db.vlog == 4 && db.nd <= 1 && db.css == 16 && db.cds == 16 && whole_tiles &&
+        if (nsrc >= kSumPiecesSources && db.vlog == 4 && db.nd <= 1 && db.css == 16 && db.cds == 16 && db.shift == 0 && whole_tiles &&
             tiles * kUnroll <= 0x7FFFFFFFull) {
             const uint32_t items = static_cast<uint32_t>(tiles * kUnroll);
             SumSources ss{};
@@ -1138,8 +1220,11 @@ int ddl_sum_boxes(const ddl_box_t* box, const void* const* srcs, int nsrc, int e
     }
     ddl_box_t in = *box;
     in.src = srcs[0];
+    // An element may be written twice unless a source lies where the result goes.
+    bool in_place = false;
+    for (int q = 0; q < nsrc; ++q) in_place = in_place || srcs[q] == box->dst;
     std::vector<DevBox> pieces;
-    if (int rc = lower_box(in, elem_size, true, &pieces)) return rc;
+    if (int rc = lower_box(in, elem_size, true, !in_place, &pieces)) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (dtype) {
         case DDL_DT_F32: return launch_sum<float>(pieces, srcs, nsrc, divisor, s);

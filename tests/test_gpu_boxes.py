@@ -153,6 +153,65 @@ def test_equal_boxes_pack_and_unpack_bit_exact(ops, dtype, rows, strip, nbox, ax
     assert torch.equal(bits(y.cpu()), want)
 
 
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32, torch.float64])
+@pytest.mark.parametrize("run", [1, 3, 5, 7, 15, 17, 31, 33, 751, 1025, 8200])
+@pytest.mark.parametrize("pitch", [0, 1, 6])
+def test_boxes_of_odd_runs_at_any_address(ops, dtype, run, pitch):
+    """Copies and clears whose runs are no whole number of vectors, at addresses and pitches that are multiples of the
+    element alone: the last vector of a run starts earlier and moves some bytes twice.  Bit for bit, and nothing outside
+    the boxes.  Two neighbouring boxes a launch: short runs of one row are moved tile by tile in turn (also accumulated
+    and moved out)."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(run * 8 + pitch)
+    rows = 3 if run > 1000 else 67
+    left = run + 1
+    width = left + run + pitch
+    x_cpu = random_bits((2, rows, width), dtype, gen)
+    x = x_cpu.cuda()
+    boxes = [(slice(0, 2), slice(0, rows), slice(0, run)), (slice(0, 2), slice(0, rows), slice(left, left + run))]
+    plan = ops.BoxPlan.from_slices(x, boxes)
+    pools = [torch.zeros(2 * rows * run + 5, dtype=dtype, device="cuda") for _ in boxes]
+    bufs = [pool[1:1 + 2 * rows * run].view(2, rows, run) for pool in pools]     # one element past an aligned address
+    plan.pack(x, bufs)
+    for sl, buf, pool in zip(boxes, bufs, pools):
+        assert torch.equal(bits(buf.cpu()), bits(x_cpu[sl]))
+        assert not bits(pool.cpu())[0] and not bits(pool.cpu())[-4:].any()
+    y_cpu = random_bits((2, rows, width), dtype, gen)
+    y = y_cpu.cuda()
+    plan.unpack(y, bufs)
+    want = bits(y_cpu).clone()
+    for sl in boxes:
+        want[sl] = bits(x_cpu)[sl]
+    assert torch.equal(bits(y.cpu()), want)
+    plan.zero(y)
+    for sl in boxes:
+        want[sl] = 0
+    assert torch.equal(bits(y.cpu()), want)
+    strides, dense = ops.contiguous_strides(x.shape), ops.contiguous_strides((2, rows, run))
+    entries = [(0, sl[2].start, 1 + k, 0, [2, rows, run], strides, dense) for k, sl in enumerate(boxes)]
+    ops.BoxLaunch(entries, x.element_size()).run([x.data_ptr()] + [b.data_ptr() for b in bufs], op=_lib.DDL_OP_MOVE)
+    want = bits(x_cpu).clone()
+    for sl, buf in zip(boxes, bufs):
+        assert torch.equal(bits(buf.cpu()), bits(x_cpu)[sl])
+        want[sl] = 0
+    assert torch.equal(bits(x.cpu()), want)
+    if dtype.is_floating_point:
+        z_cpu = torch.randn(2, rows, width, generator=gen).to(dtype)
+        add = [torch.randn(2, rows, run, generator=gen).to(dtype) for _ in boxes]
+        z = z_cpu.cuda()
+        plan.unpack(z, [a.cuda() for a in add], accumulate=True)
+        for sl, a in zip(boxes, add):
+            z_cpu[sl] += a
+        assert torch.equal(bits(z.cpu()), bits(z_cpu))
+        total = torch.zeros(2 * rows * run + 5, dtype=dtype, device="cuda")
+        into, full = total[3:3 + 2 * rows * run].view(2, rows, run), tuple(slice(0, n) for n in (2, rows, run))
+        ops.sum_boxes([z, z], boxes[1], into, full)
+        assert torch.equal(bits(into.cpu()), bits(z_cpu[boxes[1]] + z_cpu[boxes[1]]))
+        assert not bits(total.cpu())[:3].any() and not bits(total.cpu())[-2:].any()
+        ops.sum_boxes([into, into], full, into, full)                           # in place: no element is read after it is written
+        assert torch.equal(bits(into.cpu()), bits((z_cpu[boxes[1]] * 2) * 2))
+
+
 def test_pack_from_non_contiguous_tensor(ops):
     gen = torch.Generator().manual_seed(11)
     base = random_bits((9, 12, 10), torch.float32, gen).cuda()
