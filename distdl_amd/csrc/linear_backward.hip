@@ -18,74 +18,7 @@ namespace {
 
 constexpr int kTile = 64;      // elements per tile edge
 constexpr int kBlock = 256;
-
-// dst[c, r] = src[r, c] for 16-bit elements.  A 64 x 64 tile goes through LDS:
-// rows are read 16 bytes per lane, the transposed rows are put together from
-// 2-byte LDS reads and written 16 bytes per lane.  The LDS row pitch of 66
-// elements (33 dwords) spreads a column over all banks.
-__global__ __launch_bounds__(kBlock) void transpose16_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
-                                                             int64_t rows, int64_t cols, int64_t ld_src, int64_t ld_dst,
-                                                             int tiles_c, int vec_ok) {
-    __shared__ uint16_t tile[kTile][kTile + 2];
-    const int tr = blockIdx.x / tiles_c, tc = blockIdx.x - tr * tiles_c;
-    const int64_t r0 = static_cast<int64_t>(tr) * kTile, c0 = static_cast<int64_t>(tc) * kTile;
-    const int t = threadIdx.x;
-    // load: 8 lanes per row (8 x 8 elements), 32 rows per pass
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const int r = (t >> 3) + 32 * p, c = (t & 7) * 8;
-        const int64_t gr = r0 + r, gc = c0 + c;
-        uint16_t v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (gr < rows) {
-            const uint16_t* s = src + gr * ld_src + gc;
-            if (vec_ok && gc + 8 <= cols) {
-                const uint4 q = *reinterpret_cast<const uint4*>(s);
-                v[0] = q.x & 0xFFFF; v[1] = q.x >> 16; v[2] = q.y & 0xFFFF; v[3] = q.y >> 16;
-                v[4] = q.z & 0xFFFF; v[5] = q.z >> 16; v[6] = q.w & 0xFFFF; v[7] = q.w >> 16;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (gc + e < cols) v[e] = s[e];
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; e += 2)
-            *reinterpret_cast<uint32_t*>(&tile[r][c + e]) = static_cast<uint32_t>(v[e]) | (static_cast<uint32_t>(v[e + 1]) << 16);
-    }
-    __syncthreads();
-    // store: output row = source column; 8 lanes per output row, 8 source rows each
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const int oc = (t >> 3) + 32 * p, orr = (t & 7) * 8;   // source column, first source row
-        const int64_t gc = c0 + oc, gr = r0 + orr;
-        if (gc >= cols || gr >= rows) continue;
-        uint16_t v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = tile[orr + e][oc];
-        uint16_t* d = dst + gc * ld_dst + gr;
-        if (vec_ok && gr + 8 <= rows) {
-            uint4 q;
-            q.x = v[0] | (static_cast<uint32_t>(v[1]) << 16);
-            q.y = v[2] | (static_cast<uint32_t>(v[3]) << 16);
-            q.z = v[4] | (static_cast<uint32_t>(v[5]) << 16);
-            q.w = v[6] | (static_cast<uint32_t>(v[7]) << 16);
-            *reinterpret_cast<uint4*>(d) = q;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (gr + e < rows) d[e] = v[e];
-        }
-    }
-}
-
-__device__ inline float bf16_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
-
-__device__ inline uint16_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if (f != f) return 0x7FC0;
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
-}
+constexpr uint32_t kXcds = 8;    // workgroups are dealt to the XCDs in turn
 
 // 16 bytes at the alignment of an element, which global memory takes.
 template <typename T>
@@ -95,6 +28,104 @@ __device__ inline uint4 load16(const T* p) {
     };
     const Any w = *reinterpret_cast<const Any*>(p);
     return make_uint4(w.word[0], w.word[1], w.word[2], w.word[3]);
+}
+
+__device__ inline void store16(uint16_t* p, uint4 q) {
+    struct __attribute__((packed, aligned(2))) Any {
+        uint32_t word[4];
+    };
+    *reinterpret_cast<Any*>(p) = Any{{q.x, q.y, q.z, q.w}};
+}
+
+// Elements [first, first + 8) of a row of `n`, zeros past its end.
+__device__ inline uint4 load_piece(const uint16_t* row, int64_t first, int64_t n) {
+    if (first + 8 <= n) return load16(row + first);
+    uint32_t q[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        if (first + e < n) q[e >> 1] |= static_cast<uint32_t>(row[first + e]) << (16 * (e & 1));
+    return make_uint4(q[0], q[1], q[2], q[3]);
+}
+
+// dst[c, r] = src[r, c] for 16-bit elements, and zeros in the columns rows .. width of dst.  A 64 x 64 tile goes through
+// LDS: rows are read 16 bytes per lane at whatever address they have; a lane reads 8 rows of two source columns back, 4
+// bytes each, sorts them apart and writes 16 bytes to each of two rows of dst.  The LDS row pitch of 66 elements (33
+// dwords) puts the 64 lanes of a wavefront on 64 banks.  The tiles of an XCD are neighbours, so that the lines which two
+// tiles of a row share come from its L2.  Bound by memory: dy [5066, 3572] bf16, whose rows are not 16 bytes apart, into
+// a zeroed [3572, 5072] took 52 us by 2-byte accesses, after a clear of 7; now 13.4 for both, at 5.4 TB/s.
+__global__ __launch_bounds__(kBlock) void transpose16_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
+                                                             int64_t rows, int64_t cols, int64_t ld_src, int64_t ld_dst,
+                                                             int64_t width, uint32_t tiles_c, uint32_t tiles, uint32_t per_xcd) {
+    __shared__ uint32_t tile[kTile][kTile / 2 + 1];
+    const uint32_t b = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (b >= tiles) return;
+    const uint32_t tr = b / tiles_c, tc = b - tr * tiles_c;
+    const int64_t r0 = static_cast<int64_t>(tr) * kTile, c0 = static_cast<int64_t>(tc) * kTile;
+    const int t = threadIdx.x;
+    // 8 lanes per row (8 x 8 elements), 32 rows per pass
+    uint4 q[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int64_t gr = r0 + (t >> 3) + 32 * p, gc = c0 + (t & 7) * 8;
+        q[p] = gr < rows ? load_piece(src + gr * ld_src, gc, cols) : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        uint32_t* to = &tile[(t >> 3) + 32 * p][(t & 7) * 4];
+        to[0] = q[p].x, to[1] = q[p].y, to[2] = q[p].z, to[3] = q[p].w;
+    }
+    __syncthreads();
+    // 8 lanes per pair of output rows, 8 source rows each
+    const int pair = t >> 3, first = (t & 7) * 8;
+    uint32_t even[4], odd[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t lo = tile[first + 2 * e][pair], hi = tile[first + 2 * e + 1][pair];
+        even[e] = (lo & 0xFFFFu) | (hi << 16);
+        odd[e] = (lo >> 16) | (hi & 0xFFFF0000u);
+    }
+    const int64_t gc = c0 + 2 * pair, gr = r0 + first;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (gc + h >= cols) break;
+        const uint32_t* v = h ? odd : even;
+        uint16_t* d = dst + (gc + h) * ld_dst + gr;
+        if (gr + 8 <= width) {
+            store16(d, make_uint4(v[0], v[1], v[2], v[3]));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (gr + e < width) d[e] = static_cast<uint16_t>(v[e >> 1] >> (16 * (e & 1)));
+        }
+    }
+}
+
+// dst[r, c] = src[r, c], and zeros in the columns cols .. 8 * pieces of dst, whose rows lie end to end: 16 bytes a lane.
+// [5066, 3572] bf16 in 16.7 us; a clear and a box copy took 25.
+constexpr int kPadPieces = 4;   // per lane
+
+__global__ __launch_bounds__(kBlock) void pad16_kernel(const uint16_t* __restrict__ src, uint4* __restrict__ dst, uint32_t total,
+                                                       uint32_t pieces, int64_t cols, int64_t ld_src) {
+    const uint32_t first = blockIdx.x * (kBlock * kPadPieces) + threadIdx.x;
+    uint4 q[kPadPieces];
+#pragma unroll
+    for (int p = 0; p < kPadPieces; ++p) {
+        const uint32_t i = first + p * kBlock < total ? first + p * kBlock : total - 1;
+        const uint32_t r = i / pieces;
+        q[p] = load_piece(src + static_cast<int64_t>(r) * ld_src, static_cast<int64_t>(i - r * pieces) * 8, cols);
+    }
+#pragma unroll
+    for (int p = 0; p < kPadPieces; ++p)
+        if (first + p * kBlock < total) dst[first + p * kBlock] = q[p];
+}
+
+__device__ inline float bf16_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
+
+__device__ inline uint16_t f32_to_bf16(float f) {
+    uint32_t u = __float_as_uint(f);
+    if (f != f) return 0x7FC0;
+    u += 0x7FFFu + ((u >> 16) & 1u);
+    return static_cast<uint16_t>(u >> 16);
 }
 
 // Element types of the column sum: 0 = bf16, 1 = fp16, 2 = fp32.
@@ -229,7 +260,7 @@ __global__ __launch_bounds__(kBlock) void colsum_final_kernel(const float* __res
 // they share comes from memory once and not for each of four L2 caches, and rows that
 // are not aligned are read 16 bytes a lane like others: [1024, 4096] bf16 5.7 ->
 // 3.8 us, [944, 16382] 22 -> 10.
-constexpr int kNarrow = 16, kOneBlock = 1024, kXcds = 8;
+constexpr int kNarrow = 16, kOneBlock = 1024;
 
 template <int DT>
 __global__ __launch_bounds__(kOneBlock) void colsum_one_kernel(const typename Elem<DT>::type* __restrict__ a, int64_t rows, int64_t cols,
@@ -300,21 +331,49 @@ __global__ __launch_bounds__(kOneBlock) void colsum_one_kernel(const typename El
 
 extern "C" int ddl_transpose_2d(const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld_src, int64_t ld_dst,
                                 int elem_size, void* stream) {
+    return ddl_transpose_padded(src, dst, rows, cols, ld_src, ld_dst, rows, elem_size, stream);
+}
+
+extern "C" int ddl_transpose_padded(const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld_src, int64_t ld_dst,
+                                    int64_t width, int elem_size, void* stream) {
     using namespace ddl;
-    if (rows < 0 || cols < 0 || ld_src < cols || ld_dst < rows)
+    if (rows < 0 || cols < 0 || ld_src < cols || width < rows || ld_dst < width)
         return fail(DDL_E_ARG, "transpose: rows=%lld cols=%lld ld_src=%lld ld_dst=%lld", (long long)rows, (long long)cols,
                     (long long)ld_src, (long long)ld_dst);
     if (elem_size != 2) return fail(DDL_E_UNSUPP, "transpose: element size %d (only 2-byte elements)", elem_size);
-    if (rows == 0 || cols == 0) return 0;
-    if (!src || !dst) return fail(DDL_E_ARG, "transpose: null pointer");
+    if (width == 0 || cols == 0) return 0;
+    if ((!src && rows > 0) || !dst) return fail(DDL_E_ARG, "transpose: null pointer");
     if (!aligned_to(src, 2) || !aligned_to(dst, 2)) return fail(DDL_E_ALIGN, "transpose: pointer misaligned");
-    const int64_t tiles_r = (rows + kTile - 1) / kTile, tiles_c = (cols + kTile - 1) / kTile;
-    if (tiles_r * tiles_c > 0x7FFFFFFFll || tiles_c > 0x7FFFFFFFll) return fail(DDL_E_UNSUPP, "transpose: too many tiles");
-    const int vec_ok = aligned_to(src, 16) && aligned_to(dst, 16) && ld_src % 8 == 0 && ld_dst % 8 == 0;
-    hipLaunchKernelGGL(transpose16_kernel, dim3(static_cast<uint32_t>(tiles_r * tiles_c)), dim3(kBlock), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), rows,
-                       cols, ld_src, ld_dst, static_cast<int>(tiles_c), vec_ok);
+    const int64_t tiles_r = (width + kTile - 1) / kTile, tiles_c = (cols + kTile - 1) / kTile;
+    if (tiles_c > 0x7FFFFF00ll || tiles_r > 0x7FFFFF00ll / tiles_c) return fail(DDL_E_UNSUPP, "transpose: too many tiles");
+    const uint32_t tiles = static_cast<uint32_t>(tiles_r * tiles_c), per_xcd = (tiles + kXcds - 1) / kXcds;
+    hipLaunchKernelGGL(transpose16_kernel, dim3(per_xcd * kXcds), dim3(kBlock), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), rows, cols, ld_src, ld_dst, width,
+                       static_cast<uint32_t>(tiles_c), tiles, per_xcd);
     return check_launch("transpose16_kernel");
+}
+
+extern "C" int ddl_pad_rows(const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld_src, int64_t width, int elem_size,
+                            void* stream) {
+    using namespace ddl;
+    if (rows < 0 || cols < 0 || ld_src < 0 || width < cols || width % 8 != 0)
+        return fail(DDL_E_ARG, "pad: rows=%lld cols=%lld ld_src=%lld width=%lld", (long long)rows, (long long)cols, (long long)ld_src,
+                    (long long)width);
+    if (elem_size != 2) return fail(DDL_E_UNSUPP, "pad: element size %d (only 2-byte elements)", elem_size);
+    if (rows == 0 || width == 0) return 0;
+    if ((!src && cols > 0) || !dst) return fail(DDL_E_ARG, "pad: null pointer");
+    if (!aligned_to(src, 2) || !aligned_to(dst, 16)) return fail(DDL_E_ALIGN, "pad: pointer misaligned");
+    // Lanes number the pieces in 32 bits: slabs of rows that they reach, and no row is longer than that.
+    const int64_t pieces = width / 8, most = 0x7FFF0000ll / pieces;
+    if (most < 1) return fail(DDL_E_UNSUPP, "pad: rows of %lld elements", (long long)width);
+    for (int64_t r = 0; r < rows; r += most) {
+        const uint32_t total = static_cast<uint32_t>((rows - r < most ? rows - r : most) * pieces);
+        hipLaunchKernelGGL(pad16_kernel, dim3((total + kBlock * kPadPieces - 1) / (kBlock * kPadPieces)), dim3(kBlock), 0,
+                           static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(src) + r * ld_src,
+                           static_cast<uint4*>(dst) + r * pieces, total, static_cast<uint32_t>(pieces), cols, ld_src);
+        if (int rc = check_launch("pad16_kernel")) return rc;
+    }
+    return 0;
 }
 
 namespace ddl {

@@ -800,12 +800,13 @@ _LINEAR_DTYPES = {
 
 
 def _padded_k(t, k8):
-    """``t[rows, k]`` copied into a fresh ``[rows, k8]`` tensor whose extra columns are zero."""
+    """``t[rows, k]`` (16-bit elements, rows at any pitch) copied into a fresh ``[rows, k8]`` tensor whose extra columns are
+    zero."""
     rows, k = t.shape
-    out = torch.zeros((rows, k8), dtype=t.dtype, device=t.device)
-    if rows > 0 and k > 0:
-        full = [slice(0, rows), slice(0, k)]
-        copy_box(t, full, out, full)
+    out = torch.empty((rows, k8), dtype=t.dtype, device=t.device)
+    if out.numel():
+        rc = _lib.load().ddl_pad_rows(t.data_ptr(), out.data_ptr(), rows, k, t.stride(0) if rows > 1 else k, k8, 2, _stream())
+        _lib.check(rc, "ddl_pad_rows")
     return out
 
 
@@ -904,11 +905,10 @@ def transpose_2d(src, ld_dst=None):
         src = contiguous(src)
     rows, cols = src.shape
     ld_dst = rows if ld_dst is None else ld_dst
-    alloc = torch.empty if ld_dst == rows else torch.zeros
-    dst = alloc((cols, ld_dst), dtype=src.dtype, device=src.device)
-    rc = _lib.load().ddl_transpose_2d(src.data_ptr(), dst.data_ptr(), rows, cols, src.stride(0) if rows > 1 else cols,
-                                      ld_dst, 2, _stream())
-    _lib.check(rc, "ddl_transpose_2d")
+    dst = torch.empty((cols, ld_dst), dtype=src.dtype, device=src.device)
+    rc = _lib.load().ddl_transpose_padded(src.data_ptr(), dst.data_ptr(), rows, cols, src.stride(0) if rows > 1 else cols,
+                                          ld_dst, ld_dst, 2, _stream())
+    _lib.check(rc, "ddl_transpose_padded")
     return dst
 
 

@@ -561,6 +561,17 @@ int ddl_gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride,
 int ddl_transpose_2d(const void* src, void* dst, int64_t rows, int64_t cols,
                      int64_t ld_src, int64_t ld_dst, int elem_size, void* stream);
 
+/* The same, and zeros in the columns rows .. width of dst (width <= ld_dst). */
+int ddl_transpose_padded(const void* src, void* dst, int64_t rows, int64_t cols,
+                         int64_t ld_src, int64_t ld_dst, int64_t width,
+                         int elem_size, void* stream);
+
+/* dst[r, c] = src[r, c] for c < cols and zero for cols <= c < width: rows of
+ * 2-byte elements (elem_size = 2) at any pitch (also 0) into rows of `width`, a multiple
+ * of 8, end to end from a 16-byte aligned dst. */
+int ddl_pad_rows(const void* src, void* dst, int64_t rows, int64_t cols,
+                 int64_t ld_src, int64_t width, int elem_size, void* stream);
+
 /* out[c] = sum over r < rows of a[r, c], fp32 accumulation, rounded once to
  * `dtype` (bf16, fp16 or fp32: the type of a and out), for the bias gradient.
  * `workspace` is device memory for at least `cols` floats (up to 64 * cols are

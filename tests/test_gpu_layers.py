@@ -1390,6 +1390,39 @@ def test_transpose_2d_is_bit_exact(ops, rows, cols):
     assert torch.equal(ops.transpose_2d(wide[:, 2:2 + cols]).cpu(), wide[:, 2:2 + cols].cpu().t().contiguous())
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (8, 8), (63, 65), (64, 64), (65, 127), (515, 9), (7, 1025)])
+@pytest.mark.parametrize("address,pitch", [(0, 0), (1, 1), (3, 6)])
+def test_padded_transpose_and_padded_rows_at_any_address(ops, rows, cols, address, pitch):
+    """Every bit arrives, the padding is cleared whatever was there, and nothing past it is touched; rows at any 2-byte
+    address and pitch, also one row read again and again."""
+    from distdl_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(rows * 100 + cols)
+    ld = cols + pitch
+    pool = torch.randint(-32768, 32767, (rows * ld + address,), generator=gen, dtype=torch.int16)
+    src = pool[address:].view(rows, ld)[:, :cols]
+    dev = pool.cuda()
+    ptr = dev.data_ptr() + 2 * address
+    width = (rows + 7) // 8 * 8
+    for more, start in ((0, 0), (5, 0), (3, 1)):              # columns of dst past the padding; its address in elements
+        dst = torch.full((cols * (width + more) + start + 8,), 77, dtype=torch.int16, device="cuda")
+        _lib.check(lib.ddl_transpose_padded(ptr, dst.data_ptr() + 2 * start, rows, cols, ld, width + more, width, 2, None), "t")
+        got = dst.cpu()
+        body = got[start:start + cols * (width + more)].view(cols, width + more)
+        assert torch.equal(body[:, :rows], src.t()) and not body[:, rows:width].any() and (body[:, width:] == 77).all()
+        assert (got[:start] == 77).all() and (got[-8:] == 77).all()
+    width = (cols + 7) // 8 * 8 + 8
+    for step in (ld, 0):
+        dst = torch.full((rows * width + 8,), 77, dtype=torch.int16, device="cuda")
+        _lib.check(lib.ddl_pad_rows(ptr, dst.data_ptr(), rows, cols, step, width, 2, None), "p")
+        got = dst.cpu()
+        body = got[:rows * width].view(rows, width)
+        assert torch.equal(body[:, :cols], src if step else src[:1].expand(rows, cols))
+        assert not body[:, cols:].any() and (got[-8:] == 77).all()
+    assert lib.ddl_transpose_padded(ptr, dst.data_ptr(), rows, cols, ld, rows, rows + 1, 2, None) == -1
+    assert lib.ddl_pad_rows(ptr, dst.data_ptr(), rows, cols, ld, cols + 7 - (cols + 6) % 8, 2, None) == -1
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (128, 64), (129, 65), (8192, 200), (3000, 1000)])
 def test_colsum_bf16(ops, rows, cols):
     gen = torch.Generator().manual_seed(rows + cols)
