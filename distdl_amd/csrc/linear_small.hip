@@ -698,8 +698,10 @@ Small16 plan_small16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus,
 
 // Fits of a sweep as above: 1.1 us per round of two k-tiles for a lone workgroup, 0.7 for each that a CU has to work through.
 // The other way -- operands copied into padded or transposed temporaries -- is 30 us of launches and allocations in front
-// of the product, plus the copies at 4.5 TB/s.  Measured, copies and product -> here: M 8, N 3583, K 8191 82.4 -> 21.5 us;
-// M = N = K = 1023 35.9 -> 13.5; M 2049, N 511, K 4097 86.3 -> 45.9; M 4097, N 2049, K 2049 113.7, here 121.1.
+// of the product, plus the copies at 4.5 TB/s.  Measured, copies and product -> here: M 8, N 3583, K 8191 37.6 -> 21.3 us;
+// M = N = K = 1023 20.5 -> 13.5; M 2049, N 511, K 4097 49.7 -> 48.4; M 4097, N 2049, K 2049 58.9, here 123.  The copies
+// alone are cheaper than that, what the host does for them is not: with 12 us for 30 a training step of M 4001, N 1001,
+// K 2051 goes from 184 to 217 us.
 Small16 plan_any16(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double large_us) {
     Small16 best;
     const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), ktiles = (K + BK - 1) / BK;
