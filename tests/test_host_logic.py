@@ -809,6 +809,45 @@ def test_halo_exchange_uses_the_buffers_it_is_handed(boxes_on_the_cpu):
         assert dx.tolist() == [0, 1 + 1, 2 + 2, 3 + 3, 4 + 4, 0]
 
 
+@pytest.mark.parametrize("shape,recv,send", [
+    ((5, 6), [[1, 1], [1, 1]], [[1, 1], [1, 1]]),
+    ((7, 9), [[2, 1], [1, 3]], [[1, 2], [2, 1]]),
+    ((2, 7, 6, 8), [[0, 0], [2, 2], [1, 1], [2, 2]], [[0, 0], [2, 2], [1, 1], [2, 2]]),
+    ((7, 6, 8), [[2, 0], [0, 2], [1, 1]], [[0, 2], [2, 0], [1, 1]]),      # one-sided
+    ((7, 6, 8), [[1, 1], [0, 0], [1, 1]], [[1, 1], [0, 0], [1, 1]]),      # a dimension without an exchange in between
+    ((6, 4), [[2, 2], [2, 1]], [[1, 1], [1, 1]]),                         # a bulk of one column: both strips are it
+    ((4, 5), [[2, 2], [1, 1]], [[0, 0], [3, 3]])])                        # no bulk along the first dimension
+@pytest.mark.parametrize("buffers", ["four", "missing", "shared"])
+def test_halo_strips_packed_while_ghosts_are_unpacked(boxes_on_the_cpu, monkeypatch, shape, recv, send, buffers):
+    """One launch for a dimension's ghosts and the next one's strips does what two do, one after the other; a ghost without
+    a buffer keeps what the tensor had, and a buffer that is a ghost's and the next strip's is unpacked first."""
+    from distdl_amd.backends.stub_hip.functional import halo_exchange as h
+    torch.manual_seed(len(shape) + shape[0])
+    x = torch.randn(shape)
+    results = []
+    for fused in (True, False):
+        if not fused:
+            monkeypatch.setattr(h._Plan, "_with_unpacking", staticmethod(lambda *args: None))
+        e = _Exchange(shape, recv, send)
+        buf = e.buffers(0.0)
+        for sides in buf:
+            if buffers == "missing":
+                sides[1] = None
+            elif buffers == "shared" and sides[0] is not None:
+                sides[0] = next((row[1] for row in buf if row[1] is not None), sides[0])
+        gen = torch.Generator().manual_seed(1)
+
+        def swap(P, neighbors, out_left, out_right, in_left, in_right):
+            for t in (in_left, in_right):                       # what arrives depends on what has been sent
+                if t is not None:
+                    sent = sum(float(s.double().sum()) for s in (out_left, out_right) if s is not None)
+                    t.copy_(torch.randn(t.shape, generator=gen) + sent)
+
+        monkeypatch.setattr(h, "_swap", swap)
+        results.append(e.forward(x, buf))
+    assert torch.equal(results[0], results[1])
+
+
 def test_halo_exchange_of_a_tensor_with_more_dimensions_than_the_partition(boxes_on_the_cpu):
     """The dimensions of the partition are exchanged, those behind them are left alone."""
     e = _Exchange((4, 2), [[1, 0], [0, 0]], [[1, 0], [0, 0]], dims=1)
