@@ -11,7 +11,7 @@
 //                registers between the two halves, so x is read once
 //
 // Three ways of holding a row, chosen by its length:
-//   wavefront rows  up to 2048 columns: one wavefront owns a row, each lane
+//   wavefront rows  up to 1024 columns, 2048 of aligned fp32: one wavefront owns a row, each lane
 //                   holds pieces of four elements, sums go through shuffle
 //                   butterflies; a long input keeps two rows per wavefront in
 //                   flight
@@ -21,7 +21,7 @@
 //   streamed rows   anything longer, and more rows than one launch has wavefronts for: a
 //                   workgroup walks the row once per reduction
 // Rows whose length, pitch or address are no multiples of four elements are held in
-// the same way; only the end of such a row is fetched element by element.
+// the same way; the last piece of such a row ends with it.
 #include "ddl_common.h"
 
 #include "ln_elements.h"
@@ -33,7 +33,10 @@ constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxParts = 256;
-constexpr int kWaveRowCols = 2048;     // longest row a wavefront keeps in registers
+// The longest row a wavefront keeps in registers: of aligned fp32, and of anything else, whose pieces of four are half as
+// wide or cross lines.  By a wavefront and by a workgroup: [32000, 2048] fp32 89 and 95 us, [45000, 1200] 73 and 76; but
+// bf16 62 and 42, 59 and 42; [32000, 2045] bf16 115 and 53, fp32 96 and 99; [45000, 1201] bf16 125 and 44, fp32 88 and 79.
+constexpr int kWaveRowCols = 2048, kNarrowRowCols = 1024;
 constexpr int kBlockRowCols = 16384;   // longest row a workgroup keeps in registers
 
 struct PartCounts {
@@ -45,11 +48,17 @@ __device__ inline float sq4(float4 v, float m) {
     const float a = v.x - m, b = v.y - m, c = v.z - m, d = v.w - m;
     return (a * a + b * b) + (c * c + d * d);
 }
+// Of all but the first n elements.
 template <bool ANY>
-__device__ inline float sq_piece(float4 v, float m, int n) {   // of the first n elements
-    if (!ANY || n >= 4) return sq4(v, m);
-    const float a = v.x - m, b = n > 1 ? v.y - m : 0.f, c = n > 2 ? v.z - m : 0.f;
-    return (a * a + b * b) + c * c;
+__device__ inline float sum_piece(float4 v, int n) {
+    if (!ANY || n <= 0) return sum4(v);
+    return ((n > 1 ? 0.f : v.y) + (n > 2 ? 0.f : v.z)) + (n > 3 ? 0.f : v.w);
+}
+template <bool ANY>
+__device__ inline float sq_end(float4 v, float m, int n) {
+    if (!ANY || n <= 0) return sq4(v, m);
+    const float b = n > 1 ? 0.f : v.y - m, c = n > 2 ? 0.f : v.z - m, d = n > 3 ? 0.f : v.w - m;
+    return (b * b + c * c) + d * d;
 }
 __device__ inline float4 norm4(float4 v, float mean, float rstd) {
     return make_float4((v.x - mean) * rstd, (v.y - mean) * rstd, (v.z - mean) * rstd, (v.w - mean) * rstd);
@@ -130,7 +139,7 @@ struct LnArgs {
 // --------------------------------------------------------- wavefront rows --
 
 // One wavefront per row, NV pieces of four per lane (cols <= 256 NV), RPW rows of a
-// wavefront in flight at once.  ANY: rows of any length, pitch and address.
+// wavefront in flight at once.  ANY: rows of at least four columns, of any length, pitch and address.
 template <typename T, int NV, int RPW, int MODE, bool AFFINE, bool ANY>
 __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int64_t rows_first, int64_t ld_first, int cols_first,
                                                        const LnArgs a_rest, const PartCounts pc) {
@@ -147,14 +156,19 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
     const int64_t r0 = wave * RPW;
     const int64_t rows = a.rows;
     const int nv = (a.cols + 3) >> 2;
+    // The last piece of a row ends with it: its first elements are the end of the piece before, are left out of the sums and
+    // written twice.  (Fetched element by element instead, the branch kept the other loads from being in flight: [30000, 801]
+    // bf16 41 us, here 28; [8192, 1023] fp32 15.1, here 11.9.)
+    auto column = [&](int c) { return ANY && c == nv - 1 ? a.cols - 4 : 4 * c; };
+    auto again = [&](int c) { return ANY && c == nv - 1 ? 4 * nv - a.cols : 0; };
     float4 g[NV], b[NV];
     if (MODE != kStats && AFFINE) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int c = lane + k * kWave;
             if (c < nv) {
-                g[k] = load_piece<ANY>(static_cast<const T*>(a.gamma) + 4 * c, a.cols - 4 * c);
-                b[k] = load_piece<ANY>(static_cast<const T*>(a.beta) + 4 * c, a.cols - 4 * c);
+                g[k] = load_piece<ANY>(static_cast<const T*>(a.gamma) + column(c));
+                b[k] = load_piece<ANY>(static_cast<const T*>(a.beta) + column(c));
             }
         }
     }
@@ -178,7 +192,7 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int c = lane + k * kWave;
-            v[i][k] = (r < rows && c < nv) ? load_piece<ANY>(x + r * a.ld + 4 * c, a.cols - 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[i][k] = (r < rows && c < nv) ? load_piece<ANY>(x + r * a.ld + column(c)) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
     const float inv = 1.0f / static_cast<float>(a.cols);
@@ -192,12 +206,12 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
         } else {
             float s = 0.f;
 #pragma unroll
-            for (int k = 0; k < NV; ++k) s += sum4(v[i][k]);
+            for (int k = 0; k < NV; ++k) s += sum_piece<ANY>(v[i][k], again(lane + k * kWave));
             mean = wave_sum(s) * inv;
             float q = 0.f;
 #pragma unroll
             for (int k = 0; k < NV; ++k)
-                if (lane + k * kWave < nv) q += sq_piece<ANY>(v[i][k], mean, a.cols - 4 * (lane + k * kWave));
+                if (lane + k * kWave < nv) q += sq_end<ANY>(v[i][k], mean, again(lane + k * kWave));
             q = wave_sum(q);
             if (MODE == kStats || MODE == kJoined) {
                 if (lane == 0) reinterpret_cast<float2*>(a.stats)[r] = make_float2(mean, q);
@@ -219,7 +233,7 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
             if (c < nv) {
                 float4 o = norm4(v[i][k], mean, rstd);
                 if (AFFINE) o = affine4(g[k], o, b[k]);
-                store_piece<ANY>(y + r * a.ldy + 4 * c, o, a.cols - 4 * c);
+                store_piece<ANY>(y + r * a.ldy + column(c), o);
             }
         }
     }
@@ -227,11 +241,12 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
 
 // --------------------------------------------------------- workgroup rows --
 
-// V elements of a row as they lie in memory, 8 or 16 bytes; global memory takes them at the alignment of four elements.
-template <typename T, int V>
+// V elements of a row as they lie in memory, 8 or 16 bytes; global memory takes them at the alignment of four elements, or
+// of one (ANY).
+template <typename T, int V, bool ANY>
 struct RowPiece {
     static_assert(V % 4 == 0, "pieces are quartets of elements");
-    struct __attribute__((packed, aligned(4 * sizeof(T)))) Raw {
+    struct __attribute__((packed, aligned((ANY ? 1 : 4) * sizeof(T)))) Raw {
         uint32_t word[V * sizeof(T) / 4];
     };
     static __device__ Raw load(const T* p) { return *reinterpret_cast<const Raw*>(p); }
@@ -246,7 +261,6 @@ struct RowPiece {
     // The same streaming stores as store4, as one access.
     static __device__ void store(T* p, const float4 (&v)[V / 4]) {
         typedef uint32_t words __attribute__((ext_vector_type(V * sizeof(T) / 4)));
-        typedef words any __attribute__((aligned(4 * sizeof(T))));
         words o;
 #pragma unroll
         for (int q = 0; q < V / 4; ++q) {
@@ -260,7 +274,12 @@ struct RowPiece {
                 o[2 * q] = *reinterpret_cast<const uint32_t*>(&a), o[2 * q + 1] = *reinterpret_cast<const uint32_t*>(&b);
             }
         }
-        __builtin_nontemporal_store(o, reinterpret_cast<any*>(p));
+        if constexpr (ANY) {
+            store_stream(p, o);
+        } else {
+            typedef words any __attribute__((aligned(4 * sizeof(T))));
+            __builtin_nontemporal_store(o, reinterpret_cast<any*>(p));
+        }
     }
 };
 
@@ -279,21 +298,26 @@ __device__ inline float group_sum(float v, float* scratch) {
     return t;
 }
 
-// Rows whose columns, pitch and address are multiples of four elements: a workgroup per row, thread t holding the V-element
-// pieces t + THREADS k, k < NP, as they lie in memory.  A workgroup walks several rows; gamma and beta stay in its registers
+// A workgroup per row, thread t holding the V-element pieces t + THREADS k, k < NP, as they lie in memory; rows whose
+// columns, pitch and address are multiples of four elements, or (ANY) of any length, pitch and address.  A workgroup walks several rows; gamma and beta stay in its registers
 // and the next row is on its way while this one is summed.  Bound by HBM.  With one row per workgroup gamma and beta were
 // twice the row's own traffic in L2, the loads 8 bytes a lane in 16-bit types, and nothing was in flight while the row was
 // reduced: [8192, 8192] bf16 with statistics 68 to 82 us, here 48 (5.6 TB/s; a copy reaches 5.9); [4096, 8192] fp32 53 -> 48;
 // [20000, 2560] bf16 41 -> 33, with the other workers' statistics in memory 69 -> 39; [64, 8192] bf16 6.0 -> 3.9.
-template <typename T, int V, int THREADS, int NP, int MODE, bool AFFINE>
+// Unaligned, with the end of a row fetched element by element: [8000, 8191] bf16 116 us, here 55; [5461, 6143] normalised
+// 50 -> 23.
+template <typename T, int V, int THREADS, int NP, int MODE, bool AFFINE, bool ANY>
 __global__ __launch_bounds__(THREADS) void ln_group_rows(const LnArgs a, const PartCounts pc) {
-    typedef RowPiece<T, V> P;
+    typedef RowPiece<T, V, ANY> P;
     typedef typename P::Raw Raw;
     __shared__ float scratch[2][THREADS / kWave];
     const T* __restrict__ x = static_cast<const T*>(a.x);
     T* __restrict__ y = static_cast<T*>(a.y);
     const int t = threadIdx.x, lane = t & (kWave - 1);
-    const int pieces = a.cols / V;
+    const int pieces = (a.cols + V - 1) / V;
+    // The end of a row as in ln_wave_rows.
+    auto column = [&](int c) { return ANY && c == pieces - 1 ? a.cols - V : V * c; };
+    auto again = [&](int c) { return ANY && c == pieces - 1 ? V * pieces - a.cols : 0; };
     const float inv = 1.0f / static_cast<float>(a.cols);
     constexpr bool kPairs = MODE == kNorm || MODE == kJoined;   // takes the workers' {mean, M2} from memory
     Raw v[NP], g[NP], b[NP];
@@ -303,7 +327,7 @@ __global__ __launch_bounds__(THREADS) void ln_group_rows(const LnArgs a, const P
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
             const int c = t + k * THREADS;
-            if (c < pieces) to[k] = P::load(x + r * a.ld + V * c);
+            if (c < pieces) to[k] = P::load(x + r * a.ld + column(c));
         }
     };
     int64_t r = blockIdx.x;
@@ -313,8 +337,8 @@ __global__ __launch_bounds__(THREADS) void ln_group_rows(const LnArgs a, const P
         for (int k = 0; k < NP; ++k) {
             const int c = t + k * THREADS;
             if (c < pieces) {
-                g[k] = P::load(static_cast<const T*>(a.gamma) + V * c);
-                b[k] = P::load(static_cast<const T*>(a.beta) + V * c);
+                g[k] = P::load(static_cast<const T*>(a.gamma) + column(c));
+                b[k] = P::load(static_cast<const T*>(a.beta) + column(c));
             }
         }
     }
@@ -334,14 +358,14 @@ __global__ __launch_bounds__(THREADS) void ln_group_rows(const LnArgs a, const P
             for (int k = 0; k < NP; ++k)
                 if (t + k * THREADS < pieces)
 #pragma unroll
-                    for (int q = 0; q < V / 4; ++q) s += sum4(P::quad(v[k], q));
+                    for (int q = 0; q < V / 4; ++q) s += sum_piece<ANY>(P::quad(v[k], q), again(t + k * THREADS) - 4 * q);
             mean = group_sum<THREADS>(s, scratch[0]) * inv;
             float m2 = 0.f;
 #pragma unroll
             for (int k = 0; k < NP; ++k)
                 if (t + k * THREADS < pieces)
 #pragma unroll
-                    for (int q = 0; q < V / 4; ++q) m2 += sq4(P::quad(v[k], q), mean);
+                    for (int q = 0; q < V / 4; ++q) m2 += sq_end<ANY>(P::quad(v[k], q), mean, again(t + k * THREADS) - 4 * q);
             m2 = group_sum<THREADS>(m2, scratch[1]);
             if ((MODE == kStats || MODE == kJoined) && t == 0) reinterpret_cast<float2*>(a.stats)[r] = make_float2(mean, m2);
             if (MODE == kJoined)
@@ -365,7 +389,7 @@ __global__ __launch_bounds__(THREADS) void ln_group_rows(const LnArgs a, const P
                         o[q] = norm4(P::quad(v[k], q), mean, rstd);
                         if (AFFINE) o[q] = affine4(P::quad(g[k], q), o[q], P::quad(b[k], q));
                     }
-                    P::store(y + r * a.ldy + V * c, o);
+                    P::store(y + r * a.ldy + column(c), o);
                 }
             }
         }
@@ -373,67 +397,6 @@ __global__ __launch_bounds__(THREADS) void ln_group_rows(const LnArgs a, const P
             first = first_next;
 #pragma unroll
             for (int k = 0; k < NP; ++k) v[k] = v_next[k];
-        }
-    }
-}
-
-// Rows of any length, pitch and address: one workgroup per row, NV pieces of four per thread (cols <= 1024 NV); the grid
-// walks the rows.
-template <typename T, int NV, int MODE, bool AFFINE>
-__global__ __launch_bounds__(kBlock) void ln_block_rows(const LnArgs a, const PartCounts pc) {
-    __shared__ float scratch[kWavesPerBlock];
-    const T* __restrict__ x = static_cast<const T*>(a.x);
-    T* __restrict__ y = static_cast<T*>(a.y);
-    const int t = threadIdx.x, lane = t & (kWave - 1);
-    const int nv = (a.cols + 3) >> 2;
-    const float inv = 1.0f / static_cast<float>(a.cols);
-    for (int64_t r = blockIdx.x; r < a.rows; r += gridDim.x) {
-        float2 first = make_float2(0.f, 0.f);
-        if ((MODE == kNorm || MODE == kJoined) && lane < a.nparts) first = load_part(a.part_stats, a.rows, r, lane);
-        float4 v[NV];
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const int c = t + k * kBlock;
-            v[k] = c < nv ? load_piece<true>(x + r * a.ld + 4 * c, a.cols - 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        float mean, rstd;
-        if (MODE == kNorm) {
-            // every wavefront combines the pairs for itself: no exchange needed
-            combine_parts(a.part_stats, a.rows, r, a.nparts, pc, a.eps, lane, first, lane < a.nparts ? pc.inv_n[lane] : 0.f,
-                          &mean, &rstd);
-        } else {
-            float s = 0.f;
-#pragma unroll
-            for (int k = 0; k < NV; ++k) s += sum4(v[k]);
-            mean = block_sum(s, scratch) * inv;
-            float q = 0.f;
-#pragma unroll
-            for (int k = 0; k < NV; ++k)
-                if (t + k * kBlock < nv) q += sq_piece<true>(v[k], mean, a.cols - 4 * (t + k * kBlock));
-            q = block_sum(q, scratch);
-            if (MODE == kStats || MODE == kJoined) {
-                if (t == 0) reinterpret_cast<float2*>(a.stats)[r] = make_float2(mean, q);
-                if (MODE == kStats) continue;
-            }
-            if (MODE == kJoined)
-                combine_parts(a.part_stats, a.rows, r, a.nparts, pc, a.eps, lane, lane == a.my_part ? make_float2(mean, q) : first,
-                              lane < a.nparts ? pc.inv_n[lane] : 0.f, &mean, &rstd);
-            else
-                rstd = 1.0f / sqrtf(q * inv + a.eps);
-        }
-        if (t == 0) {
-            if (a.mean_out) a.mean_out[r] = mean;
-            if (a.rstd_out) a.rstd_out[r] = rstd;
-        }
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const int c = t + k * kBlock;
-            if (c < nv) {
-                float4 o = norm4(v[k], mean, rstd);
-                if (AFFINE) o = affine4(load_piece<true>(static_cast<const T*>(a.gamma) + 4 * c, a.cols - 4 * c), o,
-                                        load_piece<true>(static_cast<const T*>(a.beta) + 4 * c, a.cols - 4 * c));
-                store_piece<true>(y + r * a.ldy + 4 * c, o, a.cols - 4 * c);
-            }
         }
     }
 }
@@ -527,55 +490,43 @@ void launch_wave(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
         launch_wave_rpw<T, MODE, AFFINE, ANY, NV, 1>(a, pc, s);
 }
 
-template <typename T, int MODE, bool AFFINE, int NV>
-void launch_block(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
-    const uint32_t blocks = static_cast<uint32_t>(a.rows < (1 << 20) ? a.rows : (1 << 20));
-    hipLaunchKernelGGL((ln_block_rows<T, NV, MODE, AFFINE>), dim3(blocks), dim3(kBlock), 0, s, a, pc);
-}
-
 // Rows per workgroup of ln_group_rows: enough to share gamma and beta, few enough that every CU has several workgroups.
 constexpr int64_t kGroupRows = 8;
 
-template <typename T, int MODE, bool AFFINE, int V, int THREADS, int NP>
+template <typename T, int MODE, bool AFFINE, bool ANY, int V, int THREADS, int NP>
 void launch_group(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     int dev = 0;
     const int64_t waves = 16 * compute_units(dev);
     int64_t per = a.rows * (THREADS / kWave) / waves;
     per = per < 1 ? 1 : per > kGroupRows ? kGroupRows : per;
     const int64_t blocks = (a.rows + per - 1) / per;
-    hipLaunchKernelGGL((ln_group_rows<T, V, THREADS, NP, MODE, AFFINE>), dim3(static_cast<uint32_t>(blocks < (1 << 20) ? blocks : (1 << 20))), dim3(THREADS), 0, s, a, pc);
+    hipLaunchKernelGGL((ln_group_rows<T, V, THREADS, NP, MODE, AFFINE, ANY>), dim3(static_cast<uint32_t>(blocks < (1 << 20) ? blocks : (1 << 20))), dim3(THREADS), 0, s, a, pc);
 }
 
-template <typename T, int MODE, bool AFFINE, int V>
+template <typename T, int MODE, bool AFFINE, bool ANY, int V>
 void launch_group_pieces(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
-    const int pieces = a.cols / V;   // up to 16384 / V
-    if (pieces <= 512) launch_group<T, MODE, AFFINE, V, 256, 2>(a, pc, s);
-    else if (pieces <= 1024) launch_group<T, MODE, AFFINE, V, 256, 4>(a, pc, s);
-    else if (pieces <= 2048) launch_group<T, MODE, AFFINE, V, 512, 4>(a, pc, s);
-    else launch_group<T, MODE, AFFINE, V, 1024, 4>(a, pc, s);
+    const int pieces = (a.cols + V - 1) / V;   // up to 16384 / V
+    if (pieces <= 512) launch_group<T, MODE, AFFINE, ANY, V, 256, 2>(a, pc, s);
+    else if (pieces <= 1024) launch_group<T, MODE, AFFINE, ANY, V, 256, 4>(a, pc, s);
+    else if (pieces <= 2048) launch_group<T, MODE, AFFINE, ANY, V, 512, 4>(a, pc, s);
+    else launch_group<T, MODE, AFFINE, ANY, V, 1024, 4>(a, pc, s);
 }
 
 // Rows of up to kBlockRowCols columns, held in registers.
 template <typename T, int MODE, bool AFFINE, bool ANY>
 int launch_held(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     const int cols = a.cols;
-    if (cols <= kWaveRowCols) {
+    if (cols <= (sizeof(T) == 4 && !ANY ? kWaveRowCols : kNarrowRowCols)) {
         if (cols <= 256) launch_wave<T, MODE, AFFINE, ANY, 1>(a, pc, s);
         else if (cols <= 512) launch_wave<T, MODE, AFFINE, ANY, 2>(a, pc, s);
         else if (cols <= 1024) launch_wave<T, MODE, AFFINE, ANY, 4>(a, pc, s);
         else launch_wave<T, MODE, AFFINE, ANY, 8>(a, pc, s);
         return check_launch("ln_wave_rows");
     }
-    if constexpr (!ANY) {
-        if (sizeof(T) == 2 && cols % 8 == 0) launch_group_pieces<T, MODE, AFFINE, 16 / static_cast<int>(sizeof(T))>(a, pc, s);
-        else launch_group_pieces<T, MODE, AFFINE, 4>(a, pc, s);
-        return check_launch("ln_group_rows");
-    } else {
-        if (cols <= 4096) launch_block<T, MODE, AFFINE, 4>(a, pc, s);
-        else if (cols <= 8192) launch_block<T, MODE, AFFINE, 8>(a, pc, s);
-        else launch_block<T, MODE, AFFINE, 16>(a, pc, s);
-        return check_launch("ln_block_rows");
-    }
+    constexpr int kWide = 16 / static_cast<int>(sizeof(T));
+    if (ANY || cols % kWide == 0) launch_group_pieces<T, MODE, AFFINE, ANY, kWide>(a, pc, s);
+    else if constexpr (kWide != 4 && !ANY) launch_group_pieces<T, MODE, AFFINE, ANY, 4>(a, pc, s);
+    return check_launch("ln_group_rows");
 }
 
 template <typename T, int MODE, bool AFFINE>
@@ -586,7 +537,7 @@ int launch_typed(const LnArgs& a, const PartCounts& pc, bool vec, hipStream_t s)
     if (vec && cols <= kBlockRowCols && (one_launch || MODE == kJoined)) return launch_held<T, MODE, AFFINE, false>(a, pc, s);
     if constexpr (MODE != kJoined) {
         // Rows that start at any element: held as well, instead of read element by element once per reduction.
-        if (cols <= kBlockRowCols && one_launch) return launch_held<T, MODE, AFFINE, true>(a, pc, s);
+        if (cols >= 4 && cols <= kBlockRowCols && one_launch) return launch_held<T, MODE, AFFINE, true>(a, pc, s);
     }
     if constexpr (MODE == kJoined) {
         return fail(DDL_E_UNSUPP, "ln stats+normalize: rows of more than %d columns take the two-launch form", kBlockRowCols);

@@ -38,7 +38,40 @@ constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kStrip = 64;     // columns per workgroup of the parameter kernel
 
-template <typename T, bool VEC>
+constexpr int kAhead = 4;   // pieces of a row that a lane requests together
+
+// Four elements of dy, x and gamma.  ANY: at any address.
+template <typename T, bool ANY>
+struct BwdPiece {
+    float4 d, v, g;
+    __device__ void load(const T* dy, const T* x, const T* gamma, int64_t c) {
+        d = load_piece<ANY>(dy + c);
+        v = load_piece<ANY>(x + c);
+        g = gamma ? load_piece<ANY>(gamma + c) : make_float4(1.f, 1.f, 1.f, 1.f);
+    }
+};
+
+// Column at which the piece from `c` on is fetched.  ANY: the last piece of a row of four columns and more ends with the
+// row, and its first elements are those of the piece in front of it once more: left out of sums, written twice.  (A branch
+// for the end of a row keeps the loads of the other pieces from being in flight.)
+template <bool ANY, typename I>
+__device__ inline I piece_column(I c, I cols) {
+    return ANY && c + 4 > cols ? cols - 4 : c;
+}
+
+// The piece without the elements that the one in front of it has.
+template <bool ANY>
+__device__ inline float4 own_elements(float4 d, int again) {
+    if (ANY && again > 0) {
+        d.x = 0.f;
+        if (again > 1) d.y = 0.f;
+        if (again > 2) d.z = 0.f;
+    }
+    return d;
+}
+
+// ANY: rows of any length, pitch and address ([5461, 6143] bf16 81 us element by element, here 26; ln_bwd_input 68, here 36).
+template <typename T, bool ANY>
 __global__ __launch_bounds__(kBlock) void ln_bwd_partial(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows,
                                                          int64_t cols, int64_t ld_dy, int64_t ld_x,
                                                          const float* __restrict__ mean, const float* __restrict__ rstd,
@@ -50,21 +83,26 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_partial(const T* __restrict__ d
     const T* dyr = dy + r * ld_dy;
     const T* xr = x + r * ld_x;
     float s1 = 0.f, s2 = 0.f;
-    if (VEC) {
-        for (int64_t c = lane * 4; c < cols; c += kWave * 4) {
-            const float4 d = load4(dyr + c);
-            const float4 v = load4(xr + c);
-            float4 g = make_float4(1.f, 1.f, 1.f, 1.f);
-            if (gamma) g = load4(gamma + c);
-            const float g0 = d.x * g.x, g1 = d.y * g.y, g2 = d.z * g.z, g3 = d.w * g.w;
-            s1 += (g0 + g1) + (g2 + g3);
-            s2 += (g0 * ((v.x - m) * rs) + g1 * ((v.y - m) * rs)) + (g2 * ((v.z - m) * rs) + g3 * ((v.w - m) * rs));
+    if (ANY && cols < 4) {
+        if (lane < cols) {
+            s1 = load1(dyr + lane) * (gamma ? load1(gamma + lane) : 1.f);
+            s2 = s1 * ((load1(xr + lane) - m) * rs);
         }
     } else {
-        for (int64_t c = lane; c < cols; c += kWave) {
-            const float g = load1(dyr + c) * (gamma ? load1(gamma + c) : 1.f);
-            s1 += g;
-            s2 += g * ((load1(xr + c) - m) * rs);
+        for (int64_t first = lane * 4; first < cols; first += kAhead * kWave * 4) {
+            BwdPiece<T, ANY> p[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k)
+                if (first + k * (kWave * 4) < cols) p[k].load(dyr, xr, gamma, piece_column<ANY>(first + k * (kWave * 4), cols));
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int64_t c = first + k * (kWave * 4);
+                if (c >= cols) break;
+                const float4 d = own_elements<ANY>(p[k].d, static_cast<int>(c - piece_column<ANY>(c, cols))), v = p[k].v, g = p[k].g;
+                const float g0 = d.x * g.x, g1 = d.y * g.y, g2 = d.z * g.z, g3 = d.w * g.w;
+                s1 += (g0 + g1) + (g2 + g3);
+                s2 += (g0 * ((v.x - m) * rs) + g1 * ((v.y - m) * rs)) + (g2 * ((v.z - m) * rs) + g3 * ((v.w - m) * rs));
+            }
         }
     }
     s1 = wave_sum(s1);
@@ -83,7 +121,7 @@ __device__ inline float dx_value(float dyv, float gv, float xv, float m, float r
     return rs * q;
 }
 
-template <typename T, bool VEC>
+template <typename T, bool ANY>
 __device__ inline void ln_bwd_input_body(uint32_t block, const T* __restrict__ dy, const T* __restrict__ x, int64_t rows,
                                          int64_t cols, int64_t ld_dy, int64_t ld_x, const float* __restrict__ mean,
                                          const float* __restrict__ rstd, const T* __restrict__ gamma,
@@ -107,60 +145,46 @@ __device__ inline void ln_bwd_input_body(uint32_t block, const T* __restrict__ d
     // reduced: the reduction waits for the gathered pairs, and the row should
     // not wait behind it (one memory round trip instead of two for rows of up
     // to 1024 columns).
-    constexpr int kAhead = 4;
-    float4 d0[kAhead], v0[kAhead], g0[kAhead];
-    if (VEC) {
+    const bool tiny = ANY && cols < 4;
+    BwdPiece<T, ANY> p[kAhead];
+    auto fetch = [&](int64_t first) {
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) {
-            const int64_t c = lane * 4 + static_cast<int64_t>(k) * (kWave * 4);
-            g0[k] = make_float4(1.f, 1.f, 1.f, 1.f);
-            if (c < cols) {
-                d0[k] = load4(dyr + c);
-                v0[k] = load4(xr + c);
-                if (gamma) g0[k] = load4(gamma + c);
-            }
-        }
-    }
+        for (int k = 0; k < kAhead; ++k)
+            if (first + k * (kWave * 4) < cols) p[k].load(dyr, xr, gamma, piece_column<ANY>(first + k * (kWave * 4), cols));
+    };
+    int64_t first = lane * 4;
+    if (!tiny) fetch(first);
     const float S1 = wave_sum(p1) * weight, S2 = wave_sum(p2) * weight;   // already times a_p
-    if (VEC) {
+    if (tiny) {
+        if (lane < cols) store1(dxr + lane, dx_value(load1(dyr + lane), gamma ? load1(gamma + lane) : 1.f, load1(xr + lane), m, rs, S1, S2));
+        return;
+    }
+    while (true) {
 #pragma unroll
         for (int k = 0; k < kAhead; ++k) {
-            const int64_t c = lane * 4 + static_cast<int64_t>(k) * (kWave * 4);
+            const int64_t c = first + k * (kWave * 4);
             if (c < cols) {
                 float4 o;
-                o.x = dx_value(d0[k].x, g0[k].x, v0[k].x, m, rs, S1, S2);
-                o.y = dx_value(d0[k].y, g0[k].y, v0[k].y, m, rs, S1, S2);
-                o.z = dx_value(d0[k].z, g0[k].z, v0[k].z, m, rs, S1, S2);
-                o.w = dx_value(d0[k].w, g0[k].w, v0[k].w, m, rs, S1, S2);
-                store4(dxr + c, o);
+                o.x = dx_value(p[k].d.x, p[k].g.x, p[k].v.x, m, rs, S1, S2);
+                o.y = dx_value(p[k].d.y, p[k].g.y, p[k].v.y, m, rs, S1, S2);
+                o.z = dx_value(p[k].d.z, p[k].g.z, p[k].v.z, m, rs, S1, S2);
+                o.w = dx_value(p[k].d.w, p[k].g.w, p[k].v.w, m, rs, S1, S2);
+                store_piece<ANY>(dxr + piece_column<ANY>(c, cols), o);   // dx is not read again here: streaming store
             }
         }
-        for (int64_t c = lane * 4 + static_cast<int64_t>(kAhead) * (kWave * 4); c < cols; c += kWave * 4) {
-            const float4 d = load4(dyr + c);
-            const float4 v = load4(xr + c);
-            float4 g = make_float4(1.f, 1.f, 1.f, 1.f);
-            if (gamma) g = load4(gamma + c);
-            float4 o;
-            o.x = dx_value(d.x, g.x, v.x, m, rs, S1, S2);
-            o.y = dx_value(d.y, g.y, v.y, m, rs, S1, S2);
-            o.z = dx_value(d.z, g.z, v.z, m, rs, S1, S2);
-            o.w = dx_value(d.w, g.w, v.w, m, rs, S1, S2);
-            store4(dxr + c, o);   // dx is not read again here: streaming store
-        }
-    } else {
-        for (int64_t c = lane; c < cols; c += kWave) {
-            store1(dxr + c, dx_value(load1(dyr + c), gamma ? load1(gamma + c) : 1.f, load1(xr + c), m, rs, S1, S2));
-        }
+        first += kAhead * kWave * 4;
+        if (first >= cols) break;
+        fetch(first);
     }
 }
 
-template <typename T, bool VEC>
+template <typename T, bool ANY>
 __global__ __launch_bounds__(kBlock) void ln_bwd_input(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows,
                                                        int64_t cols, int64_t ld_dy, int64_t ld_x,
                                                        const float* __restrict__ mean, const float* __restrict__ rstd,
                                                        const T* __restrict__ gamma, const float* __restrict__ part_sums,
                                                        int nparts, float weight, T* __restrict__ dx, int64_t ld_dx) {
-    ln_bwd_input_body<T, VEC>(blockIdx.x, dy, x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, part_sums, nparts, weight, dx, ld_dx);
+    ln_bwd_input_body<T, ANY>(blockIdx.x, dy, x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, part_sums, nparts, weight, dx, ld_dx);
 }
 
 // Workgroup (strip, split): rows [split * rows_per_split, ...) of a 64-column
@@ -272,7 +296,7 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_params_final(const float* __res
 // workgroups (one per 64-column strip) add up the partial column sums -- a chain
 // of dependent loads, so they start first -- and the rest write dx.  The two
 // parts are independent.
-template <typename T, bool VEC>
+template <typename T, bool ANY>
 __global__ __launch_bounds__(kBlock) void ln_bwd_input_final(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows,
                                                              int64_t cols, int64_t ld_dy, int64_t ld_x,
                                                              const float* __restrict__ mean, const float* __restrict__ rstd,
@@ -283,7 +307,7 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_input_final(const T* __restrict
     if (blockIdx.x < final_blocks)
         ln_bwd_params_final_body<T, 8>(blockIdx.x, partial, cols, splits, dgamma, dbeta);
     else
-        ln_bwd_input_body<T, VEC>(blockIdx.x - final_blocks, dy, x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, part_sums, nparts,
+        ln_bwd_input_body<T, ANY>(blockIdx.x - final_blocks, dy, x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, part_sums, nparts,
                                weight, dx, ld_dx);
 }
 
@@ -306,7 +330,7 @@ struct DxArgs {
 // partial has the layout of ln_bwd_params_partial.  WITH_DX: the sums of the
 // whole row are complete once this worker's are (it holds the row whole, or the
 // other workers' pairs are in memory), so dx is written in the same pass, from
-// the registers that hold the row.  ANY: rows of any length, pitch and address.
+// the registers that hold the row.  ANY: rows of at least four columns, of any length, pitch and address.
 template <typename T, int NV, bool WITH_DX, bool ANY>
 __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows,
                                                               int64_t cols, int64_t ld_dy, int64_t ld_x,
@@ -324,7 +348,7 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
     for (int k = 0; k < NV; ++k) {
         const int c = lane + k * kWave;
         g[k] = make_float4(1.f, 1.f, 1.f, 1.f);
-        if (gamma && c < nv) g[k] = load_piece<ANY>(gamma + 4 * c, n - 4 * c);
+        if (gamma && c < nv) g[k] = load_piece<ANY>(gamma + piece_column<ANY>(4 * c, n));
         ca[k] = cb[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     constexpr int RU = NV <= 2 ? 4 : 2;   // rows whose loads are in flight together
@@ -346,8 +370,8 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
                 const int c = lane + k * kWave;
                 d[u][k] = v[u][k] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (on && c < nv) {
-                    d[u][k] = load_piece<ANY>(dy + r * ld_dy + 4 * c, n - 4 * c);
-                    v[u][k] = load_piece<ANY>(x + r * ld_x + 4 * c, n - 4 * c);
+                    d[u][k] = load_piece<ANY>(dy + r * ld_dy + piece_column<ANY>(4 * c, n));
+                    v[u][k] = load_piece<ANY>(x + r * ld_x + piece_column<ANY>(4 * c, n));
                 }
             }
         }
@@ -359,7 +383,7 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
 #pragma unroll
             for (int k = 0; k < NV; ++k) {
                 // columns past the row hold zeros in d, so they add nothing
-                const float4 dd = d[u][k], vv = v[u][k];
+                const float4 dd = own_elements<ANY>(d[u][k], 4 * (lane + k * kWave) - piece_column<ANY>(4 * (lane + k * kWave), n)), vv = v[u][k];
                 const float h0 = (vv.x - m[u]) * rs[u], h1 = (vv.y - m[u]) * rs[u], h2 = (vv.z - m[u]) * rs[u], h3 = (vv.w - m[u]) * rs[u];
                 const float g0 = dd.x * g[k].x, g1 = dd.y * g[k].y, g2 = dd.z * g[k].z, g3 = dd.w * g[k].w;
                 s1 += (g0 + g1) + (g2 + g3);
@@ -386,7 +410,7 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
                     o.y = dx_value(dd.y, g[k].y, vv.y, m[u], rs[u], S1, S2);
                     o.z = dx_value(dd.z, g[k].z, vv.z, m[u], rs[u], S1, S2);
                     o.w = dx_value(dd.w, g[k].w, vv.w, m[u], rs[u], S1, S2);
-                    store_piece<ANY>(dxr + 4 * c, o, n - 4 * c);
+                    store_piece<ANY>(dxr + piece_column<ANY>(4 * c, n), o);
                 }
             }
         }
@@ -394,6 +418,15 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int c4 = (lane + k * kWave) * 4;
+        if (ANY && c4 + 4 > n) {
+            if (c4 >= n) continue;
+            const int from = n - 4;
+            const float a4[4] = {ca[k].x, ca[k].y, ca[k].z, ca[k].w}, b4[4] = {cb[k].x, cb[k].y, cb[k].z, cb[k].w};
+#pragma unroll
+            for (int e = 1; e < 4; ++e)
+                if (from + e >= c4) fold[0][wave][from + e] = a4[e], fold[1][wave][from + e] = b4[e];
+            continue;
+        }
         *reinterpret_cast<float4*>(&fold[0][wave][c4]) = ca[k];
         *reinterpret_cast<float4*>(&fold[1][wave][c4]) = cb[k];
     }
@@ -407,8 +440,9 @@ __global__ __launch_bounds__(kFusedBlock) void ln_bwd_partial_cols(const T* __re
     }
 }
 
-// Unaligned rows of fewer columns stay with the separate passes: [30000, 801] bf16 107 -> 71 us in one pass, [8192, 1023]
-// fp32 49 -> 27, but [2048, 333] 10.4 -> 14 and [100000, 63] bf16 68 -> 92 (few lanes have a piece, and most rows' ends).
+// Unaligned rows of fewer columns stay with the separate passes: measured with their ends fetched element by element,
+// [30000, 801] bf16 107 -> 71 us in one pass (now 47), [8192, 1023] fp32 49 -> 27 (now 19), but [2048, 333] 10.4 -> 14 and
+// [100000, 63] bf16 68 -> 92 (few lanes have a piece).
 constexpr int64_t kAnyCols = 512;
 
 template <typename T, bool WITH_DX, bool ANY>
@@ -428,43 +462,47 @@ void launch_partial_cols(const T* dy, const T* x, int64_t rows, int64_t cols, in
 
 // Rows that do not fit a wavefront's registers, or are no multiple of four
 // elements: the pass of ln_bwd_partial_cols with a workgroup per row.  Thread t
-// keeps the V-element pieces t + THREADS k, k < NV, of gamma and of the column
+// keeps the pieces of four t + THREADS k, k < NV, of gamma and of the column
 // sums in registers for all rows of its split; RU rows are loaded while the RU rows
 // before them are summed, and the only barrier per RU rows is the exchange of the
 // wavefronts' row sums (double-buffered in LDS).  Bound by HBM: dy and x are read
 // once and dx written once.  [8192, 8192] bf16 measured, row sums + column sums + dx
-// in separate passes 45 + 65 + 82 us, here together (see ddl_ln_bwd_whole_rows).
-template <typename T, int V>
-struct Piece;
-template <typename T>
-struct Piece<T, 4> {
-    typedef std::conditional_t<sizeof(T) == 4, float4, uint2> raw;
-    static __device__ void get(const raw& r, float (&f)[4]) {
-        const float4 q = load4(reinterpret_cast<const T*>(&r));
+// in separate passes 45 + 65 + 82 us, here together (see ddl_ln_bwd_whole_rows).  ANY:
+// rows of any length, pitch and address, [8000, 8191] bf16 100 us one element a lane,
+// here 81; [32000, 2045] 153 -> 102; the same in fp32 197 -> 141.
+template <typename T, bool ANY>
+struct Piece {
+    struct __attribute__((packed, aligned((ANY ? 1 : 4) * sizeof(T)))) Raw {
+        uint32_t word[sizeof(T)];   // four elements
+    };
+    static __device__ Raw fetch(const T* p) { return *reinterpret_cast<const Raw*>(p); }
+    static __device__ void get(const Raw& r, float (&f)[4]) {
+        struct __attribute__((aligned(4 * sizeof(T)))) Quad {
+            uint32_t word[sizeof(T)];
+        } w;
+#pragma unroll
+        for (int i = 0; i < static_cast<int>(sizeof(T)); ++i) w.word[i] = r.word[i];
+        const float4 q = load4(reinterpret_cast<const T*>(&w));
         f[0] = q.x, f[1] = q.y, f[2] = q.z, f[3] = q.w;
     }
-    static __device__ void put(T* p, const float (&f)[4]) { store4(p, make_float4(f[0], f[1], f[2], f[3])); }
-};
-template <typename T>
-struct Piece<T, 1> {
-    typedef T raw;
-    static __device__ void get(const raw& r, float (&f)[1]) { f[0] = load1(&r); }
-    static __device__ void put(T* p, const float (&f)[1]) { store1(p, f[0]); }
+    static __device__ void put(T* p, const float (&f)[4]) { store_piece<ANY>(p, make_float4(f[0], f[1], f[2], f[3])); }
 };
 
-template <typename T, int THREADS, int V, int NV, int RU, bool WITH_DX>
+template <typename T, int THREADS, int NV, int RU, bool WITH_DX, bool ANY>
 __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows, int64_t cols,
                                                              int64_t ld_dy, int64_t ld_x, const float* __restrict__ mean,
                                                              const float* __restrict__ rstd, const T* __restrict__ gamma,
                                                              float* __restrict__ sums, int64_t rows_per_split, float* __restrict__ partial,
                                                              float weight, T* __restrict__ dx, int64_t ld_dx) {
 #pragma clang fp contract(off)   // both instantiations round alike
-    typedef Piece<T, V> P;
-    typedef typename P::raw Raw;
+    constexpr int V = 4;
+    typedef Piece<T, ANY> P;
+    typedef typename P::Raw Raw;
     constexpr int kWaves = THREADS / kWave;
     __shared__ float2 row_sums[2][RU][kWaves];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int pieces = static_cast<int>(cols / V);
+    const int n = static_cast<int>(cols), pieces = (n + V - 1) / V;
+    auto column = [&](int c) { return piece_column<ANY>(V * c, n); };
     const int64_t r_begin = static_cast<int64_t>(blockIdx.x) * rows_per_split;
     const int64_t r_end = r_begin + rows_per_split < rows ? r_begin + rows_per_split : rows;
     Raw g[NV];
@@ -472,7 +510,7 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int c = threadIdx.x + k * THREADS;
-        if (gamma && c < pieces) g[k] = *reinterpret_cast<const Raw*>(gamma + V * c);
+        if (gamma && c < pieces) g[k] = P::fetch(gamma + column(c));
 #pragma unroll
         for (int e = 0; e < V; ++e) ca[k][e] = cb[k][e] = 0.f;
     }
@@ -485,8 +523,8 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
             for (int k = 0; k < NV; ++k) {
                 const int c = threadIdx.x + k * THREADS;
                 if (c < pieces) {
-                    d[u][k] = *reinterpret_cast<const Raw*>(dy + r * ld_dy + V * c);
-                    v[u][k] = *reinterpret_cast<const Raw*>(x + r * ld_x + V * c);
+                    d[u][k] = P::fetch(dy + r * ld_dy + column(c));
+                    v[u][k] = P::fetch(x + r * ld_x + column(c));
                 }
             }
         }
@@ -516,6 +554,11 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
                 P::get(d[u][k], dd);
                 P::get(v[u][k], vv);
                 gain(k, gg);
+                if (ANY) {
+                    const int c = threadIdx.x + k * THREADS;
+                    const float4 own = own_elements<ANY>(make_float4(dd[0], dd[1], dd[2], dd[3]), V * c - column(c));
+                    dd[0] = own.x, dd[1] = own.y, dd[2] = own.z, dd[3] = own.w;
+                }
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
                     const float h = (vv[e] - m[u]) * rs[u], t = dd[e] * gg[e];
@@ -550,7 +593,7 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
                     gain(k, gg);
 #pragma unroll
                     for (int e = 0; e < V; ++e) o[e] = dx_value(dd[e], gg[e], vv[e], m[u], rs[u], S1, S2);
-                    P::put(dx + r * ld_dx + V * c, o);
+                    P::put(dx + r * ld_dx + column(c), o);
                 }
             }
         }
@@ -569,7 +612,10 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
         const int c = threadIdx.x + k * THREADS;
         if (c >= pieces) continue;
 #pragma unroll
-        for (int e = 0; e < V; ++e) out[V * c + e] = ca[k][e], out[cols + V * c + e] = cb[k][e];
+        for (int e = 0; e < V; ++e) {
+            const int at = column(c) + e;
+            if (!ANY || at >= V * c) out[at] = ca[k][e], out[cols + at] = cb[k][e];
+        }
     }
 }
 
@@ -581,27 +627,25 @@ void launch_block_rows(bool vec, const T* dy, const T* x, int64_t rows, int64_t 
                        const float* rstd, const T* gamma, float* sums, int64_t splits, float* partial, float weight, T* dx, int64_t ld_dx,
                        hipStream_t s) {
     const int64_t rows_per_split = (rows + splits - 1) / splits;
-    auto go = [&](auto threads, auto v, auto nv, auto ru) {
+    auto go_as = [&](auto threads, auto nv, auto ru, auto any) {
         constexpr int kThreads = decltype(threads)::value;
-        hipLaunchKernelGGL((ln_bwd_block_rows<T, kThreads, decltype(v)::value, decltype(nv)::value, decltype(ru)::value, WITH_DX>),
+        hipLaunchKernelGGL((ln_bwd_block_rows<T, kThreads, decltype(nv)::value, decltype(ru)::value, WITH_DX, decltype(any)::value>),
                            dim3(static_cast<uint32_t>(splits)), dim3(kThreads), 0, s, dy, x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, sums,
                            rows_per_split, partial, weight, dx, ld_dx);
+    };
+    auto go = [&](auto threads, auto nv, auto ru) {
+        if (vec) go_as(threads, nv, ru, std::false_type{});
+        else go_as(threads, nv, ru, std::true_type{});
     };
     const std::integral_constant<int, 1> c1{};
     const std::integral_constant<int, 2> c2{};
     const std::integral_constant<int, 4> c4{};
-    const std::integral_constant<int, 8> c8{};
     const std::integral_constant<int, 512> c512{};
     const std::integral_constant<int, 1024> c1024{};
-    if (vec) {
-        if (cols <= 2048) go(c512, c4, c1, c4);
-        else if (cols <= 4096) go(c1024, c4, c1, c4);
-        else if (cols <= 8192) go(c1024, c4, c2, c2);
-        else go(c1024, c4, c4, c1);
-    } else {
-        if (cols <= 4096) go(c1024, c1, c4, c2);
-        else go(c1024, c1, c8, c1);
-    }
+    if (cols <= 2048) go(c512, c1, c4);
+    else if (cols <= 4096) go(c1024, c1, c4);
+    else if (cols <= 8192) go(c1024, c2, c2);
+    else go_as(c1024, c4, c1, std::false_type{});
 }
 
 // Can rows be read four elements at a time?  elem = bytes per element.
@@ -666,9 +710,9 @@ extern "C" int ddl_ln_bwd_partial(const void* dy, const void* x, int dtype, int6
     with_ln_element(dtype, [&](auto* tag) {
         using T = std::remove_pointer_t<decltype(tag)>;
         if (vec)
-            hipLaunchKernelGGL((ln_bwd_partial<T, true>), dim3(blocks), dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums);
-        else
             hipLaunchKernelGGL((ln_bwd_partial<T, false>), dim3(blocks), dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums);
+        else
+            hipLaunchKernelGGL((ln_bwd_partial<T, true>), dim3(blocks), dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums);
     });
     return check_launch("ln_bwd_partial");
 }
@@ -691,10 +735,10 @@ extern "C" int ddl_ln_bwd_input(const void* dy, const void* x, int dtype, int64_
     with_ln_element(dtype, [&](auto* tag) {
         using T = std::remove_pointer_t<decltype(tag)>;
         if (vec)
-            hipLaunchKernelGGL((ln_bwd_input<T, true>), dim3(blocks), dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
+            hipLaunchKernelGGL((ln_bwd_input<T, false>), dim3(blocks), dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
                                as<T>(gamma), part_sums, nparts, weight, as<T>(dx), ld_dx);
         else
-            hipLaunchKernelGGL((ln_bwd_input<T, false>), dim3(blocks), dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
+            hipLaunchKernelGGL((ln_bwd_input<T, true>), dim3(blocks), dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
                                as<T>(gamma), part_sums, nparts, weight, as<T>(dx), ld_dx);
     });
     return check_launch("ln_bwd_input");
@@ -807,11 +851,11 @@ extern "C" int ddl_ln_bwd_input_params(const void* dy, const void* x, int dtype,
     with_ln_element(dtype, [&](auto* tag) {
         using T = std::remove_pointer_t<decltype(tag)>;
         if (vec)
-            hipLaunchKernelGGL((ln_bwd_input_final<T, true>), grid, dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
+            hipLaunchKernelGGL((ln_bwd_input_final<T, false>), grid, dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
                                as<T>(gamma), part_sums, nparts, weight, as<T>(dx), ld_dx, static_cast<uint32_t>(strips), workspace,
                                static_cast<int>(splits), as<T>(dgamma), as<T>(dbeta));
         else
-            hipLaunchKernelGGL((ln_bwd_input_final<T, false>), grid, dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
+            hipLaunchKernelGGL((ln_bwd_input_final<T, true>), grid, dim3(kBlock), 0, s, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd,
                                as<T>(gamma), part_sums, nparts, weight, as<T>(dx), ld_dx, static_cast<uint32_t>(strips), workspace,
                                static_cast<int>(splits), as<T>(dgamma), as<T>(dbeta));
     });

@@ -86,49 +86,47 @@ __device__ inline void store1(float* p, float v) { *p = v; }
 __device__ inline void store1(bf16_t* p, float v) { p->bits = static_cast<uint16_t>(f32_to_bf16(v)); }
 __device__ inline void store1(__half* p, float v) { *p = __float2half_rn(v); }
 
-// Up to four elements at any address: a piece of a row whose length, pitch or
-// start is no multiple of four elements.  Whole pieces are one load or store
-// (global memory takes them at element alignment), the last n < 4 elements of a
-// row one by one; elements past n read as zeros.
-template <typename T>
-struct PieceBits {
-    typedef std::conditional_t<sizeof(T) == 4, float4, uint2> raw;
-    struct __attribute__((packed, aligned(sizeof(T)))) Any {
-        uint32_t word[sizeof(T)];   // four elements
-    };
-};
+// Two or four words, at the alignment of a 16-bit element, as a streaming store.
+__device__ inline void store_stream(void* p, uint32_t __attribute__((ext_vector_type(2))) v) {
+    typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
+    typedef u32x2_v any __attribute__((aligned(2)));
+    __builtin_nontemporal_store(v, static_cast<any*>(p));
+}
+__device__ inline void store_stream(void* p, uint32_t __attribute__((ext_vector_type(4))) v) {
+    typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
+    typedef u32x4_v any __attribute__((aligned(2)));
+    __builtin_nontemporal_store(v, static_cast<any*>(p));
+}
+
+// Four elements; ANY: at any address (global memory takes them at element alignment).
 template <bool ANY, typename T>
-__device__ inline float4 load_piece(const T* p, int n) {
-    if (!ANY) return load4(p);
-    if (n >= 4) {
-        typename PieceBits<T>::raw r;
-        const typename PieceBits<T>::Any a = *reinterpret_cast<const typename PieceBits<T>::Any*>(p);
+__device__ inline float4 load_piece(const T* p) {
+    if constexpr (ANY) {
+        struct __attribute__((packed, aligned(sizeof(T)))) Any {
+            uint32_t word[sizeof(T)];   // four elements
+        };
+        std::conditional_t<sizeof(T) == 4, float4, uint2> r;
+        const Any a = *reinterpret_cast<const Any*>(p);
         __builtin_memcpy(&r, &a, sizeof(r));
         return load4(reinterpret_cast<const T*>(&r));
+    } else {
+        return load4(p);
     }
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (n > 0) v.x = load1(p);
-    if (n > 1) v.y = load1(p + 1);
-    if (n > 2) v.z = load1(p + 2);
-    return v;
 }
 template <bool ANY, typename T>
-__device__ inline void store_piece(T* p, float4 v, int n) {
-    if (!ANY) {
+__device__ inline void store_piece(T* p, float4 v) {
+    typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
+    if constexpr (!ANY) {
         store4(p, v);
-        return;
+    } else if constexpr (sizeof(T) == 4) {
+        store_stream(p, u32x4_v{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)});
+    } else if constexpr (std::is_same_v<T, bf16_t>) {
+        store_stream(p, u32x2_v{f32x2_to_bf16(v.x, v.y), f32x2_to_bf16(v.z, v.w)});
+    } else {
+        const __half2 a = __floats2half2_rn(v.x, v.y), b = __floats2half2_rn(v.z, v.w);
+        store_stream(p, u32x2_v{*reinterpret_cast<const uint32_t*>(&a), *reinterpret_cast<const uint32_t*>(&b)});
     }
-    if (n >= 4) {
-        T e[4];
-        store1(e, v.x), store1(e + 1, v.y), store1(e + 2, v.z), store1(e + 3, v.w);
-        typename PieceBits<T>::Any a;
-        __builtin_memcpy(&a, e, sizeof(a));
-        *reinterpret_cast<typename PieceBits<T>::Any*>(p) = a;
-        return;
-    }
-    if (n > 0) store1(p, v.x);
-    if (n > 1) store1(p + 1, v.y);
-    if (n > 2) store1(p + 2, v.z);
 }
 
 // Calls fn(T{}) with the element type that `dtype` names; false for any other dtype.

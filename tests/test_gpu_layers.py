@@ -572,6 +572,54 @@ def test_layer_norm_of_long_rows_walked_by_workgroups(ops, dtype, rows, cols, pa
         assert bool(((mean[part].double() - m).abs() <= 4e-6 * 4).all()) and bool(((rstd[part].double() - r).abs() <= 4e-6 * r).all())
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 2049), (9, 2050), (70, 2055), (1030, 4093), (300, 8185), (5, 8193), (6, 16383)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shift,pad", [(0, 0), (1, 0), (3, 5)])
+def test_layer_norm_of_long_rows_at_any_address(ops, dtype, rows, cols, shift, pad):
+    """Rows that end inside a piece, at any address and pitch: y, the statistics, the backward's row sums and dx against
+    float64; nothing next to the rows is written, and infinities stay in their row."""
+    gen = torch.Generator(device="cuda").manual_seed(rows + cols)
+
+    def at(rows, cols, pad, scale, offset):
+        pool = (torch.randn(rows * (cols + pad) + shift + 8, generator=gen, device="cuda") * scale + offset).to(dtype)
+        return pool[shift:shift + rows * (cols + pad)].view(rows, cols + pad)[:, :cols]
+
+    x, dy = at(rows, cols, pad, 2, 0.5), at(rows, cols, pad, 1, 0)
+    gamma, beta = at(1, cols, 0, 0.1, 1)[0], at(1, cols, 0, 0.1, 0)[0]
+    bad = rows - 1
+    keep = torch.ones(rows, dtype=torch.bool, device="cuda")
+    if rows > 1:
+        x[bad, cols - 1] = float("inf")
+        keep[bad] = False
+    y, mean, rstd = ops.layer_norm(x, gamma, beta, 1e-3, want_stats=True)
+    stats = ops.ln_partial_stats(x)
+    two = ops.ln_normalize_affine(x, torch.stack([stats, stats]), [cols, cols], gamma, beta, 1e-3)
+    sums = ops.ln_backward_partial(dy, x, mean, rstd, gamma)
+    dx = ops.ln_backward_input(dy, x, mean, rstd, gamma, torch.stack([sums, sums]), 0.5 / cols)
+    ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for part in keep.nonzero().flatten().split(512):
+        x64, d64 = x[part].double(), dy[part].double()
+        m = x64.mean(1, keepdim=True)
+        r = ((x64 - m).square().mean(1, keepdim=True) + 1e-3).rsqrt()
+        h = (x64 - m) * r
+        want = h * gamma.double() + beta.double()
+        # one rounding of the result and a few units of fp32 sums (values up to 12, |x| rstd up to 6)
+        assert bool(((y[part].double() - want).abs() <= ulp * want.abs() + 4e-6 * 8).all())
+        assert bool(((two[part].double() - want).abs() <= ulp * want.abs() + 4e-6 * 8).all())
+        assert bool(((mean[part].double() - m[:, 0]).abs() <= 4e-6 * 4).all()) and bool(((rstd[part].double() - r[:, 0]).abs() <= 4e-6 * r[:, 0]).all())
+        g = d64 * gamma.double()
+        s1, s2 = g.sum(1, keepdim=True), (g * h).sum(1, keepdim=True)
+        # fp32 sums of cols terms in 64 lanes of fours: a chain of cols / 256 additions and ten more, of |g| and |g h|
+        unit = 2.0 ** -24 * (cols / 256 + 10)
+        assert bool(((sums[part, :1].double() - s1).abs() <= unit * g.abs().sum(1, keepdim=True)).all())
+        assert bool(((sums[part, 1:].double() - s2).abs() <= (unit + 8e-6) * (g.abs() * (h.abs() + 1)).sum(1, keepdim=True)).all())
+        want = r * (g - (s1 + h * s2) / cols)
+        assert bool(((dx[part].double() - want).abs() <= ulp * want.abs() + 4e-6 * (g.abs() * r + 1)).all())
+    if rows > 1:
+        assert bool(y[bad].isnan().any()) and bool(dx[bad].isnan().any())
+        assert not bool(y[keep].isnan().any()) and not bool(dx[keep].isnan().any())
+
+
 @pytest.mark.parametrize("rows,cols,pad", [(1, 1028, 0), (5, 1025, 0), (37, 2048, 4), (3, 2052, 0), (66, 4096, 1), (1029, 4097, 0),
                                            (9, 8192, 0), (7, 8191, 0), (6, 8196, 0), (10, 16384, 8), (8200, 1032, 0),
                                            (1, 513, 0), (70, 514, 3), (65, 1023, 0), (300, 768, 1)])
