@@ -11,11 +11,11 @@
 //                registers between the two halves, so x is read once
 //
 // Three ways of holding a row, chosen by its length:
-//   wavefront rows  up to 1024 columns, 2048 of aligned fp32: one wavefront owns a row, each lane
+//   wavefront rows  up to 2048 columns (1024 unaligned, 256 in 16-bit types): one wavefront owns a row, each lane
 //                   holds pieces of four elements, sums go through shuffle
 //                   butterflies; a long input keeps two rows per wavefront in
 //                   flight
-//   workgroup rows  up to 16384 columns: a workgroup of 256 to 1024 threads owns
+//   workgroup rows  up to 16384 columns: a workgroup of 64 to 1024 threads owns
 //                   a row, still in registers, sums go through the wavefronts
 //                   and a word of LDS for each; it walks up to eight rows
 //   streamed rows   anything longer, and more rows than one launch has wavefronts for: a
@@ -33,10 +33,11 @@ constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxParts = 256;
-// The longest row a wavefront keeps in registers: of aligned fp32, and of anything else, whose pieces of four are half as
-// wide or cross lines.  By a wavefront and by a workgroup: [32000, 2048] fp32 89 and 95 us, [45000, 1200] 73 and 76; but
-// bf16 62 and 42, 59 and 42; [32000, 2045] bf16 115 and 53, fp32 96 and 99; [45000, 1201] bf16 125 and 44, fp32 88 and 79.
-constexpr int kWaveRowCols = 2048, kNarrowRowCols = 1024;
+// The longest row that ln_wave_rows takes: of aligned fp32, of unaligned fp32, and in 16-bit types, whose pieces of four are
+// half as wide.  ln_wave_rows and ln_group_rows: [32000, 2048] fp32 89 and 95 us, [45000, 1200] 73 and 76; unaligned
+// [45000, 1201] 88 and 79, [32000, 2045] 96 and 99; bf16 [32000, 2048] 62 and 42, [32768, 1024] 24.0 and 20.8, [65536, 512]
+// 25.6 and 21.8, [1000, 1024] 3.8 and 3.6; unaligned [32000, 2045] 115 and 53, [30000, 801] 28 and 20.3, [60000, 301] 27 and 18.6.
+constexpr int kWaveRowCols = 2048, kWaveRowColsAny = 1024, kWaveRowCols16 = 256;
 constexpr int kBlockRowCols = 16384;   // longest row a workgroup keeps in registers
 
 struct PartCounts {
@@ -157,8 +158,8 @@ __global__ __launch_bounds__(kBlock) void ln_wave_rows(const void* x_first, int6
     const int64_t rows = a.rows;
     const int nv = (a.cols + 3) >> 2;
     // The last piece of a row ends with it: its first elements are the end of the piece before, are left out of the sums and
-    // written twice.  (Fetched element by element instead, the branch kept the other loads from being in flight: [30000, 801]
-    // bf16 41 us, here 28; [8192, 1023] fp32 15.1, here 11.9.)
+    // written twice.  (Fetched element by element instead, the branch kept the other loads from being in flight: [8192, 1023]
+    // fp32 15.1 us, here 11.9.)
     auto column = [&](int c) { return ANY && c == nv - 1 ? a.cols - 4 : 4 * c; };
     auto again = [&](int c) { return ANY && c == nv - 1 ? 4 * nv - a.cols : 0; };
     float4 g[NV], b[NV];
@@ -506,7 +507,9 @@ void launch_group(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
 template <typename T, int MODE, bool AFFINE, bool ANY, int V>
 void launch_group_pieces(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     const int pieces = (a.cols + V - 1) / V;   // up to 16384 / V
-    if (pieces <= 512) launch_group<T, MODE, AFFINE, ANY, V, 256, 2>(a, pc, s);
+    if (sizeof(T) == 2 && pieces <= 64) launch_group<T, MODE, AFFINE, ANY, V, 64, 1>(a, pc, s);
+    else if (sizeof(T) == 2 && pieces <= 128) launch_group<T, MODE, AFFINE, ANY, V, 64, 2>(a, pc, s);
+    else if (pieces <= 512) launch_group<T, MODE, AFFINE, ANY, V, 256, 2>(a, pc, s);
     else if (pieces <= 1024) launch_group<T, MODE, AFFINE, ANY, V, 256, 4>(a, pc, s);
     else if (pieces <= 2048) launch_group<T, MODE, AFFINE, ANY, V, 512, 4>(a, pc, s);
     else launch_group<T, MODE, AFFINE, ANY, V, 1024, 4>(a, pc, s);
@@ -516,11 +519,13 @@ void launch_group_pieces(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
 template <typename T, int MODE, bool AFFINE, bool ANY>
 int launch_held(const LnArgs& a, const PartCounts& pc, hipStream_t s) {
     const int cols = a.cols;
-    if (cols <= (sizeof(T) == 4 && !ANY ? kWaveRowCols : kNarrowRowCols)) {
+    if (cols <= (sizeof(T) == 2 ? kWaveRowCols16 : ANY ? kWaveRowColsAny : kWaveRowCols)) {
         if (cols <= 256) launch_wave<T, MODE, AFFINE, ANY, 1>(a, pc, s);
-        else if (cols <= 512) launch_wave<T, MODE, AFFINE, ANY, 2>(a, pc, s);
-        else if (cols <= 1024) launch_wave<T, MODE, AFFINE, ANY, 4>(a, pc, s);
-        else launch_wave<T, MODE, AFFINE, ANY, 8>(a, pc, s);
+        if constexpr (sizeof(T) == 4) {
+            if (cols > 1024) launch_wave<T, MODE, AFFINE, ANY, 8>(a, pc, s);
+            else if (cols > 512) launch_wave<T, MODE, AFFINE, ANY, 4>(a, pc, s);
+            else if (cols > 256) launch_wave<T, MODE, AFFINE, ANY, 2>(a, pc, s);
+        }
         return check_launch("ln_wave_rows");
     }
     constexpr int kWide = 16 / static_cast<int>(sizeof(T));

@@ -572,7 +572,8 @@ def test_layer_norm_of_long_rows_walked_by_workgroups(ops, dtype, rows, cols, pa
         assert bool(((mean[part].double() - m).abs() <= 4e-6 * 4).all()) and bool(((rstd[part].double() - r).abs() <= 4e-6 * r).all())
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 2049), (9, 2050), (70, 2055), (1030, 4093), (300, 8185), (5, 8193), (6, 16383)])
+@pytest.mark.parametrize("rows,cols", [(3, 256), (1, 257), (70, 511), (33, 512), (65, 516), (9, 1023), (40, 1024), (5, 1025), (1, 2049),
+                                       (9, 2050), (70, 2055), (1030, 4093), (300, 8185), (5, 8193), (6, 16383)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shift,pad", [(0, 0), (1, 0), (3, 5)])
 def test_layer_norm_of_long_rows_at_any_address(ops, dtype, rows, cols, shift, pad):
