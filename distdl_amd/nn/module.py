@@ -1,6 +1,6 @@
 """Base class of every layer (reference: nn/module.py:6-112): binds the backend
-selected at construction time and re-runs the layer's setup ahead of a call
-whenever the structure of the input changes."""
+selected at construction time and re-runs the layer's setup from a forward
+pre-hook whenever the structure of the input changes."""
 
 import torch
 
@@ -14,12 +14,7 @@ class Module(torch.nn.Module):
         super().__init__()
         self._distdl_backend = backends.backend
         self._distdl_is_setup = False
-
-    def __call__(self, *args, **kwargs):
-        # In front of torch's call and not registered with it: a module with a hook of its own goes torch's long way on
-        # every call, and layers are made of layers.
-        self._distdl_forward_pre_hook(self, args)
-        return super().__call__(*args, **kwargs)
+        self.register_forward_pre_hook(self._distdl_forward_pre_hook)
 
     @staticmethod
     def _distdl_forward_pre_hook(self, input):

@@ -392,6 +392,41 @@ def test_setup_reruns_when_input_structure_changes():
     assert [int(v) for v in layer.output_tensor_structure.shape] == [3, 8]
 
 
+class _ExchangeSetup(HaloExchange):
+    """The exchange without its launches."""
+
+    def forward(self, input):
+        return input
+
+
+@pytest.mark.parametrize("where", ["prepended", "global", "added"])
+@pytest.mark.parametrize("change", ["pad", "cast"])
+def test_setup_sees_the_input_of_the_pre_hooks_in_front_of_it(where, change):
+    """A layer's set-up is the first forward pre-hook registered with the module: torch runs global pre-hooks and prepended
+    ones ahead of it, so it works on what they return; hooks added after it come after it."""
+    def hook(module, args):
+        x, = args
+        return torch.nn.functional.pad(x, (1, 1, 1, 1)) if change == "pad" else x.to(torch.bfloat16)
+
+    P = SimWorld(4, device=torch.device("cpu")).partition(0).create_partition_inclusive(range(4)).create_cartesian_topology_partition([2, 2])
+    width = np.array([[0, 1], [0, 1]])
+    layer = _ExchangeSetup(P, width, width, width, buffer_manager=BufferManager(device=torch.device("cpu")))
+    if where == "global":
+        handle = torch.nn.modules.module.register_module_forward_pre_hook(hook)
+    else:
+        handle = layer.register_forward_pre_hook(hook, prepend=where == "prepended")
+    try:
+        out = layer(torch.zeros(8, 8))
+        again = layer(torch.zeros(12, 8))
+    finally:
+        handle.remove()
+    assert (tuple(out.shape), tuple(again.shape), out.dtype) == \
+        (((10, 10), (14, 10), torch.float32) if change == "pad" else ((8, 8), (12, 8), torch.bfloat16))
+    seen = torch.zeros(12, 8) if where == "added" else again
+    assert [layer.slices[d][3][d] for d in range(2)] == [slice(n - 1, n, None) for n in seen.shape]
+    assert layer.buffers[0][3].dtype == seen.dtype
+
+
 # ------------------------------------------------------------ buffers --------
 
 def test_expandable_buffer_views_and_growth():
