@@ -2,24 +2,33 @@
 // y[M,N] = a[M,K] . b[N,K]^T + bias[N], fp32 in and out.
 //
 // An fp32 value is the sum of three bf16 values, exactly: its rounding to bf16, the
-// rounding of what is left, and what is left then (8 + 8 + 8 significant bits).  Of the
-// nine products of two such sums the three smallest are below 2^-25 of the product and
-// are left out; the other six go through v_mfma_f32_32x32x16_bf16, which accumulates in
-// fp32.  That is 192 cycles for 32 x 32 x 16 where v_mfma_f32_32x32x2_f32 takes 512, and
-// the sums are rounded once for 16 products instead of once for two: over sizes of 64 to
-// 8192 and all layouts the error against float64 is 0.85 of the fp32 instruction's for
-// sums of the same length (K 6575 1.3e-6 and 1.5e-6).
+// rounding of what is left, and what is left then (8 + 8 + 8 significant bits), as
+// published by Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", 2019).  Of the nine products of two such sums the smallest is
+// below 2^-33 of the product and left out; the other eight go through
+// v_mfma_f32_32x32x16_bf16, which accumulates in fp32: 256 cycles for 32 x 32 x 16 where
+// v_mfma_f32_32x32x2_f32 takes 512.
 //
-// Bound by issue: while a CU's four wavefronts multiply, they split (six instructions
-// an element) and read six fragments per four products; matrix instructions fill half
-// of the cycles, 190 to 197 TFLOP/s at most where the fp32 instruction ends at 148.
-// Measured, fp32 instruction (64 x 64 or 256 x 256 tiles) -> here: M 256, N 3551, K 6575 125 ->
-// 94 us, M 3551, N 6575, K 256 185 -> 98, M = N = K = 2048 137 -> 93, 4096 975 -> 755, M 1024,
-// N 8192, K 8192 1827 -> 701; below about 20 us the smaller tiles are faster.
+// The products of the first parts have an accumulator of their own; they are rounded
+// once per 16 terms, and a term that is zero rounds nothing.  The seven others, together
+// below 2^-7 of them, have a second one, added once at the end.  (All in one accumulator
+// round once per part-product at its full size: 0.5 to 1.5 times the fp32 instruction's
+// error, the more the fewer terms are not zero.  With the six largest products alone a
+// sum of one term is 1.025 times as far off.)  Error against float64 in the 2-norm,
+// fp32 instruction -> here, M = N = 1408, K 8192, share of x that is not zero: all 1.62e-6 -> 0.40e-6, a quarter
+// 0.81e-6 -> 0.23e-6, a hundredth 0.164e-6 -> 0.055e-6, one element a row 0.0253e-6 both.
+//
+// Bound by the matrix instructions' power and, in small products, by issue: while a CU's
+// wavefronts multiply, they split (seven instructions an element).  158 to 160 TFLOP/s
+// at most where the fp32 instruction ends at 148.  Measured, fp32 instruction (64 x 64 or
+// 256 x 256 tiles) -> here, operands along k or along their rows: M 256, N 3551, K 6575
+// 116 -> 101 to 106 us, M 3551, N 6575, K 256 147 to 169 -> 99 to 105, M = N = K = 2048 140 -> 122
+// to 128, 4096 968 -> 858 to 897, M 1024, N 8192, K 8192 1050 to 1075 -> 861 to 903; below about 20 us
+// the smaller tiles are faster.
 //
 //   workgroup  256 threads = 4 wavefronts (2 x 2), tile 128 x 128 x 16(k); a wavefront
 //              has 2 x 2 blocks of 32 x 32
-//   global     a thread fetches eight k of a row of each operand into registers, four
+//   global     a thread fetches eight k of a row of each operand into registers, three
 //              k-tiles ahead: 32 bytes of the row, or eight rows' worth of dwords for
 //              an operand contiguous along its rows.  Any pitch, length and
 //              4-byte-aligned address
@@ -48,7 +57,8 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBlock = 256;
 constexpr int kTile = 128, BK = 16;
-constexpr int kAhead = 4;               // k-tiles in flight from memory
+constexpr int kAhead = 3;               // k-tiles in flight from memory
+constexpr int kTurns = 2 * kAhead;      // k-tiles until both the registers and the two stages of LDS come round
 constexpr int kRowSpan = 2 * BK;        // bytes of a row in a plane
 constexpr int kPlane = kTile * kRowSpan, kOperand = 3 * kPlane, kStage = 2 * kOperand;   // a stage: the w planes, then the x planes
 constexpr int kOutPitch = 68;           // floats of a row of results in LDS: 64 and room for 16 rows on 64 banks
@@ -143,14 +153,14 @@ __global__ __launch_bounds__(kBlock, 2) void gemm32_split(const Part32 p, int sp
     const int64_t ktiles = (K + BK - 1) / BK, per = (ktiles + splits - 1) / splits;
     const int64_t t_begin = split * per < ktiles ? split * per : ktiles, t_end = t_begin + per < ktiles ? t_begin + per : ktiles;
 
-    floatx16 acc[2][2];   // [n block][m block]
+    floatx16 acc[2][2], rest[2][2];   // [n block][m block]: the products of the first parts, and all others
     auto clear = [&]() {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = rest[i][j][e] = 0.f;
     };
     clear();
     Fetch<WT> fw;
@@ -164,29 +174,37 @@ __global__ __launch_bounds__(kBlock, 2) void gemm32_split(const Part32 p, int sp
     };
     auto multiply = [&](const char* at, auto&& between) {
         bf16x8 a[3][2], b[3][2];
-#pragma unroll
-        for (int s = 0; s < 3; ++s)
+        auto read = [&](int s) {
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 a[s][i] = fragment(at, s, sub_w + i);
                 b[s][i] = fragment(at + kOperand, s, sub_x + i);
             }
-        between();
-        auto term = [&](int sw, int sx) {
+        };
+        auto term = [&](floatx16 (&to)[2][2], int sw, int sx) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[sw][i], b[sx][j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) to[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[sw][i], b[sx][j], to[i][j], 0, 0, 0);
         };
-        term(2, 0), term(0, 2), term(1, 1), term(1, 0), term(0, 1), term(0, 0);   // small terms first
-        // Splitting and storing the next k-tile goes into the shadow of the matrix instructions, five at a time: left alone,
-        // the compiler puts all of it in front of them (2048 x 2048 x 2048 107 us instead of 93).
-        __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);      // LDS reads
+        // Splitting and storing the next k-tile goes into the shadow of the matrix instructions, six at a time: left alone,
+        // the compiler puts all of it in front of them (six part-products: 2048 x 2048 x 2048 107 us instead of 93).
+        auto alternate = [](auto reads, auto products) {
+            __builtin_amdgcn_sched_group_barrier(0x100, decltype(reads)::value, 0);    // LDS reads
 #pragma unroll
-        for (int i = 0; i < 24; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a matrix instruction
-            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);   // others of the vector ALU
-        }
+            for (int i = 0; i < decltype(products)::value; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a matrix instruction
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);   // others of the vector ALU
+            }
+        };
+        // The third parts are read when twelve products are under way: all at once they would not fit the registers.
+        read(0), read(1);
+        between();
+        term(acc, 0, 0), term(rest, 1, 1), term(rest, 1, 0), term(rest, 0, 1);
+        read(2);
+        term(rest, 2, 1), term(rest, 1, 2), term(rest, 2, 0), term(rest, 0, 2);
+        alternate(std::integral_constant<int, 8>{}, std::integral_constant<int, 12>{});
+        alternate(std::integral_constant<int, 4>{}, std::integral_constant<int, 20>{});
     };
     if (t_begin < full) {
         // The loads are never skipped (past the last whole k-tile that one is loaded again): with a branch around them the
@@ -207,14 +225,13 @@ __global__ __launch_bounds__(kBlock, 2) void gemm32_split(const Part32 p, int sp
         int64_t t = t_begin;
         while (true) {
 #pragma unroll
-            for (int i = 0; i < kAhead; ++i) {
+            for (int i = 0; i < kTurns; ++i) {
                 // This wavefront's part of k-tile t is in LDS and its reads of the other stage have returned; the loads stay in flight.
                 asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
                 multiply(lds + (i & 1) * kStage, [&]() {
-                    constexpr int kRing = kAhead - 1;
-                    fw.store(vw[(i + 1) & kRing], lds + ((i + 1) & 1) * kStage);
-                    fx.store(vx[(i + 1) & kRing], lds + ((i + 1) & 1) * kStage + kOperand);
-                    load((i + 1) & kRing);
+                    fw.store(vw[(i + 1) % kAhead], lds + ((i + 1) & 1) * kStage);
+                    fx.store(vx[(i + 1) % kAhead], lds + ((i + 1) & 1) * kStage + kOperand);
+                    load((i + 1) % kAhead);
                 });
                 if (++t == full) break;
             }
@@ -275,6 +292,15 @@ __global__ __launch_bounds__(kBlock, 2) void gemm32_split(const Part32 p, int sp
         }
     }
 
+    else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = acc[i][j][e] + rest[i][j][e];
+    }
+
     // Lane holds row m = l32 and columns n = 8 g + 4 kh + {0..3} of a block in acc[4 g + {0..3}].
     auto quad = [&](int i, int j, int g) { return floatx4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]}; };
     if (splits > 1) {   // block (m, n) of the tile is number m + 4 n, as gemm32_small_sum counts them
@@ -333,23 +359,23 @@ int launch(Part32 part, int splits, float* partial, hipStream_t s) {
 
 }  // namespace
 
-// The estimates are fits to a sweep over M, N, K of 5 .. 8192 on all operand layouts, in microseconds: 3 + for each tile that a
-// CU has to work through 2.5 and, per 32 of its reduction, 1.1 (few CUs at work) to 1.37 (all) + for splits a second launch (2.3,
-// and 5 for what it and the workspace cost the host) and the partial tiles at 5 TB/s.
+// The estimates are fits to a sweep over M, N, K of 64 .. 8192 on all operand layouts, in microseconds: 6 + for each tile that a
+// CU has to work through 4.5 and, per 32 of its reduction, 1.57 (few CUs at work) to 1.72 (all) + for splits a second launch (2.3,
+// and 5 for what it and the workspace cost the host) and the partial tiles at 5 TB/s.  Over 66 sizes in three layouts the way they
+// choose is on average 1.1 % slower than the faster of both kernels and all splits.
 Small32 plan_split32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, const Small32& other) {
     Small32 best;
     const int64_t ktiles = (K + BK - 1) / BK, tiles = ((M + kTile - 1) / kTile) * ((N + kTile - 1) / kTile);
-    // A launch has fewer than 2^32 threads, 256 per tile.  Sums of one or two terms, which the fp32 instruction rounds correctly,
-    // are 1.1 to 1.4 times as far off here (from three terms on 0.9 and less).
-    if (tiles > 0xFFFFFF || K < 3) return best;
+    if (tiles > 0xFFFFFF) return best;   // a launch has fewer than 2^32 threads, 256 per tile
     double best_us = other.groups ? other.us : 1e30;
     for (const int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
         if (splits > 1 && (tiles * splits > 4 * static_cast<int64_t>(cus) || ktiles < 8 * splits || tiles * splits * kTile * kTile > workspace)) break;
-        // Fewer, longer sums than the other way are only taken where this kernel's smaller rounding error makes up for it.
-        if (4 * splits < 3 * other.groups * other.splits) continue;
+        // Fewer, longer sums than the other way are only taken where this kernel's smaller rounding error makes up for it (0.24 to
+        // 0.34 of the other's for dense sums of the same length; it grows by their square root).
+        if (4 * splits < other.groups * other.splits) continue;
         const int64_t all = tiles * splits, per_cu = (all + cus - 1) / cus, kt = (ktiles + splits - 1) / splits;
         const double fill = all < cus ? static_cast<double>(all) / cus : 1.0;
-        double us = 3 + per_cu * (2.5 + 0.5 * static_cast<double>(kt) * (1.1 + 0.27 * fill));
+        double us = 6 + per_cu * (4.5 + 0.5 * static_cast<double>(kt) * (1.57 + 0.15 * fill));
         if (splits > 1) us += 7.3 + static_cast<double>(all) * kTile * kTile * 8 / 5e6;
         if (us >= best_us) continue;
         best_us = best.us = us;

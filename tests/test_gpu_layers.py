@@ -6,6 +6,8 @@ relative, Linear bf16 within 2e-2 relative, Embedding bit-exact.  "Relative" is
 taken with respect to the magnitude of the exact (fp64 oracle) result, with an
 absolute floor of the same size because normalised outputs cross zero."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -1949,7 +1951,7 @@ def test_gemm_f32_tiled_kernel_reads_every_operand_layout(ops, a_t, b_t, M, N, K
     # enough work for the 256 x 256 tiles, wide and narrow ones
     (4096, 4352, 1540, 4, False)])
 def test_gemm_f32_products_of_every_size_and_pitch(ops, a_t, b_t, M, N, K, pad, splits):
-    """Integer operands (every sum is exact in fp32) at the sizes where the small fp32 tiles can go wrong, with and
+    """Integer operands (every sum is exact in fp32) at the sizes where the fp32 tiles can go wrong, with and
     without the workspace that lets them split the reduction, on buffers that end where the operands end."""
     from distdl_amd import _lib
     gen = torch.Generator().manual_seed(M + 3 * N + K + 2 * a_t + b_t)
@@ -1974,14 +1976,35 @@ def test_gemm_f32_products_of_every_size_and_pitch(ops, a_t, b_t, M, N, K, pad, 
         assert (got[:, N:] == 77.0).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(1300, 1411, 3), (1281, 1408, 15), (1280, 1409, 16), (1300, 1411, 17), (1279, 1410, 33), (1300, 1411, 79), (129, 1411, 4099),
-                                   (2049, 130, 1000), (128, 128, 8200)])
+class _Plan32(ctypes.Structure):
+    _fields_ = [("groups", ctypes.c_int), ("edge", ctypes.c_int), ("us", ctypes.c_double), ("splits", ctypes.c_int), ("workspace", ctypes.c_int64)]
+
+
+def _plan32(M, N, K, a_t=False, b_t=False):
+    """What the library's dispatch (ddl::plan32) takes for an fp32 product of operands end to end on this GPU: `edge` 128 for
+    the tiles of bf16 parts, else `groups` for the small ones."""
+    from distdl_amd import _lib
+    plan = _lib.load()._ZN3ddl6plan32Elllllllil
+    plan.restype, plan.argtypes = _Plan32, [ctypes.c_int64] * 7 + [ctypes.c_int, ctypes.c_int64]
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return plan(*((1, M) if a_t else (K, 1)), *((1, N) if b_t else (K, 1)), M, N, K, cus, 2 ** 62)
+
+
+@pytest.mark.parametrize("M,N,K,splits", [
+    # small tiles
+    (1300, 1411, 3, 0), (1281, 1408, 15, 0), (1280, 1409, 16, 0), (1300, 1411, 17, 0), (1279, 1410, 33, 0), (1300, 1411, 79, 0), (129, 1411, 4099, 0),
+    (2049, 130, 1000, 0), (128, 128, 8200, 0),
+    # 128 x 128 tiles of bf16 parts
+    (3300, 3411, 3, 1), (3281, 3408, 15, 1), (3280, 3409, 16, 1), (3300, 3411, 17, 1), (3279, 3410, 33, 1), (3300, 3411, 79, 1), (3300, 3411, 100, 1),
+    (257, 3411, 4099, 3), (2049, 513, 2000, 3), (640, 640, 8200, 8)])
 @pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
-def test_gemm_f32_by_exact_bf16_parts(ops, a_t, b_t, M, N, K):
+def test_gemm_f32_by_exact_bf16_parts(ops, a_t, b_t, M, N, K, splits):
     """Products large enough for 128 x 128 tiles on the bf16 matrix cores: partial tiles, every remainder of the k-tiles, the
-    reduction in one piece and split, rows of odd length that start anywhere, operands as they lie.  The error against float64
-    is that of fp32 sums (K/16 additions of six parts, each rounded once), and no larger than the fp32 matrix instruction's
+    reduction in one piece and split, rows of odd length that start anywhere, operands as they lie; and products next to them
+    that small tiles take.  The error against float64 is that of fp32 sums, and no larger than the fp32 matrix instruction's
     was (1.5e-6 for the longest of these sums, in the 2-norm)."""
+    plan = _plan32(M, N, K, a_t, b_t)
+    assert (plan.edge, plan.splits if plan.edge else 0) == ((128, splits) if splits else (0, 0))
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
 
     def operand(rows, transposed):
@@ -2001,12 +2024,12 @@ def test_gemm_f32_by_exact_bf16_parts(ops, a_t, b_t, M, N, K):
     assert bool(((out.double() - want).abs() <= (K + 2) * 2.0 ** -24 * (a64.abs() @ b64.abs().t() + bias.double().abs())).all())
 
 
-@pytest.mark.parametrize("K", [48, 1000])
-def test_gemm_f32_of_values_that_bf16_parts_cannot_carry(ops, K):
+@pytest.mark.parametrize("M,N,K,edge", [(1400, 1400, 48, 0), (1400, 1400, 1000, 0), (3300, 3300, 48, 128), (3300, 3300, 1000, 128)])
+def test_gemm_f32_of_values_that_bf16_parts_cannot_carry(ops, M, N, K, edge):
     """Infinities, NaN, values next to the largest float and large ones, rows so small that their parts would be denormal, and zeros: the
     products are those of fp32 arithmetic, and tiles without such values are not touched by the others."""
+    assert _plan32(M, N, K).edge == edge
     gen = torch.Generator(device="cuda").manual_seed(K)
-    M = N = 1400
     x, w = torch.randn(M, K, generator=gen, device="cuda"), torch.randn(N, K, generator=gen, device="cuda")
     plain = ops.linear(x, w)
     x[5, 3], x[6, 4], x[140, 7] = float("inf"), float("-inf"), float("nan")
@@ -2029,8 +2052,42 @@ def test_gemm_f32_of_values_that_bf16_parts_cannot_carry(ops, K):
     untouched = torch.ones(M, dtype=torch.bool)
     untouched[:256] = untouched[256:384] = untouched[512:640] = False     # the tiles' rows
     columns = torch.ones(N, dtype=torch.bool)
-    columns[:128] = columns[896:1024] = columns[1280:] = False
+    columns[:128] = columns[896:1024] = columns[1280:1408] = False
     assert torch.equal(got[untouched][:, columns], plain.cpu()[untouched][:, columns])
+
+
+def _sums_of_fp32(x, w):
+    """x w^T with one rounding to fp32 per term, in the order of k."""
+    out = torch.zeros(x.shape[0], w.shape[0], device="cuda")
+    for k in range(x.shape[1]):
+        out = (out.double() + x[:, k, None].double() * w[None, :, k].double()).float()
+    return out
+
+
+@pytest.mark.parametrize("density", [1.0, 0.25, 0.1, 0.01, 0])
+@pytest.mark.parametrize("M,N,K,a_t,b_t,edge", [(3300, 3411, 100, False, False, 128), (3300, 3411, 100, True, True, 128), (640, 640, 8200, False, True, 128)])
+def test_gemm_f32_error_of_sparse_operands(ops, M, N, K, a_t, b_t, edge, density):
+    """Sums of few terms that are not zero: adding zeros rounds nothing in fp32 arithmetic, so the error against float64 is to
+    stay below that of one rounding to fp32 per term.  With one such term in a row (density 0) the result is its product,
+    rounded once; on bf16 parts the sum of the smaller parts is rounded eight times besides, at less than 2^-7 of the result,
+    which moves that rounding by 2^-4 of its unit at most."""
+    assert _plan32(M, N, K, a_t, b_t).edge == edge
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    x, w = torch.randn(M, K, generator=gen, device="cuda"), torch.randn(N, K, generator=gen, device="cuda")
+    if density == 0:
+        x *= torch.nn.functional.one_hot(torch.randint(0, K, (M,), generator=gen, device="cuda"), K)
+    else:
+        x *= torch.rand(M, K, generator=gen, device="cuda") < density
+    a, sa = (x.t().contiguous(), (1, M)) if a_t else (x, (K, 1))
+    b, sb = (w.t().contiguous(), (1, N)) if b_t else (w, (K, 1))
+    out = torch.empty(M, N, device="cuda")
+    ops._gemm(a, *sa, b, *sb, None, out, ops._LINEAR_DTYPES[torch.float32], M, N, K)
+    want = x.double() @ w.double().t()
+    error = out.double() - want
+    if density == 0:
+        assert bool((error.abs() <= (1 + 2.0 ** -4) * 2.0 ** -24 * want.abs()).all())
+    else:
+        assert float(error.norm()) <= float((_sums_of_fp32(x, w).double() - want).norm())
 
 
 def test_gemm_f32_tiled_kernel_random_and_odd_depth(ops):
