@@ -4,7 +4,9 @@
 // An fp32 value is the sum of three bf16 values, exactly: its rounding to bf16, the
 // rounding of what is left, and what is left then (8 + 8 + 8 significant bits), as
 // published by Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial
-// Intelligence Datatype For Higher-Precision Computations", 2019).  Of the nine products of two such sums the smallest is
+// Intelligence Datatype For Higher-Precision Computations", 2019).  Elements are
+// multiplied by 2^24 first: then no part of any of them, denormal ones included, is
+// below bf16's normal range.  Of the nine products of two such sums the smallest is
 // below 2^-33 of the product and left out; the other eight go through
 // v_mfma_f32_32x32x16_bf16, which accumulates in fp32: 256 cycles for 32 x 32 x 16 where
 // v_mfma_f32_32x32x2_f32 takes 512.
@@ -39,10 +41,11 @@
 //   splits     workgroups share the reduction of a tile through a workspace, whose
 //              sums gemm32_small_sum adds
 //
-// What the split cannot carry is found on the way: every thread keeps the largest
-// magnitude of the rows it fetches.  Tiles with infinities, magnitudes whose product
-// comes near the largest float, or a row that is all below 2^-96 (whose smallest part
-// would be denormal) are computed again from memory on v_mfma_f32_32x32x2_f32.
+// What the parts cannot carry is found on the way: every thread keeps the largest
+// magnitude that it fetches.  Tiles with infinities, elements from 2^100 on, or
+// elements whose product times the length of the reduction reaches 2^78 (which scaled
+// might pass the largest float) are computed again from memory on
+// v_mfma_f32_32x32x2_f32.
 #include "gemm32_small.h"
 #include "gemm_tiles.h"
 #include <type_traits>
@@ -62,7 +65,8 @@ constexpr int kTurns = 2 * kAhead;      // k-tiles until both the registers and 
 constexpr int kRowSpan = 2 * BK;        // bytes of a row in a plane
 constexpr int kPlane = kTile * kRowSpan, kOperand = 3 * kPlane, kStage = 2 * kOperand;   // a stage: the w planes, then the x planes
 constexpr int kOutPitch = 68;           // floats of a row of results in LDS: 64 and room for 16 rows on 64 banks
-constexpr float kTiny = 0x1p-96f, kHuge = 0x1p120f;
+constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;   // of an element before it is split, of a result
+constexpr float kHuge = 0x1p100f, kMost = 0x1p78f;       // what elements and sums may reach, unscaled
 
 typedef PartOf<float> Part32;
 
@@ -126,7 +130,7 @@ struct Fetch {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             most = fmaxf(fmaxf(most, fabsf(v[2 * e])), fabsf(v[2 * e + 1]));
-            split2(v[2 * e], v[2 * e + 1], w[0][e], w[1][e], w[2][e]);
+            split2(v[2 * e] * kScale, v[2 * e + 1] * kScale, w[0][e], w[1][e], w[2][e]);
         }
         char* at = planes + chunk_at(row, octet);
 #pragma unroll
@@ -252,23 +256,15 @@ __global__ __launch_bounds__(kBlock, 2) void gemm32_split(const Part32 p, int sp
         __syncthreads();
     }
 
-    // Largest magnitudes of the tile's rows, and of each operand's part of the tile.
-    uint32_t* const row_most = reinterpret_cast<uint32_t*>(lds);   // floats >= 0 compare like integers
-    for (int i = threadIdx.x; i < 2 * kTile + 2; i += kBlock) row_most[i] = 0;
+    // Largest magnitudes of the operands' parts of the tile.
+    uint32_t* const largest = reinterpret_cast<uint32_t*>(lds);   // floats >= 0 compare like integers
+    if (threadIdx.x < 2) largest[threadIdx.x] = 0;
     __syncthreads();
-    atomicMax(&row_most[fw.row], __float_as_uint(fw.most));
-    atomicMax(&row_most[kTile + fx.row], __float_as_uint(fx.most));
+    atomicMax(&largest[0], __float_as_uint(fw.most));
+    atomicMax(&largest[1], __float_as_uint(fx.most));
     __syncthreads();
-    bool odd = false;
-    static_assert(kBlock == 2 * kTile, "a thread per row");
-    {
-        const float most = __uint_as_float(row_most[threadIdx.x]);
-        odd = most > 0.f && most < kTiny;
-        atomicMax(&row_most[2 * kTile + (threadIdx.x >= kTile ? 1 : 0)], row_most[threadIdx.x]);
-    }
-    odd = __syncthreads_or(odd);
-    const float most_w = __uint_as_float(row_most[2 * kTile]), most_x = __uint_as_float(row_most[2 * kTile + 1]);
-    odd = odd || !(most_w < kHuge) || !(most_x < kHuge) || !(most_w * most_x < kHuge);
+    const float most_w = __uint_as_float(largest[0]), most_x = __uint_as_float(largest[1]);
+    const bool odd = !(most_w < kHuge) || !(most_x < kHuge) || !(most_w * most_x * static_cast<float>((t_end - t_begin) * BK) < kMost);
     if (odd) {   // the same in all threads
         clear();
         auto element = [&](const float* base, bool transposed, int64_t row, int64_t rows, int64_t ld, int64_t k) {
@@ -298,7 +294,7 @@ __global__ __launch_bounds__(kBlock, 2) void gemm32_split(const Part32 p, int sp
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[i][j][e] = acc[i][j][e] + rest[i][j][e];
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = (acc[i][j][e] + rest[i][j][e]) * kUnscale;
     }
 
     // Lane holds row m = l32 and columns n = 8 g + 4 kh + {0..3} of a block in acc[4 g + {0..3}].

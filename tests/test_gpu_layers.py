@@ -2090,6 +2090,35 @@ def test_gemm_f32_error_of_sparse_operands(ops, M, N, K, a_t, b_t, edge, density
         assert float(error.norm()) <= float((_sums_of_fp32(x, w).double() - want).norm())
 
 
+@pytest.mark.parametrize("M,N,K,a_t,b_t,edge", [(3300, 3411, 48, False, False, 128), (3300, 3411, 100, True, True, 128), (640, 640, 8200, False, True, 128),
+                                                (1300, 1411, 48, False, False, 0)])
+def test_gemm_f32_of_rows_of_mixed_magnitudes(ops, M, N, K, a_t, b_t, edge):
+    """Elements of one row from the smallest denormal to ordinary ones, next to zeros: every product is as exact as in fp32
+    arithmetic, also where the small elements alone meet large ones of the other operand and make up the result."""
+    assert _plan32(M, N, K, a_t, b_t).edge == edge
+    gen = torch.Generator(device="cuda").manual_seed(K)
+
+    def mixed(rows, least, most):
+        exponent = torch.randint(least, most + 1, (rows, K), generator=gen, device="cuda")
+        keep = torch.rand(rows, K, generator=gen, device="cuda") < 0.1
+        return (torch.randn(rows, K, generator=gen, device="cuda", dtype=torch.float64) * torch.pow(2.0, exponent.double()) * keep).float()
+    x, w = mixed(M, -149, 4), mixed(N, -20, 60)
+    x[:128, 0], w[:, 0] = 1.0, 0.0
+    x[:128, 1:] = 0.0
+    x[:128, 1] = torch.randn(128, generator=gen, device="cuda") * 2.0 ** -118        # the whole result of these rows ...
+    w[:64, 1] = torch.randn(64, generator=gen, device="cuda") * 2.0 ** 97            # ... with parts of bf16
+    w[256:300, 1] = torch.randn(44, generator=gen, device="cuda") * 2.0 ** 117       # ... and with elements too large for them
+    a, sa = (x.t().contiguous(), (1, M)) if a_t else (x, (K, 1))
+    b, sb = (w.t().contiguous(), (1, N)) if b_t else (w, (K, 1))
+    out = torch.empty(M, N, device="cuda")
+    ops._gemm(a, *sa, b, *sb, None, out, ops._LINEAR_DTYPES[torch.float32], M, N, K)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert bool(((out.double() - want).abs() <= (K + 2) * 2.0 ** -24 * size + 2.0 ** -149 * K).all())
+    one = (x[:128] != 0).sum(1) == 2                 # 1 and the small element: one product
+    narrow = (out.double() - want).abs()[:128][one][:, :300]
+    assert bool((narrow <= (1 + 2.0 ** -4) * 2.0 ** -24 * size[:128][one][:, :300] + 2.0 ** -149).all())
+
+
 def test_gemm_f32_tiled_kernel_random_and_odd_depth(ops):
     """Random operands through the tiled fp32 kernel: both operands read along
     their rows, so the reduction length may be anything (here 1003, no multiple
