@@ -541,8 +541,11 @@ int launch_typed(const LnArgs& a, const PartCounts& pc, bool vec, hipStream_t s)
     const bool one_launch = cols > kWaveRowCols || (cols > 512 ? a.rows : (a.rows + 1) / 2) * kWave <= 0xFFFFFF00ll;
     if (vec && cols <= kBlockRowCols && (one_launch || MODE == kJoined)) return launch_held<T, MODE, AFFINE, false>(a, pc, s);
     if constexpr (MODE != kJoined) {
-        // Rows that start at any element: held as well, instead of read element by element once per reduction.
-        if (cols >= 4 && cols <= kBlockRowCols && one_launch) return launch_held<T, MODE, AFFINE, true>(a, pc, s);
+        // Rows that start at any element: held as well, instead of read element by element once per reduction.  Not in place
+        // with the statistics from memory: the last piece of a row starts on elements of the one in front of it, which another
+        // lane may have stored by then (where the row is reduced first, all of it has been read).
+        const bool in_place = MODE == kNorm && a.x == a.y;
+        if (cols >= 4 && cols <= kBlockRowCols && one_launch && !in_place) return launch_held<T, MODE, AFFINE, true>(a, pc, s);
     }
     if constexpr (MODE == kJoined) {
         return fail(DDL_E_UNSUPP, "ln stats+normalize: rows of more than %d columns take the two-launch form", kBlockRowCols);

@@ -145,7 +145,9 @@ __device__ inline void ln_bwd_input_body(uint32_t block, const T* __restrict__ d
     // reduced: the reduction waits for the gathered pairs, and the row should
     // not wait behind it (one memory round trip instead of two for rows of up
     // to 1024 columns).
-    const bool tiny = ANY && cols < 4;
+    // Element by element where a row is shorter than a piece, and in place, where the last piece would start on elements that
+    // have been stored.
+    const bool by_element = ANY && (cols < 4 || dx == dy || dx == x);
     BwdPiece<T, ANY> p[kAhead];
     auto fetch = [&](int64_t first) {
 #pragma unroll
@@ -153,10 +155,10 @@ __device__ inline void ln_bwd_input_body(uint32_t block, const T* __restrict__ d
             if (first + k * (kWave * 4) < cols) p[k].load(dyr, xr, gamma, piece_column<ANY>(first + k * (kWave * 4), cols));
     };
     int64_t first = lane * 4;
-    if (!tiny) fetch(first);
+    if (!by_element) fetch(first);
     const float S1 = wave_sum(p1) * weight, S2 = wave_sum(p2) * weight;   // already times a_p
-    if (tiny) {
-        if (lane < cols) store1(dxr + lane, dx_value(load1(dyr + lane), gamma ? load1(gamma + lane) : 1.f, load1(xr + lane), m, rs, S1, S2));
+    if (by_element) {
+        for (int64_t c = lane; c < cols; c += kWave) store1(dxr + c, dx_value(load1(dyr + c), gamma ? load1(gamma + c) : 1.f, load1(xr + c), m, rs, S1, S2));
         return;
     }
     while (true) {

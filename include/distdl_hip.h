@@ -215,7 +215,8 @@ int ddl_ln_partial_stats(const void* x, int dtype, int64_t rows, int64_t cols,
  *   part_stats [nparts][rows][2]  fp32 (this worker's own partials included)
  *   part_cols  [nparts]           host array: columns n_p held by each worker
  *   gamma/beta [cols] or NULL (both or neither)
- *   mean_out/rstd_out [rows] fp32 or NULL: the combined statistics, for backward. */
+ *   mean_out/rstd_out [rows] fp32 or NULL: the combined statistics, for backward.
+ * In this call and the next two y may be x (ldy = ld); else the two must not overlap. */
 int ddl_ln_normalize_affine(const void* x, int dtype, int64_t rows, int64_t cols,
                             int64_t ld, const float* part_stats,
                             int nparts, const int64_t* part_cols,
@@ -287,8 +288,9 @@ int ddl_ln_normalize_affine_f32(const float* x, int64_t rows, int64_t cols,
  * dy, x, gamma, dx, dgamma and dbeta are of `dtype` (DDL_DT_F32, DDL_DT_BF16 or
  * DDL_DT_F16: autograd hands gradients over in the type of the tensors); mean,
  * rstd, the sums and the workspace are fp32, as is all arithmetic, and results
- * are rounded once when stored.  The _f32 forms are the same calls with
- * dtype = DDL_DT_F32. */
+ * are rounded once when stored.  Here and in the calls below dx may be dy or x
+ * (same pitch); else it must not overlap them.  The _f32 forms are the same calls
+ * with dtype = DDL_DT_F32. */
 int ddl_ln_bwd_partial(const void* dy, const void* x, int dtype, int64_t rows,
                        int64_t cols, int64_t ld_dy, int64_t ld_x,
                        const float* mean, const float* rstd,

@@ -104,6 +104,63 @@ def test_layernorm_config1_rank0(ops):
     assert np.allclose(got, want[..., :256].reshape(-1, 256).numpy(), rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cols,pad", [(3, 0), (5, 0), (257, 0), (513, 1), (1021, 0), (1025, 0), (1027, 2), (2051, 0), (4097, 0), (8191, 1), (16383, 0), (16391, 0), (1024, 0), (4096, 4)])
+def test_layernorm_in_place_through_the_c_abi(ops, dtype, cols, pad):
+    """y written over x, dx over dy and over x, at lengths where a row's last piece starts on elements of the one in front of
+    it -- in the same lane's next request, another lane's, another wavefront's -- and at aligned ones.  The results are
+    those in memory of its own, but for a product and a sum that may be rounded together or one by one."""
+    from distdl_amd import _lib
+    lib, rows, stream = _lib.load(), 37, torch.cuda.current_stream().cuda_stream
+    dt, pitch = ops._LN_DTYPES[dtype], cols + pad
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")
+    x, dy = rnd(rows, pitch).to(dtype), rnd(rows, pitch).to(dtype)
+    gamma, beta = (1 + 0.1 * rnd(cols)).to(dtype), (0.1 * rnd(cols)).to(dtype)
+    stats = torch.stack((0.1 * rnd(1, rows), cols * (1 + 0.1 * rnd(1, rows).abs())), dim=2).contiguous()
+    sums, mean, rstd = rnd(1, rows, 2), torch.empty(rows, device="cuda"), torch.empty(rows, device="cuda")
+    work, widths = torch.empty(2 * 256 * cols, device="cuda"), _lib.i64_array([cols])
+    p = lambda t: t.data_ptr()
+
+    def normalize(src, dst):
+        return lib.ddl_ln_normalize_affine(p(src), dt, rows, cols, pitch, p(stats), 1, widths, p(gamma), p(beta), 1e-5, p(dst), pitch, p(mean), p(rstd), stream)
+
+    def whole(src, dst):
+        return lib.ddl_layer_norm(p(src), dt, rows, cols, pitch, p(gamma), p(beta), 1e-5, p(dst), pitch, p(mean), p(rstd), stream)
+
+    def dx(dy, x, dst):
+        return lib.ddl_ln_bwd_input(p(dy), p(x), dt, rows, cols, pitch, pitch, p(mean), p(rstd), p(gamma), p(sums), 1, 1.0 / cols, p(dst), pitch, stream)
+
+    def dx_params(dy, x, dst):
+        dg, db, scratch = torch.empty(cols, dtype=dtype, device="cuda"), torch.empty(cols, dtype=dtype, device="cuda"), torch.empty(rows, 2, device="cuda")
+        rc = lib.ddl_ln_bwd_partial_params(p(dy), p(x), dt, rows, cols, pitch, pitch, p(mean), p(rstd), p(gamma), p(scratch), p(work), work.numel(), stream)
+        return rc or lib.ddl_ln_bwd_input_params(p(dy), p(x), dt, rows, cols, pitch, pitch, p(mean), p(rstd), p(gamma), p(sums), 1, 1.0 / cols, p(dst), pitch,
+                                                 p(work), work.numel(), p(dg), p(db), stream)
+
+    def dx_whole(dy, x, dst):
+        dg, db = torch.empty(cols, dtype=dtype, device="cuda"), torch.empty(cols, dtype=dtype, device="cuda")
+        return lib.ddl_ln_bwd_whole_rows(p(dy), p(x), dt, rows, cols, pitch, pitch, p(mean), p(rstd), p(gamma), 1.0 / cols, p(dst), pitch, p(work), work.numel(),
+                                         p(dg), p(db), stream)
+    one = {torch.float32: 2.0 ** -22, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+
+    def same(got, want):
+        got, want = got[:, :cols].double(), want[:, :cols].double()
+        assert bool(((got - want).abs() <= one * (want.abs() + 8)).all()) if dtype == torch.float32 else bool(((got - want).abs() <= one * want.abs() + 2.0 ** -21).all())
+    for call in (normalize, whole):
+        apart, here = torch.full_like(x, 77), x.clone()
+        _lib.check(call(x, apart), "out of place")
+        _lib.check(call(here, here), "in place")
+        same(here, apart)
+        assert torch.equal(here[:, cols:], x[:, cols:])
+    for call in [dx, dx_params] + ([dx_whole] if 512 < cols <= 8192 else []):
+        apart = torch.full_like(x, 77)
+        _lib.check(call(dy, x, apart), "out of place")
+        for over in "dy", "x":
+            here = (dy if over == "dy" else x).clone()
+            _lib.check(call(here, x, here) if over == "dy" else call(dy, here, here), "in place")
+            same(here, apart)
+
+
 @pytest.mark.parametrize("cols", [[4, 4], [64, 64, 64], [300, 212], [1000, 24], [2048], [7, 9], [4100, 4100],
                                   [20000, 100], [8] * 70, [4] * 200, [2052, 4096], [8192, 16384], [16388, 12000],
                                   [4101, 33]])
