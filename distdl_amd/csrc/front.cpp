@@ -141,7 +141,7 @@ bool ln_backward_operands(const Tensor& dy, const Tensor& x2d, const Tensor& mea
            (!gamma || (plain(*gamma) && gamma->scalar_type() == x2d.scalar_type() && gamma->numel() == x2d.size(1)));
 }
 
-// Rows this worker holds whole: dx and the parameters' gradients in one pass.
+// Rows this worker holds whole: dx and the parameters' gradients in one pass.  dy may have any shape of as many elements.
 std::optional<std::tuple<Tensor, Tensor, Tensor>> ln_backward_whole(const Tensor& dy, const Tensor& x2d, const Tensor& mean, const Tensor& rstd,
                                                                     const MaybeTensor& gamma, const MaybeShape& gamma_shape, const MaybeShape& beta_shape) {
     if (!ln_backward_operands(dy, x2d, mean, rstd, gamma)) return std::nullopt;
@@ -169,7 +169,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> ln_backward_whole(const Tensor
 // Rows shared with other workers: this worker's row sums and partial column sums ...
 std::optional<std::tuple<Tensor, Tensor>> ln_backward_partial_params(const Tensor& dy, const Tensor& x2d, const Tensor& mean, const Tensor& rstd,
                                                                      const MaybeTensor& gamma) {
-    if (!ln_backward_operands(dy, x2d, mean, rstd, gamma)) return std::nullopt;
+    if (!ln_backward_operands(dy, x2d, mean, rstd, gamma) || dy.sizes() != x2d.sizes()) return std::nullopt;
     const int64_t rows = x2d.size(0), cols = x2d.size(1);
     Tensor sums = floats(dy, {rows, 2}), work = floats(dy, {2 * clamped((rows + 31) / 32, 256) * cols});
     check(ddl_ln_bwd_partial_params(dy.data_ptr(), x2d.data_ptr(), float_code(x2d), rows, cols, cols, cols, mean.data_ptr<float>(), rstd.data_ptr<float>(),
@@ -182,7 +182,7 @@ std::optional<std::tuple<Tensor, Tensor>> ln_backward_partial_params(const Tenso
 std::optional<std::tuple<Tensor, Tensor, Tensor>> ln_backward_input_params(const Tensor& dy, const Tensor& x2d, const Tensor& mean, const Tensor& rstd,
                                                                            const MaybeTensor& gamma, const Tensor& part_sums, double weight,
                                                                            const Tensor& work, const MaybeShape& gamma_shape, const MaybeShape& beta_shape) {
-    if (!ln_backward_operands(dy, x2d, mean, rstd, gamma) || !plain(part_sums) || !plain(work) || part_sums.scalar_type() != at::kFloat ||
+    if (!ln_backward_operands(dy, x2d, mean, rstd, gamma) || dy.sizes() != x2d.sizes() || !plain(part_sums) || !plain(work) || part_sums.scalar_type() != at::kFloat ||
         work.scalar_type() != at::kFloat || part_sums.dim() != 3 || part_sums.size(1) != x2d.size(0) || part_sums.size(2) != 2)
         return std::nullopt;
     const int64_t rows = x2d.size(0), cols = x2d.size(1);
@@ -212,7 +212,8 @@ MaybeTensor embedding_gather(const Tensor& weight, const Tensor& ids, int64_t lo
 
 MaybeTensor embedding_backward(const Tensor& dy, const Tensor& ids, int64_t lo, int64_t hi, int64_t padding_idx, bool by_freq) {
     const int dt = float_code(dy);
-    if (!dt || !plain(dy) || !id_tensor(ids) || dy.dim() != ids.dim() + 1 || dy.sizes().slice(0, ids.dim()) != ids.sizes() || hi < lo) return std::nullopt;
+    if (!dt || !plain(dy) || !id_tensor(ids) || dy.dim() != ids.dim() + 1 || dy.sizes().slice(0, ids.dim()) != ids.sizes() || dy.size(-1) == 0 || hi < lo)
+        return std::nullopt;
     const int64_t dim = dy.size(-1), rows = hi - lo, n = ids.numel();
     const int64_t few = 3 * rows + 1 + n, all = ddl_embedding_backward_workspace(n, rows), elems = few > all ? few : all;
     Tensor dw = at::empty({rows, dim}, dy.options()), work = at::empty({elems}, dy.options().dtype(at::kInt));

@@ -140,6 +140,12 @@ def test_layer_norm_adjoint_of_shared_rows(both, dtype, rows, cols):
     both(lambda: step(_randn(rows, cols + 1, dtype=dtype)[:, :cols], x, gamma))
     both(lambda: step(dy, x.double(), gamma))
     both(lambda: step(dy, x, gamma.cpu()))
+    # as many elements in another shape
+    work = hip_ops.ln_backward_partial_params(dy, x, mean, rstd, gamma)[1]
+    for other in dy.view(cols, rows), dy.view(1, rows, cols), dy.view(-1):
+        for refused in (lambda: hip_ops.ln_backward_partial_params(other, x, mean, rstd, gamma),
+                        lambda: hip_ops.ln_backward_input_params(other, x, mean, rstd, gamma, parts, 0.25 / cols, work)):
+            assert both(refused)[0] is ValueError
 
 
 @pytest.mark.parametrize("dtype", DTYPES + [torch.float64])
@@ -158,6 +164,7 @@ def test_embedding_and_its_adjoint(both, dtype, idt):
     both(lambda: hip_ops.embedding_backward(dy, ids.t().contiguous().t(), 3, 23))
     both(lambda: hip_ops.embedding_backward(dy, ids[:4], 3, 23))
     both(lambda: hip_ops.embedding_backward(dy[:0], ids[:0], 3, 23))
+    both(lambda: hip_ops.embedding_backward(dy[..., :0], ids, 3, 23))
 
 
 @pytest.mark.parametrize("dtype", DTYPES + [torch.float64, torch.int32, torch.int64, torch.uint8])
