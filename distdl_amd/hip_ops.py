@@ -175,7 +175,6 @@ class BoxLaunch:
         entries = [e for e in entries if min(e[4], default=1) > 0]
         self.elem_size = elem_size
         self.n = len(entries)
-        self._type = _lib.ddl_box_t * self.n
         self._bases, packed = [], []
         for src, src_off, dst, dst_off, shape, src_strides, dst_strides in entries:
             nd = len(shape)
@@ -186,6 +185,9 @@ class BoxLaunch:
             self._bases.append((src, int(src_off) * elem_size, dst, int(dst_off) * elem_size))
         self._template = b"".join(packed)
         self._boxes = None
+
+    def __getstate__(self):
+        return {**self.__dict__, "_boxes": None}      # a copy makes its own
 
     def run(self, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
         if self.n == 0:

@@ -2,8 +2,10 @@
 the golden vectors, overlap lists and buffer pools of the layers, the loopback
 transport, error behaviour, and the C-ABI surface.  No kernel is launched here."""
 
+import copy
 import ctypes
 import os
+import pickle
 import re
 
 import numpy as np
@@ -778,7 +780,7 @@ def boxes_on_the_cpu(monkeypatch):
             return
         element = {4: ctypes.c_float, 8: ctypes.c_double}[launch.elem_size]
         assert op != _lib.DDL_OP_ADD or dtype == _lib.DDL_DT_F32
-        boxes = launch._type.from_buffer_copy(launch._template)
+        boxes = (_lib.ddl_box_t * launch.n).from_buffer_copy(launch._template)
         sides = []
         for box, (src, src_off, dst, dst_off) in zip(boxes, launch._bases):
             at = []
@@ -920,6 +922,19 @@ def test_halo_adjoint_of_ghosts_that_share_elements_or_have_no_buffer(boxes_on_t
     dx, = torch.autograd.grad(e.forward(x, buffers), x, torch.tensor([1.0, 2.0, 3.0, 4.0]))
     assert buffers[0][1].raw_buffer.tolist() == [1]
     assert dx.tolist() == [0, 2, 3, 0]
+
+
+def test_launches_and_plans_that_have_run_can_be_copied():
+    """The native half of a launch is made in its first run and does not go along."""
+    from distdl_amd import hip_ops
+    launch = hip_ops.BoxLaunch([(0, 0, 1, 5, [2, 3], [3, 1], [4, 1])], 4)
+    launch._boxes = _lib.front().Boxes(launch._template, launch._bases, 4)
+    plan = hip_ops.HaloPadPlan([1, 2, 6, 7], [[0, 0], [0, 0], [1, 1], [1, 1]], [[0, 0], [0, 0], [0, 1], [0, 1]], [[0, 0], [0, 0], [0, 1], [0, 1]])
+    plan._crops[4] = launch
+    for again in copy.deepcopy(launch), pickle.loads(pickle.dumps(launch)), copy.deepcopy(plan)._crops[4]:
+        assert again is not launch and again._boxes is None
+        assert (again.n, again.elem_size, again._template, again._bases) == (1, 4, launch._template, launch._bases)
+    assert launch._boxes is not None
 
 
 def test_gathered_pieces_of_other_extents_are_refused():
