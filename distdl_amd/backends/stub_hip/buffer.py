@@ -52,7 +52,10 @@ class ExpandableBuffer:
         self.get_view(tuple(view_shape))
 
     def get_view(self, view_shape):
-        view = self.views.get(view_shape) if type(view_shape) is tuple else None
+        try:
+            view = self.views.get(view_shape)
+        except TypeError:                  # a list, or extents that do not hash
+            view = None
         if view is None:
             view_shape = tuple(int(s) for s in view_shape)
             view = self.views.get(view_shape)

@@ -442,6 +442,8 @@ def test_expandable_buffer_views_and_growth():
     assert buf.capacity == 20 and w.shape == (4, 5)
     assert buf.get_view((2, 3)).flatten().tolist() == [0, 1, 2, 3, 4, 5]
     assert buf.get_view((2, 3)).data_ptr() == w.data_ptr() == buf.raw_buffer.data_ptr()
+    for extents in (np.array(2), np.array(3)), [2, 3], np.array([2, 3]), torch.Size([2, 3]), (2.0, np.int64(3)):
+        assert buf.get_view(extents) is buf.get_view((2, 3))
     buf.expand(10)
     assert buf.capacity == 20
 
