@@ -388,51 +388,48 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
     }
     __syncthreads();
     const int32_t all_long = long_rows;
-    for (int32_t first = 0; first < all_long; first += kLongRows) {
+    static_assert(kBitsPerWindow / (kRankTokens + 1) <= kLongRows, "no call has more long rows whose tokens fit the bits");
+#pragma unroll
+    for (int k = 0; k < kRows; ++k)
+        if (long_at[k] >= 0) {
+            long_begin[long_at[k]] = begins[k];
+            long_end[long_at[k]] = begins[k] + n[k];
+        }
+    for (int32_t h = 0; h < all_long; ++h) {
+        uint32_t* const bits = reinterpret_cast<uint32_t*>(counters);
+        static_assert(kBitWords == kSegmentRows, "a bit per token number where the counters were");
+        constexpr int kWords = kBitWords / kBucketBlock;
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < kRows; ++k)
-            if (long_at[k] >= first && long_at[k] < first + kLongRows) {
-                long_begin[long_at[k] - first] = begins[k];
-                long_end[long_at[k] - first] = begins[k] + n[k];
-            }
-        const int32_t here = all_long - first < kLongRows ? all_long - first : kLongRows;
-        for (int32_t h = 0; h < here; ++h) {
-            uint32_t* const bits = reinterpret_cast<uint32_t*>(counters);
-            static_assert(kBitWords == kSegmentRows, "a bit per token number where the counters were");
-            constexpr int kWords = kBitWords / kBucketBlock;
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k < kWords; ++k) bits[t + k * kBucketBlock] = 0;
-            __syncthreads();
-            const int32_t begin = long_begin[h], end = long_end[h];
-            for (int32_t i = begin + t; i < end; i += kBucketBlock) {
-                const int32_t at = tokens <= kHeldTokens ? held[i - stretch] : a.bucket[i];
-                atomicOr(&bits[at >> 5], 1u << (at & 31));
-            }
-            __syncthreads();
-            uint32_t mine[kWords];
-            int32_t sum = 0;
-#pragma unroll
-            for (int k = 0; k < kWords; ++k) {
-                mine[k] = bits[t * kWords + k];
-                sum += __popc(mine[k]);
-            }
-            int32_t up_to = sum;
-#pragma unroll
-            for (int off = 1; off < kWave; off <<= 1) {
-                const int32_t up = __shfl_up(up_to, off, kWave);
-                if (lane >= off) up_to += up;
-            }
-            if (lane == kWave - 1) wave_total[wave] = up_to;
-            __syncthreads();
-            int32_t rank = begin + up_to - sum;
-#pragma unroll
-            for (int k = 0; k < kBucketBlock / kWave; ++k) rank += k < wave ? wave_total[k] : 0;
-#pragma unroll
-            for (int k = 0; k < kWords; ++k)
-                for (uint32_t w = mine[k]; w; w &= w - 1) a.bucket[rank++] = (t * kWords + k) * 32 + __ffs(w) - 1;
+        for (int k = 0; k < kWords; ++k) bits[t + k * kBucketBlock] = 0;
+        __syncthreads();
+        const int32_t begin = long_begin[h], end = long_end[h];
+        for (int32_t i = begin + t; i < end; i += kBucketBlock) {
+            const int32_t at = tokens <= kHeldTokens ? held[i - stretch] : a.bucket[i];
+            atomicOr(&bits[at >> 5], 1u << (at & 31));
         }
+        __syncthreads();
+        uint32_t mine[kWords];
+        int32_t sum = 0;
+#pragma unroll
+        for (int k = 0; k < kWords; ++k) {
+            mine[k] = bits[t * kWords + k];
+            sum += __popc(mine[k]);
+        }
+        int32_t up_to = sum;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int32_t up = __shfl_up(up_to, off, kWave);
+            if (lane >= off) up_to += up;
+        }
+        if (lane == kWave - 1) wave_total[wave] = up_to;
+        __syncthreads();
+        int32_t rank = begin + up_to - sum;
+#pragma unroll
+        for (int k = 0; k < kBucketBlock / kWave; ++k) rank += k < wave ? wave_total[k] : 0;
+#pragma unroll
+        for (int k = 0; k < kWords; ++k)
+            for (uint32_t w = mine[k]; w; w &= w - 1) a.bucket[rank++] = (t * kWords + k) * 32 + __ffs(w) - 1;
     }
 }
 
@@ -508,7 +505,7 @@ struct ReduceArgs {
     int32_t passes;         // groups of columns per row of the ordinary path
     int32_t rows_per_block;
     int32_t hot_above;      // rows of more tokens are hot
-    int32_t hot_chunks;     // 256-byte pieces of a row
+    int32_t hot_chunks;     // pieces of kHotBytes of a row
     int32_t scale_by_freq;
     __device__ Row of(int64_t row) const { return meta[(row & ((1 << shift) - 1)) * segment_rows + (row >> shift)]; }
 };
@@ -535,8 +532,8 @@ constexpr int kListTokens = 1024;
 constexpr int kWordsPerThread = kBitWords / kBlock;
 
 struct HotShared {
-    float column[kHotBytes / 2][kHotPitch];          // a batch in fp32, column by column: the adding wavefront reads four tokens at once
-    uint32_t bits[kBitWords];                        // a bit per token number, or the bucket being ordered
+    alignas(16) float column[kHotBytes / 2][kHotPitch];   // a batch in fp32, column by column: the adding wavefront reads four tokens at once
+    alignas(16) uint32_t bits[kBitWords];            // a bit per token number, or the bucket being ordered
     int32_t list[kListTokens];                       // tokens in ascending order
     int32_t wave_total[kWavesPerBlock];
 };

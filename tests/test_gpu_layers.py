@@ -1013,6 +1013,23 @@ def test_embedding_layer_full_window_matches_torch():
     assert torch.equal(torch.cat(outs, dim=-1), want)
 
 
+def test_embedding_backward_as_many_long_rows_in_a_segment_as_there_can_be(ops):
+    """255 rows of 513 tokens each, 256 rows apart, so that one workgroup of the bucketing has all of them in its segment and
+    orders every bucket by a bit per token number; sums in the order of the tokens, so repeated calls agree bit for bit."""
+    rows, dim, tokens = 5 + 256 * 254 + 40, 20, 131072
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    ids = (5 + 256 * (torch.arange(tokens, device="cuda") % 255))
+    ids[255 * 513:] = 7                                        # and 257 tokens of a row of another segment
+    ids = ids[torch.randperm(tokens, generator=gen, device="cuda")]
+    dy = torch.randn(tokens, dim, generator=gen, device="cuda")
+    got = ops.embedding_backward(dy, ids, 0, rows)
+    want, size = torch.zeros(rows, dim, dtype=torch.float64, device="cuda"), torch.zeros(rows, dim, dtype=torch.float64, device="cuda")
+    want.index_add_(0, ids, dy.double())
+    size.index_add_(0, ids, dy.double().abs())
+    assert bool(((got.double() - want).abs() <= 513 * 2.0 ** -24 * size).all())
+    assert torch.equal(ops.embedding_backward(dy, ids, 0, rows), got)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("norm_type", [1.0, 2.0, 3.0, float("inf")])
 @pytest.mark.parametrize("dim,idt", [(1, torch.int64), (7, torch.int32), (64, torch.int64), (300, torch.int32), (4100, torch.int64)])
