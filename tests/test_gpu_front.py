@@ -76,7 +76,7 @@ def test_linear_and_its_adjoint(both, dtype, m, n, k, pitch):
     both(lambda: hip_ops.linear(x, w))
     for need in ((True, True, True), (True, False, False), (False, True, True), (False, False, True)):
         both(lambda: hip_ops.linear_backward(x, w, dy, *need))
-    if x.numel() and dtype == torch.float32:
+    if x.numel() and (dtype == torch.float32 or all(v % 8 == 0 for v in (n, k, pitch))):
         assert both.taken == 6
     # operands that are not contiguous, off a 16-byte boundary, of other types or other lengths, on the host
     off = torch.empty(x.numel() + 1, dtype=dtype, device="cuda")[1:].view(x.shape).copy_(x)
@@ -85,11 +85,13 @@ def test_linear_and_its_adjoint(both, dtype, m, n, k, pitch):
     both(lambda: hip_ops.linear(x.transpose(0, -1).contiguous().transpose(0, -1), w, b))
     both(lambda: hip_ops.linear(x, w.t().contiguous().t(), b))
     both(lambda: hip_ops.linear_backward(x, w, dy.transpose(0, -1).contiguous().transpose(0, -1)))
+    taken = both.taken
     for bad in (lambda: hip_ops.linear(x.double(), w), lambda: hip_ops.linear(x, w.double()), lambda: hip_ops.linear(x, w, b.double()),
                 lambda: hip_ops.linear(x, w, b[:-1]), lambda: hip_ops.linear(x, w[0]), lambda: hip_ops.linear(x[..., :-1], w),
                 lambda: hip_ops.linear(x.cpu(), w), lambda: hip_ops.linear(x, w.cpu()), lambda: hip_ops.linear_backward(x, w, dy.double()),
                 lambda: hip_ops.linear_backward(x, w, dy.cpu())):
         both(bad)
+    assert both.taken == taken
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -137,15 +139,16 @@ def test_layer_norm_adjoint_of_shared_rows(both, dtype, rows, cols):
     both(lambda: step(dy, x, None))
     both(lambda: step(dy, x, gamma, want_beta=False))
     assert both.taken == 6
-    both(lambda: step(_randn(rows, cols + 1, dtype=dtype)[:, :cols], x, gamma))
+    work = hip_ops.ln_backward_partial_params(dy, x, mean, rstd, gamma)[1]
+    both(lambda: step(_randn(rows + 1, cols + 1, dtype=dtype)[:rows, :cols], x, gamma))
     both(lambda: step(dy, x.double(), gamma))
     both(lambda: step(dy, x, gamma.cpu()))
     # as many elements in another shape
-    work = hip_ops.ln_backward_partial_params(dy, x, mean, rstd, gamma)[1]
     for other in dy.view(cols, rows), dy.view(1, rows, cols), dy.view(-1):
         for refused in (lambda: hip_ops.ln_backward_partial_params(other, x, mean, rstd, gamma),
                         lambda: hip_ops.ln_backward_input_params(other, x, mean, rstd, gamma, parts, 0.25 / cols, work)):
             assert both(refused)[0] is ValueError
+    assert both.taken == 6 or rows == 1       # (one row is contiguous at any pitch)
 
 
 @pytest.mark.parametrize("dtype", DTYPES + [torch.float64])
@@ -155,14 +158,21 @@ def test_embedding_and_its_adjoint(both, dtype, idt):
     w, ids, dy = _randn(20, 12, dtype=dtype), torch.arange(30, device="cuda").reshape(5, 6).to(idt) % 27, _randn(5, 6, 12, dtype=dtype)
     for t in (w, _randn(20, 15, dtype=dtype)[:, :12], w.t().contiguous().t(), w[:19], w.cpu()):
         both(lambda: hip_ops.embedding_gather(t, ids, 3, 23))
+    known = idt != torch.int16
+    assert both.taken == known                # the first
     both(lambda: hip_ops.embedding_gather(w, ids.t(), 3, 23))
+    assert both.taken == known
     both(lambda: hip_ops.embedding_gather(w, ids[:0], 3, 23))
+    assert both.taken == 2 * known
     for pad in (None, 5):
         both(lambda: hip_ops.embedding_backward(dy, ids, 3, 23, pad))
         both(lambda: hip_ops.embedding_backward(dy, ids, 3, 23, pad, True))
+    adjoints = 4 * (known and dtype != torch.float64)
+    assert both.taken == 2 * known + adjoints
     both(lambda: hip_ops.embedding_backward(dy.transpose(0, 2).contiguous().transpose(0, 2), ids, 3, 23))
     both(lambda: hip_ops.embedding_backward(dy, ids.t().contiguous().t(), 3, 23))
     both(lambda: hip_ops.embedding_backward(dy, ids[:4], 3, 23))
+    assert both.taken == 2 * known + adjoints
     both(lambda: hip_ops.embedding_backward(dy[:0], ids[:0], 3, 23))
     both(lambda: hip_ops.embedding_backward(dy[..., :0], ids, 3, 23))
 
@@ -179,7 +189,9 @@ def test_gather_and_reduce_scatter_slabs(both, dtype, axis, divisor):
     pieces = {"all": [(10 * _randn(4, 7, 6, seed=q)).to(dtype) for q in range(3)]}
     world.transport.set_gather_provider("tag", lambda P, t: list(pieces["all"]))
     both(lambda: all_gather.gather_slabs(P, local, axis, "tag"))
+    assert both.taken == (axis != 3)
     both(lambda: all_gather.reduce_scatter_slabs(P, local, axis, "tag", divisor))
+    assert both.taken == 0 if axis == 3 else 2 - (dtype == torch.uint8)
     both(lambda: all_gather.gather_slabs(P, local.transpose(0, 2).contiguous().transpose(0, 2), axis, "tag"))
     both(lambda: all_gather.reduce_scatter_slabs(P, local.transpose(0, 2).contiguous().transpose(0, 2), axis, "tag", divisor))
     if axis == 1:       # pieces of different lengths, without elements, of another shape, off a 16-byte boundary of each other

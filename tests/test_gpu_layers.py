@@ -1992,11 +1992,12 @@ def test_gemm_16_bit_random_within_tolerance_and_ragged_depth(ops, a_t, b_t):
 
 @pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K,pad", [(4060, 1000, 40, 0), (4096, 4352, 132, 4), (16384, 256, 36, 8), (4100, 1004, 288, 0)])
-def test_gemm_f32_tiled_kernel_reads_every_operand_layout(ops, a_t, b_t, M, N, K, pad):
-    """Products large enough for the 256-wide fp32 tiles (at least 64 of them), in
-    every combination of operand layouts, with integer operands: every sum is
+def test_gemm_f32_large_products_read_every_operand_layout(ops, a_t, b_t, M, N, K, pad):
+    """Products of some thousand rows or columns (tiles of 64 x 64 and of 128 x 128),
+    in every combination of operand layouts, with integer operands: every sum is
     exact in fp32, so the result must equal the fp64 product -- tiles that
-    straddle M, N and K, pitched operands, the wide / narrow column split."""
+    straddle M, N and K, pitched operands.  (Integers this small are one bf16
+    part; test_gemm_f32_by_exact_bf16_parts has all three.)"""
     from distdl_amd import _lib
     gen = torch.Generator().manual_seed(M + 3 * N + K + 2 * a_t + b_t)
     a = torch.randint(-3, 4, (M, K), generator=gen).float()
@@ -2022,7 +2023,7 @@ def test_gemm_f32_tiled_kernel_reads_every_operand_layout(ops, a_t, b_t, M, N, K
     (1030, 517, 131, 0, False), (2050, 1027, 100, 2, False),
     # the reduction split over groups of wavefronts, and over workgroups, unequal shares
     (201, 263, 1033, 1, False), (201, 263, 2501, 1, True), (64, 100, 4095, 0, True),
-    # enough work for the 256 x 256 tiles, wide and narrow ones
+    # enough work for the 128 x 128 tiles
     (4096, 4352, 1540, 4, False)])
 def test_gemm_f32_products_of_every_size_and_pitch(ops, a_t, b_t, M, N, K, pad, splits):
     """Integer operands (every sum is exact in fp32) at the sizes where the fp32 tiles can go wrong, with and
@@ -2193,13 +2194,14 @@ def test_gemm_f32_of_rows_of_mixed_magnitudes(ops, M, N, K, a_t, b_t, edge):
     assert bool((narrow <= (1 + 2.0 ** -4) * 2.0 ** -24 * size[:128][one][:, :300] + 2.0 ** -149).all())
 
 
-def test_gemm_f32_tiled_kernel_random_and_odd_depth(ops):
-    """Random operands through the tiled fp32 kernel: both operands read along
+def test_gemm_f32_large_products_random_and_odd_depth(ops):
+    """Random operands through the 128 x 128 tiles: both operands read along
     their rows, so the reduction length may be anything (here 1003, no multiple
     of the k-tile or of a vector); and the forward layout with K = 1000."""
     from distdl_amd import _lib
     for a_t, b_t, K in ((True, True, 1003), (False, False, 1000)):
         M, N = 4096, 1024
+        assert _plan32(M, N, K, a_t, b_t).edge == 128
         gen = torch.Generator().manual_seed(K)
         a = torch.randn(M, K, generator=gen)
         b = 0.02 * torch.randn(N, K, generator=gen)
