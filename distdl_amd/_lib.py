@@ -8,6 +8,7 @@ callers below raise instead of computing something else.
 
 import ctypes
 import os
+import sys
 from ctypes import POINTER
 from ctypes import c_char_p
 from ctypes import c_double
@@ -176,8 +177,8 @@ def front():
         try:
             from . import _front as module
         except ImportError as e:
-            raise HipLibraryMissing(f"distdl_amd._front is not built or does not load ({e}); run `make -C "
-                                    f"{os.path.join(_HERE, 'csrc')}` (or __graft_entry__.build()).") from e
+            raise HipLibraryMissing(f"distdl_amd._front is not built for this interpreter or does not load ({e}); run `make -C "
+                                    f"{os.path.join(_HERE, 'csrc')} PYTHON={sys.executable}` (or __graft_entry__.build()).") from e
         _front = module
     return _front
 
