@@ -1,11 +1,22 @@
 """Base class of every layer (reference: nn/module.py:6-112): binds the backend
-selected at construction time and re-runs the layer's setup from a forward
-pre-hook whenever the structure of the input changes."""
+selected at construction time and re-runs the layer's setup as the first of the
+module's forward pre-hooks whenever the structure of the input changes.
+
+A module with a hook of its own goes torch's long way on every call, and layers
+are made of layers (a decode step of the all-gather linear layer 17.6 us, without them 15.2).  So the
+setup runs in front of torch's call while there is no other hook that could tell
+the difference, and is registered, ahead of the hooks of the module, once there is:
+global pre-hooks and prepended ones change the input before the setup sees it, and
+forward hooks may be called for a setup that raises."""
 
 import torch
 
 from .. import backends
 from .. import config
+
+# torch's hooks of all modules; None in a torch that keeps them elsewhere
+_PRE_HOOKS = getattr(torch.nn.modules.module, "_global_forward_pre_hooks", None)
+_HOOKS = getattr(torch.nn.modules.module, "_global_forward_hooks", None)
 
 
 class Module(torch.nn.Module):
@@ -14,7 +25,26 @@ class Module(torch.nn.Module):
         super().__init__()
         self._distdl_backend = backends.backend
         self._distdl_is_setup = False
-        self.register_forward_pre_hook(self._distdl_forward_pre_hook)
+        self._distdl_is_hooked = False
+        if _PRE_HOOKS is None or _HOOKS is None:
+            self._distdl_register_setup()
+
+    def _distdl_register_setup(self):
+        if not self._distdl_is_hooked:
+            self._distdl_is_hooked = True
+            super().register_forward_pre_hook(self._distdl_forward_pre_hook, prepend=True)
+
+    def register_forward_pre_hook(self, *args, **kwargs):
+        self._distdl_register_setup()
+        return super().register_forward_pre_hook(*args, **kwargs)
+
+    def __call__(self, *args, **kwargs):
+        if not self._distdl_is_hooked:
+            if self._forward_pre_hooks or self._forward_hooks or _PRE_HOOKS or _HOOKS:
+                self._distdl_register_setup()
+            else:
+                self._distdl_forward_pre_hook(self, args)
+        return super().__call__(*args, **kwargs)
 
     @staticmethod
     def _distdl_forward_pre_hook(self, input):

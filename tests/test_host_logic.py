@@ -401,20 +401,30 @@ class _ExchangeSetup(HaloExchange):
         return input
 
 
-@pytest.mark.parametrize("where", ["prepended", "global", "added"])
+def _exchange_setup():
+    P = SimWorld(4, device=torch.device("cpu")).partition(0).create_partition_inclusive(range(4)).create_cartesian_topology_partition([2, 2])
+    width = np.array([[0, 1], [0, 1]])
+    return _ExchangeSetup(P, width, width, width, buffer_manager=BufferManager(device=torch.device("cpu")))
+
+
+@pytest.mark.parametrize("called_before", [False, True])
+@pytest.mark.parametrize("where", ["prepended", "global", "added", "inserted"])
 @pytest.mark.parametrize("change", ["pad", "cast"])
-def test_setup_sees_the_input_of_the_pre_hooks_in_front_of_it(where, change):
+def test_setup_sees_the_input_of_the_pre_hooks_in_front_of_it(where, change, called_before):
     """A layer's set-up is the first forward pre-hook registered with the module: torch runs global pre-hooks and prepended
     ones ahead of it, so it works on what they return; hooks added after it come after it."""
     def hook(module, args):
         x, = args
         return torch.nn.functional.pad(x, (1, 1, 1, 1)) if change == "pad" else x.to(torch.bfloat16)
 
-    P = SimWorld(4, device=torch.device("cpu")).partition(0).create_partition_inclusive(range(4)).create_cartesian_topology_partition([2, 2])
-    width = np.array([[0, 1], [0, 1]])
-    layer = _ExchangeSetup(P, width, width, width, buffer_manager=BufferManager(device=torch.device("cpu")))
+    layer = _exchange_setup()
+    if called_before:
+        assert layer(torch.zeros(6, 6)).shape == (6, 6) and layer.slices[1][3][1] == slice(5, 6, None)
     if where == "global":
         handle = torch.nn.modules.module.register_module_forward_pre_hook(hook)
+    elif where == "inserted":
+        handle = torch.utils.hooks.RemovableHandle(layer._forward_pre_hooks)
+        layer._forward_pre_hooks[handle.id] = hook
     else:
         handle = layer.register_forward_pre_hook(hook, prepend=where == "prepended")
     try:
@@ -424,9 +434,41 @@ def test_setup_sees_the_input_of_the_pre_hooks_in_front_of_it(where, change):
         handle.remove()
     assert (tuple(out.shape), tuple(again.shape), out.dtype) == \
         (((10, 10), (14, 10), torch.float32) if change == "pad" else ((8, 8), (12, 8), torch.bfloat16))
-    seen = torch.zeros(12, 8) if where == "added" else again
+    seen = again if where in ("prepended", "global") else torch.zeros(12, 8)
     assert [layer.slices[d][3][d] for d in range(2)] == [slice(n - 1, n, None) for n in seen.shape]
     assert layer.buffers[0][3].dtype == seen.dtype
+    assert layer(torch.zeros(9, 9)).shape == (9, 9) and layer.slices[1][3][1] == slice(8, 9, None)
+
+
+@pytest.mark.parametrize("everywhere", [False, True])
+def test_forward_hooks_that_are_always_called_are_called_for_a_setup_that_raises(everywhere):
+    layer, called = _exchange_setup(), []
+
+    def hook(module, args, out):
+        called.append(out)
+    layer.forward = lambda input: pytest.fail("no forward without a set-up")
+    layer._distdl_module_setup = lambda input: 1 / 0
+    handle = torch.nn.modules.module.register_module_forward_hook(hook, always_call=True) if everywhere else \
+        layer.register_forward_hook(hook, always_call=True)
+    try:
+        with pytest.raises(ZeroDivisionError):
+            layer(torch.zeros(8, 8))
+    finally:
+        handle.remove()
+    assert called == [None]
+
+
+def test_setup_runs_once_per_call():
+    """In front of torch's call or as a hook of the module, never both."""
+    layer, seen = _exchange_setup(), []
+    requires_reset = layer._distdl_module_requires_reset
+    layer._distdl_module_requires_reset = lambda input: seen.append(input[0].shape) or requires_reset(input)
+    layer(torch.zeros(4, 4))
+    handle = layer.register_forward_pre_hook(lambda module, args: None)
+    layer(torch.zeros(5, 5))
+    handle.remove()
+    layer(torch.zeros(6, 6))
+    assert seen == [(4, 4), (5, 5), (6, 6)]
 
 
 # ------------------------------------------------------------ buffers --------
