@@ -21,8 +21,9 @@
 // 0.81e-6 -> 0.23e-6, a hundredth 0.164e-6 -> 0.055e-6, one element a row 0.0253e-6 both.
 //
 // Bound by the matrix instructions' power and, in small products, by issue: while a CU's
-// wavefronts multiply, they split (seven instructions an element).  158 to 160 TFLOP/s
-// at most where the fp32 instruction ends at 148.  Measured, fp32 instruction (64 x 64 or
+// wavefronts multiply, they split (seven instructions an element).  149 to 160 TFLOP/s
+// in large products, where the fp32 instruction ends at 148 (M 8192, N 3584, K 8192 3.06 to
+// 3.10 ms, its adjoint 3.10 and 3.22).  Measured, fp32 instruction (64 x 64 or
 // 256 x 256 tiles) -> here, operands along k or along their rows: M 256, N 3551, K 6575
 // 116 -> 101 to 106 us, M 3551, N 6575, K 256 147 to 169 -> 99 to 105, M = N = K = 2048 140 -> 122
 // to 128, 4096 968 -> 858 to 897, M 1024, N 8192, K 8192 1050 to 1075 -> 861 to 903; below about 20 us
