@@ -1,4 +1,4 @@
-// The 16-bit products that linear_small.hip computes, and when.
+// The 16-bit products that linear_small.hip and linear_any.hip compute, and when.
 #ifndef DDL_GEMM16_SMALL_H
 #define DDL_GEMM16_SMALL_H
 #include "gemm16_elements.h"
@@ -8,10 +8,11 @@ namespace ddl {
 typedef PartOf<uint16_t> Part16;
 
 struct Small16 {
-    enum Kind { kNone, kSkinny, kTiles, kAny };
+    enum Kind { kNone, kSkinny, kTiles, kAny, kThin };
     Kind kind = kNone;
     int groups = 1;              // kTiles: groups of wavefronts of a workgroup the reduction is split over (1 or 2)
-    int splits = 1;              // kTiles: workgroups the reduction of a tile is split over
+    int edge = 1;                // kAny: tiles of 64 (1) or 128 (2) rows and columns
+    int splits = 1;              // kTiles, kAny: workgroups the reduction of a tile is split over
     int64_t workspace = 0;       // floats for the splits' sums
 };
 
@@ -19,11 +20,13 @@ struct Small16 {
 // `large_us`, the estimate for the large tiles (microseconds).
 Small16 plan_small16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double large_us);
 
-// The same for operands that are not aligned to 16 bytes (kAny, or kNone): against `large_us` and copying both operands.
-Small16 plan_any16(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double large_us);
+// The same of linear_any.hip for operands that are not aligned to 16 bytes (kAny, kThin or kNone): against `large_us` and
+// copying both operands.
+Small16 plan_any16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double large_us);
 
 // Launches the product of `part` (its tile counts are set here) as planned; `partial` holds the splits' sums.
 int run_small16(const char* who, const Small16& plan, bool f16, bool xt, bool wt, const Part16& part, float* partial, int dev, hipStream_t s);
+int run_any16(const Small16& plan, bool f16, bool xt, bool wt, const Part16& part, float* partial, hipStream_t s);
 
 }  // namespace ddl
 #endif  // DDL_GEMM16_SMALL_H

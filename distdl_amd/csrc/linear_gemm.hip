@@ -517,23 +517,28 @@ Plan16 plan16(bool at, bool bt, int64_t M, int64_t N, int64_t K, int cus, int64_
     return plan;
 }
 
-// Can an operand with `rows` rows be read from wherever it lies (gemm16_any)?
+// Can an operand with `rows` rows be read from wherever it lies (linear_any.hip)?
 bool readable_anywhere(const Operand16& o, int64_t rows, int64_t K) {
     if (o.row_stride != 1 && o.k_stride != 1) return false;
     return o.transposed() ? rows >= 8 && o.ld() >= rows : rows == 1 || o.ld() >= K;
 }
 
-// How gemm16_any computes the product of such operands, if it does.  Whether it does is a matter of sizes and strides (the
-// caller copies the operands otherwise, and has no such way out later); the workspace only decides how.
-Small16 plan_anywhere(const Operand16& a, const Operand16& b, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace) {
+// How linear_any.hip computes the product of such operands, if it does.  Whether it does is a matter of sizes and strides (the
+// caller copies the operands otherwise, and has no such way out later); the workspace only decides how.  `leeway`: by how many
+// microseconds copying them may be the faster way.
+Small16 plan_anywhere(const Operand16& a, const Operand16& b, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double leeway) {
     if (!readable_anywhere(a, M, K) || !readable_anywhere(b, N, K)) return Small16{};
-    const double large = plan16(a.transposed(), b.transposed(), M, N, K, cus, 0).large;
-    const Small16 best = plan_any16(M, N, K, cus, INT64_MAX, large);
-    return best.kind == Small16::kNone || best.workspace <= workspace ? best : plan_any16(M, N, K, cus, workspace, 1e30);
+    const bool at = a.transposed(), bt = b.transposed();
+    const double large = plan16(at, bt, M, N, K, cus, 0).large;
+    const Small16 best = plan_any16(at, bt, M, N, K, cus, INT64_MAX, large + leeway);
+    return best.kind == Small16::kNone || best.workspace <= workspace ? best : plan_any16(at, bt, M, N, K, cus, workspace, 1e30);
 }
 
+// The product itself is computed for callers that do not have the copies, too, up to here.
+constexpr double kLeeway = 18;
+
 // y[M, N] = a[M, K] . b[N, K]^T + bias in 16-bit elements.  `workspace` (may be null) for the sums of a split reduction;
-// `anywhere`: operands that are not aligned to 16 bytes are taken where gemm16_any is the way to read them.
+// `anywhere`: operands that are not aligned to 16 bytes are taken where linear_any.hip reads them.
 int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* bias, uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
            float* workspace, int64_t workspace_elems, bool anywhere, void* stream) {
     if (M < 0 || N < 0 || K < 0 || ldy < N)
@@ -545,11 +550,11 @@ int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* 
         !(aligned_to(a.p, 16) && aligned_to(b.p, 16) && pitches_ok(a, M, K) && pitches_ok(b, N, K))) {
         int dev = 0;
         const int cus = compute_units(dev);
-        const Small16 any = plan_anywhere(a, b, M, N, K, cus, workspace ? workspace_elems : 0);
+        const Small16 any = plan_anywhere(a, b, M, N, K, cus, workspace ? workspace_elems : 0, kLeeway);
         if (any.kind != Small16::kNone) {
             Part16 p{};
             p.x = a.p, p.w = b.p, p.bias = bias, p.y = y, p.M = M, p.N = N, p.K = K, p.ldx = a.ld(), p.ldw = b.ld(), p.ldy = ldy;
-            return run_small16(who, any, f16, a.transposed(), b.transposed(), p, workspace, dev, static_cast<hipStream_t>(stream));
+            return run_any16(any, f16, a.transposed(), b.transposed(), p, workspace, static_cast<hipStream_t>(stream));
         }
     }
     if (int rc = check_operand(who, "a", a, M, K)) return rc;
@@ -660,7 +665,7 @@ extern "C" int ddl_gemm_in_place(int dtype, int aligned, int64_t a_row_stride, i
         return check_operand("gemm", "a", a, M, K) == 0 && check_operand("gemm", "b", b, N, K) == 0;
     int dev = 0;
     const int cus = compute_units(dev);
-    return plan_anywhere(a, b, M, N, K, cus, INT64_MAX).kind != Small16::kNone;
+    return plan_anywhere(a, b, M, N, K, cus, INT64_MAX, 0).kind != Small16::kNone;
 }
 
 extern "C" int64_t ddl_gemm_workspace_at(int dtype, int aligned, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride,
@@ -673,7 +678,7 @@ extern "C" int64_t ddl_gemm_workspace_at(int dtype, int aligned, int64_t a_row_s
     if (dtype != DDL_DT_BF16 && dtype != DDL_DT_F16) return 0;
     const Operand16 a{nullptr, a_row_stride, a_k_stride}, b{nullptr, b_row_stride, b_k_stride};
     if (aligned && pitches_ok(a, M, K) && pitches_ok(b, N, K)) return plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX).small.workspace;
-    return plan_anywhere(a, b, M, N, K, cus, INT64_MAX).workspace;
+    return plan_anywhere(a, b, M, N, K, cus, INT64_MAX, kLeeway).workspace;
 }
 
 extern "C" int64_t ddl_gemm_workspace(int dtype, int64_t a_row_stride, int64_t a_k_stride, int64_t b_row_stride, int64_t b_k_stride,

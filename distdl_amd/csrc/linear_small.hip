@@ -24,47 +24,13 @@
 //   even these tiles are too few, the reduction is split over `splits` workgroups per
 //   tile; their fp32 sums go through a workspace and gemm16_small_sum adds them in the
 //   order of the splits.
-#include "gemm16_elements.h"
-#include "gemm16_small.h"
+#include "gemm16_parts.h"
 #include <type_traits>
 
 namespace ddl {
 namespace {
 
 constexpr int BK = kRowBytes / 2;   // 16-bit elements of a k-tile
-
-template <bool F16>
-__device__ inline floatx4 mfma(const bf16x8& a, const bf16x8& b, const floatx4& c) {
-    if (F16) {
-        typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
-        f16x8 ha, hb;
-        __builtin_memcpy(&ha, &a, 16);
-        __builtin_memcpy(&hb, &b, 16);
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(ha, hb, c, 0, 0, 0);
-    }
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// Four consecutive columns n .. n + 3 of output row m.
-template <bool F16>
-__device__ inline void store_four(uint16_t* __restrict__ y, int64_t ldy, int64_t m, int64_t n, int64_t N, const float* v) {
-    uint16_t o[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = f32_to_elem<F16>(v[e]);
-    uint16_t* dst = y + m * ldy + n;
-    if (n + 3 < N) {   // global memory takes the eight bytes at any alignment
-        typedef uint32_t words __attribute__((ext_vector_type(2)));
-        typedef words any __attribute__((aligned(2)));
-        words pk;
-        pk[0] = static_cast<uint32_t>(o[0]) | (static_cast<uint32_t>(o[1]) << 16);
-        pk[1] = static_cast<uint32_t>(o[2]) | (static_cast<uint32_t>(o[3]) << 16);
-        *reinterpret_cast<any*>(dst) = pk;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (n + e < N) dst[e] = o[e];
-    }
-}
 
 // ---- up to 64 rows ---------------------------------------------------------
 
@@ -361,228 +327,6 @@ __global__ __launch_bounds__(KG * NWM * NWN * 64) void gemm16_small(const Part16
     }
 }
 
-// Sum of the splits' partial tiles, bias, rounding.  A thread per lane register quartet of the product kernel.
-template <bool F16, int NWM, int NWN, int TM, int TN>
-__global__ __launch_bounds__(256) void gemm16_small_sum(const Part16 p, int splits, const float* __restrict__ partial) {
-    constexpr int BM = 16 * NWM * TM, BN = 16 * NWN * TN, kQuartets = BM * BN / 4;
-    const int ntiles = p.tiles_m * p.tiles_n;
-    constexpr int kBlocks = kQuartets / 256;
-    static_assert(kBlocks * 256 == kQuartets, "tile does not split into workgroups");
-    const int tile = static_cast<int>(blockIdx.x) / kBlocks;
-    const int q = (static_cast<int>(blockIdx.x) - tile * kBlocks) * 256 + threadIdx.x;
-    int tm, tn;
-    tile_of_workgroup(tile, p.tiles_m, p.tiles_n, tm, tn);
-    const int lane = q & 63, block = (q >> 6) % (TN * TM), wave = (q >> 6) / (TN * TM);
-    const int64_t m = static_cast<int64_t>(tm) * BM + ((wave % NWM) * TM + block % TM) * 16 + (lane & 15);
-    const int64_t n = static_cast<int64_t>(tn) * BN + ((wave / NWM) * TN + block / TM) * 16 + 4 * (lane >> 4);
-    if (m >= p.M || n >= p.N) return;
-    const floatx4* src = reinterpret_cast<const floatx4*>(partial) + static_cast<int64_t>(tile) * kQuartets + q;
-    const int64_t stride = static_cast<int64_t>(ntiles) * kQuartets;
-    floatx4 s = {0.f, 0.f, 0.f, 0.f};
-    int k = 0;
-    for (; k + 4 <= splits; k += 4) {
-        floatx4 v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = src[(k + u) * stride];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) s += v[u];
-    }
-    for (; k < splits; ++k) s += src[k * stride];
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = s[e] + (p.bias && n + e < p.N ? elem_to_f32<F16>(p.bias[n + e]) : 0.f);
-    store_four<F16>(p.y, p.ldy, m, n, p.N, v);
-}
-
-// ---- small tiles of operands at any address and pitch ------------------------
-
-// 16 bytes from a 2-byte-aligned address (one global load; only requests into LDS need 4-byte alignment).
-struct __attribute__((packed, aligned(2))) Unaligned16 {
-    uint32_t word[4];
-};
-
-// gemm16_small for operands whose rows start at any element: the same tiles, layouts and fragment reads, but a tile comes
-// through registers (two tiles ahead, two wavefront groups that take alternate k-tiles, two stages of LDS each).  Chunks
-// that straddle K, and in the last k-tile of an operand read along rows whose number is no multiple of eight (a chunk there
-// runs over into the next k-line, which the last one has not), are put together from single elements.
-// It replaces copying such operands into padded or transposed temporaries, see the rule in plan_any16.
-template <bool F16, bool XT, bool WT>
-__global__ __launch_bounds__(512) void gemm16_any(const Part16 p, int splits, float* __restrict__ partial) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];
-    constexpr int NWM = 2, TM = 2, TN = 2, NW = 4, KG = 2, J = 2;   // 64 x 64: two 1 KiB pieces per wavefront and operand
-    constexpr int kStage = 128 * kRowBytes, kX = 64 * kRowBytes;
-    const int ntiles = p.tiles_m * p.tiles_n;
-    const int split = static_cast<int>(blockIdx.x) / ntiles, tile = static_cast<int>(blockIdx.x) - split * ntiles;
-    int tm, tn;
-    tile_of_workgroup(tile, p.tiles_m, p.tiles_n, tm, tn);
-    const int64_t M = p.M, N = p.N, K = p.K, m0 = static_cast<int64_t>(tm) * 64, n0 = static_cast<int64_t>(tn) * 64;
-    const int lane = threadIdx.x & 63, group = __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * 64));
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - group * NW;
-    const int l16 = lane & 15, kg = lane >> 4;
-    const int sub_w = (wave / NWM) * TN, sub_x = (wave % NWM) * TM;
-    const int ktiles = static_cast<int>((K + BK - 1) / BK);
-    const bool w_over = WT && N % 8 != 0, x_over = XT && M % 8 != 0;
-    const int full_tiles = static_cast<int>((w_over || x_over ? K - 1 : K) / BK);
-    const int per = (ktiles + splits - 1) / splits;
-    const int t_begin = split * per < ktiles ? split * per : ktiles, t_end = t_begin + per < ktiles ? t_begin + per : ktiles;
-    char* const ring = lds + group * (2 * kStage);
-
-    const uint16_t* const base_w = WT ? p.w + n0 : p.w + n0 * p.ldw;
-    const uint16_t* const base_x = XT ? p.x + m0 : p.x + m0 * p.ldx;
-    const int64_t step_w = WT ? p.ldw * BK : BK, step_x = XT ? p.ldx * BK : BK;   // elements from one k-tile to the next
-    auto chunk_k = [&](bool transposed, int i) {
-        const int row = i * 8 + (lane >> 3);
-        return transposed ? 8 * (i & 7) + (lane >> 3) : ((lane & 7) ^ ((row >> 1) & 7)) * 8;
-    };
-    auto chunk_row = [&](bool transposed, int i, int64_t origin, int64_t rows) -> int {
-        if (!transposed) {
-            const int row = i * 8 + (lane >> 3);
-            return origin + row < rows ? row : static_cast<int>(rows - 1 - origin);
-        }
-        const int k = chunk_k(true, i), h = ((k >> 1) & 1) | (((k >> 3) & 1) << 1);
-        const int col = (i >> 3) * 64 + ((lane & 7) ^ (h << 1)) * 8;
-        return origin + col < rows ? col : 0;
-    };
-    int64_t off_w[J], off_x[J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-        const int i = NW * j + wave;
-        off_w[j] = WT ? chunk_k(WT, i) * p.ldw + chunk_row(WT, i, n0, N) : chunk_row(WT, i, n0, N) * p.ldw + chunk_k(WT, i);
-        off_x[j] = XT ? chunk_k(XT, i) * p.ldx + chunk_row(XT, i, m0, M) : chunk_row(XT, i, m0, M) * p.ldx + chunk_k(XT, i);
-    }
-    auto careful = [&](bool transposed, const uint16_t* base, int64_t at, int t, int i, int64_t origin, int64_t rows) -> uint4 {
-        const int64_t k = static_cast<int64_t>(t) * BK + chunk_k(transposed, i), r = origin + chunk_row(transposed, i, origin, rows);
-        uint32_t v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const bool inside = transposed ? k < K && r + e < rows : k + e < K;
-            const uint32_t f = base[inside ? at + e : 0];   // the tile's first element otherwise
-            v[e] = inside ? f : 0u;
-        }
-        return make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
-    };
-    struct Regs {
-        uint4 w[J], x[J];
-    };
-    auto load = [&](int t, Regs& r) {
-        if (t >= t_end) return;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int64_t at_w = off_w[j] + t * step_w, at_x = off_x[j] + t * step_x;
-            if (t < full_tiles) {
-                const Unaligned16 a = *reinterpret_cast<const Unaligned16*>(base_w + at_w), b = *reinterpret_cast<const Unaligned16*>(base_x + at_x);
-                r.w[j] = make_uint4(a.word[0], a.word[1], a.word[2], a.word[3]);
-                r.x[j] = make_uint4(b.word[0], b.word[1], b.word[2], b.word[3]);
-            } else {
-                r.w[j] = careful(WT, base_w, at_w, t, NW * j + wave, n0, N);
-                r.x[j] = careful(XT, base_x, at_x, t, NW * j + wave, m0, M);
-            }
-        }
-    };
-    auto stash = [&](int t, int slot, const Regs& r) {
-        if (t >= t_end) return;
-        char* stage = ring + slot * kStage;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            *reinterpret_cast<uint4*>(stage + (NW * j + wave) * 1024 + lane * 16) = r.w[j];
-            *reinterpret_cast<uint4*>(stage + kX + (NW * j + wave) * 1024 + lane * 16) = r.x[j];
-        }
-    };
-    const int tr_lane = (8 * kg + (l16 >> 2)) * 128 + (l16 & 3) * 8;
-    const int tr_h = (((l16 >> 3) & 1) | ((kg & 1) << 1)) << 5;
-    typedef short short4v __attribute__((ext_vector_type(4)));
-    typedef short short8v __attribute__((ext_vector_type(8)));
-    typedef __attribute__((address_space(3))) short4v* lds_short4;
-    auto fragment = [&](auto transposed, const char* tile_base, int sub, int ks) -> bf16x8 {
-        bf16x8 out;
-        if (decltype(transposed)::value) {
-            const char* q = tile_base + (sub >> 2) * 8192 + ks * (32 * 128) + (tr_lane + (((sub & 3) << 5) ^ tr_h));
-            const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(q));
-            const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(q + 4 * 128));
-            const short8v both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            __builtin_memcpy(&out, &both, 16);
-        } else {
-            out = *reinterpret_cast<const bf16x8*>(tile_base + sub * (16 * kRowBytes) + l16 * kRowBytes + (((4 * ks + kg) ^ ((l16 >> 1) & 7)) << 4));
-        }
-        return out;
-    };
-    floatx4 acc[TN][TM];
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const int rounds = (t_end - t_begin + KG - 1) / KG;
-    auto tile_at = [&](int r) { return t_begin + r * KG + group; };
-    // Round r: tile r is in LDS slot r % 2, tile r + 1 in `next`; tile r + 2 is requested into `after`.
-    auto round = [&](int r, int slot, Regs& next, Regs& after) {
-        __syncthreads();   // tile r is complete; nobody reads the other slot any more
-        load(tile_at(r + 2), after);
-        const char* wt = ring + slot * kStage;
-        if (tile_at(r) < t_end) {
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                bf16x8 fw[TN], fx[TM];
-#pragma unroll
-                for (int a = 0; a < TN; ++a) fw[a] = fragment(std::integral_constant<bool, WT>{}, wt, sub_w + a, ks);
-#pragma unroll
-                for (int b = 0; b < TM; ++b) fx[b] = fragment(std::integral_constant<bool, XT>{}, wt + kX, sub_x + b, ks);
-#pragma unroll
-                for (int a = 0; a < TN; ++a)
-#pragma unroll
-                    for (int b = 0; b < TM; ++b) acc[a][b] = mfma<F16>(fw[a], fx[b], acc[a][b]);
-            }
-        }
-        stash(tile_at(r + 1), slot ^ 1, next);
-    };
-    Regs ra, rb;
-    load(tile_at(0), ra);
-    load(tile_at(1), rb);
-    stash(tile_at(0), 0, ra);
-    for (int r = 0; r < rounds; r += 2) {
-        round(r, 0, rb, ra);
-        if (r + 1 < rounds) round(r + 1, 1, ra, rb);   // the same in all wavefronts
-    }
-    __syncthreads();
-    floatx4* fold = reinterpret_cast<floatx4*>(lds);
-    if (group > 0) {
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-            for (int b = 0; b < TM; ++b) fold[(wave * (TN * TM) + a * TM + b) * 64 + lane] = acc[a][b];
-    }
-    __syncthreads();
-    if (group > 0) return;
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] += fold[(wave * (TN * TM) + a * TM + b) * 64 + lane];
-    if (splits > 1) {
-        floatx4* dst = reinterpret_cast<floatx4*>(partial) + (static_cast<int64_t>(blockIdx.x) * NW + wave) * (TN * TM * 64) + lane;
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-            for (int b = 0; b < TM; ++b) dst[(a * TM + b) * 64] = acc[a][b];
-        return;
-    }
-#pragma unroll
-    for (int a = 0; a < TN; ++a) {
-        const int64_t n = n0 + (sub_w + a) * 16 + 4 * kg;
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (p.bias) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < N) bv[e] = elem_to_f32<F16>(p.bias[n + e]);
-        }
-#pragma unroll
-        for (int b = 0; b < TM; ++b) {
-            const int64_t m = m0 + (sub_x + b) * 16 + l16;
-            if (m >= M) continue;
-            const float v[4] = {acc[a][b][0] + bv[0], acc[a][b][1] + bv[1], acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]};
-            store_four<F16>(p.y, p.ldy, m, n, N, v);
-        }
-    }
-}
-
 constexpr int kStages = 4;
 
 // Kernel functions whose dynamic LDS size has been raised on a device (first use, any thread): a flag per instantiation.
@@ -619,20 +363,7 @@ int launch_small(const char* who, const Part16& part, int splits, float* partial
 }
 
 template <bool F16, bool XT, bool WT>
-int launch_any(Part16 part, int splits, float* partial, hipStream_t s) {
-    part.tiles_m = static_cast<int>((part.M + 63) / 64), part.tiles_n = static_cast<int>((part.N + 63) / 64);
-    const int ntiles = part.tiles_m * part.tiles_n;
-    hipLaunchKernelGGL((gemm16_any<F16, XT, WT>), dim3(static_cast<uint32_t>(ntiles * splits)), dim3(512), 4 * 128 * kRowBytes, s, part, splits, partial);
-    if (int rc = check_launch("gemm16_any")) return rc;
-    if (splits == 1) return 0;
-    hipLaunchKernelGGL((gemm16_small_sum<F16, 2, 2, 2, 2>), dim3(static_cast<uint32_t>(ntiles * 4)), dim3(256), 0, s, part, splits,
-                       static_cast<const float*>(partial));
-    return check_launch("gemm16_small_sum");
-}
-
-template <bool F16, bool XT, bool WT>
 int launch_kind(const char* who, const Small16& plan, Part16 part, float* partial, int dev, hipStream_t s) {
-    if (plan.kind == Small16::kAny) return launch_any<F16, XT, WT>(part, plan.splits, partial, s);
     part.tiles_m = static_cast<int>((part.M + 63) / 64), part.tiles_n = static_cast<int>((part.N + 63) / 64);
     if (plan.groups == 2) return launch_small<F16, XT, WT, 2, 2, 2, 2, 2>(who, part, plan.splits, partial, dev, s);
     return launch_small<F16, XT, WT, 2, 2, 2, 2, 1>(who, part, plan.splits, partial, dev, s);
@@ -692,29 +423,6 @@ Small16 plan_small16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus,
         const double step = per_cu > 1 ? 0.19 * per_cu : 0.30;
         take(3.8 + kt * step + (per_cu > 2 ? per_cu - 2 : 0) * 1.4 + sum, Small16::kTiles, 1, splits);
         take(3.9 + ((kt + 1) / 2) * 0.375 * per_cu + (per_cu - 1) * 1.4 + sum, Small16::kTiles, 2, splits);
-    }
-    return best;
-}
-
-// Fits of a sweep as above: 1.1 us per round of two k-tiles for a lone workgroup, 0.7 for each that a CU has to work through.
-// The other way -- operands copied into padded or transposed temporaries -- is 30 us of launches and allocations in front
-// of the product, plus the copies at 4.5 TB/s.  Measured, copies and product -> here: M 8, N 3583, K 8191 37.6 -> 21.3 us;
-// M = N = K = 1023 20.5 -> 13.5; M 2049, N 511, K 4097 49.7 -> 48.4; M 4097, N 2049, K 2049 58.9, here 123.  The copies
-// alone are cheaper than that, what the host does for them is not: with 12 us for 30 a training step of M 4001, N 1001,
-// K 2051 goes from 184 to 217 us.
-Small16 plan_any16(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace, double large_us) {
-    Small16 best;
-    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), ktiles = (K + BK - 1) / BK;
-    if (tiles > 16 * static_cast<int64_t>(cus)) return best;
-    double best_us = 30 + large_us + (static_cast<double>(M) + N) * K * 4 / 4.5e6;
-    for (const int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        if (splits > 1 && (tiles * splits > 4 * static_cast<int64_t>(cus) || ktiles < 4 * splits || tiles * splits * 4096 > workspace)) break;
-        const int64_t per_cu = (tiles * splits + cus - 1) / cus, rounds = ((ktiles + splits - 1) / splits + 1) / 2;
-        const double us = 4 + rounds * (per_cu > 1 ? 0.7 * per_cu : 1.1) + (per_cu > 2 ? per_cu - 2 : 0) * 1.4 +
-                          (splits > 1 ? 7.5 + tiles * splits * 0.0066 : 0);
-        if (us >= best_us) continue;
-        best_us = us;
-        best.kind = Small16::kAny, best.splits = splits, best.workspace = splits > 1 ? tiles * splits * 4096 : 0;
     }
     return best;
 }
