@@ -183,6 +183,47 @@ def front():
     return _front
 
 
+def extension():
+    """The extension module itself, for the objects that layers make of its classes."""
+    front()
+    from . import _front as module
+    return module
+
+
+_callbacks = {}
+
+
+def callback(fn):
+    """``fn``, a function of a module, as native code calls it."""
+    made = _callbacks.get(fn)
+    if made is None:
+        made = _callbacks[fn] = extension().Callback(fn)
+    return made
+
+
+def buffers_moved():
+    """Some pooled buffer has been reallocated: native launches on the old ones are not used any more."""
+    module = sys.modules.get(__package__ + "._front")
+    if module is not None:
+        module.buffers_moved()
+
+
+def buffers_epoch():
+    return extension().buffers_epoch()
+
+
+class Own:
+    """A place for native objects that a layer makes when it first needs them; a copy of the layer makes its own."""
+
+    __slots__ = ("value",)
+
+    def __init__(self):
+        self.value = None
+
+    def __reduce__(self):
+        return Own, ()
+
+
 def check(rc, what):
     if rc != 0:
         msg = load().ddl_last_error().decode("utf-8", "replace")

@@ -11,6 +11,7 @@ dtype so that layers sharing a manager share memory.
 import numpy as np
 import torch
 
+from ... import _lib
 from . import device as _device
 
 
@@ -43,6 +44,7 @@ class ExpandableBuffer:
         self.raw_buffer = grown
         self.capacity = new_capacity
         self.views = {shape: self._carve(shape) for shape in self.views}
+        _lib.buffers_moved()       # last: who has seen the old views has seen the old count, too
 
     def _carve(self, view_shape):
         volume = int(np.prod(view_shape, dtype=np.int64))

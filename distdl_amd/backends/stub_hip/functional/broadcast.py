@@ -5,12 +5,13 @@ transport (identity for a solo rank that owns the data; copies between rank
 threads, summed with the box kernel, under loopback) so that layers storing
 weights on a sub-grid work end to end, gradients included."""
 
-__all__ = ["BroadcastFunction", "route_of"]
+__all__ = ["BroadcastFunction", "route_of", "stays"]
 
 import torch
 
 from .... import hip_ops
 from ....utilities.torch import zero_volume_tensor
+from ..transport import SoloTransport
 
 
 def route_of(P_send, P_recv, kind):
@@ -20,6 +21,12 @@ def route_of(P_send, P_recv, kind):
     if route is None or route.kind != kind:
         raise ValueError(f"P_send / P_recv were not made by this backend's create_{kind}_partition_to")
     return route
+
+
+def stays(P_send, P_recv):
+    """Whether a broadcast or a reduction between these leaves the tensor where it is, and its gradient too: the live rank of a
+    solo transport, in both partitions."""
+    return P_send.active and P_recv.active and type(P_send._world.transport) is SoloTransport
 
 
 class BroadcastFunction(torch.autograd.Function):

@@ -12,8 +12,9 @@ adjoint walks the dimensions backwards: move the ghosts out (pack and clear, one
 launch), swap, ADD what arrives into the bulk.
 """
 
-__all__ = ["HaloExchangeFunction"]
+__all__ = ["HaloExchangeFunction", "native_exchange"]
 
+import functools
 import math
 import operator
 
@@ -24,6 +25,7 @@ from .... import hip_ops
 from ....utilities.slicing import compute_nd_slice_shape
 from ....utilities.torch import zero_volume_tensor
 from ..partition import PROC_NULL
+from ..transport import SoloTransport
 
 _LTAG = 0
 _RTAG = 1
@@ -183,6 +185,22 @@ def _views(buffers, plan, tensor, bases):
     return out
 
 
+def _before(plan, i, bases):
+    """The launches ahead of the messages of dimension ``i``: the ghosts of the one before are unpacked, this one's strips
+    packed.  One launch for both, unless a strip goes into a buffer that still holds a ghost."""
+    if i == len(plan.dims):
+        return [plan.dims[-1][2]] if plan.dims else []
+    _, pack, _, both = plan.dims[i]
+    if i == 0:
+        return [pack]
+    return [both] if both is not None and not _share(bases, i) else [plan.dims[i - 1][2], pack]
+
+
+def _in_order(plan, bases):
+    """All launches of a forward exchange that sends no messages."""
+    return [plan.first] + [launch for i in range(len(plan.dims) + 1) for launch in _before(plan, i, bases)]
+
+
 def _share(bases, i):
     """Is one of dimension ``i``'s bulk buffers a ghost buffer of dimension ``i - 1``?"""
     ghosts = {bases[4 * i - 2 + _LEFT_GHOST], bases[4 * i - 2 + _RIGHT_GHOST]} - {0}
@@ -204,6 +222,60 @@ def _swap(P_x, neighbor_ranks_i, out_left, out_right, in_left, in_right):
         sends.append((rrank, out_right, _RTAG))
     if sends or recvs:
         P_x._world.transport.exchange(P_x, sends, recvs)
+
+
+def _adjoint(P_x, slices, buffers, neighbor_ranks, grad_output):
+    """In place on the incoming gradient, as the reference (:98)."""
+    if not grad_output.is_contiguous():
+        raise ValueError("HaloExchange adjoint needs a contiguous gradient")
+
+    hip_ops._require_gpu(grad_output)
+    plan = _plan(P_x.dim, slices, buffers, grad_output, False)
+    bases = [0, grad_output.data_ptr()]
+    views = _views(buffers, plan, grad_output, bases)
+    add_dtype = hip_ops._ADD_DTYPES.get(grad_output.dtype)
+    if add_dtype is None and plan.adds:
+        raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
+    for i in reversed(range(len(views))):
+        lbb, lgb, rbb, rgb = views[i]
+        _, out, clear, adds = plan.dims[i]
+        out.run(bases, op=_lib.DDL_OP_COPY if clear else _lib.DDL_OP_MOVE)
+        if clear:
+            clear.zero(grad_output)
+        _swap(P_x, neighbor_ranks[i], lgb, rgb, lbb, rbb)
+        for launch in adds:
+            launch.run(bases, op=_lib.DDL_OP_ADD, dtype=add_dtype)
+    return grad_output
+
+
+def native_exchange(input, P_x, slices, buffers, neighbor_ranks):
+    """Forward and, if it requires gradients, adjoint for tensors like ``input`` as native moves, where no message is sent
+    between their launches (the live rank of a solo transport).  None otherwise, and where the general way raises or clears
+    ghosts in a launch of its own."""
+    if not P_x.active or P_x.size == 1 or type(P_x._world.transport) is not SoloTransport or not input.is_cuda:
+        return None
+    epoch, bases = _lib.buffers_epoch(), [0, 0]
+    adjoint = None
+    try:
+        plan = _plan(P_x.dim, slices, buffers, input, True)
+        views = [v for sides in _views(buffers, plan, input, bases) for v in sides]
+        if input.requires_grad:
+            like = torch.empty(input.shape, dtype=input.dtype, device="meta")       # contiguous, as the result and its gradient are
+            adjoint = _plan(P_x.dim, slices, buffers, like, False)
+    except (RuntimeError, ValueError):
+        return None
+    forward = hip_ops.native_moves(epoch, input, tuple(input.shape),
+                                   [(launch, _lib.DDL_OP_COPY, _lib.DDL_DT_BITS) for launch in _in_order(plan, bases)], views)
+    if adjoint is None:
+        return forward, None
+    add_dtype = hip_ops._ADD_DTYPES.get(input.dtype)
+    if add_dtype is None or any(clear for _, _, clear, _ in adjoint.dims):
+        return None
+    back = []
+    for _, out, _, adds in reversed(adjoint.dims):
+        back += [(out, _lib.DDL_OP_MOVE, _lib.DDL_DT_BITS)] + [(launch, _lib.DDL_OP_ADD, add_dtype) for launch in adds]
+    return forward, hip_ops.native_moves(epoch, like, None, back, views,
+                                         general=functools.partial(_adjoint, P_x, slices, buffers, neighbor_ranks))
 
 
 class HaloExchangeFunction(torch.autograd.Function):
@@ -231,20 +303,12 @@ class HaloExchangeFunction(torch.autograd.Function):
         bases = [src.data_ptr(), output.data_ptr()]
         views = _views(buffers, plan, output, bases)
         plan.first.run(bases)
-        pending = None          # ghosts that have arrived and are not unpacked yet
         for i, (lbb, lgb, rbb, rgb) in enumerate(views):
-            _, pack, unpack, both = plan.dims[i]
-            # One launch for both, unless a strip goes into a buffer that still holds a ghost.
-            if pending is not None and both is not None and not _share(bases, i):
-                both.run(bases)
-            else:
-                if pending is not None:
-                    pending.run(bases)
-                pack.run(bases)
+            for launch in _before(plan, i, bases):
+                launch.run(bases)
             _swap(P_x, neighbor_ranks[i], lbb, rbb, lgb, rgb)
-            pending = unpack
-        if pending is not None:
-            pending.run(bases)
+        for launch in _before(plan, len(views), bases):
+            launch.run(bases)
         return output
 
     @staticmethod
@@ -255,25 +319,6 @@ class HaloExchangeFunction(torch.autograd.Function):
         if P_x.size == 1:
             return grad_output, None, None, None, None
 
-        # In place on the incoming gradient, as the reference (:98).
         ctx.mark_dirty(grad_output)
-        if not grad_output.is_contiguous():
-            raise ValueError("HaloExchange adjoint needs a contiguous gradient")
-
-        hip_ops._require_gpu(grad_output)
-        plan = _plan(P_x.dim, slices, buffers, grad_output, False)
-        bases = [0, grad_output.data_ptr()]
-        views = _views(buffers, plan, grad_output, bases)
-        add_dtype = hip_ops._ADD_DTYPES.get(grad_output.dtype)
-        if add_dtype is None and plan.adds:
-            raise ValueError(f"accumulating unpack is not available for {grad_output.dtype}")
-        for i in reversed(range(len(views))):
-            lbb, lgb, rbb, rgb = views[i]
-            _, out, clear, adds = plan.dims[i]
-            out.run(bases, op=_lib.DDL_OP_COPY if clear else _lib.DDL_OP_MOVE)
-            if clear:
-                clear.zero(grad_output)
-            _swap(P_x, ctx.neighbor_ranks[i], lgb, rgb, lbb, rbb)
-            for launch in adds:
-                launch.run(bases, op=_lib.DDL_OP_ADD, dtype=add_dtype)
+        _adjoint(P_x, slices, buffers, ctx.neighbor_ranks, grad_output)
         return grad_output, None, None, None, None

@@ -13,14 +13,18 @@ is not zero-filled first when the incoming boxes tile it completely (they
 always do for a valid pair of partitions).
 """
 
-__all__ = ["RepartitionFunction"]
+__all__ = ["RepartitionFunction", "native_repartition"]
+
+import functools
 
 import numpy as np
 import torch
 
+from .... import _lib
 from .... import hip_ops
 from ....utilities.torch import zero_volume_tensor
 from .. import buffer as _buffer
+from ..transport import SoloTransport
 
 _FWD_TAG = 111
 _ADJ_TAG = 113
@@ -190,6 +194,43 @@ def _move(src, P_union, dtype, P_src, src_overlaps, src_buffers, P_dst, dst_over
     return out
 
 
+def _adjoint(P_union, dtype, P_y, P_y_to_x_overlaps, P_y_to_x_buffers, P_x, P_x_to_y_overlaps, P_x_to_y_buffers, x_shape, preserve_batch,
+             grad_output):
+    """The same movement with the two overlap lists exchanged; the boxes are disjoint, so it copies and never adds
+    (reference :344-346)."""
+    return _move(grad_output.detach(), P_union, dtype, P_y, P_y_to_x_overlaps, P_y_to_x_buffers, P_x, P_x_to_y_overlaps, P_x_to_y_buffers,
+                 x_shape, preserve_batch, _ADJ_TAG)
+
+
+def native_repartition(input, P_union, x_global_structure, x_local_structure, y_local_structure, P_x, P_x_to_y_overlaps, P_x_to_y_buffers,
+                       P_y, P_y_to_x_overlaps, P_y_to_x_buffers, preserve_batch):
+    """Forward and, if it requires gradients, adjoint for tensors like ``input`` as native moves, where no message is sent
+    between their launches: the live rank of a solo transport that is in both partitions.  None otherwise."""
+    dtype = x_global_structure.dtype
+    if not (P_union.active and P_x.active and P_y.active and type(P_union._world.transport) is SoloTransport and input.is_cuda) or \
+       input.dtype != dtype:
+        return None
+    x_shape, y_shape = tuple(int(n) for n in x_local_structure.shape), tuple(int(n) for n in y_local_structure.shape)
+    if tuple(input.shape) != x_shape:
+        return None
+    general = functools.partial(_adjoint, P_union, dtype, P_y, P_y_to_x_overlaps, P_y_to_x_buffers, P_x, P_x_to_y_overlaps, P_x_to_y_buffers,
+                                x_local_structure.shape, preserve_batch)
+    out, epoch = [None, None], _lib.buffers_epoch()
+    directions = [(input, y_shape, None, (P_x, P_x_to_y_overlaps, P_x_to_y_buffers, P_y, P_y_to_x_overlaps, P_y_to_x_buffers))]
+    if input.requires_grad:
+        directions.append((torch.empty(y_shape, dtype=dtype, device="meta"), x_shape, general,
+                           (P_y, P_y_to_x_overlaps, P_y_to_x_buffers, P_x, P_x_to_y_overlaps, P_x_to_y_buffers)))
+    for i, (src, shape, back, args) in enumerate(directions):
+        plan = _move_plan(src, dtype, *args, shape)
+        views = plan.send_views + plan.recv_views
+        if plan.zero_fill or any(v is not None and not v.is_cuda for v in views):
+            return None
+        # slot 2 is address 0: the plan's boxes name their buffers by address, and the buffers stay with the object
+        out[i] = hip_ops.native_moves(epoch, src, shape, [(plan.first, _lib.DDL_OP_COPY, _lib.DDL_DT_BITS),
+                                                          (plan.second, _lib.DDL_OP_COPY, _lib.DDL_DT_BITS)], [None] + views, general=back)
+    return out
+
+
 class RepartitionFunction(torch.autograd.Function):
 
     @staticmethod
@@ -223,10 +264,8 @@ class RepartitionFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        """Adjoint: the same movement with the two overlap lists exchanged; the
-        boxes are disjoint, so it copies and never adds (reference :344-346)."""
-        grad_input = _move(grad_output.detach(), ctx.P_union, ctx.x_global_structure.dtype,
-                           ctx.P_y, ctx.P_y_to_x_overlaps, ctx.P_y_to_x_buffers,
-                           ctx.P_x, ctx.P_x_to_y_overlaps, ctx.P_x_to_y_buffers,
-                           ctx.x_local_structure.shape if ctx.P_x.active else None, ctx.preserve_batch, _ADJ_TAG)
+        grad_input = _adjoint(ctx.P_union, ctx.x_global_structure.dtype,
+                              ctx.P_y, ctx.P_y_to_x_overlaps, ctx.P_y_to_x_buffers,
+                              ctx.P_x, ctx.P_x_to_y_overlaps, ctx.P_x_to_y_buffers,
+                              ctx.x_local_structure.shape if ctx.P_x.active else None, ctx.preserve_batch, grad_output)
         return grad_input, None, None, None, None, None, None, None, None, None, None, None

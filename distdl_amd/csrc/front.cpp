@@ -8,26 +8,9 @@
 // the callers in hip_ops.py then go their general way, which converts, copies or
 // raises.  A failing entry point raises RuntimeError as _lib.check does.  The
 // interpreter lock is released while a function runs.
-#include <c10/hip/HIPStream.h>
-#include <torch/extension.h>
+#include "front.h"
 
-#include <optional>
-#include <string>
-#include <tuple>
-#include <vector>
-
-#include "../../include/distdl_hip.h"
-
-namespace {
-
-using at::Tensor;
-typedef std::optional<Tensor> MaybeTensor;
-
-void check(int rc, const char* what) {
-    if (rc != 0) throw std::runtime_error(std::string(what) + " failed with code " + std::to_string(rc) + ": " + ddl_last_error());
-}
-
-void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+namespace ddl_front {
 
 int float_code(const Tensor& t) {   // 0: none of the three
     switch (t.scalar_type()) {
@@ -38,6 +21,8 @@ int float_code(const Tensor& t) {   // 0: none of the three
     }
 }
 
+namespace {
+
 int sum_code(const Tensor& t) {
     switch (t.scalar_type()) {
         case at::kDouble: return DDL_DT_F64;
@@ -47,23 +32,29 @@ int sum_code(const Tensor& t) {
     }
 }
 
-bool plain(const Tensor& t) { return t.is_cuda() && t.is_contiguous(); }
-bool multiple(const void* p, int64_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; }
-const void* pointer(const MaybeTensor& t) { return t ? t->data_ptr() : nullptr; }
-void* pointer(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 Tensor floats(const Tensor& like, at::IntArrayRef shape) { return at::empty(shape, like.options().dtype(at::kFloat)); }
 Tensor shaped(const Tensor& like, const std::optional<std::vector<int64_t>>& shape) { return shape ? at::empty(*shape, like.options()) : Tensor(); }
 int64_t clamped(int64_t n, int64_t most) { return n < 1 ? 1 : n > most ? most : n; }
 
+}  // namespace
+
 // ---------------------------------------------------------------- linear --
 
-MaybeTensor linear(const Tensor& x, const Tensor& w, const MaybeTensor& bias) {
+// Is `w` the [n, k] matrix of a product with `x`, in any number of dimensions of which the leading ones have one element?
+static bool weight_matrix(const Tensor& w, const Tensor& x) {
+    if (!w.is_cuda() || w.scalar_type() != x.scalar_type() || w.dim() < 2) return false;
+    for (int64_t d = 0; d < w.dim() - 2; ++d)
+        if (w.size(d) != 1) return false;
+    return w.size(-2) > 0 && w.size(-1) > 0 && (w.size(-1) == 1 || w.stride(-1) == 1);
+}
+
+MaybeTensor product(const Tensor& x, const Tensor& w, const MaybeTensor& bias) {
     const int dt = float_code(x);
-    if (!dt || !plain(x) || !w.is_cuda() || w.scalar_type() != x.scalar_type() || w.dim() != 2 || x.dim() < 1 || x.numel() == 0) return std::nullopt;
-    const int64_t n = w.size(0), k = w.size(1);
-    if (n == 0 || k == 0 || x.size(-1) != k || (k > 1 && w.stride(1) != 1)) return std::nullopt;
+    if (!dt || !plain(x) || !weight_matrix(w, x) || x.dim() < 1 || x.numel() == 0) return std::nullopt;
+    const int64_t n = w.size(-2), k = w.size(-1);
+    if (x.size(-1) != k) return std::nullopt;
     if (bias && (!plain(*bias) || bias->scalar_type() != x.scalar_type() || bias->numel() != n)) return std::nullopt;
-    const int64_t m = x.numel() / k, ldw = n > 1 ? w.stride(0) : k;
+    const int64_t m = x.numel() / k, ldw = n > 1 ? w.stride(-2) : k;
     const void *px = x.data_ptr(), *pw = w.data_ptr();
     const bool aligned = multiple(px, 16) && multiple(pw, 16);
     if (dt != DDL_DT_F32 && !(k % 8 == 0 && aligned && (n <= 1 || ldw % 8 == 0)) && !ddl_gemm_in_place(dt, aligned, k, 1, ldw, 1, m, n, k))
@@ -78,14 +69,14 @@ MaybeTensor linear(const Tensor& x, const Tensor& w, const MaybeTensor& bias) {
     return y;
 }
 
-std::optional<std::tuple<Tensor, Tensor, Tensor>> linear_backward(const Tensor& x, const Tensor& w, const Tensor& dy, bool need_x, bool need_w,
-                                                                  bool need_b) {
+std::optional<std::tuple<Tensor, Tensor, Tensor>> product_backward(const Tensor& x, const Tensor& w, const Tensor& dy, bool need_x, bool need_w,
+                                                                  const MaybeShape& bias_shape) {
     const int dt = float_code(x);
-    if (!dt || !plain(x) || !plain(dy) || !w.is_cuda() || w.scalar_type() != x.scalar_type() || dy.scalar_type() != x.scalar_type() || w.dim() != 2)
-        return std::nullopt;
-    const int64_t n = w.size(0), k = w.size(1);
-    if (n == 0 || k == 0 || x.numel() == 0 || (k > 1 && w.stride(1) != 1) || x.numel() % k != 0) return std::nullopt;
-    const int64_t m = x.numel() / k, ldw = n > 1 ? w.stride(0) : k;
+    if (!dt || !plain(x) || !plain(dy) || !weight_matrix(w, x) || dy.scalar_type() != x.scalar_type()) return std::nullopt;
+    const int64_t n = w.size(-2), k = w.size(-1);
+    const bool need_b = bias_shape.has_value();
+    if (x.numel() == 0 || x.numel() % k != 0) return std::nullopt;
+    const int64_t m = x.numel() / k, ldw = n > 1 ? w.stride(-2) : k;
     if (dy.numel() != m * n) return std::nullopt;
     const void *px = x.data_ptr(), *pw = w.data_ptr(), *pdy = dy.data_ptr();
     if (dt != DDL_DT_F32) {   // the conditions of hip_ops.linear_backward for reading every operand where it lies
@@ -100,8 +91,8 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> linear_backward(const Tensor& 
     }
     Tensor dx, dw, db, work;
     if (need_x) dx = at::empty(x.sizes(), x.options());
-    if (need_w) dw = at::empty({n, k}, x.options());
-    if (need_b) db = at::empty({n}, x.options());
+    if (need_w) dw = at::empty(w.sizes(), x.options());
+    if (need_b) db = at::empty(*bias_shape, x.options());
     const bool aligned = multiple(px, 16) && multiple(pw, 16) && multiple(pdy, 16);
     const int64_t elems = ddl_linear_backward_workspace_at(dt, aligned, m, n, k, k, ldw, n, need_x, need_w, need_b);
     if (elems) work = floats(x, {elems});
@@ -113,8 +104,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> linear_backward(const Tensor& 
 
 // ------------------------------------------------------------ layer norm --
 
-// y, the rows as [rows, cols], mean, rstd, gamma as [cols]
-typedef std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> Normalized;
+namespace {
 
 bool ln_operands(const Tensor& x, const MaybeTensor& gamma, const MaybeTensor& beta, int64_t cols) {
     if (!float_code(x) || !plain(x) || cols < 1 || x.numel() == 0 || x.numel() % cols != 0 || gamma.has_value() != beta.has_value()) return false;
@@ -122,6 +112,8 @@ bool ln_operands(const Tensor& x, const MaybeTensor& gamma, const MaybeTensor& b
     return plain(*gamma) && plain(*beta) && gamma->scalar_type() == x.scalar_type() && beta->scalar_type() == x.scalar_type() &&
            gamma->numel() == cols && beta->numel() == cols;
 }
+
+}  // namespace
 
 std::optional<Normalized> layer_norm(const Tensor& x, const MaybeTensor& gamma, const MaybeTensor& beta, int64_t cols, double eps) {
     if (!ln_operands(x, gamma, beta, cols)) return std::nullopt;
@@ -133,13 +125,15 @@ std::optional<Normalized> layer_norm(const Tensor& x, const MaybeTensor& gamma, 
     return Normalized(y, x.detach().view({rows, cols}), mean, rstd, gamma ? gamma->detach().view({cols}) : Tensor());
 }
 
-typedef std::optional<std::vector<int64_t>> MaybeShape;   // of a parameter's gradient, if that is wanted
+namespace {
 
 bool ln_backward_operands(const Tensor& dy, const Tensor& x2d, const Tensor& mean, const Tensor& rstd, const MaybeTensor& gamma) {
     return float_code(x2d) && plain(dy) && plain(x2d) && plain(mean) && plain(rstd) && x2d.dim() == 2 && x2d.numel() > 0 &&
            dy.scalar_type() == x2d.scalar_type() && dy.numel() == x2d.numel() &&
            (!gamma || (plain(*gamma) && gamma->scalar_type() == x2d.scalar_type() && gamma->numel() == x2d.size(1)));
 }
+
+}  // namespace
 
 // Rows this worker holds whole: dx and the parameters' gradients in one pass.  dy may have any shape of as many elements.
 std::optional<std::tuple<Tensor, Tensor, Tensor>> ln_backward_whole(const Tensor& dy, const Tensor& x2d, const Tensor& mean, const Tensor& rstd,
@@ -196,7 +190,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> ln_backward_input_params(const
 
 // ------------------------------------------------------------- embedding --
 
-bool id_tensor(const Tensor& ids) { return plain(ids) && (ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt); }
+static bool id_tensor(const Tensor& ids) { return plain(ids) && (ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt); }
 
 MaybeTensor embedding_gather(const Tensor& weight, const Tensor& ids, int64_t lo, int64_t hi) {
     if (!plain(weight) || weight.dim() != 2 || weight.size(0) != hi - lo || !id_tensor(ids)) return std::nullopt;
@@ -225,41 +219,29 @@ MaybeTensor embedding_backward(const Tensor& dy, const Tensor& ids, int64_t lo, 
 
 // ----------------------------------------------------------------- boxes --
 
-// The boxes of one launch with everything but the base addresses: a call adds those
-// of the slots.  Calls only read the object.
-class Boxes {
-public:
-    typedef std::tuple<size_t, int64_t, size_t, int64_t> Place;   // source slot and byte offset, destination slot and byte offset
-    // descriptors: ddl_box_t after ddl_box_t, without the pointers.
-    Boxes(const std::string& descriptors, const std::vector<Place>& places, int elem_size) : places_(places), elem_size_(elem_size) {
-        if (descriptors.size() != places.size() * sizeof(ddl_box_t)) throw std::invalid_argument("Boxes: descriptors and places disagree");
-        boxes_.resize(places.size());
-        if (!places.empty()) memcpy(boxes_.data(), descriptors.data(), descriptors.size());
-        for (const Place& p : places) {
-            if (std::get<0>(p) >= bases_) bases_ = std::get<0>(p) + 1;
-            if (std::get<2>(p) >= bases_) bases_ = std::get<2>(p) + 1;
-        }
+Boxes::Boxes(const std::string& descriptors, const std::vector<Place>& places, int elem_size) : places_(places), elem_size_(elem_size) {
+    if (descriptors.size() != places.size() * sizeof(ddl_box_t)) throw std::invalid_argument("Boxes: descriptors and places disagree");
+    boxes_.resize(places.size());
+    if (!places.empty()) memcpy(boxes_.data(), descriptors.data(), descriptors.size());
+    for (const Place& p : places) {
+        if (std::get<0>(p) >= bases_) bases_ = std::get<0>(p) + 1;
+        if (std::get<2>(p) >= bases_) bases_ = std::get<2>(p) + 1;
     }
-    void run(const std::vector<int64_t>& bases, int op, int dtype) const {
-        if (boxes_.empty()) return;
-        if (bases.size() < bases_) throw std::invalid_argument("Boxes: too few base addresses");
-        std::vector<ddl_box_t> boxes(boxes_);
-        for (size_t i = 0; i < boxes.size(); ++i) {
-            boxes[i].src = reinterpret_cast<const void*>(bases[std::get<0>(places_[i])] + std::get<1>(places_[i]));
-            boxes[i].dst = reinterpret_cast<void*>(bases[std::get<2>(places_[i])] + std::get<3>(places_[i]));
-        }
-        check(ddl_copy_boxes(boxes.data(), static_cast<int>(boxes.size()), elem_size_, op, dtype, current_stream()), "ddl_copy_boxes");
-    }
+}
 
-private:
-    std::vector<ddl_box_t> boxes_;
-    std::vector<Place> places_;
-    size_t bases_ = 0;
-    int elem_size_;
-};
+void Boxes::run(const std::vector<int64_t>& bases, int op, int dtype) const {
+    if (boxes_.empty()) return;
+    if (bases.size() < bases_) throw std::invalid_argument("Boxes: too few base addresses");
+    std::vector<ddl_box_t> boxes(boxes_);
+    for (size_t i = 0; i < boxes.size(); ++i) {
+        boxes[i].src = reinterpret_cast<const void*>(bases[std::get<0>(places_[i])] + std::get<1>(places_[i]));
+        boxes[i].dst = reinterpret_cast<void*>(bases[std::get<2>(places_[i])] + std::get<3>(places_[i]));
+    }
+    check(ddl_copy_boxes(boxes.data(), static_cast<int>(boxes.size()), elem_size_, op, dtype, current_stream()), "ddl_copy_boxes");
+}
 
 // The sum over the sources, in order, of elements [start, start + extent) along `axis`, each divided first.
-MaybeTensor sum_slab(const std::vector<Tensor>& srcs, int64_t axis, int64_t start, int64_t extent, double divisor) {
+static MaybeTensor sum_slab(const std::vector<Tensor>& srcs, int64_t axis, int64_t start, int64_t extent, double divisor) {
     if (srcs.empty() || srcs.size() > 64) return std::nullopt;
     const Tensor& first = srcs[0];
     const int dt = sum_code(first), nd = static_cast<int>(first.dim());
@@ -288,7 +270,7 @@ MaybeTensor sum_slab(const std::vector<Tensor>& srcs, int64_t axis, int64_t star
 }
 
 // The pieces joined along `axis`.
-MaybeTensor join(const Tensor& local, const std::vector<Tensor>& parts, int64_t axis) {
+static MaybeTensor join(const Tensor& local, const std::vector<Tensor>& parts, int64_t axis) {
     const int nd = static_cast<int>(local.dim());
     if (parts.empty() || nd < 1 || nd > DDL_MAX_DIMS || axis < 0 || axis >= nd || !local.is_cuda()) return std::nullopt;
     auto shape = local.sizes().vec();
@@ -321,13 +303,20 @@ MaybeTensor join(const Tensor& local, const std::vector<Tensor>& parts, int64_t 
     return out;
 }
 
-}  // namespace
+}  // namespace ddl_front
 
 PYBIND11_MODULE(_front, m) {
     namespace py = pybind11;
+    using namespace ddl_front;
     typedef py::call_guard<py::gil_scoped_release> unlocked;
-    m.def("linear", &linear, unlocked());
-    m.def("linear_backward", &linear_backward, unlocked());
+    // as hip_ops has them: the weight as a matrix, its bias as a vector
+    m.def("linear", [](const Tensor& x, const Tensor& w, const MaybeTensor& bias) { return w.dim() == 2 ? product(x, w, bias) : std::nullopt; }, unlocked());
+    m.def("linear_backward",
+          [](const Tensor& x, const Tensor& w, const Tensor& dy, bool need_x, bool need_w, bool need_b) -> std::optional<std::tuple<Tensor, Tensor, Tensor>> {
+              if (w.dim() != 2) return std::nullopt;
+              return product_backward(x, w, dy, need_x, need_w, need_b ? MaybeShape(std::vector<int64_t>{w.size(0)}) : std::nullopt);
+          },
+          unlocked());
     m.def("layer_norm", &layer_norm, unlocked());
     m.def("ln_backward_whole", &ln_backward_whole, unlocked());
     m.def("ln_backward_partial_params", &ln_backward_partial_params, unlocked());
@@ -336,9 +325,10 @@ PYBIND11_MODULE(_front, m) {
     m.def("embedding_backward", &embedding_backward, unlocked());
     m.def("sum_slab", &sum_slab, unlocked());
     m.def("join", &join, unlocked());
-    py::class_<Boxes>(m, "Boxes")
+    py::class_<Boxes, std::shared_ptr<Boxes>>(m, "Boxes")
         .def(py::init([](const py::bytes& descriptors, const std::vector<Boxes::Place>& places, int elem_size) {
             return new Boxes(static_cast<std::string>(descriptors), places, elem_size);
         }))
         .def("run", &Boxes::run, unlocked());
+    define_nodes(m);
 }

@@ -189,13 +189,27 @@ class BoxLaunch:
     def __getstate__(self):
         return {**self.__dict__, "_boxes": None}      # a copy makes its own
 
-    def run(self, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
-        if self.n == 0:
-            return
+    def native(self):
         boxes = self._boxes
         if boxes is None:
             boxes = self._boxes = _lib.front().Boxes(self._template, self._bases, self.elem_size)
-        boxes.run(bases, op, dtype)
+        return boxes
+
+    def run(self, bases, op=_lib.DDL_OP_COPY, dtype=_lib.DDL_DT_BITS):
+        if self.n:
+            self.native().run(bases, op, dtype)
+
+
+def native_moves(epoch, src, out_shape, launches, buffers=(), staging=None, general=None):
+    """The launches of one direction of a data movement as one native object (``Moves`` of csrc/front_nodes.cpp): for tensors of
+    the shape, strides and type of ``src``, into a new tensor of ``out_shape`` (None: in place).  ``launches`` are ``(BoxLaunch,
+    operation, element type)``, their slots 0 the tensor, 1 the result (in place: 1 the tensor), 2 and on ``buffers``;
+    ``general`` is the way through Python for any other tensor; ``epoch`` is ``_lib.buffers_epoch()`` from before the buffers
+    were looked at."""
+    extension = _lib.extension()
+    steps = [(launch.native(), op, dtype) for launch, op, dtype in launches if launch.n]
+    return extension.Moves(list(src.shape), list(src.stride()), src.dtype, None if out_shape is None else list(out_shape), steps,
+                           list(buffers), staging, None if general is None else extension.Callback(general), epoch)
 
 
 def copy_box(src, src_slices, dst, dst_slices, accumulate=False):
@@ -354,6 +368,48 @@ class HaloPadPlan:
                 shape.append(self.padded_shape[j] - self.recv[j][0] - self.recv[j][1])
         return tuple(shape)
 
+    def _checked_slabs(self, dtype, ghost_bufs, bulk_bufs):
+        """The ghost and the bulk slabs in the order of the entry point's pointers, None where there is none."""
+        out = []
+        for kind, bufs in (("ghost", ghost_bufs), ("bulk", bulk_bufs)):
+            slabs = [None] * (2 * self.ndim)
+            out.append(slabs)
+            if bufs is None:
+                continue
+            for place, d, s, shape in self._slabs[kind]:
+                buf = bufs[d][s]
+                if buf is None:
+                    continue
+                _require_gpu(buf)
+                if buf.shape != shape or not buf.is_contiguous() or buf.dtype != dtype:
+                    raise ValueError(f"halo_pad_exchange: {kind} slab ({d},{s}) must be contiguous {shape}, "
+                                     f"got {tuple(buf.shape)}")
+                slabs[place] = buf
+        return out
+
+    def moves(self, epoch, x, ghost_bufs, bulk_bufs):
+        """``run`` for tensors like ``x`` and, if it requires gradients, ``crop`` for those of the result, as native moves."""
+        staging = ([v for p in self.pad for v in p], [v for p in self.recv for v in p], [v for p in self.send for v in p],
+                   *self._checked_slabs(x.dtype, ghost_bufs, bulk_bufs))
+        forward = native_moves(epoch, x, self.padded_shape, [], staging=staging)
+        if not x.requires_grad:
+            return forward, None
+        padded = torch.empty(self.padded_shape, dtype=x.dtype, device="meta")
+        crop = self._crop_launch(x.element_size())
+        return forward, native_moves(epoch, padded, self.x_shape, [(crop, _lib.DDL_OP_COPY, _lib.DDL_DT_BITS)], general=self._general_crop)
+
+    def _general_crop(self, padded):
+        return self.crop(padded.detach())
+
+    def _crop_launch(self, elem_size):
+        launch = self._crops.get(elem_size)
+        if launch is None:
+            strides = contiguous_strides(self.padded_shape)
+            launch = self._crops[elem_size] = BoxLaunch(
+                [(0, sum(p[0] * st for p, st in zip(self.pad, strides)), 1, 0, self.x_shape, strides, contiguous_strides(self.x_shape))],
+                elem_size)
+        return launch
+
     def run(self, x, ghost_bufs, bulk_bufs, out=None, kernel=_lib.DDL_HALO_AUTO):
         """ghost_bufs / bulk_bufs: ``[ndim][2]`` nested lists of tensors or None.
         ``kernel``: ``DDL_HALO_AUTO`` (library's choice), ``DDL_HALO_ROWS`` or
@@ -365,20 +421,8 @@ class HaloPadPlan:
             out = torch.empty(self.padded_shape, dtype=x.dtype, device=x.device)
         elif tuple(out.shape) != self.padded_shape or not out.is_contiguous() or out.dtype != x.dtype:
             raise ValueError("halo_pad_exchange: bad output tensor")
-        gptr, bptr = [None] * (2 * self.ndim), [None] * (2 * self.ndim)
-        dtype = x.dtype
-        for kind, bufs, ptrs in (("ghost", ghost_bufs, gptr), ("bulk", bulk_bufs, bptr)):
-            if bufs is None:
-                continue
-            for place, d, s, shape in self._slabs[kind]:
-                buf = bufs[d][s]
-                if buf is None:
-                    continue
-                _require_gpu(buf)
-                if buf.shape != shape or not buf.is_contiguous() or buf.dtype != dtype:
-                    raise ValueError(f"halo_pad_exchange: {kind} slab ({d},{s}) must be contiguous {shape}, "
-                                     f"got {tuple(buf.shape)}")
-                ptrs[place] = buf.data_ptr()
+        ghosts, bulk = self._checked_slabs(x.dtype, ghost_bufs, bulk_bufs)
+        gptr, bptr = [_ptr(t) for t in ghosts], [_ptr(t) for t in bulk]
         rc = _lib.load().ddl_halo_pad_exchange(x.data_ptr(), out.data_ptr(), self.shape_arr, self.ndim,
                                                x.element_size(), self.pad_arr, self.recv_arr, self.send_arr,
                                                _lib.ptr_array(gptr), _lib.ptr_array(bptr), int(kernel), _stream())
@@ -390,12 +434,7 @@ class HaloPadPlan:
         out = torch.empty(self.x_shape, dtype=padded.dtype, device=padded.device)
         if padded.shape == self.padded_shape and padded.is_contiguous():
             _require_gpu(padded)
-            launch = self._crops.get(padded.element_size())
-            if launch is None:
-                strides = contiguous_strides(self.padded_shape)
-                launch = self._crops[padded.element_size()] = BoxLaunch(
-                    [(0, sum(p[0] * st for p, st in zip(self.pad, strides)), 1, 0, self.x_shape, strides, contiguous_strides(self.x_shape))],
-                    padded.element_size())
+            launch = self._crop_launch(padded.element_size())
             launch.run([padded.data_ptr(), out.data_ptr()])
             return out
         inner = [slice(p[0], p[0] + n) for p, n in zip(self.pad, self.x_shape)]

@@ -1,6 +1,7 @@
 """Broadcast layer stand-in (reference: nn/broadcast.py).  The collective itself
 is outside this build; see backends/stub_hip/functional/broadcast.py."""
 
+from .. import _lib
 from ..utilities.torch import TensorStructure
 from .module import Module
 
@@ -25,7 +26,12 @@ class Broadcast(Module):
     def forward(self, input):
         if self.identity or not (self.P_x.active or self.P_y.active):
             return input
-        Function = self._distdl_backend.functional.broadcast.BroadcastFunction
+        functional = self._distdl_backend.functional.broadcast
+        if self.scale_backward is None and functional.stays(self.P_send, self.P_recv):
+            out = _lib.front().alias(input)
+            if out is not None:
+                return out
+        Function = functional.BroadcastFunction
         # Positional arguments as in the reference (nn/broadcast.py:215-221).
         return Function.apply(input, self.P_send, self.P_recv, self.preserve_batch, TensorStructure(input), None,
                               self.scale_backward)

@@ -14,6 +14,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 
+from .. import _lib
 from .. import hip_ops
 from ..backends.stub_hip import buffer as _buffer
 from ..utilities.slicing import assemble_slices
@@ -146,6 +147,7 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         self.needed_slices = None
         self.halo_layer = None
         self._staging_plan = None
+        self._moves = _lib.Own()      # (what they are for, staging and its adjoint as native moves or None)
         self._distdl_is_setup = False
         self._input_tensor_structure = TensorStructure()
 
@@ -171,6 +173,7 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         self._input_tensor_structure = TensorStructure(input[0])
         if not self.P_x.active:
             return
+        self._moves.value = None
         backend = self._distdl_backend
         x_global_structure = backend.assemble_global_tensor_structure(input[0], self.P_x)
         x_global_shape_after_pad = np.asarray(x_global_structure.shape) + 2 * self.global_padding
@@ -189,6 +192,8 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         self.needed_slices = assemble_slices(needed_ranges[:, 0], needed_ranges[:, 1])
 
         total_padding = self.local_padding + self.halo_shape
+        self._nothing_to_stage = total_padding.sum() == 0 and self.P_x.size == 1
+        self._window = [(int(sl.start), int(sl.stop)) for sl in self.needed_slices]
         self._pad_only_plan = hip_ops.HaloPadPlan(input[0].shape, total_padding,
                                                   np.zeros_like(total_padding), np.zeros_like(total_padding))
         self._staging_plan = hip_ops.HaloPadPlan(input[0].shape, total_padding, recv_buffer_shape, send_buffer_shape)
@@ -226,22 +231,34 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
 
     def stage_input(self, input):
         """Padded, exchanged and cropped input of the local convolution."""
-        total_padding = self.local_padding + self.halo_shape
         transport = self.P_x._world.transport
-        if total_padding.sum() == 0 and self.P_x.size == 1:
+        if self._nothing_to_stage:
             return input
         if getattr(transport, "ghosts_preloaded", False):
-            ghost, bulk = self._fused_slabs(input)
-            exchanged = _HaloStaging.apply(input, self._staging_plan, ghost, bulk)
+            moves = self._moves.value
+            key = (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, _buffer.reallocations())
+            if moves is None or moves[0] != key:
+                moves = self._moves.value = self._native_staging(input)
+            exchanged = None if moves[1] is None else _lib.front().move(input, *moves[1])
+            if exchanged is None:
+                exchanged = _HaloStaging.apply(input, self._staging_plan, *self._fused_slabs(input))
         else:
             padded = _HaloStaging.apply(input, self._pad_only_plan, None, None)
             exchanged = self.halo_layer(padded)
-        crop = tuple(slice(int(sl.start), int(sl.stop)) for sl in self.needed_slices)
-        if all(sl.start == 0 and sl.stop == n for sl, n in zip(crop, exchanged.shape)):
+        if all(start == 0 and stop == n for (start, stop), n in zip(self._window, exchanged.shape)):
             return exchanged
+        crop = tuple(slice(start, stop) for start, stop in self._window)
         # A window smaller than the padded tensor (strided or unbalanced
         # geometries): handed to the convolution as a contiguous tensor.
         return _Crop.apply(exchanged, crop)
+
+    def _native_staging(self, input):
+        """(what they are for, staging and its adjoint as native moves or None)"""
+        self._fused_slabs(input)          # what is to be reallocated is so from here on
+        epoch, key = _lib.buffers_epoch(), (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, _buffer.reallocations())
+        if not input.is_cuda or not input.is_contiguous() or tuple(input.shape) != self._staging_plan.x_shape:
+            return key, None
+        return key, self._staging_plan.moves(epoch, input, *self._fused_slabs(input))
 
     def _fused_slabs(self, input):
         """Ghost and bulk slabs of the fused pass as ``[dim][side]`` tables of

@@ -9,6 +9,7 @@ extension for vocabulary-sharded tables: the local table then holds rows
 
 import torch
 
+from .. import _lib
 from .. import config
 from .. import hip_ops
 from ..utilities.slicing import compute_subshape
@@ -35,6 +36,11 @@ class _EmbeddingShard(torch.autograd.Function):
         lo, hi, padding_idx, scale_grad_by_freq = ctx.window
         dw = hip_ops.embedding_backward(grad_output, ids, lo, hi, padding_idx, scale_grad_by_freq)
         return dw, None, None, None, None, None
+
+
+def _general_backward(grad_output, ids, lo, hi, padding_idx, scale_grad_by_freq):
+    """The adjoint for what its native form does not take."""
+    return hip_ops.embedding_backward(grad_output, ids, lo, hi, padding_idx, scale_grad_by_freq)
 
 
 class DistributedEmbedding(Module):
@@ -155,5 +161,9 @@ class DistributedEmbedding(Module):
             # As F.embedding does: in place on the tensor that is looked up (every
             # worker scales its own columns by their own norm), outside autograd.
             hip_ops.embedding_renorm(weight.detach(), input, self.vocab_lo, self.vocab_hi, self.max_norm, self.norm_type)
+        out = _lib.front().embedding_shard(weight, input, self.vocab_lo, self.vocab_hi, self.padding_idx, bool(self.scale_grad_by_freq),
+                                           _lib.callback(_general_backward))
+        if out is not None:
+            return out
         return _EmbeddingShard.apply(weight, input, self.vocab_lo, self.vocab_hi, self.padding_idx,
                                      bool(self.scale_grad_by_freq))

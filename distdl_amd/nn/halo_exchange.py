@@ -2,6 +2,8 @@
 
 import numpy as np
 
+from .. import _lib
+from ..backends.stub_hip import buffer as _buffer
 from ..utilities.torch import TensorStructure
 from .module import Module
 
@@ -49,6 +51,7 @@ class HaloExchange(Module):
 
         self.slices = None
         self.buffers = None
+        self._moves = _lib.Own()      # (what they are for, forward and adjoint as native moves or None)
 
         if buffer_manager is None:
             buffer_manager = self._distdl_backend.BufferManager()
@@ -64,6 +67,7 @@ class HaloExchange(Module):
         return assemble_halo_slices(x_local_shape, recv_buffer_shape, send_buffer_shape)
 
     def _distdl_module_setup(self, input):
+        self._moves.value = None
         if self.P_x.active:
             SliceTable = self._distdl_backend.functional.halo_exchange.SliceTable
             self.slices = SliceTable(self._assemble_slices(input[0].shape, self.recv_buffer_shape,
@@ -87,7 +91,16 @@ class HaloExchange(Module):
         return self._input_tensor_structure != TensorStructure(input[0])
 
     def forward(self, input):
-        Function = self._distdl_backend.functional.halo_exchange.HaloExchangeFunction
         if not self.P_x.active:
             return input
-        return Function.apply(input, self.P_x, self.slices, self.buffers, self.neighbor_ranks)
+        functional = self._distdl_backend.functional.halo_exchange
+        args = (self.P_x, self.slices, self.buffers, self.neighbor_ranks)
+        key = (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, type(self.P_x._world.transport), _buffer.reallocations())
+        moves = self._moves.value
+        if moves is None or moves[0] != key:
+            moves = self._moves.value = (key, functional.native_exchange(input, *args))
+        if moves[1] is not None:
+            y = _lib.front().move(input, *moves[1])
+            if y is not None:
+                return y
+        return functional.HaloExchangeFunction.apply(input, *args)

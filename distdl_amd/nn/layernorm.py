@@ -12,6 +12,7 @@ Inputs may be float32, bfloat16 or float16, forward and backward; sums, means
 and reciprocal deviations are float32 and results are rounded once.
 """
 
+import functools
 import numbers
 
 import numpy as np
@@ -74,6 +75,51 @@ def _shard_forward(input, weight, bias, P_reduce, part_cols, eps, part_cols_arr,
     return y.view(input.shape), x2d, mean, rstd, gamma
 
 
+def _gather_sums(P_reduce, sums):
+    return P_reduce._world.transport.allgather(P_reduce, sums, tag=BWD_SUMS_TAG).contiguous()
+
+
+def _shard_backward(P_reduce, nparts, grad_output, x2d, mean, rstd, gamma, need_x, w_shape, b_shape):
+    """Adjoint of one shard: ``(dx, dw, db)``; the shapes of the parameters are None where no gradient of theirs is wanted."""
+    cols, want_w, want_b = x2d.shape[1], w_shape is not None, b_shape is not None
+    dy2d = grad_output.detach().reshape(-1, cols)
+    if dy2d.dtype != x2d.dtype:
+        dy2d = dy2d.to(x2d.dtype)
+    if dy2d.shape[1] > 1 and dy2d.stride(1) != 1:
+        dy2d = hip_ops.contiguous(dy2d)
+    dx = dw = db = None
+    fused = need_x and (want_w or want_b)        # two launches instead of four
+    if need_x and nparts == 1 and hip_ops.ln_backward_one_pass_supported(dy2d, x2d, gamma):
+        # rows held whole: this worker's sums are the row's sums, so dx comes out of the pass that forms them
+        dx, dw, db = hip_ops.ln_backward_one_pass(dy2d, x2d, mean, rstd, gamma, 1.0 / cols, want_gamma=want_w,
+                                                  want_beta=want_b)
+        dx = dx.view(grad_output.shape)
+    elif fused and nparts == 1 and hip_ops.ln_backward_whole_rows_supported(dy2d, x2d, gamma):
+        dx, dw, db = hip_ops.ln_backward_whole_rows(dy2d, x2d, mean, rstd, gamma, 1.0 / cols, want_w, want_b)
+        dx = dx.view(grad_output.shape)
+    elif need_x:
+        if fused:
+            sums, work = hip_ops.ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma)
+        else:
+            sums = hip_ops.ln_backward_partial(dy2d, x2d, mean, rstd, gamma)
+        if nparts > 1:
+            gathered = _gather_sums(P_reduce, sums)
+        else:
+            gathered = sums.unsqueeze(0)
+        weight_a = 1.0 / (nparts * cols)
+        if fused:
+            dx, dw, db = hip_ops.ln_backward_input_params(dy2d, x2d, mean, rstd, gamma, gathered, weight_a, work,
+                                                          want_w, want_b)
+        else:
+            dx = hip_ops.ln_backward_input(dy2d, x2d, mean, rstd, gamma, gathered, weight_a)
+        dx = dx.view(grad_output.shape)
+    elif want_w or want_b:
+        dw, db = hip_ops.ln_backward_params(dy2d, x2d, mean, rstd, want_w, want_b)
+    dw = None if dw is None else dw.view(w_shape)
+    db = None if db is None else db.view(b_shape)
+    return dx, dw, db
+
+
 class _LayerNormShard(torch.autograd.Function):
     """Local shard of a layer norm whose statistics span ``P_reduce``, and its
     adjoint: the gradient autograd derives from the reference's forward
@@ -93,48 +139,13 @@ class _LayerNormShard(torch.autograd.Function):
         x2d, mean, rstd, gamma = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad[:3]
         w_shape, b_shape = ctx.param_shapes
-        want_w, want_b = need_w and w_shape is not None, need_b and b_shape is not None
+        w_shape, b_shape = w_shape if need_w else None, b_shape if need_b else None
         if need_x and ctx.nparts == 1:
-            grads = _lib.front().ln_backward_whole(grad_output, x2d, mean, rstd, gamma, w_shape if want_w else None,
-                                                   b_shape if want_b else None)
+            grads = _lib.front().ln_backward_whole(grad_output, x2d, mean, rstd, gamma, w_shape, b_shape)
             if grads is not None:
                 return grads + (None, None, None, None, None)
-        dy2d = grad_output.detach().reshape(-1, ctx.cols)
-        if dy2d.dtype != x2d.dtype:
-            dy2d = dy2d.to(x2d.dtype)
-        if dy2d.shape[1] > 1 and dy2d.stride(1) != 1:
-            dy2d = hip_ops.contiguous(dy2d)
-        dx = dw = db = None
-        fused = need_x and (want_w or want_b)        # two launches instead of four
-        if need_x and ctx.nparts == 1 and hip_ops.ln_backward_one_pass_supported(dy2d, x2d, gamma):
-            # rows held whole: this worker's sums are the row's sums, so dx comes out of the pass that forms them
-            dx, dw, db = hip_ops.ln_backward_one_pass(dy2d, x2d, mean, rstd, gamma, 1.0 / ctx.cols, want_gamma=want_w,
-                                                      want_beta=want_b)
-            dx = dx.view(grad_output.shape)
-        elif fused and ctx.nparts == 1 and hip_ops.ln_backward_whole_rows_supported(dy2d, x2d, gamma):
-            dx, dw, db = hip_ops.ln_backward_whole_rows(dy2d, x2d, mean, rstd, gamma, 1.0 / ctx.cols, want_w, want_b)
-            dx = dx.view(grad_output.shape)
-        elif need_x:
-            if fused:
-                sums, work = hip_ops.ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma)
-            else:
-                sums = hip_ops.ln_backward_partial(dy2d, x2d, mean, rstd, gamma)
-            if ctx.nparts > 1:
-                gathered = ctx.P_reduce._world.transport.allgather(ctx.P_reduce, sums, tag=BWD_SUMS_TAG).contiguous()
-            else:
-                gathered = sums.unsqueeze(0)
-            weight_a = 1.0 / (ctx.nparts * ctx.cols)
-            if fused:
-                dx, dw, db = hip_ops.ln_backward_input_params(dy2d, x2d, mean, rstd, gamma, gathered, weight_a, work,
-                                                              want_w, want_b)
-            else:
-                dx = hip_ops.ln_backward_input(dy2d, x2d, mean, rstd, gamma, gathered, weight_a)
-            dx = dx.view(grad_output.shape)
-        elif want_w or want_b:
-            dw, db = hip_ops.ln_backward_params(dy2d, x2d, mean, rstd, want_w, want_b)
-        dw = None if dw is None else dw.view(w_shape)
-        db = None if db is None else db.view(b_shape)
-        return dx, dw, db, None, None, None, None, None
+        grads = _shard_backward(ctx.P_reduce, ctx.nparts, grad_output, x2d, mean, rstd, gamma, need_x, w_shape, b_shape)
+        return grads + (None, None, None, None, None)
 
 
 class DistributedLayerNorm(Module):
@@ -190,6 +201,7 @@ class DistributedLayerNorm(Module):
         self._checked_shape = None                               # last input shape found consistent with part_cols
         self._stats_buffers = {}                                 # rows -> gathered statistics buffer [P, rows, 2]
         self._call_plan = None                                   # what _forward_contiguous worked out for the last shape
+        self._adjoint_calls = _lib.Own()                         # what the native adjoint calls in Python
 
         if self.elementwise_affine:
             # Parameters live on the workers with index 0 in every dimension that
@@ -236,9 +248,9 @@ class DistributedLayerNorm(Module):
         self.weight_buffer = self.broadcast(self.weight)
         self.bias_buffer = self.broadcast(self.bias)
 
-    def _forward_contiguous(self, input, weight, bias):
-        """The forward of ``_shard_forward`` for a contiguous input when no
-        gradient is recorded: everything that only depends on the input's
+    def _forward_contiguous(self, input, weight, bias, keep=False):
+        """The forward of ``_shard_forward`` for a contiguous input, with the
+        rows' mean and reciprocal deviation if ``keep``: everything that only depends on the input's
         shape (row and column counts, the gathered-statistics buffer and the
         address of this worker's slot in it) is worked out once per shape, and a
         call is the two entry points with the transport's gather between -- or
@@ -265,6 +277,10 @@ class DistributedLayerNorm(Module):
             raise ValueError(f"DistributedLayerNorm parameters hold {weight.numel()} / {bias.numel()} elements, "
                              f"the local rows hold {cols}")
         y = torch.empty_like(input)
+        mean = rstd = mean_ptr = rstd_ptr = None
+        if keep:
+            mean, rstd = torch.empty(rows, dtype=torch.float32, device=input.device), torch.empty(rows, dtype=torch.float32, device=input.device)
+            mean_ptr, rstd_ptr = mean.data_ptr(), rstd.data_ptr()
         stream = hip_ops._stream()
         gamma = None if weight is None else weight.data_ptr()
         beta = None if bias is None else bias.data_ptr()
@@ -272,7 +288,7 @@ class DistributedLayerNorm(Module):
            (weight is None or (weight.data_ptr() % quad == 0 and bias.data_ptr() % quad == 0)) and \
            P_reduce._world.transport.peers_gathered_ahead(P_reduce, gathered, tag=STATS_TAG):
             rc = lib.ddl_ln_stats_normalize(input.data_ptr(), dt, rows, cols, cols, gathered.data_ptr(), nparts, P_reduce.rank,
-                                            self._part_cols_arr, gamma, beta, self.eps, y.data_ptr(), cols, None, None,
+                                            self._part_cols_arr, gamma, beta, self.eps, y.data_ptr(), cols, mean_ptr, rstd_ptr,
                                             stream)
             if rc:
                 _lib.check(rc, "ddl_ln_stats_normalize")
@@ -282,16 +298,35 @@ class DistributedLayerNorm(Module):
                 _lib.check(rc, "ddl_ln_partial_stats")
             P_reduce._world.transport.allgather_into(P_reduce, gathered, tag=STATS_TAG)
             rc = lib.ddl_ln_normalize_affine(input.data_ptr(), dt, rows, cols, cols, gathered.data_ptr(), nparts,
-                                             self._part_cols_arr, gamma, beta, self.eps, y.data_ptr(), cols, None, None,
+                                             self._part_cols_arr, gamma, beta, self.eps, y.data_ptr(), cols, mean_ptr, rstd_ptr,
                                              stream)
             if rc:
                 _lib.check(rc, "ddl_ln_normalize_affine")
         else:
             rc = lib.ddl_layer_norm(input.data_ptr(), dt, rows, cols, cols, gamma, beta, self.eps, y.data_ptr(), cols,
-                                    None, None, stream)
+                                    mean_ptr, rstd_ptr, stream)
             if rc:
                 _lib.check(rc, "ddl_layer_norm")
-        return y
+        return (y, mean, rstd) if keep else y
+
+    def _forward_native(self, input, weight, bias):
+        """y with its adjoint as a native node, or None where the general way takes the operands."""
+        P_reduce, nparts = self.allreduce.P_allreduce, len(self.part_cols)
+        calls = self._adjoint_calls.value
+        if calls is None:
+            made = _lib.extension().Callback
+            calls = self._adjoint_calls.value = (made(functools.partial(_gather_sums, P_reduce)),
+                                                 made(functools.partial(_shard_backward, P_reduce, nparts)))
+        if nparts == 1:
+            return _lib.front().layer_norm_shard(input, weight, bias, self.part_cols[0], self.eps, calls[1])
+        if not P_reduce.active or not input.is_cuda or not input.is_contiguous() or \
+           not (weight is None or (weight.is_contiguous() and bias.is_contiguous())):
+            return None
+        if input.numel() == 0 or not _lib.front().unobserved(input, weight, bias):
+            return None
+        with torch.no_grad():       # a gather may copy its parts
+            y, mean, rstd = self._forward_contiguous(input, weight, bias, keep=True)
+        return _lib.front().layer_norm_node(input, weight, bias, y, mean, rstd, nparts, *calls)
 
     def forward(self, input):
         if not self.P_x.active:
@@ -324,5 +359,8 @@ class DistributedLayerNorm(Module):
                 return self._forward_contiguous(input, weight, bias)
             return _shard_forward(input, weight, bias, self.allreduce.P_allreduce, self.part_cols, self.eps,
                                   self._part_cols_arr, self._stats_buffers, False)[0]
+        y = self._forward_native(input, weight, bias)
+        if y is not None:
+            return y
         return _LayerNormShard.apply(input, weight, bias, self.allreduce.P_allreduce, self.part_cols, self.eps,
                                      self._part_cols_arr, self._stats_buffers)

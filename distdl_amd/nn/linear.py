@@ -7,6 +7,7 @@ __all__ = ["DistributedLinear"]
 
 import torch
 
+from .. import _lib
 from .. import hip_ops
 from ..utilities.slicing import compute_subshape
 from .broadcast import Broadcast
@@ -33,9 +34,27 @@ class _LinearShard(torch.autograd.Function):
         return hip_ops.linear_backward(x, weight, grad_output, need_x, need_w, need_b and ctx.has_bias)
 
 
-def linear_shard(x, weight, bias):
+def _general_backward(x, weight, grad_output, need_x, need_w, bias_shape):
+    """The adjoint for what its native form does not take; ``weight`` in any number of dimensions, ``bias_shape`` None where
+    its gradient is not wanted."""
+    if grad_output.dtype != x.dtype:
+        grad_output = grad_output.detach().to(x.dtype)
+    dx, dw, db = hip_ops.linear_backward(x, weight.detach().view(weight.shape[-2:]), grad_output, need_x, need_w, bias_shape is not None)
+    return dx, None if dw is None else dw.view(weight.shape), None if db is None else db.view(bias_shape)
+
+
+def linear_shard(x, weight, bias, out_features=-1, in_features=-1):
     """``x @ weight.T + bias`` on the HIP kernels: bfloat16 and float16 on the
-    tuned MFMA kernel, float32 (the layers' default) on the fp32 one."""
+    tuned MFMA kernel, float32 (the layers' default) on the fp32 one.  ``weight``
+    and ``bias`` as the parameters of a layer lie, ``[1, ..., out, in]`` and
+    ``[1, ..., out, 1]`` with the features the layer says."""
+    y = _lib.front().linear_shard(x, weight, bias, _lib.callback(_general_backward))
+    if y is not None:
+        return y
+    if weight.dim() != 2:
+        weight = weight.view(out_features, in_features)
+    if bias is not None and bias.dim() != 1:
+        bias = bias.view(weight.shape[-2])
     if x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or weight.dtype != x.dtype:
         raise NotImplementedError(f"the linear shard kernels take bfloat16, float16 or float32 operands of one type "
                                   f"(got x {x.dtype}, weight {weight.dtype})")

@@ -125,16 +125,16 @@ class DistributedLinearAllGather(Module):
             return input
         input = self.all_gather(input)
         if self.weight_buffer is None:
-            weight = self.broadcast_weight(self.weight).view(-1, self.in_features)
+            weight = self.broadcast_weight(self.weight)
         else:
             weight = self.weight_buffer
             self.weight_buffer = None
         if self.bias is not None:
             if self.bias_buffer is None:
-                bias = self.broadcast_bias(self.bias).view(weight.shape[-2])
+                bias = self.broadcast_bias(self.bias)
             else:
                 bias = self.bias_buffer
                 self.bias_buffer = None
         else:
             bias = None
-        return linear_shard(input, weight, bias)
+        return linear_shard(input, weight, bias, in_features=self.in_features)

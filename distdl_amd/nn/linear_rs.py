@@ -143,16 +143,16 @@ class DistributedLinearReduceScatter(Module):
         if not self.P_x.active:
             return input
         if self.weight_buffer is None:
-            weight = self.broadcast_weight(self.weight).view(self.out_features, -1)
+            weight = self.broadcast_weight(self.weight)
         else:
             weight = self.weight_buffer
             self.weight_buffer = None
         if self.bias is not None:
             if self.bias_buffer is None:
-                bias = self.broadcast_bias(self.bias).view(self.out_features)
+                bias = self.broadcast_bias(self.bias)
             else:
                 bias = self.bias_buffer
                 self.bias_buffer = None
         else:
             bias = None
-        return self.reduce_scatter(linear_shard(input, weight, bias))
+        return self.reduce_scatter(linear_shard(input, weight, bias, out_features=self.out_features))

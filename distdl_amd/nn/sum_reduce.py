@@ -3,6 +3,7 @@ held on ``P_x`` are summed onto ``P_y`` along the dimensions in which ``P_y`` ha
 one worker, by the reference's broadcast rules read backwards.  The collective
 itself is outside this build; see backends/stub_hip/functional/sum_reduce.py."""
 
+from .. import _lib
 from ..utilities.torch import TensorStructure
 from .module import Module
 
@@ -25,6 +26,10 @@ class SumReduce(Module):
     def forward(self, input):
         if self.identity or not (self.P_x.active or self.P_y.active):
             return input
+        if self._distdl_backend.functional.broadcast.stays(self.P_send, self.P_recv):
+            out = _lib.front().alias(input)
+            if out is not None:
+                return out
         Function = self._distdl_backend.functional.sum_reduce.SumReduceFunction
         # Positional arguments as in the reference (nn/sum_reduce.py:205-211).
         return Function.apply(input, self.P_send, self.P_recv, self.preserve_batch, TensorStructure(input), None)
