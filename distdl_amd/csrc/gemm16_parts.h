@@ -41,15 +41,16 @@ __device__ inline void store_four(uint16_t* __restrict__ y, int64_t ldy, int64_t
     }
 }
 
-// Sum of the splits' partial tiles, bias, rounding.  A thread per lane register quartet of the product kernel.
+// Sum of the splits' partial tiles, bias, rounding, by workgroup `workgroup` of 256 threads: a thread per lane register quartet of
+// the product kernel.
 template <bool F16, int NWM, int NWN, int TM, int TN>
-__global__ __launch_bounds__(256) void gemm16_small_sum(const Part16 p, int splits, const float* __restrict__ partial) {
+__device__ inline void sum_splits(const Part16& p, int splits, const float* __restrict__ partial, int workgroup) {
     constexpr int BM = 16 * NWM * TM, BN = 16 * NWN * TN, kQuartets = BM * BN / 4;
     const int ntiles = p.tiles_m * p.tiles_n;
     constexpr int kBlocks = kQuartets / 256;
     static_assert(kBlocks * 256 == kQuartets, "tile does not split into workgroups");
-    const int tile = static_cast<int>(blockIdx.x) / kBlocks;
-    const int q = (static_cast<int>(blockIdx.x) - tile * kBlocks) * 256 + threadIdx.x;
+    const int tile = workgroup / kBlocks;
+    const int q = (workgroup - tile * kBlocks) * 256 + threadIdx.x;
     int tm, tn;
     tile_of_workgroup(tile, p.tiles_m, p.tiles_n, tm, tn);
     const int lane = q & 63, block = (q >> 6) % (TN * TM), wave = (q >> 6) / (TN * TM);
@@ -72,6 +73,11 @@ __global__ __launch_bounds__(256) void gemm16_small_sum(const Part16 p, int spli
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = s[e] + (p.bias && n + e < p.N ? elem_to_f32<F16>(p.bias[n + e]) : 0.f);
     store_four<F16>(p.y, p.ldy, m, n, p.N, v);
+}
+
+template <bool F16, int NWM, int NWN, int TM, int TN>
+__global__ __launch_bounds__(256) void gemm16_small_sum(const Part16 p, int splits, const float* __restrict__ partial) {
+    sum_splits<F16, NWM, NWN, TM, TN>(p, splits, partial, blockIdx.x);
 }
 
 }  // namespace

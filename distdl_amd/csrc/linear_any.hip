@@ -19,9 +19,17 @@
 //   Tiles of 128 x 128 move half the bytes per flop (0.6 us per k-tile and CU against
 //   1.0 for four of 64 x 64), smaller ones fill the chip: see plan_any16.
 //
+// linear16_adjoint (dx, dw and db of a linear shard).
+//   Bound by launches and by CUs that have nothing to do: each of the three leaves most of the
+//   chip idle when it is small, and waits for the one before.  Workgroups of all of them in one
+//   launch, the product with the longer workgroups first: M 336, N 77, K 603 bf16 14.6 -> 5.7 us,
+//   M 120, N 2258, K 3584 41.7 -> 15.4, M 718, N 821, K 5156 60.2 -> 32.8, M 1024, N 4096, K 1024
+//   (aligned, before: requests into LDS, tiles of 128 x 256) 38.3 -> 30.0.  See plan_adjoint16.
+//
 // gemm16_thin (K below 8, at least one operand read along k).
 //   A reduction shorter than a 16-byte load.  Bound by the result's stores; an output
 //   element per lane.
+#include "colsum.h"
 #include "gemm16_parts.h"
 #include <type_traits>
 
@@ -30,15 +38,6 @@ namespace {
 
 constexpr int BK = kRowBytes / 2;   // 16-bit elements of a k-tile
 constexpr int kAnyThreads = 256;
-
-// 16 bytes from a 2-byte-aligned address (one global load).
-__device__ inline uint4 load16(const uint16_t* p) {
-    struct __attribute__((packed, aligned(2))) Any {
-        uint32_t word[4];
-    };
-    const Any a = *reinterpret_cast<const Any*>(p);
-    return make_uint4(a.word[0], a.word[1], a.word[2], a.word[3]);
-}
 
 // The eight elements of `v` from number `s` on, zeros behind them.
 __device__ inline uint4 drop(uint4 v, int s) {
@@ -225,6 +224,11 @@ __device__ __forceinline__ void any_product(const Part16& p, int block, int spli
             for (int b = 0; b < TM; ++b) dst[(a * TM + b) * 64] = acc[a][b];
         return;
     }
+    // Through LDS, so that whole row segments of the tile leave 16 bytes a lane, at any address: with eight bytes a lane, as a
+    // wavefront holds them, the adjoint of M 23, N 6400, K 2496 took 32.8 us, here 30.6.
+    constexpr int kPitch = 2 * B + 16;   // staggers consecutive rows over the banks
+    static_assert(B * kPitch <= 2 * kStage, "the result does not fit where the operands were");
+    __syncthreads();   // nobody reads the operands any more
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
         const int64_t c = n0 + (sub_w + a) * 16 + 4 * kg;
@@ -236,10 +240,29 @@ __device__ __forceinline__ void any_product(const Part16& p, int block, int spli
         }
 #pragma unroll
         for (int b = 0; b < TM; ++b) {
-            const int64_t m = m0 + (sub_x + b) * 16 + l16;
-            if (m >= M) continue;
-            const float v[4] = {acc[a][b][0] + bv[0], acc[a][b][1] + bv[1], acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]};
-            store_four<F16>(p.y, p.ldy, m, c, N, v);
+            uint32_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = f32_to_elem<F16>(acc[a][b][e] + bv[e]);
+            *reinterpret_cast<uint2*>(lds + ((sub_x + b) * 16 + l16) * kPitch + ((sub_w + a) * 16 + 4 * kg) * 2) = make_uint2(o[0] | o[1] << 16, o[2] | o[3] << 16);
+        }
+    }
+    __syncthreads();
+    constexpr int kChunks = B / 8;   // of a row
+#pragma unroll
+    for (int q = 0; q < B * kChunks / kAnyThreads; ++q) {
+        const int at = q * kAnyThreads + threadIdx.x, row = at / kChunks, chunk = at % kChunks;
+        const int64_t m = m0 + row, c = n0 + chunk * 8;
+        if (m >= M || c >= N) continue;
+        const uint4 v = *reinterpret_cast<const uint4*>(lds + row * kPitch + chunk * 16);
+        uint16_t* const dst = p.y + m * p.ldy + c;
+        if (c + 8 <= N) {
+            typedef u32x4 any __attribute__((aligned(2)));
+            *reinterpret_cast<any*>(dst) = u32x4{v.x, v.y, v.z, v.w};
+        } else {
+            const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (c + e < N) dst[e] = static_cast<uint16_t>(words[e >> 1] >> (16 * (e & 1)));
         }
     }
 }
@@ -249,6 +272,57 @@ template <bool F16, bool XT, bool WT, int T>
 __global__ __launch_bounds__(kAnyThreads, T == 2 ? 2 : 4) void gemm16_any(const Part16 p, int splits, float* __restrict__ partial) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     any_product<F16, XT, WT, T>(p, blockIdx.x, splits, partial, lds);
+}
+
+// The adjoint of a linear shard in one launch: dx = dy . w and dw = dy^T . x by tiles of 64 TX and 64 TW, db = column sums of dy.
+struct Adjoint16 {
+    Part16 dx, dw;
+    int splits_x, splits_w, blocks_x, blocks_w;   // workgroups of the products; of the sums of their splits
+    int first_w;                                  // dw's workgroups come first
+    float *partial_x, *partial_w;
+    const uint16_t* dy;
+    int64_t rows, cols, lddy;
+    void* db;
+    int strips;
+};
+
+constexpr int kFirstStrips = 64;
+
+template <bool F16, int TX, int TW>
+__global__ __launch_bounds__(kAnyThreads, TX == 2 || TW == 2 ? 2 : 4) void linear16_adjoint(const Adjoint16 p) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    // Few strips of column sums come first, each a long chain of loads; many would keep the products waiting.
+    const int products = p.blocks_x + p.blocks_w, first = p.strips <= kFirstStrips ? p.strips : 0;
+    const int b = static_cast<int>(blockIdx.x) - first, x = p.first_w ? b - p.blocks_w : b, w = p.first_w ? b : b - p.blocks_x;
+    if (b < 0 || b >= products) {
+        typedef typename Elem<F16 ? 1 : 0>::type T;
+        colsum_strip<F16 ? 1 : 0, kAnyThreads, 4>(reinterpret_cast<const T*>(p.dy), p.rows, p.cols, p.lddy, static_cast<T*>(p.db), b < 0 ? blockIdx.x : b - products,
+                                                   p.strips, lds);
+    } else if (x >= 0 && x < p.blocks_x) {
+        any_product<F16, false, true, TX>(p.dx, x, p.splits_x, p.partial_x, lds);
+    } else {
+        any_product<F16, true, true, TW>(p.dw, w, p.splits_w, p.partial_w, lds);
+    }
+}
+
+// The sums of the splits of both products; a product in one piece has no workgroups.
+template <bool F16, int TX, int TW>
+__global__ __launch_bounds__(256) void linear16_adjoint_sum(const Adjoint16 p, int blocks_x) {
+    const int b = blockIdx.x;
+    if (b < blocks_x) sum_splits<F16, 2, 2, 2 * TX, 2 * TX>(p.dx, p.splits_x, p.partial_x, b);
+    else sum_splits<F16, 2, 2, 2 * TW, 2 * TW>(p.dw, p.splits_w, p.partial_w, b - blocks_x);
+}
+
+template <bool F16, int TX, int TW>
+int launch_adjoint(const Adjoint16& p, hipStream_t s) {
+    constexpr int lds_bytes = 4 * 64 * (TX > TW ? TX : TW) * kRowBytes;
+    static_assert(colsum_lds_bytes(0, kAnyThreads) <= lds_bytes, "the column sums do not fit");
+    hipLaunchKernelGGL((linear16_adjoint<F16, TX, TW>), dim3(static_cast<uint32_t>(p.blocks_x + p.blocks_w + p.strips)), dim3(kAnyThreads), lds_bytes, s, p);
+    if (int rc = check_launch("linear16_adjoint")) return rc;
+    const int sum_x = p.splits_x > 1 ? p.blocks_x / p.splits_x * 4 * TX * TX : 0, sum_w = p.splits_w > 1 ? p.blocks_w / p.splits_w * 4 * TW * TW : 0;
+    if (sum_x + sum_w == 0) return 0;
+    hipLaunchKernelGGL((linear16_adjoint_sum<F16, TX, TW>), dim3(static_cast<uint32_t>(sum_x + sum_w)), dim3(256), 0, s, p, sum_x);
+    return check_launch("linear16_adjoint_sum");
 }
 
 template <bool F16>
@@ -331,11 +405,79 @@ Small16 plan_any16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus, i
             if (us < once_us) us = once_us;
             if (splits > 1) us += 5.5 + static_cast<double>(workgroups) * floats * 8 / 8e6;
             if (us >= best_us) continue;
-            best_us = us;
+            best_us = best.us = us;
             best.kind = Small16::kAny, best.edge = edge, best.splits = splits, best.workspace = splits > 1 ? workgroups * floats : 0;
         }
     }
     return best;
+}
+
+// Both products on one chip at the same time: a workgroup's k-tile takes what it does above, the rounds of all of them are
+// shared by the CUs, and the longest one is the least it can take; 4.1 or 6.1 as above, 5.5 for the launch that adds splits.
+// The other way is `apart_us` for the products and 4.5 for the column sum, and 3 for each of the two further launches, of
+// which 2 are the host's, where that may be what a step waits for.  Measured over 10 100 sizes (M, N 16 .. 8192, K 32 .. 8192,
+// some aligned): on average 2.03 times as fast as the launches one after the other, at worst 0.80 (M 5848, N 24, K 1408 aligned,
+// 22.9 -> 28.6 us; M 8192, N 512, K 1024 40.3 -> 42.1).
+AdjointPlan16 plan_adjoint16(int64_t M, int64_t N, int64_t K, bool want_db, int cus, int64_t workspace, double apart_us) {
+    AdjointPlan16 best;
+    // operands along their rows have at least eight, dy read along n as well
+    if (M < 8 || N < 8 || K < 8 || (want_db && M > kAdjointRows)) return best;
+    const double launch_us = apart_us < 35 ? 3 : 1;
+    double best_us = apart_us + (want_db ? 4.5 + launch_us : 0) + launch_us;
+    const int64_t strips = want_db ? (N + kNarrow - 1) / kNarrow : 0;
+    double least_us = 3 + 2 * (static_cast<double>(M) * N + (static_cast<double>(M) + N) * K * 2) / 6e6;   // operands and results once
+    if (want_db && 4 + M * 0.0016 > least_us) least_us = 4 + M * 0.0016;                                       // one strip of the column sums
+    for (int edges = 0; edges < 4; ++edges) {
+        const int64_t ex = 1 + (edges & 1), ew = 1 + (edges >> 1);
+        auto tiles = [](int64_t rows, int64_t cols, int64_t e) { return ((rows + 64 * e - 1) / (64 * e)) * ((cols + 64 * e - 1) / (64 * e)); };
+        const int64_t tiles_x = tiles(M, K, ex), tiles_w = tiles(N, K, ew), kx = (N + BK - 1) / BK, kw = (M + BK - 1) / BK;
+        const int64_t resident = (ex == 1 && ew == 1 ? 4 : 2) * static_cast<int64_t>(cus);
+        if (tiles_x + tiles_w > 16 * static_cast<int64_t>(cus)) continue;
+        const double cx = ex == 1 ? 0.25 : 0.62, cw = ew == 1 ? 0.25 : 0.62;
+        for (const int sx : {1, 2, 3, 4, 6, 8}) {
+            if (sx > 1 && (tiles_x * sx > resident || kx < 2 * sx)) break;
+            for (const int sw : {1, 2, 3, 4, 6, 8}) {
+                const int64_t bx = tiles_x * sx, bw = tiles_w * sw;
+                const int64_t floats = (sx > 1 ? bx * ex * ex : 0) * 4096 + (sw > 1 ? bw * ew * ew : 0) * 4096;
+                if ((sw > 1 && (bx + bw > resident || kw < 2 * sw)) || floats > workspace) break;
+                const double nx = static_cast<double>((kx + sx - 1) / sx), nw = static_cast<double>((kw + sw - 1) / sw);
+                const double all = (bx * (nx * cx + (ex == 1 ? 0.85 : 2.5)) + bw * (nw * cw + (ew == 1 ? 0.85 : 2.5))) / cus;
+                const double longest = nx * cx > nw * cw ? nx * cx : nw * cw;
+                double us = (ex == 1 && ew == 1 ? 4.1 : 6.1) + (all * 1.15 > longest ? all * 1.15 : longest) + static_cast<double>(strips) / cus;
+                if (us < least_us) us = least_us;
+                if (floats) us += 5.5 + static_cast<double>(floats) * 8 / 8e6;
+                if (us >= best_us) continue;
+                best_us = us;
+                best.edge_x = static_cast<int>(ex), best.edge_w = static_cast<int>(ew), best.splits_x = sx, best.splits_w = sw, best.workspace = floats;
+                best.first_w = nw * cw > nx * cx;
+            }
+        }
+    }
+    return best;
+}
+
+int run_adjoint16(const AdjointPlan16& plan, bool f16, const Part16& dx, const Part16& dw, void* db, float* workspace, hipStream_t s) {
+    Adjoint16 p{};
+    p.dx = dx, p.dw = dw, p.splits_x = plan.splits_x, p.splits_w = plan.splits_w, p.first_w = plan.first_w;
+    auto tile = [](Part16& part, int edge) {
+        part.tiles_m = static_cast<int>((part.M + 64 * edge - 1) / (64 * edge)), part.tiles_n = static_cast<int>((part.N + 64 * edge - 1) / (64 * edge));
+        return part.tiles_m * part.tiles_n;
+    };
+    p.blocks_x = tile(p.dx, plan.edge_x) * plan.splits_x, p.blocks_w = tile(p.dw, plan.edge_w) * plan.splits_w;
+    p.partial_x = workspace, p.partial_w = workspace + (plan.splits_x > 1 ? static_cast<int64_t>(p.blocks_x) * plan.edge_x * plan.edge_x * 4096 : 0);
+    p.dy = dx.x, p.rows = dx.M, p.cols = dx.K, p.lddy = dx.ldx, p.db = db;
+    p.strips = db ? static_cast<int>((p.cols + kNarrow - 1) / kNarrow) : 0;
+    const int kind = (f16 ? 4 : 0) + (plan.edge_x == 2 ? 2 : 0) + (plan.edge_w == 2 ? 1 : 0);
+    switch (kind) {
+        case 0: return launch_adjoint<false, 1, 1>(p, s);
+        case 1: return launch_adjoint<false, 1, 2>(p, s);
+        case 2: return launch_adjoint<false, 2, 1>(p, s);
+        case 3: return launch_adjoint<false, 2, 2>(p, s);
+        case 4: return launch_adjoint<true, 1, 1>(p, s);
+        case 5: return launch_adjoint<true, 1, 2>(p, s);
+        case 6: return launch_adjoint<true, 2, 1>(p, s);
+        default: return launch_adjoint<true, 2, 2>(p, s);
+    }
 }
 
 int run_any16(const Small16& plan, bool f16, bool xt, bool wt, const Part16& part, float* partial, hipStream_t s) {

@@ -9,26 +9,14 @@
 // and x where they lie (ddl_gemm_ws), db is a column sum with fp32 accumulation.
 // Large 16-bit products whose operands cannot be read in place are transposed
 // into temporaries by the caller (ddl_transpose_2d) and go through ddl_linear.
-#include "ddl_common.h"
-
-#include <hip/hip_fp16.h>
+#include "colsum.h"
+#include "gemm16_small.h"
 
 namespace ddl {
 namespace {
 
 constexpr int kTile = 64;      // elements per tile edge
 constexpr int kBlock = 256;
-constexpr uint32_t kXcds = 8;    // workgroups are dealt to the XCDs in turn
-
-// 16 bytes at the alignment of an element, which global memory takes.
-template <typename T>
-__device__ inline uint4 load16(const T* p) {
-    struct __attribute__((packed, aligned(sizeof(T)))) Any {
-        uint32_t word[4];
-    };
-    const Any w = *reinterpret_cast<const Any*>(p);
-    return make_uint4(w.word[0], w.word[1], w.word[2], w.word[3]);
-}
 
 __device__ inline void store16(uint16_t* p, uint4 q) {
     struct __attribute__((packed, aligned(2))) Any {
@@ -119,64 +107,6 @@ __global__ __launch_bounds__(kBlock) void pad16_kernel(const uint16_t* __restric
         if (first + p * kBlock < total) dst[first + p * kBlock] = q[p];
 }
 
-__device__ inline float bf16_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
-
-__device__ inline uint16_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if (f != f) return 0x7FC0;
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
-}
-
-// Element types of the column sum: 0 = bf16, 1 = fp16, 2 = fp32.
-template <int DT>
-struct Elem;
-template <>
-struct Elem<0> {
-    typedef uint16_t type;
-    static __device__ float load(const uint16_t* p) { return bf16_to_f32(*p); }
-    static __device__ void store(uint16_t* p, float f) { *p = f32_to_bf16(f); }
-    static __device__ void load8(const uint16_t* p, float (&v)[8]) {
-        const uint4 q = load16(p);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[2 * e] = __uint_as_float(w[e] << 16);
-            v[2 * e + 1] = __uint_as_float(w[e] & 0xFFFF0000u);
-        }
-    }
-};
-template <>
-struct Elem<1> {
-    typedef __half type;
-    static __device__ float load(const __half* p) { return __half2float(*p); }
-    static __device__ void store(__half* p, float f) { *p = __float2half_rn(f); }
-    static __device__ void load8(const __half* p, float (&v)[8]) {
-        const uint4 q = load16(p);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&w[e]));
-            v[2 * e] = f.x;
-            v[2 * e + 1] = f.y;
-        }
-    }
-};
-template <>
-struct Elem<2> {
-    typedef float type;
-    static __device__ float load(const float* p) { return *p; }
-    static __device__ void store(float* p, float f) { *p = f; }
-    static __device__ void load8(const float* p, float (&v)[8]) {
-        load4(p, *reinterpret_cast<float(*)[4]>(&v[0]));
-        load4(p + 4, *reinterpret_cast<float(*)[4]>(&v[4]));
-    }
-    static __device__ void load4(const float* p, float (&v)[4]) {
-        const uint4 q = load16(p);
-        v[0] = __uint_as_float(q.x), v[1] = __uint_as_float(q.y), v[2] = __uint_as_float(q.z), v[3] = __uint_as_float(q.w);
-    }
-};
-
 // Stage 1 of the column sum: workgroup (strip, split) adds rows
 // [split * rows_per_split, ...) of a 64-column strip in fp32 and writes 64
 // partial sums to partial[split, col].  8 lanes cover the 64 columns of a row,
@@ -252,78 +182,14 @@ __global__ __launch_bounds__(kBlock) void colsum_final_kernel(const float* __res
     }
 }
 
-// The column sum of few rows in one launch: a workgroup per 16 columns adds all
-// rows, 16 / E lanes per row (E elements of 16 bytes each, at any address), LDS
-// folds the row groups.  The two stages above are two launches and a workspace
-// for what is a few microseconds of reading: [777, 333] fp32 5.0 + 4.7 us, [1024,
-// 4096] bf16 4.9 + 3.9 us.  Neighbouring strips go to one XCD, so that a 128-byte line
-// they share comes from memory once and not for each of four L2 caches, and rows that
-// are not aligned are read 16 bytes a lane like others: [1024, 4096] bf16 5.7 ->
-// 3.8 us, [944, 16382] 22 -> 10.
-constexpr int kNarrow = 16, kOneBlock = 1024;
+// The column sum of few rows in one launch, see colsum.h.
+constexpr int kOneBlock = 1024;
 
 template <int DT>
 __global__ __launch_bounds__(kOneBlock) void colsum_one_kernel(const typename Elem<DT>::type* __restrict__ a, int64_t rows, int64_t cols,
                                                                int64_t ld, typename Elem<DT>::type* __restrict__ out) {
-    typedef typename Elem<DT>::type T;
-    constexpr int E = 16 / static_cast<int>(sizeof(T)), kPieces = kNarrow / E, kGroups = kOneBlock / kPieces;
-    __shared__ float fold[kGroups][kNarrow + 1];
-    __shared__ float half[kOneBlock / kNarrow][kNarrow];
-    const int t = threadIdx.x, g = t / kPieces, c = t % kPieces * E;
-    const uint32_t per = gridDim.x / kXcds, whole = per * kXcds;   // hardware deals workgroups round-robin over the XCDs
-    const int64_t c0 = static_cast<int64_t>(blockIdx.x < whole ? blockIdx.x % kXcds * per + blockIdx.x / kXcds : blockIdx.x) * kNarrow;
-    const int64_t gc = c0 + c;
-    float acc[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) acc[e] = 0.f;
-    // The last vector of a row ends with it: its first `back` columns are the vector's before it, added there.
-    const int back = gc + E > cols ? static_cast<int>(gc + E - cols) : 0;
-    if (back < E && gc >= back) {
-        const T* const first = a + (gc - back);
-#pragma unroll 4
-        for (int64_t r = g; r < rows; r += kGroups) {
-            float v[E];
-            if constexpr (sizeof(T) == 2) Elem<DT>::load8(first + r * ld, v);
-            else Elem<DT>::load4(first + r * ld, v);
-#pragma unroll
-            for (int e = 0; e < E; ++e) acc[e] += v[e];
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e)
-            if (e >= back) fold[g][c + e - back] = acc[e];
-    } else if (back < E) {   // rows shorter than a vector
-        for (int64_t r = g; r < rows; r += kGroups)
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                if (gc + e < cols) acc[e] += Elem<DT>::load(a + r * ld + gc + e);
-#pragma unroll
-        for (int e = 0; e < E; ++e) fold[g][c + e] = acc[e];
-    }
-    __syncthreads();
-    constexpr int kParts = kOneBlock / kNarrow;   // threads per column
-    const int col = t % kNarrow, part = t / kNarrow;
-    // Sums of many partial sums go pairwise: added one after the other, 64 of them lose a third more to rounding in fp32 than
-    // the two stages do.
-    constexpr int kMine = kGroups / kParts;
-    float mine[kMine];
-#pragma unroll
-    for (int k = 0; k < kMine; ++k) mine[k] = fold[part + k * kParts][col];
-#pragma unroll
-    for (int d = kMine / 2; d > 0; d /= 2)
-#pragma unroll
-        for (int k = 0; k < d; ++k) mine[k] += mine[k + d];
-    half[part][col] = mine[0];
-    __syncthreads();
-    if (t < kNarrow && c0 + t < cols) {
-        float r[kParts];
-#pragma unroll
-        for (int k = 0; k < kParts; ++k) r[k] = half[k][t];
-#pragma unroll
-        for (int d = kParts / 2; d > 0; d /= 2)
-#pragma unroll
-            for (int k = 0; k < d; ++k) r[k] += r[k + d];
-        Elem<DT>::store(out + c0 + t, r[0]);
-    }
+    __shared__ char lds[colsum_lds_bytes(DT, kOneBlock)];
+    colsum_strip<DT, kOneBlock, 1>(a, rows, cols, ld, out, blockIdx.x, gridDim.x, lds);
 }
 
 }  // namespace
@@ -434,6 +300,12 @@ extern "C" int ddl_colsum(const void* a, int dtype, int64_t rows, int64_t cols, 
     return run_colsum<2>(a, rows, cols, ld, out, workspace, splits, rows_per_split, strips, s);
 }
 
+namespace ddl {
+
+AdjointPlan16 adjoint16(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy, bool aligned, bool want_db, int64_t workspace);
+
+}  // namespace ddl
+
 extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                                                     int64_t lddy, int want_dx, int want_dw, int want_db) {
     // The products and the column sum run one after the other, so they share the workspace.  If not all operands are
@@ -441,6 +313,15 @@ extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int6
     int64_t most = 0;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     auto take = [&](int64_t elems) { most = elems > most ? elems : most; };
+    if (dtype != DDL_DT_F32 && want_dx && want_dw) {   // both in one launch, with a part of the workspace each
+        const bool inside = want_db && M <= ddl::kAdjointRows;
+        const ddl::AdjointPlan16 plan = ddl::adjoint16(M, N, K, ldx, ldw, lddy, aligned != 0, inside, INT64_MAX);
+        if (plan.edge_x) {
+            take(plan.workspace);
+            want_dx = want_dw = 0;
+            if (inside) want_db = 0;
+        }
+    }
     for (int both = aligned ? 1 : 0; both < 2; ++both) {
         if (want_dx) take(ddl_gemm_workspace_at(dtype, both, lddy, 1, 1, ldw, M, K, N));
         if (want_dw) take(ddl_gemm_workspace_at(dtype, both, 1, lddy, 1, ldx, N, K, M));
@@ -462,6 +343,22 @@ extern "C" int ddl_linear_backward(const void* x, const void* w, const void* dy,
     using namespace ddl;
     if (M < 1 || N < 1 || K < 1) return fail(DDL_E_ARG, "linear backward: M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
     if (!dy || (dx && !w) || (dw && !x)) return fail(DDL_E_ARG, "linear backward: null pointer");
+    if (dtype != DDL_DT_F32 && dx && dw && aligned_to(x, 2) && aligned_to(w, 2) && aligned_to(dy, 2) && aligned_to(dx, 2) && aligned_to(dw, 2) && aligned_to(db, 2) &&
+        (!workspace || aligned_to(workspace, 16))) {
+        const bool aligned = aligned_to(x, 16) && aligned_to(w, 16) && aligned_to(dy, 16);
+        const int64_t room = workspace ? workspace_elems : 0;
+        const bool inside = db && M <= kAdjointRows;
+        const AdjointPlan16 plan = adjoint16(M, N, K, ldx, ldw, lddy, aligned, inside, room);
+        if (plan.edge_x) {
+            Part16 to_x{}, to_w{};
+            to_x.x = static_cast<const uint16_t*>(dy), to_x.ldx = lddy, to_x.w = static_cast<const uint16_t*>(w), to_x.ldw = ldw;
+            to_x.y = static_cast<uint16_t*>(dx), to_x.ldy = K, to_x.M = M, to_x.N = K, to_x.K = N;
+            to_w.x = static_cast<const uint16_t*>(dy), to_w.ldx = lddy, to_w.w = static_cast<const uint16_t*>(x), to_w.ldw = ldx;
+            to_w.y = static_cast<uint16_t*>(dw), to_w.ldy = K, to_w.M = N, to_w.N = K, to_w.K = M;
+            const int rc = run_adjoint16(plan, dtype == DDL_DT_F16, to_x, to_w, inside ? db : nullptr, workspace, static_cast<hipStream_t>(stream));
+            return rc || inside || !db ? rc : ddl_colsum(dy, dtype, M, N, lddy, db, workspace, workspace_elems, stream);
+        }
+    }
     // dx[m, j] = sum_n dy[m, n] w[n, j]: rows of the second operand are the columns of w
     if (dx)
         if (int rc = ddl_gemm_ws(dy, lddy, 1, w, 1, ldw, nullptr, dx, dtype, K, M, K, N, workspace, workspace_elems, stream)) return rc;

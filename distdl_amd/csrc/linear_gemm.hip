@@ -537,6 +537,16 @@ Small16 plan_anywhere(const Operand16& a, const Operand16& b, int64_t M, int64_t
 // The product itself is computed for callers that do not have the copies, too, up to here.
 constexpr double kLeeway = 18;
 
+// Estimate for one product, as it is computed when it is alone; negative where it is not (the caller copies the operands).
+double alone_us(const Operand16& a, const Operand16& b, bool aligned, int64_t M, int64_t N, int64_t K, int cus) {
+    if (aligned && pitches_ok(a, M, K) && pitches_ok(b, N, K)) {
+        const Plan16 plan = plan16(a.transposed(), b.transposed(), M, N, K, cus, INT64_MAX);
+        return plan.small.kind != Small16::kNone ? plan.small.us : plan.large;
+    }
+    const Small16 any = plan_anywhere(a, b, M, N, K, cus, INT64_MAX, kLeeway);
+    return any.kind == Small16::kNone ? -1 : any.kind == Small16::kThin ? 8 : any.us;
+}
+
 // y[M, N] = a[M, K] . b[N, K]^T + bias in 16-bit elements.  `workspace` (may be null) for the sums of a split reduction;
 // `anywhere`: operands that are not aligned to 16 bytes are taken where linear_any.hip reads them.
 int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* bias, uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
@@ -605,6 +615,23 @@ int gemm16(const char* who, bool f16, Operand16 a, Operand16 b, const uint16_t* 
 }
 
 }  // namespace
+}  // namespace ddl
+
+namespace ddl {
+
+// How the adjoint of a 16-bit linear shard is computed in one launch, if it is (edge_x 0 otherwise): where the two products
+// would each be computed with their operands as they lie.
+AdjointPlan16 adjoint16(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy, bool aligned, bool want_db, int64_t workspace) {
+    int dev = 0;
+    const int cus = compute_units(dev);
+    const Operand16 dy{nullptr, lddy, 1}, dy_t{nullptr, 1, lddy}, w{nullptr, 1, ldw}, x{nullptr, 1, ldx};
+    if (M < 2 || N < 2 || K < 2 || !readable_anywhere(dy, M, N) || !readable_anywhere(w, K, N) || !readable_anywhere(dy_t, N, M) || !readable_anywhere(x, K, M))
+        return AdjointPlan16{};
+    const double dx_us = alone_us(dy, w, aligned, M, K, N, cus), dw_us = alone_us(dy_t, x, aligned, N, K, M, cus);
+    if (dx_us < 0 || dw_us < 0) return AdjointPlan16{};
+    return plan_adjoint16(M, N, K, want_db, cus, workspace, dx_us + dw_us);
+}
+
 }  // namespace ddl
 
 namespace ddl {

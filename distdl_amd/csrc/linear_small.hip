@@ -406,7 +406,7 @@ Small16 plan_small16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus,
     auto take = [&](double us, Small16::Kind kind, int groups, int splits) {
         if (us < hbm_us) us = hbm_us;
         if (us >= best_us) return;
-        best_us = us;
+        best_us = best.us = us;
         best.kind = kind, best.groups = groups, best.splits = splits, best.workspace = splits > 1 ? tiles * splits * 4096 : 0;
     };
     if (M <= 64 && !xt && !wt && N <= 0x7FFFFF) {

@@ -49,3 +49,38 @@ def test_products_of_operands_at_any_address(dtype, a_t, b_t, M, N, K, pad, shif
         _lib.check(rc, "ddl_gemm_ws")
         assert torch.equal(out[:, :N].double(), want)
         assert (out[:, N:] == 77.0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,pad,shift", [
+    # one k-tile and one element more, 64 x 64 tiles, an odd length of every kind; 128 x 128 tiles of either product; both with
+    # split reductions; as many rows as the column sums take there, and one more; aligned throughout
+    (8, 8, 8, 0, 0), (65, 64, 66, 1, 1), (97, 77, 603, 0, 0), (718, 821, 2056, 0, 3), (2048, 1024, 1024, 0, 0), (3001, 130, 257, 2, 0),
+    (16384, 24, 40, 0, 0), (16385, 17, 33, 0, 1), (9, 5001, 1200, 0, 0), (1200, 9, 5001, 1, 0)])
+def test_adjoint_of_a_linear_shard_in_one_launch(dtype, M, N, K, pad, shift):
+    """dx, dw and db on integers, equal to the sums in 64 bits; with the workspace asked for, half of it and none; what surrounds the
+    operands is NaN, and the products alone, which take other kernels, give the same."""
+    from distdl_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+
+    def draw(rows, cols, keep):
+        t = torch.randint(-1, 2, (rows, cols), generator=gen, device="cuda")
+        return (t * (torch.rand(rows, cols, generator=gen, device="cuda") < keep)).to(dtype)
+    x, w, dy = draw(M, K, min(1.0, 40.0 / M)), draw(N, K, min(1.0, 40.0 / N)), draw(M, N, min(1.0, 2000.0 / M))
+    want = [dy.double() @ w.double(), dy.double().T @ x.double(), dy.double().sum(0)]
+    assert max(t.abs().max() for t in want) <= 256
+    (bx, px, (ldx, _)), (bw, pw, (ldw, _)), (bd, pd, (ldd, _)) = [_strided(t, False, pad, shift) for t in (x, w, dy)]
+    lib, dt = _lib.load(), _lib.DDL_DT_BF16 if dtype == torch.bfloat16 else _lib.DDL_DT_F16
+    aligned = int(pad == 0 and shift % 8 == 0)
+    stream = torch.cuda.current_stream().cuda_stream
+    for wanted in ((1, 1, 1), (1, 1, 0), (1, 0, 1), (0, 1, 0)):
+        elems = lib.ddl_linear_backward_workspace_at(dt, aligned, M, N, K, ldx, ldw, ldd, *wanted)
+        for n in {elems, elems // 2, 0} if wanted[2] == 0 or M <= 4096 else {elems}:
+            work = torch.full((n,), float("nan"), device="cuda") if n else None
+            outs = [torch.full((s + 8,), 77.0, dtype=dtype, device="cuda") if on else None for s, on in zip((M * K, N * K, N), wanted)]
+            rc = lib.ddl_linear_backward(px, pw, pd, *[None if o is None else o.data_ptr() for o in outs], dt, M, N, K, ldx, ldw, ldd,
+                                         None if work is None else work.data_ptr(), n, stream)
+            _lib.check(rc, "ddl_linear_backward")
+            for o, t in zip(outs, want):
+                if o is not None:
+                    assert torch.equal(o[:-8].view(t.shape).double(), t) and (o[-8:] == 77.0).all()
