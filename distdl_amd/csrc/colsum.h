@@ -10,6 +10,7 @@ namespace ddl {
 
 constexpr uint32_t kColsumXcds = 8;    // workgroups are dealt to the XCDs in turn
 constexpr int kNarrow = 16;            // columns of a strip
+constexpr int kFirstStrips = 64;       // so many strips go ahead of the products they share a launch with
 
 namespace {
 

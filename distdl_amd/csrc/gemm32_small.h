@@ -50,6 +50,18 @@ Small32 plan_split32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace
 // Launches the product of `part` (its tile counts are set here) as planned; `partial` holds the splits' sums.
 int run_small32(const char* who, const Small32& plan, bool xt, bool wt, const PartOf<float>& part, float* partial, int dev, hipStream_t s);
 
+// The adjoint of a linear shard, dx[M, K], dw[N, K] and db[N] from dy[M, N], in one launch (and one that adds split reductions).
+struct AdjointPlan32 {
+    int groups_x = 0, groups_w = 0;     // tiles, as in Small32; 0: not taken
+    int splits_x = 1, splits_w = 1;
+    bool first_w = false;
+    int64_t workspace = 0;
+};
+AdjointPlan32 plan_adjoint32(int64_t M, int64_t N, int64_t K, bool want_db, int cus, int64_t workspace, const Small32& x, const Small32& w);
+
+// `dx` and `dw` describe the products dy . w and dy^T . x, `db` may be null.
+int run_adjoint32(const AdjointPlan32& plan, const PartOf<float>& dx, const PartOf<float>& dw, float* db, float* workspace, hipStream_t s);
+
 int run_split32(const Small32& plan, bool xt, bool wt, const PartOf<float>& part, float* partial, hipStream_t s);
 
 // Adds the splits' sums and the bias: `partial` holds, split by split and tile by tile, blocks x blocks (2 or 4) blocks of

@@ -286,8 +286,6 @@ struct Adjoint16 {
     int strips;
 };
 
-constexpr int kFirstStrips = 64;
-
 template <bool F16, int TX, int TW>
 __global__ __launch_bounds__(kAnyThreads, TX == 2 || TW == 2 ? 2 : 4) void linear16_adjoint(const Adjoint16 p) {
     extern __shared__ __attribute__((aligned(16))) char lds[];

@@ -11,6 +11,7 @@
 // into temporaries by the caller (ddl_transpose_2d) and go through ddl_linear.
 #include "colsum.h"
 #include "gemm16_small.h"
+#include "gemm32_small.h"
 
 namespace ddl {
 namespace {
@@ -303,6 +304,19 @@ extern "C" int ddl_colsum(const void* a, int dtype, int64_t rows, int64_t cols, 
 namespace ddl {
 
 AdjointPlan16 adjoint16(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy, bool aligned, bool want_db, int64_t workspace);
+Small32 plan32(int64_t a_rs, int64_t a_ks, int64_t b_rs, int64_t b_ks, int64_t M, int64_t N, int64_t K, int cus, int64_t workspace);
+
+constexpr int64_t kAdjointRows32 = 2048;   // longer column sums stay in two stages, whose partial sums are shorter
+
+// The same in fp32: where both products go to linear_f32_small.hip.
+static AdjointPlan32 adjoint32(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy, bool want_db, int64_t workspace) {
+    int dev = 0;
+    const int cus = compute_units(dev);
+    // strides of 1 and 1 say nothing about the order of an operand
+    if (M < 2 || N < 2 || K < 2 || ldx < 2 || ldw < 2 || lddy < 2) return AdjointPlan32{};
+    const Small32 x = plan32(lddy, 1, 1, ldw, M, K, N, cus, INT64_MAX), w = plan32(1, lddy, 1, ldx, N, K, M, cus, INT64_MAX);
+    return plan_adjoint32(M, N, K, want_db, cus, workspace, x, w);
+}
 
 }  // namespace ddl
 
@@ -313,11 +327,19 @@ extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int6
     int64_t most = 0;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     auto take = [&](int64_t elems) { most = elems > most ? elems : most; };
-    if (dtype != DDL_DT_F32 && want_dx && want_dw) {   // both in one launch, with a part of the workspace each
-        const bool inside = want_db && M <= ddl::kAdjointRows;
-        const ddl::AdjointPlan16 plan = ddl::adjoint16(M, N, K, ldx, ldw, lddy, aligned != 0, inside, INT64_MAX);
-        if (plan.edge_x) {
+    if (want_dx && want_dw) {   // both in one launch, with a part of the workspace each
+        const bool inside = want_db && M <= (dtype == DDL_DT_F32 ? ddl::kAdjointRows32 : ddl::kAdjointRows);
+        bool taken;
+        if (dtype == DDL_DT_F32) {
+            const ddl::AdjointPlan32 plan = ddl::adjoint32(M, N, K, ldx, ldw, lddy, inside, INT64_MAX);
+            taken = plan.groups_x != 0;
             take(plan.workspace);
+        } else {
+            const ddl::AdjointPlan16 plan = ddl::adjoint16(M, N, K, ldx, ldw, lddy, aligned != 0, inside, INT64_MAX);
+            taken = plan.edge_x != 0;
+            take(plan.workspace);
+        }
+        if (taken) {
             want_dx = want_dw = 0;
             if (inside) want_db = 0;
         }
@@ -356,6 +378,20 @@ extern "C" int ddl_linear_backward(const void* x, const void* w, const void* dy,
             to_w.x = static_cast<const uint16_t*>(dy), to_w.ldx = lddy, to_w.w = static_cast<const uint16_t*>(x), to_w.ldw = ldx;
             to_w.y = static_cast<uint16_t*>(dw), to_w.ldy = K, to_w.M = N, to_w.N = K, to_w.K = M;
             const int rc = run_adjoint16(plan, dtype == DDL_DT_F16, to_x, to_w, inside ? db : nullptr, workspace, static_cast<hipStream_t>(stream));
+            return rc || inside || !db ? rc : ddl_colsum(dy, dtype, M, N, lddy, db, workspace, workspace_elems, stream);
+        }
+    }
+    if (dtype == DDL_DT_F32 && dx && dw && aligned_to(x, 4) && aligned_to(w, 4) && aligned_to(dy, 4) && aligned_to(dx, 4) && aligned_to(dw, 4) &&
+        aligned_to(db, 4) && (!workspace || aligned_to(workspace, 16))) {
+        const bool inside = db && M <= kAdjointRows32;
+        const AdjointPlan32 plan = adjoint32(M, N, K, ldx, ldw, lddy, inside, workspace ? workspace_elems : 0);
+        if (plan.groups_x) {
+            PartOf<float> to_x{}, to_w{};
+            to_x.x = static_cast<const float*>(dy), to_x.ldx = lddy, to_x.w = static_cast<const float*>(w), to_x.ldw = ldw;
+            to_x.y = static_cast<float*>(dx), to_x.ldy = K, to_x.M = M, to_x.N = K, to_x.K = N;
+            to_w.x = static_cast<const float*>(dy), to_w.ldx = lddy, to_w.w = static_cast<const float*>(x), to_w.ldw = ldx;
+            to_w.y = static_cast<float*>(dw), to_w.ldy = K, to_w.M = N, to_w.N = K, to_w.K = M;
+            const int rc = run_adjoint32(plan, to_x, to_w, inside ? static_cast<float*>(db) : nullptr, workspace, static_cast<hipStream_t>(stream));
             return rc || inside || !db ? rc : ddl_colsum(dy, dtype, M, N, lddy, db, workspace, workspace_elems, stream);
         }
     }

@@ -25,6 +25,13 @@
 // element.  (The addresses there are selected, not branched on: with branches the
 // compiler kept 360 registers, one workgroup fit on a CU, and the kernel took 1.4 times
 // as long.)
+//
+// linear32_adjoint is dx, dw and db of a linear shard in one launch, for products whose
+// workgroups are all resident at once: alone each of the three leaves CUs idle and waits
+// for the one before.  M 777, N 333, K 1024 28.1 -> 21.0 us, M 97, N 77, K 603 10.9 -> 5.3, M 108, N
+// 192, K 5376 15.8 -> 10.5, M = N = K = 1024 53.9 -> 40.9.  With more workgroups the products fill
+// the chip one after the other, and the one launch is slower (M 2078, N 6152, K 276 162, here 243).
+#include "colsum.h"
 #include "gemm_tiles.h"
 #include "gemm32_small.h"
 #include <type_traits>
@@ -37,15 +44,15 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 constexpr int BK = kRowBytes / 4;   // floats of a k-tile
 typedef PartOf<float> Part32;
 
+// Workgroup `number` of the tiles_m x tiles_n x splits of a product.
 template <bool XT, bool WT, int NWM, int NWN, int KG, int STAGES>
-__global__ __launch_bounds__(256) void gemm32_small(const Part32 p, int splits, float* __restrict__ partial) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];
+__device__ __forceinline__ void small_product(const Part32& p, int number, int splits, float* __restrict__ partial, char* lds) {
     constexpr int NW = NWM * NWN, BM = 32 * NWM, BN = 32 * NWN;
     static_assert(NW * KG == 4, "four wavefronts per workgroup");
     constexpr int JW_W = BN / 8 / NW, JW_X = BM / 8 / NW;   // request instructions (1 KiB each) per wavefront and tile
     constexpr int kStage = (BM + BN) * kRowBytes, kX = BN * kRowBytes;   // a stage holds the w tile and then the x tile
     const int ntiles = p.tiles_m * p.tiles_n;
-    const int split = static_cast<int>(blockIdx.x) / ntiles, tile = static_cast<int>(blockIdx.x) - split * ntiles;
+    const int split = number / ntiles, tile = number - split * ntiles;
     int tm, tn;
     tile_of_workgroup(tile, p.tiles_m, p.tiles_n, tm, tn);
     const int64_t M = p.M, N = p.N, K = p.K;
@@ -191,7 +198,7 @@ __global__ __launch_bounds__(256) void gemm32_small(const Part32 p, int splits, 
             for (int g = 0; g < 4; ++g) quad[g] += fold[((i * NW + wave) * 4 + g) * 64 + lane];
     }
     if (splits > 1) {   // lane order, so that the partial sums are written and read in whole lines
-        floatx4* dst = reinterpret_cast<floatx4*>(partial) + (static_cast<int64_t>(blockIdx.x) * NW + wave) * 256 + lane;
+        floatx4* dst = reinterpret_cast<floatx4*>(partial) + (static_cast<int64_t>(number) * NW + wave) * 256 + lane;
 #pragma unroll
         for (int g = 0; g < 4; ++g) dst[g * 64] = quad[g];
         return;
@@ -205,19 +212,25 @@ __global__ __launch_bounds__(256) void gemm32_small(const Part32 p, int splits, 
     }
 }
 
-// Sum of the splits' partial tiles and bias.  A thread per quartet of columns.
+template <bool XT, bool WT, int NWM, int NWN, int KG, int STAGES>
+__global__ __launch_bounds__(256) void gemm32_small(const Part32 p, int splits, float* __restrict__ partial) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    small_product<XT, WT, NWM, NWN, KG, STAGES>(p, blockIdx.x, splits, partial, lds);
+}
+
+// Sum of the splits' partial tiles and bias, workgroup `number`: a thread per quartet of columns.
 template <int NWM, int NWN>
-__global__ __launch_bounds__(256) void gemm32_small_sum(const Part32 p, int splits, const float* __restrict__ partial) {
+__device__ inline void sum_splits(const Part32& p, int splits, const float* __restrict__ partial, int number) {
     constexpr int NW = NWM * NWN;   // one workgroup per 32 x 32 block
     const int ntiles = p.tiles_m * p.tiles_n;
-    const int tile = static_cast<int>(blockIdx.x) / NW, wave = static_cast<int>(blockIdx.x) - tile * NW;
+    const int tile = number / NW, wave = number - tile * NW;
     int tm, tn;
     tile_of_workgroup(tile, p.tiles_m, p.tiles_n, tm, tn);
     const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
     const int64_t m = static_cast<int64_t>(tm) * (32 * NWM) + wave % NWM * 32 + (lane & 31);
     const int64_t n = static_cast<int64_t>(tn) * (32 * NWN) + wave / NWM * 32 + 8 * g + 4 * (lane >> 5);
     if (m >= p.M || n >= p.N) return;
-    const floatx4* src = reinterpret_cast<const floatx4*>(partial) + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const floatx4* src = reinterpret_cast<const floatx4*>(partial) + static_cast<int64_t>(number) * 256 + threadIdx.x;
     const int64_t stride = static_cast<int64_t>(ntiles) * NW * 256;
     floatx4 s = {0.f, 0.f, 0.f, 0.f};
     int k = 0;
@@ -230,6 +243,11 @@ __global__ __launch_bounds__(256) void gemm32_small_sum(const Part32 p, int spli
     }
     for (; k < splits; ++k) s += src[k * stride];
     store_four(p.y + m * p.ldy + n, n, p.N, s + bias_of(p.bias, n, p.N));
+}
+
+template <int NWM, int NWN>
+__global__ __launch_bounds__(256) void gemm32_small_sum(const Part32 p, int splits, const float* __restrict__ partial) {
+    sum_splits<NWM, NWN>(p, splits, partial, blockIdx.x);
 }
 
 template <int NWM, int NWN>
@@ -262,6 +280,67 @@ int launch_shape(const char* who, const Small32& plan, const Part32& part, float
     return launch<XT, WT, 2, 2, 1>(who, part, plan.splits, partial, dev, s);
 }
 
+// The adjoint of a linear shard in one launch: dx = dy . w and dw = dy^T . x in tiles of GX and GW groups, db = column sums of dy.
+struct Adjoint32 {
+    Part32 dx, dw;
+    int splits_x, splits_w, blocks_x, blocks_w;   // workgroups of the products
+    int first_w;                                  // dw's come first
+    float *partial_x, *partial_w;
+    float* db;
+    int strips;
+};
+
+// By groups: wavefronts along m and n, stages (two workgroups per CU with one and two groups).
+template <int G>
+struct Shape32 {
+    static constexpr int NWM = G == 1 ? 2 : 1, NWN = G == 4 ? 1 : 2, STAGES = G == 1 ? 4 : 3;
+    static constexpr int kLds = G * STAGES * 32 * (NWM + NWN) * kRowBytes;
+};
+
+template <int GX, int GW>
+__global__ __launch_bounds__(256) void linear32_adjoint(const Adjoint32 p) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    typedef Shape32<GX> X;
+    typedef Shape32<GW> W;
+    // Few strips of column sums come first, each a long chain of loads; many would keep the products waiting.
+    const int products = p.blocks_x + p.blocks_w, first = p.strips <= kFirstStrips ? p.strips : 0;
+    const int b = static_cast<int>(blockIdx.x) - first, x = p.first_w ? b - p.blocks_w : b, w = p.first_w ? b : b - p.blocks_x;
+    if (b < 0 || b >= products)
+        colsum_strip<2, 256, 4>(p.dx.x, p.dx.M, p.dx.K, p.dx.ldx, p.db, b < 0 ? blockIdx.x : b - products, p.strips, lds);
+    else if (x >= 0 && x < p.blocks_x)
+        small_product<false, true, X::NWM, X::NWN, GX, X::STAGES>(p.dx, x, p.splits_x, p.partial_x, lds);
+    else
+        small_product<true, true, W::NWM, W::NWN, GW, W::STAGES>(p.dw, w, p.splits_w, p.partial_w, lds);
+}
+
+template <int GX, int GW>
+__global__ __launch_bounds__(256) void linear32_adjoint_sum(const Adjoint32 p, int blocks_x) {
+    const int b = blockIdx.x;
+    if (b < blocks_x) sum_splits<Shape32<GX>::NWM, Shape32<GX>::NWN>(p.dx, p.splits_x, p.partial_x, b);
+    else sum_splits<Shape32<GW>::NWM, Shape32<GW>::NWN>(p.dw, p.splits_w, p.partial_w, b - blocks_x);
+}
+
+template <int GX, int GW>
+int launch_adjoint(const Adjoint32& p, int dev, hipStream_t s) {
+    static std::atomic<bool> reserved[kMaxDevices];
+    typedef Shape32<GX> X;
+    typedef Shape32<GW> W;
+    constexpr int lds_bytes = X::kLds > W::kLds ? X::kLds : W::kLds;
+    static_assert(colsum_lds_bytes(2, 256) <= lds_bytes, "the column sums do not fit");
+    const auto kernel = linear32_adjoint<GX, GW>;
+    if (lds_bytes > 65536 && !reserved[dev].load(std::memory_order_acquire)) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+        if (e != hipSuccess) return fail(static_cast<int>(e), "linear backward: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+        reserved[dev].store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(p.blocks_x + p.blocks_w + p.strips)), dim3(256), lds_bytes, s, p);
+    if (int rc = check_launch("linear32_adjoint")) return rc;
+    const int sum_x = p.splits_x > 1 ? p.blocks_x / p.splits_x * X::NWM * X::NWN : 0, sum_w = p.splits_w > 1 ? p.blocks_w / p.splits_w * W::NWM * W::NWN : 0;
+    if (sum_x + sum_w == 0) return 0;
+    hipLaunchKernelGGL((linear32_adjoint_sum<GX, GW>), dim3(static_cast<uint32_t>(sum_x + sum_w)), dim3(256), 0, s, p, sum_x);
+    return check_launch("linear32_adjoint_sum");
+}
+
 }  // namespace
 
 // The estimates are fits to a sweep over M, N, K of 5 .. 16384 on all operand layouts, in microseconds: 4 + per k-tile (per
@@ -292,6 +371,78 @@ Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace
         }
     }
     return best;
+}
+
+// Both products on one chip at the same time, next to `x` and `w`, how they are computed alone: a round of a workgroup (k-tiles of
+// all its groups) is 0.52 us of its CU's matrix cores and at least 0.7 long.  No element is summed in fewer pieces than alone.
+// The other way has 4.5 for the column sum, and 3 for each of the two further launches, of which 2 are the host's, where that may
+// be what a step waits for.  All workgroups are resident at once: where there are more, the products fill the chip one by one.
+AdjointPlan32 plan_adjoint32(int64_t M, int64_t N, int64_t K, bool want_db, int cus, int64_t workspace, const Small32& x, const Small32& w) {
+    AdjointPlan32 best;
+    if (!x.groups || x.edge || !w.groups || w.edge) return best;
+    const double apart_us = x.us + w.us, launch_us = apart_us < 35 ? 3 : 1;
+    double best_us = apart_us + (want_db ? 4.5 + launch_us : 0) + launch_us;
+    double least_us = 3 + 4 * (static_cast<double>(M) * N + (static_cast<double>(M) + N) * K * 2) / 6e6;   // operands and results once
+    if (want_db && 4 + M * 0.0032 > least_us) least_us = 4 + M * 0.0032;                                   // one strip of the column sums
+    const double strips = want_db ? static_cast<double>((N + kNarrow - 1) / kNarrow) : 0;
+    auto tiles = [](int64_t rows, int64_t cols, int g) {
+        const int64_t bm = g == 1 ? 64 : 32, bn = g == 4 ? 32 : 64;
+        return ((rows + bm - 1) / bm) * ((cols + bn - 1) / bn);
+    };
+    auto floats = [](int64_t blocks, int g) { return blocks * (g == 1 ? 4096 : g == 2 ? 2048 : 1024); };
+    const int64_t kx = (N + BK - 1) / BK, kw = (M + BK - 1) / BK;
+    for (const int gx : {1, 2, 4}) {
+        for (const int gw : {1, 2, 4}) {
+            const int64_t tiles_x = tiles(M, K, gx), tiles_w = tiles(N, K, gw), most = (gx == 4 || gw == 4 ? 1 : 2) * static_cast<int64_t>(cus);
+            for (const int sx : {1, 2, 3, 4, 6, 8}) {
+                if (tiles_x * sx > most || (sx > 1 && kx < 2 * sx * gx)) break;
+                if (gx * sx < x.groups * x.splits) continue;
+                for (const int sw : {1, 2, 3, 4, 6, 8}) {
+                    const int64_t bx = tiles_x * sx, bw = tiles_w * sw, sums = (sx > 1 ? floats(bx, gx) : 0) + (sw > 1 ? floats(bw, gw) : 0);
+                    if (bx + bw > most || (sw > 1 && kw < 2 * sw * gw)) break;
+                    if (sums > workspace) break;
+                    if (gw * sw < w.groups * w.splits) continue;
+                    const int64_t nx = ((kx + sx - 1) / sx + gx - 1) / gx, nw = ((kw + sw - 1) / sw + gw - 1) / gw;
+                    const double ex = gx == 1 ? 1.0 : gx == 2 ? 1.3 : 2.0, ew = gw == 1 ? 1.0 : gw == 2 ? 1.3 : 2.0;
+                    const double all = (bx * (nx * 0.52 + ex) + bw * (nw * 0.52 + ew)) / cus * 1.1, longest = (nx > nw ? nx : nw) * 0.7;
+                    double us = 4.5 + (all > longest ? all : longest) + strips / cus;
+                    if (us < least_us) us = least_us;
+                    if (sums) us += 5.5 + static_cast<double>(sums) * 8 / 5e6;
+                    if (us >= best_us) continue;
+                    best_us = us;
+                    best.groups_x = gx, best.groups_w = gw, best.splits_x = sx, best.splits_w = sw, best.workspace = sums, best.first_w = nw > nx;
+                }
+            }
+        }
+    }
+    return best;
+}
+
+int run_adjoint32(const AdjointPlan32& plan, const PartOf<float>& dx, const PartOf<float>& dw, float* db, float* workspace, hipStream_t s) {
+    Adjoint32 p{};
+    p.dx = dx, p.dw = dw, p.splits_x = plan.splits_x, p.splits_w = plan.splits_w, p.first_w = plan.first_w;
+    auto tile = [](Part32& part, int g) {
+        const int64_t bm = g == 1 ? 64 : 32, bn = g == 4 ? 32 : 64;
+        part.tiles_m = static_cast<int>((part.M + bm - 1) / bm), part.tiles_n = static_cast<int>((part.N + bn - 1) / bn);
+        return part.tiles_m * part.tiles_n;
+    };
+    p.blocks_x = tile(p.dx, plan.groups_x) * plan.splits_x, p.blocks_w = tile(p.dw, plan.groups_w) * plan.splits_w;
+    p.partial_x = workspace;
+    p.partial_w = workspace + (plan.splits_x > 1 ? static_cast<int64_t>(p.blocks_x) * (plan.groups_x == 1 ? 4096 : plan.groups_x == 2 ? 2048 : 1024) : 0);
+    p.db = db, p.strips = db ? static_cast<int>((dx.K + kNarrow - 1) / kNarrow) : 0;
+    int dev = 0;
+    compute_units(dev);
+    switch (plan.groups_x * 8 + plan.groups_w) {
+        case 9: return launch_adjoint<1, 1>(p, dev, s);
+        case 10: return launch_adjoint<1, 2>(p, dev, s);
+        case 12: return launch_adjoint<1, 4>(p, dev, s);
+        case 17: return launch_adjoint<2, 1>(p, dev, s);
+        case 18: return launch_adjoint<2, 2>(p, dev, s);
+        case 20: return launch_adjoint<2, 4>(p, dev, s);
+        case 33: return launch_adjoint<4, 1>(p, dev, s);
+        case 34: return launch_adjoint<4, 2>(p, dev, s);
+        default: return launch_adjoint<4, 4>(p, dev, s);
+    }
 }
 
 int run_small32(const char* who, const Small32& plan, bool xt, bool wt, const PartOf<float>& part, float* partial, int dev, hipStream_t s) {

@@ -14,7 +14,7 @@ def _strided(t, transposed, pad, shift):
     buf = torch.full((shift + (t.shape[0] - 1) * ld + t.shape[1],), float("nan"), dtype=t.dtype, device="cuda")
     view = buf[shift:].as_strided(t.shape, (ld, 1))
     view.copy_(t)
-    return buf, buf.data_ptr() + 2 * shift, (1, ld) if transposed else (ld, 1)
+    return buf, buf.data_ptr() + t.element_size() * shift, (1, ld) if transposed else (ld, 1)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -51,12 +51,20 @@ def test_products_of_operands_at_any_address(dtype, a_t, b_t, M, N, K, pad, shif
         assert (out[:, N:] == 77.0).all()
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,N,K,pad,shift", [
+_ADJOINTS = [
     # one k-tile and one element more, 64 x 64 tiles, an odd length of every kind; 128 x 128 tiles of either product; both with
     # split reductions; as many rows as the column sums take there, and one more; aligned throughout
     (8, 8, 8, 0, 0), (65, 64, 66, 1, 1), (97, 77, 603, 0, 0), (718, 821, 2056, 0, 3), (2048, 1024, 1024, 0, 0), (3001, 130, 257, 2, 0),
-    (16384, 24, 40, 0, 0), (16385, 17, 33, 0, 1), (9, 5001, 1200, 0, 0), (1200, 9, 5001, 1, 0)])
+    (16384, 24, 40, 0, 0), (16385, 17, 33, 0, 1), (9, 5001, 1200, 0, 0), (1200, 9, 5001, 1, 0)]
+_ADJOINTS_32 = [
+    # fewer elements than a k-tile, one more than one, tiles of every size for either product, split reductions, as many rows as the
+    # column sums take there and one more, more tiles than one launch takes
+    (2, 2, 2, 0, 0), (5, 3, 7, 1, 1), (33, 31, 35, 0, 0), (97, 77, 603, 0, 3), (777, 333, 1024, 0, 0), (104, 1256, 960, 0, 0), (108, 192, 5376, 2, 1),
+    (2048, 24, 40, 0, 0), (2049, 17, 33, 0, 1), (512, 512, 512, 0, 0), (1500, 130, 257, 3, 0), (2500, 900, 300, 0, 0)]
+
+
+@pytest.mark.parametrize("dtype,M,N,K,pad,shift", [(dt, *c) for dt in (torch.bfloat16, torch.float16) for c in _ADJOINTS] +
+                         [(torch.float32, *c) for c in _ADJOINTS_32])
 def test_adjoint_of_a_linear_shard_in_one_launch(dtype, M, N, K, pad, shift):
     """dx, dw and db on integers, equal to the sums in 64 bits; with the workspace asked for, half of it and none; what surrounds the
     operands is NaN, and the products alone, which take other kernels, give the same."""
@@ -70,12 +78,12 @@ def test_adjoint_of_a_linear_shard_in_one_launch(dtype, M, N, K, pad, shift):
     want = [dy.double() @ w.double(), dy.double().T @ x.double(), dy.double().sum(0)]
     assert max(t.abs().max() for t in want) <= 256
     (bx, px, (ldx, _)), (bw, pw, (ldw, _)), (bd, pd, (ldd, _)) = [_strided(t, False, pad, shift) for t in (x, w, dy)]
-    lib, dt = _lib.load(), _lib.DDL_DT_BF16 if dtype == torch.bfloat16 else _lib.DDL_DT_F16
+    lib, dt = _lib.load(), {torch.bfloat16: _lib.DDL_DT_BF16, torch.float16: _lib.DDL_DT_F16, torch.float32: _lib.DDL_DT_F32}[dtype]
     aligned = int(pad == 0 and shift % 8 == 0)
     stream = torch.cuda.current_stream().cuda_stream
     for wanted in ((1, 1, 1), (1, 1, 0), (1, 0, 1), (0, 1, 0)):
         elems = lib.ddl_linear_backward_workspace_at(dt, aligned, M, N, K, ldx, ldw, ldd, *wanted)
-        for n in {elems, elems // 2, 0} if wanted[2] == 0 or M <= 4096 else {elems}:
+        for n in {elems, elems // 2, 0} if wanted[2] == 0 or M <= 2048 else {elems}:
             work = torch.full((n,), float("nan"), device="cuda") if n else None
             outs = [torch.full((s + 8,), 77.0, dtype=dtype, device="cuda") if on else None for s, on in zip((M * K, N * K, N), wanted)]
             rc = lib.ddl_linear_backward(px, pw, pd, *[None if o is None else o.data_ptr() for o in outs], dt, M, N, K, ldx, ldw, ldd,
