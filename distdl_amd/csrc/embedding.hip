@@ -1,8 +1,7 @@
 // DistributedEmbedding shard gather (reference: nn/embedding.py:244-246,
 // torch.nn.functional.embedding on the local table).  out[t] is row ids[t]-lo of
 // the table when lo <= ids[t] < hi and a row of zero bits otherwise.  Rows are
-// opaque bytes: one wavefront moves one token's row as 16-byte vectors, eight
-// vectors per lane in flight; misses issue no loads at all.
+// opaque bytes, moved 16 at a time.
 //
 // max_norm (the renormalisation F.embedding performs before the lookup): the
 // rows that are looked up are flagged, then one wavefront per flagged row forms
@@ -17,64 +16,133 @@ namespace {
 constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
-constexpr int kInFlight = 8;
-// The gather runs two tokens per workgroup.  Workgroups go to the eight XCDs in
-// turn, so a workgroup's bytes decide which address bits an XCD's stores agree
-// in: with rows of 8 KiB, four tokens per workgroup (bits 15-17) take 200.0 us on
-// configuration 3, two (14-16) 199.0, one 198.0 -- and eight (16-18) 210.
-constexpr int kGatherBlock = 128;
-constexpr int kGatherWaves = kGatherBlock / kWave;
+constexpr uint32_t kXcds = 8;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-template <typename V, typename IdT>
-__global__ __launch_bounds__(kGatherBlock) void gather_rows(const char* __restrict__ weight, int64_t ldw_bytes, int64_t nvec,
-                                                      const IdT* __restrict__ ids, int64_t n_ids, int64_t lo, int64_t hi,
-                                                      char* __restrict__ out) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kGatherWaves + threadIdx.x / kWave;
-    if (t >= n_ids) return;
+// How the rows are moved: as vectors of 16 bytes with streaming stores.  Bound by HBM, and
+// for misses by how the stores of a moment lie in it; nothing is in a cache when a step gets
+// here, so all was measured on tables, ids and outputs that change from call to call, with the
+// adjoint behind each call.
+//
+// gather_rows: 256 lanes per row, which fill it or most of it, 4 KiB after 4 KiB; its id is a
+// scalar.  131 072 ids into [16032, 4096] bf16, of which one in eight hits, 255 us with the
+// adjoint (one wavefront per row, eight vectors in flight, 275; 512 lanes 286; 256 with two
+// vectors each at a time 271; gather_vectors 279).
+// gather_vectors: the vectors of the whole output in a row, two per lane of 512, for rows that
+// 256 lanes do not fill: 60 000 ids into [16000, 3000], one in eight hits, 103 us (by rows 118,
+// by wavefronts 127).
+// ANY: rows or addresses that are no multiples of 16 bytes, any of them; the last vector
+// of a row ends with it, and neighbouring workgroups run on one XCD, whose L2 puts the lines
+// together that two of them write: 32 768 ids into [6155, 3895] bf16 114 -> 71 us, 8 416
+// into [65590, 2863] 41 -> 18, 224 into [1944, 4051] fp32 10.6 -> 4.5 (before: a vector of
+// an element's size per lane).
+template <bool ANY>
+__device__ inline u32x4 load_vector(const char* p) {
+    typedef u32x4 any __attribute__((aligned(1)));
+    return ANY ? *reinterpret_cast<const any*>(p) : *reinterpret_cast<const u32x4*>(p);
+}
+template <bool ANY>
+__device__ inline void store_vector(char* p, u32x4 v) {
+    typedef u32x4 any __attribute__((aligned(1)));
+    if (ANY) __builtin_nontemporal_store(v, reinterpret_cast<any*>(p));
+    else __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+}
+template <bool ANY>
+__device__ inline uint32_t block_number() {   // hardware deals workgroups round-robin over the XCDs
+    const uint32_t per = gridDim.x / kXcds, whole = per * kXcds;
+    return ANY && blockIdx.x < whole ? blockIdx.x % kXcds * per + blockIdx.x / kXcds : blockIdx.x;
+}
+
+template <bool ANY, typename IdT>
+__global__ __launch_bounds__(kBlock) void gather_rows(const char* __restrict__ weight, int64_t ldw_bytes, uint32_t nvec, int64_t last,
+                                                      const IdT* __restrict__ ids, int64_t lo, int64_t hi, char* __restrict__ out, int64_t row_bytes) {
+    const uint32_t t = block_number<ANY>();
     const int64_t id = static_cast<int64_t>(ids[t]);
-    const bool hit = id >= lo && id < hi;
-    V* dst = reinterpret_cast<V*>(out + t * nvec * static_cast<int64_t>(sizeof(V)));
-    if (!hit) {
-        V z;
-        __builtin_memset(&z, 0, sizeof(V));
-        for (int64_t c = lane; c < nvec; c += kWave) __builtin_nontemporal_store(z, dst + c);
-        return;
-    }
-    const V* src = reinterpret_cast<const V*>(weight + (id - lo) * ldw_bytes);
-    for (int64_t c0 = 0; c0 < nvec; c0 += kWave * kInFlight) {
-        V v[kInFlight];
-#pragma unroll
-        for (int k = 0; k < kInFlight; ++k) {
-            const int64_t c = c0 + lane + k * kWave;
-            if (c < nvec) v[k] = src[c];
-        }
-#pragma unroll
-        for (int k = 0; k < kInFlight; ++k) {
-            const int64_t c = c0 + lane + k * kWave;
-            if (c < nvec) __builtin_nontemporal_store(v[k], dst + c);
-        }
+    char* const dst = out + static_cast<int64_t>(t) * row_bytes;
+    auto place = [&](uint32_t c) { return ANY && c + 1 == nvec ? last : static_cast<int64_t>(c) * 16; };
+    if (id >= lo && id < hi) {
+        const char* const src = weight + (id - lo) * ldw_bytes;
+        for (uint32_t c = threadIdx.x; c < nvec; c += kBlock) store_vector<ANY>(dst + place(c), load_vector<ANY>(src + place(c)));
+    } else {
+        for (uint32_t c = threadIdx.x; c < nvec; c += kBlock) store_vector<ANY>(dst + place(c), u32x4{0, 0, 0, 0});
     }
 }
 
-template <typename V>
-int launch_gather(const void* w, int64_t ldw_bytes, int64_t row_bytes, const void* ids, int i64, int64_t n, int64_t lo,
-                  int64_t hi, void* out, hipStream_t s) {
-    const int64_t nvec = row_bytes / static_cast<int64_t>(sizeof(V));
-    const int64_t blocks = (n + kGatherWaves - 1) / kGatherWaves;
-    if (blocks > 0x7FFFFFFFll) return fail(DDL_E_UNSUPP, "embedding gather: more than 2^32 ids in one call");
-    if (i64)
-        hipLaunchKernelGGL((gather_rows<V, int64_t>), dim3(static_cast<uint32_t>(blocks)), dim3(kGatherBlock), 0, s,
-                           static_cast<const char*>(w), ldw_bytes, nvec, static_cast<const int64_t*>(ids), n, lo, hi,
-                           static_cast<char*>(out));
-    else
-        hipLaunchKernelGGL((gather_rows<V, int32_t>), dim3(static_cast<uint32_t>(blocks)), dim3(kGatherBlock), 0, s,
-                           static_cast<const char*>(w), ldw_bytes, nvec, static_cast<const int32_t*>(ids), n, lo, hi,
-                           static_cast<char*>(out));
-    return check_launch("gather_rows");
+constexpr int kGatherBlock = 512, kGatherVectors = 2;
+
+template <bool ANY, typename IdT>
+__global__ __launch_bounds__(kGatherBlock) void gather_vectors(const char* __restrict__ weight, int64_t ldw_bytes, uint32_t nvec, FastDiv by_nvec,
+                                                               int64_t last, const IdT* __restrict__ ids, uint32_t total, int64_t lo, int64_t hi,
+                                                               char* __restrict__ out, int64_t row_bytes) {
+    const uint32_t first = block_number<ANY>() * (kGatherBlock * kGatherVectors) + threadIdx.x;
+    u32x4 v[kGatherVectors];
+    int64_t to[kGatherVectors];
+#pragma unroll
+    for (int u = 0; u < kGatherVectors; ++u) {
+        const uint32_t i = first + u * kGatherBlock < total ? first + u * kGatherBlock : total - 1, t = fd_div(i, by_nvec), c = i - t * nvec;
+        const int64_t id = static_cast<int64_t>(ids[t]);
+        const int64_t at = ANY && c + 1 == nvec ? last : static_cast<int64_t>(c) * 16;
+        to[u] = static_cast<int64_t>(t) * row_bytes + at;
+        v[u] = u32x4{0, 0, 0, 0};
+        if (id >= lo && id < hi) {   // misses issue no load
+            v[u] = load_vector<ANY>(weight + (id - lo) * ldw_bytes + at);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kGatherVectors; ++u)
+        if (first + u * kGatherBlock < total) store_vector<ANY>(out + to[u], v[u]);
+}
+
+// Rows of less than 16 bytes: an element per lane.
+template <typename V, typename IdT>
+__global__ __launch_bounds__(kBlock) void gather_elements(const char* __restrict__ weight, int64_t ldw_bytes, uint32_t dim, FastDiv by_dim,
+                                                          const IdT* __restrict__ ids, uint32_t total, int64_t lo, int64_t hi, V* __restrict__ out) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= total) return;
+    const uint32_t t = fd_div(i, by_dim), c = i - t * dim;
+    const int64_t id = static_cast<int64_t>(ids[t]);
+    V v = 0;
+    if (id >= lo && id < hi) v = reinterpret_cast<const V*>(weight + (id - lo) * ldw_bytes)[c];
+    out[i] = v;
+}
+
+// Lanes are numbered in 31 bits, and a launch has fewer than 2^32 threads: slabs of as many ids as that takes.
+template <typename IdT>
+int launch_gather(const char* w, int64_t ldw_bytes, int64_t row_bytes, int64_t elem, const IdT* ids, int64_t n, int64_t lo, int64_t hi, char* out, hipStream_t s) {
+    const bool vectors = row_bytes >= 16, any = ((row_bytes | ldw_bytes | reinterpret_cast<intptr_t>(w) | reinterpret_cast<intptr_t>(out)) & 15) != 0;
+    const int64_t lanes = vectors ? (row_bytes + 15) / 16 : row_bytes / elem;
+    const bool by_rows = vectors && lanes * 10 >= (lanes + kBlock - 1) / kBlock * kBlock * 9;
+    const int64_t most = by_rows ? 0xFFFFFF : 0x7FFF0000ll / lanes;
+    if (lanes > 0x7FFF0000ll) return fail(DDL_E_UNSUPP, "embedding gather: rows of %lld bytes", (long long)row_bytes);
+    const FastDiv div = make_fastdiv(static_cast<uint32_t>(lanes));
+    for (int64_t first = 0; first < n; first += most) {
+        const int64_t count = n - first < most ? n - first : most;
+        const uint32_t per_row = static_cast<uint32_t>(lanes), total = static_cast<uint32_t>(by_rows ? 0 : count * lanes);
+        char* const to = out + first * row_bytes;
+        const IdT* const from = ids + first;
+        if (by_rows) {
+            const auto kernel = any ? gather_rows<true, IdT> : gather_rows<false, IdT>;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(count)), dim3(kBlock), 0, s, w, ldw_bytes, per_row, row_bytes - 16, from, lo, hi, to, row_bytes);
+        } else if (vectors) {
+            constexpr uint32_t kWidth = kGatherBlock * kGatherVectors;
+            const auto kernel = any ? gather_vectors<true, IdT> : gather_vectors<false, IdT>;
+            hipLaunchKernelGGL(kernel, dim3((total + kWidth - 1) / kWidth), dim3(kGatherBlock), 0, s, w, ldw_bytes, per_row, div, row_bytes - 16, from, total, lo,
+                               hi, to, row_bytes);
+        } else {
+            const dim3 grid((total + kBlock - 1) / kBlock), block(kBlock);
+            if (elem == 1)
+                hipLaunchKernelGGL((gather_elements<uint8_t, IdT>), grid, block, 0, s, w, ldw_bytes, per_row, div, from, total, lo, hi, reinterpret_cast<uint8_t*>(to));
+            else if (elem == 2)
+                hipLaunchKernelGGL((gather_elements<uint16_t, IdT>), grid, block, 0, s, w, ldw_bytes, per_row, div, from, total, lo, hi, reinterpret_cast<uint16_t*>(to));
+            else if (elem == 4)
+                hipLaunchKernelGGL((gather_elements<uint32_t, IdT>), grid, block, 0, s, w, ldw_bytes, per_row, div, from, total, lo, hi, reinterpret_cast<uint32_t*>(to));
+            else
+                hipLaunchKernelGGL((gather_elements<uint64_t, IdT>), grid, block, 0, s, w, ldw_bytes, per_row, div, from, total, lo, hi, reinterpret_cast<uint64_t*>(to));
+        }
+        if (int rc = check_launch("embedding gather")) return rc;
+    }
+    return 0;
 }
 
 __global__ __launch_bounds__(kBlock) void renorm_clear(int32_t* __restrict__ flags, int64_t rows) {
@@ -185,12 +253,9 @@ extern "C" int ddl_embedding_gather(const void* weight, int64_t dim, int64_t ldw
     if (!aligned_to(out, elem_size) || !aligned_to(weight, elem_size))
         return fail(DDL_E_ALIGN, "embedding gather: table or output not aligned to the element size");
     const int64_t row_bytes = dim * elem_size, ldw_bytes = ldw * elem_size;
-    const uint64_t bits = static_cast<uint64_t>(row_bytes) | static_cast<uint64_t>(ldw_bytes) |
-                          reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(out);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if ((bits & 15) == 0) return launch_gather<u32x4>(weight, ldw_bytes, row_bytes, ids, ids_is_i64, n_ids, lo, hi, out, s);
-    if ((bits & 7) == 0) return launch_gather<u32x2>(weight, ldw_bytes, row_bytes, ids, ids_is_i64, n_ids, lo, hi, out, s);
-    if ((bits & 3) == 0) return launch_gather<uint32_t>(weight, ldw_bytes, row_bytes, ids, ids_is_i64, n_ids, lo, hi, out, s);
-    if ((bits & 1) == 0) return launch_gather<uint16_t>(weight, ldw_bytes, row_bytes, ids, ids_is_i64, n_ids, lo, hi, out, s);
-    return launch_gather<uint8_t>(weight, ldw_bytes, row_bytes, ids, ids_is_i64, n_ids, lo, hi, out, s);
+    const char* const w = static_cast<const char*>(weight);
+    char* const to = static_cast<char*>(out);
+    if (ids_is_i64) return launch_gather(w, ldw_bytes, row_bytes, elem_size, static_cast<const int64_t*>(ids), n_ids, lo, hi, to, s);
+    return launch_gather(w, ldw_bytes, row_bytes, elem_size, static_cast<const int32_t*>(ids), n_ids, lo, hi, to, s);
 }
