@@ -16,11 +16,11 @@
 // four launches of a repartition of [8, 4001, 6001] bf16 over four workers and its
 // adjoint 278, now 146; of [5, 1531, 3077] 43, now 31.)
 //
-// Device side: a workgroup moves tiles of 1024 vectors shaped TR rows x TC
+// Device side: a workgroup moves a tile of 256 or 512 vectors shaped TR rows x TC
 // columns, TC a power of two (see columns_of_tile), so a vector's row and
 // column inside its tile are bit fields of its number; only the row needs
 // multiply-high divisions, and only when more than one outer dimension is left.
-// Workgroups are persistent (they stride over the tile sequence of the launch),
+// Workgroups of launches with more than a million tiles stride over them,
 // loads and stores are non-temporal, and nothing but the box table -- passed by
 // value as kernel arguments and read with scalar loads -- is read besides the
 // payload.
@@ -41,7 +41,15 @@ constexpr int kUnroll = 4;
 constexpr uint32_t kTileVecs = kThreads * kUnroll;
 constexpr uint32_t kTileLog = 10;  // log2(kTileVecs)
 static_assert((1u << kTileLog) == kTileVecs, "tile size must be 2^kTileLog");
-constexpr uint32_t kPersistentBlocks = 4096;  // 16 per CU
+constexpr uint32_t tile_log(int vectors) { return vectors == 4 ? kTileLog : vectors == 2 ? kTileLog - 1 : kTileLog - 2; }   // of a lane
+constexpr uint32_t kPersistentBlocks = 1u << 20;   // workgroups of a launch; more tiles than that are strided over
+constexpr uint32_t kSumBlocks = 4096;              // of the sum kernels, 16 per CU
+// A box kernel's lanes move two vectors each, or one in launches of less than this: a lane's vectors wait for its addresses
+// and for each other, and with fewer of them there are more workgroups to hide that.  Crop and pad of [1, 32, 128^3] fp32 with
+// its adjoint: 191 us with four (and 4096 workgroups that stride), 181 with two, 201 with one.  Strips of an exchange of
+// [2, 5, 27^3] fp32 between eight workers and its adjoint, eleven launches: 52 us with four, 45 with two, 42 with one.  A
+// repartition of [5, 1531, 3077] bf16 between four workers, 735 thousand vectors a launch: 30 us, 29 and 33.
+constexpr uint64_t kFewVectors = 1u << 19;
 constexpr uint32_t kXcds = 8;                 // workgroups are dealt to the XCDs in turn
 constexpr uint64_t kMaxVecs = (1ull << 31) - kTileVecs;
 constexpr uint64_t kLongRunBytes = 64 << 10;   // boxes whose innermost runs are at least this long are interleaved within a launch
@@ -210,9 +218,9 @@ typedef const DevBox* DevBoxPtr;
 // entries beyond a box's own count hold extent 1 and stride 0).  Every table
 // field is fetched unconditionally at the top, so the scalar loads are issued
 // together and waited for once per tile.
-template <int ND>
-__device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_t (&soff)[kUnroll], int64_t (&doff)[kUnroll],
-                                             bool (&live)[kUnroll]) {
+template <int ND, int U>
+__device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_t (&soff)[U], int64_t (&doff)[U], bool (&live)[U]) {
+    constexpr uint32_t kLog = tile_log(U);
     const uint32_t col_tiles = bx->col_tiles;
     const uint32_t tc_log = bx->tc_log;
     const uint32_t ct_mul = bx->ct_mul, ct_shr = bx->ct_shr;
@@ -231,13 +239,13 @@ __device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_
     }
     const uint32_t row_tile = col_tiles == 1 ? tile : (__umulhi(tile, ct_mul) >> ct_shr);  // wave-uniform
     const uint32_t col_tile = tile - row_tile * col_tiles;
-    const uint32_t row0 = row_tile << (kTileLog - tc_log);
+    const uint32_t row0 = row_tile << (kLog - tc_log);
     const uint32_t col0 = col_tile << tc_log;
     const uint32_t tc = 1u << tc_log;
     // wave-uniform; not a tile with a vector that starts earlier
-    const bool interior = col0 + tc + (shift != 0 ? 1u : 0u) <= cols && row0 + (kTileVecs >> tc_log) <= rows;
+    const bool interior = col0 + tc + (shift != 0 ? 1u : 0u) <= cols && row0 + ((1u << kLog) >> tc_log) <= rows;
     if (ND <= 1 && interior) {
-        // Whole tile inside the box and rows addressed by one stride: the four
+        // Whole tile inside the box and rows addressed by one stride: the
         // vectors of a lane differ by wave-uniform steps, so one position is
         // computed and the others follow by addition.
         const uint32_t j = threadIdx.x;
@@ -249,23 +257,23 @@ __device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_
             dof += static_cast<int64_t>(r) * dds[0];
         }
         // step of kThreads vectors: columns while they fit the tile row, rows after that
-        int64_t sstep[kUnroll], dstep[kUnroll];
+        int64_t sstep[U], dstep[U];
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
+        for (int u = 0; u < U; ++u) {
             const uint32_t jj = u * kThreads;                 // uniform
             const uint32_t dc = jj & (tc - 1u), dr = jj >> tc_log;
             sstep[u] = static_cast<int64_t>(dc) * css + (ND > 0 ? static_cast<int64_t>(dr) * dss[0] : 0);
             dstep[u] = static_cast<int64_t>(dc) * cds + (ND > 0 ? static_cast<int64_t>(dr) * dds[0] : 0);
         }
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
+        for (int u = 0; u < U; ++u) {
             soff[u] = so + sstep[u];
             doff[u] = dof + dstep[u];
             live[u] = true;
         }
     } else {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
+        for (int u = 0; u < U; ++u) {
             const uint32_t j = threadIdx.x + u * kThreads;   // vector number inside the tile
             uint32_t col = col0 + (j & (tc - 1u));
             uint32_t r = row0 + (j >> tc_log);
@@ -295,34 +303,34 @@ __device__ __forceinline__ void tile_offsets(DevBoxPtr bx, uint32_t tile, int64_
     }
 }
 
-template <int OP, typename T, typename V, int ND>
+template <int OP, typename T, typename V, int ND, int U>
 __device__ inline void move_tile(DevBoxPtr bx, uint32_t tile) {
-    int64_t soff[kUnroll], doff[kUnroll];
-    bool live[kUnroll];
-    tile_offsets<ND>(bx, tile, soff, doff, live);
+    int64_t soff[U], doff[U];
+    bool live[U];
+    tile_offsets<ND, U>(bx, tile, soff, doff, live);
     char* const dst = bx->dst;
     if constexpr (OP == OP_ZERO) {
         V z;
         __builtin_memset(&z, 0, sizeof(V));
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) __builtin_nontemporal_store(z, reinterpret_cast<V*>(dst + doff[u]));
+        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(z, reinterpret_cast<V*>(dst + doff[u]));
         return;
     }
     const char* const src = bx->src;
-    V val[kUnroll];
+    V val[U];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) val[u] = __builtin_nontemporal_load(reinterpret_cast<const V*>(src + soff[u]));
+    for (int u = 0; u < U; ++u) val[u] = __builtin_nontemporal_load(reinterpret_cast<const V*>(src + soff[u]));
     if constexpr (OP == OP_ADD) {
         if constexpr (sizeof(V) >= sizeof(T)) {
-            V cur[kUnroll];
+            V cur[U];
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) cur[u] = *reinterpret_cast<const V*>(dst + doff[u]);
+            for (int u = 0; u < U; ++u) cur[u] = *reinterpret_cast<const V*>(dst + doff[u]);
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) val[u] = add_vectors<T, V>(cur[u], val[u]);
+            for (int u = 0; u < U; ++u) val[u] = add_vectors<T, V>(cur[u], val[u]);
         }
         // An accumulation must happen exactly once per element.
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < U; ++u)
             if (live[u]) *reinterpret_cast<V*>(dst + doff[u]) = val[u];
         return;
     }
@@ -331,7 +339,7 @@ __device__ inline void move_tile(DevBoxPtr bx, uint32_t tile) {
         V z;
         __builtin_memset(&z, 0, sizeof(V));
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < U; ++u)
             if (live[u]) {
                 *reinterpret_cast<V*>(dst + doff[u]) = val[u];
                 *reinterpret_cast<V*>(const_cast<char*>(src) + soff[u]) = z;
@@ -339,30 +347,29 @@ __device__ inline void move_tile(DevBoxPtr bx, uint32_t tile) {
         return;
     }
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) __builtin_nontemporal_store(val[u], reinterpret_cast<V*>(dst + doff[u]));
+    for (int u = 0; u < U; ++u) __builtin_nontemporal_store(val[u], reinterpret_cast<V*>(dst + doff[u]));
 }
 
-template <int OP, typename T, typename V>
+template <int OP, typename T, typename V, int U>
 __device__ inline void move_tile_nd(DevBoxPtr bx, uint32_t tile, uint32_t nd) {
     if (nd == 0)
-        move_tile<OP, T, V, 0>(bx, tile);
+        move_tile<OP, T, V, 0, U>(bx, tile);
     else if (nd == 1)
-        move_tile<OP, T, V, 1>(bx, tile);
+        move_tile<OP, T, V, 1, U>(bx, tile);
     else if (nd == 2)
-        move_tile<OP, T, V, 2>(bx, tile);
+        move_tile<OP, T, V, 2, U>(bx, tile);
     else
-        move_tile<OP, T, V, kMaxDevDims>(bx, tile);
+        move_tile<OP, T, V, kMaxDevDims, U>(bx, tile);
 }
 
-template <int OP, typename T>
+template <int OP, typename T, int U>
 __global__ __launch_bounds__(kThreads) void box_kernel(const Batch bt_by_value) {
 #if defined(__HIP_DEVICE_COMPILE__)
     BatchPtr bt = (BatchPtr)__builtin_amdgcn_kernarg_segment_ptr();
 #else
     BatchPtr bt = &bt_by_value;
 #endif
-    // Persistent workgroups: each walks the launch's tile sequence with a
-    // stride of the grid, so a few thousand workgroups serve any volume.
+    // A workgroup has one tile, unless there are more than a launch has workgroups.
     const uint32_t nbox = bt->nbox;
     const uint32_t ntiles = bt->ntiles;
     const uint32_t rr_div = bt->rr.div, rr_mul = bt->rr.mul, rr_shr = bt->rr.shr;
@@ -385,11 +392,11 @@ __global__ __launch_bounds__(kThreads) void box_kernel(const Batch bt_by_value) 
         DevBoxPtr bx = &bt->box[bi];
         const uint32_t nd = bx->nd;
         switch (bx->vlog) {
-            case 4: move_tile_nd<OP, T, u32x4>(bx, tile, nd); break;
-            case 3: move_tile_nd<OP, T, u32x2>(bx, tile, nd); break;
-            case 2: move_tile_nd<OP, T, u32x1>(bx, tile, nd); break;
-            case 1: move_tile_nd<OP, T, u16x1>(bx, tile, nd); break;
-            default: move_tile_nd<OP, T, uint8_t>(bx, tile, nd); break;
+            case 4: move_tile_nd<OP, T, u32x4, U>(bx, tile, nd); break;
+            case 3: move_tile_nd<OP, T, u32x2, U>(bx, tile, nd); break;
+            case 2: move_tile_nd<OP, T, u32x1, U>(bx, tile, nd); break;
+            case 1: move_tile_nd<OP, T, u16x1, U>(bx, tile, nd); break;
+            default: move_tile_nd<OP, T, uint8_t, U>(bx, tile, nd); break;
         }
     }
 }
@@ -599,7 +606,7 @@ __device__ inline void sum_tile(SumArgsPtr sa, uint32_t tile) {
     DevBoxPtr bx = &sa->box;
     int64_t soff[kUnroll], doff[kUnroll];
     bool live[kUnroll];
-    tile_offsets<ND>(bx, tile, soff, doff, live);
+    tile_offsets<ND, kUnroll>(bx, tile, soff, doff, live);
     const char* const src = bx->src;
     const uint32_t nsrc = sa->nsrc;
     const double divisor = sa->divisor, reciprocal = sa->reciprocal;
@@ -774,13 +781,13 @@ struct HostDim {
     int64_t n, ss, ds;
 };
 
-// log2 of the columns of a tile of vectors of 2^vlog bytes: the power of two that covers the box, at most 1024; or a smaller
+// log2 of the columns of a tile of vectors of 2^vlog bytes: the power of two that covers the box, at most the tile's vectors; or a smaller
 // one of at least 512 bytes, the widest of which no more than an eighth lies past the box, or the one of which the least
 // does.  Lanes past the box repeat its last vector.  (Narrower tiles cover a box still better and make a wavefront's
 // addresses scatter: strips of 43 fp32 in tiles of 16 columns 12 us, in one of 64 8 to 10.)
-inline uint32_t columns_of_tile(uint32_t cols, uint32_t vlog) {
+inline uint32_t columns_of_tile(uint32_t cols, uint32_t vlog, uint32_t most) {
     uint32_t log = 0;
-    while (log < kTileLog && (1u << log) < cols) ++log;
+    while (log < most && (1u << log) < cols) ++log;
     uint32_t best = log;
     uint64_t least = ~0ull;
     for (uint32_t l = log; l == log || l + vlog >= 9; --l) {
@@ -789,6 +796,15 @@ inline uint32_t columns_of_tile(uint32_t cols, uint32_t vlog) {
         if (covered * 8 <= static_cast<uint64_t>(cols) * 9) return best;
     }
     return best;
+}
+
+// Lays the box out in tiles of 2^most vectors.
+inline void lay_out(DevBox& db, uint32_t most) {
+    db.tc_log = columns_of_tile(db.cols, db.vlog, most);
+    db.col_tiles = (db.cols + (1u << db.tc_log) - 1) >> db.tc_log;
+    const FastDiv ct = make_fastdiv(db.col_tiles);
+    db.ct_mul = ct.mul;
+    db.ct_shr = ct.shr;
 }
 
 // Rewrites one box in bytes, merges what can be merged and appends the
@@ -895,15 +911,10 @@ int lower_box(const ddl_box_t& in, int elem_size, bool has_src, bool twice, std:
         db.css = inner.ss;
         db.cds = inner.ds;
         db.rows = static_cast<uint32_t>(total / static_cast<uint64_t>(inner.n));
-        const uint32_t tc_log = columns_of_tile(db.cols, vlog);
-        db.tc_log = tc_log;
         db.shift = shift;
-        db.col_tiles = (db.cols + (1u << tc_log) - 1) >> tc_log;
-        const FastDiv ct = make_fastdiv(db.col_tiles);
-        db.ct_mul = ct.mul;
-        db.ct_shr = ct.shr;
         db.nd = static_cast<uint32_t>(p.d.size() - 1);
         db.vlog = vlog;
+        lay_out(db, kTileLog);
         for (int d = 0; d < kMaxDevDims; ++d) {
             // Unused entries (extent 1, stride 0) sit at the slow end so that the
             // general instantiation may decompose all kMaxDevDims of them.
@@ -927,7 +938,7 @@ int lower_box(const ddl_box_t& in, int elem_size, bool has_src, bool twice, std:
 
 // Whether the boxes of a batch differ in their base addresses only and consist
 // of whole tiles, so that uniform_copy_kernel can move them.
-constexpr uint64_t kUniformMaxTiles = 16384;   // 256 MiB a launch: beyond that the persistent kernel's fewer, longer-lived workgroups serve as well
+constexpr uint64_t kUniformMaxTiles = 16384;   // 256 MiB a launch: beyond that the general kernel serves as well
 inline bool uniform_batch(const Batch& bt, uint32_t n, uint64_t tiles) {
     const DevBox& a = bt.box[0];
     if (n < 1 || tiles > kUniformMaxTiles || tiles % n != 0 || tiles / n > 65535) return false;
@@ -997,23 +1008,36 @@ inline bool share_lines(const Batch& bt, uint32_t n, bool equal) {
     return src || dst;
 }
 
+// Numbers the tiles of the boxes, laid out in tiles of 2^log vectors; returns how many there are.
+inline uint64_t number_tiles(Batch& bt, uint32_t n, uint32_t log) {
+    uint64_t tiles = 0;
+    for (uint32_t k = 0; k < n; ++k) {
+        const uint64_t tr = (1u << log) >> bt.box[k].tc_log;  // rows per tile
+        bt.box[k].first_tile = bt.first_tile[k] = static_cast<uint32_t>(tiles);
+        tiles += static_cast<uint64_t>(bt.box[k].col_tiles) * ((bt.box[k].rows + tr - 1) / tr);
+    }
+    return tiles;
+}
+
 template <int OP, typename T>
 int launch_batches(const std::vector<DevBox>& boxes, hipStream_t stream) {
     size_t i = 0;
     while (i < boxes.size()) {
         Batch bt{};
-        uint64_t tiles = 0;
+        uint64_t vectors = 0;
         uint32_t n = 0;
-        while (i < boxes.size() && n < kBatch) {
-            const uint64_t tr = kTileVecs >> boxes[i].tc_log;  // rows per tile
-            const uint64_t t = static_cast<uint64_t>(boxes[i].col_tiles) * ((boxes[i].rows + tr - 1) / tr);
-            if (n > 0 && tiles + t > 0x7FFFFFFFull) break;
-            bt.box[n] = boxes[i];
-            bt.box[n].first_tile = static_cast<uint32_t>(tiles);
-            bt.first_tile[n] = static_cast<uint32_t>(tiles);
-            tiles += t;
-            ++n;
-            ++i;
+        while (i < boxes.size() && n < kBatch) {   // tiles are numbered in 31 bits, whatever their size
+            const uint64_t v = static_cast<uint64_t>(boxes[i].cols) * boxes[i].rows;
+            if (n > 0 && vectors + v > kMaxVecs) break;
+            vectors += v;
+            bt.box[n++] = boxes[i++];
+        }
+        uint64_t tiles = number_tiles(bt, n, kTileLog);
+        const bool uniform = OP == OP_COPY && uniform_batch(bt, n, tiles);
+        const int each = vectors < kFewVectors ? 1 : 2;
+        if (!uniform) {
+            for (uint32_t k = 0; k < n; ++k) lay_out(bt.box[k], tile_log(each));
+            tiles = number_tiles(bt, n, tile_log(each));
         }
         bt.nbox = n;
         bt.ntiles = static_cast<uint32_t>(tiles);
@@ -1043,7 +1067,7 @@ int launch_batches(const std::vector<DevBox>& boxes, hipStream_t stream) {
         }
         const bool interleave = equal && (long_runs || scatter);
         bt.rr = interleave ? make_fastdiv(n) : FastDiv{0, 0, 0, 0};
-        if (OP == OP_COPY && uniform_batch(bt, n, tiles)) {
+        if (uniform) {
             if (int rc = launch_uniform(bt, n, static_cast<uint32_t>(tiles / n), interleave, stream)) return rc;
             continue;
         }
@@ -1056,7 +1080,8 @@ int launch_batches(const std::vector<DevBox>& boxes, hipStream_t stream) {
             most = kPersistentBlocks / (kXcds * n) * (kXcds * n);
         }
         const uint32_t blocks = tiles < most ? static_cast<uint32_t>(tiles) : most;
-        hipLaunchKernelGGL((box_kernel<OP, T>), dim3(blocks), dim3(kThreads), 0, stream, bt);
+        const auto kernel = each == 1 ? box_kernel<OP, T, 1> : box_kernel<OP, T, 2>;
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, stream, bt);
         if (int rc = check_launch("box_kernel")) return rc;
     }
     return 0;
@@ -1186,7 +1211,7 @@ int launch_sum(const std::vector<DevBox>& pieces, const void* const* srcs, int n
             if (int rc = check_launch("sum_pieces_kernel")) return rc;
             continue;
         }
-        const uint32_t blocks = tiles < kPersistentBlocks ? static_cast<uint32_t>(tiles) : kPersistentBlocks;
+        const uint32_t blocks = tiles < kSumBlocks ? static_cast<uint32_t>(tiles) : kSumBlocks;
         if (sa.divide == kDivNone)
             hipLaunchKernelGGL((sum_kernel<T, kDivNone>), dim3(blocks), dim3(kThreads), 0, stream, sa);
         else if (sa.divide == kDivReciprocal)

@@ -241,6 +241,37 @@ def test_accumulating_unpack_matches_torch_add(ops, dtype, tol):
     assert torch.equal(bits(y.cpu()), bits(want))
 
 
+@pytest.mark.parametrize("rows,run", [(2047, 4093), (2049, 4099), (1, 300), (513, 60)])
+def test_boxes_at_the_number_of_vectors_a_lane_moves(ops, rows, run):
+    """Lanes move one vector each up to 2^19 vectors in a launch and two from there: boxes on both sides of that line, of
+    odd runs and with rows that do not fill a tile, copied both ways, accumulated, cleared and moved out, bit for bit."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(rows)
+    x_cpu = torch.randint(-9, 10, (rows, run + 3), generator=gen).float()
+    x = x_cpu.cuda()
+    sl = (slice(0, rows), slice(1, run + 1))
+    plan = ops.BoxPlan.from_slices(x, [sl])
+    buf = torch.full((rows, run), -1.0, device="cuda")
+    plan.pack(x, [buf])
+    assert torch.equal(buf.cpu(), x_cpu[sl])
+    plan.unpack(x, [buf], accumulate=True)
+    want = x_cpu.clone()
+    want[sl] *= 2
+    assert torch.equal(x.cpu(), want)
+    plan.unpack(x, [buf])
+    assert torch.equal(x.cpu(), x_cpu)
+    strides = ops.contiguous_strides(x_cpu.shape)
+    out = torch.full((rows, run), -1.0, device="cuda")
+    entry = (0, 1, 1, 0, [rows, run], strides, ops.contiguous_strides([rows, run]))
+    ops.BoxLaunch([entry], 4).run([x.data_ptr(), out.data_ptr()], op=_lib.DDL_OP_MOVE)
+    want = x_cpu.clone()
+    want[sl] = 0
+    assert torch.equal(out.cpu(), x_cpu[sl]) and torch.equal(x.cpu(), want)
+    x = x_cpu.cuda()
+    plan.zero(x)
+    assert torch.equal(x.cpu(), want)
+
+
 def test_copy_box_strided_to_strided(ops):
     gen = torch.Generator().manual_seed(21)
     src = random_bits((7, 40, 9), torch.bfloat16, gen).cuda()
