@@ -9,6 +9,14 @@
 // `splits` workgroups share the reduction of a tile through a workspace;
 // gemm32_small_sum adds their sums in the order of the splits.
 //
+// A wavefront multiplies one half of a k-tile while the other half, or the first half of the next k-tile, comes
+// from LDS, and the requests go out one or two per matrix instruction: where a CU has one workgroup, nothing else
+// fills these waits.  All reads of a k-tile first, then its products: a round 0.78 us in two groups and 0.68 in
+// one, here 0.57 and 0.54, of which the matrix cores take 0.43 (M 777, N 333, K 1024 17.0 -> 13.0 us, its adjoint
+// 22.0 -> 19.4; M = N = K = 1024 26.0 -> 20.9; M 399, N 1115, K 3264 1.5 times as fast; 4000 products of up to 8e9
+// operations 1.09 times, their adjoints 1.04).  The last rounds, with decisions in them, have a loop of their own:
+// with those in the only loop M 777 took 14.9.
+//
 // Tiles go from global memory straight into LDS through a ring of stages: k-tiles of
 // 32 floats; an operand contiguous along k in rows of 128 bytes whose 16-byte chunks are
 // XOR-ed with (row >> 1) & 7 (lane (r = lane % 32, h = lane / 32) reads chunk 2 g + h of row
@@ -28,8 +36,8 @@
 //
 // linear32_adjoint is dx, dw and db of a linear shard in one launch, for products whose
 // workgroups are all resident at once: alone each of the three leaves CUs idle and waits
-// for the one before.  M 777, N 333, K 1024 28.1 -> 21.0 us, M 97, N 77, K 603 10.9 -> 5.3, M 108, N
-// 192, K 5376 15.8 -> 10.5, M = N = K = 1024 53.9 -> 40.9.  With more workgroups the products fill
+// for the one before.  M 777, N 333, K 1024 28.1 -> 19.4 us, M 97, N 77, K 603 10.9 -> 5.3, M 108, N
+// 192, K 5376 15.8 -> 10.5, M = N = K = 1024 53.9 -> 38.5.  With more workgroups the products fill
 // the chip one after the other, and the one launch is slower (M 2078, N 6152, K 276 162, here 243).
 #include "colsum.h"
 #include "gemm_tiles.h"
@@ -112,13 +120,16 @@ __device__ __forceinline__ void small_product(const Part32& p, int number, int s
         }
         *reinterpret_cast<floatx4*>(dst + lane * 16) = floatx4{v[0], v[1], v[2], v[3]};
     };
+    constexpr int J = JW_W + JW_X;
+    auto request_piece = [&](int j, int t, char* stage) {
+        if (j < JW_W) dma16(buf_w, off_w[j], t * step_w, stage + (NW * j + wave) * 1024);
+        else dma16(buf_x, off_x[j - JW_W], t * step_x, stage + kX + (NW * (j - JW_W) + wave) * 1024);
+    };
     auto request = [&](int t, int slot) {
         char* stage = ring + slot * kStage;
         if (t < full_tiles) {
 #pragma unroll
-            for (int j = 0; j < JW_W; ++j) dma16(buf_w, off_w[j], t * step_w, stage + (NW * j + wave) * 1024);
-#pragma unroll
-            for (int j = 0; j < JW_X; ++j) dma16(buf_x, off_x[j], t * step_x, stage + kX + (NW * j + wave) * 1024);
+            for (int j = 0; j < J; ++j) request_piece(j, t, stage);
         } else {
 #pragma unroll
             for (int j = 0; j < JW_W; ++j) careful(WT, base_w, off_w[j], step_w, t, NW * j + wave, n0, N, stage + (NW * j + wave) * 1024);
@@ -146,38 +157,82 @@ __device__ __forceinline__ void small_product(const Part32& p, int number, int s
     // Group i takes k-tiles t_begin + i, + KG, ...; all groups walk the same number of rounds, for the barriers.
     const int rounds = (t_end - t_begin + KG - 1) / KG;
     auto tile_at = [&](int r) { return t_begin + r * KG + group; };
-#pragma unroll
-    for (int i = 0; i < STAGES - 1; ++i)
+#pragma unroll 1   // unrolled, the instructions of four requests are what a short product waits for
+    for (int i = 0; i < STAGES; ++i)
         if (tile_at(i) < t_end) request(tile_at(i), i);
-    int slot = 0;
-#pragma unroll 1
-    for (int r = 0; r < rounds; ++r) {
-        // This wavefront's requests of tile r have landed (those of the STAGES - 2 tiles behind it may be in flight if all
-        // went out as requests) and its LDS reads of tile r - 1 have returned: behind the barrier tile r is readable and
-        // the slot of tile r - 1 is free.
-        const int last = tile_at(r + STAGES - 2);
+    // Requests up to tile r - 1 of this group have landed and this wavefront's LDS reads have returned; the `behind` tiles
+    // from r on may be in flight if all went out as requests.
+    auto landed = [&](int r, auto behind) {
+        const int last = tile_at(r + decltype(behind)::value - 1);
         if (last < t_end && last < full_tiles)
-            __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((STAGES - 2) * (JW_W + JW_X)));
+            __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(decltype(behind)::value * J));
         else
             __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (tile_at(r + STAGES - 1) < t_end) request(tile_at(r + STAGES - 1), slot == 0 ? STAGES - 1 : slot - 1);
-        if (KG > 1 && tile_at(r) >= t_end) continue;   // the last round of a group that has one tile less
+    };
+    floatx4 fw[4], fx[4];
+    auto read_half = [&](int slot, auto half) {
+        constexpr int g0 = decltype(half)::value * 2;
         const char* wt = ring + slot * kStage;
         const char* xt = wt + kX;
-        floatx4 fw[4], fx[4];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
+        for (int g = g0; g < g0 + 2; ++g) {
             fw[g] = fragment(std::integral_constant<bool, WT>{}, wt, sub_w, g);
             fx[g] = fragment(std::integral_constant<bool, XT>{}, xt, sub_x, g);
         }
-        __builtin_amdgcn_sched_barrier(0);   // all reads first: left alone, the compiler puts each pair in front of its MFMAs
+        __builtin_amdgcn_sched_barrier(0);   // left alone, the compiler puts each pair in front of its MFMAs
+    };
+    auto multiply = [&](auto half, auto from, auto upto) {   // instructions [from, upto) of eight
+        constexpr int g0 = decltype(half)::value * 2;
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fw[g][e], fx[g][e], acc, 0, 0, 0);
+        for (int i = decltype(from)::value; i < decltype(upto)::value; ++i)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fw[g0 + i / 4][i % 4], fx[g0 + i / 4][i % 4], acc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    typedef std::integral_constant<int, 0> First;
+    typedef std::integral_constant<int, 1> Second;
+    typedef std::integral_constant<int, 8> End;
+    // Seven instructions on one half of a k-tile hide the reads of the other half, or of the first half of the next k-tile.
+    // The one in front of the reads has waited for what came before them.
+    landed(1, std::integral_constant<int, STAGES - 1>{});
+    read_half(0, First{});
+    int slot = 0, r = 0;
+    // While all that is requested goes out as requests: nothing to decide, and an instruction's shadow has at most two of them.
+    const int plain = (t_end < full_tiles ? t_end : full_tiles) - t_begin - group;   // tiles of the range, counted from the group's first
+#pragma unroll 1
+    for (; (r + STAGES) * KG < plain; ++r) {
+        multiply(First{}, First{}, Second{});
+        read_half(slot, Second{});
+        multiply(First{}, Second{}, End{});
+        __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((STAGES - 2) * J));   // tile r + 1 is readable, the slot of tile r free
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        char* const stage = ring + slot * kStage;
         slot = slot + 1 == STAGES ? 0 : slot + 1;
+        multiply(Second{}, First{}, Second{});
+        read_half(slot, First{});
+#pragma unroll
+        for (int i = 1; i < 8; ++i) {
+#pragma unroll
+            for (int j = (i - 1) * J / 7; j < i * J / 7; ++j) request_piece(j, tile_at(r + STAGES), stage);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fw[2 + i / 4][i % 4], fx[2 + i / 4][i % 4], acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll 1
+    for (; r < rounds; ++r) {
+        if (KG > 1 && tile_at(r) >= t_end) break;   // the last round of a group that has one tile less
+        multiply(First{}, First{}, Second{});
+        read_half(slot, Second{});
+        multiply(First{}, Second{}, End{});
+        if (r + 1 < rounds) landed(r + 2, std::integral_constant<int, STAGES - 2>{});
+        const int next = slot + 1 == STAGES ? 0 : slot + 1;
+        multiply(Second{}, First{}, Second{});
+        read_half(next, First{});   // behind the last tile what the slot holds, for nothing
+        if (tile_at(r + STAGES) < t_end) request(tile_at(r + STAGES), slot);
+        multiply(Second{}, Second{}, End{});
+        slot = next;
     }
     // Lane holds row m = l32 and columns n = 8 g + 4 kh + {0..3} in acc[4 g + {0..3}].
     floatx4 quad[4];
@@ -347,9 +402,10 @@ int launch_adjoint(const Adjoint32& p, int dev, hipStream_t s) {
 // round of one k-tile for every group) 0.68 for a lone 64 x 64 tile, 0.52 for each that a CU has to work through, 0.78 in
 // two or four groups + the epilogue of every further tile + for splits a second launch (2.3, and 5 for
 // what it and the workspace cost the host, which many callers wait for) and the partial tiles at 5 TB/s.
-// Measured, general kernel of 128 x 128 tiles -> here: M 777, N 333, K 1024 107.2 -> 17.7 (two groups; 15.7 in three
-// splits, which the host's share makes the slower call); its adjoint M 777, N 1024, K 333 45.4 -> 12.4 and M 333, N 1024, K 777, both operands along their rows, 84.1 ->
-// 15.6; M 8, N 4096, K 4096 365 -> 20.
+// They were fitted before the loop's halves overlapped, which takes 0.54, 0.48 and 0.57 where they say 0.68, 0.52 and 0.78; with
+// those the choice is no better (4000 shapes, the product 1.02 times as fast and its adjoint as fast, single ones 0.6 to 1.6:
+// fewer splits of long reductions, and products that linear_f32_split.hip has the lead in).
+// Measured, general kernel of 128 x 128 tiles -> here: M 777, N 333, K 1024 107.2 -> 13.0 (two groups); M 8, N 4096, K 4096 365 -> 16.3.
 Small32 plan_small32(int64_t M, int64_t N, int64_t K, int cus, int64_t workspace) {
     Small32 best;
     const int64_t ktiles = (K + BK - 1) / BK;

@@ -1,5 +1,6 @@
 """16-bit products of operands at any address and pitch: the tiles of 64 and of 128 rows and columns, whole and split reductions,
-the k-tile that needs care, reductions shorter than a load.  (The small tiles' own cases are in test_gpu_layers.py.)"""
+the k-tile that needs care, reductions shorter than a load; and the rings of the fp32 products.  (The small tiles' own cases are in
+test_gpu_layers.py.)"""
 
 import pytest
 import torch
@@ -49,6 +50,29 @@ def test_products_of_operands_at_any_address(dtype, a_t, b_t, M, N, K, pad, shif
         _lib.check(rc, "ddl_gemm_ws")
         assert torch.equal(out[:, :N].double(), want)
         assert (out[:, N:] == 77.0).all()
+
+
+@pytest.mark.parametrize("a_t,b_t", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N", [(33, 31), (777, 333), (1024, 1021)])
+def test_fp32_reductions_around_the_ring_of_stages(a_t, b_t, M, N):
+    """Four, two and one group of wavefronts that take alternate k-tiles of 32 through rings of four: reductions that fill the
+    rings or not, leave the last groups a tile less, end with a k-tile of one element or one short of a whole one.  Integers, so
+    equal to the sums in 64 bits."""
+    from distdl_amd import _lib
+    lib = _lib.load()
+    for tiles in (1, 3, 4, 5, 7, 9, 10, 16, 17, 19, 21, 34):
+        for K in (32 * tiles - 1, 32 * tiles, 32 * tiles + 1):
+            gen = torch.Generator(device="cuda").manual_seed(M + K)
+            a, b = (torch.randint(-4, 5, (n, K), generator=gen, device="cuda").float() for n in (M, N))
+            _, pa, (a_rs, a_ks) = kept_a = _strided(a, a_t, 0, 0)
+            _, pb, (b_rs, b_ks) = kept_b = _strided(b, b_t, 1, 1)
+            out = torch.full((M, N + 1), 77.0, device="cuda")
+            rc = lib.ddl_gemm_ws(pa, a_rs, a_ks, pb, b_rs, b_ks, None, out.data_ptr(), _lib.DDL_DT_F32, N + 1, M, N, K, None, 0,
+                                 torch.cuda.current_stream().cuda_stream)
+            _lib.check(rc, "ddl_gemm_ws")
+            assert torch.equal(out[:, :N].double(), a.double() @ b.double().T), K
+            assert (out[:, N] == 77.0).all()
+            del kept_a, kept_b
 
 
 _ADJOINTS = [
