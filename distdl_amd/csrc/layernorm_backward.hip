@@ -688,6 +688,23 @@ int64_t param_splits(int64_t rows, int64_t cols, int64_t workspace_elems, int64_
     return splits;
 }
 
+// Row splits of the sums over rows and columns together (ddl_ln_bwd_partial_params), for rows that ln_bwd_block_rows takes: one
+// of 1024 threads fills a CU, so four rows each up to half the CUs; from there on eight, because the launch behind it reads the
+// column sums of every split.  The times are at ddl_ln_bwd_partial_params.
+int64_t block_row_splits(int64_t rows) {
+    const int64_t four = (rows + 3) / 4, eight = (rows + 7) / 8;
+    const int64_t splits = four < 128 ? four : eight < 128 ? 128 : eight < 256 ? eight : 256;
+    return splits > 0 ? splits : 1;
+}
+
+bool by_block_rows(int64_t cols) { return cols > 4 * kWave * 4 && cols <= block_rows_cols(false); }
+
+// With less room than that: splits for the two passes one after the other.
+int64_t joint_splits(int64_t rows, int64_t cols, int64_t workspace_elems) {
+    const int64_t splits = block_row_splits(rows);
+    return by_block_rows(cols) && workspace_elems / (2 * cols) >= splits ? splits : param_splits(rows, cols, workspace_elems);
+}
+
 template <typename T>
 const T* as(const void* p) { return static_cast<const T*>(p); }
 template <typename T>
@@ -785,7 +802,7 @@ extern "C" int ddl_ln_bwd_partial_params(const void* dy, const void* x, int dtyp
     if (!elem) return fail(DDL_E_UNSUPP, "ln backward sums: dtype %d (f32, bf16, f16 only)", dtype);
     if (int rc = check_rows("ln backward sums", rows, cols, ld_dy, ld_x)) return rc;
     if (!workspace) return fail(DDL_E_ARG, "ln backward sums: null workspace");
-    const int64_t splits = param_splits(rows, cols, workspace_elems);
+    const int64_t splits = joint_splits(rows, cols, workspace_elems);
     if (splits < 1) return fail(DDL_E_ARG, "ln backward sums: workspace of %lld floats is smaller than 2 x %lld", (long long)workspace_elems, (long long)cols);
     if (rows > 0 && (!dy || !x || !mean || !rstd || !sums)) return fail(DDL_E_ARG, "ln backward sums: null pointer");
     if (!elems_aligned(elem, {dy, x, gamma}) || !aligned_to(mean, 4) || !aligned_to(rstd, 4) || !aligned_to(sums, 8) || !aligned_to(workspace, 4))
@@ -803,9 +820,11 @@ extern "C" int ddl_ln_bwd_partial_params(const void* dy, const void* x, int dtyp
         });
         return check_launch("ln_bwd_partial_cols");
     }
-    // One read of dy and x instead of two, where every CU gets a split: [8192, 8192] bf16 with the dx launch 187 -> 132 us,
-    // but [1024, 8192] (32 splits) 43 -> 58 and rows of a few hundred elements 10.6 -> 24.
-    if (splits == 256 && cols > 4 * kWave * 4 && cols <= block_rows_cols(vec)) {
+    // One read of dy and x instead of two.  Event time with the dx launch, the two passes -> here: [5727, 4352] bf16 62.9 -> 49.3
+    // us, fp32 103.9 -> 78.6; [2607, 2000] 20.9 -> 18.0; [1500, 5501] 40.5 -> 29.8; [1000, 4000] 25.2 -> 21.8; [512, 2176] 17.0 ->
+    // 13.3; [256, 8192] 29.5 -> 22.7; fp32 rows of 1028 to 1531 columns are alike around 1000 of them (14.3 and 14.5).  In splits
+    // of 32 rows [1024, 8192] took 58 us instead of 43.  Rows longer than those of by_block_rows: where every CU gets a split.
+    if ((by_block_rows(cols) && splits == block_row_splits(rows)) || (splits == 256 && cols > 4 * kWave * 4 && cols <= block_rows_cols(vec))) {
         with_ln_element(dtype, [&](auto* tag) {
             using T = std::remove_pointer_t<decltype(tag)>;
             launch_block_rows<T, false>(vec, as<T>(dy), as<T>(x), rows, cols, ld_dy, ld_x, mean, rstd, as<T>(gamma), sums, splits, workspace, 0.f,
@@ -837,7 +856,7 @@ extern "C" int ddl_ln_bwd_input_params(const void* dy, const void* x, int dtype,
     if (int rc = check_rows("ln backward input", rows, cols, ld_dy, ld_x)) return rc;
     if (ld_dx < cols || nparts < 1) return fail(DDL_E_ARG, "ln backward input: ld_dx=%lld nparts=%d", (long long)ld_dx, nparts);
     if (!workspace) return fail(DDL_E_ARG, "ln backward input: null workspace");
-    const int64_t splits = param_splits(rows, cols, workspace_elems);
+    const int64_t splits = joint_splits(rows, cols, workspace_elems);
     if (splits < 1) return fail(DDL_E_ARG, "ln backward input: workspace of %lld floats is smaller than 2 x %lld", (long long)workspace_elems, (long long)cols);
     if (rows > 0 && (!dy || !x || !mean || !rstd || !part_sums || !dx)) return fail(DDL_E_ARG, "ln backward input: null pointer");
     if (!elems_aligned(elem, {dy, x, gamma, dx, dgamma, dbeta}) || !aligned_to(mean, 4) || !aligned_to(rstd, 4) || !aligned_to(part_sums, 8) ||

@@ -622,6 +622,14 @@ def _ln_param_workspace(rows, cols, device):
     return torch.empty(2 * splits * cols, dtype=torch.float32, device=device)
 
 
+def _ln_joint_workspace(rows, cols, device):
+    """For ``ddl_ln_bwd_partial_params``: rows of 1025 to 8192 columns are summed in splits of four to eight rows."""
+    if not 1024 < cols <= 8192:
+        return _ln_param_workspace(rows, cols, device)
+    splits = max(1, min(256, max(min((rows + 3) // 4, 128), (rows + 7) // 8)))
+    return torch.empty(2 * splits * cols, dtype=torch.float32, device=device)
+
+
 def ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma):
     """``ln_backward_partial`` plus, in the same pass, the partial column sums
     for the parameter gradients.  Returns (sums [rows, 2], workspace); hand the
@@ -633,7 +641,7 @@ def ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma):
     ld_dy, ld_x = _rows2d(dy2d, "ln_backward_partial_params"), _rows2d(x2d, "ln_backward_partial_params")
     rows, cols = x2d.shape
     sums = torch.empty((rows, 2), dtype=torch.float32, device=x2d.device)
-    work = _ln_param_workspace(rows, cols, x2d.device)
+    work = _ln_joint_workspace(rows, cols, x2d.device)
     dt = _ln_bwd_dtype("ln_backward_partial_params", dy2d, x2d, gamma)
     rc = _lib.load().ddl_ln_bwd_partial_params(dy2d.data_ptr(), x2d.data_ptr(), dt, rows, cols, ld_dy, ld_x,
                                                mean.data_ptr(), rstd.data_ptr(), _ptr(gamma), sums.data_ptr(),

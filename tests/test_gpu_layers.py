@@ -713,6 +713,44 @@ def test_layer_norm_backward_of_long_whole_rows(ops, rows, cols, pad, dtype):
             assert bool((err <= ulp * want.abs() + 2e-6 * size).all()), float(err.max())
 
 
+@pytest.mark.parametrize("rows,cols,pad", [(1, 1025, 0), (4, 8192, 0), (5, 1028, 3), (509, 1026, 0), (513, 2049, 1), (1023, 1536, 0), (1025, 1100, 0),
+                                           (2049, 1025, 0), (9, 8193, 0), (3, 1024, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layer_norm_row_and_column_sums_in_one_pass(ops, rows, cols, pad, dtype):
+    """Row sums and column sums of shared rows where the number of row splits changes, with the room that the layer hands
+    over and with room for fewer splits and for one, against float64."""
+    gen = torch.Generator().manual_seed(rows * 11 + cols)
+    store = torch.randn(2, rows, cols + pad, generator=gen).to(dtype)
+    gamma = (1 + 0.1 * torch.randn(cols, generator=gen)).to(dtype)
+    mean, rstd = 0.1 * torch.randn(rows, generator=gen), 1 + 0.1 * torch.rand(rows, generator=gen)
+    x, dy = store[0, :, :cols].double(), store[1, :, :cols].double()
+    xhat = (x - mean.double()[:, None]) * rstd.double()[:, None]
+    g = dy * gamma.double()
+    want = ((g.sum(1), 4 * cols ** 0.5), ((g * xhat).sum(1), 4 * cols ** 0.5), ((dy * xhat).sum(0), 4 * rows ** 0.5), (dy.sum(0), 4 * rows ** 0.5))
+    sg, gg, mg, rg = store.cuda(), gamma.cuda(), mean.cuda(), rstd.cuda()
+    xg, dyg = sg[0, :, :cols], sg[1, :, :cols]
+    from distdl_amd import _lib
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    code = _lib.DDL_DT_F32 if dtype == torch.float32 else _lib.DDL_DT_BF16
+    ulp = 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -8
+    def by_hand(room):   # ddl_* with room for as many splits
+        sums, work = torch.empty(rows, 2, device="cuda"), torch.empty(2 * room * cols, device="cuda")
+        dx, dg, db = torch.empty(rows, cols, dtype=dtype, device="cuda"), torch.empty_like(gg), torch.empty_like(gg)
+        at = (dyg.data_ptr(), xg.data_ptr(), code, rows, cols, cols + pad, cols + pad, mg.data_ptr(), rg.data_ptr(), gg.data_ptr())
+        assert lib.ddl_ln_bwd_partial_params(*at, sums.data_ptr(), work.data_ptr(), work.numel(), stream) == 0
+        assert lib.ddl_ln_bwd_input_params(*at, sums.data_ptr(), 1, 1.0 / cols, dx.data_ptr(), cols, work.data_ptr(), work.numel(), dg.data_ptr(),
+                                           db.data_ptr(), stream) == 0
+        return sums, dg, db
+    def by_layer():
+        sums, work = ops.ln_backward_partial_params(dyg, xg, mg, rg, gg)
+        return (sums, *ops.ln_backward_input_params(dyg, xg, mg, rg, gg, sums.unsqueeze(0).contiguous(), 1.0 / cols, work)[1:])
+    for sums, dg, db in (by_layer(), by_hand(256), by_hand((rows + 31) // 32), by_hand(1)):
+        # fp32 sums of terms around one: a few units of sqrt(terms); parameters rounded once to their type
+        for (value, size), got, rounding in zip(want, (sums[:, 0], sums[:, 1], dg, db), (0, 0, ulp, ulp)):
+            err = (got.cpu().double() - value).abs()
+            assert bool((err <= rounding * value.abs() + 2e-6 * size).all()), float(err.max())
+
+
 @pytest.mark.parametrize("dtype,ulp", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)])
 @pytest.mark.parametrize("cols", [[256, 256], [300, 212], [7, 9], [2048], [1030]])
 def test_layernorm_backward_16_bit_elements(ops, dtype, ulp, cols):
