@@ -583,7 +583,6 @@ __device__ inline V div_vector(V s, double d, double r) {
 
 constexpr int kMaxSumSources = 64;
 constexpr int kSumPiecesSources = 5;        // from this many sources on, whole-tile boxes take sum_pieces_kernel
-constexpr uint32_t kSumGroup = 2;   // 2: 27.6 us for eight [4,2048,1024] bf16 slabs, 1: 29.5 us, 4: 31.0 us (registers cost more wavefronts than the loads gain)
 
 struct SumArgs {
     DevBox box;                        // src: the box in source 0
@@ -601,60 +600,66 @@ typedef const SumArgs __attribute__((address_space(4))) * SumArgsPtr;
 typedef const SumArgs* SumArgsPtr;
 #endif
 
-template <typename T, typename V, int ND, uint32_t MODE>
+// U vectors of a lane, eight loads in flight: four vectors of two sources, or one of eight where a launch of the former would
+// have few workgroups (its chain is short of loads, not of bandwidth).  Four -> one vector a lane: [372, 242] of eight bf16 sources
+// 6.7 -> 4.0 us, [1784, 434] 7.3 -> 5.4, fp32 11.3 -> 8.4, [2322, 32] bf16 7.5 -> 3.9, but fp32 [6296, 406] 18.1 -> 19.4 (from
+// kFewVectors on).  With two to four sources the rest of the eight loads is for nothing: bf16 [372, 483] of four 5.1 -> 3.8, but
+// [1784, 868] 5.9 -> 6.2 and of two 6.8 -> 9.2 (from an eighth of that on).
+template <typename T, typename V, int ND, uint32_t MODE, int U>
 __device__ inline void sum_tile(SumArgsPtr sa, uint32_t tile) {
     DevBoxPtr bx = &sa->box;
-    int64_t soff[kUnroll], doff[kUnroll];
-    bool live[kUnroll];
-    tile_offsets<ND, kUnroll>(bx, tile, soff, doff, live);
+    int64_t soff[U], doff[U];
+    bool live[U];
+    tile_offsets<ND, U>(bx, tile, soff, doff, live);
     const char* const src = bx->src;
     const uint32_t nsrc = sa->nsrc;
     const double divisor = sa->divisor, reciprocal = sa->reciprocal;
-    // Sources are fetched kSumGroup at a time (all their loads issued before the first addition) and added in order.
-    V acc[kUnroll];
-    for (uint32_t q0 = 0; q0 < nsrc; q0 += kSumGroup) {
-        V val[kSumGroup][kUnroll];
+    constexpr uint32_t kGroup = 8 / U;
+    // Sources are fetched kGroup at a time (all their loads issued before the first addition) and added in order.
+    V acc[U];
+    for (uint32_t q0 = 0; q0 < nsrc; q0 += kGroup) {
+        V val[kGroup][U];
 #pragma unroll
-        for (uint32_t g = 0; g < kSumGroup; ++g) {
+        for (uint32_t g = 0; g < kGroup; ++g) {
             const uint32_t q = q0 + g < nsrc ? q0 + g : nsrc - 1;   // past the end: the last source again, fetched and not added
             const char* const sq = src + sa->delta[q];
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) val[g][u] = __builtin_nontemporal_load(reinterpret_cast<const V*>(sq + soff[u]));
+            for (int u = 0; u < U; ++u) val[g][u] = __builtin_nontemporal_load(reinterpret_cast<const V*>(sq + soff[u]));
         }
 #pragma unroll
-        for (uint32_t g = 0; g < kSumGroup; ++g) {
+        for (uint32_t g = 0; g < kGroup; ++g) {
             if (q0 + g >= nsrc) break;
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) val[g][u] = div_vector<T, V, MODE>(val[g][u], divisor, reciprocal);
+            for (int u = 0; u < U; ++u) val[g][u] = div_vector<T, V, MODE>(val[g][u], divisor, reciprocal);
             if (q0 + g == 0) {
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u) acc[u] = val[g][u];
+                for (int u = 0; u < U; ++u) acc[u] = val[g][u];
             } else {
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u) acc[u] = add_vectors<T, V>(acc[u], val[g][u]);
+                for (int u = 0; u < U; ++u) acc[u] = add_vectors<T, V>(acc[u], val[g][u]);
             }
         }
     }
     // The destination may be one of the sources: an element is written by the one lane that owns it.
     char* const dst = bx->dst;
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
+    for (int u = 0; u < U; ++u)
         if (live[u]) __builtin_nontemporal_store(acc[u], reinterpret_cast<V*>(dst + doff[u]));
 }
 
-template <typename T, typename V, uint32_t MODE>
+template <typename T, typename V, uint32_t MODE, int U>
 __device__ inline void sum_tile_nd(SumArgsPtr sa, uint32_t tile, uint32_t nd) {
     if (nd == 0)
-        sum_tile<T, V, 0, MODE>(sa, tile);
+        sum_tile<T, V, 0, MODE, U>(sa, tile);
     else if (nd == 1)
-        sum_tile<T, V, 1, MODE>(sa, tile);
+        sum_tile<T, V, 1, MODE, U>(sa, tile);
     else if (nd == 2)
-        sum_tile<T, V, 2, MODE>(sa, tile);
+        sum_tile<T, V, 2, MODE, U>(sa, tile);
     else
-        sum_tile<T, V, kMaxDevDims, MODE>(sa, tile);
+        sum_tile<T, V, kMaxDevDims, MODE, U>(sa, tile);
 }
 
-template <typename T, uint32_t MODE>
+template <typename T, uint32_t MODE, int U>
 __global__ __launch_bounds__(kThreads) void sum_kernel(const SumArgs args_by_value) {
 #if defined(__HIP_DEVICE_COMPILE__)
     SumArgsPtr sa = (SumArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
@@ -666,13 +671,13 @@ __global__ __launch_bounds__(kThreads) void sum_kernel(const SumArgs args_by_val
     for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         // A vector holds whole elements: the host lowers the box with the element size as the narrowest vector.
         if (vlog == 4)
-            sum_tile_nd<T, u32x4, MODE>(sa, tile, nd);
+            sum_tile_nd<T, u32x4, MODE, U>(sa, tile, nd);
         else if (vlog == 3) {
-            if constexpr (sizeof(T) <= 8) sum_tile_nd<T, u32x2, MODE>(sa, tile, nd);
+            if constexpr (sizeof(T) <= 8) sum_tile_nd<T, u32x2, MODE, U>(sa, tile, nd);
         } else if (vlog == 2) {
-            if constexpr (sizeof(T) <= 4) sum_tile_nd<T, u32x1, MODE>(sa, tile, nd);
+            if constexpr (sizeof(T) <= 4) sum_tile_nd<T, u32x1, MODE, U>(sa, tile, nd);
         } else {
-            if constexpr (sizeof(T) <= 2) sum_tile_nd<T, u16x1, MODE>(sa, tile, nd);
+            if constexpr (sizeof(T) <= 2) sum_tile_nd<T, u16x1, MODE, U>(sa, tile, nd);
         }
     }
 }
@@ -1211,13 +1216,22 @@ int launch_sum(const std::vector<DevBox>& pieces, const void* const* srcs, int n
             if (int rc = check_launch("sum_pieces_kernel")) return rc;
             continue;
         }
-        const uint32_t blocks = tiles < kSumBlocks ? static_cast<uint32_t>(tiles) : kSumBlocks;
+        const bool few = static_cast<uint64_t>(sa.box.cols) * sa.box.rows < (nsrc > 4 ? kFewVectors : kFewVectors / 8);
+        if (few) {
+            lay_out(sa.box, tile_log(1));
+            const uint64_t rows_each = (1u << tile_log(1)) >> sa.box.tc_log;
+            sa.ntiles = static_cast<uint32_t>(sa.box.col_tiles * ((sa.box.rows + rows_each - 1) / rows_each));
+        }
+        const uint32_t blocks = sa.ntiles < kSumBlocks ? sa.ntiles : kSumBlocks;
+#define DDL_LAUNCH_SUM(MODE) \
+    hipLaunchKernelGGL((few ? sum_kernel<T, MODE, 1> : sum_kernel<T, MODE, kUnroll>), dim3(blocks), dim3(kThreads), 0, stream, sa)
         if (sa.divide == kDivNone)
-            hipLaunchKernelGGL((sum_kernel<T, kDivNone>), dim3(blocks), dim3(kThreads), 0, stream, sa);
+            DDL_LAUNCH_SUM(kDivNone);
         else if (sa.divide == kDivReciprocal)
-            hipLaunchKernelGGL((sum_kernel<T, kDivReciprocal>), dim3(blocks), dim3(kThreads), 0, stream, sa);
+            DDL_LAUNCH_SUM(kDivReciprocal);
         else
-            hipLaunchKernelGGL((sum_kernel<T, kDivDivide>), dim3(blocks), dim3(kThreads), 0, stream, sa);
+            DDL_LAUNCH_SUM(kDivDivide);
+#undef DDL_LAUNCH_SUM
         if (int rc = check_launch("sum_kernel")) return rc;
     }
     return 0;

@@ -732,6 +732,19 @@ def test_sum_boxes_of_many_sources_over_whole_tiles(ops, dtype, nsrc, rows, row_
         assert torch.equal(bits(dev[2].cpu())[untouched], bits(srcs[2])[untouched])
 
 
+@pytest.mark.parametrize("nsrc,rows,cols", [(2, 255, 2056), (2, 256, 2048), (4, 257, 2056), (5, 1023, 4104), (5, 1025, 4096), (9, 700, 13), (8, 3, 2055),
+                                            (8, 2000, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sum_boxes_on_either_side_of_one_vector_a_lane(ops, dtype, nsrc, rows, cols):
+    """Boxes of just under and just over the vectors up to which a lane has one, and of few and narrow ones, divided by three."""
+    gen = torch.Generator().manual_seed(nsrc + rows + cols)
+    srcs = [torch.randn(rows, cols + 3, generator=gen).to(dtype) for _ in range(nsrc)]
+    box, full = (slice(0, rows), slice(2, 2 + cols)), (slice(0, rows), slice(0, cols))
+    out = torch.zeros(rows, cols, dtype=dtype, device="cuda")
+    ops.sum_boxes([t.cuda() for t in srcs], box, out, full, 3)
+    assert torch.equal(bits(out.cpu()), bits(_sequential_sum([t[box] for t in srcs], 3)))
+
+
 def test_sum_boxes_in_place_and_fallbacks(ops):
     """The destination may be one of the sources (scaling a gradient in place);
     sources that are not 16 bytes apart, or more than 64 of them, go through
