@@ -226,3 +226,20 @@ def test_linear_of_more_rows_than_small_tiles_have_workgroups_for(ops):
     w = torch.full((1, 1), 1.5, device="cuda")
     y = ops.linear(x, w)
     assert y.shape == x.shape and torch.equal(y, x.mul_(1.5))
+
+
+def test_layer_norm_backward_takes_the_last_rows_first(ops):
+    """dy, x and dx of just more than 256 MiB together: rows are walked from the last to the first.  Column sums of small
+    integers are exact; dx against the same rows in a call of their own, which are walked the other way."""
+    rows, cols = 43700, 1025
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x, dy = (torch.randint(-4, 5, (rows, cols), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    gamma = torch.randint(1, 3, (cols,), generator=gen, device="cuda").to(torch.bfloat16)
+    mean, rstd = torch.zeros(rows, device="cuda"), torch.ones(rows, device="cuda")
+    assert 3 * x.numel() * 2 > 1 << 28
+    dx, dg, db = ops.ln_backward_whole_rows(dy, x, mean, rstd, gamma, 1.0 / cols)
+    assert torch.equal(dg, (dy.double() * x.double()).sum(0).to(torch.bfloat16)) and torch.equal(db, dy.double().sum(0).to(torch.bfloat16))
+    for first in (0, 21850, rows - 700):
+        part = slice(first, first + 700)
+        alone, _, _ = ops.ln_backward_whole_rows(dy[part], x[part], mean[part], rstd[part], gamma, 1.0 / cols)
+        assert torch.equal(alone, dx[part])
