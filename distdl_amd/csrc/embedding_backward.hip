@@ -14,7 +14,8 @@
 //   emb_bwd_split    tokens of a chunk of ids sorted by segment; segment s owns the rows s, s + G, s + 2 G, ... of the
 //                    table (frequent ids are neighbours in a vocabulary sorted by frequency: so they spread)
 //   emb_bwd_buckets  a workgroup per segment: counts and places its tokens with counters in LDS.  Nothing has to be cleared,
-//                    and a row that many tokens share costs LDS atomics of one workgroup
+//                    and a row that many tokens share costs LDS atomics of one workgroup.  Few tokens are read by every
+//                    workgroup, without emb_bwd_split in front
 //   with less workspace than these take, or a table of more than 2^23 rows, four launches instead:
 //   emb_bwd_clear    counters = 0
 //   emb_bwd_count    count[row]++ per token in the window
@@ -168,7 +169,9 @@ __global__ __launch_bounds__(kBlock) void emb_bwd_fill(const IdT* __restrict__ i
 // Bound by latency: launches, LDS atomics, a few dependent trips to L2.  Measured, four launches -> two: 131072 uniform
 // tokens over 128256 ids, 16032 of them rows, 20 -> 10.5 us; as in text (11000 tokens on one row) 92 -> 28 us; 8192 tokens as
 // in text over 50304 rows 19 -> 16 us with the buckets left in order, which takes the hot rows' kernel 6 us less; 16 tokens
-// 7.6 -> 7.3 us.  (One launch whose workgroups each look at all tokens: 7 us for 8192 tokens, but 24 for 131072, 79 as in text.)
+// 7.6 -> 7.3 us.  Up to kOneTokens tokens one launch, whose workgroups each look at all of them, does (24 us for 131072 tokens, 79 as
+// in text).  The whole gradient, two launches -> one: 8192 tokens as in text, [50304, 512] fp32 41.7 -> 39.8 us, 2048 33.3 -> 29.8;
+// 4000, [2000, 64] 26.3 -> 22.7; 856, [2538, 1210] bf16 14.7 -> 11.7; 16, [125, 64] 9.7 -> 7.3.
 constexpr int kSplitBlock = 256;
 constexpr int kBucketBlock = 1024;
 constexpr int kChunks = 1024;                     // chunks of tokens, at most
@@ -177,6 +180,10 @@ constexpr int kSegments = 2048;                   // segments, at most; a power 
 constexpr int kHeldTokens = 4096;                 // tokens of a segment that are placed in LDS first
 constexpr int kLongRows = 256;
 constexpr int32_t kOrdered = 0x40000000;          // in an entry of the hot list: the row's bucket is in ascending order
+constexpr int32_t kLong = 0x20000000;             // of the slots of emb_bwd_buckets<.., true>: more than kRankTokens tokens
+constexpr int kOneTokens = 8192;                  // bucketed in one launch: up to so many tokens,
+constexpr int kOneRows = 1024;                    // 256 segments of up to so many rows
+constexpr int kHotSlots = 512;                    // slots of hot rows, at most
 constexpr int kRankTokens = 2 * kBlock;           // up to so many tokens of a row are ordered by counting the smaller ones
 constexpr int kBitWords = 4096;                   // more of them by a bit per token number
 constexpr int kBitsPerWindow = kBitWords * 32;
@@ -194,6 +201,12 @@ struct SplitArgs {
     int32_t* totals;                              // entries at the end of the hot list, entries at its front
     int32_t hot_most;                             // entries the hot list has room for
 };
+
+// Slots of hot rows that the segments up to one whose tokens end at `tokens` have: one for every kHotAbove + 1 tokens and one
+// more for each segment.
+constexpr int kHotAbove = 32;                        // rows of more tokens are hot: what half a wavefront's lanes order, and as long as
+                                                     // the ordinary walk stays below the time of everything else (with 64: 24 us, with 32: 17)
+__host__ __device__ inline int32_t hot_slots(int32_t tokens, int32_t segments) { return tokens / (kHotAbove + 1) + segments; }
 
 template <typename IdT>
 __global__ __launch_bounds__(kSplitBlock) void emb_bwd_split(const IdT* __restrict__ ids, const SplitArgs a) {
@@ -259,9 +272,15 @@ __device__ inline int32_t count_up(int32_t* counters, int32_t row) {
     return __builtin_amdgcn_readfirstlane(base) + before;
 }
 
-static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const SplitArgs a) {
-    __shared__ int32_t counters[kSegmentRows];
-    __shared__ int32_t upto[kChunks + 1], from[kChunks];   // tokens of this segment in the chunks below; where its own begin
+// ONE: without emb_bwd_split in front; each workgroup looks at all tokens and keeps its segment's in LDS.  Its hot rows go into slots
+// of its own, for there is no launch in front that could clear a counter.
+template <typename IdT, bool ONE>
+__global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const IdT* __restrict__ ids, const SplitArgs a) {
+    constexpr int kSegRows = ONE ? kOneRows : kSegmentRows;
+    __shared__ int32_t counters[kSegRows];
+    __shared__ int32_t upto[ONE ? 1 : kChunks + 1], from[ONE ? 1 : kChunks];   // tokens of this segment in the chunks below; where its own begin
+    __shared__ uint16_t my_token[ONE ? kOneTokens : 1], my_row[ONE ? kOneTokens : 1];
+    __shared__ int32_t my_tokens, my_hot;
     __shared__ int32_t wave_total[kBucketBlock / kWave], wave_base[kBucketBlock / kWave];
     __shared__ int32_t held[kHeldTokens];
     __shared__ uint16_t held_row[kHeldTokens];
@@ -271,34 +290,68 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
     if (t == 0) long_rows = 0;
     const int32_t rows = s < a.rows ? ((a.rows - 1 - s) >> a.shift) + 1 : 0;   // of this segment
     for (int i = t; i < rows; i += kBucketBlock) counters[i] = 0;
-    // A thread per chunk.  The tokens of lower segments in all chunks are the place of this segment's stretch.
-    static_assert(kChunks == kBucketBlock, "a thread per chunk");
-    int32_t len = 0, lower = 0;
-    if (t < a.chunks) {
-        const int32_t* const o = a.offsets + static_cast<int64_t>(t) * (a.segments + 1) + s;
-        lower = o[0];
-        len = o[1] - lower;
-        from[t] = lower;
-    }
-    int32_t incl = len, base = lower;
+    int32_t tokens = 0, run = 0;                  // of this segment; of the segments below: where this one's stretch begins
+    if constexpr (ONE) {
+        if (t == 0) my_tokens = my_hot = 0;
+        __syncthreads();
+        int32_t lower = 0;
+        constexpr int kEach = kOneTokens / kBucketBlock;
+        int32_t r[kEach];
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int32_t up = __shfl_up(incl, off, kWave);
-        if (lane >= off) incl += up;
-        base += __shfl_xor(base, off, kWave);
-    }
-    if (lane == kWave - 1) wave_total[wave] = incl, wave_base[wave] = base;
-    __syncthreads();
-    int32_t before = 0, tokens = 0, run = 0;
+        for (int k = 0; k < kEach; ++k) {
+            const int64_t i = t + k * kBucketBlock;
+            r[k] = i < a.n_ids ? static_cast<int32_t>(token_row(ids, i, a.lo, a.lo + a.rows, a.padding_idx)) : -1;
+        }
 #pragma unroll
-    for (int k = 0; k < kBucketBlock / kWave; ++k) {
-        before += k < wave ? wave_total[k] : 0;
-        tokens += wave_total[k];
-        run += wave_base[k];
+        for (int k = 0; k < kEach; ++k) {
+            const int32_t segment = r[k] & (a.segments - 1);
+            const bool mine = r[k] >= 0 && segment == s;
+            lower += r[k] >= 0 && segment < s ? 1 : 0;
+            const uint64_t all = __ballot(mine);
+            if (all == 0) continue;                    // the same in all lanes
+            const int32_t before = __popcll(all & ((1ull << lane) - 1));
+            int32_t first = 0;
+            if (lane == 0) first = atomicAdd(&my_tokens, __popcll(all));
+            const int32_t at = __builtin_amdgcn_readfirstlane(first) + before;
+            if (mine) my_token[at] = static_cast<uint16_t>(t + k * kBucketBlock), my_row[at] = static_cast<uint16_t>(r[k] >> a.shift);
+        }
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) lower += __shfl_xor(lower, off, kWave);
+        if (lane == kWave - 1) wave_base[wave] = lower;
+        __syncthreads();
+        tokens = my_tokens;
+#pragma unroll
+        for (int k = 0; k < kBucketBlock / kWave; ++k) run += wave_base[k];
+    } else {
+        // A thread per chunk.  The tokens of lower segments in all chunks are the place of this segment's stretch.
+        static_assert(kChunks == kBucketBlock, "a thread per chunk");
+        int32_t len = 0, lower = 0;
+        if (t < a.chunks) {
+            const int32_t* const o = a.offsets + static_cast<int64_t>(t) * (a.segments + 1) + s;
+            lower = o[0];
+            len = o[1] - lower;
+            from[t] = lower;
+        }
+        int32_t incl = len, base = lower;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int32_t up = __shfl_up(incl, off, kWave);
+            if (lane >= off) incl += up;
+            base += __shfl_xor(base, off, kWave);
+        }
+        if (lane == kWave - 1) wave_total[wave] = incl, wave_base[wave] = base;
+        __syncthreads();
+        int32_t before = 0;
+#pragma unroll
+        for (int k = 0; k < kBucketBlock / kWave; ++k) {
+            before += k < wave ? wave_total[k] : 0;
+            tokens += wave_total[k];
+            run += wave_base[k];
+        }
+        upto[t + 1] = before + incl;
+        if (t == 0) upto[0] = 0;
+        __syncthreads();
     }
-    upto[t + 1] = before + incl;
-    if (t == 0) upto[0] = 0;
-    __syncthreads();
     // Where this segment's token i < tokens is: in the chunk c with upto[c] <= i < upto[c + 1].
     auto place = [&](int32_t i) {
         int32_t c = 0;
@@ -307,16 +360,27 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
             if (upto[c + half] <= i) c += half;
         return c * a.chunk_tokens + from[c] + (i - upto[c]);
     };
+    auto look = [&](int32_t i, int32_t& row, int32_t& token) {
+        if constexpr (ONE) {
+            row = my_row[i], token = my_token[i];
+        } else {
+            const int64_t at = place(i);
+            row = a.row[at], token = a.token[at];
+        }
+    };
     // The first kBucketBlock tokens, mostly all, stay in registers.
     int32_t row_first = -1, token_first = 0;
     if (t < tokens) {
-        const int64_t at = place(t);
-        row_first = a.row[at], token_first = a.token[at];
+        look(t, row_first, token_first);
         count_up(counters, row_first);
     }
-    for (int32_t i = t + kBucketBlock; i < tokens; i += kBucketBlock) count_up(counters, a.row[place(i)]);
+    for (int32_t i = t + kBucketBlock; i < tokens; i += kBucketBlock) {
+        int32_t row, token;
+        look(i, row, token);
+        count_up(counters, row);
+    }
     __syncthreads();
-    constexpr int kRows = kSegmentRows / kBucketBlock;
+    constexpr int kRows = kSegRows / kBucketBlock;
     const int per = (rows + kBucketBlock - 1) / kBucketBlock;   // consecutive rows of a thread
     int32_t n[kRows], begins[kRows], long_at[kRows], total = 0;
     const int32_t run_first = run;                              // where this segment's stretch begins
@@ -326,7 +390,7 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
         n[k] = k < per && t * per + k < rows ? counters[t * per + k] : 0;
         total += n[k];
     }
-    incl = total;
+    int32_t incl = total;
 #pragma unroll
     for (int off = 1; off < kWave; off <<= 1) {
         const int32_t up = __shfl_up(incl, off, kWave);
@@ -347,7 +411,11 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
         run += n[k];
         meta[r].count = n[k], meta[r].end = run;
         // Long rows from the front of the list, so that their workgroups start first; the others from its end.
-        if (n[k] > kRankTokens) {
+        if constexpr (ONE) {
+            if (n[k] > kRankTokens) long_at[k] = atomicAdd(&long_rows, 1);
+            if (n[k] > a.hot_above)
+                a.hot[hot_slots(run_first, s) + atomicAdd(&my_hot, 1)] = ((r << a.shift) + s) | (n[k] > kRankTokens ? kOrdered | kLong : tokens <= kHeldTokens ? kOrdered : 0);
+        } else if (n[k] > kRankTokens) {
             if (a.n_ids <= kBitsPerWindow) long_at[k] = atomicAdd(&long_rows, 1);
             a.hot[atomicAdd(&a.totals[1], 1)] = ((r << a.shift) + s) | (a.n_ids <= kBitsPerWindow ? kOrdered : 0);
         } else if (n[k] > a.hot_above) {
@@ -355,6 +423,10 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
         }
     }
     __syncthreads();
+    if constexpr (ONE) {   // the slots that are left
+        const int32_t end = hot_slots(s + 1 < a.segments ? run_first + tokens : static_cast<int32_t>(a.n_ids), s + 1);
+        for (int32_t i = hot_slots(run_first, s) + my_hot + t; i < end; i += kBucketBlock) a.hot[i] = -1;
+    }
     // The buckets, in ascending order where that is cheap: the workgroups that share a hot row's columns need not each do it.
     const int32_t stretch = run_first;
     if (tokens <= kHeldTokens) {
@@ -364,8 +436,9 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
         };
         if (row_first >= 0) hold(row_first, token_first);
         for (int32_t i = t + kBucketBlock; i < tokens; i += kBucketBlock) {
-            const int64_t at = place(i);
-            hold(a.row[at], a.token[at]);
+            int32_t row, token;
+            look(i, row, token);
+            hold(row, token);
         }
         __syncthreads();
         for (int32_t i = t; i < tokens; i += kBucketBlock) {   // a counter holds the end of its row now, which is where the next begins
@@ -382,8 +455,9 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
     } else {
         if (row_first >= 0) a.bucket[count_up(counters, row_first)] = token_first;
         for (int32_t i = t + kBucketBlock; i < tokens; i += kBucketBlock) {
-            const int64_t at = place(i);
-            a.bucket[count_up(counters, a.row[at])] = a.token[at];
+            int32_t row, token;
+            look(i, row, token);
+            a.bucket[count_up(counters, row)] = token;
         }
     }
     __syncthreads();
@@ -397,8 +471,8 @@ static __global__ __launch_bounds__(kBucketBlock) void emb_bwd_buckets(const Spl
         }
     for (int32_t h = 0; h < all_long; ++h) {
         uint32_t* const bits = reinterpret_cast<uint32_t*>(counters);
-        static_assert(kBitWords == kSegmentRows, "a bit per token number where the counters were");
-        constexpr int kWords = kBitWords / kBucketBlock;
+        static_assert((ONE ? kOneTokens : kBitsPerWindow) <= 32 * kSegRows, "a bit per token number where the counters were");
+        constexpr int kWords = kSegRows / kBucketBlock;
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < kWords; ++k) bits[t + k * kBucketBlock] = 0;
@@ -507,6 +581,7 @@ struct ReduceArgs {
     int32_t hot_above;      // rows of more tokens are hot
     int32_t hot_chunks;     // pieces of kHotBytes of a row
     int32_t scale_by_freq;
+    int32_t slots;          // not 0: hot rows are in this many slots, some of them empty, and `totals` holds nothing
     __device__ Row of(int64_t row) const { return meta[(row & ((1 << shift) - 1)) * segment_rows + (row >> shift)]; }
 };
 
@@ -523,8 +598,6 @@ struct ReduceArgs {
 // read back in ascending order, kListTokens at a time.  The bits have LDS of their
 // own: in the stage's they had to be set again, by a walk over the whole bucket,
 // for every kListTokens (2^20 tokens of one row, 256 bytes each: 1267 ms, now 59).
-constexpr int kHotAbove = 32;                        // rows of more tokens are hot: what half a wavefront's lanes order, and as long as
-                                                     // the ordinary walk stays below the time of everything else (with 64: 24 us, with 32: 17)
 constexpr int kHotBytes = 64;
 constexpr int kHotBatch = 256;                       // tokens per batch
 constexpr int kHotPitch = kHotBatch + 4;             // 16 floats apart for the four lanes that store a token: no two on one bank
@@ -534,7 +607,8 @@ constexpr int kWordsPerThread = kBitWords / kBlock;
 struct HotShared {
     alignas(16) float column[kHotBytes / 2][kHotPitch];   // a batch in fp32, column by column: the adding wavefront reads four tokens at once
     alignas(16) uint32_t bits[kBitWords];            // a bit per token number, or the bucket being ordered
-    int32_t list[kListTokens];                       // tokens in ascending order
+    int32_t list[kListTokens + kHotSlots];           // tokens in ascending order; behind them the hot rows found in the slots
+    int32_t slots[4][kWavesPerBlock];
     int32_t wave_total[kWavesPerBlock];
 };
 
@@ -695,12 +769,35 @@ __device__ inline void hot_row(HotShared& sh, const ReduceArgs& a, int64_t row, 
 template <typename E>
 __global__ __launch_bounds__(kBlock) void emb_bwd_hot(const ReduceArgs a) {
     __shared__ HotShared sh;
-    const int32_t listed = a.totals[1];
-    const int32_t more = a.hot_most ? a.totals[0] : a.of(a.rows - 1).count > a.hot_above ? 1 : 0;
+    int32_t* const found = sh.list + kListTokens;         // of the slots: long rows first
+    int32_t listed, more = 0;
+    if (a.slots) {
+        static_assert(kHotSlots == 2 * kBlock, "two slots a thread");
+        const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+        const int32_t e0 = t < a.slots ? a.hot[t] : -1, e1 = t + kBlock < a.slots ? a.hot[t + kBlock] : -1;
+        uint64_t in[4] = {__ballot(e0 >= 0 && (e0 & kLong)), __ballot(e1 >= 0 && (e1 & kLong)), __ballot(e0 >= 0 && !(e0 & kLong)), __ballot(e1 >= 0 && !(e1 & kLong))};
+        if (lane < 4) sh.slots[lane][wave] = __popcll(lane == 0 ? in[0] : lane == 1 ? in[1] : lane == 2 ? in[2] : in[3]);
+        __syncthreads();
+        listed = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            int32_t at = listed;
+#pragma unroll
+            for (int k = 0; k < kWavesPerBlock; ++k) {
+                at += k < wave ? sh.slots[q][k] : 0;
+                listed += sh.slots[q][k];
+            }
+            if ((in[q] >> lane) & 1) found[at + __popcll(in[q] & ((1ull << lane) - 1))] = (q & 1 ? e1 : e0) & ~kLong;
+        }
+        __syncthreads();
+    } else {
+        listed = a.totals[1];
+        more = a.hot_most ? a.totals[0] : a.of(a.rows - 1).count > a.hot_above ? 1 : 0;
+    }
     const int32_t items = (listed + more) * a.hot_chunks;
     for (int32_t item = static_cast<int32_t>(blockIdx.x); item < items; item += static_cast<int32_t>(gridDim.x)) {
         const int32_t which = item / a.hot_chunks;
-        const int32_t entry = which < listed ? a.hot[which] : a.hot_most ? a.hot[a.hot_most - 1 - (which - listed)] : static_cast<int32_t>(a.rows) - 1;
+        const int32_t entry = which < listed ? (a.slots ? found[which] : a.hot[which]) : a.hot_most ? a.hot[a.hot_most - 1 - (which - listed)] : static_cast<int32_t>(a.rows) - 1;
         const bool ordered = a.hot_most && (entry & kOrdered);
         hot_row<E>(sh, a, ordered ? entry & ~kOrdered : entry, ordered, item - which * a.hot_chunks);
     }
@@ -843,7 +940,7 @@ Split plan_split(int64_t n_ids, int64_t rows) {
     if (p.chunk_tokens < 1024) p.chunk_tokens = 1024;
     p.chunks = static_cast<int>((n_ids + p.chunk_tokens - 1) / p.chunk_tokens);
     const int64_t segments = 1ll << p.shift;
-    p.elems = 2 * segments * p.segment_rows + 2 + 3 * n_ids + p.chunks * (segments + 1) + n_ids / (kHotAbove + 1) + 1;
+    p.elems = 2 * segments * p.segment_rows + 2 + 3 * n_ids + p.chunks * (segments + 1) + hot_slots(static_cast<int32_t>(n_ids), static_cast<int32_t>(segments));
     return p;
 }
 
@@ -875,8 +972,13 @@ int run(const void* dy, int dtype, int64_t dim, int64_t ld_dy, const IdT* ids, i
         b.hot = b.offsets + static_cast<int64_t>(b.chunks) * (b.segments + 1);
         a.meta = b.meta, a.bucket = b.bucket, a.hot = b.hot, a.totals = b.totals;
         a.shift = b.shift, a.segment_rows = b.segment_rows, a.hot_most = b.hot_most;
-        hipLaunchKernelGGL((emb_bwd_split<IdT>), dim3(static_cast<uint32_t>(b.chunks)), dim3(kSplitBlock), 0, s, ids, b);
-        hipLaunchKernelGGL(emb_bwd_buckets, dim3(static_cast<uint32_t>(b.segments)), dim3(kBucketBlock), 0, s, b);
+        if (n_ids <= kOneTokens && b.segments == 256 && b.segment_rows <= kOneRows) {
+            a.slots = hot_slots(static_cast<int32_t>(n_ids), b.segments);
+            hipLaunchKernelGGL((emb_bwd_buckets<IdT, true>), dim3(static_cast<uint32_t>(b.segments)), dim3(kBucketBlock), 0, s, ids, b);
+        } else {
+            hipLaunchKernelGGL((emb_bwd_split<IdT>), dim3(static_cast<uint32_t>(b.chunks)), dim3(kSplitBlock), 0, s, ids, b);
+            hipLaunchKernelGGL((emb_bwd_buckets<IdT, false>), dim3(static_cast<uint32_t>(b.segments)), dim3(kBucketBlock), 0, s, ids, b);
+        }
     } else {
         // 3 rows + 1 + n_ids integers: the hot list has at most rows - 1 entries
         Row* const meta = reinterpret_cast<Row*>(ws);           // [rows]

@@ -1346,6 +1346,52 @@ def test_embedding_backward_bucketing_by_segments(ops, rows, tokens, hot):
     assert bool(((got.double() - want).abs() <= 2.0 ** -24 * count * size).all())    # one rounding per addition
 
 
+@pytest.mark.parametrize("rows,tokens,kind", [
+    (50304, 8192, "text"), (50304, 8193, "text"),          # the most tokens that one launch buckets, and one more
+    (262144, 8192, "spread"), (262145, 8192, "spread"),    # the most rows of its segments, and one more
+    (3, 8192, "text"), (1, 8192, "text"),                  # rows of thousands of tokens: more than a segment holds in LDS
+    (700, 8192, "misses"), (256 * 20, 8184, "all hot"),    # most tokens outside of the table; every segment with a hot row
+    (1000, 513, "one"), (1000, 512, "one"), (1000, 33, "one"), (1000, 32, "one"), (255, 1, "spread"), (1000, 40, "none")])
+@pytest.mark.parametrize("idt", [torch.int64, torch.int32])
+def test_embedding_backward_in_one_bucketing_launch(ops, rows, tokens, kind, idt):
+    """Tokens bucketed in one launch (or in two) give what the general launches give, bit for bit."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(rows + tokens)
+    lo, dim = 17, 24
+    if kind == "text":
+        ids = (torch.exp(torch.rand(tokens, generator=gen, dtype=torch.float64) * np.log(rows + 1)).long() - 1).clamp_(0, rows - 1) + lo
+    elif kind == "misses":
+        ids = torch.randint(0, 20 * rows, (tokens,), generator=gen)
+    elif kind == "all hot":   # 248 rows of 33 tokens each, in different segments
+        ids = torch.arange(tokens)[torch.randperm(tokens, generator=gen)] % 248 + 256 * (torch.arange(1) + 19) + lo
+    elif kind == "one":
+        ids = torch.full((tokens,), lo + rows - 1)
+    elif kind == "none":
+        ids = torch.full((tokens,), lo + rows)
+    else:
+        ids = torch.randint(0, rows, (tokens,), generator=gen) + lo
+        ids[0] = lo + rows - 1
+    ids = ids.to(idt).cuda()
+    dy = torch.randn(tokens, dim, generator=gen).cuda()
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    got = []
+    for words in (3 * rows + 1 + tokens, max(3 * rows + 1 + tokens, lib.ddl_embedding_backward_workspace(tokens, rows))):
+        work = torch.randint(-2 ** 31, 2 ** 31, (words,), generator=gen).to(torch.int32).cuda()   # whatever it held before
+        dw = torch.full((rows, dim), float("nan"), device="cuda")
+        _lib.check(lib.ddl_embedding_backward(dy.data_ptr(), _lib.DDL_DT_F32, dim, dim, ids.data_ptr(), int(idt == torch.int64), tokens, lo, lo + rows, lo + 5,
+                                              0, dw.data_ptr(), dim, work.data_ptr(), work.numel(), stream), "ddl_embedding_backward")
+        got.append(dw)
+    assert torch.equal(got[0], got[1])
+    assert torch.equal(ops.embedding_backward(dy, ids, lo, lo + rows, padding_idx=lo + 5), got[0])
+    want = torch.zeros(rows + 1, dim, dtype=torch.float64)
+    at = ids.cpu().long() - lo
+    at[(at < 0) | (at >= rows) | (at == 5)] = rows
+    want.index_add_(0, at, dy.cpu().double())
+    # fp32 sums of up to `tokens` standard normal terms, one after the other
+    most = int(torch.bincount(at, minlength=rows + 1)[:rows].max())
+    assert bool(((got[0].cpu().double() - want[:rows]).abs() <= 2.0 ** -24 * most * 4 * max(most, 1) ** 0.5 + 1e-12).all())
+
+
 def test_embedding_backward_of_one_row_takes_time_in_proportion_to_its_tokens(ops):
     """Every token the same id: exact sums (small integers), and four times the tokens take about four times as long (4.5
     measured; ordering the bucket anew for every 1024 of its tokens made it 22)."""
