@@ -395,6 +395,10 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     // see its writes above; no other wavefront touches this region.
     asm volatile("" ::: "memory");
     static_assert((TM * 16 * kChunks) % 64 == 0, "block does not split into whole wavefront passes");
+    // y is not read again here: streaming stores, where rows start on lines.  Others share a line between two wavefronts' 128 bytes,
+    // which the L2 puts together of ordinary stores only: M 8192, N 8188, K 64 102 -> 48 us (N 8192 45), N 8191, K 256 89 -> 66,
+    // N 4092, K 512 61 -> 46; M 4100, N 8191, K 128 46 -> 35.
+    const bool lines = ((reinterpret_cast<uintptr_t>(y) | static_cast<uintptr_t>(2 * ldy)) & 127) == 0;
 #pragma unroll 4
     for (int p = 0; p < TM * 16 * kChunks / 64; ++p) {
         const int idx = p * 64 + lane;
@@ -405,12 +409,13 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
         if (m >= M || n >= N) continue;
         uint16_t* dst = y + m * ldy + n;
         if (n + 8 <= N) {
-            // y is not read again here: a streaming store, at the alignment of an element (global memory takes any)
+            // at the alignment of an element (global memory takes any)
             typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
             typedef u32x4 any __attribute__((aligned(2)));
             u32x4 nv;
             nv[0] = v.x, nv[1] = v.y, nv[2] = v.z, nv[3] = v.w;
-            __builtin_nontemporal_store(nv, reinterpret_cast<any*>(dst));
+            if (lines) __builtin_nontemporal_store(nv, reinterpret_cast<any*>(dst));
+            else *reinterpret_cast<any*>(dst) = nv;
         } else {
             const uint32_t words[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
