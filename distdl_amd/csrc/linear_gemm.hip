@@ -399,6 +399,7 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     // which the L2 puts together of ordinary stores only: M 8192, N 8188, K 64 102 -> 48 us (N 8192 45), N 8191, K 256 89 -> 66,
     // N 4092, K 512 61 -> 46; M 4100, N 8191, K 128 46 -> 35.
     const bool lines = ((reinterpret_cast<uintptr_t>(y) | static_cast<uintptr_t>(2 * ldy)) & 127) == 0;
+    auto leave = [&](auto streaming) {   // a loop each: of two stores on one path the compiler makes one, an ordinary one
 #pragma unroll 4
     for (int p = 0; p < TM * 16 * kChunks / 64; ++p) {
         const int idx = p * 64 + lane;
@@ -414,7 +415,7 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
             typedef u32x4 any __attribute__((aligned(2)));
             u32x4 nv;
             nv[0] = v.x, nv[1] = v.y, nv[2] = v.z, nv[3] = v.w;
-            if (lines) __builtin_nontemporal_store(nv, reinterpret_cast<any*>(dst));
+            if constexpr (decltype(streaming)::value) __builtin_nontemporal_store(nv, reinterpret_cast<any*>(dst));
             else *reinterpret_cast<any*>(dst) = nv;
         } else {
             const uint32_t words[4] = {v.x, v.y, v.z, v.w};
@@ -423,6 +424,9 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
                 if (n + e < N) dst[e] = static_cast<uint16_t>(words[e >> 1] >> (16 * (e & 1)));
         }
     }
+    };
+    if (lines) leave(std::true_type{});
+    else leave(std::false_type{});
 }
 
 constexpr int kThreads = 512;
