@@ -148,6 +148,13 @@ class _LayerNormShard(torch.autograd.Function):
         return grads + (None, None, None, None, None)
 
 
+def _takes_addresses(input, weight, bias):
+    """May the kernels be handed these operands by their addresses?  The general way converts, or says what is wrong: parameters
+    that are not on the GPU, or a bias of another type than the input (the weight's has been looked at)."""
+    return input.is_cuda and input.is_contiguous() and \
+        (weight is None or (weight.is_cuda and bias.is_cuda and bias.dtype == input.dtype and weight.is_contiguous() and bias.is_contiguous()))
+
+
 class DistributedLayerNorm(Module):
     r"""Layer normalisation over the last ``len(normalized_shape)`` dimensions of
     a tensor partitioned by ``P_x``; those dimensions may themselves be
@@ -319,8 +326,7 @@ class DistributedLayerNorm(Module):
                                                  made(functools.partial(_shard_backward, P_reduce, nparts)))
         if nparts == 1:
             return _lib.front().layer_norm_shard(input, weight, bias, self.part_cols[0], self.eps, calls[1])
-        if not P_reduce.active or not input.is_cuda or not input.is_contiguous() or \
-           not (weight is None or (weight.is_contiguous() and bias.is_contiguous())):
+        if not P_reduce.active or not _takes_addresses(input, weight, bias):
             return None
         if input.numel() == 0 or not _lib.front().unobserved(input, weight, bias):
             return None
@@ -355,7 +361,7 @@ class DistributedLayerNorm(Module):
         wants_grad = torch.is_grad_enabled() and (input.requires_grad or (weight is not None and weight.requires_grad) or
                                                   (bias is not None and bias.requires_grad))
         if not wants_grad:      # nothing to record: skip the autograd machinery and the statistics kept for backward
-            if input.is_cuda and input.is_contiguous() and (weight is None or (weight.is_contiguous() and bias.is_contiguous())):
+            if _takes_addresses(input, weight, bias):
                 return self._forward_contiguous(input, weight, bias)
             return _shard_forward(input, weight, bias, self.allreduce.P_allreduce, self.part_cols, self.eps,
                                   self._part_cols_arr, self._stats_buffers, False)[0]

@@ -1032,3 +1032,49 @@ def test_column_sums_of_more_columns_than_one_launch_has_threads_for_take_two():
             assert lib.ddl_linear_backward_workspace(dt, 8, cols, 1, 1, 1, cols, 0, 0, 1) == floats
         assert lib.ddl_linear_backward_workspace(dt, rows, 64, 1, 1, 1, 64, 0, 0, 1) == 0
         assert lib.ddl_linear_backward_workspace(dt, rows + 1, 64, 1, 1, 1, 64, 0, 0, 1) == -(-(rows + 1) // 128) * 64
+
+
+class _OnGpu(torch.Tensor):
+    """A tensor of the CPU that says it is on the GPU, for checks in front of a launch."""
+    is_cuda = True
+
+
+@pytest.mark.parametrize("workers", [1, 4])
+@pytest.mark.parametrize("trains", [True, False])
+@pytest.mark.parametrize("wrong", [None, "weight", "bias", "bias type"])
+def test_layer_norm_hands_the_kernels_parameters_of_the_inputs_kind_only(monkeypatch, workers, trains, wrong):
+    """Parameters left on the CPU and a bias of another type than the input's raise, before an entry point gets their addresses."""
+    from distdl_amd import hip_ops
+    from distdl_amd.nn import DistributedLayerNorm
+    called = []
+
+    class Entries:
+
+        def __init__(self, **answers):
+            self.answers = answers
+
+        def __getattr__(self, name):
+            def entry(*args):
+                called.append(name)
+                return self.answers.get(name, 0)
+            return entry
+    P = SimWorld(workers, device="cpu").partition(0).create_partition_inclusive(list(range(workers))).create_cartesian_topology_partition([1, 1, workers])
+    layer = DistributedLayerNorm(P, [8 * workers], device="cpu")
+    for name in "weight", "bias":
+        kept = torch.ones_like(getattr(layer, name)).detach()
+        if wrong == "bias type" and name == "bias":
+            kept = kept.to(torch.bfloat16)
+        setattr(layer, name, torch.nn.Parameter(kept if wrong == name else kept.as_subclass(_OnGpu)))
+    x = torch.randn(2, 3, 8).as_subclass(_OnGpu)
+    monkeypatch.setattr(_lib, "_lib", Entries())
+    monkeypatch.setattr(_lib, "_front", Entries(unobserved=True, layer_norm=None, layer_norm_shard=None))
+    monkeypatch.setattr(_lib, "extension", Entries)
+    monkeypatch.setattr(hip_ops, "_stream", lambda: None)
+    with torch.set_grad_enabled(trains):
+        if wrong is None:
+            layer(x)
+        else:
+            with pytest.raises((ValueError, RuntimeError), match="on cpu|gamma / beta"):
+                layer(x)
+    taking = {"ddl_layer_norm", "ddl_ln_stats_normalize", "ddl_ln_normalize_affine"} & set(called)
+    assert bool(taking) == (wrong is None)
