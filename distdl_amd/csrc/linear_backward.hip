@@ -327,10 +327,11 @@ extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int6
     int64_t most = 0;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     auto take = [&](int64_t elems) { most = elems > most ? elems : most; };
-    if (want_dx && want_dw) {   // both in one launch, with a part of the workspace each
-        const bool inside = want_db && M <= (dtype == DDL_DT_F32 ? ddl::kAdjointRows32 : ddl::kAdjointRows);
+    const bool wide = dtype == DDL_DT_F32, narrow = dtype == DDL_DT_BF16 || dtype == DDL_DT_F16;
+    if (want_dx && want_dw && (wide || narrow)) {   // both in one launch, with a part of the workspace each
+        const bool inside = want_db && M <= (wide ? ddl::kAdjointRows32 : ddl::kAdjointRows);
         bool taken;
-        if (dtype == DDL_DT_F32) {
+        if (wide) {
             const ddl::AdjointPlan32 plan = ddl::adjoint32(M, N, K, ldx, ldw, lddy, inside, INT64_MAX);
             taken = plan.groups_x != 0;
             take(plan.workspace);
@@ -365,8 +366,8 @@ extern "C" int ddl_linear_backward(const void* x, const void* w, const void* dy,
     using namespace ddl;
     if (M < 1 || N < 1 || K < 1) return fail(DDL_E_ARG, "linear backward: M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
     if (!dy || (dx && !w) || (dw && !x)) return fail(DDL_E_ARG, "linear backward: null pointer");
-    if (dtype != DDL_DT_F32 && dx && dw && aligned_to(x, 2) && aligned_to(w, 2) && aligned_to(dy, 2) && aligned_to(dx, 2) && aligned_to(dw, 2) && aligned_to(db, 2) &&
-        (!workspace || aligned_to(workspace, 16))) {
+    if ((dtype == DDL_DT_BF16 || dtype == DDL_DT_F16) && dx && dw && aligned_to(x, 2) && aligned_to(w, 2) && aligned_to(dy, 2) && aligned_to(dx, 2) &&
+        aligned_to(dw, 2) && aligned_to(db, 2) && (!workspace || aligned_to(workspace, 16))) {
         const bool aligned = aligned_to(x, 16) && aligned_to(w, 16) && aligned_to(dy, 16);
         const int64_t room = workspace ? workspace_elems : 0;
         const bool inside = db && M <= kAdjointRows;

@@ -1078,3 +1078,16 @@ def test_layer_norm_hands_the_kernels_parameters_of_the_inputs_kind_only(monkeyp
                 layer(x)
     taking = {"ddl_layer_norm", "ddl_ln_stats_normalize", "ddl_ln_normalize_affine"} & set(called)
     assert bool(taking) == (wrong is None)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 64, 64), (777, 333, 1024), (4096, 2048, 2048)])
+def test_adjoint_of_a_linear_shard_refuses_element_types_it_has_no_kernel_for(M, N, K):
+    """No launch (there is no GPU here, it would fail with the runtime's error) and no room for one, in any combination of outputs."""
+    lib = _lib.load()
+    there = ctypes.addressof(ctypes.create_string_buffer(64)) // 16 * 16 + 16
+    for dtype in (_lib.DDL_DT_BITS, _lib.DDL_DT_F64, _lib.DDL_DT_I32, _lib.DDL_DT_I64, 77, -1):
+        for wanted in ((1, 1, 1), (1, 1, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1)):
+            outs = [there if on else None for on in wanted]
+            assert lib.ddl_linear_backward(there, there, there, *outs, dtype, M, N, K, K, K, N, there, 1 << 30, None) == -5, (dtype, wanted)
+            if not wanted[2]:
+                assert lib.ddl_linear_backward_workspace(dtype, M, N, K, K, K, N, *wanted) == 0
