@@ -9,7 +9,8 @@
 //
 // Every function answers None where torch wants to see what happens or where the
 // node would drop something: under a tracer, a dispatch mode or a functorch transform, for
-// tensors with tangents, for subclasses that dispatch to Python.  The callers then
+// tensors with tangents, for subclasses of torch.Tensor (but for parameters), which
+// may want their own type back.  The callers then
 // apply their torch.autograd.Function.  Tensors are saved as SavedVariables: hooks on
 // saved tensors, checks of versions and of a second pass work as for any node.
 #include "front.h"
@@ -18,6 +19,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -41,7 +43,8 @@ bool unobserved() {
 bool ordinary(const Tensor& t) {
     constexpr c10::DispatchKeySet kSeen({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched,
                                          c10::DispatchKey::Functionalize});
-    return !t.key_set().has_any(kSeen) && !t._fw_grad(0).defined();
+    const PyObject* const object = t.unsafeGetTensorImpl()->pyobj_slot()->load_pyobj();   // the caller's reference keeps it
+    return !t.key_set().has_any(kSeen) && !t._fw_grad(0).defined() && (!object || THPVariable_CheckExact(const_cast<PyObject*>(object)));
 }
 bool ordinary(const MaybeTensor& t) { return !t || ordinary(*t); }
 

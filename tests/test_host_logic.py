@@ -1091,3 +1091,32 @@ def test_adjoint_of_a_linear_shard_refuses_element_types_it_has_no_kernel_for(M,
             assert lib.ddl_linear_backward(there, there, there, *outs, dtype, M, N, K, K, K, N, there, 1 << 30, None) == -5, (dtype, wanted)
             if not wanted[2]:
                 assert lib.ddl_linear_backward_workspace(dtype, M, N, K, K, K, N, *wanted) == 0
+
+
+def _grid_layers():
+    """A broadcast onto and a sum from a grid of four workers, as the live rank has them: what it holds stays where it is."""
+    from distdl_amd.nn import Broadcast
+    from distdl_amd.nn import SumReduce
+    team = SimWorld(4, device="cpu").partition(0)
+    one = team.create_partition_inclusive([0]).create_cartesian_topology_partition([1, 1])
+    grid = team.create_partition_inclusive([0, 1, 2, 3]).create_cartesian_topology_partition([1, 4])
+    return [Broadcast(one, grid), SumReduce(grid, one)]
+
+
+class _Tagged(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_tensors_that_stay_keep_their_type(which):
+    """A subclass of torch.Tensor comes back, with gradients and without; a parameter comes back as a tensor."""
+    layer = _grid_layers()[which]
+    plain = torch.randn(3, 4)
+    for x in (plain.as_subclass(_Tagged), plain.clone().as_subclass(_Tagged).requires_grad_(True)):
+        for grad in (True, False):
+            with torch.set_grad_enabled(grad):
+                y = layer(x)
+            assert type(y) is _Tagged and y.requires_grad == (grad and x.requires_grad) and y.data_ptr() == x.data_ptr()
+    layer(x).sum().backward()
+    assert torch.equal(x.grad, torch.ones(3, 4))
+    assert type(layer(torch.nn.Parameter(plain))) is type(layer(plain)) is torch.Tensor
