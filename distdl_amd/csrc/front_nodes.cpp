@@ -22,6 +22,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/dynamo/compiled_autograd.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 
@@ -84,27 +85,115 @@ typedef std::shared_ptr<Callback> Shared;
 
 typedef std::tuple<MaybeTensor, MaybeTensor, MaybeTensor> Three;
 
-// (The lock is not held while Python is called.)
-struct ShardNode : Node {
+// The gradients that a pass asks for, and those that a node was made for: bit i for input i.
+struct Asked {
+    uint32_t now = 0, ever = 0;
+};
+inline bool has(uint32_t bits, int i) { return (bits >> i) & 1; }
+
+// What tells two adjoints apart, for a compiled pass that is used again.
+class Key {
+public:
+    Key& operator()(int64_t v) {
+        bytes_.append(reinterpret_cast<const char*>(&v), sizeof(v));
+        return *this;
+    }
+    Key& operator()(at::IntArrayRef v) {
+        (*this)(static_cast<int64_t>(v.size()));
+        for (const int64_t n : v) (*this)(n);
+        return *this;
+    }
+    Key& operator()(const MaybeShape& v) { return v ? (*this)(at::IntArrayRef(*v)) : (*this)(int64_t{-1}); }
+    template <typename T>
+    Key& operator()(const std::shared_ptr<T>& v) {   // a compiled pass holds it, so no other object has its address
+        return (*this)(static_cast<int64_t>(reinterpret_cast<intptr_t>(v.get())));
+    }
+    const std::string& bytes() const { return bytes_; }
+
+private:
+    std::string bytes_;
+};
+
+// The node of an adjoint A: `A::run(saved tensors, gradient, asked)` computes the gradients, `A::identify(key)` adds all that A
+// holds.  Unpacking runs hooks on saved tensors under the lock, as torch's nodes do; the adjoint runs without it.
+//
+// A compiled pass (torch's compiled autograd) keeps the adjoint as one opaque call: it copies A, and hands in the saved
+// tensors and the gradient of the pass it runs in.
+template <typename A>
+struct ShardNode final : Node {
+    A adjoint;
     std::vector<SavedVariable> saved;
-    void save(const Tensor& t) { saved.emplace_back(t, false); }
-    void save(const MaybeTensor& t) { saved.emplace_back(t ? *t : Tensor(), false); }
+    uint32_t present = 0;   // saved tensors that are there
+    void save(const Tensor& t) {
+        present |= (t.defined() ? 1u : 0u) << saved.size();
+        saved.emplace_back(t, false);
+    }
+    std::string name() const override { return A::kName; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
         for (SavedVariable& s : saved) s.reset_data();
     }
+    variable_list apply(variable_list&& grads) override {
+        return adjoint.run(unpacked(), grads[0].defined() ? grads[0] : input_metadata(0).zeros_like(), asked());
+    }
+    void compiled_args(torch::dynamo::autograd::CompiledNodeArgs& args) const override {
+        const auto& meta = input_metadata(0);
+        Key key;
+        key(int64_t{present})(int64_t{asked().now})(int64_t{asked().ever});
+        key(static_cast<int64_t>(c10::typeMetaToScalarType(meta.dtype())))(int64_t{meta.device().index()});
+        for (const c10::SymInt& n : meta.shape_as_dim_vector()) key(n.expect_int());
+        adjoint.identify(key);
+        args.collect(key.bytes());
+        for (const SavedVariable& s : saved) args.collect(s, false);
+    }
+    variable_list apply_with_saved(const variable_list& grads, torch::dynamo::autograd::SwapSavedVariables& swap) override {
+        namespace compiled = torch::dynamo::autograd;
+        for (SavedVariable& s : saved) swap.before(s);
+        std::vector<Tensor> there;
+        for (const Tensor& t : unpacked())
+            if (t.defined()) there.push_back(t);
+        compiled::PackedArgs packed;
+        packed.pack(there);
+        compiled::functional_apply_t call = [adjoint = adjoint, present = present, count = saved.size(), asked = asked(), meta = input_metadata(0)](
+                                                const variable_list& given, const compiled::ivalue_list& packed_args) {
+            compiled::PackedArgs args(packed_args);
+            const auto tensors = args.template unpack<std::vector<Tensor>>();
+            std::vector<Tensor> kept(count);
+            for (size_t i = 0, k = 0; i < count; ++i)
+                if (has(present, static_cast<int>(i))) kept[i] = tensors.at(k++);
+            return adjoint.run(kept, given[0].defined() ? given[0] : meta.zeros_like(), asked);
+        };
+        const auto& compiler = compiled::getPyCompilerInterface();
+        const std::string bound = compiler->bind_function(swap.get_py_compiler(), name(), std::move(call), {compiled::IValuePacker<std::vector<Tensor>>::packed_type()},
+                                                          /*is_custom_function=*/true, /*is_traceable=*/false);
+        auto results = compiler->call_function(swap.get_py_compiler(), "apply_functional", bound, grads, packed.vec(),
+                                               compiled::IValuePacker<std::vector<std::optional<torch::autograd::InputMetadata>>>::pack(compiled::get_input_metadata(next_edges())));
+        for (SavedVariable& s : saved) swap.after(s);
+        return results;
+    }
+
+private:
     std::vector<Tensor> unpacked() {
         std::lock_guard<std::mutex> lock(mutex_);
         std::vector<Tensor> tensors;
         for (SavedVariable& s : saved) tensors.push_back(s.unpack());
         return tensors;
     }
-    Tensor gradient(variable_list& grads) { return grads[0].defined() ? grads[0] : input_metadata(0).zeros_like(); }
+    Asked asked() const {
+        Asked a;
+        for (int i = 0; i < static_cast<int>(num_outputs()); ++i) {
+            a.now |= (task_should_compute_output(i) ? 1u : 0u) << i;
+            a.ever |= (should_compute_output(i) ? 1u : 0u) << i;
+        }
+        return a;
+    }
 };
 
-template <typename N>
-std::shared_ptr<N> make_node(std::initializer_list<MaybeTensor> inputs) {
-    std::shared_ptr<N> node(new N, torch::autograd::deleteNode);
+// y's node, for the inputs given.
+template <typename A>
+std::shared_ptr<ShardNode<A>> make_node(A adjoint, std::initializer_list<MaybeTensor> inputs) {
+    std::shared_ptr<ShardNode<A>> node(new ShardNode<A>, torch::autograd::deleteNode);
+    node->adjoint = std::move(adjoint);
     torch::autograd::edge_list edges;
     for (const MaybeTensor& t : inputs) edges.push_back(t ? torch::autograd::impl::gradient_edge(*t) : torch::autograd::Edge());
     node->set_next_edges(std::move(edges));
@@ -119,14 +208,14 @@ variable_list listed(const Three& t) {
 
 // ---------------------------------------------------------------- linear --
 
-struct LinearShardBackward : ShardNode {
+struct LinearShard {
+    static constexpr const char* kName = "LinearShardBackward";
     std::vector<int64_t> bias_shape;
     Shared general;
-    std::string name() const override { return "LinearShardBackward"; }
-    variable_list apply(variable_list&& grads) override {
-        const std::vector<Tensor> kept = unpacked();
-        const Tensor &x = kept[0], &w = kept[1], dy = gradient(grads);
-        const bool need_x = task_should_compute_output(0), need_w = task_should_compute_output(1), need_b = task_should_compute_output(2);
+    void identify(Key& key) const { key(at::IntArrayRef(bias_shape))(general); }
+    variable_list run(const std::vector<Tensor>& kept, const Tensor& dy, const Asked& asked) const {
+        const Tensor &x = kept[0], &w = kept[1];
+        const bool need_x = has(asked.now, 0), need_w = has(asked.now, 1), need_b = has(asked.now, 2);
         auto res = product_backward(x, w, dy, need_x, need_w, need_b ? MaybeShape(bias_shape) : std::nullopt);
         if (res) return {std::get<0>(*res), std::get<1>(*res), std::get<2>(*res)};
         return listed(general->call<Three>(x, w, dy, need_x, need_w, need_b ? MaybeShape(bias_shape) : std::nullopt));
@@ -141,29 +230,27 @@ MaybeTensor linear_shard(const Tensor& x, const Tensor& w, const MaybeTensor& bi
         y = product(x, w, bias);
     }
     if (!y || !at::GradMode::is_enabled() || !(wanted(x) || wanted(w) || wanted(bias))) return y;
-    auto node = make_node<LinearShardBackward>({x, w, bias});
+    auto node = make_node(LinearShard{bias ? bias->sizes().vec() : std::vector<int64_t>(), general}, {x, w, bias});
     node->save(x);
     node->save(w);
-    if (bias) node->bias_shape = bias->sizes().vec();
-    node->general = general;
     torch::autograd::create_gradient_edge(*y, node);
     return y;
 }
 
 // ------------------------------------------------------------ layer norm --
 
-struct LayerNormShardBackward : ShardNode {
+struct LayerNormShard {
+    static constexpr const char* kName = "LayerNormShardBackward";
     MaybeShape gamma_shape, beta_shape;
     int64_t workers = 1;
     Shared gather, general;   // gather: this worker's row sums -> those of all workers
-    std::string name() const override { return "LayerNormShardBackward"; }
-    variable_list apply(variable_list&& grads) override {
-        const std::vector<Tensor> kept = unpacked();
-        const Tensor &x2d = kept[0], &mean = kept[1], &rstd = kept[2], dy = gradient(grads);
+    void identify(Key& key) const { key(gamma_shape)(beta_shape)(workers)(gather)(general); }
+    variable_list run(const std::vector<Tensor>& kept, const Tensor& dy, const Asked& asked) const {
+        const Tensor &x2d = kept[0], &mean = kept[1], &rstd = kept[2];
         const MaybeTensor gamma = defined(kept[3]);
         // Those that require gradients, whether or not this pass asks for them: the order of the sums hangs on it.
-        const bool need_x = should_compute_output(0);
-        const MaybeShape for_gamma = should_compute_output(1) ? gamma_shape : std::nullopt, for_beta = should_compute_output(2) ? beta_shape : std::nullopt;
+        const bool need_x = has(asked.ever, 0);
+        const MaybeShape for_gamma = has(asked.ever, 1) ? gamma_shape : std::nullopt, for_beta = has(asked.ever, 2) ? beta_shape : std::nullopt;
         std::optional<std::tuple<Tensor, Tensor, Tensor>> res;
         if (need_x && workers == 1) {
             res = ln_backward_whole(dy, x2d, mean, rstd, gamma, for_gamma, for_beta);
@@ -187,14 +274,12 @@ MaybeTensor normalized(const Tensor& x, const MaybeTensor& gamma, const MaybeTen
                        const Shared& gather, const Shared& general) {
     if (!res) return std::nullopt;
     Tensor y = std::get<0>(*res);
-    auto node = make_node<LayerNormShardBackward>({x, gamma, beta});
+    auto shape = [](const MaybeTensor& t) { return t ? MaybeShape(t->sizes().vec()) : std::nullopt; };
+    auto node = make_node(LayerNormShard{shape(gamma), shape(beta), workers, gather, general}, {x, gamma, beta});
     node->save(std::get<1>(*res));
     node->save(std::get<2>(*res));
     node->save(std::get<3>(*res));
     node->save(std::get<4>(*res));
-    if (gamma) node->gamma_shape = gamma->sizes().vec();
-    if (beta) node->beta_shape = beta->sizes().vec();
-    node->workers = workers, node->gather = gather, node->general = general;
     torch::autograd::create_gradient_edge(y, node);
     return y;
 }
@@ -221,16 +306,16 @@ Tensor layer_norm_node(const Tensor& x, const MaybeTensor& gamma, const MaybeTen
 
 // ------------------------------------------------------------- embedding --
 
-struct EmbeddingShardBackward : ShardNode {
+struct EmbeddingShard {
+    static constexpr const char* kName = "EmbeddingShardBackward";
     int64_t lo = 0, hi = 0;
     std::optional<int64_t> padding_idx;
     bool by_freq = false;
     Shared general;
-    std::string name() const override { return "EmbeddingShardBackward"; }
-    variable_list apply(variable_list&& grads) override {
-        const std::vector<Tensor> kept = unpacked();
-        const Tensor &ids = kept[0], dy = gradient(grads);
-        if (!task_should_compute_output(0)) return {Tensor()};
+    void identify(Key& key) const { key(lo)(hi)(int64_t{padding_idx.has_value()})(padding_idx.value_or(0))(int64_t{by_freq})(general); }
+    variable_list run(const std::vector<Tensor>& kept, const Tensor& dy, const Asked& asked) const {
+        const Tensor& ids = kept[0];
+        if (!has(asked.now, 0)) return {Tensor()};
         const MaybeTensor dw = embedding_backward(dy, ids, lo, hi, padding_idx.value_or(-1), by_freq);
         if (dw) return {*dw};
         return {general->call<Tensor>(dy, ids, lo, hi, padding_idx, by_freq)};
@@ -242,9 +327,8 @@ MaybeTensor embedding_shard(const Tensor& weight, const Tensor& ids, int64_t lo,
     if (!unobserved() || !ordinary(weight) || !ordinary(ids) || !float_code(weight)) return std::nullopt;
     MaybeTensor y = embedding_gather(weight, ids, lo, hi);
     if (!y || !at::GradMode::is_enabled() || !wanted(weight)) return y;
-    auto node = make_node<EmbeddingShardBackward>({weight});
+    auto node = make_node(EmbeddingShard{lo, hi, padding_idx, by_freq, general}, {weight});
     node->save(ids);
-    node->lo = lo, node->hi = hi, node->padding_idx = padding_idx, node->by_freq = by_freq, node->general = general;
     torch::autograd::create_gradient_edge(*y, node);
     return y;
 }
@@ -312,58 +396,52 @@ private:
     int64_t epoch_;
 };
 
-struct MoveBackward : ShardNode {
-    std::shared_ptr<Moves> adjoint;
-    std::string name() const override { return "MoveBackward"; }
-    variable_list apply(variable_list&& grads) override {
-        const Tensor dy = gradient(grads);
-        return {adjoint->takes(dy) ? adjoint->run(dy) : adjoint->general(dy)};
-    }
+struct Move {
+    static constexpr const char* kName = "MoveBackward";
+    std::shared_ptr<Moves> moves;
+    void identify(Key& key) const { key(moves); }
+    variable_list run(const std::vector<Tensor>&, const Tensor& dy, const Asked&) const { return {moves->takes(dy) ? moves->run(dy) : moves->general(dy)}; }
 };
 
 MaybeTensor move(const Tensor& x, const std::shared_ptr<Moves>& forward, const std::shared_ptr<Moves>& adjoint) {
     const bool graph = at::GradMode::is_enabled() && wanted(x);
     if (!forward->takes(x) || (graph && !adjoint) || !unobserved() || !ordinary(x)) return std::nullopt;
     Tensor y = forward->run(x);
-    if (graph) {
-        auto node = make_node<MoveBackward>({x});
-        node->adjoint = adjoint;
-        torch::autograd::create_gradient_edge(y, node);
-    }
+    if (graph) torch::autograd::create_gradient_edge(y, make_node(Move{adjoint}, {x}));
     return y;
 }
 
 // ----------------------------------------------------------------- alias --
 
 // What a rank that is alone hands to itself: a result of its own on the same memory.
-struct AliasBackward : ShardNode {
-    std::string name() const override { return "AliasBackward"; }
-    variable_list apply(variable_list&& grads) override { return {gradient(grads)}; }
+struct Alias {
+    static constexpr const char* kName = "AliasBackward";
+    void identify(Key&) const {}
+    variable_list run(const std::vector<Tensor>&, const Tensor& dy, const Asked&) const { return {dy}; }
 };
 
 MaybeTensor alias(const Tensor& x) {
     if (!unobserved() || !ordinary(x)) return std::nullopt;
     Tensor y = x.detach();
-    if (at::GradMode::is_enabled() && wanted(x)) torch::autograd::create_gradient_edge(y, make_node<AliasBackward>({x}));
+    if (at::GradMode::is_enabled() && wanted(x)) torch::autograd::create_gradient_edge(y, make_node(Alias{}, {x}));
     return y;
 }
 
 // ---------------------------------------------------------------- Python --
 
 // y, computed from x in Python, with an adjoint in Python.
-struct CallBackward : ShardNode {
-    Shared adjoint;
-    std::string name() const override { return "CallBackward"; }
-    variable_list apply(variable_list&& grads) override { return {adjoint->call<Tensor>(gradient(grads))}; }
+struct Call {
+    static constexpr const char* kName = "CallBackward";
+    Shared function;
+    void identify(Key& key) const { key(function); }
+    variable_list run(const std::vector<Tensor>&, const Tensor& dy, const Asked&) const { return {function->call<Tensor>(dy)}; }
 };
 
 bool attachable(const Tensor& x) { return at::GradMode::is_enabled() && wanted(x) && unobserved() && ordinary(x); }
 
 Tensor attach(Tensor y, const Tensor& x, const Shared& adjoint) {
     if (y.requires_grad() || !at::isFloatingType(y.scalar_type())) throw std::invalid_argument("attach: a result with a history of its own");
-    auto node = make_node<CallBackward>({x});
-    node->adjoint = adjoint;
-    torch::autograd::create_gradient_edge(y, node);
+    torch::autograd::create_gradient_edge(y, make_node(Call{adjoint}, {x}));
     return y;
 }
 

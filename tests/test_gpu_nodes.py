@@ -292,3 +292,19 @@ def test_passes_of_several_threads():
         t.join()
     torch.cuda.synchronize()
     assert not errors
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_compiled_autograd_runs_through_the_nodes(general, name):
+    """The bits of an ordinary pass, under the compiled one as it is recorded, with other values, and for another layer alike."""
+    from torch._dynamo import compiled_autograd
+    for seed in (5, 6):
+        layer, x, params = _case(name)
+        wanted = ([x] if x.is_floating_point() else []) + params
+        dy = _randn(*layer(x).shape, dtype=params[0].dtype if params else x.dtype, seed=seed)
+        want = [_step(layer, x, wanted, k * dy) for k in (1, 2)] + [_step(layer, x, wanted[-1:], dy)]
+        with compiled_autograd._enable(lambda graph: graph):
+            got = [_step(layer, x, wanted, k * dy) for k in (1, 2)] + [_step(layer, x, wanted[-1:], dy)]
+        for a, b in zip(got, want):
+            _same(a, b)
+        assert type(layer(x).grad_fn).__name__ != type(general(lambda: layer(x)).grad_fn).__name__

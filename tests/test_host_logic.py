@@ -1120,3 +1120,47 @@ def test_tensors_that_stay_keep_their_type(which):
     layer(x).sum().backward()
     assert torch.equal(x.grad, torch.ones(3, 4))
     assert type(layer(torch.nn.Parameter(plain))) is type(layer(plain)) is torch.Tensor
+
+
+class _Drop(torch.autograd.Function):
+
+    @staticmethod
+    def forward(ctx, x):
+        return x * 2
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_compiled_autograd_runs_through_layers_whose_tensor_stays(which):
+    """The same gradients as without it: for new values and shapes, for some of the inputs, in a second pass, and where none arrives."""
+    from torch._dynamo import compiled_autograd
+    layer = _grid_layers()[which]
+
+    def passes():
+        out = []
+        for n in (3, 3, 5):
+            x, w = torch.randn(n, generator=torch.Generator().manual_seed(n + len(out))).requires_grad_(True), torch.ones(n, requires_grad=True)
+            z = (layer(x) ** 2 * layer(layer(w))).sum()
+            out += torch.autograd.grad(z, [w], retain_graph=True)
+            out += torch.autograd.grad(z, [x, w])
+            (_Drop.apply(layer(x)) + 1).sum().backward()
+            out.append(x.grad)
+        return out
+    want = passes()
+    with compiled_autograd._enable(lambda graph: graph):
+        got = passes()
+    assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_compiled_autograd_tells_adjoints_in_python_apart():
+    from torch._dynamo import compiled_autograd
+    ext = _lib.extension()
+    with compiled_autograd._enable(lambda graph: graph):
+        for factor in (2.0, 3.0, 2.0):
+            x = torch.ones(4, requires_grad=True)
+            y = ext.attach(x.detach() * factor, x, ext.Callback(lambda g, f=factor: g * f))
+            y.sum().backward()
+            assert torch.equal(x.grad, torch.full((4,), factor))
