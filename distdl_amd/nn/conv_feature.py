@@ -147,7 +147,7 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         self.needed_slices = None
         self.halo_layer = None
         self._staging_plan = None
-        self._moves = _lib.Own()      # (what they are for, staging and its adjoint as native moves or None)
+        self._moves = _lib.Own()      # (what they are for, staging and its adjoint as native moves, see HaloExchange)
         self._distdl_is_setup = False
         self._input_tensor_structure = TensorStructure()
 
@@ -238,8 +238,10 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
             moves = self._moves.value
             key = (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, _buffer.reallocations())
             if moves is None or moves[0] != key:
-                moves = self._moves.value = self._native_staging(input)
-            exchanged = None if moves[1] is None else _lib.front().move(input, *moves[1])
+                moves = self._moves.value = (key, None)
+            elif moves[1] is None:
+                moves = self._moves.value = (key, self._native_staging(input))
+            exchanged = _lib.front().move(input, *moves[1]) if moves[1] else None
             if exchanged is None:
                 exchanged = _HaloStaging.apply(input, self._staging_plan, *self._fused_slabs(input))
         else:
@@ -253,12 +255,12 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         return _Crop.apply(exchanged, crop)
 
     def _native_staging(self, input):
-        """(what they are for, staging and its adjoint as native moves or None)"""
+        """Staging and its adjoint as native moves, () where the general way takes the input."""
         self._fused_slabs(input)          # what is to be reallocated is so from here on
-        epoch, key = _lib.buffers_epoch(), (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, _buffer.reallocations())
+        epoch = _lib.buffers_epoch()
         if not input.is_cuda or not input.is_contiguous() or tuple(input.shape) != self._staging_plan.x_shape:
-            return key, None
-        return key, self._staging_plan.moves(epoch, input, *self._fused_slabs(input))
+            return ()
+        return self._staging_plan.moves(epoch, input, *self._fused_slabs(input))
 
     def _fused_slabs(self, input):
         """Ghost and bulk slabs of the fused pass as ``[dim][side]`` tables of

@@ -76,7 +76,7 @@ class Repartition(Module):
         self.buffer_manager = buffer_manager
         self.P_x_to_y_buffers = None
         self.P_y_to_x_buffers = None
-        self._moves = _lib.Own()      # (what they are for, forward and adjoint as native moves or None)
+        self._moves = _lib.Own()      # (what they are for, forward and adjoint as native moves, see HaloExchange)
 
         self._distdl_is_setup = False
         self._input_tensor_structure = TensorStructure()
@@ -189,8 +189,10 @@ class Repartition(Module):
         key = (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, type(transport), _buffer.reallocations())
         moves = self._moves.value
         if moves is None or moves[0] != key:
-            moves = self._moves.value = (key, functional.native_repartition(input, *args))
-        if moves[1] is not None:
+            moves = self._moves.value = (key, None)
+        elif moves[1] is None:
+            moves = self._moves.value = (key, functional.native_repartition(input, *args) or ())
+        if moves[1]:
             y = _lib.front().move(input, *moves[1])
             if y is not None:
                 return y
