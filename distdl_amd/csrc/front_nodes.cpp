@@ -417,7 +417,8 @@ MaybeTensor move(const Tensor& x, const std::shared_ptr<Moves>& forward, const s
 struct Alias {
     static constexpr const char* kName = "AliasBackward";
     void identify(Key&) const {}
-    variable_list run(const std::vector<Tensor>&, const Tensor& dy, const Asked&) const { return {dy}; }
+    // No layer's adjoint has a history of its own, so a second derivative does not go through this one either.
+    variable_list run(const std::vector<Tensor>&, const Tensor& dy, const Asked&) const { return {at::GradMode::is_enabled() ? dy.detach() : dy}; }
 };
 
 MaybeTensor alias(const Tensor& x) {

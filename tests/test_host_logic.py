@@ -1122,6 +1122,14 @@ def test_tensors_that_stay_keep_their_type(which):
     assert type(layer(torch.nn.Parameter(plain))) is type(layer(plain)) is torch.Tensor
 
 
+@pytest.mark.parametrize("which", [0, 1])
+def test_adjoints_of_tensors_that_stay_have_no_history(which):
+    """As those of every other layer: a gradient made for a second pass ends there."""
+    layer, x = _grid_layers()[which], torch.randn(3, requires_grad=True)
+    grad, = torch.autograd.grad((layer(x) ** 3).sum(), x, create_graph=True)
+    assert torch.equal(grad, 3 * x.detach() ** 2) and not grad.requires_grad
+
+
 class _Drop(torch.autograd.Function):
 
     @staticmethod
