@@ -128,6 +128,7 @@ SIGNATURES = {
     "ddl_linear_backward_workspace_at": (c_int64, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int,
                                                    c_int]),
     "ddl_linear_backward_workspace": (c_int64, [c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_int]),
+    "ddl_linear_backward_plan": (c_int, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int64, c_void_p]),
     "ddl_linear_backward": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64,
                                     c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p]),
     "ddl_gemm_f32": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64,

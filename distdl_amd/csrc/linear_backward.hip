@@ -13,6 +13,8 @@
 #include "gemm16_small.h"
 #include "gemm32_small.h"
 
+#include <type_traits>
+
 namespace ddl {
 namespace {
 
@@ -318,7 +320,41 @@ static AdjointPlan32 adjoint32(int64_t M, int64_t N, int64_t K, int64_t ldx, int
     return plan_adjoint32(M, N, K, want_db, cus, workspace, x, w);
 }
 
+// dx, dw and, `inside`, db in one launch, if that is how they are computed.
+struct OneLaunch {
+    bool taken = false, inside = false;
+    AdjointPlan32 wide;
+    AdjointPlan16 narrow;
+};
+
+static OneLaunch one_launch(int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy, bool aligned, bool want_db, int64_t workspace) {
+    OneLaunch plan;
+    if (dtype == DDL_DT_F32) {
+        plan.inside = want_db && M <= kAdjointRows32;
+        plan.wide = adjoint32(M, N, K, ldx, ldw, lddy, plan.inside, workspace);
+        plan.taken = plan.wide.groups_x != 0;
+    } else if (dtype == DDL_DT_BF16 || dtype == DDL_DT_F16) {
+        plan.inside = want_db && M <= kAdjointRows;
+        plan.narrow = adjoint16(M, N, K, ldx, ldw, lddy, aligned, plan.inside, workspace);
+        plan.taken = plan.narrow.edge_x != 0;
+    }
+    return plan;
+}
+
 }  // namespace ddl
+
+extern "C" int ddl_linear_backward_plan(int dtype, int aligned, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t lddy, int want_db,
+                                        int64_t workspace_elems, int* plan) {
+    using namespace ddl;
+    if (M < 1 || N < 1 || K < 1 || !plan) return 0;
+    const OneLaunch one = one_launch(dtype, M, N, K, ldx, ldw, lddy, aligned != 0, want_db != 0, workspace_elems);
+    if (!one.taken) return 0;
+    const bool wide = dtype == DDL_DT_F32;
+    plan[0] = wide ? one.wide.groups_x : one.narrow.edge_x, plan[1] = wide ? one.wide.groups_w : one.narrow.edge_w;
+    plan[2] = wide ? one.wide.splits_x : one.narrow.splits_x, plan[3] = wide ? one.wide.splits_w : one.narrow.splits_w;
+    plan[4] = one.inside;
+    return 1;
+}
 
 extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                                                     int64_t lddy, int want_dx, int want_dw, int want_db) {
@@ -327,22 +363,12 @@ extern "C" int64_t ddl_linear_backward_workspace_at(int dtype, int aligned, int6
     int64_t most = 0;
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     auto take = [&](int64_t elems) { most = elems > most ? elems : most; };
-    const bool wide = dtype == DDL_DT_F32, narrow = dtype == DDL_DT_BF16 || dtype == DDL_DT_F16;
-    if (want_dx && want_dw && (wide || narrow)) {   // both in one launch, with a part of the workspace each
-        const bool inside = want_db && M <= (wide ? ddl::kAdjointRows32 : ddl::kAdjointRows);
-        bool taken;
-        if (wide) {
-            const ddl::AdjointPlan32 plan = ddl::adjoint32(M, N, K, ldx, ldw, lddy, inside, INT64_MAX);
-            taken = plan.groups_x != 0;
-            take(plan.workspace);
-        } else {
-            const ddl::AdjointPlan16 plan = ddl::adjoint16(M, N, K, ldx, ldw, lddy, aligned != 0, inside, INT64_MAX);
-            taken = plan.edge_x != 0;
-            take(plan.workspace);
-        }
-        if (taken) {
+    if (want_dx && want_dw) {   // both in one launch, with a part of the workspace each
+        const ddl::OneLaunch plan = ddl::one_launch(dtype, M, N, K, ldx, ldw, lddy, aligned != 0, want_db != 0, INT64_MAX);
+        if (plan.taken) {
+            take(plan.wide.workspace + plan.narrow.workspace);
             want_dx = want_dw = 0;
-            if (inside) want_db = 0;
+            if (plan.inside) want_db = 0;
         }
     }
     for (int both = aligned ? 1 : 0; both < 2; ++both) {
@@ -366,34 +392,26 @@ extern "C" int ddl_linear_backward(const void* x, const void* w, const void* dy,
     using namespace ddl;
     if (M < 1 || N < 1 || K < 1) return fail(DDL_E_ARG, "linear backward: M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
     if (!dy || (dx && !w) || (dw && !x)) return fail(DDL_E_ARG, "linear backward: null pointer");
-    if ((dtype == DDL_DT_BF16 || dtype == DDL_DT_F16) && dx && dw && aligned_to(x, 2) && aligned_to(w, 2) && aligned_to(dy, 2) && aligned_to(dx, 2) &&
-        aligned_to(dw, 2) && aligned_to(db, 2) && (!workspace || aligned_to(workspace, 16))) {
+    const int es = dtype == DDL_DT_F32 ? 4 : 2;
+    if (dx && dw && aligned_to(x, es) && aligned_to(w, es) && aligned_to(dy, es) && aligned_to(dx, es) && aligned_to(dw, es) && aligned_to(db, es) &&
+        (!workspace || aligned_to(workspace, 16))) {
         const bool aligned = aligned_to(x, 16) && aligned_to(w, 16) && aligned_to(dy, 16);
-        const int64_t room = workspace ? workspace_elems : 0;
-        const bool inside = db && M <= kAdjointRows;
-        const AdjointPlan16 plan = adjoint16(M, N, K, ldx, ldw, lddy, aligned, inside, room);
-        if (plan.edge_x) {
-            Part16 to_x{}, to_w{};
-            to_x.x = static_cast<const uint16_t*>(dy), to_x.ldx = lddy, to_x.w = static_cast<const uint16_t*>(w), to_x.ldw = ldw;
-            to_x.y = static_cast<uint16_t*>(dx), to_x.ldy = K, to_x.M = M, to_x.N = K, to_x.K = N;
-            to_w.x = static_cast<const uint16_t*>(dy), to_w.ldx = lddy, to_w.w = static_cast<const uint16_t*>(x), to_w.ldw = ldx;
-            to_w.y = static_cast<uint16_t*>(dw), to_w.ldy = K, to_w.M = N, to_w.N = K, to_w.K = M;
-            const int rc = run_adjoint16(plan, dtype == DDL_DT_F16, to_x, to_w, inside ? db : nullptr, workspace, static_cast<hipStream_t>(stream));
-            return rc || inside || !db ? rc : ddl_colsum(dy, dtype, M, N, lddy, db, workspace, workspace_elems, stream);
-        }
-    }
-    if (dtype == DDL_DT_F32 && dx && dw && aligned_to(x, 4) && aligned_to(w, 4) && aligned_to(dy, 4) && aligned_to(dx, 4) && aligned_to(dw, 4) &&
-        aligned_to(db, 4) && (!workspace || aligned_to(workspace, 16))) {
-        const bool inside = db && M <= kAdjointRows32;
-        const AdjointPlan32 plan = adjoint32(M, N, K, ldx, ldw, lddy, inside, workspace ? workspace_elems : 0);
-        if (plan.groups_x) {
-            PartOf<float> to_x{}, to_w{};
-            to_x.x = static_cast<const float*>(dy), to_x.ldx = lddy, to_x.w = static_cast<const float*>(w), to_x.ldw = ldw;
-            to_x.y = static_cast<float*>(dx), to_x.ldy = K, to_x.M = M, to_x.N = K, to_x.K = N;
-            to_w.x = static_cast<const float*>(dy), to_w.ldx = lddy, to_w.w = static_cast<const float*>(x), to_w.ldw = ldx;
-            to_w.y = static_cast<float*>(dw), to_w.ldy = K, to_w.M = N, to_w.N = K, to_w.K = M;
-            const int rc = run_adjoint32(plan, to_x, to_w, inside ? static_cast<float*>(db) : nullptr, workspace, static_cast<hipStream_t>(stream));
-            return rc || inside || !db ? rc : ddl_colsum(dy, dtype, M, N, lddy, db, workspace, workspace_elems, stream);
+        const OneLaunch plan = one_launch(dtype, M, N, K, ldx, ldw, lddy, aligned, db != nullptr, workspace ? workspace_elems : 0);
+        if (plan.taken) {
+            auto run = [&](auto* element, auto&& launch) {
+                using T = std::remove_pointer_t<decltype(element)>;
+                PartOf<T> to_x{}, to_w{};
+                to_x.x = static_cast<const T*>(dy), to_x.ldx = lddy, to_x.w = static_cast<const T*>(w), to_x.ldw = ldw;
+                to_x.y = static_cast<T*>(dx), to_x.ldy = K, to_x.M = M, to_x.N = K, to_x.K = N;
+                to_w.x = static_cast<const T*>(dy), to_w.ldx = lddy, to_w.w = static_cast<const T*>(x), to_w.ldw = ldx;
+                to_w.y = static_cast<T*>(dw), to_w.ldy = K, to_w.M = N, to_w.N = K, to_w.K = M;
+                return launch(to_x, to_w, plan.inside ? db : nullptr);
+            };
+            const hipStream_t s = static_cast<hipStream_t>(stream);
+            const int rc = dtype == DDL_DT_F32
+                               ? run(static_cast<float*>(nullptr), [&](auto& to_x, auto& to_w, void* sums) { return run_adjoint32(plan.wide, to_x, to_w, static_cast<float*>(sums), workspace, s); })
+                               : run(static_cast<uint16_t*>(nullptr), [&](auto& to_x, auto& to_w, void* sums) { return run_adjoint16(plan.narrow, dtype == DDL_DT_F16, to_x, to_w, sums, workspace, s); });
+            return rc || plan.inside || !db ? rc : ddl_colsum(dy, dtype, M, N, lddy, db, workspace, workspace_elems, stream);
         }
     }
     // dx[m, j] = sum_n dy[m, n] w[n, j]: rows of the second operand are the columns of w

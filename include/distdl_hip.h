@@ -549,6 +549,15 @@ int ddl_linear_backward(const void* x, const void* w, const void* dy, void* dx,
                         void* dw, void* db, int dtype, int64_t M, int64_t N,
                         int64_t K, int64_t ldx, int64_t ldw, int64_t lddy,
                         float* workspace, int64_t workspace_elems, void* stream);
+/* How ddl_linear_backward computes dx and dw where both are wanted, given that many
+ * floats of workspace (16-byte aligned).  0: one after the other.  1: in one launch, with
+ * plan[0], plan[1] the tiles of dx and dw (16-bit types: 1 or 2 for 64 or 128 rows and
+ * columns; fp32: 1, 2 or 4 groups of wavefronts that share a reduction), plan[2], plan[3]
+ * the workgroups that share one of dx and of dw, and plan[4] whether db is summed there
+ * too. */
+int ddl_linear_backward_plan(int dtype, int aligned, int64_t M, int64_t N,
+                             int64_t K, int64_t ldx, int64_t ldw, int64_t lddy,
+                             int want_db, int64_t workspace_elems, int* plan);
 int ddl_gemm_f32(const float* a, int64_t a_row_stride, int64_t a_k_stride,
                  const float* b, int64_t b_row_stride, int64_t b_k_stride,
                  const float* bias, float* y, int64_t ldy,

@@ -2,6 +2,8 @@
 the k-tile that needs care, reductions shorter than a load; and the rings of the fp32 products.  (The small tiles' own cases are in
 test_gpu_layers.py.)"""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -76,15 +78,52 @@ def test_fp32_reductions_around_the_ring_of_stages(a_t, b_t, M, N):
 
 
 _ADJOINTS = [
-    # one k-tile and one element more, 64 x 64 tiles, an odd length of every kind; 128 x 128 tiles of either product; both with
-    # split reductions; as many rows as the column sums take there, and one more; aligned throughout
+    # one k-tile and one element more, 64 x 64 tiles, an odd length of every kind; 128 x 128 tiles of both products and of dx;
+    # split reductions of either; many rows and few columns, without db in one launch; one row more than the column sums take
+    # there; aligned throughout
     (8, 8, 8, 0, 0), (65, 64, 66, 1, 1), (97, 77, 603, 0, 0), (718, 821, 2056, 0, 3), (2048, 1024, 1024, 0, 0), (3001, 130, 257, 2, 0),
     (16384, 24, 40, 0, 0), (16385, 17, 33, 0, 1), (9, 5001, 1200, 0, 0), (1200, 9, 5001, 1, 0)]
 _ADJOINTS_32 = [
-    # fewer elements than a k-tile, one more than one, tiles of every size for either product, split reductions, as many rows as the
-    # column sums take there and one more, more tiles than one launch takes
+    # too few rows and too many tiles for one launch, which go one after the other (the first two, the last); fewer elements than a
+    # k-tile, split reductions, as many rows as the column sums take there and one more
     (2, 2, 2, 0, 0), (5, 3, 7, 1, 1), (33, 31, 35, 0, 0), (97, 77, 603, 0, 3), (777, 333, 1024, 0, 0), (104, 1256, 960, 0, 0), (108, 192, 5376, 2, 1),
     (2048, 24, 40, 0, 0), (2049, 17, 33, 0, 1), (512, 512, 512, 0, 0), (1500, 130, 257, 3, 0), (2500, 900, 300, 0, 0)]
+
+
+# What one launch is made of, and the sizes that take it with room for all splits: (tiles of dx and dw, workgroups that share a
+# reduction of each, db summed there too), see ddl_linear_backward_plan.
+_PLANNED = [
+    ((1, 1, 1, 1, 1), (65, 64, 66, 1, 1)), ((1, 1, 8, 1, 1), (8, 2064, 8, 3, 3)), ((1, 1, 1, 3, 1), (2412, 9, 9, 0, 1)),
+    ((1, 1, 8, 2, 1), (512, 1928, 8, 3, 3)),        # dw's partial sums lie behind those of dx
+    ((1, 2, 1, 1, 1), (8, 840, 6480, 1, 0)), ((1, 2, 1, 4, 1), (6324, 2436, 105, 0, 0)),
+    ((2, 1, 1, 1, 1), (836, 8, 7779, 8, 8)), ((2, 1, 1, 3, 1), (16384, 130, 257, 0, 1)),   # as many rows as the column sums take there
+    ((2, 2, 1, 1, 1), (472, 66, 7510, 3, 3)), ((2, 2, 1, 6, 1), (4098, 66, 1151, 0, 1)), ((2, 2, 2, 6, 1), (6844, 2509, 71, 0, 1)),
+    ((1, 1, 1, 8, 0), (16385, 17, 33, 0, 1))]       # one row more
+_PLANNED_32 = [
+    ((1, 1, 1, 1, 1), (3, 8, 8, 1, 0)), ((1, 2, 1, 1, 1), (37, 8, 8, 1, 0)), ((1, 2, 1, 2, 1), (394, 8, 2105, 3, 3)),
+    ((1, 2, 3, 1, 1), (1282, 1815, 199, 3, 3)), ((1, 4, 1, 1, 1), (67, 8, 9, 0, 1)), ((1, 4, 1, 8, 1), (2048, 16, 9, 0, 1)),
+    ((2, 1, 1, 1, 1), (2, 33, 8, 3, 3)), ((2, 1, 2, 1, 1), (2, 232, 2852, 0, 0)), ((2, 2, 1, 1, 1), (38, 35, 9, 3, 3)),
+    ((2, 2, 1, 2, 1), (255, 35, 1392, 1, 0)), ((2, 2, 2, 1, 1), (41, 232, 1406, 3, 3)), ((2, 2, 2, 2, 1), (267, 247, 508, 0, 0)),
+    ((2, 4, 1, 1, 1), (78, 36, 10, 3, 3)), ((2, 4, 1, 6, 1), (1647, 36, 9, 0, 0)), ((2, 4, 8, 1, 1), (335, 1483, 34, 0, 0)),
+    ((2, 4, 1, 8, 0), (2499, 33, 9, 8, 8)), ((4, 1, 1, 1, 1), (2, 81, 8, 0, 1)), ((4, 1, 4, 1, 1), (2, 1402, 10, 0, 1)),
+    ((4, 2, 1, 1, 1), (34, 77, 9, 0, 1)), ((4, 2, 4, 1, 1), (36, 1322, 10, 1, 0)), ((4, 4, 1, 1, 1), (65, 77, 8, 3, 3)),
+    ((4, 4, 1, 8, 1), (2028, 67, 8, 8, 8)), ((4, 4, 4, 1, 1), (71, 1411, 8, 0, 0)), ((4, 4, 6, 2, 1), (537, 1510, 11, 0, 1)),
+    (None, (2500, 900, 300, 0, 0)), (None, (2, 2, 2, 0, 0))]
+
+
+@pytest.mark.parametrize("dtype,plan,case", [(dt, *c) for dt in (torch.bfloat16, torch.float16) for c in _PLANNED] +
+                         [(torch.float32, *c) for c in _PLANNED_32])
+def test_every_form_of_the_adjoint_in_one_launch(dtype, plan, case):
+    """The sizes go where this list says, and the results are exact there."""
+    from distdl_amd import _lib
+    M, N, K, pad, shift = case
+    lib, dt = _lib.load(), {torch.bfloat16: _lib.DDL_DT_BF16, torch.float16: _lib.DDL_DT_F16, torch.float32: _lib.DDL_DT_F32}[dtype]
+    sizes = (int(pad % 8 == 0 and shift % 8 == 0), M, N, K, K + pad, K + pad, N + pad)
+    elems = lib.ddl_linear_backward_workspace_at(dt, *sizes, 1, 1, 1)
+    got = (ctypes.c_int * 5)()
+    taken = lib.ddl_linear_backward_plan(dt, *sizes, 1, elems, got)
+    assert (tuple(got) if taken else None) == plan
+    test_adjoint_of_a_linear_shard_in_one_launch(dtype, M, N, K, pad, shift)
 
 
 @pytest.mark.parametrize("dtype,M,N,K,pad,shift", [(dt, *c) for dt in (torch.bfloat16, torch.float16) for c in _ADJOINTS] +
