@@ -24,9 +24,10 @@ def route_of(P_send, P_recv, kind):
 
 
 def stays(P_send, P_recv):
-    """Whether a broadcast or a reduction between these leaves the tensor where it is, and its gradient too: the live rank of a
-    solo transport, in both partitions."""
-    return P_send.active and P_recv.active and type(P_send._world.transport) is SoloTransport
+    """Whether a broadcast or a reduction between these leaves the tensor where it is, and its gradient too, so that a native
+    node may take the call: the live rank of a solo transport, in both partitions.  torch.compile cannot look into native code,
+    but into the Functions, which one graph then holds with what is around them."""
+    return P_send.active and P_recv.active and type(P_send._world.transport) is SoloTransport and not torch.compiler.is_compiling()
 
 
 class BroadcastFunction(torch.autograd.Function):

@@ -1172,3 +1172,17 @@ def test_compiled_autograd_tells_adjoints_in_python_apart():
             y = ext.attach(x.detach() * factor, x, ext.Callback(lambda g, f=factor: g * f))
             y.sum().backward()
             assert torch.equal(x.grad, torch.full((4,), factor))
+
+
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("grad", [True, False])
+def test_layers_whose_tensor_stays_compile_into_one_graph(which, grad):
+    """torch.compile(fullgraph=True) raises at a native call that it cannot look into."""
+    layer, x = _grid_layers()[which], torch.arange(6.).view(2, 3).requires_grad_(grad)
+    layer(x)
+    torch._dynamo.reset()
+    y = torch.compile(lambda t: layer(t * 2) ** 2, fullgraph=True, backend="aot_eager")(x)
+    assert torch.equal(y, 4 * x ** 2)
+    if grad:
+        y.sum().backward()
+        assert torch.equal(x.grad, 8 * x)
