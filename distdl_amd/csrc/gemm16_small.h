@@ -37,7 +37,7 @@ struct AdjointPlan16 {
 constexpr int64_t kAdjointRows = 16384;      // of dy, for its column sums
 
 // Against `apart_us`, the estimate for the two products one after the other.
-AdjointPlan16 plan_adjoint16(int64_t M, int64_t N, int64_t K, bool want_db, int cus, int64_t workspace, double apart_us);
+AdjointPlan16 plan_adjoint16(int64_t M, int64_t N, int64_t K, bool aligned, bool want_db, int cus, int64_t workspace, double apart_us);
 
 // `dx` and `dw` describe the products as run_any16 has them (dy . w and dy^T . x), `db` may be null.
 int run_adjoint16(const AdjointPlan16& plan, bool f16, const Part16& dx, const Part16& dw, void* db, float* workspace, hipStream_t s);

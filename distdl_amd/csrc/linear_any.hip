@@ -413,16 +413,25 @@ Small16 plan_any16(bool xt, bool wt, int64_t M, int64_t N, int64_t K, int cus, i
 // Both products on one chip at the same time: a workgroup's k-tile takes what it does above, the rounds of all of them are
 // shared by the CUs, and the longest one is the least it can take; 4.1 or 6.1 as above, 5.5 for the launch that adds splits.
 // The other way is `apart_us` for the products and 4.5 for the column sum, and 3 for each of the two further launches, of
-// which 2 are the host's, where that may be what a step waits for.  Measured over 10 100 sizes (M, N 16 .. 8192, K 32 .. 8192,
-// some aligned): on average 2.03 times as fast as the launches one after the other, at worst 0.80 (M 5848, N 24, K 1408 aligned,
-// 22.9 -> 28.6 us; M 8192, N 512, K 1024 40.3 -> 42.1).
-AdjointPlan16 plan_adjoint16(int64_t M, int64_t N, int64_t K, bool want_db, int cus, int64_t workspace, double apart_us) {
+// which 2 are the host's, where that may be what a step waits for.
+// The best of these is taken if it also holds against what they leave out (careful_us): a long reduction in one piece takes 1.55
+// times as long where rows are not aligned, and where it is by far the longest it waits for the other product's workgroups while
+// not all are resident; the column sums take up to 2 ns a row; large products one after the other take 1.15 times `apart_us`.
+// Three launches and one, of calls that therefore stay with three: M 5848, N 24, K 1408 aligned 22.9 and 29.6 us, M 8983, N 47,
+// K 1624 39.6 and 62.1, M 8572, N 137, K 827 39.9 and 69.6, M 9975, N 17, K 37 19.6 and 28.2.  GPU time of 2204 calls for which
+// the first estimate is for one launch (M 16 .. 16384, N 8 .. 8192, K 32 .. 8192, half of them aligned), in a replayed graph, which
+// leaves out the host's share: 2069 take it, 1.5 times as fast as the three, 42 of them less than 0.95 times and at worst
+// 0.79 (the former rule: 140 and 0.57); 12 of the 135 others would be faster by more than 5 % in one launch, at most 1.14 times.
+// Of 1504 more calls with M above 2000, N up to 1024, drawn after the rule was made: 1312 take it, 1.3 times as fast, 75 less than 0.95
+// times and at worst 0.62 (M 2146, N 19, K 931: 12.8 and 20.5 us; the former rule: 206 and 0.57), 24 of 192 lose, at most 1.24 times.
+AdjointPlan16 plan_adjoint16(int64_t M, int64_t N, int64_t K, bool aligned, bool want_db, int cus, int64_t workspace, double apart_us) {
     AdjointPlan16 best;
     // operands along their rows have at least eight, dy read along n as well
     if (M < 8 || N < 8 || K < 8 || (want_db && M > kAdjointRows)) return best;
     const double launch_us = apart_us < 35 ? 3 : 1;
-    double best_us = apart_us + (want_db ? 4.5 + launch_us : 0) + launch_us;
+    const double other_us = apart_us + (want_db ? 4.5 + launch_us : 0) + launch_us;
     const int64_t strips = want_db ? (N + kNarrow - 1) / kNarrow : 0;
+    double best_us = other_us, careful_us = 0;
     double least_us = 3 + 2 * (static_cast<double>(M) * N + (static_cast<double>(M) + N) * K * 2) / 6e6;   // operands and results once
     if (want_db && 4 + M * 0.0016 > least_us) least_us = 4 + M * 0.0016;                                       // one strip of the column sums
     for (int edges = 0; edges < 4; ++edges) {
@@ -439,19 +448,23 @@ AdjointPlan16 plan_adjoint16(int64_t M, int64_t N, int64_t K, bool want_db, int 
                 const int64_t floats = (sx > 1 ? bx * ex * ex : 0) * 4096 + (sw > 1 ? bw * ew * ew : 0) * 4096;
                 if ((sw > 1 && (bx + bw > resident || kw < 2 * sw)) || floats > workspace) break;
                 const double nx = static_cast<double>((kx + sx - 1) / sx), nw = static_cast<double>((kw + sw - 1) / sw);
-                const double all = (bx * (nx * cx + (ex == 1 ? 0.85 : 2.5)) + bw * (nw * cw + (ew == 1 ? 0.85 : 2.5))) / cus;
-                const double longest = nx * cx > nw * cw ? nx * cx : nw * cw;
-                double us = (ex == 1 && ew == 1 ? 4.1 : 6.1) + (all * 1.15 > longest ? all * 1.15 : longest) + static_cast<double>(strips) / cus;
-                if (us < least_us) us = least_us;
-                if (floats) us += 5.5 + static_cast<double>(floats) * 8 / 8e6;
+                const double all_x = bx * (nx * cx + (ex == 1 ? 0.85 : 2.5)) / cus, all_w = bw * (nw * cw + (ew == 1 ? 0.85 : 2.5)) / cus;
+                const double all = (all_x + all_w) * 1.15, longest = nx * cx > nw * cw ? nx * cx : nw * cw;
+                const double start_us = (ex == 1 && ew == 1 ? 4.1 : 6.1) + static_cast<double>(strips) / cus;
+                const double sums_us = floats ? 5.5 + static_cast<double>(floats) * 8 / 8e6 : 0;
+                double us = start_us + (all > longest ? all : longest);
+                us = (us > least_us ? us : least_us) + sums_us;
                 if (us >= best_us) continue;
-                best_us = us;
+                best_us = careful_us = us;
                 best.edge_x = static_cast<int>(ex), best.edge_w = static_cast<int>(ew), best.splits_x = sx, best.splits_w = sw, best.workspace = floats;
                 best.first_w = nw * cw > nx * cx;
+                double chain = longest * (aligned ? 1 : 1.55);
+                if (bx + bw > resident && chain > 1.5 * (all_x + all_w)) chain += 0.75 * (best.first_w ? all_x : all_w);
+                for (const double t : {start_us + chain, want_db ? 4 + M * 0.002 : 0}) careful_us = t + sums_us > careful_us ? t + sums_us : careful_us;
             }
         }
     }
-    return best;
+    return careful_us < (apart_us < 35 ? 1 : 1.15) * other_us ? best : AdjointPlan16{};
 }
 
 int run_adjoint16(const AdjointPlan16& plan, bool f16, const Part16& dx, const Part16& dw, void* db, float* workspace, hipStream_t s) {

@@ -638,7 +638,7 @@ AdjointPlan16 adjoint16(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ld
         return AdjointPlan16{};
     const double dx_us = alone_us(dy, w, aligned, M, K, N, cus), dw_us = alone_us(dy_t, x, aligned, N, K, M, cus);
     if (dx_us < 0 || dw_us < 0) return AdjointPlan16{};
-    return plan_adjoint16(M, N, K, want_db, cus, workspace, dx_us + dw_us);
+    return plan_adjoint16(M, N, K, aligned, want_db, cus, workspace, dx_us + dw_us);
 }
 
 }  // namespace ddl

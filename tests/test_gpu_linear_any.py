@@ -96,9 +96,9 @@ _PLANNED = [
     ((1, 1, 1, 1, 1), (65, 64, 66, 1, 1)), ((1, 1, 8, 1, 1), (8, 2064, 8, 3, 3)), ((1, 1, 1, 3, 1), (2412, 9, 9, 0, 1)),
     ((1, 1, 8, 2, 1), (512, 1928, 8, 3, 3)),        # dw's partial sums lie behind those of dx
     ((1, 2, 1, 1, 1), (8, 840, 6480, 1, 0)), ((1, 2, 1, 4, 1), (6324, 2436, 105, 0, 0)),
-    ((2, 1, 1, 1, 1), (836, 8, 7779, 8, 8)), ((2, 1, 1, 3, 1), (16384, 130, 257, 0, 1)),   # as many rows as the column sums take there
+    ((2, 1, 1, 1, 1), (836, 8, 7779, 8, 8)), ((2, 1, 1, 3, 1), (16384, 310, 266, 8, 8)),   # as many rows as the column sums take there
     ((2, 2, 1, 1, 1), (472, 66, 7510, 3, 3)), ((2, 2, 1, 6, 1), (4098, 66, 1151, 0, 1)), ((2, 2, 2, 6, 1), (6844, 2509, 71, 0, 1)),
-    ((1, 1, 1, 8, 0), (16385, 17, 33, 0, 1))]       # one row more
+    ((1, 1, 1, 8, 0), (16385, 10, 8, 0, 0))]       # one row more
 _PLANNED_32 = [
     ((1, 1, 1, 1, 1), (3, 8, 8, 1, 0)), ((1, 2, 1, 1, 1), (37, 8, 8, 1, 0)), ((1, 2, 1, 2, 1), (394, 8, 2105, 3, 3)),
     ((1, 2, 3, 1, 1), (1282, 1815, 199, 3, 3)), ((1, 4, 1, 1, 1), (67, 8, 9, 0, 1)), ((1, 4, 1, 8, 1), (2048, 16, 9, 0, 1)),

@@ -1186,3 +1186,15 @@ def test_layers_whose_tensor_stays_compile_into_one_graph(which, grad):
     if grad:
         y.sum().backward()
         assert torch.equal(x.grad, 8 * x)
+
+
+@pytest.mark.parametrize("aligned,M,N,K,taken", [
+    # dw is one long reduction beside more tiles of dx than are resident, at aligned rows and at others
+    (1, 5848, 24, 1408, 0), (0, 5848, 24, 1408, 0), (0, 8983, 47, 1624, 0), (0, 8572, 137, 827, 0), (0, 12212, 179, 1060, 0),
+    # long column sums
+    (0, 12065, 73, 149, 0), (0, 9975, 17, 37, 0),
+    (0, 336, 77, 603, 1), (1, 120, 2258, 3584, 1), (0, 718, 821, 5156, 1), (1, 1024, 4096, 1024, 1), (0, 2276, 456, 3299, 1), (1, 8192, 512, 512, 1)])
+def test_adjoint_of_a_linear_shard_in_one_launch_where_that_is_the_faster_way(aligned, M, N, K, taken):
+    lib, pad, plan = _lib.load(), 1 - aligned, (ctypes.c_int * 5)()
+    for dtype in (_lib.DDL_DT_BF16, _lib.DDL_DT_F16):
+        assert lib.ddl_linear_backward_plan(dtype, aligned, M, N, K, K + pad, K + pad, N + pad, 1, 1 << 40, plan) == taken
