@@ -86,6 +86,7 @@ SIGNATURES = {
                                  c_void_p, c_int, c_float, c_void_p, c_int64, c_void_p]),
     "ddl_ln_bwd_params": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_void_p, c_int64, c_void_p]),
+    "ddl_ln_bwd_partial_params_workspace": (c_int64, [c_int64, c_int64]),
     "ddl_ln_bwd_partial_params": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,
                                           c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "ddl_ln_bwd_input_params": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,

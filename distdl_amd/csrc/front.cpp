@@ -8,7 +8,6 @@
 // the callers in hip_ops.py then go their general way, which converts, copies or
 // raises.  A failing entry point raises RuntimeError as _lib.check does.  The
 // interpreter lock is released while a function runs.
-#include <algorithm>
 #include "front.h"
 
 namespace ddl_front {
@@ -161,22 +160,12 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> ln_backward_whole(const Tensor
     return std::make_tuple(dx, dg, db);
 }
 
-namespace {
-
-// As many splits as ddl_ln_bwd_partial_params makes given the room.
-int64_t joint_splits(int64_t rows, int64_t cols) {
-    if (cols <= 1024 || cols > 8192) return clamped((rows + 31) / 32, 256);
-    return std::max(clamped((rows + 3) / 4, 128), clamped((rows + 7) / 8, 256));
-}
-
-}  // namespace
-
 // Rows shared with other workers: this worker's row sums and partial column sums ...
 std::optional<std::tuple<Tensor, Tensor>> ln_backward_partial_params(const Tensor& dy, const Tensor& x2d, const Tensor& mean, const Tensor& rstd,
                                                                      const MaybeTensor& gamma) {
     if (!ln_backward_operands(dy, x2d, mean, rstd, gamma) || dy.sizes() != x2d.sizes()) return std::nullopt;
     const int64_t rows = x2d.size(0), cols = x2d.size(1);
-    Tensor sums = floats(dy, {rows, 2}), work = floats(dy, {2 * joint_splits(rows, cols) * cols});
+    Tensor sums = floats(dy, {rows, 2}), work = floats(dy, {ddl_ln_bwd_partial_params_workspace(rows, cols)});
     check(ddl_ln_bwd_partial_params(dy.data_ptr(), x2d.data_ptr(), float_code(x2d), rows, cols, cols, cols, mean.data_ptr<float>(), rstd.data_ptr<float>(),
                                     pointer(gamma), sums.data_ptr<float>(), work.data_ptr<float>(), work.numel(), current_stream()),
           "ddl_ln_bwd_partial_params");

@@ -802,6 +802,12 @@ extern "C" int ddl_ln_bwd_params(const void* dy, const void* x, int dtype, int64
     return rc;
 }
 
+extern "C" int64_t ddl_ln_bwd_partial_params_workspace(int64_t rows, int64_t cols) {
+    using namespace ddl;
+    if (rows < 0 || cols < 1) return 0;
+    return 2 * cols * joint_splits(rows, cols, 512 * cols);
+}
+
 extern "C" int ddl_ln_bwd_partial_params(const void* dy, const void* x, int dtype, int64_t rows, int64_t cols, int64_t ld_dy,
                                          int64_t ld_x, const float* mean, const float* rstd, const void* gamma, float* sums,
                                          float* workspace, int64_t workspace_elems, void* stream) {

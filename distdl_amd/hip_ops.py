@@ -623,11 +623,8 @@ def _ln_param_workspace(rows, cols, device):
 
 
 def _ln_joint_workspace(rows, cols, device):
-    """For ``ddl_ln_bwd_partial_params``: rows of 1025 to 8192 columns are summed in splits of four to eight rows."""
-    if not 1024 < cols <= 8192:
-        return _ln_param_workspace(rows, cols, device)
-    splits = max(1, min(256, max(min((rows + 3) // 4, 128), (rows + 7) // 8)))
-    return torch.empty(2 * splits * cols, dtype=torch.float32, device=device)
+    """For ``ddl_ln_bwd_partial_params``."""
+    return torch.empty(_lib.load().ddl_ln_bwd_partial_params_workspace(rows, cols), dtype=torch.float32, device=device)
 
 
 def ln_backward_partial_params(dy2d, x2d, mean, rstd, gamma):

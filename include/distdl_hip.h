@@ -332,8 +332,10 @@ int ddl_ln_bwd_params_f32(const float* dy, const float* x, int64_t rows,
  *                               from the partial sums in `workspace`
  *
  * Both calls take the same rows, cols, workspace and workspace_elems (at least
- * 2 * cols floats, up to 512 * cols are used); the second must follow the first
+ * 2 * cols floats, up to 512 * cols are used; ddl_ln_bwd_partial_params_workspace
+ * says how many the fastest way takes); the second must follow the first
  * on the same stream.  Element types as above; _f32 forms likewise. */
+int64_t ddl_ln_bwd_partial_params_workspace(int64_t rows, int64_t cols);
 int ddl_ln_bwd_partial_params(const void* dy, const void* x, int dtype,
                               int64_t rows, int64_t cols, int64_t ld_dy,
                               int64_t ld_x, const float* mean,

@@ -1198,3 +1198,17 @@ def test_adjoint_of_a_linear_shard_in_one_launch_where_that_is_the_faster_way(al
     lib, pad, plan = _lib.load(), 1 - aligned, (ctypes.c_int * 5)()
     for dtype in (_lib.DDL_DT_BF16, _lib.DDL_DT_F16):
         assert lib.ddl_linear_backward_plan(dtype, aligned, M, N, K, K + pad, K + pad, N + pad, 1, 1 << 40, plan) == taken
+
+
+def test_layer_norm_adjoint_is_handed_the_room_that_the_library_asks_for():
+    """Splits of four to eight rows for rows of 1025 to 8192 columns, of 32 for others; never more than a caller may have to give."""
+    from distdl_amd import hip_ops
+    lib = _lib.load()
+    for cols in (1, 1024, 1025, 4352, 8192, 8193, 16384):
+        for rows in (0, 1, 4, 5, 32, 33, 511, 512, 513, 1024, 1025, 2048, 8191, 8192, 100000):
+            elems = lib.ddl_ln_bwd_partial_params_workspace(rows, cols)
+            each = 32 if not 1024 < cols <= 8192 else 4 if rows <= 512 else 8 if rows >= 1024 else None
+            splits = 128 if each is None else max(1, min(256, -(-rows // each)))
+            assert elems == 2 * cols * splits <= 512 * cols, (rows, cols)
+            assert hip_ops._ln_joint_workspace(rows, cols, "cpu").numel() == elems
+    assert lib.ddl_ln_bwd_partial_params_workspace(-1, 8) == lib.ddl_ln_bwd_partial_params_workspace(8, 0) == 0
