@@ -147,7 +147,7 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         self.needed_slices = None
         self.halo_layer = None
         self._staging_plan = None
-        self._moves = _lib.Own()      # (what they are for, staging and its adjoint as native moves, see HaloExchange)
+        self._moves = _lib.Own()      # (what they are for, staging and its adjoint as native moves), see hip_ops.kept_moves
         self._distdl_is_setup = False
         self._input_tensor_structure = TensorStructure()
 
@@ -235,13 +235,12 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         if self._nothing_to_stage:
             return input
         if getattr(transport, "ghosts_preloaded", False):
-            moves = self._moves.value
             key = (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, _buffer.reallocations())
-            if moves is None or moves[0] != key:
-                moves = self._moves.value = (key, None)
-            elif moves[1] is None:
-                moves = self._moves.value = (key, self._native_staging(input))
-            exchanged = _lib.front().move(input, *moves[1]) if moves[1] else None
+            if self._moves.value is None or self._moves.value[0] != key:
+                self._fused_slabs(input)          # what is to be reallocated is so from here on
+                key = key[:-1] + (_buffer.reallocations(),)
+            moves = hip_ops.kept_moves(self._moves, key, input, lambda: self._native_staging(input))
+            exchanged = _lib.front().move(input, *moves) if moves else None
             if exchanged is None:
                 exchanged = _HaloStaging.apply(input, self._staging_plan, *self._fused_slabs(input))
         else:
@@ -255,11 +254,10 @@ class DistributedFeatureConvBase(Module, HaloMixin, ConvMixin):
         return _Crop.apply(exchanged, crop)
 
     def _native_staging(self, input):
-        """Staging and its adjoint as native moves, () where the general way takes the input."""
-        self._fused_slabs(input)          # what is to be reallocated is so from here on
+        """Staging and its adjoint as native moves, None where the general way takes the input."""
         epoch = _lib.buffers_epoch()
         if not input.is_cuda or not input.is_contiguous() or tuple(input.shape) != self._staging_plan.x_shape:
-            return ()
+            return None
         return self._staging_plan.moves(epoch, input, *self._fused_slabs(input))
 
     def _fused_slabs(self, input):

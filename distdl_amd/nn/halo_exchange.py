@@ -3,6 +3,7 @@
 import numpy as np
 
 from .. import _lib
+from .. import hip_ops
 from ..backends.stub_hip import buffer as _buffer
 from ..utilities.torch import TensorStructure
 from .module import Module
@@ -51,9 +52,7 @@ class HaloExchange(Module):
 
         self.slices = None
         self.buffers = None
-        # (what they are for, forward and adjoint as native moves): made when an input like the last one comes again, () where
-        # the general way takes it.  Made for every new input they cost a layer whose input keeps changing 25 of 175 us a call.
-        self._moves = _lib.Own()
+        self._moves = _lib.Own()      # (what they are for, forward and adjoint as native moves), see hip_ops.kept_moves
 
         if buffer_manager is None:
             buffer_manager = self._distdl_backend.BufferManager()
@@ -98,13 +97,9 @@ class HaloExchange(Module):
         functional = self._distdl_backend.functional.halo_exchange
         args = (self.P_x, self.slices, self.buffers, self.neighbor_ranks)
         key = (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, type(self.P_x._world.transport), _buffer.reallocations())
-        moves = self._moves.value
-        if moves is None or moves[0] != key:
-            moves = self._moves.value = (key, None)
-        elif moves[1] is None:
-            moves = self._moves.value = (key, functional.native_exchange(input, *args) or ())
-        if moves[1]:
-            y = _lib.front().move(input, *moves[1])
+        moves = hip_ops.kept_moves(self._moves, key, input, lambda: functional.native_exchange(input, *args))
+        if moves:
+            y = _lib.front().move(input, *moves)
             if y is not None:
                 return y
         return functional.HaloExchangeFunction.apply(input, *args)

@@ -3,6 +3,7 @@
 import numpy as np
 
 from .. import _lib
+from .. import hip_ops
 from ..backends.stub_hip import buffer as _buffer
 from ..utilities.slicing import compute_nd_slice_shape
 from ..utilities.slicing import compute_subshape
@@ -76,7 +77,7 @@ class Repartition(Module):
         self.buffer_manager = buffer_manager
         self.P_x_to_y_buffers = None
         self.P_y_to_x_buffers = None
-        self._moves = _lib.Own()      # (what they are for, forward and adjoint as native moves, see HaloExchange)
+        self._moves = _lib.Own()      # (what they are for, forward and adjoint as native moves), see hip_ops.kept_moves
 
         self._distdl_is_setup = False
         self._input_tensor_structure = TensorStructure()
@@ -187,13 +188,9 @@ class Repartition(Module):
                 self.P_y, self.P_y_to_x_overlaps, self.P_y_to_x_buffers, self.preserve_batch)
         transport = self.P_union._world.transport if self.P_union.active else None
         key = (input.shape, input.stride(), input.dtype, input.device, input.requires_grad, type(transport), _buffer.reallocations())
-        moves = self._moves.value
-        if moves is None or moves[0] != key:
-            moves = self._moves.value = (key, None)
-        elif moves[1] is None:
-            moves = self._moves.value = (key, functional.native_repartition(input, *args) or ())
-        if moves[1]:
-            y = _lib.front().move(input, *moves[1])
+        moves = hip_ops.kept_moves(self._moves, key, input, lambda: functional.native_repartition(input, *args))
+        if moves:
+            y = _lib.front().move(input, *moves)
             if y is not None:
                 return y
         return functional.RepartitionFunction.apply(input, *args)

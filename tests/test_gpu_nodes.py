@@ -311,16 +311,25 @@ def test_compiled_autograd_runs_through_the_nodes(general, name):
 
 
 @pytest.mark.parametrize("name", ["repartition", "exchange", "staging"])
-def test_layers_whose_input_keeps_changing_make_no_moves(monkeypatch, name):
-    """Moves are made when an input like the last one comes again, and give what the general way did before them."""
+def test_when_moves_are_made(monkeypatch, name):
+    """At once where a gradient is recorded, else when an input like the last one comes again; they give what the general way does."""
     from distdl_amd import hip_ops
     layer, x, _ = _case(name)
     made, real = [], hip_ops.native_moves
     monkeypatch.setattr(hip_ops, "native_moves", lambda *args, **kwargs: made.append(1) or real(*args, **kwargs))
-    plain, outs = x.detach(), []
-    for t in (x, plain, x, plain, x, x, x):
+    plain, outs, counts = x.detach(), [], []
+
+    def call(t):
         _fill(layer)
+        made.clear()
         outs.append(layer(t).detach())
-    assert len(made) == 2           # the last but one pass: forward and adjoint
+        counts.append(len(made))
+    with torch.no_grad():
+        for t in (x, plain, x, plain, plain, plain):
+            call(t)
+        assert counts == [0, 0, 0, 0, 1, 0]
+    for t in (x, x, plain, plain, x):
+        call(t)
+    assert counts[6:] == [2, 0, 0, 1, 2]           # forward and adjoint
     for out in outs:
         assert torch.equal(out, outs[0])
