@@ -589,10 +589,10 @@ struct ReduceArgs {
 // ---- hot rows ----
 // A workgroup owns 64 bytes of columns of one row.  What takes time is the
 // memory round trip, not the additions, so all threads fetch the pieces of the
-// next two batches of 256 tokens (128 in emb_bwd_sums) -- four lanes a token, 16 bytes a lane -- while one
+// next two batches -- four lanes a token, 16 bytes a lane -- while one
 // wavefront adds a batch in token order out of LDS, a column per lane: the sums stay strictly sequential per column with 512 tokens in
-// flight.  (With 256 bytes of columns and batches of 64 tokens a row of 11000 tokens
-// of 512 bytes took 370 us, here 100; 483 tokens of 2 KiB 20 us, here 9.  A wavefront
+// flight in emb_bwd_hot (batches of 256), 256 in emb_bwd_sums (of 128).  (With 256 bytes of columns and batches of 64 tokens a row of
+// 11000 tokens of 512 bytes took 370 us, in emb_bwd_hot 100; 483 tokens of 2 KiB 20 us and 9.  A wavefront
 // that walks its columns alone keeps 32 tokens in flight in the same registers: 55 us.)
 // The order of the tokens, where emb_bwd_buckets has not made it: up to 512 by counting the smaller ones, more through
 // a bit per token number in LDS (16 KiB for a window of 131072 of them) that is

@@ -401,29 +401,29 @@ __device__ __forceinline__ void gemm_tile(const Part& part, int tile_id, char* l
     const bool lines = ((reinterpret_cast<uintptr_t>(y) | static_cast<uintptr_t>(2 * ldy)) & 127) == 0;
     auto leave = [&](auto streaming) {   // a loop each: of two stores on one path the compiler makes one, an ordinary one
 #pragma unroll 4
-    for (int p = 0; p < TM * 16 * kChunks / 64; ++p) {
-        const int idx = p * 64 + lane;
-        const int row = idx / kChunks, chunk = idx % kChunks;
-        const int64_t m = m0 + wm + row;
-        const int64_t n = n0 + wn + chunk * 8;
-        const uint4 v = *reinterpret_cast<const uint4*>(region + row * kPitch + ((chunk ^ swz(row)) << 4));
-        if (m >= M || n >= N) continue;
-        uint16_t* dst = y + m * ldy + n;
-        if (n + 8 <= N) {
-            // at the alignment of an element (global memory takes any)
-            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-            typedef u32x4 any __attribute__((aligned(2)));
-            u32x4 nv;
-            nv[0] = v.x, nv[1] = v.y, nv[2] = v.z, nv[3] = v.w;
-            if constexpr (decltype(streaming)::value) __builtin_nontemporal_store(nv, reinterpret_cast<any*>(dst));
-            else *reinterpret_cast<any*>(dst) = nv;
-        } else {
-            const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+        for (int p = 0; p < TM * 16 * kChunks / 64; ++p) {
+            const int idx = p * 64 + lane;
+            const int row = idx / kChunks, chunk = idx % kChunks;
+            const int64_t m = m0 + wm + row;
+            const int64_t n = n0 + wn + chunk * 8;
+            const uint4 v = *reinterpret_cast<const uint4*>(region + row * kPitch + ((chunk ^ swz(row)) << 4));
+            if (m >= M || n >= N) continue;
+            uint16_t* dst = y + m * ldy + n;
+            if (n + 8 <= N) {
+                // at the alignment of an element (global memory takes any)
+                typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+                typedef u32x4 any __attribute__((aligned(2)));
+                u32x4 nv;
+                nv[0] = v.x, nv[1] = v.y, nv[2] = v.z, nv[3] = v.w;
+                if constexpr (decltype(streaming)::value) __builtin_nontemporal_store(nv, reinterpret_cast<any*>(dst));
+                else *reinterpret_cast<any*>(dst) = nv;
+            } else {
+                const uint32_t words[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (n + e < N) dst[e] = static_cast<uint16_t>(words[e >> 1] >> (16 * (e & 1)));
+                for (int e = 0; e < 8; ++e)
+                    if (n + e < N) dst[e] = static_cast<uint16_t>(words[e >> 1] >> (16 * (e & 1)));
+            }
         }
-    }
     };
     if (lines) leave(std::true_type{});
     else leave(std::false_type{});
