@@ -491,11 +491,11 @@ struct Piece {
 };
 
 template <typename T, int THREADS, int NV, int RU, bool WITH_DX, bool ANY>
-__global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict__ dy, const T* __restrict__ x, int64_t rows, int64_t cols,
-                                                             int64_t ld_dy, int64_t ld_x, const float* __restrict__ mean,
+__global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict__ dy, const T* __restrict__ x, int64_t cols, int64_t ld_dy,
+                                                             int64_t ld_x, const float* __restrict__ mean,
                                                              const float* __restrict__ rstd, const T* __restrict__ gamma,
-                                                             float* __restrict__ sums, bool backwards, float* __restrict__ partial,
-                                                             float weight, T* __restrict__ dx, int64_t ld_dx) {
+                                                             float* __restrict__ sums, int rows_each, int rows_over, bool backwards,
+                                                             float* __restrict__ partial, float weight, T* __restrict__ dx, int64_t ld_dx) {
 #pragma clang fp contract(off)   // both instantiations round alike
     constexpr int V = 4;
     typedef Piece<T, ANY> P;
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int n = static_cast<int>(cols), pieces = (n + V - 1) / V;
     auto column = [&](int c) { return piece_column<ANY>(V * c, n); };
-    const int64_t splits = gridDim.x, own = blockIdx.x < rows ? (rows - 1 - blockIdx.x) / splits + 1 : 0;   // rows of this split
+    const int64_t splits = gridDim.x, own = rows_each + (static_cast<int>(blockIdx.x) < rows_over ? 1 : 0);   // rows of this split
     const int64_t first = backwards ? blockIdx.x + (own - 1) * splits : blockIdx.x, step = backwards ? -splits : splits;
     auto row_at = [&](int64_t i) { return first + i * step; };
     Raw g[NV];
@@ -541,7 +541,9 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
     float m[RU], rs[RU];
     if (own > 0) fetch(0, d, v, m, rs);
     int parity = 0;
-    for (int64_t r0 = 0; r0 < own; r0 += RU, parity ^= 1) {
+    // Left in the middle, where `more` is false: with that as a condition of its own besides the loop's, the compiler sees a way round
+    // on which the next rows' loads have not been waited for, and waits for each of them in front of the next.
+    for (int64_t r0 = 0; own > 0; r0 += RU, parity ^= 1) {
         Raw d_next[RU][NV], v_next[RU][NV];
         float m_next[RU], rs_next[RU];
         const bool more = r0 + RU < own;
@@ -590,6 +592,11 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
                 for (int k = 0; k < NV; ++k) {
                     const int c = threadIdx.x + k * THREADS;
                     if (c >= pieces) continue;
+                    if constexpr (NV * sizeof(T) == 16) {   // formed again: kept since the sums, h and t go to scratch memory
+                        asm volatile("" : "+v"(m[u]));
+#pragma unroll
+                        for (int i = 0; i < static_cast<int>(sizeof(T)); ++i) asm volatile("" : "+v"(d[u][k].word[i]));
+                    }
                     float dd[V], vv[V], gg[V], o[V];
                     P::get(d[u][k], dd);
                     P::get(v[u][k], vv);
@@ -600,13 +607,12 @@ __global__ __launch_bounds__(THREADS) void ln_bwd_block_rows(const T* __restrict
                 }
             }
         }
-        if (more) {
+        if (!more) break;
 #pragma unroll
-            for (int u = 0; u < RU; ++u) {
-                m[u] = m_next[u], rs[u] = rs_next[u];
+        for (int u = 0; u < RU; ++u) {
+            m[u] = m_next[u], rs[u] = rs_next[u];
 #pragma unroll
-                for (int k = 0; k < NV; ++k) d[u][k] = d_next[u][k], v[u][k] = v_next[u][k];
-            }
+            for (int k = 0; k < NV; ++k) d[u][k] = d_next[u][k], v[u][k] = v_next[u][k];
         }
     }
     float* out = partial + static_cast<int64_t>(blockIdx.x) * 2 * cols;
@@ -630,6 +636,8 @@ constexpr int64_t block_rows_cols(bool vec) { return vec ? 16384 : 8192; }
 // Training step of [8192, 8192] bf16, a run of rows to each workgroup -> so: 124.7 -> 123.3 us, with dy written right in front of it
 // (and counted) 179.4 -> 171.0; [60000, 1100] 282.5 -> 271.7; fp32 [8192, 4096] 171.6 -> 170.1.  Smaller ones are better off
 // in the usual order: [2048, 6000] 45.4 -> 44.9, but 46.2 with the last rows first.
+// Rows of more than 8192 columns fill the registers.  With the two remarks in the kernel left out, runs of rows -> in turn: fp32 [1175, 8216]
+// 31 -> 78 us, [2885, 11276] 82 -> 191, bf16 [2562, 11816] 45.6 -> 52.1; with them alike in bf16 and 1.02 to 1.09 times as fast in fp32.
 constexpr int64_t kInfinityCache = 256ll << 20;
 
 template <typename T, bool WITH_DX>
@@ -637,11 +645,12 @@ void launch_block_rows(bool vec, const T* dy, const T* x, int64_t rows, int64_t 
                        const float* rstd, const T* gamma, float* sums, int64_t splits, float* partial, float weight, T* dx, int64_t ld_dx,
                        hipStream_t s) {
     const bool backwards = 3 * rows * cols * static_cast<int64_t>(sizeof(T)) > kInfinityCache;
+    const int rows_each = static_cast<int>(rows / splits), rows_over = static_cast<int>(rows % splits);
     auto go_as = [&](auto threads, auto nv, auto ru, auto any) {
         constexpr int kThreads = decltype(threads)::value;
         hipLaunchKernelGGL((ln_bwd_block_rows<T, kThreads, decltype(nv)::value, decltype(ru)::value, WITH_DX, decltype(any)::value>),
-                           dim3(static_cast<uint32_t>(splits)), dim3(kThreads), 0, s, dy, x, rows, cols, ld_dy, ld_x, mean, rstd, gamma, sums,
-                           backwards, partial, weight, dx, ld_dx);
+                           dim3(static_cast<uint32_t>(splits)), dim3(kThreads), 0, s, dy, x, cols, ld_dy, ld_x, mean, rstd, gamma, sums,
+                           rows_each, rows_over, backwards, partial, weight, dx, ld_dx);
     };
     auto go = [&](auto threads, auto nv, auto ru) {
         if (vec) go_as(threads, nv, ru, std::false_type{});
