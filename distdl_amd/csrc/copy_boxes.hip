@@ -16,11 +16,11 @@
 // four launches of a repartition of [8, 4001, 6001] bf16 over four workers and its
 // adjoint 278, now 146; of [5, 1531, 3077] 43, now 31.)
 //
-// Device side: a workgroup moves a tile of 256 or 512 vectors shaped TR rows x TC
+// Device side: a workgroup moves tiles of 256, 512 or 1024 vectors shaped TR rows x TC
 // columns, TC a power of two (see columns_of_tile), so a vector's row and
 // column inside its tile are bit fields of its number; only the row needs
 // multiply-high divisions, and only when more than one outer dimension is left.
-// Workgroups of launches with more than a million tiles stride over them,
+// Workgroups of launches with many tiles stride over them,
 // loads and stores are non-temporal, and nothing but the box table -- passed by
 // value as kernel arguments and read with scalar loads -- is read besides the
 // payload.
@@ -43,13 +43,18 @@ constexpr uint32_t kTileLog = 10;  // log2(kTileVecs)
 static_assert((1u << kTileLog) == kTileVecs, "tile size must be 2^kTileLog");
 constexpr uint32_t tile_log(int vectors) { return vectors == 4 ? kTileLog : vectors == 2 ? kTileLog - 1 : kTileLog - 2; }   // of a lane
 constexpr uint32_t kPersistentBlocks = 1u << 20;   // workgroups of a launch; more tiles than that are strided over
-constexpr uint32_t kSumBlocks = 4096;              // of the sum kernels, 16 per CU
-// A box kernel's lanes move two vectors each, or one in launches of less than this: a lane's vectors wait for its addresses
-// and for each other, and with fewer of them there are more workgroups to hide that.  Crop and pad of [1, 32, 128^3] fp32 with
-// its adjoint: 191 us with four (and 4096 workgroups that stride), 181 with two, 201 with one.  Strips of an exchange of
-// [2, 5, 27^3] fp32 between eight workers and its adjoint, eleven launches: 52 us with four, 45 with two, 42 with one.  A
-// repartition of [5, 1531, 3077] bf16 between four workers, 735 thousand vectors a launch: 30 us, 29 and 33.
+constexpr uint32_t kStrideBlocks = 4096;           // of the sum kernels and of box kernels with four vectors a lane, 16 per CU
+// Vectors that a lane of a box kernel moves: it waits for its addresses and for each of its vectors, and with fewer of them there are
+// more workgroups to hide that, which cost more than they hide where there are many.  Of single boxes, time with four (and 4096
+// workgroups that stride) over that with one and two: less than 2^16 vectors 1.12 to 1.29 and 1.08 to 1.16; up to 2^18 1.02 to 1.17 and 1.02
+// to 1.13; up to 2^19 0.85 to 1.03 and 0.97 to 1.09; more than that by op and width: copies of 16-byte vectors 0.77 to 0.92 with one, with two
+// 0.87 to 0.97 up to 2^20 and 0.98 to 1.09 from there on; narrower ones and accumulation 0.50 to 0.90 and 0.71 to 0.96 (bf16 [130, 351, 302] added at
+// odd addresses 47 us with four, 71 with two).  Crop and pad of [1, 32, 128^3] fp32 with its adjoint: 191 us with four, 181 with two, 201 with
+// one.  Strips of an exchange of [2, 5, 27^3] fp32 between eight workers and its adjoint, eleven launches: 52, 45 and 42.
 constexpr uint64_t kFewVectors = 1u << 19;
+inline int vectors_of_a_lane(uint64_t vectors, bool streams) {   // streams: copies and zeros of 16-byte vectors
+    return vectors < kFewVectors / 2 ? 1 : vectors < kFewVectors || (streams && vectors >= 2 * kFewVectors) ? 2 : 4;
+}
 constexpr uint32_t kXcds = 8;                 // workgroups are dealt to the XCDs in turn
 constexpr uint64_t kMaxVecs = (1ull << 31) - kTileVecs;
 constexpr uint64_t kLongRunBytes = 64 << 10;   // boxes whose innermost runs are at least this long are interleaved within a launch
@@ -1039,7 +1044,9 @@ int launch_batches(const std::vector<DevBox>& boxes, hipStream_t stream) {
         }
         uint64_t tiles = number_tiles(bt, n, kTileLog);
         const bool uniform = OP == OP_COPY && uniform_batch(bt, n, tiles);
-        const int each = vectors < kFewVectors ? 1 : 2;
+        bool streams = OP == OP_COPY || OP == OP_ZERO;
+        for (uint32_t k = 0; k < n; ++k) streams = streams && bt.box[k].vlog == 4;
+        const int each = vectors_of_a_lane(vectors, streams);
         if (!uniform) {
             for (uint32_t k = 0; k < n; ++k) lay_out(bt.box[k], tile_log(each));
             tiles = number_tiles(bt, n, tile_log(each));
@@ -1076,16 +1083,17 @@ int launch_batches(const std::vector<DevBox>& boxes, hipStream_t stream) {
             if (int rc = launch_uniform(bt, n, static_cast<uint32_t>(tiles / n), interleave, stream)) return rc;
             continue;
         }
-        uint32_t most = kPersistentBlocks;
+        const uint32_t workgroups = each == 4 ? kStrideBlocks : kPersistentBlocks;
+        uint32_t most = workgroups;
         if (tiles < 0x40000000ull && share_lines(bt, n, equal)) {
             bt.rr = make_fastdiv(n);
             bt.rr.pad = static_cast<uint32_t>(tiles / n);
             tiles = (tiles / n + kXcds - 1) / kXcds * kXcds * n;
             bt.ntiles = static_cast<uint32_t>(tiles);
-            most = kPersistentBlocks / (kXcds * n) * (kXcds * n);
+            most = workgroups / (kXcds * n) * (kXcds * n);
         }
         const uint32_t blocks = tiles < most ? static_cast<uint32_t>(tiles) : most;
-        const auto kernel = each == 1 ? box_kernel<OP, T, 1> : box_kernel<OP, T, 2>;
+        const auto kernel = each == 1 ? box_kernel<OP, T, 1> : each == 2 ? box_kernel<OP, T, 2> : box_kernel<OP, T, kUnroll>;
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, stream, bt);
         if (int rc = check_launch("box_kernel")) return rc;
     }
@@ -1222,7 +1230,7 @@ int launch_sum(const std::vector<DevBox>& pieces, const void* const* srcs, int n
             const uint64_t rows_each = (1u << tile_log(1)) >> sa.box.tc_log;
             sa.ntiles = static_cast<uint32_t>(sa.box.col_tiles * ((sa.box.rows + rows_each - 1) / rows_each));
         }
-        const uint32_t blocks = sa.ntiles < kSumBlocks ? sa.ntiles : kSumBlocks;
+        const uint32_t blocks = sa.ntiles < kStrideBlocks ? sa.ntiles : kStrideBlocks;
 #define DDL_LAUNCH_SUM(MODE) \
     hipLaunchKernelGGL((few ? sum_kernel<T, MODE, 1> : sum_kernel<T, MODE, kUnroll>), dim3(blocks), dim3(kThreads), 0, stream, sa)
         if (sa.divide == kDivNone)

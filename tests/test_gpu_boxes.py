@@ -272,6 +272,31 @@ def test_boxes_at_the_number_of_vectors_a_lane_moves(ops, rows, run):
     assert torch.equal(x.cpu(), want)
 
 
+@pytest.mark.parametrize("op", ["copy", "add", "move"])
+@pytest.mark.parametrize("rows,run", [(1, 2 ** 18 - 1), (1, 2 ** 18 + 1), (513, 1023), (1, 2 ** 19 + 1), (1027, 1023), (1, 4096 * 1024 + 513)])
+def test_narrow_boxes_at_the_number_of_vectors_a_lane_moves(ops, op, rows, run):
+    """Elements of two bytes at odd places, one vector each: on either side of one, two and four a lane, and of more tiles than a launch
+    of four a lane has workgroups.  What lies between the rows stays as it is."""
+    from distdl_amd import _lib
+    gen = torch.Generator().manual_seed(run)
+    pitch = run + 3
+    x = torch.randint(-90, 90, (rows * pitch + 1,), generator=gen).to(torch.bfloat16).cuda()
+    out = torch.randint(-90, 90, (rows * pitch + 2,), generator=gen).to(torch.bfloat16).cuda()
+    want_x, want = x.clone(), out.clone()
+    src, dst = want_x[1:].view(rows, pitch)[:, :run], want[2:].view(rows, pitch)[:, :run]
+    if op == "add":
+        dst += src
+    else:
+        dst.copy_(src)
+    if op == "move":
+        src.zero_()
+    entry = (0, 1, 1, 2, (rows, run), (pitch, 1), (pitch, 1))
+    code = {"copy": _lib.DDL_OP_COPY, "add": _lib.DDL_OP_ADD, "move": _lib.DDL_OP_MOVE}[op]
+    ops.BoxLaunch([entry], 2).run([x.data_ptr(), out.data_ptr()], op=code, dtype=_lib.DDL_DT_BF16 if op == "add" else _lib.DDL_DT_BITS)
+    torch.cuda.synchronize()
+    assert torch.equal(bits(x), bits(want_x)) and torch.equal(bits(out), bits(want))
+
+
 def test_copy_box_strided_to_strided(ops):
     gen = torch.Generator().manual_seed(21)
     src = random_bits((7, 40, 9), torch.bfloat16, gen).cuda()
