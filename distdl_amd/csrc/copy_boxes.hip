@@ -50,10 +50,12 @@ constexpr uint32_t kStrideBlocks = 4096;           // of the sum kernels and of 
 // to 1.13; up to 2^19 0.85 to 1.03 and 0.97 to 1.09; more than that by op and width: copies of 16-byte vectors 0.77 to 0.92 with one, with two
 // 0.87 to 0.97 up to 2^20 and 0.98 to 1.09 from there on; narrower ones and accumulation 0.50 to 0.90 and 0.71 to 0.96 (bf16 [130, 351, 302] added at
 // odd addresses 47 us with four, 71 with two).  Crop and pad of [1, 32, 128^3] fp32 with its adjoint: 191 us with four, 181 with two, 201 with
-// one.  Strips of an exchange of [2, 5, 27^3] fp32 between eight workers and its adjoint, eleven launches: 52, 45 and 42.
+// one.  Where single vectors lie far apart, in the source or the result, copies and sums wait for memory more, and two are taken for all of
+// them: two slabs [1, 32, 130, 130, 1] fp32 out of rows of 130 13.8 us with two, 15.2 with four; into such rows 32.5 and 35.6.  Strips of an
+// exchange of [2, 5, 27^3] fp32 between eight workers and its adjoint, eleven launches: 52, 45 and 42.
 constexpr uint64_t kFewVectors = 1u << 19;
-inline int vectors_of_a_lane(uint64_t vectors, bool streams) {   // streams: copies and zeros of 16-byte vectors
-    return vectors < kFewVectors / 2 ? 1 : vectors < kFewVectors || (streams && vectors >= 2 * kFewVectors) ? 2 : 4;
+inline int vectors_of_a_lane(uint64_t vectors, bool streams, bool apart) {   // streams: copies and zeros of 16-byte vectors
+    return vectors < kFewVectors / 2 ? 1 : vectors < kFewVectors || apart || (streams && vectors >= 2 * kFewVectors) ? 2 : 4;
 }
 constexpr uint32_t kXcds = 8;                 // workgroups are dealt to the XCDs in turn
 constexpr uint64_t kMaxVecs = (1ull << 31) - kTileVecs;
@@ -1044,9 +1046,12 @@ int launch_batches(const std::vector<DevBox>& boxes, hipStream_t stream) {
         }
         uint64_t tiles = number_tiles(bt, n, kTileLog);
         const bool uniform = OP == OP_COPY && uniform_batch(bt, n, tiles);
-        bool streams = OP == OP_COPY || OP == OP_ZERO;
-        for (uint32_t k = 0; k < n; ++k) streams = streams && bt.box[k].vlog == 4;
-        const int each = vectors_of_a_lane(vectors, streams);
+        bool streams = OP == OP_COPY || OP == OP_ZERO, apart = OP == OP_COPY || OP == OP_ADD;
+        for (uint32_t k = 0; k < n; ++k) {
+            streams = streams && bt.box[k].vlog == 4;
+            apart = apart && std::max(bt.box[k].css, bt.box[k].cds) > (1 << bt.box[k].vlog);
+        }
+        const int each = vectors_of_a_lane(vectors, streams, apart);
         if (!uniform) {
             for (uint32_t k = 0; k < n; ++k) lay_out(bt.box[k], tile_log(each));
             tiles = number_tiles(bt, n, tile_log(each));
